@@ -12,7 +12,7 @@ import sys
 import numpy as np
 import torch
 
-sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "realtime-vla_amd"))
+sys.path.insert(0, os.path.abspath("realtime-vla_amd"))      # of the tree this is run in, which need not be the one this file lies in
 
 import synthetic as syn  # noqa: E402
 from dm0_infer import DM0Inference  # noqa: E402
