@@ -147,7 +147,7 @@ int rtvla_prepare(rtvla_ctx* ctx, void* hip_stream);
  * (rtvla_tile_layout_version, raised whenever that layout changes).  A caller may save that region and, in a later
  * process with the same weights bound, copy it back to the start of the workspace and call rtvla_prepare_with_tiles
  * instead of rtvla_prepare: it does everything rtvla_prepare does except the re-tiling. */
-#define RTVLA_TILE_LAYOUT_VERSION 2
+#define RTVLA_TILE_LAYOUT_VERSION 3
 size_t rtvla_tiled_bytes(const rtvla_ctx* ctx);
 int rtvla_tile_layout_version(void);
 int rtvla_prepare_with_tiles(rtvla_ctx* ctx, void* hip_stream);

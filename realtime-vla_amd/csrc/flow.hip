@@ -1,0 +1,969 @@
+// The action expert's flow-matching loop as ONE resident kernel (replaces the decoder-side launches of
+// /root/reference/pi0_infer.py:886-1230, pi05_infer.py:22-523 and dm0_infer.py:763-872).
+//
+// With at most 128 rows every GEMM of the loop is a few microseconds of latency: as launches, a layer is six dependent ones that
+// cost 2.3 us each before they do anything, and every one of them starts with cold L2s, because an XCD's L2 does not carry lines
+// across a launch boundary.  Here 256 workgroups, one per CU, stay resident for the whole loop and meet at barriers instead.
+//
+// Split of the work: the 8 XCDs are the ranks of a tensor-parallel group.  XCD x owns query head x (Pi0 / Pi05: 8 heads, one K/V head
+// whose new rows every XCD computes for itself; DM0: K/V head x with its two query heads) and one eighth of the MLP's hidden columns.
+// Everything an XCD produces for itself (q, k, v, probabilities, attention output, hidden, the residual stream) stays in memory that
+// only this XCD touches and is exchanged through its L2: plain stores, loads that pass the L1 (sc1), a barrier of 32 flags.  Only the
+// output and down projections produce sums over XCDs: each XCD writes its fp32 partial through to memory and CU r of every XCD waits
+// for the CUs r of the other seven (8 flags), then sums the tiles those eight produced in a fixed order.  A layer is
+//   qkv | logits + exp | P V | O partial || sum + residual | gate, up | down partial || sum + residual |      (| XCD barrier, || 8-CU barrier)
+// Measured on MI355X: XCD barrier 0.35 us (1.02 us with 1 KB stored per workgroup before it and 32 KB read after it, 1.43 us with
+// 64 KB), a barrier over all CUs 1.6 us, a dependent launch 2.3 us empty and 4.4-5.0 us as part of a layer.
+//
+// A CU holds RH of the 2 RH row tiles (CU parity) and the columns of one of 16 groups, so the activations of a phase are read once
+// into half the CUs each and the weights twice per XCD (once from memory).  The eight compute waves split K and reduce through LDS; a
+// ninth wave does the waiting, so that the compute waves can have the next phase's weights on the way while it polls.
+//
+// All workgroups have to be resident at once: the launcher keeps one flow kernel per device in flight, and a wait that lasts longer
+// than FLOW_WAIT_TICKS ends (the kernel then runs to its end without waiting and the actions become NaN), so the grid always drains.
+#include "kernels.h"
+#include <algorithm>
+#include <atomic>
+
+namespace {
+
+constexpr int FW = 8;                                    // compute waves
+constexpr int FLOW_THREADS = (FW + 2) * 64;              // + the wave that posts and polls flags, + the wave that fetches ahead
+constexpr unsigned long long FLOW_WAIT_TICKS = 200000000ull;      // 2 s of the 100 MHz counter
+constexpr float NEG_BIG = -1.0e30f;
+constexpr int SQ_BYTES = FW * 4 * 64;
+
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+typedef const __attribute__((address_space(4))) FlowP cFlowP;
+constexpr int SC1 = 16, SYS = 17;                        // cache policy of the buffer instructions: past the L1 / through to memory
+
+RTVLA_DEVICE rsrc_t make_rsrc(const void* base, unsigned bytes) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, 0x00027000); }
+RTVLA_DEVICE bf16x8 ld16(rsrc_t r, int off) { return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, SC1)); }
+RTVLA_DEVICE bf16x4 ld8(rsrc_t r, int off) { return __builtin_bit_cast(bf16x4, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, SC1)); }
+RTVLA_DEVICE float ld4(rsrc_t r, int off) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, SC1)); }
+RTVLA_DEVICE void st8(rsrc_t r, int off, bf16x4 v) { __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, off, 0, 0); }
+RTVLA_DEVICE void st16(rsrc_t r, int off, bf16x8 v) { __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, off, 0, 0); }
+RTVLA_DEVICE int ft_off(int row, int col, int cols32) { return (((row >> 4) * cols32 + (col >> 5)) * 64 + (row & 15) + 16 * ((col & 31) >> 3)) * 16 + (col & 7) * 2; }
+RTVLA_DEVICE int frag_off(int rt, int kb, int cols32, int lane) { return ((rt * cols32 + kb) * 64 + lane) * 16; }
+RTVLA_DEVICE bf16x8 ldw(const bf16_t* tiles, int nb, int kb, int K32p, int lane) { return *(const bf16x8*)(tiles + ((size_t)nb * K32p + kb) * 512 + lane * 8); }
+RTVLA_DEVICE bf16x8 cat44(bf16x4 lo, bf16x4 hi) {
+    bf16x8 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { v[j] = lo[j]; v[4 + j] = hi[j]; }
+    return v;
+}
+
+// The ids a phase starts from, hidden from the optimiser: every address in a phase follows from them, and all of those are loop
+// invariants that would be hoisted out of the layer loop into far more registers than there are.
+#define FLOW_IDS                                                                                     \
+    int lane = lane_, w = w_, x = x_, r = r_;                                                        \
+    asm volatile("" : "+v"(lane), "+s"(w), "+s"(x), "+s"(r));                                        \
+    [[maybe_unused]] const int g = lane >> 4, lr = lane & 15, half = r & 1, grp = r >> 1
+
+// A wait with an end: after FLOW_WAIT_TICKS the wave notes it in `abort`, stops waiting and runs to the end of the program.
+struct Patience {
+    unsigned long long t0 = 0;
+    int n = 0;
+    bool lost = false;
+    RTVLA_DEVICE void spin(FlowSync* sync, int lane) {
+        if ((++n & 255) != 0) return;
+        const unsigned long long now = __builtin_amdgcn_s_memrealtime();
+        if (n == 256) t0 = now;
+        else if (now - t0 > FLOW_WAIT_TICKS) {
+            lost = true;
+            if (lane == 0) atomicOr_system(&sync->abort, 1u);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+    }
+};
+
+// D[16 x 16] = A[16 x 16] B[16 x 16] of one half (4 elements per lane) of two 16 x 32 fragments
+RTVLA_DEVICE f32x4 mfma16k16(bf16x8 a, bf16x8 b, int hi) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    const bf16x4 a4 = {a[4 * hi], a[4 * hi + 1], a[4 * hi + 2], a[4 * hi + 3]}, b4 = {b[4 * hi], b[4 * hi + 1], b[4 * hi + 2], b[4 * hi + 3]};
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a4), __builtin_bit_cast(s16x4, b4), f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+}
+
+// what differs between the models' action experts
+template <int MODEL> struct Cfg;
+template <> struct Cfg<FLOW_PI0> {
+    static constexpr int HD = 256, HEADS = 1, AT = 3, ET = 2, EGRP = 16, FK = 2, FWAVES = 8, HID = 512, WD_K32 = 128;
+};
+template <> struct Cfg<FLOW_PI05> : Cfg<FLOW_PI0> {};
+template <> struct Cfg<FLOW_DM0> {
+    static constexpr int HD = 128, HEADS = 2, AT = 2, ET = 1, EGRP = 12, FK = 1, FWAVES = 6, HID = 192, WD_K32 = 64;
+};
+
+template <int MODEL, int RH>
+__global__ __launch_bounds__(FLOW_THREADS)
+void flow_kernel(FlowP kernel_args) {
+    using C = Cfg<MODEL>;
+    constexpr bool PI05 = MODEL == FLOW_PI05, DM0 = MODEL == FLOW_DM0;
+    constexpr int RTP = 2 * RH;                          // row tiles of the suffix
+    constexpr int QRT = RTP * C::HEADS;                  // row tiles of the queries of one XCD
+    constexpr int QRTP = QRT <= 2 ? 2 : QRT <= 4 ? 4 : 8;
+    constexpr int KD = C::HD / 32, DT = C::HD / 16, NDT = DT * QRTP / 32;      // d tiles per CU of the P V phase
+    constexpr int MC = RH < 2 ? RH : 2;                  // row tiles per pass of a GEMM phase (registers)
+    constexpr int HID32 = C::HID / 32;
+    constexpr int AK = (C::AT * RH + 7) / 8, SK = (4 * RH + 7) / 8;            // finished tiles per wave of the qkv and of the 4-column-tile phases
+    static_assert(QRT <= 8 && NDT >= 1, "row tiles of one XCD");
+
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    f32x4* const red = (f32x4*)smem;                                           // [wave][tile][64]
+    float* const sq = (float*)(smem + FW * 4 * RH * 1024);                     // [wave][RH * 16] row sums of squares; [2][wave][16] maxima and sums of P V
+    int* const sh = (int*)(smem + FW * 4 * RH * 1024 + SQ_BYTES);
+
+    // The parameters are read from the kernel-argument segment where they are used: hoisted out of the loops they would not fit the
+    // scalar registers.  prm() hides the pointer from the optimiser so that each phase loads its own.
+    auto prm = []() __attribute__((always_inline)) -> cFlowP& {
+        auto q = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(q));
+        return *(cFlowP*)q;
+    };
+
+    const int tid = threadIdx.x, lane_ = tid & 63;
+    const int w_ = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // the XCD this workgroup runs on and its number among the XCD's workgroups
+    if (tid == 0) {
+        const int xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7;         // HW_REG_XCC_ID
+        sh[0] = xcc;
+        sh[1] = (int)atomicAdd(&kernel_args.sync->rank[xcc * 32], 1u);
+    }
+    __syncthreads();
+    const int x_ = __builtin_amdgcn_readfirstlane(sh[0]), r_ = __builtin_amdgcn_readfirstlane(sh[1]);
+    if (r_ >= 32) { if (tid == 0) atomicOr(&kernel_args.sync->abort, 1u); return; }       // not 32 workgroups per XCD: the others give up waiting
+    const int step0 = kernel_args.step0, step1 = kernel_args.step1, layer0 = kernel_args.layer0, layer1 = kernel_args.layer1;
+    const bool begin = kernel_args.begin != 0, end = kernel_args.end != 0;
+    const bool keep_in = layer0 == layer1;                                     // (a single stage: the new stream goes back to the caller's buffer)
+    auto bar = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+    // ============ the waiting wave posts and polls the flags, the fetching wave pulls what comes up into the XCD's L2; both meet the
+    // ============ compute waves at every barrier
+    auto walk = [&](auto&& local, auto&& slot) __attribute__((always_inline)) {
+        if (!begin) local();
+        for (int t = step0; t < step1; ++t) {
+            if (begin) {
+                local();
+                if (!PI05) { bar(); if (!keep_in) local(); }
+            }
+            for (int l = layer0; l < layer1; ++l) {
+                slot(0, t, l); bar(); local();                                 // qkv
+                slot(1, t, l); local();                                        // logits
+                slot(2, t, l); bar(); local();                                 // P V
+                slot(3, t, l); bar(); slot(4, t, l); local();                  // output projection, exchange, sum
+                slot(5, t, l); bar(); local();                                 // gate, up
+                slot(6, t, l); bar(); slot(7, t, l); local();                  // down projection, exchange, sum
+            }
+            if (end) {
+                bar(); bar();
+                if (t + 1 < step1) local();
+            }
+        }
+    };
+    if (w_ == FW) {
+        const int lane = lane_, x = x_;
+        const unsigned* const flags = kernel_args.sync->lflag + x * 256 + lane * 4;      // 32 workgroups x 8 compute waves, 4 flags per lane
+        unsigned ep = 0;
+        Patience patience;
+        walk([&]() __attribute__((always_inline)) {
+                 ++ep;
+                 while (!patience.lost) {
+                     u32x4 v;
+                     asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=v"(v) : "v"(flags) : "memory");
+                     if (__all((int)(v[0] - ep) >= 0 && (int)(v[1] - ep) >= 0 && (int)(v[2] - ep) >= 0 && (int)(v[3] - ep) >= 0)) break;
+                     patience.spin(kernel_args.sync, lane);
+                 }
+                 patience.n = 0;
+                 bar();
+             },
+             [](int, int, int) __attribute__((always_inline)) {});
+        return;
+    }
+    if (w_ == FW + 1) {
+        // One word of every 128-byte line is loaded into a scrap of LDS: the line is then in this XCD's L2 when the compute waves ask for
+        // it, two to five phases later.  The 32 workgroups of an XCD share the lines out; a slot is 0.5 - 1 MB per XCD.
+        const unsigned scrap = (unsigned)(FW * 4 * RH * 1024 + SQ_BYTES + 64);
+        typedef const __attribute__((address_space(1))) void* gptr_t;
+        typedef __attribute__((address_space(3))) void* lptr_t;
+        auto touch = [&](const void* base, int first, int bytes, int lines64) __attribute__((always_inline)) {      // lines64 x 64 lines from byte `first` of `bytes`
+            for (int i = 0; i < lines64; ++i) {
+                const int off = min(first + (i * 64 + lane_) * 128, bytes - 128);
+                __builtin_amdgcn_global_load_lds((gptr_t)((const char*)base + off), (lptr_t)(smem + scrap), 4, 0, 0);
+            }
+        };
+        const int KBp = (kernel_args.prefix + 31) >> 5;
+        walk(bar, [&](int k, int t, int l) __attribute__((always_inline)) {
+            cFlowP& p = prm();
+            const int x = x_, r = r_;
+            int tn = t, ln = l + 1;                                            // the layer after this one
+            if (ln == layer1) { ln = layer0; tn = t + 1 < step1 ? t + 1 : t; }
+            if (k <= 2) {                                                      // gate and up tiles of this layer: 2 x 32 KB of every workgroup, in thirds
+                if (r < C::HID / 16) {
+                    const size_t o = (size_t)(PI05 ? t * p.layers + l : l) * p.wg_stride + (size_t)(x * (C::HID / 16) + r) * 32 * 512;
+                    if (k == 0) touch(p.wg + o, 0, 32768, 3);
+                    if (k == 1) { touch(p.wg + o, 3 * 8192, 32768, 1); touch(p.wu + o, 0, 32768, 2); }
+                    if (k == 2) touch(p.wu + o, 2 * 8192, 32768, 2);
+                }
+            } else if (k == 3) {                                               // down projection of this layer: this XCD's K slice of two column tiles
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    touch(p.wd + (size_t)l * p.wd_stride + ((size_t)(2 * r + j) * C::WD_K32 + x * HID32) * 512, 0, HID32 * 1024, (HID32 + 7) / 8);
+            } else if (k == 4 || k == 5) {                                     // qkv of the next layer: AT * 16 tiles of 32 KB
+                const bf16_t* base = p.wqkv + (size_t)(PI05 ? tn * p.layers + ln : ln) * p.wqkv_stride;
+                const int hf = r * C::AT + (k == 4 ? 0 : 1);                   // half tiles of 16 KB, AT per workgroup
+                auto half_tile = [&](int h) __attribute__((always_inline)) {
+                    const int grp = (h >> 1) & 15, j = (h >> 1) >> 4;
+                    const int nb = DM0 ? (j == 0 ? x * 16 + grp : (grp < 8 ? 128 + x * 8 + grp : 192 + x * 8 + grp - 8)) : (j == 0 ? x * 16 + grp : j == 1 ? 128 + grp : 144 + grp);
+                    touch(base + (size_t)nb * 32 * 512, (h & 1) * 16384, 32768, 2);
+                };
+                half_tile(hf);
+                if (k == 5 && C::AT == 3) half_tile(hf + 1);
+            } else if (k == 6) {                                               // cached K and V^T of the next layer
+                const size_t o = (size_t)(DM0 ? ln * 8 + x : ln) * p.kv_stride;
+                for (int kb = r; kb < KBp; kb += 32) touch(p.kcache + o + (size_t)kb * 2 * KD * 512, 0, 2 * KD * 1024, 2 * KD / 8);
+                constexpr int SH = 32 / DT;                                    // workgroups per 16-wide d tile
+                const int vb = KBp * 1024 / SH;
+                touch(p.vcache + o + (size_t)(r / SH) * (p.ldvt >> 5) * 512, (r % SH) * vb, KBp * 1024, (vb + 8191) >> 13);
+            } else {                                                           // output projection of the next layer
+#pragma unroll
+                for (int j = 0; j < 2; ++j) touch(p.wo + (size_t)ln * p.wo_stride + ((size_t)(2 * r + j) * 64 + x * 8) * 512, 0, 8192, 1);
+            }
+        });
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                       // nothing may land in LDS after the workgroup has ended
+        return;
+    }
+
+    // ================================================= the compute waves =================================================
+    const rsrc_t priv = make_rsrc(kernel_args.priv + (size_t)x_ * kernel_args.priv_stride, (unsigned)kernel_args.priv_stride);
+    const rsrc_t part = make_rsrc(kernel_args.part, kernel_args.part_bytes);
+    const int rows = kernel_args.rows;
+    const int KBp = (kernel_args.prefix + 31) >> 5, KB = KBp + ((rows + 31) >> 5);       // 32-key blocks: cached prefix, all
+    int vl = kernel_args.prefix;
+    if (kernel_args.valid_len) vl = max(0, min(*kernel_args.valid_len, vl));
+    const float sc2 = kernel_args.scale * 1.4426950408889634f;
+    // this wave's stores are done -> its flag; `pre` runs while the waiting wave polls the flags of the XCD's 256 compute waves
+    unsigned ep = 0;
+    const unsigned* const my_flag = kernel_args.sync->lflag + x_ * 256 + r_ * FW + w_;
+    auto sync = [&](auto&& pre) __attribute__((always_inline)) {
+        ++ep;
+        asm volatile("s_waitcnt vmcnt(0)\n\tglobal_store_dword %0, %1, off" ::"v"(my_flag), "v"(ep) : "memory");      // (every lane stores the same word)
+        pre();
+        bar();
+    };
+
+    // ---- one GEMM phase: NT column tiles x RH row tiles, K of this wave = NK blocks; partial sums to LDS ----
+    // `swap`: tile index from which on the product is taken as rows x columns instead of columns x rows
+    auto gemm = [&]<int NT, int NK>(const bf16x8 (&wt)[NT][NK], int a_base, int a_cols32, int kb0, bool with_sq, int swap) __attribute__((always_inline)) {
+        FLOW_IDS;
+#pragma unroll
+        for (int m0 = 0; m0 < RH; m0 += MC) {
+            bf16x8 a[MC][NK];
+#pragma unroll
+            for (int m = 0; m < MC; ++m)
+#pragma unroll
+                for (int i = 0; i < NK; ++i)
+                    if (m0 + m < RH) a[m][i] = ld16(priv, a_base + frag_off(half * RH + m0 + m, kb0 + i, a_cols32, lane));
+            f32x4 acc[MC][NT];
+#pragma unroll
+            for (int m = 0; m < MC; ++m)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < NK; ++i)
+#pragma unroll
+                for (int m = 0; m < MC; ++m)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
+                        if (m0 + m < RH) acc[m][t] = t >= swap ? mfma16(a[m][i], wt[t][i], acc[m][t]) : mfma16(wt[t][i], a[m][i], acc[m][t]);
+            if (with_sq) {
+#pragma unroll
+                for (int m = 0; m < MC; ++m) {
+                    if (m0 + m >= RH) continue;
+                    float s = 0.f, s1 = 0.f;
+#pragma unroll
+                    for (int i = 0; i < NK; ++i)
+#pragma unroll
+                        for (int j = 0; j < 8; j += 4) {
+                            const bf16x2 v = {a[m][i][j], a[m][i][j + 1]}, v1 = {a[m][i][j + 2], a[m][i][j + 3]};
+                            s = __builtin_amdgcn_fdot2_f32_bf16(v, v, s, false);
+                            s1 = __builtin_amdgcn_fdot2_f32_bf16(v1, v1, s1, false);
+                        }
+                    s = rows_sum(s + s1);
+                    if (g == 0) sq[w * (RH * 16) + (m0 + m) * 16 + lr] = s;
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < MC; ++m)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    if (m0 + m < RH) red[((size_t)w * (NT * RH) + t * RH + m0 + m) * 64 + lane] = acc[m][t];
+        }
+    };
+    auto tile_sum = [&](int lane, int ntiles, int u, int waves) __attribute__((always_inline)) {
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ww = 0; ww < FW; ++ww) if (ww < waves) v += red[((size_t)ww * ntiles + u) * 64 + lane];
+        return v;
+    };
+    auto row_factor = [&](int row_in_half) __attribute__((always_inline)) {    // RMS factor of one row of this CU's half
+        float t = 0.f;
+#pragma unroll
+        for (int ww = 0; ww < FW; ++ww) t += sq[ww * (RH * 16) + row_in_half];
+        const float f = rsqrtf(t * (1.0f / 1024.0f) + 1e-6f);
+        return MODEL == FLOW_PI0 ? round_bf16(f) : f;
+    };
+
+    // ---- weights of the phases ----
+    auto a_tile = [](int x, int grp, int t) __attribute__((always_inline)) {                  // column tile of the QKV matrix
+        if constexpr (DM0) return t == 0 ? x * 16 + grp : (grp < 8 ? 128 + x * 8 + grp : 192 + x * 8 + grp - 8);
+        else return t == 0 ? x * 16 + grp : t == 1 ? 128 + grp : 144 + grp;
+    };
+    auto load_a = [&](cFlowP& p, int t, int l, bf16x8 (&wA)[C::AT][4]) __attribute__((always_inline)) {
+        FLOW_IDS;
+        const bf16_t* base = p.wqkv + (size_t)(PI05 ? t * p.layers + l : l) * p.wqkv_stride;
+#pragma unroll
+        for (int j = 0; j < C::AT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) wA[j][i] = ldw(base, a_tile(x, grp, j), w * 4 + i, 32, lane);
+    };
+    auto load_c = [&](cFlowP& p, int l, bf16x8 (&wC)[4][1]) __attribute__((always_inline)) {
+        FLOW_IDS;
+        const bf16_t* base = p.wo + (size_t)l * p.wo_stride;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) wC[j][0] = ldw(base, grp * 4 + j, x * 8 + w, 64, lane);
+    };
+    auto load_e = [&](cFlowP& p, int t, int l, int part, bf16x8 (&wE)[2 * C::ET][4]) __attribute__((always_inline)) {
+        FLOW_IDS;
+        const size_t o = (size_t)(PI05 ? t * p.layers + l : l) * p.wg_stride;
+        const int hb = x * (C::HID / 16) + min(grp, C::EGRP - 1) * C::ET;       // (loads are not made conditional anywhere: the compiler spills around it)
+#pragma unroll
+        for (int j = part * C::ET; j < (part + 1) * C::ET; ++j)                // part 0: gate, 1: up
+#pragma unroll
+            for (int i = 0; i < 4; ++i) wE[j][i] = ldw((j < C::ET ? p.wg : p.wu) + o, hb + j % C::ET, w * 4 + i, 32, lane);
+    };
+    auto load_f = [&](cFlowP& p, int l, bf16x8 (&wF)[4][C::FK]) __attribute__((always_inline)) {
+        FLOW_IDS;
+        const bf16_t* base = p.wd + (size_t)l * p.wd_stride;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < C::FK; ++i) wF[j][i] = ldw(base, grp * 4 + j, x * HID32 + min(w, C::FWAVES - 1) * C::FK + i, C::WD_K32, lane);
+    };
+
+    // ---- qkv: RMS factor (Pi0, Pi05), RoPE, new K / V rows ----
+    auto pre_qkv = [&](cFlowP& p, int t, int l, bf16x8 (&wA)[C::AT][4], bf16x4 (&pre_cs)[AK]) __attribute__((always_inline)) {
+        FLOW_IDS;
+        load_a(p, t, l, wA);
+        if constexpr (!DM0) {
+#pragma unroll
+            for (int k = 0; k < AK; ++k) {
+                const int u = w + 8 * k;
+                pre_cs[k] = load4(p.rope + (size_t)min((half * RH + u % RH) * 16 + lr, rows - 1) * 256 + grp * 16 + 4 * g);
+            }
+        }
+    };
+    auto qkv = [&](cFlowP& p, int t, int l, const bf16x8 (&wA)[C::AT][4], const bf16x4 (&pre_cs)[AK]) __attribute__((always_inline)) {
+        FLOW_IDS;
+        constexpr int NT = C::AT;
+        gemm.template operator()<NT, 4>(wA, p.off_x, 32, w * 4, true, DM0 ? (grp >= 8 ? 1 : 9) : 2);
+        bar();
+        if (w < FW) {
+#pragma unroll
+            for (int k = 0; k < (NT * RH + 7) / 8; ++k) {
+                const int u = w + 8 * k;
+                if (NT * RH % FW != 0 && u >= NT * RH) continue;
+                const int j = u / RH, m = u % RH;
+                f32x4 v = tile_sum(lane, NT * RH, u, FW);
+                const int row0 = (half * RH + m) * 16;
+                if constexpr (DM0) {
+                    // raw products, rounded as the reference's QKV buffer; V carries the row's RMS factor, Q and K get it with their norm
+                    if (j == 0) st8(priv, p.off_q + ft_off(((grp >> 3) * RTP) * 16 + row0 + lr, (grp & 7) * 16 + 4 * g, KD), pack4(v));
+                    else if (grp < 8) st8(priv, p.off_k + ft_off(row0 + lr, grp * 16 + 4 * g, KD), pack4(v));
+                    else {
+                        const int d = (grp - 8) * 16 + lr, key = row0 + 4 * g;
+                        f32x4 o;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o[e] = round_bf16(v[e]) * row_factor(m * 16 + 4 * g + e);
+                        st8(priv, p.off_v + (((d >> 4) * 4 + (key >> 5)) * 64 + (d & 15) + 16 * ((key & 15) >> 2)) * 16 + 8 * ((key & 31) >> 4), pack4(o));
+                    }
+                } else if (j < 2) {
+                    v *= row_factor(m * 16 + lr);
+                    const int n0 = grp * 16 + 4 * g;
+                    if constexpr (PI05) v += *(const f32x4*)(p.bias_qkv + (size_t)(t * p.layers + l) * 2560 + (j == 0 ? x * 256 : 2048) + n0);
+                    const bf16x4 cs = pre_cs[k];
+                    const float c0 = bf2f(cs[0]), s0 = bf2f(cs[1]), c1 = bf2f(cs[2]), s1 = bf2f(cs[3]);
+                    const bf16x4 o = pack4(v[0] * c0 - v[1] * s0, v[1] * c0 + v[0] * s0, v[2] * c1 - v[3] * s1, v[3] * c1 + v[2] * s1);
+                    const int row = row0 + lr;
+                    st8(priv, (j == 0 ? p.off_q : p.off_k) + ft_off(row, n0, 8), o);
+                    // the cache rows behind the prefix, as the reference keeps them (nothing here reads them back)
+                    if (j == 1 && x == 0 && row < rows) store4(p.kcache + (size_t)l * p.kv_stride + ft_index(p.prefix + row, n0, 8), o);
+                } else {                                                       // V: lane holds 4 keys of one column
+                    const int d = grp * 16 + lr, key = row0 + 4 * g;
+                    float b = 0.f;
+                    if constexpr (PI05) b = p.bias_qkv[(size_t)(t * p.layers + l) * 2560 + 2304 + d];
+                    f32x4 o;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[e] = v[e] * row_factor(m * 16 + 4 * g + e) + b;
+                    const bf16x4 pk = pack4(o);
+                    st8(priv, p.off_v + (((d >> 4) * 4 + (key >> 5)) * 64 + (d & 15) + 16 * ((key & 15) >> 2)) * 16 + 8 * ((key & 31) >> 4), pk);
+                    if (x == 0) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (key + e < rows) p.vcache[(size_t)l * p.kv_stride + vt_index(d, p.prefix + key + e, p.ldvt >> 5)] = pk[e];
+                    }
+                }
+            }
+            if constexpr (DM0) {                                               // the row factors, once per row half
+                if (grp == 0 && w == FW - 1 && lane < RH * 16) {
+                    const float f = row_factor(lane);
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, f), priv, p.off_f + (half * RH * 16 + lane) * 4, 0, 0);
+                }
+            }
+        }
+    };
+
+    // DM0: factor, RMS norm over the head's 128 features, norm weight, rotary embedding on adjacent pairs; lane holds 8 features per block
+    auto dm0_qk = [&](cFlowP& p, int g, bf16x8 (&v)[KD], int tok, const bf16_t* nw) __attribute__((always_inline)) {
+        const float f = ld4(priv, p.off_f + tok * 4);
+        const int rr = min(tok, rows - 1);
+        bf16x8 cs[KD], ww[KD];
+#pragma unroll
+        for (int kd = 0; kd < KD; ++kd) { cs[kd] = *(const bf16x8*)(p.rope + (size_t)rr * 128 + kd * 32 + 8 * g); ww[kd] = *(const bf16x8*)(nw + kd * 32 + 8 * g); }
+        float y[KD][8], s = 0.f;
+#pragma unroll
+        for (int kd = 0; kd < KD; ++kd)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) { y[kd][j] = bf2f(v[kd][j]) * f; s += y[kd][j] * y[kd][j]; }
+        const float inv = rsqrtf(rows_sum(s) * (1.0f / 128.0f) + 1e-6f);
+#pragma unroll
+        for (int kd = 0; kd < KD; ++kd)
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                const float a = y[kd][j] * inv * bf2f(ww[kd][j]), b = y[kd][j + 1] * inv * bf2f(ww[kd][j + 1]);
+                const float c = bf2f(cs[kd][j]), sn = bf2f(cs[kd][j + 1]);
+                v[kd][j] = f2bf(a * c - b * sn); v[kd][j + 1] = f2bf(b * c + a * sn);
+            }
+    };
+
+    // ---- logits of (query row tile, 16 keys) per wave and their exponentials relative to the row maximum over those 16 keys ----
+    // Workgroup: the 32-key blocks r, r + 32, ...; wave: one half of the block (w & 1), row tiles (w >> 1), + 4, ...
+    auto load_k = [&](cFlowP& p, int lane, int x, int l, int nt, int kb, bf16x8 (&kf)[KD]) __attribute__((always_inline)) {
+        const bf16_t* base = p.kcache + (size_t)(DM0 ? l * 8 + x : l) * p.kv_stride;
+#pragma unroll
+        for (int kd = 0; kd < KD; ++kd) kf[kd] = *(const bf16x8*)(base + ((size_t)((kb * 2 + nt) * KD + kd) * 64 + lane) * 8);
+    };
+    auto pre_logits = [&](cFlowP& p, int l, bf16x8 (&kf)[KD]) __attribute__((always_inline)) {
+        FLOW_IDS;
+        load_k(p, lane, x, l, w & 1, min(r, KBp - 1), kf);
+    };
+    auto logits = [&](cFlowP& p, int l, bf16x8 (&kf)[KD]) __attribute__((always_inline)) {
+        FLOW_IDS;
+        const int nt = w & 1;
+        for (int kb = r; kb < KB; kb += 32) {
+            if (kb >= KBp) {
+#pragma unroll
+                for (int kd = 0; kd < KD; ++kd) kf[kd] = ld16(priv, p.off_k + frag_off((kb - KBp) * 2 + nt, kd, KD, lane));
+                if constexpr (DM0) dm0_qk(p, g, kf, ((kb - KBp) * 2 + nt) * 16 + lr, p.knorm + (size_t)l * 128);
+            } else if (kb >= 32) load_k(p, lane, x, l, nt, kb, kf);
+            // the keys of this lane: 4 g .. 4 g + 3 of the 16; visible are those below `lim` (of the state row, among the new keys, only the first)
+            const int key = nt * 16 + 4 * g;
+            const int lim = kb < KBp ? vl - kb * 32 : rows - (kb - KBp) * 32;
+            const int lim_state = kb < KBp ? lim : KBp == kb ? 1 : 0;
+            for (int rt = w >> 1; rt < QRT; rt += 4) {
+                bf16x8 qf[KD];
+#pragma unroll
+                for (int kd = 0; kd < KD; ++kd) qf[kd] = ld16(priv, p.off_q + frag_off(rt, kd, KD, lane));
+                const int tok = (rt % RTP) * 16 + lr;
+                if constexpr (DM0) dm0_qk(p, g, qf, tok, p.qnorm + (size_t)l * 128);
+                f32x4 st = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int kd = 0; kd < KD; ++kd) st = mfma16(kf[kd], qf[kd], st);
+                const int lm = (MODEL == FLOW_PI0 && tok == 0) ? lim_state : lim;      // the state token sees the prefix and itself
+                float mx = NEG_BIG;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    st[e] = key + e < lm ? st[e] * sc2 : NEG_BIG;
+                    mx = fmaxf(mx, st[e]);
+                }
+                mx = rows_max(mx);
+                float sum = 0.f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    st[e] = key + e < lm ? __builtin_amdgcn_exp2f(st[e] - mx) : 0.f;
+                    sum += st[e];
+                }
+                sum = rows_sum(sum);
+                // this half's four probabilities of the lane's 16-byte piece of the P^T fragment
+                st8(priv, p.off_p + ((rt * KB + kb) * 64 + lane) * 16 + nt * 8, pack4(st));
+                if (g == 0) __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(mx), __float_as_uint(sum)}, priv, p.off_m + ((rt * KB + kb) * 16 + lr) * 16 + nt * 8, 0, 0);
+            }
+        }
+    };
+
+    // ---- O = P V for one query row tile and NDT 16-wide column tiles; the waves split the key blocks, every 16 keys with their own factor ----
+    constexpr int VB = 4;                                                      // blocks of a wave per trip (32 key blocks per workgroup)
+    auto load_v = [&](cFlowP& p, int lane, int x, int pdg, int l, int kb, bf16x8 (&v)[NDT]) __attribute__((always_inline)) {
+        const bf16_t* base = p.vcache + (size_t)(DM0 ? l * 8 + x : l) * p.kv_stride;
+#pragma unroll
+        for (int d = 0; d < NDT; ++d) v[d] = *(const bf16x8*)(base + ((size_t)((pdg * NDT + d) * (p.ldvt >> 5) + kb) * 64 + lane) * 8);
+    };
+    auto pre_pv = [&](cFlowP& p, int l, bf16x8 (&vf)[VB][NDT]) __attribute__((always_inline)) {
+        FLOW_IDS;
+        const int pdg = r / QRTP;
+#pragma unroll
+        for (int i = 0; i < VB; ++i) load_v(p, lane, x, pdg, l, min(w + FW * i, KBp - 1), vf[i]);
+    };
+    auto pv = [&](cFlowP& p, int l, bf16x8 (&vf)[VB][NDT]) __attribute__((always_inline)) {
+        FLOW_IDS;
+        const int prt = r % QRTP, pdg = r / QRTP;
+        if (QRT == QRTP || prt < QRT) {
+            f32x4 o[NDT];
+#pragma unroll
+            for (int d = 0; d < NDT; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+            float M = NEG_BIG, L = 0.f;
+            for (int b0 = 0; b0 < KB; b0 += VB * FW) {
+                bf16x8 pf[VB];
+                f32x4 mo[VB];                                                  // {max, sum} of both halves
+#pragma unroll
+                for (int i = 0; i < VB; ++i) {
+                    const int kb = min(b0 + w + FW * i, KB - 1);
+                    mo[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(priv, p.off_m + ((prt * KB + kb) * 16 + lr) * 16, 0, SC1));
+                    pf[i] = ld16(priv, p.off_p + ((prt * KB + kb) * 64 + lane) * 16);
+                }
+#pragma unroll
+                for (int i = 0; i < VB; ++i) {
+                    const int kb = b0 + w + FW * i;
+                    if (kb >= KBp && kb < KB)
+#pragma unroll
+                        for (int d = 0; d < NDT; ++d) vf[i][d] = ld16(priv, p.off_v + (((pdg * NDT + d) * 4 + kb - KBp) * 64 + lane) * 16);
+                    else if (b0 > 0) load_v(p, lane, x, pdg, l, min(kb, KBp - 1), vf[i]);
+                }
+                float m = M;
+#pragma unroll
+                for (int i = 0; i < VB; ++i)
+                    if (b0 + w + FW * i < KB) m = fmaxf(m, fmaxf(mo[i][0], mo[i][2]));
+                if (b0 > 0) {
+                    const float f = __builtin_amdgcn_exp2f(M - m);
+                    L *= f;
+#pragma unroll
+                    for (int d = 0; d < NDT; ++d) o[d] *= f;
+                }
+                M = m;
+#pragma unroll
+                for (int i = 0; i < VB; ++i) {
+                    const bool in = b0 + w + FW * i < KB;
+                    const float f0 = in ? __builtin_amdgcn_exp2f(mo[i][0] - M) : 0.f, f1 = in ? __builtin_amdgcn_exp2f(mo[i][2] - M) : 0.f;
+                    L += f0 * mo[i][1] + f1 * mo[i][3];
+#pragma unroll
+                    for (int d = 0; d < NDT; ++d) o[d] += f0 * mfma16k16(vf[i][d], pf[i], 0) + f1 * mfma16k16(vf[i][d], pf[i], 1);
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < NDT; ++d) red[((size_t)w * NDT + d) * 64 + lane] = o[d];
+            if (g == 0) { sq[w * 16 + lr] = M; sq[FW * 16 + w * 16 + lr] = L; }
+        }
+        bar();
+        if (w < NDT && (QRT == QRTP || prt < QRT)) {
+            float mw[FW], M = NEG_BIG, L = 0.f;
+#pragma unroll
+            for (int ww = 0; ww < FW; ++ww) { mw[ww] = sq[ww * 16 + lr]; M = fmaxf(M, mw[ww]); }
+            f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ww = 0; ww < FW; ++ww) {
+                const float f = __builtin_amdgcn_exp2f(mw[ww] - M);
+                L += f * sq[FW * 16 + ww * 16 + lr];
+                v += f * red[((size_t)ww * NDT + w) * 64 + lane];
+            }
+            v *= L > 0.f ? 1.0f / L : 0.f;
+            const int tok = (prt % RTP) * 16 + lr, col = (prt / RTP) * C::HD + (pdg * NDT + w) * 16 + 4 * g;
+            st8(priv, p.off_o + ft_off(tok, col, 8), pack4(v));
+        }
+    };
+
+    // ---- partial sums over this XCD's share of K, exchanged with the CUs r of the other XCDs ----
+    // The values are their own flags: a buffer is all ones (a NaN no sum produces) until its values arrive, so a reader polls the data
+    // and saves the write acknowledgement, the flag and a second read.  Three buffers take turns: once the partials of exchange e are
+    // here, every peer has read exchange e - 1, so that buffer of this workgroup is set to ones again; it is written next in exchange
+    // e + 2, which a peer only looks at after it has received this workgroup's exchange e + 1, sent behind a wait for those ones.
+    // Tile layout: 64 bytes per row, so that the rows past the last one are neither written nor read.
+    int ex = 0;                                                                // exchange number modulo 3
+    Patience patience;
+    auto part_off = [&](int buf, int y, int r, int u, int lane) __attribute__((always_inline)) {
+        return (((buf * 8 + y) * 32 + r) * (4 * RH) + u) * 1024 + ((lane & 15) * 4 + (lane >> 4)) * 16;
+    };
+    auto store_part = [&](int waves, f32x4 (&own)[SK]) __attribute__((always_inline)) {
+        FLOW_IDS;
+#pragma unroll
+        for (int k = 0; k < SK; ++k) {
+            const int u = w + 8 * k;
+            if (4 * RH % FW == 0 || u < 4 * RH) {
+                own[k] = tile_sum(lane, 4 * RH, u, waves);
+                if ((half * RH + u % RH) * 16 + lr < rows) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, own[k]), part, part_off(ex, x, r, u, lane), 0, SYS);
+            }
+        }
+    };
+    // The peers' tiles are requested, then `pre` (weights of the next phase) runs in their shadow; what had not arrived is asked for again.
+    auto sum_residual = [&](cFlowP& p, bool keep, const f32x4 (&own)[SK], const bf16_t* gp, auto&& pre) __attribute__((always_inline)) {
+        FLOW_IDS;
+#pragma unroll
+        for (int k = 0; k < SK; ++k) {
+            const int u = w + 8 * k, row = (half * RH + u % RH) * 16 + lr, col = (grp * 4 + u / RH) * 16 + 4 * g;
+            const bool in = (4 * RH % FW == 0 || u < 4 * RH) && row < rows;
+            // (this XCD's own tile is at hand: its request, like those of rows past the end, is moved behind the end of the buffer, where
+            // the hardware returns zero and reads nothing)
+            auto load = [&](int y) __attribute__((always_inline)) {
+                return __builtin_amdgcn_raw_buffer_load_b128(part, in && y != x ? part_off(ex, y, r, u, lane) : 0x7fffff00, 0, SYS);
+            };
+            u32x4 v[8];
+#pragma unroll
+            for (int y = 0; y < 8; ++y) v[y] = load(y);
+            const bf16x4 xold = ld8(priv, p.off_x + ft_off(row, col, 32));
+            bf16x4 gate = {};
+            if constexpr (PI05) gate = load4(gp + col);
+            if (k == 0) {
+                __builtin_amdgcn_sched_barrier(0);
+                pre();
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            for (;;) {
+                bool missing = false;
+#pragma unroll
+                for (int y = 0; y < 8; ++y)
+                    if (__any(v[y][0] == ~0u || v[y][1] == ~0u || v[y][2] == ~0u || v[y][3] == ~0u)) { v[y] = load(y); missing = true; }
+                if (!missing || patience.lost) break;
+                patience.spin(p.sync, lane);
+            }
+            patience.n = 0;
+            if (in) {
+                f32x4 sum = {0.f, 0.f, 0.f, 0.f};                              // in the order of the XCDs on each of them
+#pragma unroll
+                for (int y = 0; y < 8; ++y) sum += y == x ? own[k] : __builtin_bit_cast(f32x4, v[y]);
+                if constexpr (PI05) for (int e = 0; e < 4; ++e) sum[e] *= bf2f(gate[e]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[e] += bf2f(xold[e]);
+                const bf16x4 o = pack4(sum);
+                st8(priv, p.off_x + ft_off(row, col, 32), o);
+                if (keep && x == 0) store4(p.x + ft_index(row, col, 32), o);
+            }
+        }
+        ex = ex == 2 ? 0 : ex + 1;
+    };
+    auto reset_part = [&]() __attribute__((always_inline)) {                   // of the exchange before the one just summed; runs behind the next flag
+        FLOW_IDS;
+        const int last = ex == 2 ? 0 : ex + 1;                                 // two back from the one to come
+#pragma unroll
+        for (int k = 0; k < SK; ++k) {
+            const int u = w + 8 * k;
+            if ((4 * RH % FW == 0 || u < 4 * RH) && (half * RH + u % RH) * 16 + lr < rows)
+                __builtin_amdgcn_raw_buffer_store_b128(u32x4{~0u, ~0u, ~0u, ~0u}, part, part_off(last, x, r, u, lane), 0, SYS);
+        }
+    };
+
+    // ---- gate / up ----
+    auto mlp_up = [&](cFlowP& p, int t, int l, const bf16x8 (&wE)[2 * C::ET][4]) __attribute__((always_inline)) {
+        FLOW_IDS;
+        constexpr int NT = 2 * C::ET;
+        if (C::EGRP == 16 || grp < C::EGRP) gemm.template operator()<NT, 4>(wE, p.off_x, 32, w * 4, true, 9);
+        bar();
+        if (w < C::ET * RH && (C::EGRP == 16 || grp < C::EGRP)) {
+            const int j = w / RH, m = w % RH;
+            f32x4 gv = tile_sum(lane, NT * RH, w, FW), uv = tile_sum(lane, NT * RH, C::ET * RH + w, FW);
+            const float f = row_factor(m * 16 + lr);
+            gv *= f; uv *= f;
+            const int hc = (grp * C::ET + j) * 16 + 4 * g;
+            if constexpr (PI05) {
+                const size_t o = (size_t)(t * p.layers + l) * 4096 + x * C::HID + hc;
+                gv += *(const f32x4*)(p.bias_gate + o); uv += *(const f32x4*)(p.bias_up + o);
+            }
+            f32x4 h;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = (DM0 ? siluf(gv[e]) : gelu_tanh(gv[e])) * uv[e];
+            st8(priv, p.off_h + ft_off((half * RH + m) * 16 + lr, hc, HID32), pack4(h));
+        }
+    };
+
+    // ---- start of a flow step: noise -> input projection (+ SiLU, MLP) -> residual stream ----
+    const int s0 = MODEL == FLOW_PI0 ? 1 : 0;                                  // action rows follow the state token
+    auto action_in = [&](cFlowP& p, int t) __attribute__((always_inline)) {
+        FLOW_IDS;
+        const bool first = t == step0;
+#pragma unroll
+        for (int k = 0; k < (2 * RTP + 7) / 8; ++k) {
+            const int u = w + 8 * k;
+            if (2 * RTP % FW != 0 && u >= 2 * RTP) continue;
+            const int ct = 2 * r + (u & 1), rt = u >> 1;
+            const int arow = max(0, min(rt * 16 + lr - s0, rows - s0 - 1));
+            const bf16x8 nz = first ? *(const bf16x8*)(p.noise + arow * 32 + 8 * g) : ld16(priv, p.off_n + arow * 64 + 16 * g);
+            const bf16x8 wi = ldw(p.win, ct, 0, 4, lane);
+            const bf16x4 b = load4(p.bin + (PI05 ? 0 : (size_t)t * 1024) + ct * 16 + 4 * g);
+            f32x4 v = {bf2f(b[0]), bf2f(b[1]), bf2f(b[2]), bf2f(b[3])};
+            v = mfma16(wi, nz, v);
+            if constexpr (!PI05) for (int e = 0; e < 4; ++e) v[e] = siluf(v[e]);
+            st8(priv, (PI05 ? p.off_x : p.off_xin) + ft_off(rt * 16 + lr, ct * 16 + 4 * g, 32), pack4(v));
+        }
+    };
+    auto pre_mlp_in = [&](cFlowP& p, bf16x8 (&wM)[4][4]) __attribute__((always_inline)) {
+        FLOW_IDS;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) wM[j][i] = ldw(p.wmlp, grp * 4 + j, w * 4 + i, 32, lane);
+    };
+    auto mlp_in = [&](cFlowP& p, bool keep, const bf16x8 (&wM)[4][4]) __attribute__((always_inline)) {
+        FLOW_IDS;
+        gemm.template operator()<4, 4>(wM, p.off_xin, 32, w * 4, false, 9);
+        bar();
+        {
+#pragma unroll
+            for (int k = 0; k < SK; ++k) {
+                const int u = w + 8 * k;
+                if (4 * RH % FW != 0 && u >= 4 * RH) continue;
+                f32x4 v = tile_sum(lane, 4 * RH, u, FW);
+                const int row = (half * RH + u % RH) * 16 + lr, col = (grp * 4 + u / RH) * 16 + 4 * g;
+                const bf16x4 b = load4(p.bmlp + col);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] += bf2f(b[e]);
+                bf16x4 o = pack4(v);
+                if (MODEL == FLOW_PI0 && row == 0) o = load4(p.state_x + col);
+                st8(priv, p.off_x + ft_off(row, col, 32), o);
+                if (keep && x == 0) store4(p.x + ft_index(row, col, 32), o);
+            }
+        }
+    };
+
+    // ---- end of a flow step: final norm, output projection, Euler update of the noise (CU: one 16 x 16 tile) ----
+    auto euler = [&](cFlowP& p, int t) __attribute__((always_inline)) {
+        FLOW_IDS;
+        const int urt = r >> 1, uct = r & 1;
+        const bool first = t == step0, last = t == step1 - 1;
+        const int row = urt * 16 + lr, arow = row - s0;
+        bf16x8 a[4], wU[4];
+        if (urt < RTP) {
+            float s = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) wU[i] = ldw(p.wout, uct, w * 4 + i, 32, lane);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a[i] = ld16(priv, p.off_x + frag_off(urt, w * 4 + i, 32, lane));
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 8; j += 2) {
+                    const bf16x2 v = {a[i][j], a[i][j + 1]};
+                    s = __builtin_amdgcn_fdot2_f32_bf16(v, v, s, false);
+                }
+            s = rows_sum(s);
+            if (g == 0) sq[w * (RH * 16) + lr] = s;
+        }
+        bar();
+        if (urt < RTP) {
+            if constexpr (PI05) {                                              // adaptive norm: x f (1 + scale) + shift before the product
+                const float f = row_factor(lr);
+                const bf16_t* st = p.style_final + (size_t)t * 3072;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const bf16x8 sc = *(const bf16x8*)(st + (w * 4 + i) * 32 + 8 * g), shf = *(const bf16x8*)(st + 1024 + (w * 4 + i) * 32 + 8 * g);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) a[i][j] = f2bf(bf2f(a[i][j]) * f * (1.0f + bf2f(sc[j])) + bf2f(shf[j]));
+                }
+            }
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc = mfma16(wU[i], a[i], acc);
+            red[(size_t)w * 64 + lane] = acc;
+        }
+        bar();
+        if (w == 0 && urt < RTP && arow >= 0 && row < rows) {
+            const int col = uct * 16 + 4 * g;
+            f32x4 v = tile_sum(lane, 1, 0, FW);
+            if constexpr (!PI05) v *= row_factor(lr);
+            const bf16x4 b = load4(p.bout + col);
+            const bf16x4 old = first ? load4(p.noise + arow * 32 + col) : ld8(priv, p.off_n + arow * 64 + col * 2);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = v[e] + bf2f(b[e]) + bf2f(old[e]);
+            const bf16x4 o = pack4(v);
+            st8(priv, p.off_n + arow * 64 + col * 2, o);
+            if (last && x == 0) {
+                unsigned bad;
+                asm volatile("global_load_dword %0, %1, off sc0 sc1\n\ts_waitcnt vmcnt(0)" : "=v"(bad) : "v"(&p.sync->abort) : "memory");
+                const float nan = __uint_as_float(0x7fc00000u);
+                store4(p.noise_out + arow * 32 + col, bad ? pack4(nan, nan, nan, nan) : o);
+            }
+        }
+    };
+
+    // ---- the program (the waiting wave above walks through the same one) ----
+    auto nothing = []() __attribute__((always_inline)) {};
+    auto copy_x = [&](bool in) __attribute__((always_inline)) {
+        FLOW_IDS;
+        cFlowP& p = prm();
+        for (int i = r * FW + w; i < RTP * 32; i += 32 * FW) {
+            const size_t at = ((size_t)i * 64 + lane) * 8;
+            if (in) st16(priv, p.off_x + (i * 64 + lane) * 16, *(const bf16x8*)(p.x + at));
+            else if (x == 0) *(bf16x8*)(p.x + at) = ld16(priv, p.off_x + (i * 64 + lane) * 16);
+        }
+    };
+    bf16x8 wA[C::AT][4];
+    bf16x4 cs[AK];
+    if (!begin) {                                                              // a single stage: the stream comes from the caller's buffer
+        copy_x(true);
+        sync([&]() __attribute__((always_inline)) { pre_qkv(prm(), step0, layer0 < layer1 ? layer0 : 0, wA, cs); });
+    }
+    for (int t = step0; t < step1; ++t) {
+        if (begin) {
+            action_in(prm(), t);
+            if constexpr (PI05) {
+                sync([&]() __attribute__((always_inline)) { pre_qkv(prm(), t, layer0, wA, cs); });
+                if (keep_in) copy_x(false);
+            } else {
+                bf16x8 wM[4][4];
+                sync([&]() __attribute__((always_inline)) { pre_mlp_in(prm(), wM); });
+                mlp_in(prm(), keep_in, wM);
+                if (!keep_in) sync([&]() __attribute__((always_inline)) { pre_qkv(prm(), t, layer0, wA, cs); });
+            }
+        }
+        for (int l = layer0; l < layer1; ++l) {
+            const bool lastl = l == layer1 - 1;
+            qkv(prm(), t, l, wA, cs);
+            {
+                bf16x8 kf[KD];
+                sync([&]() __attribute__((always_inline)) { pre_logits(prm(), l, kf); });
+                logits(prm(), l, kf);
+            }
+            {
+                bf16x8 vf[VB][NDT];
+                sync([&]() __attribute__((always_inline)) { pre_pv(prm(), l, vf); });
+                pv(prm(), l, vf);
+            }
+            {
+                bf16x8 wE[2 * C::ET][4];
+                f32x4 own[SK];
+                {
+                    bf16x8 wC[4][1];
+                    sync([&]() __attribute__((always_inline)) { load_c(prm(), l, wC); load_e(prm(), t, l, 0, wE); });
+                    gemm.template operator()<4, 1>(wC, prm().off_o, 8, w_, false, 9);
+                }
+                bar();
+                store_part(FW, own);
+                cFlowP& p = prm();
+                sum_residual(p, false, own, PI05 ? p.style_attn + ((size_t)t * p.layers + l) * 3072 + 2048 : nullptr,
+                             [&]() __attribute__((always_inline)) { load_e(prm(), t, l, 1, wE); });
+                sync(reset_part);
+                mlp_up(prm(), t, l, wE);
+            }
+            {
+                f32x4 own[SK];
+                {
+                    bf16x8 wF[4][C::FK];
+                    sync([&]() __attribute__((always_inline)) { load_f(prm(), l, wF); });
+                    if (C::FWAVES == FW || w_ < C::FWAVES) gemm.template operator()<4, C::FK>(wF, prm().off_h, HID32, w_ * C::FK, false, 9);
+                }
+                bar();
+                store_part(C::FWAVES, own);
+                cFlowP& p = prm();
+                sum_residual(p, lastl, own, PI05 ? p.style_ffn + ((size_t)t * p.layers + l) * 3072 + 2048 : nullptr,
+                             [&]() __attribute__((always_inline)) { pre_qkv(prm(), t, lastl ? l : l + 1, wA, cs); });      // (after the last layer for nothing)
+            }
+            sync(reset_part);
+        }
+        if (end) {
+            euler(prm(), t);
+            if (t + 1 < step1) sync(nothing);
+        }
+    }
+}
+
+// zeroes the flags, sets the exchange buffers to ones and, for Pi0, projects the state token (row 0 of the residual stream, the same in every flow step)
+__global__ __launch_bounds__(256) void flow_init_kernel(FlowSync* sync, uint4* part, int part16, const bf16_t* state, const bf16_t* w, const bf16_t* b, bf16_t* out) {
+    const int i = blockIdx.x * 256 + threadIdx.x, n = gridDim.x * 256;
+    unsigned* s = (unsigned*)sync;
+    for (int k = i; k < (int)(sizeof(FlowSync) / 4); k += n) s[k] = 0;
+    for (int k = i; k < part16; k += n) part[k] = uint4{~0u, ~0u, ~0u, ~0u};
+    if (state && i < 1024) {
+        float acc = bf2f(b[i]);
+        bf16_t wc[32];
+#pragma unroll
+        for (int k = 0; k < 32; ++k) wc[k] = w[(size_t)k * 1024 + i];
+#pragma unroll
+        for (int k = 0; k < 32; ++k) acc += bf2f(state[k]) * bf2f(wc[k]);
+        out[i] = f2bf(acc);
+    }
+}
+
+__global__ __launch_bounds__(FLOW_THREADS) void flow_check_kernel(FlowSync* sync) {
+    if (threadIdx.x != 0) return;
+    const int xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7;
+    if (atomicAdd(&sync->rank[xcc * 32], 1u) >= 32u) atomicOr(&sync->abort, 1u);
+    __hip_atomic_fetch_add(&sync->lflag[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+    while (__hip_atomic_load(&sync->lflag[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < 256u)
+        if (__builtin_amdgcn_s_memrealtime() - t0 > 5000000ull) { atomicOr(&sync->abort, 1u); break; }      // 50 ms
+}
+
+template <int MODEL, int RH>
+int launch_inst(const FlowP& p, hipStream_t s) {
+    const size_t smem = std::max((size_t)FW * 4 * RH * 1024 + SQ_BYTES + 64 + 256, (size_t)96 * 1024);      // more than half a CU's LDS: one workgroup per CU
+    auto kern = flow_kernel<MODEL, RH>;
+    static std::atomic<uint64_t> done{0};
+    if (int rc = ensure_dynamic_lds((const void*)kern, smem, done)) return rc;
+    hipLaunchKernelGGL(kern, dim3(256), dim3(FLOW_THREADS), smem, s, p);
+    return hipGetLastError() == hipSuccess ? 0 : 5;
+}
+
+}  // namespace
+
+int flow_row_pairs(int rows) { return (rows + 31) / 32; }
+
+size_t flow_layout(FlowP* p, int qtiles, int blocks, int hidden) {
+    size_t at = 0;
+    auto take = [&](size_t bytes) { const int o = (int)at; at += (bytes + 255) & ~(size_t)255; return o; };
+    p->off_x = take(128 * 1024 * 2); p->off_xin = take(128 * 1024 * 2);
+    p->off_q = take((size_t)std::max(qtiles, 8) * 16 * 256 * 2); p->off_k = take(128 * 256 * 2); p->off_v = take(256 * 128 * 2);
+    p->off_o = take(128 * 256 * 2); p->off_h = take((size_t)128 * hidden * 2); p->off_n = take(128 * 32 * 2); p->off_f = take(128 * 4);
+    p->off_m = take((size_t)qtiles * blocks * 16 * 16); p->off_p = take((size_t)qtiles * blocks * 1024);
+    return (at + 4095) & ~(size_t)4095;
+}
+
+void launch_flow_init(FlowSync* sync, float* part, unsigned part_bytes, const bf16_t* state, const bf16_t* w, const bf16_t* b, bf16_t* out, hipStream_t s) {
+    hipLaunchKernelGGL(flow_init_kernel, dim3(512), dim3(256), 0, s, sync, (uint4*)part, (int)(part_bytes / 16), state, w, b, out);
+}
+
+int launch_flow(const FlowP& p, int model, hipStream_t s) {
+    if (p.rows < 1 || p.rows > (model == FLOW_DM0 ? 64 : 128) || p.prefix < 1 || (p.ldvt & 31) || p.ldvt < p.prefix + p.rows) return 1;
+    if (p.step0 < 0 || p.step1 <= p.step0 || p.layer0 < 0 || p.layer1 < p.layer0 || p.layer1 > p.layers) return 1;
+    if (p.begin && !p.end && p.step1 != p.step0 + 1) return 1;
+    const int rh = flow_row_pairs(p.rows);
+    if (model == FLOW_PI0) {
+        switch (rh) { case 1: return launch_inst<FLOW_PI0, 1>(p, s); case 2: return launch_inst<FLOW_PI0, 2>(p, s); case 3: return launch_inst<FLOW_PI0, 3>(p, s); case 4: return launch_inst<FLOW_PI0, 4>(p, s); }
+    } else if (model == FLOW_PI05) {
+        switch (rh) { case 1: return launch_inst<FLOW_PI05, 1>(p, s); case 2: return launch_inst<FLOW_PI05, 2>(p, s); case 3: return launch_inst<FLOW_PI05, 3>(p, s); case 4: return launch_inst<FLOW_PI05, 4>(p, s); }
+    } else if (model == FLOW_DM0) {
+        switch (rh) { case 1: return launch_inst<FLOW_DM0, 1>(p, s); case 2: return launch_inst<FLOW_DM0, 2>(p, s); }
+    }
+    return 2;
+}
+
+// Whether the flow kernel's assumption holds here: 256 workgroups of its size are resident together, 32 on each of 8 XCDs (not so on
+// a partitioned device or under a CU mask).  Tried once per device with a kernel that does nothing else; every wait in it ends.
+bool flow_supported(FlowSync* sync, hipStream_t s) {
+    static std::atomic<int> known[64];                                         // 0: not tried, 1: yes, 2: no
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+    if (const int k = known[dev].load(std::memory_order_acquire)) return k == 1;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
+    bool ok = cus == 256;
+    if (ok) {
+        const size_t smem = 96 * 1024;
+        unsigned bad = 1;
+        ok = hipFuncSetAttribute((const void*)flow_check_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) == hipSuccess;
+        if (ok) {
+            launch_flow_init(sync, nullptr, 0, nullptr, nullptr, nullptr, nullptr, s);
+            hipLaunchKernelGGL(flow_check_kernel, dim3(256), dim3(FLOW_THREADS), smem, s, sync);
+            ok = hipGetLastError() == hipSuccess && hipMemcpyAsync(&bad, &sync->abort, sizeof bad, hipMemcpyDeviceToHost, s) == hipSuccess &&
+                 hipStreamSynchronize(s) == hipSuccess && bad == 0;
+        }
+    }
+    known[dev].store(ok ? 1 : 2, std::memory_order_release);
+    return ok;
+}

@@ -168,6 +168,38 @@ int launch_flash_attention(const AttnP& p, int hd, hipStream_t s);
 // SigLIP attention: q, k fragment-tiled [views*16][256][96], vt tiled [views*16][80][256], out row-major
 void launch_vision_attention(const bf16_t* q, const bf16_t* k, const bf16_t* vt, bf16_t* out, int views, hipStream_t s);
 
+// ----- the action expert's flow loop as one resident kernel (csrc/flow.hip) ------------------------------------
+enum FlowModel { FLOW_PI0 = 0, FLOW_PI05, FLOW_DM0 };
+struct FlowSync { unsigned rank[8 * 32], lflag[8 * 256], abort, pad[31]; };
+struct FlowP {
+    // program: flow steps [step0, step1), each: input projection (begin), layers [layer0, layer1), output projection + Euler (end)
+    int step0, step1, layer0, layer1, begin, end;
+    int layers, rows, prefix;                  // layers of the model, suffix rows (state token included), prefix rows as allocated
+    const int* valid_len;                      // visible prefix rows, or null: all
+    float scale;
+    // tiled weights of layer 0 (Pi05 qkv / gate / up: of flow step 0, layer 0) and the distance to the next one, in elements
+    const bf16_t *wqkv, *wo, *wg, *wu, *wd; size_t wqkv_stride, wo_stride, wg_stride, wd_stride;
+    const float *bias_qkv, *bias_gate, *bias_up;                        // Pi05: shift * W of the adaptive norms
+    const bf16_t *style_attn, *style_ffn, *style_final;                 // Pi05: [scale | shift | gate]
+    const bf16_t *win, *bin, *wmlp, *bmlp, *wout, *bout;                // input projection (tiled), its bias (per step but for Pi05), input MLP, output projection
+    const bf16_t *qnorm, *knorm;                                        // DM0
+    const bf16_t* rope;                        // [row][256] (DM0: 128)
+    const bf16_t* state_x;                     // Pi0: the projected state token
+    bf16_t *kcache, *vcache; size_t kv_stride; int ldvt;
+    const bf16_t* noise; bf16_t* noise_out;    // [chunk][32], may be the same
+    bf16_t* x;                                 // residual stream, fragment-tiled: read by programs without `begin`, written by all
+    char* priv; size_t priv_stride;            // memory of one XCD's own, 8 of them
+    int off_x, off_xin, off_q, off_k, off_v, off_o, off_h, off_n, off_f, off_m, off_p;
+    float* part; unsigned part_bytes;          // fp32 partial sums exchanged between the XCDs
+    FlowSync* sync;
+};
+int flow_row_pairs(int rows);                  // the kernel's row-tile pairs (template argument) for that many suffix rows
+// byte offsets inside one XCD's memory; returns its size.  qrows: query row tiles per XCD, blocks: 32-key blocks, hidden: MLP columns per XCD
+size_t flow_layout(FlowP* p, int qtiles, int blocks, int hidden);
+void launch_flow_init(FlowSync* sync, float* part, unsigned part_bytes, const bf16_t* state, const bf16_t* w, const bf16_t* b, bf16_t* out, hipStream_t s);
+int launch_flow(const FlowP& p, int model, hipStream_t s);
+bool flow_supported(FlowSync* sync, hipStream_t s);      // whether the current device can run it (tried once per device; synchronises then)
+
 // Row-major q [tokens][kv_heads][group][hd], k / v [keys][kv_heads][hd] -> the kernels' layouts per K/V head b: Q fragment-tiled
 // [row = local token * group + head][hd_pad] at qt + b' * q_bstride, K fragment-tiled [key][hd_pad], V^T tiled [hd][keys_pad];
 // with seq > 0 the tokens / keys form independent sequences of `seq` (SigLIP views) and b' = sequence * kv_heads + b.  The

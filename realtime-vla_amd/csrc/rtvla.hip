@@ -11,6 +11,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -51,6 +52,8 @@ struct rtvla_ctx {
     size_t act_begin = 0;          // activations start here (cleared at prepare)
     char* ws = nullptr;
     bool prepared = false;
+    bool flow = false;             // the flow loop runs as one resident kernel (csrc/flow.hip); false: as launches, see flow_supported()
+    FlowP flow_p{};                // its private-memory layout (build_tables)
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     hipStream_t timing_stream = nullptr;     // the measurement helpers capture graphs, which the null stream cannot
@@ -174,6 +177,17 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
     return bc;
 }
 
+// what the resident flow kernel needs besides the model's buffers
+void add_flow_buffers(rtvla_ctx* c, int heads, int hidden) {
+    const int rh = flow_row_pairs(c->S_d);
+    c->flow_p.priv_stride = flow_layout(&c->flow_p, 2 * rh * heads, (c->S_e + 31) / 32 + (c->S_d + 31) / 32, hidden);
+    c->add_buf("flow_priv", 8, (int64_t)c->flow_p.priv_stride / 4, (int64_t)c->flow_p.priv_stride / 4, 4);
+    c->flow_p.part_bytes = 3u * 8 * 32 * 4 * rh * 1024;
+    c->add_buf("flow_part", 1, c->flow_p.part_bytes / 4, c->flow_p.part_bytes / 4, 4);
+    c->add_buf("flow_sync", 1, sizeof(FlowSync) / 4, sizeof(FlowSync) / 4, 4);
+    c->add_buf("flow_state_x", 1, 1024, 1024);
+}
+
 int build_tables(rtvla_ctx* c) {
     const rtvla_dims& d = c->d;
     const int64_t V = d.vision_layers, L = d.llm_layers, v = d.num_views, ch = d.chunk_size;
@@ -270,6 +284,7 @@ int build_tables(rtvla_ctx* c) {
     c->add_tiled("t_decoder_ffn_up_w", 1024, 4096, L);
     c->add_tiled("t_decoder_ffn_down_w", 4096, 1024, L);
     c->add_tiled("t_decoder_out_proj_w", 1024, 32, 1);
+    c->add_tiled("t_decoder_action_in_w", 32, 1024, 1);
     if (!pi05) {
         c->add_tiled("t_decoder_action_mlp_w", 1024, 1024, 1);
     } else {
@@ -322,6 +337,7 @@ int build_tables(rtvla_ctx* c) {
     const int64_t pmax = std::max(S_v * 1152, S_e * 2048) * 8;
     c->add_buf("splitk_partial", 1, pmax, pmax, 4);
     c->add_buf("attn_partial", 1, ATTN_PARTIAL_FLOATS, ATTN_PARTIAL_FLOATS, 4);
+    add_flow_buffers(c, 1, 512);
     return 0;
 }
 
@@ -402,6 +418,7 @@ int build_tables_dm0(rtvla_ctx* c) {
     c->add_tiled("t_decoder_ffn_down_w", 2048, 1024, L);              // K = 1536 zero-padded to the 2048 the streaming kernel takes
     c->add_tiled("t_decoder_action_mlp_w", 1024, 1024, 1);
     c->add_tiled("t_decoder_out_proj_w", 1024, 32, 1);
+    c->add_tiled("t_decoder_action_in_w", 32, 1024, 1);
     c->act_begin = c->ws_bytes;
     const int64_t M = n * DM0_SEQ_PAD;                                       // every image owns 2720 rows of the row-major ViT buffers
     c->add_buf("const_ones", 1, 1024, 1024);
@@ -436,6 +453,7 @@ int build_tables_dm0(rtvla_ctx* c) {
     const int64_t pmax = std::max(M * 1024, P * 2048) * 8;
     c->add_buf("splitk_partial", 1, pmax, pmax, 4);
     c->add_buf("attn_partial", 1, ATTN_PARTIAL_FLOATS, ATTN_PARTIAL_FLOATS, 4);
+    add_flow_buffers(c, 2, 192);
     return 0;
 }
 
@@ -559,10 +577,52 @@ struct Sched {
         SkinnyP p{}; p.a_tiled = 1; p.a_row0 = a_row0; p.out_tiled = 1; p.out_row0 = out_row0; return p;
     }
 
+    // Flow steps [step0, step1), each with its input projection (begin), layers [layer0, layer1) and Euler update (end), in one launch of
+    // the resident kernel
+    void flow(int step0, int step1, int layer0, int layer1, bool begin, bool end, const char* what) {
+        const bool dm0 = d.model == RTVLA_DM0;
+        FlowP p = c->flow_p;
+        p.step0 = step0; p.step1 = step1; p.layer0 = layer0; p.layer1 = layer1; p.begin = begin; p.end = end;
+        p.layers = d.llm_layers; p.rows = c->S_d; p.prefix = c->S_e; p.valid_len = valid_len();
+        p.scale = dm0 ? 0.08838834764831845f : 0.0625f;
+        p.wqkv = c->TW(pi05 ? "t_decoder_attn_qkv_ada" : "t_decoder_attn_qkv_w"); p.wqkv_stride = c->BI(pi05 ? "t_decoder_attn_qkv_ada" : "t_decoder_attn_qkv_w").ld;
+        p.wo = c->TW("t_decoder_attn_o_w"); p.wo_stride = c->BI("t_decoder_attn_o_w").ld;
+        p.wg = c->TW(pi05 ? "t_decoder_ffn_gate_ada" : "t_decoder_ffn_gate_w"); p.wu = c->TW(pi05 ? "t_decoder_ffn_up_ada" : "t_decoder_ffn_up_w");
+        p.wg_stride = c->BI("t_decoder_ffn_gate_w").ld;
+        p.wd = c->TW("t_decoder_ffn_down_w"); p.wd_stride = c->BI("t_decoder_ffn_down_w").ld;
+        p.win = c->TW("t_decoder_action_in_w"); p.wout = c->TW("t_decoder_out_proj_w");
+        p.rope = c->W("decoder_rope_weights"); p.ldvt = c->keys_pad;
+        if (pi05) {
+            p.bias_qkv = c->B<float>("decoder_ada_bias_qkv"); p.bias_gate = c->B<float>("decoder_ada_bias_gate"); p.bias_up = c->B<float>("decoder_ada_bias_up");
+            p.style_attn = c->B("decoder_style_attn"); p.style_ffn = c->B("decoder_style_ffn"); p.style_final = c->B("decoder_style_final");
+            p.bin = c->W("decoder_action_in_proj_b"); p.bout = c->B("decoder_out_proj_b_scaled");
+        } else {
+            p.bin = c->W("decoder_action_fused_time_biases"); p.bout = c->W("decoder_action_fused_out_proj_b");
+            p.wmlp = c->TW("t_decoder_action_mlp_w"); p.bmlp = c->W("decoder_action_mlp_b");
+        }
+        if (dm0) {
+            p.qnorm = c->W("decoder_q_norm_w"); p.knorm = c->W("decoder_k_norm_w");
+            p.kcache = c->B("kv_K"); p.vcache = c->B("kv_Vt"); p.kv_stride = (size_t)c->keys_pad * 128;
+        } else {
+            p.kcache = Kc(0); p.vcache = Vt(0); p.kv_stride = (size_t)c->keys_pad * 256;
+        }
+        p.noise = c->W("diffusion_noise"); p.noise_out = c->W("diffusion_noise"); p.x = c->B("decoder_x");
+        p.priv = (char*)c->B<float>("flow_priv"); p.part = c->B<float>("flow_part"); p.sync = (FlowSync*)c->B<float>("flow_sync");
+        bf16_t* const sx = c->B("flow_state_x");
+        p.state_x = sx;
+        if (c->want("flow init")) {
+            const bool st = begin && !pi05 && !dm0;
+            launch_flow_init(p.sync, p.part, p.part_bytes, st ? c->W("observation_state_normalized") : nullptr, st ? c->W("decoder_state_in_proj_w") : nullptr, st ? c->W("decoder_state_in_proj_b") : nullptr, sx, s);
+            c->note(0, "flow init");
+        }
+        if (c->want(what)) c->note(launch_flow(p, dm0 ? FLOW_DM0 : pi05 ? FLOW_PI05 : FLOW_PI0, s), what);
+    }
+
     void suffix_init() {}
 
     void suffix_step_begin(int t) {
         const int ch = d.chunk_size;
+        if (c->flow) { flow(t, t + 1, 0, 0, true, false, "flow step begin"); return; }
         if (!pi05) {
             // state token -> row 0 of the residual stream (re-projected every step: the stream is updated in place) and the fused
             // action/time input projection + SiLU -> decoder_x_buf, as ONE launch: the two are independent
@@ -587,6 +647,7 @@ struct Sched {
 
     void suffix_layer(int t, int i) {
         const int S_d = c->S_d, S_e = c->S_e, L = d.llm_layers;
+        if (c->flow) { flow(t, t + 1, i, i + 1, false, false, "flow layer"); return; }
         const int norm = pi05 ? SN_ADARMS : SN_RMS;
         const bf16_t* st_attn = pi05 ? c->B("decoder_style_attn") + ((size_t)t * L + i) * 3072 : nullptr;
         const bf16_t* st_ffn = pi05 ? c->B("decoder_style_ffn") + ((size_t)t * L + i) * 3072 : nullptr;
@@ -621,6 +682,7 @@ struct Sched {
 
     void suffix_step_end(int t) {
         const int ch = d.chunk_size;
+        if (c->flow) { flow(t, t + 1, 0, 0, false, true, "flow step end"); return; }
         SkinnyP e{}; e.a_tiled = 1; e.out = c->W("diffusion_noise"); e.ldo = 32;       // noise stays row-major [chunk][32]
         if (!pi05) {
             e.a_row0 = 1;                                                               // action rows follow the state token
@@ -728,6 +790,7 @@ struct Sched {
     // dm0_infer.py:763-780
     void dm0_step_begin(int t) {
         const int ch = d.chunk_size;
+        if (c->flow) { flow(t, t + 1, 0, 0, true, false, "flow step begin"); return; }
         if (c->want("action in")) {
             launch_small_linear(c->W("diffusion_noise"), 32, c->W("decoder_action_fused_in_proj_w"), c->W("decoder_action_fused_time_biases", 1024, t % 10),
                                 c->B("decoder_x_buf"), 1024, ch, 32, 1024, 1, 1, 0, s);
@@ -740,6 +803,7 @@ struct Sched {
     // dm0_infer.py:782-851
     void dm0_suffix_layer(int t, int i) {
         const int ch = d.chunk_size, P = c->S_e, kp = c->keys_pad;
+        if (c->flow) { flow(t, t + 1, i, i + 1, false, false, "flow layer"); return; }
         SkinnyP q{}; q.a_tiled = 1; q.out = c->B("decoder_qkv"); q.ldo = 4096; q.bias = c->B("const_zeros");
         skinny(c->B("decoder_x"), 1024, ch, c->TW("t_decoder_attn_qkv_w", i), nullptr, 1024, 4096, SN_NONE, nullptr, SK_BIAS, q, "suffix qkv");
         if (c->want("suffix qk-norm rope")) {
@@ -765,6 +829,7 @@ struct Sched {
 
     // dm0_infer.py:863-872, :99-120
     void dm0_step_end(int t) {
+        if (c->flow) { flow(t, t + 1, 0, 0, false, true, "flow step end"); return; }
         SkinnyP e{}; e.a_tiled = 1; e.out = c->W("diffusion_noise"); e.ldo = 32; e.bias = c->W("decoder_action_fused_out_proj_b"); e.factor_f32 = 1;
         skinny(c->B("decoder_x"), 1024, d.chunk_size, c->TW("t_decoder_out_proj_w"), nullptr, 1024, 32, SN_RMS, nullptr, SK_RES, e, "euler");
     }
@@ -798,6 +863,7 @@ struct Sched {
             launch_pretile_padded(c->W("decoder_ffn_down_w", (size_t)1536 * 1024, i), 1536, 2048, 1024, c->TW("t_decoder_ffn_down_w", i), s);
         tile("decoder_action_mlp_w", "t_decoder_action_mlp_w", 1024, 1024, 1);
         tile("decoder_action_fused_out_proj_w", "t_decoder_out_proj_w", 1024, 32, 1);
+        tile("decoder_action_fused_in_proj_w", "t_decoder_action_in_w", 32, 1024, 1);
     }
 
     int dm0_stage(int st, int layer, int step) {
@@ -822,6 +888,7 @@ struct Sched {
         for (int i = 0; i < d.vision_layers; ++i) dm0_vision_layer(i);
         dm0_project();
         for (int i = 0; i < d.llm_layers; ++i) dm0_prefix_layer(i);
+        if (c->flow) { flow(0, d.num_steps, 0, d.llm_layers, true, true, "flow loop"); return; }
         for (int t = 0; t < d.num_steps; ++t) {
             dm0_step_begin(t);
             for (int i = 0; i < d.llm_layers; ++i) dm0_suffix_layer(t, i);
@@ -858,6 +925,7 @@ struct Sched {
         project();
         suffix_init();
         for (int i = 0; i < d.llm_layers; ++i) prefix_layer(i);
+        if (c->flow) { flow(0, d.num_steps, 0, d.llm_layers, true, true, "flow loop"); return; }
         for (int t = 0; t < d.num_steps; ++t) {
             suffix_step_begin(t);
             for (int i = 0; i < d.llm_layers; ++i) suffix_layer(t, i);
@@ -891,6 +959,7 @@ struct Sched {
         tile("decoder_ffn_gate_w", "t_decoder_ffn_gate_w", 1024, 4096, L);
         tile("decoder_ffn_up_w", "t_decoder_ffn_up_w", 1024, 4096, L);
         tile("decoder_ffn_down_w", "t_decoder_ffn_down_w", 4096, 1024, L);
+        tile(pi05 ? "decoder_action_in_proj_w" : "decoder_action_fused_in_proj_w", "t_decoder_action_in_w", 32, 1024, 1);
         if (!pi05) {
             tile("decoder_action_mlp_w", "t_decoder_action_mlp_w", 1024, 1024, 1);
             tile("decoder_action_fused_out_proj_w", "t_decoder_out_proj_w", 1024, 32, 1);
@@ -957,6 +1026,46 @@ int check_ready(rtvla_ctx* c, bool need_prepared) {
 int hip_fail(rtvla_ctx* c, hipError_t e, const char* what) {
     return c->fail(RTVLA_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }
+
+// The flow kernel needs every CU of the device to itself (csrc/flow.hip): two of them, started on two streams, could each hold half of
+// the CUs and wait for the other half.  Launches that contain one are therefore chained per device: each waits for the event recorded
+// behind the one before it, if that was on another stream.  A stream that is being captured is left alone (see FlowOff).
+constexpr int MAX_DEVICES = 64;
+struct FlowGate { std::mutex m; hipEvent_t done = nullptr; hipStream_t last = nullptr; bool used = false; };
+FlowGate flow_gates[MAX_DEVICES];
+
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
+struct FlowTurn {
+    FlowGate* g = nullptr;
+    hipStream_t s;
+    hipError_t err = hipSuccess;
+    FlowTurn(const rtvla_ctx* c, hipStream_t stream) : s(stream) {
+        int dev = 0;
+        if (!c->flow || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES || capturing(s)) return;
+        g = &flow_gates[dev];
+        g->m.lock();
+        if (!g->done) err = hipEventCreateWithFlags(&g->done, hipEventDisableTiming);
+        else if (g->used && (g->last != s || s == hipStreamPerThread)) err = hipStreamWaitEvent(s, g->done, 0);
+    }
+    ~FlowTurn() {
+        if (!g) return;
+        if (err == hipSuccess && hipEventRecord(g->done, s) == hipSuccess) { g->last = s; g->used = true; }
+        g->m.unlock();
+    }
+    FlowTurn(const FlowTurn&) = delete;
+    FlowTurn& operator=(const FlowTurn&) = delete;
+};
+
+// A caller's own graph of rtvla_forward may be replayed on any stream, where nothing chains it: it gets the loop as launches.
+struct FlowOff {
+    rtvla_ctx* c; bool was;
+    FlowOff(rtvla_ctx* c_, hipStream_t s) : c(c_), was(c_->flow) { if (was && capturing(s)) c->flow = false; }
+    ~FlowOff() { c->flow = was; }
+};
 
 // A captured graph holds the addresses that were bound when it was recorded: any later binding makes it stale.
 void drop_graph(rtvla_ctx* c) {
@@ -1065,6 +1174,7 @@ int rtvla_buffer_info(const rtvla_ctx* c, int index, const char** name, size_t* 
 static int prepare_impl(rtvla_ctx* c, void* stream, bool tiles_loaded) {
     if (int rc = check_ready(c, false)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;
+    c->flow = flow_supported((FlowSync*)c->B<float>("flow_sync"), (hipStream_t)stream);
     Sched(c, (hipStream_t)stream).prepare(tiles_loaded);
     if (c->status) return c->status;
     hipError_t e = hipGetLastError();
@@ -1081,6 +1191,9 @@ int rtvla_tile_layout_version(void) { return RTVLA_TILE_LAYOUT_VERSION; }
 int rtvla_forward(rtvla_ctx* c, void* stream) {
     if (int rc = check_ready(c, true)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;
+    FlowOff off(c, (hipStream_t)stream);
+    FlowTurn turn(c, (hipStream_t)stream);
+    if (turn.err != hipSuccess) return hip_fail(c, turn.err, "waiting for another stream's flow loop");
     Sched(c, (hipStream_t)stream).forward();
     return c->status;
 }
@@ -1088,6 +1201,9 @@ int rtvla_forward(rtvla_ctx* c, void* stream) {
 int rtvla_forward_stage(rtvla_ctx* c, int stage, int layer, int step, void* stream) {
     if (int rc = check_ready(c, true)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;
+    FlowOff off(c, (hipStream_t)stream);
+    FlowTurn turn(c, (hipStream_t)stream);
+    if (turn.err != hipSuccess) return hip_fail(c, turn.err, "waiting for another stream's flow loop");
     int rc = Sched(c, (hipStream_t)stream).stage(stage, layer, step);
     if (rc) return c->fail(rc, "bad stage / layer / step");
     return c->status;
@@ -1116,6 +1232,8 @@ int rtvla_graph_capture(rtvla_ctx* c, void* stream) {
 int rtvla_graph_launch(rtvla_ctx* c, void* stream) {
     if (!c) return RTVLA_ERR_ARG;
     if (!c->exec || !c->prepared) return c->fail(RTVLA_ERR_STATE, "no graph captured since the last rtvla_bind / rtvla_prepare");
+    FlowTurn turn(c, (hipStream_t)stream);
+    if (turn.err != hipSuccess) return hip_fail(c, turn.err, "waiting for another stream's flow loop");
     hipError_t e = hipGraphLaunch(c->exec, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(c, e, "hipGraphLaunch");
     return RTVLA_OK;
@@ -1134,6 +1252,8 @@ static int time_replay(rtvla_ctx* c, hipStream_t s, int stage, int layer, int st
         if (e0 != hipSuccess) return hip_fail(c, e0, "timing stream");
         s = c->timing_stream;
     }
+    FlowTurn turn(c, s);
+    if (turn.err != hipSuccess) return hip_fail(c, turn.err, "waiting for another stream's flow loop");
     Sched sc(c, s);
     const bool cycle = layer == -1;
     const int n_layers = !cycle ? 1 : (stage == RTVLA_STAGE_VISION_LAYER ? c->d.vision_layers :
