@@ -157,6 +157,10 @@ int rtvla_prepare_with_tiles(rtvla_ctx* ctx, void* hip_stream);
  * from the bound io buffers; the result is left in `diffusion_noise`. */
 int rtvla_forward(rtvla_ctx* ctx, void* hip_stream);
 
+/* Pi05 with the prompt staged on the device: writes `n` token ids (host memory, int64, read before the call returns) into the bound
+ * prompt_token_ids and 256 * num_views + n into valid_encoder_len, as launches on the stream: no copy, nothing waits. */
+int rtvla_stage_prompt(rtvla_ctx* ctx, const int64_t* ids_host, int n, void* hip_stream);
+
 /* Enqueue a single stage (see rtvla_stage); `layer` and `step` are ignored where meaningless. */
 int rtvla_forward_stage(rtvla_ctx* ctx, int stage, int layer, int step, void* hip_stream);
 
@@ -270,22 +274,20 @@ int rtvla_attention(int kind, const void* q, const void* k, const void* v, void*
 /* Replaces _resize_with_pad + _normalize_image (test.py:104-119) for one uint8 HWC RGB image: aspect-preserving
  * bilinear resize that matches Pillow's Image.resize(BILINEAR) bit for bit, pasted centred on a black 224x224
  * canvas, then x / 255 * 2 - 1, written as bf16 [224][224][3] - i.e. straight into one view of
- * observation_images_normalized.  `scratch` holds the 8-bit intermediate of the horizontal pass
- * (rtvla_preprocess_image_scratch bytes).  RTVLA_ERR_LIMIT for shrink factors above 31. */
+ * observation_images_normalized.  One kernel with the 8-bit intermediate in LDS: `scratch` (rtvla_preprocess_image_scratch bytes)
+ * is checked and left alone.  RTVLA_ERR_LIMIT for shrink factors above 31. */
 size_t rtvla_preprocess_image_scratch(int height, int width);
 int rtvla_preprocess_image(const void* src_u8, int height, int width, void* dst_bf16, void* scratch, size_t scratch_bytes,
                            void* hip_stream);
 
-/* The same computation for callers that cannot allocate device memory or hand over a workspace (code under HIP graph
- * capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The 8-bit
- * intermediate lives in a device array that is part of the library's code object (RTVLA_STATIC_SCRATCH_BYTES, held by
- * every GPU the library is loaded on until the process ends); the call allocates nothing.  Frames whose intermediate
- * (height x resized width x 3 bytes, resized width <= 224) exceeds that size - more than 2160 rows at full width - are
- * rejected with RTVLA_ERR_LIMIT before anything is enqueued.  All calls on one GPU share the one array: calls that
- * overlap on the same GPU (different streams or threads) race; calls on one stream are ordered.  Nothing in the array
- * has to start at zero: the horizontal pass writes every byte the vertical pass reads.  The array's device address is
- * looked up on the first call on each GPU; that lookup is not stream work, so the first call on a GPU must not come while
- * `hip_stream` is being captured (RTVLA_ERR_STATE then: make one eager call first, later calls may be captured). */
+/* The same for frames as the reference's _parse_image takes them (test.py:88-94): format 0 uint8 [h][w][3], 1 float32 [h][w][3],
+ * 2 float32 [3][h][w], 3 uint8 [3][h][w]; a float value becomes the low byte of the integer 255 x truncates to, as numpy's
+ * astype(uint8).  No scratch, nothing allocated: usable under graph capture. */
+int rtvla_preprocess_frame(const void* src, int format, int height, int width, void* dst_bf16, void* hip_stream);
+
+/* rtvla_preprocess_image without the scratch argument, for frames whose 8-bit intermediate (height x resized width x 3 bytes,
+ * resized width <= 224) has at most RTVLA_STATIC_SCRATCH_BYTES - 2160 rows at full width; larger ones are rejected with
+ * RTVLA_ERR_LIMIT (rtvla_preprocess_frame takes them). */
 #define RTVLA_STATIC_SCRATCH_BYTES (2160 * 224 * 3)
 int rtvla_preprocess_image_static(const void* src_u8, int height, int width, void* dst_bf16, void* hip_stream);
 
@@ -296,12 +298,18 @@ int rtvla_preprocess_image_static(const void* src_u8, int height, int width, voi
  * index np.digitize(z, linspace(-1, 1, 257)[:-1]) - 1 as int32 [32]. */
 int rtvla_preprocess_state(const double* state, int n, const double* stat_a, const double* stat_b, int n_stats, int mode,
                            void* out_bf16, double* out_f64, int32_t* out_bins, void* hip_stream);
+/* The same with the state in host memory: it is read before the call returns and travels with the launch. */
+int rtvla_preprocess_state_host(const double* state_host, int n, const double* stat_a, const double* stat_b, int n_stats, int mode,
+                                void* out_bf16, double* out_f64, int32_t* out_bins, void* hip_stream);
 
 /* Replaces _unnormalize_actions and the delta-to-absolute step of infer (test.py:139-151, :196-201): bf16 actions
  * [chunk][32] -> float32 -> (mode 0) x * (b + 1e-6) + a or (mode 1) (x + 1) / 2 * (b - a + 1e-6) + a in double, first
  * action_dim columns, + ori_state, with the state taken off again on every 7th column.  out: double [chunk][action_dim]. */
 int rtvla_postprocess_actions(const void* actions_bf16, int chunk, const double* stat_a, const double* stat_b, int n_stats,
                               int mode, const double* ori_state, int action_dim, double* out, void* hip_stream);
+/* The same with the state in host memory, n_state values zero-padded to 32. */
+int rtvla_postprocess_actions_host(const void* actions_bf16, int chunk, const double* stat_a, const double* stat_b, int n_stats,
+                                   int mode, const double* state_host, int n_state, int action_dim, double* out, void* hip_stream);
 
 #ifdef __cplusplus
 }

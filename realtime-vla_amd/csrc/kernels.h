@@ -211,6 +211,7 @@ void launch_attn_tile_operands(const bf16_t* q, const bf16_t* k, const bf16_t* v
 // ----- small helpers ------------------------------------------------------------------------
 void launch_prompt_stage(const bf16_t* emb, int vocab, const int* ids, const int* valid_len, bf16_t* x_rows, int prompt_rows, int s_v,
                          float scale, const bf16_t* rope_full, int rope_rows, bf16_t* dec_rope, int dec_rows, hipStream_t s);
+void launch_store_ids(const int64_t* ids_host, int n, int* ids, int valid_len, int* valid_len_dst, hipStream_t s);
 void launch_im2col(const bf16_t* images, bf16_t* patches, int ldp, int views, hipStream_t s);
 void launch_copy_rows(const bf16_t* src, int lds, bf16_t* dst, int ldd, int rows, int cols, hipStream_t s);
 void launch_fill_zero(void* p, size_t bytes, hipStream_t s);

@@ -185,6 +185,14 @@ __global__ void prompt_stage_kernel(const bf16_t* __restrict__ emb, int vocab, c
     }
 }
 
+// token ids by value (up to STORE_IDS a launch) and the prefix length they give
+constexpr int STORE_IDS = 512;
+struct IdBlock { int v[STORE_IDS]; };
+__global__ void store_ids_kernel(IdBlock b, int n, int* __restrict__ ids, int valid_len, int* __restrict__ valid_len_dst) {
+    if ((int)threadIdx.x < n) ids[threadIdx.x] = b.v[threadIdx.x];
+    if (threadIdx.x == 0) *valid_len_dst = valid_len;
+}
+
 __global__ void fill_zero_kernel(uint4* p, size_t n16) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n16) p[i] = uint4{0, 0, 0, 0};
@@ -284,6 +292,18 @@ void launch_prompt_stage(const bf16_t* emb, int vocab, const int* ids, const int
                          float scale, const bf16_t* rope_full, int rope_rows, bf16_t* dec_rope, int dec_rows, hipStream_t s) {
     hipLaunchKernelGGL(prompt_stage_kernel, dim3(prompt_rows + dec_rows), dim3(256), 0, s, emb, vocab, ids, valid_len, x_rows, prompt_rows, s_v,
                        scale, rope_full, rope_rows, dec_rope, dec_rows);
+}
+
+void launch_store_ids(const int64_t* ids_host, int n, int* ids, int valid_len, int* valid_len_dst, hipStream_t s) {
+    int at = 0;
+    do {
+        IdBlock b;
+        const int m = n - at < STORE_IDS ? n - at : STORE_IDS;
+        for (int i = 0; i < m; ++i) b.v[i] = (int)ids_host[at + i];
+        for (int i = m; i < STORE_IDS; ++i) b.v[i] = 0;
+        hipLaunchKernelGGL(store_ids_kernel, dim3(1), dim3(STORE_IDS), 0, s, b, m, ids + at, valid_len, valid_len_dst);
+        at += m;
+    } while (at < n);
 }
 
 void launch_fill_zero(void* p, size_t bytes, hipStream_t s) {

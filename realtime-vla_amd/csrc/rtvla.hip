@@ -1198,6 +1198,18 @@ int rtvla_forward(rtvla_ctx* c, void* stream) {
     return c->status;
 }
 
+int rtvla_stage_prompt(rtvla_ctx* c, const int64_t* ids_host, int n, void* stream) {
+    if (!c || n < 0 || (n > 0 && !ids_host)) return RTVLA_ERR_ARG;
+    if (c->d.model != RTVLA_PI05) return c->fail(RTVLA_ERR_ARG, "only Pi05 stages its prompt on the device");
+    if (n > c->d.prompt_len) return c->fail(RTVLA_ERR_SIZE, "more token ids than prompt_len");
+    const Tensor& ids = c->T("prompt_token_ids");
+    const Tensor& vl = c->T("valid_encoder_len");
+    if (!ids.bound || !vl.bound) return c->fail(RTVLA_ERR_UNBOUND, "prompt_token_ids or valid_encoder_len not bound");
+    launch_store_ids(ids_host, n, (int*)ids.ptr, c->S_v + n, (int*)vl.ptr, (hipStream_t)stream);
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? RTVLA_OK : hip_fail(c, e, "staging token ids");
+}
+
 int rtvla_forward_stage(rtvla_ctx* c, int stage, int layer, int step, void* stream) {
     if (int rc = check_ready(c, true)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;

@@ -5,19 +5,13 @@
 //
 // The resize reproduces Pillow's `Image.resize(..., BILINEAR)` bit for bit: triangle filter with the support stretched
 // by the shrink factor, double-precision weights normalised per output pixel, 22-bit fixed point, a horizontal pass to
-// an 8-bit intermediate and a vertical pass, each rounded to nearest and clipped.  Every thread derives the weights of
-// its own output pixel (a dozen double operations per tap), so there are no coefficient tables to upload and the
-// kernels can be captured in a graph.  This file is compiled with floating-point contraction off: a fused
+// an 8-bit intermediate and a vertical pass, each rounded to nearest and clipped.  The weights are derived in the kernel
+// (a dozen double operations per tap), so there are no coefficient tables to upload and the kernels can be captured in a
+// graph.  This file is compiled with floating-point contraction off: a fused
 // multiply-add would round the weights differently from the C code being matched.
 #include "../../include/rtvla.h"
 #include "common.h"
 #include <math.h>
-#include <mutex>
-
-// 8-bit intermediate of the horizontal pass for rtvla_preprocess_image_static: part of the code object, so every
-// GPU the library runs on holds its own copy at its own address from load until the process ends.  Host code
-// never passes this name to a kernel; it uses the per-device address resolved in static_scratch_ptr().
-static __device__ __align__(256) unsigned char scratch[RTVLA_STATIC_SCRATCH_BYTES];
 
 namespace {
 
@@ -59,51 +53,152 @@ RTVLA_DEVICE int tap_weight(const Window& w, int x) {
 
 RTVLA_DEVICE int clip8(int v) { v >>= PRECISION_BITS; return v < 0 ? 0 : (v > 255 ? 255 : v); }
 
-// horizontal pass: src [h][w][3] -> tmp [h][rw][3]
-__global__ void resample_h_kernel(const uint8_t* __restrict__ src, int h, int w, int rw, uint8_t* __restrict__ tmp) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= h * rw) return;
-    const int y = idx / rw, xx = idx - y * rw;
-    const Window win = window_of(xx, w, rw);
-    int acc[3] = {1 << (PRECISION_BITS - 1), 1 << (PRECISION_BITS - 1), 1 << (PRECISION_BITS - 1)};
-    const uint8_t* row = src + ((size_t)y * w + win.first) * 3;
-    for (int x = 0; x < win.count; ++x) {
-        const int k = tap_weight(win, x);
-        acc[0] += row[x * 3 + 0] * k; acc[1] += row[x * 3 + 1] * k; acc[2] += row[x * 3 + 2] * k;
-    }
-    uint8_t* o = tmp + (size_t)idx * 3;
-    o[0] = (uint8_t)clip8(acc[0]); o[1] = (uint8_t)clip8(acc[1]); o[2] = (uint8_t)clip8(acc[2]);
+// One launch per frame: resize, pad, x / 255 * 2 - 1 -> bf16 NHWC.  A workgroup owns 32 x TH pixels of the 224 x 224 canvas.  It derives
+// the weights of its 32 columns and TH rows once (one thread per tap, into LDS), resamples the source rows its output rows need
+// across into an 8-bit LDS tile, and that tile down into the output.  Neighbouring row blocks resample the rows they share twice
+// ((TH + 2) / TH of the work for TH output rows); in exchange nothing but the frame is read and nothing but the result written, and the
+// second launch with its round trip through memory is gone.  Measured (480 x 640 uint8, one frame): two launches, each thread deriving the
+// weights of its own pixel, 11.7 us; this one 4.9 us.  TH = 4 gives large frames (many taps per pixel) twice the workgroups.
+enum FrameFormat { FRAME_U8_HWC = 0, FRAME_F32_HWC, FRAME_F32_CHW, FRAME_U8_CHW };
+constexpr int TW = 32, NT = 512;            // columns and threads of a workgroup
+struct FrameP { const uint8_t* src; int h, w, rw, rh, pad_top, pad_left, taps_x, taps_y, max_rows; bf16_t* dst; };      // taps: rounded up to 4
+
+// numpy's / torch's float -> uint8: truncation to an integer, low byte
+RTVLA_DEVICE int to_u8(float x) {
+    const float v = 255.0f * x;
+    int i = (int)v;
+    if (__builtin_expect(!(fabsf(v) < 2147483648.0f), 0)) i = (int)(long long)v;
+    return i & 255;
+}
+// four consecutive values, any alignment of 4 bytes; one load unless it would reach past `end`
+RTVLA_DEVICE f32x4 load_f4(const float* q, const float* end) {
+    f32x4 v;
+    if (q + 4 <= end) __builtin_memcpy(&v, q, 16);
+    else for (int i = 0; i < 4; ++i) v[i] = q + i < end ? q[i] : 0.f;
+    return v;
 }
 
-// vertical pass + paste on the black 224 x 224 canvas + x / 255 * 2 - 1 -> bf16 NHWC
-__global__ void resample_v_pad_norm_kernel(const uint8_t* __restrict__ tmp, int h, int rw, int rh, int pad_top, int pad_left,
-                                           bf16_t* __restrict__ dst) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= 224 * 224) return;
-    const int yy = idx / 224, xx = idx - yy * 224;
-    int v[3] = {0, 0, 0};
-    const int ry = yy - pad_top, rx = xx - pad_left;
-    if (ry >= 0 && ry < rh && rx >= 0 && rx < rw) {
-        const Window win = window_of(ry, h, rh);
-        int acc[3] = {1 << (PRECISION_BITS - 1), 1 << (PRECISION_BITS - 1), 1 << (PRECISION_BITS - 1)};
-        for (int y = 0; y < win.count; ++y) {
-            const int k = tap_weight(win, y);
-            const uint8_t* p = tmp + ((size_t)(win.first + y) * rw + rx) * 3;
-            acc[0] += p[0] * k; acc[1] += p[1] * k; acc[2] += p[2] * k;
-        }
-        v[0] = clip8(acc[0]); v[1] = clip8(acc[1]); v[2] = clip8(acc[2]);
+template <int FMT, int TH>
+__global__ __launch_bounds__(NT) void resize_kernel(FrameP p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    int4* const wx = (int4*)smem;                                              // [taps_x / 4][TW]
+    int* const wy = (int*)(wx + (p.taps_x >> 2) * TW);                         // [taps_y][TH]
+    unsigned* const inter = (unsigned*)(wy + p.taps_y * TH);                   // [row][TW], three bytes each
+    __shared__ Window win[TW + TH];
+    __shared__ bf16_t value[256];
+    const int tid = threadIdx.x, x0 = blockIdx.x * TW, y0 = blockIdx.y * TH;
+    if (tid < 256) value[tid] = f2bf((float)tid / 255.0f * 2.0f - 1.0f);
+    if (tid < TW) {
+        const int rx = x0 + tid - p.pad_left;
+        if (rx >= 0 && rx < p.rw) win[tid] = window_of(rx, p.w, p.rw); else { win[tid] = Window{}; win[tid].count = 0; }
+    } else if (tid >= 64 && tid < 64 + TH) {
+        const int ry = y0 + tid - 64 - p.pad_top;
+        if (ry >= 0 && ry < p.rh) win[TW + tid - 64] = window_of(ry, p.h, p.rh); else { win[TW + tid - 64] = Window{}; win[TW + tid - 64].count = 0; }
     }
+    __syncthreads();
+    for (int i = tid; i < p.taps_x * TW; i += NT) {
+        const int c = i % TW, t = i / TW;
+        ((int*)wx)[((t >> 2) * TW + c) * 4 + (t & 3)] = t < win[c].count ? tap_weight(win[c], t) : 0;
+    }
+    for (int i = tid; i < p.taps_y * TH; i += NT) {
+        const int rr = i % TH, t = i / TH;
+        wy[i] = t < win[TW + rr].count ? tap_weight(win[TW + rr], t) : 0;
+    }
+    // source rows of this block: the windows move down with the output row
+    int lo = 1 << 30, hi = 0;
 #pragma unroll
-    for (int c = 0; c < 3; ++c) dst[(size_t)idx * 3 + c] = f2bf((float)v[c] / 255.0f * 2.0f - 1.0f);
+    for (int i = 0; i < TH; ++i)
+        if (win[TW + i].count > 0) { lo = min(lo, win[TW + i].first); hi = max(hi, win[TW + i].first + win[TW + i].count); }
+    __syncthreads();
+    const int c = tid & (TW - 1), first = win[c].first, count = win[c].count;
+    const uintptr_t last = ((uintptr_t)p.src + (size_t)p.h * p.w * 3 - 1) & ~(uintptr_t)3;      // uint8: the dword that holds the last byte
+    if (count > 0)
+        for (int row = tid >> 5; row < hi - lo; row += NT / TW) {
+            int a0 = 1 << (PRECISION_BITS - 1), a1 = a0, a2 = a0;
+            const size_t at = (size_t)(lo + row) * p.w + first;
+            if constexpr (FMT == FRAME_U8_CHW) {
+                const size_t plane = (size_t)p.h * p.w;
+                for (int t = 0; t < count; ++t) {
+                    const int k = ((const int*)wx)[((t >> 2) * TW + c) * 4 + (t & 3)];
+                    a0 += __mul24((int)p.src[at + t], k); a1 += __mul24((int)p.src[plane + at + t], k); a2 += __mul24((int)p.src[2 * plane + at + t], k);
+                }
+            } else {
+                // Four taps at a time, and the loads of UN such groups before the first is used: with 1 - 2 workgroups per CU the pass is bound
+                // by the latency of its loads.  What lies past the window has zero weight.
+                constexpr int UN = 4;
+                for (int t0 = 0; t0 < p.taps_x; t0 += 4 * UN) {
+                    f32x4 v[UN][3];
+#pragma unroll
+                    for (int j = 0; j < UN; ++j) {
+                        const int t = t0 + 4 * j;
+                        if (t >= p.taps_x) break;
+                        if constexpr (FMT == FRAME_U8_HWC) {                   // 12 bytes, as the dwords they lie in
+                            const uintptr_t q = ((uintptr_t)p.src + at * 3 & ~(uintptr_t)3) + t * 3;
+                            if (q + 12 <= last) __builtin_memcpy(&v[j][0], (const void*)q, 16);
+                            else
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) v[j][0][i] = *(const float*)min(q + 4 * i, last);
+                        } else {
+                            const float* const f = (const float*)p.src;
+                            const size_t plane = (size_t)p.h * p.w;
+#pragma unroll
+                            for (int i = 0; i < 3; ++i) v[j][i] = load_f4(FMT == FRAME_F32_CHW ? f + i * plane + at + t : f + (at + t) * 3 + 4 * i, f + 3 * plane);
+                        }
+                    }
+#pragma unroll
+                    for (int j = 0; j < UN; ++j) {
+                        const int t = t0 + 4 * j;
+                        if (t >= p.taps_x) break;
+                        const int4 k = wx[(t >> 2) * TW + c];
+                        int u[3][4];
+                        if constexpr (FMT == FRAME_U8_HWC) {
+                            const unsigned sh = (unsigned)(((uintptr_t)p.src + at * 3) & 3);
+                            unsigned e[3];
+#pragma unroll
+                            for (int i = 0; i < 3; ++i) e[i] = __builtin_amdgcn_alignbyte(__float_as_uint(v[j][0][i + 1]), __float_as_uint(v[j][0][i]), sh);
+#pragma unroll
+                            for (int i = 0; i < 12; ++i) u[i % 3][i / 3] = (e[i >> 2] >> 8 * (i & 3)) & 255;
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < 12; ++i) {
+                                if constexpr (FMT == FRAME_F32_CHW) u[i >> 2][i & 3] = to_u8(v[j][i >> 2][i & 3]);
+                                else u[i % 3][i / 3] = to_u8(v[j][i >> 2][i & 3]);
+                            }
+                        }
+                        a0 += __mul24(u[0][0], k.x) + __mul24(u[0][1], k.y) + __mul24(u[0][2], k.z) + __mul24(u[0][3], k.w);
+                        a1 += __mul24(u[1][0], k.x) + __mul24(u[1][1], k.y) + __mul24(u[1][2], k.z) + __mul24(u[1][3], k.w);
+                        a2 += __mul24(u[2][0], k.x) + __mul24(u[2][1], k.y) + __mul24(u[2][2], k.z) + __mul24(u[2][3], k.w);
+                    }
+                }
+            }
+            inter[row * TW + c] = (unsigned)clip8(a0) | (unsigned)clip8(a1) << 8 | (unsigned)clip8(a2) << 16;
+        }
+    __syncthreads();
+    const int rr = tid / TW;
+    if (rr >= TH) return;
+    int v0 = 0, v1 = 0, v2 = 0;
+    const int vfirst = win[TW + rr].first - lo, vcount = win[TW + rr].count;
+    if (count > 0 && vcount > 0) {
+        int a0 = 1 << (PRECISION_BITS - 1), a1 = a0, a2 = a0;
+        for (int t = 0; t < vcount; ++t) {
+            const unsigned e = inter[(vfirst + t) * TW + c];
+            const int k = wy[t * TH + rr];
+            a0 += __mul24(e & 255, k); a1 += __mul24((e >> 8) & 255, k); a2 += __mul24(e >> 16, k);
+        }
+        v0 = clip8(a0); v1 = clip8(a1); v2 = clip8(a2);
+    }
+    bf16_t* o = p.dst + ((size_t)(y0 + rr) * 224 + x0 + c) * 3;
+    o[0] = value[v0]; o[1] = value[v1]; o[2] = value[v2];
 }
 
 // state: mode 0 (Pi0) (x - a) / (b + 1e-6), a = mean, b = std; mode 1 (Pi05) (x - a) / (b - a + 1e-6) * 2 - 1, a = q01, b = q99
 // (statistics and state zero-padded to 32 like _pad_to_dim); then float32 -> bf16 for the model and the 256-bin index
-__global__ void state_kernel(const double* __restrict__ state, int n, const double* __restrict__ a, const double* __restrict__ b, int n_stats,
+struct State32 { double v[32]; };      // a state handed over by value: no copy to the device, no synchronisation
+__global__ void state_kernel(const double* __restrict__ state, State32 by_value, int n, const double* __restrict__ a, const double* __restrict__ b, int n_stats,
                              int mode, bf16_t* __restrict__ out_bf16, double* __restrict__ out_f64, int32_t* __restrict__ bins) {
     const int i = threadIdx.x;
     if (i >= 32) return;
-    const double x = i < n ? state[i] : 0.0, av = i < n_stats ? a[i] : 0.0, bv = i < n_stats ? b[i] : 0.0;
+    const double x = i < n ? (state ? state[i] : by_value.v[i]) : 0.0, av = i < n_stats ? a[i] : 0.0, bv = i < n_stats ? b[i] : 0.0;
     const double z = mode == 0 ? (x - av) / (bv + 1e-6) : (x - av) / (bv - av + 1e-6) * 2.0 - 1.0;
     if (out_f64) out_f64[i] = z;
     if (out_bf16) out_bf16[i] = f2bf((float)z);
@@ -119,7 +214,7 @@ __global__ void state_kernel(const double* __restrict__ state, int n, const doub
 // actions: bf16 [chunk][32] -> float32 -> un-normalise in double -> first action_dim columns + state, gripper columns
 // (every 7th) get the state taken off again, exactly in the reference's order of operations
 __global__ void actions_kernel(const bf16_t* __restrict__ actions, int chunk, const double* __restrict__ a, const double* __restrict__ b,
-                               int n_stats, int mode, const double* __restrict__ ori_state, int action_dim, double* __restrict__ out) {
+                               int n_stats, int mode, const double* __restrict__ state, State32 by_value, int action_dim, double* __restrict__ out) {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= chunk * action_dim) return;
     const int r = idx / action_dim, d = idx - r * action_dim;
@@ -128,61 +223,77 @@ __global__ void actions_kernel(const bf16_t* __restrict__ actions, int chunk, co
     double v;
     if (mode == 0) v = (double)x * (bv + 1e-6) + av;                               // a = mean, b = std
     else v = (double)((x + 1.0f) / 2.0f) * (bv - av + 1e-6) + av;                  // a = q01, b = q99; (x + 1) / 2 stays float32
-    v = v + ori_state[d];
-    if (d % 7 == 6 && d < (action_dim / 7) * 7) v = v - ori_state[d];
+    const double ori = state ? state[d] : by_value.v[d];
+    v = v + ori;
+    if (d % 7 == 6 && d < (action_dim / 7) * 7) v = v - ori;
     out[idx] = v;
 }
 
-// geometry, limits and the two launches shared by rtvla_preprocess_image and rtvla_preprocess_image_static;
-// `get_scratch` is asked for the intermediate buffer only after every size check has passed
-template <typename GetScratch>
-int preprocess_image_impl(const void* src_u8, int height, int width, void* dst_bf16, size_t scratch_bytes, int too_small_code,
-                          GetScratch get_scratch, void* stream) {
-    if (!src_u8 || !dst_bf16 || height <= 0 || width <= 0) return RTVLA_ERR_ARG;
-    // geometry of test.py:105-116 (Python float arithmetic = C double arithmetic)
-    int rh = 224, rw = 224, pad_top = 0, pad_left = 0;
+// geometry of test.py:105-116 (Python float arithmetic = C double arithmetic) and limits
+int frame_plan(int height, int width, FrameP* p) {
+    if (height <= 0 || width <= 0) return RTVLA_ERR_ARG;
+    p->h = height; p->w = width; p->rh = p->rw = 224; p->pad_top = p->pad_left = 0;
     if (!(width == 224 && height == 224)) {
         const double rwf = (double)width / 224, rhf = (double)height / 224;
         const double ratio = rwf > rhf ? rwf : rhf;
-        rh = (int)((double)height / ratio); rw = (int)((double)width / ratio);
-        pad_top = (int)((double)(224 - rh) / 2); if (pad_top < 0) pad_top = 0;
-        pad_left = (int)((double)(224 - rw) / 2); if (pad_left < 0) pad_left = 0;
+        p->rh = (int)((double)height / ratio); p->rw = (int)((double)width / ratio);
+        p->pad_top = (int)((double)(224 - p->rh) / 2); if (p->pad_top < 0) p->pad_top = 0;
+        p->pad_left = (int)((double)(224 - p->rw) / 2); if (p->pad_left < 0) p->pad_left = 0;
     }
-    if (rh < 1 || rw < 1 || rh > 224 || rw > 224) return RTVLA_ERR_ARG;
-    const double sx = (double)width / rw, sy = (double)height / rh;
-    if ((int)ceil(sx > 1.0 ? sx : 1.0) * 2 + 1 > MAX_TAPS || (int)ceil(sy > 1.0 ? sy : 1.0) * 2 + 1 > MAX_TAPS) return RTVLA_ERR_LIMIT;
-    if (scratch_bytes < (size_t)height * rw * 3) return too_small_code;
-    uint8_t* tmp = nullptr;
-    hipStream_t s = (hipStream_t)stream;
-    if (int rc = get_scratch(&tmp, s)) return rc;
-    const int n1 = height * rw;
-    hipLaunchKernelGGL(resample_h_kernel, dim3((n1 + 255) / 256), dim3(256), 0, s, (const uint8_t*)src_u8, height, width, rw, tmp);
-    hipLaunchKernelGGL(resample_v_pad_norm_kernel, dim3((224 * 224 + 255) / 256), dim3(256), 0, s, (const uint8_t*)tmp, height, rw, rh,
-                       pad_top, pad_left, (bf16_t*)dst_bf16);
+    if (p->rh < 1 || p->rw < 1 || p->rh > 224 || p->rw > 224) return RTVLA_ERR_ARG;
+    const double sx = (double)width / p->rw, sy = (double)height / p->rh;
+    const int tx = (int)ceil(sx > 1.0 ? sx : 1.0) * 2 + 1, ty = (int)ceil(sy > 1.0 ? sy : 1.0) * 2 + 1;
+    if (tx > MAX_TAPS || ty > MAX_TAPS) return RTVLA_ERR_LIMIT;
+    p->taps_x = (tx + 3) & ~3; p->taps_y = (ty + 3) & ~3;
+    return RTVLA_OK;
+}
+
+template <int FMT, int TH>
+void launch_resize(FrameP p, hipStream_t s) {
+    const double sy = (double)p.h / p.rh;
+    p.max_rows = (int)((TH - 1) * sy) + p.taps_y + 2;                          // first row of the first window to the last row of the last
+    const size_t smem = (size_t)p.taps_x * TW * 4 + (size_t)p.taps_y * TH * 4 + (size_t)p.max_rows * TW * 4;
+    hipLaunchKernelGGL((resize_kernel<FMT, TH>), dim3(224 / TW, 224 / TH), dim3(NT), smem, s, p);
+}
+template <int FMT>
+int launch_frame(const FrameP& p, hipStream_t s) {
+    // more than 8 rows of source per output row or column: the across pass dominates, twice the workgroups share it (and LDS stays below 64 KB)
+    if (p.taps_x > 12 || p.taps_y > 12) launch_resize<FMT, 4>(p, s); else launch_resize<FMT, 8>(p, s);
+    return hipGetLastError() == hipSuccess ? RTVLA_OK : RTVLA_ERR_DEVICE;
+}
+int preprocess_frame_impl(const void* src, int format, int height, int width, void* dst_bf16, void* stream) {
+    if (!src || !dst_bf16) return RTVLA_ERR_ARG;
+    FrameP p{};
+    if (int rc = frame_plan(height, width, &p)) return rc;
+    p.src = (const uint8_t*)src; p.dst = (bf16_t*)dst_bf16;
+    switch (format) {
+        case FRAME_U8_HWC: return launch_frame<FRAME_U8_HWC>(p, (hipStream_t)stream);
+        case FRAME_F32_HWC: return launch_frame<FRAME_F32_HWC>(p, (hipStream_t)stream);
+        case FRAME_F32_CHW: return launch_frame<FRAME_F32_CHW>(p, (hipStream_t)stream);
+        case FRAME_U8_CHW: return launch_frame<FRAME_U8_CHW>(p, (hipStream_t)stream);
+    }
+    return RTVLA_ERR_ARG;
+}
+
+int launch_state(const double* dev, const double* host, int n, const double* stat_a, const double* stat_b, int n_stats, int mode, void* out_bf16, double* out_f64,
+                 int32_t* out_bins, void* stream) {
+    if ((!dev && !host) || !stat_a || !stat_b || n < 0 || n > 32 || n_stats < 0 || n_stats > 32 || (mode != 0 && mode != 1)) return RTVLA_ERR_ARG;
+    State32 v{};
+    if (!dev) for (int i = 0; i < n; ++i) v.v[i] = host[i];
+    hipLaunchKernelGGL(state_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, dev, v, n, stat_a, stat_b, n_stats, mode, (bf16_t*)out_bf16, out_f64, out_bins);
     return hipGetLastError() == hipSuccess ? RTVLA_OK : RTVLA_ERR_DEVICE;
 }
 
-// Device address of `scratch` on the current device, resolved once per device with that device current.
-constexpr int MAX_DEVICES = 64;
-std::mutex static_scratch_mutex;
-void* static_scratch_addr[MAX_DEVICES] = {};
-
-// The lookup loads the code object and is not stream work: it must not happen while `s` is being captured into a graph,
-// so a first call on a device that comes under capture is refused (RTVLA_ERR_STATE) and any earlier eager call resolves it.
-int static_scratch_ptr(uint8_t** out, hipStream_t s) {
-    int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return RTVLA_ERR_DEVICE;
-    std::lock_guard<std::mutex> lock(static_scratch_mutex);
-    if (!static_scratch_addr[dev]) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cap) != hipSuccess) return RTVLA_ERR_DEVICE;
-        if (cap != hipStreamCaptureStatusNone) return RTVLA_ERR_STATE;
-        void* ptr = nullptr;
-        if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)) != hipSuccess || !ptr) return RTVLA_ERR_DEVICE;
-        static_scratch_addr[dev] = ptr;
-    }
-    *out = (uint8_t*)static_scratch_addr[dev];
-    return RTVLA_OK;
+int launch_actions(const void* actions_bf16, int chunk, const double* stat_a, const double* stat_b, int n_stats, int mode, const double* dev, const double* host, int n_state,
+                   int action_dim, double* out, void* stream) {
+    if (!actions_bf16 || !stat_a || !stat_b || (!dev && !host) || !out || chunk <= 0 || action_dim <= 0 || action_dim > 32 || n_stats < 0 || n_stats > 32 ||
+        n_state < 0 || n_state > 32 || (mode != 0 && mode != 1)) return RTVLA_ERR_ARG;
+    State32 v{};
+    if (!dev) for (int i = 0; i < n_state; ++i) v.v[i] = host[i];
+    const int n = chunk * action_dim;
+    hipLaunchKernelGGL(actions_kernel, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)actions_bf16, chunk, stat_a, stat_b, n_stats, mode, dev, v,
+                       action_dim, out);
+    return hipGetLastError() == hipSuccess ? RTVLA_OK : RTVLA_ERR_DEVICE;
 }
 
 }  // namespace
@@ -191,34 +302,47 @@ extern "C" {
 
 size_t rtvla_preprocess_image_scratch(int height, int width) {
     if (height <= 0 || width <= 0) return 0;
-    return ((size_t)height * 224 * 3 + 255) & ~(size_t)255;       // the horizontal pass never produces more than 224 columns
+    return ((size_t)height * 224 * 3 + 255) & ~(size_t)255;       // (kept for callers of the ABI: the kernel has no intermediate in memory any more)
+}
+
+int rtvla_preprocess_frame(const void* src, int format, int height, int width, void* dst_bf16, void* stream) {
+    return preprocess_frame_impl(src, format, height, width, dst_bf16, stream);
 }
 
 int rtvla_preprocess_image(const void* src_u8, int height, int width, void* dst_bf16, void* scratch_arg, size_t scratch_bytes, void* stream) {
-    if (!scratch_arg) return RTVLA_ERR_ARG;
-    return preprocess_image_impl(src_u8, height, width, dst_bf16, scratch_bytes, RTVLA_ERR_SIZE,
-                                 [&](uint8_t** out, hipStream_t) { *out = (uint8_t*)scratch_arg; return (int)RTVLA_OK; }, stream);
+    if (!scratch_arg || !src_u8 || !dst_bf16) return RTVLA_ERR_ARG;
+    FrameP p{};
+    if (int rc = frame_plan(height, width, &p)) return rc;
+    if (scratch_bytes < (size_t)height * p.rw * 3) return RTVLA_ERR_SIZE;
+    return preprocess_frame_impl(src_u8, FRAME_U8_HWC, height, width, dst_bf16, stream);
 }
 
 int rtvla_preprocess_image_static(const void* src_u8, int height, int width, void* dst_bf16, void* stream) {
-    return preprocess_image_impl(src_u8, height, width, dst_bf16, (size_t)RTVLA_STATIC_SCRATCH_BYTES, RTVLA_ERR_LIMIT, static_scratch_ptr, stream);
+    if (!src_u8 || !dst_bf16) return RTVLA_ERR_ARG;
+    FrameP p{};
+    if (int rc = frame_plan(height, width, &p)) return rc;
+    if ((size_t)height * p.rw * 3 > (size_t)RTVLA_STATIC_SCRATCH_BYTES) return RTVLA_ERR_LIMIT;
+    return preprocess_frame_impl(src_u8, FRAME_U8_HWC, height, width, dst_bf16, stream);
 }
 
 int rtvla_preprocess_state(const double* state, int n, const double* stat_a, const double* stat_b, int n_stats, int mode,
                            void* out_bf16, double* out_f64, int32_t* out_bins, void* stream) {
-    if (!state || !stat_a || !stat_b || n < 0 || n > 32 || n_stats < 0 || n_stats > 32 || (mode != 0 && mode != 1)) return RTVLA_ERR_ARG;
-    hipLaunchKernelGGL(state_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, state, n, stat_a, stat_b, n_stats, mode, (bf16_t*)out_bf16, out_f64, out_bins);
-    return hipGetLastError() == hipSuccess ? RTVLA_OK : RTVLA_ERR_DEVICE;
+    return launch_state(state, nullptr, n, stat_a, stat_b, n_stats, mode, out_bf16, out_f64, out_bins, stream);
+}
+
+int rtvla_preprocess_state_host(const double* state_host, int n, const double* stat_a, const double* stat_b, int n_stats, int mode,
+                                void* out_bf16, double* out_f64, int32_t* out_bins, void* stream) {
+    return launch_state(nullptr, state_host, n, stat_a, stat_b, n_stats, mode, out_bf16, out_f64, out_bins, stream);
 }
 
 int rtvla_postprocess_actions(const void* actions_bf16, int chunk, const double* stat_a, const double* stat_b, int n_stats, int mode,
                               const double* ori_state, int action_dim, double* out, void* stream) {
-    if (!actions_bf16 || !stat_a || !stat_b || !ori_state || !out || chunk <= 0 || action_dim <= 0 || action_dim > 32 || n_stats < 0 || n_stats > 32 ||
-        (mode != 0 && mode != 1)) return RTVLA_ERR_ARG;
-    const int n = chunk * action_dim;
-    hipLaunchKernelGGL(actions_kernel, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)actions_bf16, chunk, stat_a, stat_b, n_stats,
-                       mode, ori_state, action_dim, out);
-    return hipGetLastError() == hipSuccess ? RTVLA_OK : RTVLA_ERR_DEVICE;
+    return launch_actions(actions_bf16, chunk, stat_a, stat_b, n_stats, mode, ori_state, nullptr, 0, action_dim, out, stream);
+}
+
+int rtvla_postprocess_actions_host(const void* actions_bf16, int chunk, const double* stat_a, const double* stat_b, int n_stats, int mode,
+                                   const double* state_host, int n_state, int action_dim, double* out, void* stream) {
+    return launch_actions(actions_bf16, chunk, stat_a, stat_b, n_stats, mode, nullptr, state_host, n_state, action_dim, out, stream);
 }
 
 }  // extern "C"

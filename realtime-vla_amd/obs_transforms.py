@@ -3,14 +3,12 @@ harness (/root/reference/test.py:88-201: `_parse_image`, `_resize_with_pad`, `_n
 `_digitize_state`, `_unnormalize_actions`, `_apply_input_transforms`, and the action post-processing of `infer`).
 The reference runs these in numpy / Pillow on the host for every observation; here each is one or two HIP kernels of
 librtvla.so writing straight into the model's input buffers.  PyTorch only owns the memory."""
-import ctypes
-
 import numpy as np
 import torch
 
 import rtvla_capi as capi
 
-_P = ctypes.c_void_p
+_VIEW_SHAPE = (224, 224, 3)
 
 
 class ObservationTransforms:
@@ -31,11 +29,12 @@ class ObservationTransforms:
             if norm_stats and group in norm_stats:
                 a = torch.tensor(np.asarray(norm_stats[group][keys[0]], dtype=np.float64)[:32], device=self.device)
                 b = torch.tensor(np.asarray(norm_stats[group][keys[1]], dtype=np.float64)[:32], device=self.device)
-                self._stats[group] = (a, b)
-        self._scratch = torch.empty(0, dtype=torch.uint8, device=self.device)
+                self._stats[group] = (a, b, int(a.numel()))
+        self._index = self.device.index if self.device.index is not None else torch.cuda.current_device()
+        self.device = torch.device("cuda", self._index)
 
     def _stream(self):
-        return _P(torch.cuda.current_stream(self.device).cuda_stream)
+        return torch._C._cuda_getCurrentRawStream(self._index)      # the bare handle: the Stream object costs more than a launch
 
     @staticmethod
     def _check(rc, what):
@@ -52,29 +51,45 @@ class ObservationTransforms:
             image = image.permute(1, 2, 0)
         return image.to(self.device).contiguous()
 
+    def _frame(self, image):
+        """(contiguous tensor on the device, its frame format, height, width): float32 and channels-first frames go to the kernel as
+        they are, everything else as _parse_image makes it."""
+        if not isinstance(image, torch.Tensor):
+            image = torch.as_tensor(image)
+        dtype = image.dtype
+        if (dtype is not torch.uint8 and dtype is not torch.float32) or image.dim() != 3:
+            image, dtype = self._parse_image(image), torch.uint8
+        chw = image.shape[0] == 3
+        h, w, c = (image.shape[1], image.shape[2], 3) if chw else image.shape
+        if c != 3 or image.dtype is not dtype:
+            raise ValueError("expected an RGB uint8 image, got shape %s dtype %s" % ((h, w, c), image.dtype))
+        if image.device != self.device:
+            image = image.to(self.device)
+        if not image.is_contiguous():
+            image = image.contiguous()
+        if dtype is torch.uint8:
+            return image, (capi.FRAME_U8_CHW if chw else capi.FRAME_U8_HWC), h, w
+        return image, (capi.FRAME_F32_CHW if chw else capi.FRAME_F32_HWC), h, w
+
     def resize_pad_normalize_into(self, image, out_view, static_scratch=False):
         """_resize_with_pad + _normalize_image of one image into out_view (bf16 [224, 224, 3], e.g. one view of the
-        model's observation_images_normalized buffer).  With static_scratch the library's built-in intermediate buffer
-        is used and nothing is allocated (frames of at most 2160 rows at full width; calls on one GPU must not overlap)."""
-        img = self._parse_image(image)
-        h, w, c = img.shape
-        if c != 3 or img.dtype != torch.uint8:
-            raise ValueError("expected an RGB uint8 image, got shape %s dtype %s" % (tuple(img.shape), img.dtype))
-        if out_view.dtype != torch.bfloat16 or tuple(out_view.shape) != (224, 224, 3) or not out_view.is_contiguous():
+        model's observation_images_normalized buffer).  Nothing is allocated for a frame that is on the device already;
+        static_scratch (frames of at most 2160 rows at full width) is kept for its callers."""
+        if out_view.dtype is not torch.bfloat16 or out_view.shape != _VIEW_SHAPE or not out_view.is_contiguous():
+            self._frame(image)                                    # (a bad image is reported first)
             raise ValueError("out_view must be a contiguous bf16 [224, 224, 3] tensor")
+        img, fmt, h, w = self._frame(image)
         if static_scratch:
-            rc = self.lib.rtvla_preprocess_image_static(_P(img.data_ptr()), h, w, _P(out_view.data_ptr()), self._stream())
+            img = self._parse_image(img)
+            rc = self.lib.rtvla_preprocess_image_static(img.data_ptr(), h, w, out_view.data_ptr(), self._stream())
             if rc == capi.ERR_LIMIT:
                 raise ValueError("a %d x %d frame does not fit the library's %d-byte static intermediate buffer (or shrinks by more "
                                  "than a factor of 31)" % (h, w, capi.STATIC_SCRATCH_BYTES))
             self._check(rc, "rtvla_preprocess_image_static")
-            self._keep = img
-            return out_view
-        need = self.lib.rtvla_preprocess_image_scratch(h, w)
-        if self._scratch.numel() < need:
-            self._scratch = torch.empty(need, dtype=torch.uint8, device=self.device)
-        self._check(self.lib.rtvla_preprocess_image(_P(img.data_ptr()), h, w, _P(out_view.data_ptr()), _P(self._scratch.data_ptr()),
-                                                    self._scratch.numel(), self._stream()), "rtvla_preprocess_image")
+        else:
+            rc = self.lib.rtvla_preprocess_frame(img.data_ptr(), fmt, h, w, out_view.data_ptr(), self._stream())
+            if rc:
+                self._check(rc, "rtvla_preprocess_frame")
         self._keep = img                                           # alive until the stream has consumed it
         return out_view
 
@@ -84,13 +99,15 @@ class ObservationTransforms:
         writes the float32 -> bf16 value into out_bf16 (the model's observation_state_normalized buffer)."""
         if "state" not in self._stats:
             return None, None
-        a, b = self._stats["state"]
-        st = torch.as_tensor(np.asarray(state, dtype=np.float64)).to(self.device)
+        a, b, n_stats = self._stats["state"]
+        st = np.ascontiguousarray(state, dtype=np.float64)         # travels with the launch
         z = torch.empty(32, dtype=torch.float64, device=self.device)
         bins = torch.empty(32, dtype=torch.int32, device=self.device) if want_bins else None
-        self._check(self.lib.rtvla_preprocess_state(_P(st.data_ptr()), int(st.numel()), _P(a.data_ptr()), _P(b.data_ptr()), int(a.numel()), self.mode,
-                                                    _P(out_bf16.data_ptr()) if out_bf16 is not None else None, _P(z.data_ptr()),
-                                                    _P(bins.data_ptr()) if bins is not None else None, self._stream()), "rtvla_preprocess_state")
+        rc = self.lib.rtvla_preprocess_state_host(st.__array_interface__["data"][0], st.size, a.data_ptr(), b.data_ptr(), n_stats, self.mode,
+                                                  out_bf16.data_ptr() if out_bf16 is not None else None, z.data_ptr(),
+                                                  bins.data_ptr() if bins is not None else None, self._stream())
+        if rc:
+            self._check(rc, "rtvla_preprocess_state_host")
         return z, bins
 
     # ---- actions ----
@@ -98,16 +115,16 @@ class ObservationTransforms:
         """test.py:196-201: un-normalise, add the current state, keep the grippers absolute -> float64 [chunk, action_dim]."""
         if "actions" not in self._stats:
             return None
-        a, b = self._stats["actions"]
-        if actions_bf16.dtype != torch.bfloat16 or actions_bf16.shape[-1] != 32 or not actions_bf16.is_contiguous():
+        a, b, n_stats = self._stats["actions"]
+        if actions_bf16.dtype is not torch.bfloat16 or actions_bf16.shape[-1] != 32 or not actions_bf16.is_contiguous():
             raise ValueError("actions must be a contiguous bf16 [chunk, 32] tensor")
-        chunk = int(actions_bf16.shape[0])
-        st = torch.zeros(32, dtype=torch.float64, device=self.device)
-        s_in = torch.as_tensor(np.asarray(ori_state, dtype=np.float64))
-        st[: s_in.numel()] = s_in.to(self.device)
-        out = torch.empty(chunk, self.action_dim, dtype=torch.float64, device=self.device)
-        self._check(self.lib.rtvla_postprocess_actions(_P(actions_bf16.data_ptr()), chunk, _P(a.data_ptr()), _P(b.data_ptr()), int(a.numel()), self.mode,
-                                                       _P(st.data_ptr()), self.action_dim, _P(out.data_ptr()), self._stream()), "rtvla_postprocess_actions")
+        chunk = actions_bf16.shape[0]
+        st = np.ascontiguousarray(ori_state, dtype=np.float64)
+        out = torch.empty((chunk, self.action_dim), dtype=torch.float64, device=self.device)
+        rc = self.lib.rtvla_postprocess_actions_host(actions_bf16.data_ptr(), chunk, a.data_ptr(), b.data_ptr(), n_stats, self.mode,
+                                                     st.__array_interface__["data"][0], st.size, self.action_dim, out.data_ptr(), self._stream())
+        if rc:
+            self._check(rc, "rtvla_postprocess_actions_host")
         return out
 
     # ---- the whole observation, as TritonInference.infer does around policy.forward (test.py:181-205) ----

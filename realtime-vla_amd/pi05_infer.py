@@ -129,8 +129,12 @@ class Pi05Inference:
         n = int(ids.shape[0])
         if n > self.max_prompt_len:
             raise ValueError(f"{n} prompt tokens exceed max_prompt_len {self.max_prompt_len}")
-        self.buffers['prompt_token_ids'][:n].copy_(ids)
-        self.buffers['valid_encoder_len'].fill_(self.num_views * 256 + n)
+        if ids.is_cuda:
+            self.buffers['prompt_token_ids'][:n].copy_(ids)
+            self.buffers['valid_encoder_len'].fill_(self.num_views * 256 + n)
+        else:
+            # the ids travel with a launch: a copy from host memory would wait for the forward before this one
+            self._engine.ctx.stage_prompt(ids.to(torch.int64).contiguous(), torch.cuda.current_stream(self._engine.device).cuda_stream)
 
     def forward_ids(self, observation_images_normalized, diffusion_noise, token_ids) -> torch.Tensor:
         """forward() for callers that tokenise themselves (no counterpart in the reference, whose tokenizer call is

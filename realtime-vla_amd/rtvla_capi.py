@@ -25,6 +25,7 @@ TILE_AUTO, TILE_SKINNY = -1, -2
 ACT_BIAS_GELU, ACT_GEGLU, ACT_SWIGLU = 1, 2, 3
 NORM_NONE, NORM_RMS, NORM_LAYER = 0, 1, 2
 ATTN_GEMMA_PREFIX, ATTN_GEMMA_SUFFIX, ATTN_GQA128_PREFIX, ATTN_GQA128_SUFFIX, ATTN_VIT64, ATTN_SIGLIP = range(6)
+FRAME_U8_HWC, FRAME_F32_HWC, FRAME_F32_CHW, FRAME_U8_CHW = range(4)
 STATIC_SCRATCH_BYTES = 2160 * 224 * 3          # RTVLA_STATIC_SCRATCH_BYTES
 
 
@@ -57,6 +58,7 @@ SYMBOLS = {
     "rtvla_tiled_bytes": (ctypes.c_size_t, [_P]),
     "rtvla_tile_layout_version": (ctypes.c_int, []),
     "rtvla_forward": (ctypes.c_int, [_P, _P]),
+    "rtvla_stage_prompt": (ctypes.c_int, [_P, _P, ctypes.c_int, _P]),
     "rtvla_forward_stage": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
     "rtvla_graph_capture": (ctypes.c_int, [_P, _P]),
     "rtvla_graph_launch": (ctypes.c_int, [_P, _P]),
@@ -81,6 +83,9 @@ SYMBOLS = {
     "rtvla_preprocess_image_scratch": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int]),
     "rtvla_preprocess_image": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, _P, _P, ctypes.c_size_t, _P]),
     "rtvla_preprocess_image_static": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, _P, _P]),
+    "rtvla_preprocess_frame": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P, _P]),
+    "rtvla_preprocess_state_host": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, ctypes.c_int, ctypes.c_int, _P, _P, _P, _P]),
+    "rtvla_postprocess_actions_host": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, ctypes.c_int, ctypes.c_int, _P, ctypes.c_int, ctypes.c_int, _P, _P]),
     "rtvla_preprocess_state": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, ctypes.c_int, ctypes.c_int, _P, _P, _P, _P]),
     "rtvla_postprocess_actions": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, ctypes.c_int, ctypes.c_int, _P, ctypes.c_int, _P, _P]),
 }
@@ -173,6 +178,10 @@ class Context:
 
     def forward(self, stream):
         self.check(self.lib.rtvla_forward(self.handle, _P(stream)))
+
+    def stage_prompt(self, ids, stream):
+        """`ids`: contiguous int64 CPU tensor, read before the call returns."""
+        self.check(self.lib.rtvla_stage_prompt(self.handle, ids.data_ptr(), ids.numel(), stream))
 
     def forward_stage(self, stage, layer, step, stream):
         self.check(self.lib.rtvla_forward_stage(self.handle, stage, layer, step, _P(stream)))

@@ -30,6 +30,24 @@ def test_image_preprocessing_matches_the_pillow_restatement_bit_exactly(h, w):
     assert torch.equal(got, want), "mismatching elements: %d" % (got != want).sum().item()
 
 
+@pytest.mark.parametrize("h,w", [(1, 1), (4, 5), (9, 300), (300, 9), (223, 225), (479, 641), (717, 1279), (2700, 1801)])
+@pytest.mark.parametrize("fmt", ["u8", "u8_chw", "f32", "f32_chw"])
+def test_frame_formats_at_the_edges_of_the_tiles(h, w, fmt):
+    """Every frame format on the device: single pixels, strips narrower than a tile, windows that end with the buffer, both tile heights."""
+    from oracle import transforms as T
+    from obs_transforms import ObservationTransforms
+    tr = ObservationTransforms("pi0")
+    img = np.random.RandomState(h * 31 + w).randint(0, 256, size=(h, w, 3)).astype(np.uint8)
+    x = img if fmt.startswith("u8") else (img.astype(np.float32) + 0.3) / 255.0
+    if fmt.endswith("chw"):
+        x = x.transpose(2, 0, 1).copy()
+    want = torch.from_numpy(T.normalize_image(T.resize_with_pad(T.parse_image(x)))).to(torch.bfloat16)      # (three rows are read as channels first)
+    frame = torch.from_numpy(x).cuda()
+    out = torch.full((224, 224, 3), 7.0, dtype=torch.bfloat16, device="cuda:0")
+    tr.resize_pad_normalize_into(frame, out)
+    assert torch.equal(out.cpu(), want)
+
+
 def test_image_inputs_float_and_chw_and_errors():
     from oracle import transforms as T
     from obs_transforms import ObservationTransforms
