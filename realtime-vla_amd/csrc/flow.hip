@@ -19,11 +19,17 @@
 // into half the CUs each and the weights twice per XCD (once from memory).  The eight compute waves split K and reduce through LDS; a
 // ninth wave does the waiting, so that the compute waves can have the next phase's weights on the way while it polls.
 //
-// All workgroups have to be resident at once: the launcher keeps one flow kernel per device in flight, and a wait that lasts longer
-// than FLOW_WAIT_TICKS ends (the kernel then runs to its end without waiting and the actions become NaN), so the grid always drains.
+// All workgroups have to be resident at once.  A process keeps one flow kernel per device in flight (rtvla.hip), but another process's
+// may be placed on half of the CUs at the same moment.  So no workgroup starts before all 256 have reported: the last one opens the
+// gate, and one that has waited too long closes it, after which all of them leave and the CUs are free.  The kernel is therefore
+// launched twice; the second launch ends at once if the first one ran (the gate and that launch: 6 us of a forward of 8 - 14 ms), and
+// the two processes' first limits differ.  Past the gate every wait still ends after FLOW_WAIT_TICKS (the kernel then runs to its end
+// without waiting and the actions become NaN, as they do where both gates were closed), so the grid always drains.
 #include "kernels.h"
 #include <algorithm>
 #include <atomic>
+#include <mutex>
+#include <unistd.h>
 
 namespace {
 
@@ -79,6 +85,30 @@ struct Patience {
     }
 };
 
+// The gate of one launch (thread 0 of each workgroup): `rank` gets the workgroup's number on its XCD, `gate` what was decided.
+enum { GATE_UNDECIDED = 0, GATE_OPEN = 1, GATE_CLOSED = 2, GATE_DONE = 3 };
+RTVLA_DEVICE void flow_gate(FlowSync* sync, int attempt, int xcc, unsigned ticks, int* rank, int* gate) {
+    auto word = [](unsigned* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    auto decide = [](unsigned* p, unsigned to) {
+        unsigned none = GATE_UNDECIDED;
+        __hip_atomic_compare_exchange_strong(p, &none, to, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    *rank = 0;
+    for (int k = 0; k < attempt; ++k)                                          // (that launch has ended)
+        if (word(&sync->gate[k]) == GATE_OPEN) { *gate = GATE_DONE; return; }
+    unsigned* const g = &sync->gate[attempt];
+    *rank = (int)atomicAdd(&sync->rank[attempt][xcc * 32], 1u);
+    if (*rank >= 32) decide(g, GATE_CLOSED);                                   // not 32 workgroups per XCD
+    else if (atomicAdd(&sync->arrived[attempt], 1u) == 255u) decide(g, GATE_OPEN);
+    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+    unsigned v;
+    while ((v = word(g)) == GATE_UNDECIDED) {
+        if (__builtin_amdgcn_s_memrealtime() - t0 > ticks) decide(g, GATE_CLOSED);
+        __builtin_amdgcn_s_sleep(1);
+    }
+    *gate = (int)v;
+}
+
 // D[16 x 16] = A[16 x 16] B[16 x 16] of one half (4 elements per lane) of two 16 x 32 fragments
 RTVLA_DEVICE f32x4 mfma16k16(bf16x8 a, bf16x8 b, int hi) {
     typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -129,11 +159,17 @@ void flow_kernel(FlowP kernel_args) {
     if (tid == 0) {
         const int xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7;         // HW_REG_XCC_ID
         sh[0] = xcc;
-        sh[1] = (int)atomicAdd(&kernel_args.sync->rank[xcc * 32], 1u);
+        flow_gate(kernel_args.sync, kernel_args.attempt, xcc, kernel_args.gate_ticks, &sh[1], &sh[2]);
     }
     __syncthreads();
     const int x_ = __builtin_amdgcn_readfirstlane(sh[0]), r_ = __builtin_amdgcn_readfirstlane(sh[1]);
-    if (r_ >= 32) { if (tid == 0) atomicOr(&kernel_args.sync->abort, 1u); return; }       // not 32 workgroups per XCD: the others give up waiting
+    if (const int gate = __builtin_amdgcn_readfirstlane(sh[2]); gate != GATE_OPEN) {
+        if (gate == GATE_CLOSED && kernel_args.attempt == FLOW_ATTEMPTS - 1) {             // no attempt left: actions nobody can take for actions
+            const int n = (kernel_args.rows - (MODEL == FLOW_PI0 ? 1 : 0)) * 32;
+            if (kernel_args.end) for (int i = tid; i < n; i += FLOW_THREADS) kernel_args.noise_out[i] = f2bf(__uint_as_float(0x7fc00000u));
+        }
+        return;
+    }
     const int step0 = kernel_args.step0, step1 = kernel_args.step1, layer0 = kernel_args.layer0, layer1 = kernel_args.layer1;
     const bool begin = kernel_args.begin != 0, end = kernel_args.end != 0;
     const bool keep_in = layer0 == layer1;                                     // (a single stage: the new stream goes back to the caller's buffer)
@@ -894,11 +930,9 @@ __global__ __launch_bounds__(256) void flow_init_kernel(FlowSync* sync, uint4* p
 __global__ __launch_bounds__(FLOW_THREADS) void flow_check_kernel(FlowSync* sync) {
     if (threadIdx.x != 0) return;
     const int xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7;
-    if (atomicAdd(&sync->rank[xcc * 32], 1u) >= 32u) atomicOr(&sync->abort, 1u);
-    __hip_atomic_fetch_add(&sync->lflag[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
-    while (__hip_atomic_load(&sync->lflag[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < 256u)
-        if (__builtin_amdgcn_s_memrealtime() - t0 > 5000000ull) { atomicOr(&sync->abort, 1u); break; }      // 50 ms
+    int rank, gate;
+    flow_gate(sync, 0, xcc, 5000000u, &rank, &gate);                           // 50 ms
+    if (gate != GATE_OPEN) atomicOr(&sync->abort, 1u);
 }
 
 template <int MODEL, int RH>
@@ -907,8 +941,15 @@ int launch_inst(const FlowP& p, hipStream_t s) {
     auto kern = flow_kernel<MODEL, RH>;
     static std::atomic<uint64_t> done{0};
     if (int rc = ensure_dynamic_lds((const void*)kern, smem, done)) return rc;
-    hipLaunchKernelGGL(kern, dim3(256), dim3(FLOW_THREADS), smem, s, p);
-    return hipGetLastError() == hipSuccess ? 0 : 5;
+    // first limit 5 - 20 ms, the last one 2 - 3.5 s; which of each differs from process to process
+    const unsigned spread = ((unsigned)getpid() * 2654435761u) >> 28;
+    FlowP q = p;
+    for (q.attempt = 0; q.attempt < FLOW_ATTEMPTS; ++q.attempt) {
+        q.gate_ticks = q.attempt < FLOW_ATTEMPTS - 1 ? 500000u + spread * 100000u : 200000000u + spread * 10000000u;
+        hipLaunchKernelGGL(kern, dim3(256), dim3(FLOW_THREADS), smem, s, q);
+        if (hipGetLastError() != hipSuccess) return 5;
+    }
+    return 0;
 }
 
 }  // namespace
@@ -948,8 +989,11 @@ int launch_flow(const FlowP& p, int model, hipStream_t s) {
 // a partitioned device or under a CU mask).  Tried once per device with a kernel that does nothing else; every wait in it ends.
 bool flow_supported(FlowSync* sync, hipStream_t s) {
     static std::atomic<int> known[64];                                         // 0: not tried, 1: yes, 2: no
+    static std::mutex trying;                                                  // two checks at once could close each other's gates
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+    if (const int k = known[dev].load(std::memory_order_acquire)) return k == 1;
+    const std::lock_guard<std::mutex> lock(trying);
     if (const int k = known[dev].load(std::memory_order_acquire)) return k == 1;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
     bool ok = cus == 256;

@@ -170,10 +170,12 @@ void launch_vision_attention(const bf16_t* q, const bf16_t* k, const bf16_t* vt,
 
 // ----- the action expert's flow loop as one resident kernel (csrc/flow.hip) ------------------------------------
 enum FlowModel { FLOW_PI0 = 0, FLOW_PI05, FLOW_DM0 };
-struct FlowSync { unsigned rank[8 * 32], lflag[8 * 256], abort, pad[31]; };
+constexpr int FLOW_ATTEMPTS = 2;               // launches of which one runs, see csrc/flow.hip
+struct FlowSync { unsigned rank[FLOW_ATTEMPTS][8 * 32], lflag[8 * 256], abort, pad[31], arrived[FLOW_ATTEMPTS], gate[FLOW_ATTEMPTS], pad2[28]; };
 struct FlowP {
     // program: flow steps [step0, step1), each: input projection (begin), layers [layer0, layer1), output projection + Euler (end)
     int step0, step1, layer0, layer1, begin, end;
+    int attempt; unsigned gate_ticks;          // set by launch_flow
     int layers, rows, prefix;                  // layers of the model, suffix rows (state token included), prefix rows as allocated
     const int* valid_len;                      // visible prefix rows, or null: all
     float scale;

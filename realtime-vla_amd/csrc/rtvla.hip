@@ -615,7 +615,7 @@ struct Sched {
             launch_flow_init(p.sync, p.part, p.part_bytes, st ? c->W("observation_state_normalized") : nullptr, st ? c->W("decoder_state_in_proj_w") : nullptr, st ? c->W("decoder_state_in_proj_b") : nullptr, sx, s);
             c->note(0, "flow init");
         }
-        if (c->want(what)) c->note(launch_flow(p, dm0 ? FLOW_DM0 : pi05 ? FLOW_PI05 : FLOW_PI0, s), what);
+        if (c->want(what)) c->note(launch_flow(p, dm0 ? FLOW_DM0 : pi05 ? FLOW_PI05 : FLOW_PI0, s), what, FLOW_ATTEMPTS);
     }
 
     void suffix_init() {}
@@ -1174,7 +1174,7 @@ int rtvla_buffer_info(const rtvla_ctx* c, int index, const char** name, size_t* 
 static int prepare_impl(rtvla_ctx* c, void* stream, bool tiles_loaded) {
     if (int rc = check_ready(c, false)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;
-    c->flow = flow_supported((FlowSync*)c->B<float>("flow_sync"), (hipStream_t)stream);
+    c->flow = !capturing((hipStream_t)stream) && flow_supported((FlowSync*)c->B<float>("flow_sync"), (hipStream_t)stream);      // (it waits for its answer)
     Sched(c, (hipStream_t)stream).prepare(tiles_loaded);
     if (c->status) return c->status;
     hipError_t e = hipGetLastError();
