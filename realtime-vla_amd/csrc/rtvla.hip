@@ -610,12 +610,12 @@ struct Sched {
         p.priv = (char*)c->B<float>("flow_priv"); p.part = c->B<float>("flow_part"); p.sync = (FlowSync*)c->B<float>("flow_sync");
         bf16_t* const sx = c->B("flow_state_x");
         p.state_x = sx;
-        if (c->want("flow init")) {
+        // one unit for the per-launch timing as well: the kernel needs the flags and the exchange buffers as its init leaves them
+        if (c->want(what)) {
             const bool st = begin && !pi05 && !dm0;
             launch_flow_init(p.sync, p.part, p.part_bytes, st ? c->W("observation_state_normalized") : nullptr, st ? c->W("decoder_state_in_proj_w") : nullptr, st ? c->W("decoder_state_in_proj_b") : nullptr, sx, s);
-            c->note(0, "flow init");
+            c->note(launch_flow(p, dm0 ? FLOW_DM0 : pi05 ? FLOW_PI05 : FLOW_PI0, s), what, 1 + FLOW_ATTEMPTS);
         }
-        if (c->want(what)) c->note(launch_flow(p, dm0 ? FLOW_DM0 : pi05 ? FLOW_PI05 : FLOW_PI0, s), what, FLOW_ATTEMPTS);
     }
 
     void suffix_init() {}
@@ -1282,7 +1282,10 @@ static int time_replay(rtvla_ctx* c, hipStream_t s, int stage, int layer, int st
     e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) { c->only = -1; return hip_fail(c, e, "hipStreamBeginCapture"); }
     int enqueued = 0;
-    for (int i = 0; i < iters && !rc; ++i)
+    // the layers of a flow step as the forward runs them: one launch of the resident kernel
+    const bool resident = cycle && launch_index < 0 && stage == RTVLA_STAGE_SUFFIX_LAYER && c->flow;
+    for (int i = 0; resident && i < iters; ++i) { sc.flow(step, step + 1, 0, n_layers, false, false, "flow layers"); enqueued += n_layers; }
+    for (int i = 0; !resident && i < iters && !rc; ++i)
         for (int l = first; l < first + n_layers && !rc; ++l) {
             c->launches = 0; c->kernels = 0;
             rc = sc.stage(stage, l, step);
