@@ -191,12 +191,15 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
     // ---- epilogue: lane (h, r) holds rows m = m0 + 32 i + r, columns n = 32 tile + 8 grp + 4 h + e ----
     // Row-major outputs go through LDS one 32-row tile at a time so that the global stores are whole
     // 16-byte chunks of contiguous row segments (256 B - 1 KB per row) instead of 8-byte pieces of 32 rows.
-    constexpr bool ROWMAJOR = (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU || EPI == EPI_PATCH || EPI == EPI_GEGLU || EPI == EPI_SWIGLU || EPI == EPI_PARTIAL);
+    constexpr bool ROWMAJOR = (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU || EPI == EPI_PATCH || EPI == EPI_GEGLU || EPI == EPI_SWIGLU || EPI == EPI_PARTIAL ||
+                              EPI == EPI_RESIDUAL);
     if constexpr (ROWMAJOR) {
-        constexpr int ESZ = (EPI == EPI_PARTIAL) ? 4 : 2;
+        constexpr bool RES = EPI == EPI_RESIDUAL;                  // staged as fp32: the residual joins on the way out, where a row's chunks are contiguous
+        constexpr int ESZ = (EPI == EPI_PARTIAL || RES) ? 4 : 2;
         constexpr int OUTW = WN * HALF * 32;                       // output columns of the workgroup
         constexpr int ROWB = OUTW * ESZ + 16;                      // padded LDS row pitch in bytes
-        constexpr int CPR = OUTW * ESZ / 16;                       // 16-byte chunks per row
+        constexpr int COLS = EPI == EPI_PARTIAL ? 4 : 8;           // columns of a 16-byte output chunk
+        constexpr int CPR = OUTW / COLS;                           // chunks per row
         constexpr int RPP = NTH / CPR;                             // rows per copy pass
         static_assert(NTH % CPR == 0 && 32 % RPP == 0, "copy-out mapping");
         unsigned char* obuf = smem_raw;
@@ -208,6 +211,14 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
         constexpr int GROUP = (3 * BM * 128) / TILE_B >= MT ? MT : ((3 * BM * 128) / TILE_B < 1 ? 1 : (3 * BM * 128) / TILE_B);
 #pragma unroll
         for (int g0 = 0; g0 < MT; g0 += GROUP) {
+          bf16x8 res[RES ? GROUP * (32 / RPP) : 1];
+          if constexpr (RES) {
+#pragma unroll
+            for (int k = 0; k < GROUP * (32 / RPP); ++k) {
+                const int mm = min(m0 + (g0 + k / (32 / RPP)) * 32 + (k % (32 / RPP)) * RPP + tid / CPR, p.M - 1), n = min(nbase + (tid % CPR) * COLS, ncols - COLS);
+                res[k] = *(const bf16x8*)(p.res + (size_t)mm * p.ldr + n);
+            }
+          }
 #pragma unroll
           for (int i = g0; i < (g0 + GROUP < MT ? g0 + GROUP : MT); ++i) {
             if (m0 + i * 32 >= p.M) continue;                                     // a row tile past the end (uniform)
@@ -247,7 +258,8 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
 #pragma unroll
                             for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
                         }
-                        *(bf16x4*)dst = pack4(v);
+                        if constexpr (RES) *(f32x4*)dst = v;
+                        else *(bf16x4*)dst = pack4(v);
                     }
                 }
             }
@@ -260,8 +272,17 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
             for (int ps = 0; ps < 32 / RPP; ++ps) {
                 const int row = ps * RPP + tid / CPR, ch = tid % CPR;
                 const int mm = m0 + i * 32 + row;
-                const int n = nbase + ch * (16 / ESZ);
+                const int n = nbase + ch * COLS;
                 if (mm < p.M && n < ncols) {
+                    if constexpr (RES) {
+                        f32x4 lo = *(const f32x4*)(tbuf + row * ROWB + ch * 32), hi = *(const f32x4*)(tbuf + row * ROWB + ch * 32 + 16);
+                        const bf16x8 rs = res[(i - g0) * (32 / RPP) + ps];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) { lo[e] += bf2f(rs[e]); hi[e] += bf2f(rs[4 + e]); }
+                        const bf16x4 a = pack4(lo), b = pack4(hi);
+                        *(uint4*)(p.out + (size_t)mm * p.ldo + n) = uint4{((const uint2*)&a)->x, ((const uint2*)&a)->y, ((const uint2*)&b)->x, ((const uint2*)&b)->y};
+                        continue;                                  // (no streaming hint: the normalising pass reads it next)
+                    }
                     const uint4 val = *(const uint4*)(tbuf + row * ROWB + ch * 16);
                     // (streaming hint: the output is read once by the next launch and should not displace the operand tiles in L2)
                     if constexpr (EPI == EPI_PARTIAL) __builtin_nontemporal_store(*(const f32x4*)&val, (f32x4*)(p.partial + (size_t)split * p.pstride + (size_t)mm * p.ldp + n));
@@ -431,7 +452,7 @@ int launch_cfg(const GemmP& p, hipStream_t s) {
     if (MT > 4 && ((sps & 1) || (stages_total & 1))) return 3;              // the large tiles consume K stages in pairs
     GemmP q = p; q.nsplit = nsplit;
     // three K-stage buffers; the row-major epilogues stage 32-row output tiles in the same memory
-    const size_t epi_bytes = (size_t)32 * (WN * HALF * 32 * (EPI == EPI_PARTIAL ? 4 : 2) + 16);
+    const size_t epi_bytes = (size_t)32 * (WN * HALF * 32 * (EPI == EPI_PARTIAL || EPI == EPI_RESIDUAL ? 4 : 2) + 16);
     const size_t smem = std::max((size_t)3 * BM * 64 * sizeof(bf16_t), epi_bytes);
     auto kern = gemm_mfma_kernel<WN, MT, NT, EPI, MIXED>;
     if (smem > 65536) {
@@ -472,6 +493,7 @@ int launch_gemm(const GemmP& p, int epi, int tile, hipStream_t s) {
         case EPI_PATCH:     return launch_epi<EPI_PATCH>(p, tile, s);
         case EPI_GEGLU:     return launch_epi<EPI_GEGLU>(p, tile, s);
         case EPI_PARTIAL:   return launch_epi<EPI_PARTIAL>(p, tile, s);
+        case EPI_RESIDUAL:  return launch_epi<EPI_RESIDUAL>(p, tile, s);
         case EPI_QKV_ROPE:  return launch_epi<EPI_QKV_ROPE>(p, tile, s);
         case EPI_VIS_QKV:   return launch_epi<EPI_VIS_QKV>(p, tile, s);
         case EPI_SWIGLU:    return launch_epi<EPI_SWIGLU>(p, tile, s);

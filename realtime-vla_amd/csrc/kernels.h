@@ -49,6 +49,7 @@ enum GemmEpilogue {
     EPI_PATCH,         // out = acc + bias + res[row % res_mod]
     EPI_GEGLU,         // out = gelu_tanh(acc(B0)) * acc(B1)
     EPI_PARTIAL,       // fp32 split-K partial
+    EPI_RESIDUAL,      // out = acc + bias + res[row], where out and res may be the same rows
     EPI_QKV_ROPE,      // Gemma prefix: bf16 -> interleaved RoPE on Q,K -> Q / K cache / transposed V cache
     EPI_VIS_QKV,       // SigLIP: +bias, Q|K row-major, V transposed per (view, head)
     EPI_SWIGLU,        // out = silu(acc(B0) * rowscale[row]) * (acc(B1) * rowscale[row])   (DM0 prefix MLP)

@@ -188,6 +188,24 @@ def test_fused_activation_epilogues_against_fp32(M, K, N, act):
     assert ran >= 3
 
 
+@pytest.mark.parametrize("M", [1, 3, 5, 2720])
+def test_layer_norm_of_1024_wide_rows_alone(M):
+    """Four rows a workgroup, so row counts off by one; against float64: half a bf16 step of the result, and of the sum's terms fp32 errors."""
+    import rtvla_capi as capi
+    lib = capi.load()
+    g = torch.Generator(device="cuda:0").manual_seed(M)
+    x = (torch.randn(M, 1024, device="cuda:0", generator=g) * 2 + 0.5).bfloat16()
+    w = (1 + 0.1 * torch.randn(1024, device="cuda:0", generator=g)).bfloat16()
+    b = (0.1 * torch.randn(1024, device="cuda:0", generator=g)).bfloat16()
+    out = torch.full((M + 1, 1024), 9.0, dtype=torch.bfloat16, device="cuda:0")
+    assert lib.rtvla_reduce_norm(None, 0, M, 1024, None, _P(x.data_ptr()), 2, _P(w.data_ptr()), _P(b.data_ptr()), ctypes.c_float(1e-5),
+                                 None, _P(out.data_ptr()), _P(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    ref = torch.nn.functional.layer_norm(x.double(), (1024,), w.double(), b.double(), 1e-5)
+    assert ((out[:M].double() - ref).abs() <= ref.abs() * 2.0 ** -8 + 1e-5).all()
+    assert (out[M] == 9.0).all()
+
+
 @pytest.mark.parametrize("M,N,nsplit,norm,has_bias,has_res", [
     (768, 1152, 2, 2, True, True),        # SigLIP O projection: split 2 + bias + residual + LayerNorm
     (768, 1152, 4, 2, True, True),        # SigLIP down projection
