@@ -235,6 +235,14 @@ void flow_kernel(FlowP kernel_args) {
             const int x = x_, r = r_;
             int tn = t, ln = l + 1;                                            // the layer after this one
             if (ln == layer1) { ln = layer0; tn = t + 1 < step1 ? t + 1 : t; }
+            // what a phase reads of a few kilobytes that nothing else has touched: norm weights (DM0), biases and gates (Pi05)
+            if constexpr (DM0) {
+                if (k == 4 && r < 2) touch((r ? p.knorm : p.qnorm) + (size_t)ln * 128, 0, 256, 1);
+            } else if constexpr (PI05) {
+                const size_t tl = (size_t)t * p.layers + l;
+                if (k == 4 && r < 2) touch(p.bias_qkv + ((size_t)tn * p.layers + ln) * 2560 + (r ? 2048 : x * 256), 0, r ? 2048 : 1024, 1);
+                if (k == 0 && r < 4) touch(r == 0 ? (const void*)(p.style_attn + tl * 3072 + 2048) : r == 1 ? (const void*)(p.style_ffn + tl * 3072 + 2048) : (const void*)((r == 2 ? p.bias_gate : p.bias_up) + tl * 4096 + x * C::HID), 0, 2048, 1);
+            }
             if (k <= 2) {                                                      // gate and up tiles of this layer: 2 x 32 KB of every workgroup, in thirds
                 if (r < C::HID / 16) {
                     const size_t o = (size_t)(PI05 ? t * p.layers + l : l) * p.wg_stride + (size_t)(x * (C::HID / 16) + r) * 32 * 512;
@@ -640,8 +648,9 @@ void flow_kernel(FlowP kernel_args) {
             }
         }
     };
-    // The peers' tiles are requested, then `pre` (weights of the next phase) runs in their shadow; what had not arrived is asked for again.
-    auto sum_residual = [&](cFlowP& p, bool keep, const f32x4 (&own)[SK], const bf16_t* gp, auto&& pre) __attribute__((always_inline)) {
+    // The peers' tiles are requested and what had not arrived is asked for again.  Nothing else may be in flight here: loads return in
+    // order, so weights requested between the two would hold up every further look (64 - 96 KB per workgroup, 1.6 - 2.5 us).
+    auto sum_residual = [&](cFlowP& p, bool keep, const f32x4 (&own)[SK], const bf16_t* gp) __attribute__((always_inline)) {
         FLOW_IDS;
 #pragma unroll
         for (int k = 0; k < SK; ++k) {
@@ -653,16 +662,11 @@ void flow_kernel(FlowP kernel_args) {
                 return __builtin_amdgcn_raw_buffer_load_b128(part, in && y != x ? part_off(ex, y, r, u, lane) : 0x7fffff00, 0, SYS);
             };
             u32x4 v[8];
-#pragma unroll
-            for (int y = 0; y < 8; ++y) v[y] = load(y);
             const bf16x4 xold = ld8(priv, p.off_x + ft_off(row, col, 32));
             bf16x4 gate = {};
             if constexpr (PI05) gate = load4(gp + col);
-            if (k == 0) {
-                __builtin_amdgcn_sched_barrier(0);
-                pre();
-                __builtin_amdgcn_sched_barrier(0);
-            }
+#pragma unroll
+            for (int y = 0; y < 8; ++y) v[y] = load(y);
             for (;;) {
                 bool missing = false;
 #pragma unroll
@@ -883,9 +887,8 @@ void flow_kernel(FlowP kernel_args) {
                 bar();
                 store_part(FW, own);
                 cFlowP& p = prm();
-                sum_residual(p, false, own, PI05 ? p.style_attn + ((size_t)t * p.layers + l) * 3072 + 2048 : nullptr,
-                             [&]() __attribute__((always_inline)) { load_e(prm(), t, l, 1, wE); });
-                sync(reset_part);
+                sum_residual(p, false, own, PI05 ? p.style_attn + ((size_t)t * p.layers + l) * 3072 + 2048 : nullptr);
+                sync([&]() __attribute__((always_inline)) { reset_part(); load_e(prm(), t, l, 1, wE); });
                 mlp_up(prm(), t, l, wE);
             }
             {
@@ -898,10 +901,9 @@ void flow_kernel(FlowP kernel_args) {
                 bar();
                 store_part(C::FWAVES, own);
                 cFlowP& p = prm();
-                sum_residual(p, lastl, own, PI05 ? p.style_ffn + ((size_t)t * p.layers + l) * 3072 + 2048 : nullptr,
-                             [&]() __attribute__((always_inline)) { pre_qkv(prm(), t, lastl ? l : l + 1, wA, cs); });      // (after the last layer for nothing)
+                sum_residual(p, lastl, own, PI05 ? p.style_ffn + ((size_t)t * p.layers + l) * 3072 + 2048 : nullptr);
             }
-            sync(reset_part);
+            sync([&]() __attribute__((always_inline)) { reset_part(); pre_qkv(prm(), t, lastl ? l : l + 1, wA, cs); });      // (after the last layer for nothing)
         }
         if (end) {
             euler(prm(), t);
