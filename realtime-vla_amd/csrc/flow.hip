@@ -38,6 +38,7 @@ constexpr int FLOW_THREADS = (FW + 2) * 64;              // + the wave that post
 constexpr unsigned long long FLOW_WAIT_TICKS = 200000000ull;      // 2 s of the 100 MHz counter
 constexpr float NEG_BIG = -1.0e30f;
 constexpr int SQ_BYTES = FW * 4 * 64;
+constexpr int ROPE_PITCH = 272;                                       // 256 bytes of a row, and 16 that move the next one to other banks
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
@@ -144,6 +145,7 @@ void flow_kernel(FlowP kernel_args) {
     f32x4* const red = (f32x4*)smem;                                           // [wave][tile][64]
     float* const sq = (float*)(smem + FW * 4 * RH * 1024);                     // [wave][RH * 16] row sums of squares; [2][wave][16] maxima and sums of P V
     int* const sh = (int*)(smem + FW * 4 * RH * 1024 + SQ_BYTES);
+    unsigned char* const rope_lds = smem + FW * 4 * RH * 1024 + SQ_BYTES + 320;       // DM0: the rotary table of the suffix rows, [row][ROPE_PITCH]
 
     // The parameters are read from the kernel-argument segment where they are used: hoisted out of the loops they would not fit the
     // scalar registers.  prm() hides the pointer from the optimiser so that each phase loads its own.
@@ -161,6 +163,9 @@ void flow_kernel(FlowP kernel_args) {
         sh[0] = xcc;
         flow_gate(kernel_args.sync, kernel_args.attempt, xcc, kernel_args.gate_ticks, &sh[1], &sh[2]);
     }
+    if constexpr (DM0)
+        for (int i = tid; i < RTP * 16 * 16; i += FLOW_THREADS)
+            *(uint4*)(rope_lds + (i >> 4) * ROPE_PITCH + (i & 15) * 16) = *(const uint4*)(kernel_args.rope + (size_t)min(i >> 4, kernel_args.rows - 1) * 128 + (i & 15) * 8);
     __syncthreads();
     const int x_ = __builtin_amdgcn_readfirstlane(sh[0]), r_ = __builtin_amdgcn_readfirstlane(sh[1]);
     if (const int gate = __builtin_amdgcn_readfirstlane(sh[2]); gate != GATE_OPEN) {
@@ -469,12 +474,11 @@ void flow_kernel(FlowP kernel_args) {
     };
 
     // DM0: factor, RMS norm over the head's 128 features, norm weight, rotary embedding on adjacent pairs; lane holds 8 features per block
-    auto dm0_qk = [&](cFlowP& p, int g, bf16x8 (&v)[KD], int tok, const bf16_t* nw) __attribute__((always_inline)) {
-        const float f = ld4(priv, p.off_f + tok * 4);
-        const int rr = min(tok, rows - 1);
+    // The rotary table comes from LDS: from memory it would be 4 KB per wave and row tile, more than the queries.
+    auto dm0_qk = [&](int g, bf16x8 (&v)[KD], float f, int tok, const bf16_t* nw) __attribute__((always_inline)) {
         bf16x8 cs[KD], ww[KD];
 #pragma unroll
-        for (int kd = 0; kd < KD; ++kd) { cs[kd] = *(const bf16x8*)(p.rope + (size_t)rr * 128 + kd * 32 + 8 * g); ww[kd] = *(const bf16x8*)(nw + kd * 32 + 8 * g); }
+        for (int kd = 0; kd < KD; ++kd) { cs[kd] = *(const bf16x8*)(rope_lds + tok * ROPE_PITCH + kd * 64 + 16 * g); ww[kd] = *(const bf16x8*)(nw + kd * 32 + 8 * g); }
         float y[KD][8], s = 0.f;
 #pragma unroll
         for (int kd = 0; kd < KD; ++kd)
@@ -492,7 +496,8 @@ void flow_kernel(FlowP kernel_args) {
     };
 
     // ---- logits of (query row tile, 16 keys) per wave and their exponentials relative to the row maximum over those 16 keys ----
-    // Workgroup: the 32-key blocks r, r + 32, ...; wave: one half of the block (w & 1), row tiles (w >> 1), + 4, ...
+    // Workgroup: the 32-key blocks r, r + 32, ...; wave: one half of the block (w & 1), row tiles (w >> 1), + 4
+    constexpr int NQ = (QRT + 3) / 4;
     auto load_k = [&](cFlowP& p, int lane, int x, int l, int nt, int kb, bf16x8 (&kf)[KD]) __attribute__((always_inline)) {
         const bf16_t* base = p.kcache + (size_t)(DM0 ? l * 8 + x : l) * p.kv_stride;
 #pragma unroll
@@ -505,26 +510,50 @@ void flow_kernel(FlowP kernel_args) {
     auto logits = [&](cFlowP& p, int l, bf16x8 (&kf)[KD]) __attribute__((always_inline)) {
         FLOW_IDS;
         const int nt = w & 1;
+        if (r >= KB) return;
+        auto new_k = [&](int kb) __attribute__((always_inline)) {
+#pragma unroll
+            for (int kd = 0; kd < KD; ++kd) kf[kd] = ld16(priv, p.off_k + frag_off((kb - KBp) * 2 + nt, kd, KD, lane));
+        };
+        auto key_row = [&](int kb) __attribute__((always_inline)) { return min(((kb - KBp) * 2 + nt) * 16 + lr, RTP * 16 - 1); };
+        // all that the first block needs is requested before any of it is used
+        bf16x8 qf[NQ][KD];
+#pragma unroll
+        for (int i = 0; i < NQ; ++i)
+#pragma unroll
+            for (int kd = 0; kd < KD; ++kd) qf[i][kd] = ld16(priv, p.off_q + frag_off(min((w >> 1) + 4 * i, QRT - 1), kd, KD, lane));
+        float fq = 0.f, fk = 0.f;
+        const int tok0 = ((w >> 1) % RTP) * 16 + lr;
+        if constexpr (DM0) fq = ld4(priv, p.off_f + tok0 * 4);                         // (both row tiles of a wave are of the same tokens)
+        if (r >= KBp) {
+            new_k(r);
+            if constexpr (DM0) fk = ld4(priv, p.off_f + key_row(r) * 4);
+        }
+        if constexpr (DM0) {
+            static_assert(NQ == 1 || RTP == 4, "row tiles four apart are of the same tokens");
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) dm0_qk(g, qf[i], fq, tok0, p.qnorm + (size_t)l * 128);
+        }
         for (int kb = r; kb < KB; kb += 32) {
             if (kb >= KBp) {
-#pragma unroll
-                for (int kd = 0; kd < KD; ++kd) kf[kd] = ld16(priv, p.off_k + frag_off((kb - KBp) * 2 + nt, kd, KD, lane));
-                if constexpr (DM0) dm0_qk(p, g, kf, ((kb - KBp) * 2 + nt) * 16 + lr, p.knorm + (size_t)l * 128);
+                if (kb >= 32) {
+                    new_k(kb);
+                    if constexpr (DM0) fk = ld4(priv, p.off_f + key_row(kb) * 4);
+                }
+                if constexpr (DM0) dm0_qk(g, kf, fk, key_row(kb), p.knorm + (size_t)l * 128);
             } else if (kb >= 32) load_k(p, lane, x, l, nt, kb, kf);
             // the keys of this lane: 4 g .. 4 g + 3 of the 16; visible are those below `lim` (of the state row, among the new keys, only the first)
             const int key = nt * 16 + 4 * g;
             const int lim = kb < KBp ? vl - kb * 32 : rows - (kb - KBp) * 32;
             const int lim_state = kb < KBp ? lim : KBp == kb ? 1 : 0;
-            for (int rt = w >> 1; rt < QRT; rt += 4) {
-                bf16x8 qf[KD];
 #pragma unroll
-                for (int kd = 0; kd < KD; ++kd) qf[kd] = ld16(priv, p.off_q + frag_off(rt, kd, KD, lane));
-                const int tok = (rt % RTP) * 16 + lr;
-                if constexpr (DM0) dm0_qk(p, g, qf, tok, p.qnorm + (size_t)l * 128);
+            for (int i = 0; i < NQ; ++i) {
+                const int rt = (w >> 1) + 4 * i;
+                if (QRT % 4 != 0 && rt >= QRT) continue;
+                const int lm = (MODEL == FLOW_PI0 && rt % RTP == 0 && lr == 0) ? lim_state : lim;      // the state token sees the prefix and itself
                 f32x4 st = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int kd = 0; kd < KD; ++kd) st = mfma16(kf[kd], qf[kd], st);
-                const int lm = (MODEL == FLOW_PI0 && tok == 0) ? lim_state : lim;      // the state token sees the prefix and itself
+                for (int kd = 0; kd < KD; ++kd) st = mfma16(kf[kd], qf[i][kd], st);
                 float mx = NEG_BIG;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -939,7 +968,7 @@ __global__ __launch_bounds__(FLOW_THREADS) void flow_check_kernel(FlowSync* sync
 
 template <int MODEL, int RH>
 int launch_inst(const FlowP& p, hipStream_t s) {
-    const size_t smem = std::max((size_t)FW * 4 * RH * 1024 + SQ_BYTES + 64 + 256, (size_t)96 * 1024);      // more than half a CU's LDS: one workgroup per CU
+    const size_t smem = std::max((size_t)FW * 4 * RH * 1024 + SQ_BYTES + 320 + (MODEL == FLOW_DM0 ? 2 * RH * 16 * ROPE_PITCH : 0), (size_t)96 * 1024);      // more than half a CU's LDS: one workgroup per CU
     auto kern = flow_kernel<MODEL, RH>;
     static std::atomic<uint64_t> done{0};
     if (int rc = ensure_dynamic_lds((const void*)kern, smem, done)) return rc;
