@@ -279,10 +279,10 @@ int launch8_cfg(const GemmP& p, hipStream_t s) {
     constexpr int HALF = Epi8<EPI>::dual ? 1 : 2;
     constexpr int ESZ = (EPI == EPI_PARTIAL) ? 4 : 2;
     const int tiles = (p.M + 31) / 32;
-    const int m_blocks = (tiles + MT - 1) / MT;
+    const int n_blocks = ((p.N16 + 1) / 2 + 4 * HALF - 1) / (4 * HALF);
+    const int m_blocks = gemm8_row_blocks(tiles, MT, n_blocks);
     int n_big = tiles - m_blocks * (MT - 1);
     if (n_big < 0) n_big = 0;
-    const int n_blocks = ((p.N16 + 1) / 2 + 4 * HALF - 1) / (4 * HALF);
     const int stages_total = p.K32p / 2;
     const int nsplit = p.nsplit < 1 ? 1 : p.nsplit;
     const int sps = (stages_total + nsplit - 1) / nsplit;
@@ -304,12 +304,19 @@ int launch8_epi(const GemmP& p, int tile, hipStream_t s) {
         case TILE8_256x256: return launch8_cfg<8, EPI>(p, s);
         case TILE8_224x256: return launch8_cfg<7, EPI>(p, s);
         case TILE8_192x256: return launch8_cfg<6, EPI>(p, s);
-        case TILE8_128x256: return launch8_cfg<4, EPI>(p, s);
+        case TILE8_128x256: if constexpr (EPI != EPI_VIT_QKV_ROPE) return launch8_cfg<4, EPI>(p, s); else return 2;
     }
     return 2;
 }
 
 }  // namespace
+
+// As many row blocks as the last round of 256 workgroups has room for: 8 160 rows by 3 072 columns in blocks of at most 224 rows are
+// 37 x 12 = 444 workgroups, two rounds whose second leaves 68 CUs idle; as 42 x 12 = 504 nearly all CUs get two smaller ones.
+int gemm8_row_blocks(int row_tiles, int mt, int n_blocks) {
+    const int least = (row_tiles + mt - 1) / mt, room = (least * n_blocks + 255) / 256 * 256 / n_blocks;
+    return mt > 4 ? std::max(least, std::min(room, row_tiles / (mt - 1))) : least;      // (the short tile runs two workgroups per CU)
+}
 
 int launch_gemm8(const GemmP& p, int epi, int tile, hipStream_t s) {
     if (p.M <= 0 || p.N16 <= 0 || p.K32p <= 0 || (p.K32p & 1) || p.a_rows <= 0 || p.bgroup < 1) return 1;

@@ -84,6 +84,7 @@ int gemm_tile_bm(int tile);
 int gemm_tile_bn(int tile);
 int launch_gemm(const GemmP& p, int epi, int tile, hipStream_t s);
 int launch_gemm8(const GemmP& p, int epi, int tile, hipStream_t s);
+int gemm8_row_blocks(int row_tiles, int mt, int n_blocks);      // row blocks of an eight-wave launch with tiles of up to mt 32-row tiles
 
 // ----- split-K reduce + bias + residual (+ gate) + normalisation -----------------------
 enum NormMode { NORM_NONE = 0, NORM_RMS, NORM_LAYER };

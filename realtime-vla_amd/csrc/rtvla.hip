@@ -114,34 +114,33 @@ constexpr int XN_LD = 2048 + 64;   // row strides that are a large power of two 
 constexpr int EHID_LD = 16384 + 64;
 constexpr int64_t ATTN_PARTIAL_FLOATS = 64 * 16 * (16 * 64 * 4 + 32);   // 64 row blocks (128 suffix rows x 8 heads) x 16 key splits of the suffix attention
 
-// Pick block tile and split-K factor from a cost model fitted to measurements on MI355X.  One K stage of a
-// workgroup takes the larger of its MFMA time (32 cycles per 32x32x16 MFMA at the ~2.05 GHz the chip sustains,
-// 75 % issue efficiency) and a latency-bound load time (0.1 us + 6.7 us per MB of operands pulled by the
-// workgroup); tiles of 64 rows run two workgroups per CU, which then share the MFMA pipe but overlap
-// their load latency; all workgroups together cannot pull more than ~20 TB/s out of L2; every launch pays a
-// fixed ramp and an epilogue that grows with the tile; split-K adds the reduce pass over the fp32 partials.
-TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittable, const char* what, int eight = 0) {
-    static const int tiles[] = {TILE_224x256, TILE_192x256, TILE_160x256, TILE_128x256, TILE_64x256, TILE_128x128, TILE_64x128};
+// Pick block tile and split-K factor from a cost model fitted to measurements on MI355X (every tile and split on 73 shapes: the GEMMs of
+// a SigLIP, Gemma, DM0 ViT and DM0 prefix layer at one to four views, weights cold).  One K stage of a workgroup takes the larger of its
+// MFMA time (32 cycles per 32x32x16 MFMA at 2.05 GHz and 48 % issue efficiency) and a latency-bound load time (0.11 us + 10.4 us per MB
+// of operands pulled by the workgroup); tiles of 64 rows run two workgroups per CU, which then share the MFMA pipe but overlap their load
+// latency; all workgroups together cannot pull more than 17 TB/s out of L2; every launch pays a fixed ramp and an epilogue that grows
+// with the tile; split-K adds the reduce pass over the fp32 partials.  Over those shapes, weighted by the launches per forward, the choice
+// is 0.46 ms off the best one in sum (1.48 ms before the fit, with a table of exceptions and without the 96-row tile): SigLIP
+// up-projection at 768 rows 128x128 15.8 -> 64x128 14.0 us, DM0 ViT output projection at 2 720 rows 64x128 17.0 -> 96x128 13.4 us.
+TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittable, const char* what, bool eight = false) {
+    static const int tiles[] = {TILE_224x256, TILE_192x256, TILE_160x256, TILE_128x256, TILE_64x256, TILE_128x128, TILE_96x128, TILE_64x128};
     static const int splits[] = {1, 2, 3, 4, 6, 8};
     { TileChoice forced; if (tuning_forced_tile(what, splittable, &forced.tile, &forced.nsplit)) return forced; }
     // measured (M = 8115, K = 1024, N = 4096, bias + GELU): the eight-wave 256 x 256 tile takes 84-89 us where the best four-wave
-    // tile takes 98-101 us; with 788 rows, with the gated epilogues and with fp32 split-K partials the four-wave tiles win
-    // (eight: 1 = bias (+ GELU) epilogue, 2 = the ViT QKV epilogue, measured 75 us with the eight-wave 128 x 256 tile against 93 us)
-    if (eight && M >= 4096 && stages <= 32 && ncols16 >= 128) return TileChoice{eight == 1 ? TILE8_256x256 : TILE8_128x256, 1};
-    // shapes where timing the launch inside a layer (weights streamed from HBM) disagrees with the model below: the K = 4304
-    // SigLIP down-projection gains from four K splits (more workgroups pulling the 9.9 MB of weights at once, 22.1 -> 19.3 us
-    // with the reduce pass at 768 rows, 20.4 -> 14.4 us at 256 rows), the 788-row prefix QKV from 96-row tiles (22.0 -> 20.5 us), and so does
-    // the SigLIP QKV GEMM at three views (768 rows as 8 x 27 = 216 workgroups, one per CU, instead of 324 on 256 CUs: 14.8 -> 12.4 us)
-    struct Measured { int ncols16, stages, splittable, m_lo, m_hi, tile, nsplit; };
-    static const Measured measured[] = {
-        {72, 68, 1, 1, 512, TILE_64x128, 4},
-        {72, 68, 1, 513, 768, TILE_128x128, 4},
-        {160, 32, 0, 769, 1024, TILE_96x128, 1},
-        {216, 18, 0, 673, 768, TILE_96x128, 1},
-    };
-    if (!dual)
-        for (const Measured& e : measured)
-            if (e.ncols16 == ncols16 && e.stages == stages && e.splittable == (splittable ? 1 : 0) && M >= e.m_lo && M <= e.m_hi) return TileChoice{e.tile, e.nsplit};
+    // tile takes 93-101 us, N = 3072 with the ViT QKV epilogue 77 us against 79-93 us; with 788 rows, with the gated epilogues and with fp32
+    // split-K partials the four-wave tiles win.  Of the eight-wave tiles the one whose rounds of 256 workgroups cost the fewest row tiles,
+    // one more per round for its ramp (5 440 rows: N = 4096 256 rows 66.3 -> 192 rows 59.4 us, N = 3072 128 rows 66.8 -> 192 rows 60.2 us)
+    if (eight && M >= 4096 && stages <= 32 && ncols16 >= 128) {
+        TileChoice c8{TILE8_256x256, 1};
+        int least = 1 << 30;
+        for (int tile : {TILE8_256x256, TILE8_224x256, TILE8_192x256}) {
+            const int cols = (ncols16 + 15) / 16, row_tiles = (M + 31) / 32;
+            const int m_blocks = gemm8_row_blocks(row_tiles, gemm_tile_bm(tile) / 32, cols);
+            const int cost = (m_blocks * cols + 255) / 256 * ((row_tiles + m_blocks - 1) / m_blocks + 1);
+            if (cost < least) { least = cost; c8.tile = tile; }
+        }
+        return c8;
+    }
     double best = 1e30; TileChoice bc{TILE_128x256, 1};
     for (int tile : tiles) {
         const int bm = gemm_tile_bm(tile);
@@ -162,14 +161,12 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
             if (bm > 128 && ((sps & 1) || (tail & 1))) continue;          // the large tiles consume K stages in pairs
             const int blocks = mb * nb * sp;
             const int per_cu = (blocks + 255) / 256;
-            const int together = std::min(occ, per_cu);
-            const int rounds = (per_cu + occ - 1) / occ;
-            const double mfma_us = mt * nt * 4 * 32 / 2050.0 / 0.75;
+            const double mfma_us = mt * nt * 4 * 32 / 2050.0 / 0.48;
             const double stage_bytes = (double)(bm + bn) * 64 * 2;
-            const double stage_us = std::max(together * mfma_us, 0.1 + stage_bytes / 1.5e5);
-            double t = std::max(rounds * sps * stage_us, blocks * (double)sps * stage_bytes / 20.0e6);
-            t += 3.5 + 2.0 + 1.2 * mt * (splittable ? 1.5 : 1.0);
-            if (splittable) t += 3.5 + (double)sp * M * ncols16 * 16 * 4.0 / 4.0e6;    // the reduce pass reads the partials at ~4 TB/s
+            const double alone_us = std::max(mfma_us, 0.11 + stage_bytes / 9.6e4), pair_us = std::max(occ * mfma_us, 0.11 + stage_bytes / 9.6e4);
+            double t = std::max((per_cu / occ * pair_us + per_cu % occ * alone_us) * sps, blocks * (double)sps * stage_bytes / 17.2e6);
+            t += 5.9 + 1.2 * mt * (splittable ? 1.5 : 1.0);
+            if (splittable) t += 2.2 + (double)sp * M * ncols16 * 16 * 4.0 / 7.5e6;    // the reduce pass over the partials
             if (t < best) { best = t; bc = TileChoice{tile, sp}; }
         }
     }
@@ -472,7 +469,7 @@ struct Sched {
         GemmP p = extra;
         p.A = A; p.lda = lda; p.a_rows = a_rows; p.M = M; p.B0 = B0; p.B1 = B1;
         p.N16 = n16_tiles(N); p.K32p = k32_padded(K); p.bgroup = bgroup;
-        const TileChoice tc = choose_tile(M, p.N16, p.K32p / 2, epi == EPI_GEGLU || epi == EPI_SWIGLU, epi == EPI_PARTIAL, what, (epi == EPI_BIAS || epi == EPI_BIAS_GELU) ? 1 : epi == EPI_VIT_QKV_ROPE ? 2 : 0);
+        const TileChoice tc = choose_tile(M, p.N16, p.K32p / 2, epi == EPI_GEGLU || epi == EPI_SWIGLU, epi == EPI_PARTIAL, what, epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_VIT_QKV_ROPE);
         p.nsplit = tc.nsplit;
         if (epi == EPI_PARTIAL) {
             p.partial = c->B<float>("splitk_partial"); p.ldp = N; p.pstride = (size_t)M * N;
@@ -1498,7 +1495,7 @@ int plan_linear_act(int M, int K, int N, int act, int tile, ActPlan* out) {
     ActPlan p{};
     p.dual = act != RTVLA_ACT_BIAS_GELU;
     p.K128 = k32_padded(K) * 32;
-    p.tile = tile >= 0 ? tile : choose_tile(M, n16_tiles(N), k32_padded(K) / 2, p.dual, false, "linear act", p.dual ? 0 : 1).tile;
+    p.tile = tile >= 0 ? tile : choose_tile(M, n16_tiles(N), k32_padded(K) / 2, p.dual, false, "linear act", !p.dual).tile;
     if (p.dual && (gemm_tile_bn(p.tile) != 256 || gemm_tile_eight_waves(p.tile))) return RTVLA_ERR_LIMIT;      // gate and up share a 256-column workgroup tile
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const int G = p.dual ? 4 : 8;
