@@ -141,6 +141,14 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
         }
         return c8;
     }
+    // row counts where a launch by itself (its weights of a few layers stay in the last-level cache) disagrees with the whole forward, which
+    // was timed with either choice: SigLIP down-projection at 768 rows 128x128 against the model's 64x128, four splits each: 60 us less a
+    // forward; SigLIP output projection at 1 024 rows, two splits against the model's three: 95 us less
+    struct Measured { int ncols16, stages, m_lo, m_hi, tile, nsplit; };
+    static const Measured measured[] = {{72, 68, 513, 768, TILE_128x128, 4}, {72, 18, 769, 1024, TILE_64x128, 2}};
+    if (splittable)
+        for (const Measured& e : measured)
+            if (e.ncols16 == ncols16 && e.stages == stages && M >= e.m_lo && M <= e.m_hi) return TileChoice{e.tile, e.nsplit};
     double best = 1e30; TileChoice bc{TILE_128x256, 1};
     for (int tile : tiles) {
         const int bm = gemm_tile_bm(tile);
@@ -150,7 +158,8 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
         const int mb = (M + bm - 1) / bm, nb = (ncols16 + bn16 - 1) / bn16;
         const int nt = bn / 128;
         // the 256-column tiles of 128 rows and more mix row blocks of bm and bm - 32 rows: average 32-row tiles per block
-        const double mt = (bm >= 128 && bn == 256) ? (double)((M + 31) / 32) / mb : bm / 32;
+        // (at least the smaller size: 256 rows in blocks of at most 224 are two blocks of 192, the rest of them padding)
+        const double mt = (bm >= 128 && bn == 256) ? std::max((double)((M + 31) / 32) / mb, bm / 32 - 1.0) : bm / 32;
         if (!dual && tile == TILE_64x256) continue;        // measured: 64x128 is never slower than 64x256 for the single-weight GEMMs
         const int occ = bm <= 64 ? 2 : 1;
         for (int sp : splits) {
@@ -167,7 +176,7 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
             double t = std::max((per_cu / occ * pair_us + per_cu % occ * alone_us) * sps, blocks * (double)sps * stage_bytes / 17.2e6);
             t += 5.9 + 1.2 * mt * (splittable ? 1.5 : 1.0);
             if (splittable) t += 2.2 + (double)sp * M * ncols16 * 16 * 4.0 / 7.5e6;    // the reduce pass over the partials
-            if (t < best) { best = t; bc = TileChoice{tile, sp}; }
+            if (t <= best) { best = t; bc = TileChoice{tile, sp}; }      // (of equals the smaller tile)
         }
     }
     tuning_report_tile(what, M, ncols16 * 16, stages, gemm_tile_bm(bc.tile), gemm_tile_bn(bc.tile), bc.nsplit, best);
