@@ -171,6 +171,16 @@ int rtvla_graph_capture(rtvla_ctx* ctx, void* hip_stream);
  * rtvla_graph_launch then returns RTVLA_ERR_STATE until rtvla_prepare and rtvla_graph_capture have run again. */
 int rtvla_graph_launch(rtvla_ctx* ctx, void* hip_stream);
 
+/* How long the flow loop's resident kernel waits before it gives way (no reference counterpart).  The kernel needs every compute unit of
+ * the device at the same moment.  While kernels of other processes or streams hold some, its first launch waits `first_ms` (default 5 - 20)
+ * and its second `second_ms` (200 - 350) for all of its workgroups to be placed; a loop that has begun waits `wait_ms` (2000) for a
+ * workgroup that does not answer.  If none of them finishes, one workgroup runs the whole loop by itself: the same actions bit for bit, in
+ * about a second instead of 5 - 7 ms.  No forward is lost.  0: does not wait at all, negative: the default. */
+int rtvla_flow_limits(rtvla_ctx* ctx, float first_ms, float second_ms, float wait_ms);
+/* Read without waiting for anything: whether the flow loop is enqueued as the resident kernel (1) or as launches (0), and of the forwards
+ * and stages that have ended so far, how many had the loop run in one workgroup (modulo 2^32).  Either pointer may be null. */
+int rtvla_flow_status(const rtvla_ctx* ctx, int32_t* resident, uint32_t* alone);
+
 /* Number of kernels the last forward (or stage) enqueued: the kernel nodes of the captured graph. */
 int rtvla_launch_count(const rtvla_ctx* ctx);
 

@@ -172,12 +172,15 @@ void launch_vision_attention(const bf16_t* q, const bf16_t* k, const bf16_t* vt,
 
 // ----- the action expert's flow loop as one resident kernel (csrc/flow.hip) ------------------------------------
 enum FlowModel { FLOW_PI0 = 0, FLOW_PI05, FLOW_DM0 };
-constexpr int FLOW_ATTEMPTS = 2;               // launches of which one runs, see csrc/flow.hip
+constexpr int FLOW_ATTEMPTS = 2;               // launches of the whole grid, of which one runs; a third, of one workgroup, runs if neither did (csrc/flow.hip)
+constexpr int FLOW_LAUNCHES = FLOW_ATTEMPTS + 1;
 struct FlowSync { unsigned rank[FLOW_ATTEMPTS][8 * 32], lflag[8 * 256], abort, pad[31], arrived[FLOW_ATTEMPTS], gate[FLOW_ATTEMPTS], pad2[28]; };
 struct FlowP {
     // program: flow steps [step0, step1), each: input projection (begin), layers [layer0, layer1), output projection + Euler (end)
     int step0, step1, layer0, layer1, begin, end;
     int attempt; unsigned gate_ticks;          // set by launch_flow
+    unsigned gate_limits[FLOW_ATTEMPTS], wait_ticks;           // in 10 ns; 0: the gate closes at once / no wait is waited out
+    unsigned* alone;                           // host memory: programs that ran in one workgroup, or null
     int layers, rows, prefix;                  // layers of the model, suffix rows (state token included), prefix rows as allocated
     const int* valid_len;                      // visible prefix rows, or null: all
     float scale;
@@ -190,17 +193,18 @@ struct FlowP {
     const bf16_t* rope;                        // [row][256] (DM0: 128)
     const bf16_t* state_x;                     // Pi0: the projected state token
     bf16_t *kcache, *vcache; size_t kv_stride; int ldvt;
-    const bf16_t* noise; bf16_t* noise_out;    // [chunk][32], may be the same
-    bf16_t* x;                                 // residual stream, fragment-tiled: read by programs without `begin`, written by all
+    const bf16_t* noise; bf16_t* noise_out;    // [chunk][32]
+    const bf16_t* x_in; bf16_t* x;             // residual stream, fragment-tiled: where programs without `begin` start, where all end
     char* priv; size_t priv_stride;            // memory of one XCD's own, 8 of them
     int off_x, off_xin, off_q, off_k, off_v, off_o, off_h, off_n, off_f, off_m, off_p;
     float* part; unsigned part_bytes;          // fp32 partial sums exchanged between the XCDs
     FlowSync* sync;
 };
+struct FlowStart { const uint4 *noise, *x; uint4 *noise_copy, *x_copy; int noise16, x16; };      // what launch_flow_init copies, in 16-byte pieces
 int flow_row_pairs(int rows);                  // the kernel's row-tile pairs (template argument) for that many suffix rows
 // byte offsets inside one XCD's memory; returns its size.  qrows: query row tiles per XCD, blocks: 32-key blocks, hidden: MLP columns per XCD
 size_t flow_layout(FlowP* p, int qtiles, int blocks, int hidden);
-void launch_flow_init(FlowSync* sync, float* part, unsigned part_bytes, const bf16_t* state, const bf16_t* w, const bf16_t* b, bf16_t* out, hipStream_t s);
+void launch_flow_init(FlowSync* sync, float* part, unsigned part_bytes, const FlowStart& start, const bf16_t* state, const bf16_t* w, const bf16_t* b, bf16_t* out, hipStream_t s);
 int launch_flow(const FlowP& p, int model, hipStream_t s);
 bool flow_supported(FlowSync* sync, hipStream_t s);      // whether the current device can run it (tried once per device; synchronises then)
 

@@ -13,9 +13,32 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <unistd.h>
 #include <vector>
 
 namespace {
+
+// Words in pinned host memory that a kernel counts in and the host reads without waiting.  One page-sized allocation per process, made
+// at the first use and never freed, so that a kernel still running when its context goes can write to it; a word is given back with its context.
+class HostWords {
+    static constexpr int COUNT = 1024;
+    std::mutex m;
+    unsigned* base = nullptr;
+    bool used[COUNT] = {};
+public:
+    unsigned* take() {
+        const std::lock_guard<std::mutex> lock(m);
+        if (!base && hipHostMalloc((void**)&base, COUNT * sizeof(unsigned), hipHostMallocPortable) != hipSuccess) { base = nullptr; (void)hipGetLastError(); return nullptr; }
+        for (int i = 0; i < COUNT; ++i)
+            if (!used[i]) { used[i] = true; __atomic_store_n(base + i, 0u, __ATOMIC_RELAXED); return base + i; }
+        return nullptr;
+    }
+    void give(unsigned* p) {
+        const std::lock_guard<std::mutex> lock(m);
+        if (p) used[p - base] = false;
+    }
+};
+HostWords host_words;
 
 struct Tensor {
     std::string name;
@@ -53,7 +76,8 @@ struct rtvla_ctx {
     char* ws = nullptr;
     bool prepared = false;
     bool flow = false;             // the flow loop runs as one resident kernel (csrc/flow.hip); false: as launches, see flow_supported()
-    FlowP flow_p{};                // its private-memory layout (build_tables)
+    FlowP flow_p{};                // its private-memory layout (build_tables) and limits (rtvla_flow_limits)
+    unsigned* flow_alone = nullptr;          // host word the flow kernel counts in: loops that ran in one workgroup (HostWords)
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     hipStream_t timing_stream = nullptr;     // the measurement helpers capture graphs, which the null stream cannot
@@ -183,6 +207,17 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
     return bc;
 }
 
+// How long the flow kernel's launches wait before they give way (csrc/flow.hip), in milliseconds; negative: the default.  The first launch
+// gives way quickly (another process's loop takes 5 - 12 ms), the second outlasts several of those; which time exactly differs from
+// process to process, so that two of them do not close and retry in step.
+void set_flow_limits(rtvla_ctx* c, float first_ms, float second_ms, float wait_ms) {
+    const unsigned spread = ((unsigned)getpid() * 2654435761u) >> 28;
+    auto ticks = [](float ms, unsigned otherwise) { return ms < 0.f ? otherwise : (unsigned)std::min((double)ms * 1e5, 4e9); };
+    c->flow_p.gate_limits[0] = ticks(first_ms, 500000u + spread * 100000u);                 // 5 - 20 ms
+    c->flow_p.gate_limits[1] = ticks(second_ms, 20000000u + spread * 1000000u);             // 200 - 350 ms
+    c->flow_p.wait_ticks = ticks(wait_ms, 200000000u);                                      // 2 s
+}
+
 // what the resident flow kernel needs besides the model's buffers
 void add_flow_buffers(rtvla_ctx* c, int heads, int hidden) {
     const int rh = flow_row_pairs(c->S_d);
@@ -192,6 +227,9 @@ void add_flow_buffers(rtvla_ctx* c, int heads, int hidden) {
     c->add_buf("flow_part", 1, c->flow_p.part_bytes / 4, c->flow_p.part_bytes / 4, 4);
     c->add_buf("flow_sync", 1, sizeof(FlowSync) / 4, sizeof(FlowSync) / 4, 4);
     c->add_buf("flow_state_x", 1, 1024, 1024);
+    c->add_buf("flow_noise", 128, 32, 32);
+    c->add_buf("flow_x", 128, 1024, 1024);
+    set_flow_limits(c, -1, -1, -1);
 }
 
 int build_tables(rtvla_ctx* c) {
@@ -624,15 +662,18 @@ struct Sched {
         } else {
             p.kcache = Kc(0); p.vcache = Vt(0); p.kv_stride = (size_t)c->keys_pad * 256;
         }
-        p.noise = c->W("diffusion_noise"); p.noise_out = c->W("diffusion_noise"); p.x = c->B("decoder_x");
+        p.noise = c->B("flow_noise"); p.noise_out = c->W("diffusion_noise"); p.x_in = c->B("flow_x"); p.x = c->B("decoder_x");
+        p.alone = c->flow_alone;
+        const FlowStart start{(const uint4*)p.noise_out, (const uint4*)p.x, (uint4*)c->B("flow_noise"), (uint4*)c->B("flow_x"), d.chunk_size * 4,
+                              begin ? 0 : flow_row_pairs(c->S_d) * 32 * 1024 / 8};
         p.priv = (char*)c->B<float>("flow_priv"); p.part = c->B<float>("flow_part"); p.sync = (FlowSync*)c->B<float>("flow_sync");
         bf16_t* const sx = c->B("flow_state_x");
         p.state_x = sx;
         // one unit for the per-launch timing as well: the kernel needs the flags and the exchange buffers as its init leaves them
         if (c->want(what)) {
             const bool st = begin && !pi05 && !dm0;
-            launch_flow_init(p.sync, p.part, p.part_bytes, st ? c->W("observation_state_normalized") : nullptr, st ? c->W("decoder_state_in_proj_w") : nullptr, st ? c->W("decoder_state_in_proj_b") : nullptr, sx, s);
-            c->note(launch_flow(p, dm0 ? FLOW_DM0 : pi05 ? FLOW_PI05 : FLOW_PI0, s), what, 1 + FLOW_ATTEMPTS);
+            launch_flow_init(p.sync, p.part, p.part_bytes, start, st ? c->W("observation_state_normalized") : nullptr, st ? c->W("decoder_state_in_proj_w") : nullptr, st ? c->W("decoder_state_in_proj_b") : nullptr, sx, s);
+            c->note(launch_flow(p, dm0 ? FLOW_DM0 : pi05 ? FLOW_PI05 : FLOW_PI0, s), what, 1 + FLOW_LAUNCHES);
         }
     }
 
@@ -1125,6 +1166,7 @@ int rtvla_destroy(rtvla_ctx* c) {
     if (!c) return RTVLA_ERR_ARG;
     drop_graph(c);
     if (c->timing_stream) hipStreamDestroy(c->timing_stream);
+    host_words.give(c->flow_alone);
     delete c;
     return RTVLA_OK;
 }
@@ -1190,6 +1232,7 @@ int rtvla_buffer_info(const rtvla_ctx* c, int index, const char** name, size_t* 
 static int prepare_impl(rtvla_ctx* c, void* stream, bool tiles_loaded) {
     if (int rc = check_ready(c, false)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;
+    if (!c->flow_alone && !capturing((hipStream_t)stream)) c->flow_alone = host_words.take();
     c->flow = !capturing((hipStream_t)stream) && flow_supported((FlowSync*)c->B<float>("flow_sync"), (hipStream_t)stream);      // (it waits for its answer)
     Sched(c, (hipStream_t)stream).prepare(tiles_loaded);
     if (c->status) return c->status;
@@ -1264,6 +1307,20 @@ int rtvla_graph_launch(rtvla_ctx* c, void* stream) {
     if (turn.err != hipSuccess) return hip_fail(c, turn.err, "waiting for another stream's flow loop");
     hipError_t e = hipGraphLaunch(c->exec, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(c, e, "hipGraphLaunch");
+    return RTVLA_OK;
+}
+
+int rtvla_flow_limits(rtvla_ctx* c, float first_ms, float second_ms, float wait_ms) {
+    if (!c || first_ms != first_ms || second_ms != second_ms || wait_ms != wait_ms) return RTVLA_ERR_ARG;
+    set_flow_limits(c, first_ms, second_ms, wait_ms);
+    drop_graph(c);                               // (the captured launches carry the limits they were recorded with)
+    return RTVLA_OK;
+}
+
+int rtvla_flow_status(const rtvla_ctx* c, int32_t* resident, uint32_t* alone) {
+    if (!c) return RTVLA_ERR_ARG;
+    if (resident) *resident = c->flow;
+    if (alone) *alone = c->flow_alone ? __atomic_load_n(c->flow_alone, __ATOMIC_RELAXED) : 0;
     return RTVLA_OK;
 }
 

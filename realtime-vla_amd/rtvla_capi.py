@@ -62,6 +62,8 @@ SYMBOLS = {
     "rtvla_forward_stage": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
     "rtvla_graph_capture": (ctypes.c_int, [_P, _P]),
     "rtvla_graph_launch": (ctypes.c_int, [_P, _P]),
+    "rtvla_flow_limits": (ctypes.c_int, [_P, ctypes.c_float, ctypes.c_float, ctypes.c_float]),
+    "rtvla_flow_status": (ctypes.c_int, [_P, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_uint32)]),
     "rtvla_launch_count": (ctypes.c_int, [_P]),
     "rtvla_time_stage": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P, ctypes.POINTER(ctypes.c_float)]),
     "rtvla_time_launch": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P,
@@ -191,6 +193,15 @@ class Context:
 
     def graph_launch(self, stream):
         self.check(self.lib.rtvla_graph_launch(self.handle, _P(stream)))
+
+    def flow_limits(self, first_ms=-1.0, second_ms=-1.0, wait_ms=-1.0):
+        self.check(self.lib.rtvla_flow_limits(self.handle, first_ms, second_ms, wait_ms))
+
+    def flow_status(self):
+        """(the loop is the resident kernel, loops that ran in one workgroup)"""
+        resident, alone = ctypes.c_int32(), ctypes.c_uint32()
+        self.check(self.lib.rtvla_flow_status(self.handle, ctypes.byref(resident), ctypes.byref(alone)))
+        return bool(resident.value), alone.value
 
     def launch_count(self):
         return self.lib.rtvla_launch_count(self.handle)

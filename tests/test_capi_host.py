@@ -62,6 +62,19 @@ def test_create_validates_dimensions(lib):
     capi.Context(capi.PI05, 3, 52, 128).close()
 
 
+def test_flow_limits_and_status_need_no_device(lib):
+    c = capi.Context(capi.PI0, 1, 0, 50)
+    assert c.flow_status() == (False, 0)
+    for limits in ((), (0, 0, 0), (-1, 1e9, 2.5)):
+        c.flow_limits(*limits)
+    for bad in ((float("nan"), 1, 1), (1, float("nan"), 1), (1, 1, float("nan"))):
+        with pytest.raises(capi.RtvlaError) as e:
+            c.flow_limits(*bad)
+        assert e.value.code == 1
+    assert lib.rtvla_flow_limits(None, 1, 1, 1) == 1 and lib.rtvla_flow_status(None, None, None) == 1
+    assert lib.rtvla_flow_status(c.handle, None, None) == 0
+
+
 def test_tensor_table_matches_the_reference_layout(lib):
     c = capi.Context(capi.PI0, 3, 20, 50)
     t = {n: (e, s, w) for n, e, s, w, _ in c.tensors()}

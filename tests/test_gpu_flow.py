@@ -53,6 +53,57 @@ def test_resident_loop_equals_the_loop_as_launches(model, views, prompt, chunk):
     assert torch.equal(m.forward(*inputs).float().cpu(), resident)
 
 
+# suffix rows at the ends of every instance's range, a prefix that ends inside a 32-key block, past one round of the attention phases, and
+# a prompt that is shorter than its allocation (Pi05)
+SHAPES = [("pi0", 1, 5, 9), ("pi0", 1, 31, 50), ("pi0", 1, 7, 95), ("pi0", 4, 40, 127), ("pi05", 1, 9, 32), ("pi05", 1, 32, 64), ("pi05", 2, 21, 96),
+          ("pi05", 1, 5, 128), ("dm0", 1, 23, 50), ("dm0", 2, 24, 50)]
+
+
+# (the limits are the host's to set: a gate without patience closes before anybody reports, a loop without patience runs to its end at once)
+@pytest.mark.parametrize("limits", [(0, 0, -1), (-1, -1, 0)], ids=["gates closed", "loop given up"])
+@pytest.mark.parametrize("model,views,prompt,chunk", SHAPES)
+def test_one_workgroup_gives_the_same_actions(model, views, prompt, chunk, limits):
+    """Whatever keeps the resident kernel from finishing, the actions are those it would have given."""
+    m, inputs = policy(model, 500 + chunk, views, prompt, chunk)
+    ctx = m._engine.ctx
+    want = m.forward(*inputs).clone()
+    before = ctx.flow_status()[1]
+    ctx.flow_limits(*limits)
+    m._engine.capture()                                                      # (its eager forward is the first without patience)
+    got = m.forward(*inputs).clone()
+    torch.cuda.synchronize()
+    assert torch.isfinite(want.float()).all() and torch.equal(got, want)
+    assert ctx.flow_status() == (True, before + 2)
+    ctx.flow_limits()
+    m._engine.capture()
+    again = m.forward(*inputs).clone()
+    torch.cuda.synchronize()
+    assert torch.equal(again, want) and ctx.flow_status() == (True, before + 2)
+
+
+@pytest.mark.parametrize("model", ["pi0", "pi05", "dm0"])
+def test_one_workgroup_gives_the_same_layer(model):
+    """The stages start from the caller's stream and noise; a loop that gave up half way has spoiled neither."""
+    import rtvla_capi as capi
+    m, inputs = policy(model, 600, 1, 20, 40)
+    e = m._engine
+    m.forward(*inputs)
+    x, noise = e.buffers["decoder_x"], e.buffers["diffusion_noise"]
+    x0, n0 = x.clone(), noise.clone()
+    results = []
+    for limits in ((-1, -1, -1), (0, 0, -1), (-1, -1, 0)):
+        e.ctx.flow_limits(*limits)
+        for stage in (capi.STAGE_SUFFIX_STEP_BEGIN, capi.STAGE_SUFFIX_LAYER, capi.STAGE_SUFFIX_STEP_END):
+            x.copy_(x0)
+            noise.copy_(n0)
+            e.run_stage(stage, 1, 3)
+            torch.cuda.synchronize()
+            results.append((x.clone(), noise.clone()))
+    for k in range(3, 9):
+        assert torch.equal(results[k][0], results[k % 3][0]) and torch.equal(results[k][1], results[k % 3][1]), k
+    assert e.ctx.flow_status() == (True, 6)
+
+
 WORKER = """
 import sys
 sys.path[:0] = %r
