@@ -10,7 +10,9 @@
  *            -> rtvla_prepare -> [rtvla_graph_capture] -> rtvla_forward / rtvla_graph_launch ...
  *            -> rtvla_destroy.
  * One context = one static shape set (views, prompt length, chunk); single host thread per
- * context; calls that enqueue work on the same context must not overlap.
+ * context; calls that enqueue work on the same context must not overlap.  Contexts on different threads and
+ * streams are independent, but for their flow loops: a loop occupies the whole device, so the loops of one process
+ * run in the order in which they were enqueued, each behind the one before it (an event on the stream; no call waits).
  */
 #ifndef RTVLA_H
 #define RTVLA_H
@@ -164,7 +166,8 @@ int rtvla_stage_prompt(rtvla_ctx* ctx, const int64_t* ids_host, int n, void* hip
 /* Enqueue a single stage (see rtvla_stage); `layer` and `step` are ignored where meaningless. */
 int rtvla_forward_stage(rtvla_ctx* ctx, int stage, int layer, int step, void* hip_stream);
 
-/* Capture rtvla_forward into a HIP graph held by the context / replay it on a stream.
+/* Capture rtvla_forward into a HIP graph held by the context / replay it on a stream.  Where the flow loop is the resident kernel, the
+ * graph holds what comes before it, and rtvla_graph_launch enqueues the loop behind the graph, in its turn among the loops of the process.
  * Replaces record_infer_graph and infer_graph.replay() (pi0_infer.py:1347-1354, :1360). */
 int rtvla_graph_capture(rtvla_ctx* ctx, void* hip_stream);
 /* A graph records the addresses bound at capture time: rtvla_bind and rtvla_bind_workspace drop it, and
@@ -181,7 +184,7 @@ int rtvla_flow_limits(rtvla_ctx* ctx, float first_ms, float second_ms, float wai
  * and stages that have ended so far, how many had the loop run in one workgroup (modulo 2^32).  Either pointer may be null. */
 int rtvla_flow_status(const rtvla_ctx* ctx, int32_t* resident, uint32_t* alone);
 
-/* Number of kernels the last forward (or stage) enqueued: the kernel nodes of the captured graph. */
+/* Number of kernels the last forward (or stage) enqueued; after rtvla_graph_capture, those of one rtvla_graph_launch. */
 int rtvla_launch_count(const rtvla_ctx* ctx);
 
 /* Measurement helper (no reference counterpart): record `stage` `iters` times back to back into a temporary HIP

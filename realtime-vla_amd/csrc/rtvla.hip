@@ -6,6 +6,7 @@
 #include "kernels.h"
 #include "tuning.h"
 
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -76,7 +77,8 @@ struct rtvla_ctx {
     char* ws = nullptr;
     bool prepared = false;
     bool flow = false;             // the flow loop runs as one resident kernel (csrc/flow.hip); false: as launches, see flow_supported()
-    FlowP flow_p{};                // its private-memory layout (build_tables) and limits (rtvla_flow_limits)
+    FlowP flow_p{};                // its private-memory layout (build_tables)
+    unsigned gate_limit[FLOW_ATTEMPTS] = {}, gate_step[FLOW_ATTEMPTS] = {};      // how long its launches wait (set_flow_limits)
     unsigned* flow_alone = nullptr;          // host word the flow kernel counts in: loops that ran in one workgroup (HostWords)
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -208,14 +210,13 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
 }
 
 // How long the flow kernel's launches wait before they give way (csrc/flow.hip), in milliseconds; negative: the default.  The first launch
-// gives way quickly (another process's loop takes 5 - 12 ms), the second outlasts several of those; which time exactly differs from
-// process to process, so that two of them do not close and retry in step.
+// gives way quickly (another process's loop takes 5 - 12 ms), the second outlasts several of those; the defaults differ by up to 15 steps
+// from process to process and from loop to loop, so that two of them do not close and retry in step.
 void set_flow_limits(rtvla_ctx* c, float first_ms, float second_ms, float wait_ms) {
-    const unsigned spread = ((unsigned)getpid() * 2654435761u) >> 28;
     auto ticks = [](float ms, unsigned otherwise) { return ms < 0.f ? otherwise : (unsigned)std::min((double)ms * 1e5, 4e9); };
-    c->flow_p.gate_limits[0] = ticks(first_ms, 500000u + spread * 100000u);                 // 5 - 20 ms
-    c->flow_p.gate_limits[1] = ticks(second_ms, 20000000u + spread * 1000000u);             // 200 - 350 ms
-    c->flow_p.wait_ticks = ticks(wait_ms, 200000000u);                                      // 2 s
+    c->gate_limit[0] = ticks(first_ms, 500000u); c->gate_step[0] = first_ms < 0.f ? 100000u : 0;                  // 5 - 20 ms
+    c->gate_limit[1] = ticks(second_ms, 20000000u); c->gate_step[1] = second_ms < 0.f ? 1000000u : 0;             // 200 - 350 ms
+    c->flow_p.wait_ticks = ticks(wait_ms, 200000000u);                                                            // 2 s
 }
 
 // what the resident flow kernel needs besides the model's buffers
@@ -501,6 +502,40 @@ int build_tables_dm0(rtvla_ctx* c) {
     return 0;
 }
 
+// The flow kernel needs every CU of the device at the same moment (csrc/flow.hip): two of them, started on two streams, could each hold half of
+// the CUs and wait for the other half.  The launches of one loop are therefore enqueued behind the loop enqueued before it on this device,
+// whichever stream that was on; what comes before a loop is not held up.  The event is waited for on the same stream too: a stream is known
+// by its handle only, and a handle may be that of a stream that has gone.  A stream that is being captured is left alone (see FlowOff).
+constexpr int MAX_DEVICES = 64;
+struct FlowGate { std::mutex m; hipEvent_t done = nullptr; bool used = false; };
+FlowGate flow_gates[MAX_DEVICES];
+
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
+struct FlowTurn {
+    FlowGate* g = nullptr;
+    hipStream_t s;
+    hipError_t err = hipSuccess;
+    FlowTurn(const rtvla_ctx* c, hipStream_t stream) : s(stream) {
+        int dev = 0;
+        if (!c || !c->flow || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES || capturing(s)) return;
+        g = &flow_gates[dev];
+        g->m.lock();
+        if (!g->done) err = hipEventCreateWithFlags(&g->done, hipEventDisableTiming);
+        else if (g->used) err = hipStreamWaitEvent(s, g->done, 0);
+    }
+    ~FlowTurn() {
+        if (!g) return;
+        if (err == hipSuccess && hipEventRecord(g->done, s) == hipSuccess) g->used = true;
+        g->m.unlock();
+    }
+    FlowTurn(const FlowTurn&) = delete;
+    FlowTurn& operator=(const FlowTurn&) = delete;
+};
+
 // ------------------------------------------------------------------------------------------------
 // schedule
 // ------------------------------------------------------------------------------------------------
@@ -509,6 +544,7 @@ struct Sched {
     hipStream_t s;
     const rtvla_dims& d;
     bool pi05;
+    bool have_turn = false;        // the caller holds the device's FlowTurn
     Sched(rtvla_ctx* c_, hipStream_t s_) : c(c_), s(s_), d(c_->d), pi05(c_->d.model == RTVLA_PI05) {}
 
     void gemm(const bf16_t* A, int lda, int a_rows, int M, const bf16_t* B0, const bf16_t* B1, int K, int N, int epi, GemmP extra, const char* what) {
@@ -671,6 +707,11 @@ struct Sched {
         p.state_x = sx;
         // one unit for the per-launch timing as well: the kernel needs the flags and the exchange buffers as its init leaves them
         if (c->want(what)) {
+            static std::atomic<unsigned> loops{0};
+            const unsigned spread = ((unsigned)getpid() * 2654435761u + loops.fetch_add(1, std::memory_order_relaxed) * 1640531527u) >> 28;
+            for (int k = 0; k < FLOW_ATTEMPTS; ++k) p.gate_limits[k] = c->gate_limit[k] + spread * c->gate_step[k];
+            FlowTurn turn(have_turn ? nullptr : c, s);
+            if (turn.err != hipSuccess) { c->note(5, "waiting for the flow loop before this one"); return; }
             const bool st = begin && !pi05 && !dm0;
             launch_flow_init(p.sync, p.part, p.part_bytes, start, st ? c->W("observation_state_normalized") : nullptr, st ? c->W("decoder_state_in_proj_w") : nullptr, st ? c->W("decoder_state_in_proj_b") : nullptr, sx, s);
             c->note(launch_flow(p, dm0 ? FLOW_DM0 : pi05 ? FLOW_PI05 : FLOW_PI0, s), what, 1 + FLOW_LAUNCHES);
@@ -940,17 +981,11 @@ struct Sched {
         return 0;
     }
 
-    void dm0_forward() {
+    void dm0_front() {
         dm0_vision_embed();
         for (int i = 0; i < d.vision_layers; ++i) dm0_vision_layer(i);
         dm0_project();
         for (int i = 0; i < d.llm_layers; ++i) dm0_prefix_layer(i);
-        if (c->flow) { flow(0, d.num_steps, 0, d.llm_layers, true, true, "flow loop"); return; }
-        for (int t = 0; t < d.num_steps; ++t) {
-            dm0_step_begin(t);
-            for (int i = 0; i < d.llm_layers; ++i) dm0_suffix_layer(t, i);
-            dm0_step_end(t);
-        }
     }
 
     int stage(int st, int layer, int step) {
@@ -975,20 +1010,26 @@ struct Sched {
     // started on an idle GPU, and cost 0.9 - 1.7 ms of every replay queued behind another one: the branch's queue then holds a barrier
     // packet that waits for the whole earlier replay, and every dispatch of the running chain takes 0.6 us longer beside it.  Pi0, 3
     // views: 12.76 ms per replay with the branch, 11.79 ms without; DM0, 1 image: 17.7 and 16.0 ms.)
-    void forward() {
-        if (d.model == RTVLA_DM0) { dm0_forward(); return; }
+    void front() {
+        if (d.model == RTVLA_DM0) { dm0_front(); return; }
         vision_embed();
         for (int i = 0; i < d.vision_layers; ++i) vision_layer(i);
         project();
         suffix_init();
         for (int i = 0; i < d.llm_layers; ++i) prefix_layer(i);
+    }
+
+    void loop() {
         if (c->flow) { flow(0, d.num_steps, 0, d.llm_layers, true, true, "flow loop"); return; }
+        const bool dm0 = d.model == RTVLA_DM0;
         for (int t = 0; t < d.num_steps; ++t) {
-            suffix_step_begin(t);
-            for (int i = 0; i < d.llm_layers; ++i) suffix_layer(t, i);
-            suffix_step_end(t);
+            if (dm0) dm0_step_begin(t); else suffix_step_begin(t);
+            for (int i = 0; i < d.llm_layers; ++i) if (dm0) dm0_suffix_layer(t, i); else suffix_layer(t, i);
+            if (dm0) dm0_step_end(t); else suffix_step_end(t);
         }
     }
+
+    void forward() { front(); loop(); }
 
     // one-time device work.  With `tiles_loaded` the re-tiled weights (the first rtvla_tiled_bytes of the workspace) were
     // filled in by the caller from a copy saved after an earlier prepare, and only the rest is done.
@@ -1083,39 +1124,6 @@ int check_ready(rtvla_ctx* c, bool need_prepared) {
 int hip_fail(rtvla_ctx* c, hipError_t e, const char* what) {
     return c->fail(RTVLA_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }
-
-// The flow kernel needs every CU of the device to itself (csrc/flow.hip): two of them, started on two streams, could each hold half of
-// the CUs and wait for the other half.  Launches that contain one are therefore chained per device: each waits for the event recorded
-// behind the one before it, if that was on another stream.  A stream that is being captured is left alone (see FlowOff).
-constexpr int MAX_DEVICES = 64;
-struct FlowGate { std::mutex m; hipEvent_t done = nullptr; hipStream_t last = nullptr; bool used = false; };
-FlowGate flow_gates[MAX_DEVICES];
-
-bool capturing(hipStream_t s) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
-}
-
-struct FlowTurn {
-    FlowGate* g = nullptr;
-    hipStream_t s;
-    hipError_t err = hipSuccess;
-    FlowTurn(const rtvla_ctx* c, hipStream_t stream) : s(stream) {
-        int dev = 0;
-        if (!c->flow || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES || capturing(s)) return;
-        g = &flow_gates[dev];
-        g->m.lock();
-        if (!g->done) err = hipEventCreateWithFlags(&g->done, hipEventDisableTiming);
-        else if (g->used && (g->last != s || s == hipStreamPerThread)) err = hipStreamWaitEvent(s, g->done, 0);
-    }
-    ~FlowTurn() {
-        if (!g) return;
-        if (err == hipSuccess && hipEventRecord(g->done, s) == hipSuccess) { g->last = s; g->used = true; }
-        g->m.unlock();
-    }
-    FlowTurn(const FlowTurn&) = delete;
-    FlowTurn& operator=(const FlowTurn&) = delete;
-};
 
 // A caller's own graph of rtvla_forward may be replayed on any stream, where nothing chains it: it gets the loop as launches.
 struct FlowOff {
@@ -1251,8 +1259,6 @@ int rtvla_forward(rtvla_ctx* c, void* stream) {
     if (int rc = check_ready(c, true)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;
     FlowOff off(c, (hipStream_t)stream);
-    FlowTurn turn(c, (hipStream_t)stream);
-    if (turn.err != hipSuccess) return hip_fail(c, turn.err, "waiting for another stream's flow loop");
     Sched(c, (hipStream_t)stream).forward();
     return c->status;
 }
@@ -1273,8 +1279,6 @@ int rtvla_forward_stage(rtvla_ctx* c, int stage, int layer, int step, void* stre
     if (int rc = check_ready(c, true)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;
     FlowOff off(c, (hipStream_t)stream);
-    FlowTurn turn(c, (hipStream_t)stream);
-    if (turn.err != hipSuccess) return hip_fail(c, turn.err, "waiting for another stream's flow loop");
     int rc = Sched(c, (hipStream_t)stream).stage(stage, layer, step);
     if (rc) return c->fail(rc, "bad stage / layer / step");
     return c->status;
@@ -1285,15 +1289,18 @@ int rtvla_graph_capture(rtvla_ctx* c, void* stream) {
     hipStream_t s = (hipStream_t)stream;
     // one eager run first: sets per-kernel attributes outside the capture and surfaces launch errors
     if (int rc = rtvla_forward(c, stream)) return rc;
+    const int kernels = c->kernels;
     hipError_t e = hipStreamSynchronize(s);
     if (e != hipSuccess) return hip_fail(c, e, "eager forward before capture");
     drop_graph(c);
     e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(c, e, "hipStreamBeginCapture");
-    c->status = 0; c->launches = 0; c->kernels = 0;
-    Sched(c, s).forward();
+    // the resident flow loop stays outside: it waits for its turn, which a graph's place in the order of the streams is not known for
+    Sched sc(c, s);
+    if (c->flow) sc.front(); else sc.forward();
     e = hipStreamEndCapture(s, &c->graph);
     if (e != hipSuccess) return hip_fail(c, e, "hipStreamEndCapture");
+    c->kernels = kernels;
     if (c->status) return c->status;
     e = hipGraphInstantiate(&c->exec, c->graph, nullptr, nullptr, 0);
     if (e != hipSuccess) return hip_fail(c, e, "hipGraphInstantiate");
@@ -1303,17 +1310,19 @@ int rtvla_graph_capture(rtvla_ctx* c, void* stream) {
 int rtvla_graph_launch(rtvla_ctx* c, void* stream) {
     if (!c) return RTVLA_ERR_ARG;
     if (!c->exec || !c->prepared) return c->fail(RTVLA_ERR_STATE, "no graph captured since the last rtvla_bind / rtvla_prepare");
-    FlowTurn turn(c, (hipStream_t)stream);
-    if (turn.err != hipSuccess) return hip_fail(c, turn.err, "waiting for another stream's flow loop");
     hipError_t e = hipGraphLaunch(c->exec, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(c, e, "hipGraphLaunch");
-    return RTVLA_OK;
+    if (!c->flow) return RTVLA_OK;
+    const int kernels = c->kernels;
+    c->status = 0; c->launches = 0;
+    Sched(c, (hipStream_t)stream).loop();
+    c->kernels = kernels;
+    return c->status;
 }
 
 int rtvla_flow_limits(rtvla_ctx* c, float first_ms, float second_ms, float wait_ms) {
     if (!c || first_ms != first_ms || second_ms != second_ms || wait_ms != wait_ms) return RTVLA_ERR_ARG;
     set_flow_limits(c, first_ms, second_ms, wait_ms);
-    drop_graph(c);                               // (the captured launches carry the limits they were recorded with)
     return RTVLA_OK;
 }
 
@@ -1340,6 +1349,7 @@ static int time_replay(rtvla_ctx* c, hipStream_t s, int stage, int layer, int st
     FlowTurn turn(c, s);
     if (turn.err != hipSuccess) return hip_fail(c, turn.err, "waiting for another stream's flow loop");
     Sched sc(c, s);
+    sc.have_turn = true;
     const bool cycle = layer == -1;
     const int n_layers = !cycle ? 1 : (stage == RTVLA_STAGE_VISION_LAYER ? c->d.vision_layers :
                                        (stage == RTVLA_STAGE_PREFIX_LAYER || stage == RTVLA_STAGE_SUFFIX_LAYER) ? c->d.llm_layers : 1);

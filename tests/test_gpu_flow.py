@@ -3,6 +3,7 @@ same weights and noise at the suffix sizes where the kernel's row tiles end, and
 import os
 import subprocess
 import sys
+import threading
 
 import pytest
 import torch
@@ -102,6 +103,51 @@ def test_one_workgroup_gives_the_same_layer(model):
     for k in range(3, 9):
         assert torch.equal(results[k][0], results[k % 3][0]) and torch.equal(results[k][1], results[k % 3][1]), k
     assert e.ctx.flow_status() == (True, 6)
+
+
+def test_policies_on_two_streams_and_threads():
+    """The loops of one process take turns, whatever streams and threads they come from; each policy's actions are those it gives alone."""
+    pairs = [policy(*args) for args in (("pi0", 701, 2, 20, 50), ("dm0", 702, 1, 24, 50))]
+    want = [m.forward(*inputs).clone() for m, inputs in pairs]
+    torch.cuda.synchronize()
+    wrong, errors = [0, 0], []
+
+    def run(k):
+        m, inputs = pairs[k]
+        try:
+            for burst in range(10):                                          # (streams come and go: a new one may have the handle of an old one)
+                stream = torch.cuda.Stream()
+                with torch.cuda.stream(stream):
+                    for _ in range(10):
+                        wrong[k] += int(not torch.equal(m.forward(*inputs), want[k]))
+        except Exception as e:                                               # (an exception in a thread is nobody's otherwise)
+            errors.append(e)
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=100)
+    assert not errors and wrong == [0, 0]
+    assert [m._engine.ctx.flow_status() for m, _ in pairs] == [(True, 0)] * 2
+
+
+def test_only_the_flow_loops_take_turns():
+    """What comes before a loop does not wait for the loops of another stream."""
+    import rtvla_capi as capi
+    (a, a_in), (b, b_in) = policy("pi0", 703, 1, 5, 50), policy("pi0", 704, 1, 5, 50)
+    a.forward(*a_in)
+    b.forward(*b_in)
+    torch.cuda.synchronize()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(first):
+        for _ in range(200):
+            a._engine.replay()
+    with torch.cuda.stream(second):
+        b._engine.run_stage(capi.STAGE_VISION_LAYER, 0)
+    second.synchronize()
+    assert not first.query()                                                 # 200 forwards against one layer
+    first.synchronize()
 
 
 WORKER = """
