@@ -180,7 +180,13 @@ int rtvla_graph_launch(rtvla_ctx* ctx, void* hip_stream);
  * workgroup that does not answer.  If none of them finishes, one workgroup runs the whole loop by itself: the same actions bit for bit, in
  * about a second instead of 5 - 7 ms.  No forward is lost.  0: does not wait at all, negative: the default. */
 int rtvla_flow_limits(rtvla_ctx* ctx, float first_ms, float second_ms, float wait_ms);
-/* Read without waiting for anything: whether the flow loop is enqueued as the resident kernel (1) or as launches (0), and of the forwards
+/* The flow loop exists as launches too: a quarter longer (Pi0 5.8 ms instead of 4.7), but any number of compute units will do.  RTVLA_FLOW_AUTO takes them under a
+ * caller's own capture, on a stream whose CU mask leaves out part of the device, and for the forwards after one whose loop had to run in one
+ * workgroup (64 of them, more if that happens again).  RTVLA_FLOW_RESIDENT leaves out the last of these, RTVLA_FLOW_LAUNCHES takes nothing
+ * else.  The two differ by roundings of the bf16 stream.  Applies to what is enqueued from here on. */
+enum rtvla_flow_route { RTVLA_FLOW_AUTO = 0, RTVLA_FLOW_RESIDENT = 1, RTVLA_FLOW_LAUNCHES = 2 };
+int rtvla_set_flow_route(rtvla_ctx* ctx, int route);
+/* Read without waiting for anything: whether the last call enqueued its flow loop as the resident kernel (1) or as launches (0), and of the forwards
  * and stages that have ended so far, how many had the loop run in one workgroup (modulo 2^32).  Either pointer may be null. */
 int rtvla_flow_status(const rtvla_ctx* ctx, int32_t* resident, uint32_t* alone);
 

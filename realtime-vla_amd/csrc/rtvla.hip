@@ -76,13 +76,18 @@ struct rtvla_ctx {
     size_t act_begin = 0;          // activations start here (cleared at prepare)
     char* ws = nullptr;
     bool prepared = false;
-    bool flow = false;             // the flow loop runs as one resident kernel (csrc/flow.hip); false: as launches, see flow_supported()
+    bool flow_able = false;        // the device can run the flow loop as one resident kernel (csrc/flow.hip), see flow_supported()
+    bool flow = false;             // the call being enqueued does; false: as launches (choose_route)
+    int flow_route = RTVLA_FLOW_AUTO;
+    unsigned flow_alone_seen = 0;  // of *flow_alone
+    int flow_rest = 0, flow_rest_next = 64, flow_calm = 0;      // forwards still to run as launches; of the next rest; resident ones since the last
     FlowP flow_p{};                // its private-memory layout (build_tables)
     unsigned gate_limit[FLOW_ATTEMPTS] = {}, gate_step[FLOW_ATTEMPTS] = {};      // how long its launches wait (set_flow_limits)
     unsigned* flow_alone = nullptr;          // host word the flow kernel counts in: loops that ran in one workgroup (HostWords)
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    hipStream_t timing_stream = nullptr;     // the measurement helpers capture graphs, which the null stream cannot
+    hipGraph_t graph = nullptr, loop_graph = nullptr;      // what comes before the flow loop; the loop as launches (when first needed)
+    hipGraphExec_t exec = nullptr, loop_exec = nullptr;
+    int front_kernels = 0, loop_kernels = 0;
+    hipStream_t own_stream = nullptr;        // for captures whose caller is on the null stream, which cannot be captured, or knows nothing of them
     std::string err;
     int launches = 0;              // scheduler launches enqueued so far (index space of rtvla_time_launch)
     int kernels = 0;               // kernels behind them (the key-split attention is two)
@@ -505,7 +510,7 @@ int build_tables_dm0(rtvla_ctx* c) {
 // The flow kernel needs every CU of the device at the same moment (csrc/flow.hip): two of them, started on two streams, could each hold half of
 // the CUs and wait for the other half.  The launches of one loop are therefore enqueued behind the loop enqueued before it on this device,
 // whichever stream that was on; what comes before a loop is not held up.  The event is waited for on the same stream too: a stream is known
-// by its handle only, and a handle may be that of a stream that has gone.  A stream that is being captured is left alone (see FlowOff).
+// by its handle only, and a handle may be that of a stream that has gone.  A stream that is being captured is left alone (see choose_route).
 constexpr int MAX_DEVICES = 64;
 struct FlowGate { std::mutex m; hipEvent_t done = nullptr; bool used = false; };
 FlowGate flow_gates[MAX_DEVICES];
@@ -1125,17 +1130,71 @@ int hip_fail(rtvla_ctx* c, hipError_t e, const char* what) {
     return c->fail(RTVLA_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// A caller's own graph of rtvla_forward may be replayed on any stream, where nothing chains it: it gets the loop as launches.
-struct FlowOff {
-    rtvla_ctx* c; bool was;
-    FlowOff(rtvla_ctx* c_, hipStream_t s) : c(c_), was(c_->flow) { if (was && capturing(s)) c->flow = false; }
-    ~FlowOff() { c->flow = was; }
-};
+// Whether work on this stream may use every CU of the device.
+bool whole_device(hipStream_t s) {
+    uint32_t mask[8] = {};                       // 256 CUs
+    if (hipExtStreamGetCUMask(s, 8, mask) != hipSuccess) { (void)hipGetLastError(); return true; }      // (the kernel's gate finds out)
+    int n = 0;
+    for (uint32_t m : mask) n += __builtin_popcount(m);
+    return n == 256;
+}
+
+// How the flow loop of this call is enqueued.  As launches: under capture (a caller's own graph may be replayed on any stream, where nothing
+// chains it); on a stream that is kept from some of the CUs, where the resident kernel never could begin (asking
+// takes 0.4 us); and for a while after a loop had
+// to run in one workgroup, because whatever held the CUs may go on doing so and launches only get slower by that: 64 forwards, four times as
+// many after every further try that fails (at most 16 384, a try of 1.1 s in 180 s), 64 again after 1 024 that did not.
+void choose_route(rtvla_ctx* c, hipStream_t s, bool whole_forward) {
+    c->flow = false;
+    if (!c->flow_able || c->flow_route == RTVLA_FLOW_LAUNCHES || capturing(s) || !whole_device(s)) return;
+    if (!c->flow_alone) c->flow_alone = host_words.take();
+    if (c->flow_alone && c->flow_route == RTVLA_FLOW_AUTO) {
+        const unsigned alone = __atomic_load_n(c->flow_alone, __ATOMIC_RELAXED);
+        if (alone != c->flow_alone_seen) {
+            c->flow_alone_seen = alone;
+            c->flow_rest = c->flow_rest_next;
+            c->flow_rest_next = std::min(4 * c->flow_rest_next, 16384);
+            c->flow_calm = 0;
+        }
+        if (c->flow_rest > 0) { c->flow_rest -= whole_forward; return; }
+        if (whole_forward && ++c->flow_calm == 1024) { c->flow_rest_next = 64; c->flow_calm = 0; }
+    }
+    c->flow = true;
+}
 
 // A captured graph holds the addresses that were bound when it was recorded: any later binding makes it stale.
 void drop_graph(rtvla_ctx* c) {
-    if (c->exec) { hipGraphExecDestroy(c->exec); c->exec = nullptr; }
-    if (c->graph) { hipGraphDestroy(c->graph); c->graph = nullptr; }
+    for (hipGraphExec_t* e : {&c->exec, &c->loop_exec}) if (*e) { hipGraphExecDestroy(*e); *e = nullptr; }
+    for (hipGraph_t* g : {&c->graph, &c->loop_graph}) if (*g) { hipGraphDestroy(*g); *g = nullptr; }
+}
+
+// Records what `enqueue` puts on the stream into a graph.
+template <typename F> int record(rtvla_ctx* c, hipStream_t s, hipGraph_t* graph, hipGraphExec_t* exec, F enqueue) {
+    hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
+    if (e != hipSuccess) return hip_fail(c, e, "hipStreamBeginCapture");
+    c->status = 0; c->launches = 0; c->kernels = 0;
+    enqueue();
+    e = hipStreamEndCapture(s, graph);
+    if (e != hipSuccess) return hip_fail(c, e, "hipStreamEndCapture");
+    if (c->status) return c->status;
+    e = hipGraphInstantiate(exec, *graph, nullptr, nullptr, 0);
+    return e == hipSuccess ? 0 : hip_fail(c, e, "hipGraphInstantiate");
+}
+
+// The flow loop behind the front graph, on the route chosen for this call.
+int launch_loop(rtvla_ctx* c, hipStream_t s) {
+    c->status = 0; c->launches = 0; c->kernels = 0;
+    if (c->flow) { Sched(c, s).loop(); return c->status; }
+    hipError_t e = hipSuccess;
+    if (!c->loop_exec) {
+        if (!c->own_stream && (e = hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking)) != hipSuccess) return hip_fail(c, e, "stream for the capture");
+        if (c->loop_graph) { hipGraphDestroy(c->loop_graph); c->loop_graph = nullptr; }
+        if (int rc = record(c, c->own_stream, &c->loop_graph, &c->loop_exec, [&] { Sched(c, c->own_stream).loop(); })) return rc;
+        c->loop_kernels = c->kernels;
+    }
+    c->kernels = c->loop_kernels;
+    e = hipGraphLaunch(c->loop_exec, s);
+    return e == hipSuccess ? 0 : hip_fail(c, e, "hipGraphLaunch");
 }
 
 }  // namespace
@@ -1173,7 +1232,7 @@ int rtvla_create(const rtvla_dims* dims, rtvla_ctx** out) {
 int rtvla_destroy(rtvla_ctx* c) {
     if (!c) return RTVLA_ERR_ARG;
     drop_graph(c);
-    if (c->timing_stream) hipStreamDestroy(c->timing_stream);
+    if (c->own_stream) hipStreamDestroy(c->own_stream);
     host_words.give(c->flow_alone);
     delete c;
     return RTVLA_OK;
@@ -1240,8 +1299,7 @@ int rtvla_buffer_info(const rtvla_ctx* c, int index, const char** name, size_t* 
 static int prepare_impl(rtvla_ctx* c, void* stream, bool tiles_loaded) {
     if (int rc = check_ready(c, false)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;
-    if (!c->flow_alone && !capturing((hipStream_t)stream)) c->flow_alone = host_words.take();
-    c->flow = !capturing((hipStream_t)stream) && flow_supported((FlowSync*)c->B<float>("flow_sync"), (hipStream_t)stream);      // (it waits for its answer)
+    c->flow_able = !capturing((hipStream_t)stream) && flow_supported((FlowSync*)c->B<float>("flow_sync"), (hipStream_t)stream);      // (it waits for its answer)
     Sched(c, (hipStream_t)stream).prepare(tiles_loaded);
     if (c->status) return c->status;
     hipError_t e = hipGetLastError();
@@ -1258,7 +1316,7 @@ int rtvla_tile_layout_version(void) { return RTVLA_TILE_LAYOUT_VERSION; }
 int rtvla_forward(rtvla_ctx* c, void* stream) {
     if (int rc = check_ready(c, true)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;
-    FlowOff off(c, (hipStream_t)stream);
+    choose_route(c, (hipStream_t)stream, true);
     Sched(c, (hipStream_t)stream).forward();
     return c->status;
 }
@@ -1278,7 +1336,7 @@ int rtvla_stage_prompt(rtvla_ctx* c, const int64_t* ids_host, int n, void* strea
 int rtvla_forward_stage(rtvla_ctx* c, int stage, int layer, int step, void* stream) {
     if (int rc = check_ready(c, true)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;
-    FlowOff off(c, (hipStream_t)stream);
+    choose_route(c, (hipStream_t)stream, false);
     int rc = Sched(c, (hipStream_t)stream).stage(stage, layer, step);
     if (rc) return c->fail(rc, "bad stage / layer / step");
     return c->status;
@@ -1293,17 +1351,10 @@ int rtvla_graph_capture(rtvla_ctx* c, void* stream) {
     hipError_t e = hipStreamSynchronize(s);
     if (e != hipSuccess) return hip_fail(c, e, "eager forward before capture");
     drop_graph(c);
-    e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
-    if (e != hipSuccess) return hip_fail(c, e, "hipStreamBeginCapture");
-    // the resident flow loop stays outside: it waits for its turn, which a graph's place in the order of the streams is not known for
-    Sched sc(c, s);
-    if (c->flow) sc.front(); else sc.forward();
-    e = hipStreamEndCapture(s, &c->graph);
-    if (e != hipSuccess) return hip_fail(c, e, "hipStreamEndCapture");
+    // the flow loop stays outside: which route it takes is known when it is launched, and the resident kernel waits for its turn then
+    if (int rc = record(c, s, &c->graph, &c->exec, [&] { Sched(c, s).front(); })) return rc;
+    c->front_kernels = c->kernels;
     c->kernels = kernels;
-    if (c->status) return c->status;
-    e = hipGraphInstantiate(&c->exec, c->graph, nullptr, nullptr, 0);
-    if (e != hipSuccess) return hip_fail(c, e, "hipGraphInstantiate");
     return RTVLA_OK;
 }
 
@@ -1312,17 +1363,21 @@ int rtvla_graph_launch(rtvla_ctx* c, void* stream) {
     if (!c->exec || !c->prepared) return c->fail(RTVLA_ERR_STATE, "no graph captured since the last rtvla_bind / rtvla_prepare");
     hipError_t e = hipGraphLaunch(c->exec, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(c, e, "hipGraphLaunch");
-    if (!c->flow) return RTVLA_OK;
-    const int kernels = c->kernels;
-    c->status = 0; c->launches = 0;
-    Sched(c, (hipStream_t)stream).loop();
-    c->kernels = kernels;
-    return c->status;
+    choose_route(c, (hipStream_t)stream, true);
+    const int rc = launch_loop(c, (hipStream_t)stream);
+    c->kernels += c->front_kernels;
+    return rc;
 }
 
 int rtvla_flow_limits(rtvla_ctx* c, float first_ms, float second_ms, float wait_ms) {
     if (!c || first_ms != first_ms || second_ms != second_ms || wait_ms != wait_ms) return RTVLA_ERR_ARG;
     set_flow_limits(c, first_ms, second_ms, wait_ms);
+    return RTVLA_OK;
+}
+
+int rtvla_set_flow_route(rtvla_ctx* c, int route) {
+    if (!c || route < RTVLA_FLOW_AUTO || route > RTVLA_FLOW_LAUNCHES) return RTVLA_ERR_ARG;
+    c->flow_route = route;
     return RTVLA_OK;
 }
 
@@ -1342,10 +1397,11 @@ static int time_replay(rtvla_ctx* c, hipStream_t s, int stage, int layer, int st
     if (!s) {
         // the null stream cannot be captured: finish what it holds, then launch and time on a stream of the context's own
         hipError_t e0 = hipStreamSynchronize(nullptr);
-        if (e0 == hipSuccess && !c->timing_stream) e0 = hipStreamCreateWithFlags(&c->timing_stream, hipStreamNonBlocking);
+        if (e0 == hipSuccess && !c->own_stream) e0 = hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking);
         if (e0 != hipSuccess) return hip_fail(c, e0, "timing stream");
-        s = c->timing_stream;
+        s = c->own_stream;
     }
+    choose_route(c, s, false);
     FlowTurn turn(c, s);
     if (turn.err != hipSuccess) return hip_fail(c, turn.err, "waiting for another stream's flow loop");
     Sched sc(c, s);

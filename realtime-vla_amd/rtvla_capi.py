@@ -25,6 +25,7 @@ TILE_AUTO, TILE_SKINNY = -1, -2
 ACT_BIAS_GELU, ACT_GEGLU, ACT_SWIGLU = 1, 2, 3
 NORM_NONE, NORM_RMS, NORM_LAYER = 0, 1, 2
 ATTN_GEMMA_PREFIX, ATTN_GEMMA_SUFFIX, ATTN_GQA128_PREFIX, ATTN_GQA128_SUFFIX, ATTN_VIT64, ATTN_SIGLIP = range(6)
+FLOW_AUTO, FLOW_RESIDENT, FLOW_LAUNCHES = range(3)
 FRAME_U8_HWC, FRAME_F32_HWC, FRAME_F32_CHW, FRAME_U8_CHW = range(4)
 STATIC_SCRATCH_BYTES = 2160 * 224 * 3          # RTVLA_STATIC_SCRATCH_BYTES
 
@@ -63,6 +64,7 @@ SYMBOLS = {
     "rtvla_graph_capture": (ctypes.c_int, [_P, _P]),
     "rtvla_graph_launch": (ctypes.c_int, [_P, _P]),
     "rtvla_flow_limits": (ctypes.c_int, [_P, ctypes.c_float, ctypes.c_float, ctypes.c_float]),
+    "rtvla_set_flow_route": (ctypes.c_int, [_P, ctypes.c_int]),
     "rtvla_flow_status": (ctypes.c_int, [_P, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_uint32)]),
     "rtvla_launch_count": (ctypes.c_int, [_P]),
     "rtvla_time_stage": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P, ctypes.POINTER(ctypes.c_float)]),
@@ -197,8 +199,11 @@ class Context:
     def flow_limits(self, first_ms=-1.0, second_ms=-1.0, wait_ms=-1.0):
         self.check(self.lib.rtvla_flow_limits(self.handle, first_ms, second_ms, wait_ms))
 
+    def set_flow_route(self, route):
+        self.check(self.lib.rtvla_set_flow_route(self.handle, route))
+
     def flow_status(self):
-        """(the loop is the resident kernel, loops that ran in one workgroup)"""
+        """(the last loop was enqueued as the resident kernel, loops that ran in one workgroup)"""
         resident, alone = ctypes.c_int32(), ctypes.c_uint32()
         self.check(self.lib.rtvla_flow_status(self.handle, ctypes.byref(resident), ctypes.byref(alone)))
         return bool(resident.value), alone.value

@@ -71,6 +71,13 @@ def test_flow_limits_and_status_need_no_device(lib):
         with pytest.raises(capi.RtvlaError) as e:
             c.flow_limits(*bad)
         assert e.value.code == 1
+    for route in (capi.FLOW_RESIDENT, capi.FLOW_LAUNCHES, capi.FLOW_AUTO):
+        c.set_flow_route(route)
+    for route in (-1, 3):
+        with pytest.raises(capi.RtvlaError) as e:
+            c.set_flow_route(route)
+        assert e.value.code == 1
+    assert lib.rtvla_set_flow_route(None, 0) == 1
     assert lib.rtvla_flow_limits(None, 1, 1, 1) == 1 and lib.rtvla_flow_status(None, None, None) == 1
     assert lib.rtvla_flow_status(c.handle, None, None) == 0
 

@@ -1,5 +1,6 @@
 """The resident flow kernel (csrc/flow.hip) against the flow loop as launches, which a caller's own graph of rtvla_forward gets: the
 same weights and noise at the suffix sizes where the kernel's row tiles end, and beside a second process on the same GPU."""
+import ctypes
 import os
 import subprocess
 import sys
@@ -8,6 +9,7 @@ import threading
 import pytest
 import torch
 
+import rtvla_capi as capi
 import synthetic as syn
 
 pytestmark = pytest.mark.gpu
@@ -69,6 +71,7 @@ def test_one_workgroup_gives_the_same_actions(model, views, prompt, chunk, limit
     ctx = m._engine.ctx
     want = m.forward(*inputs).clone()
     before = ctx.flow_status()[1]
+    ctx.set_flow_route(capi.FLOW_RESIDENT)                                   # (else the second one would be launches)
     ctx.flow_limits(*limits)
     m._engine.capture()                                                      # (its eager forward is the first without patience)
     got = m.forward(*inputs).clone()
@@ -85,9 +88,9 @@ def test_one_workgroup_gives_the_same_actions(model, views, prompt, chunk, limit
 @pytest.mark.parametrize("model", ["pi0", "pi05", "dm0"])
 def test_one_workgroup_gives_the_same_layer(model):
     """The stages start from the caller's stream and noise; a loop that gave up half way has spoiled neither."""
-    import rtvla_capi as capi
     m, inputs = policy(model, 600, 1, 20, 40)
     e = m._engine
+    e.ctx.set_flow_route(capi.FLOW_RESIDENT)
     m.forward(*inputs)
     x, noise = e.buffers["decoder_x"], e.buffers["diffusion_noise"]
     x0, n0 = x.clone(), noise.clone()
@@ -103,6 +106,60 @@ def test_one_workgroup_gives_the_same_layer(model):
     for k in range(3, 9):
         assert torch.equal(results[k][0], results[k % 3][0]) and torch.equal(results[k][1], results[k % 3][1]), k
     assert e.ctx.flow_status() == (True, 6)
+
+
+@pytest.mark.parametrize("model", ["pi0", "pi05", "dm0"])
+def test_launches_after_a_loop_in_one_workgroup(model):
+    """Whatever held the CUs may go on doing so: the next 64 forwards take the launches, then the resident kernel is tried again."""
+    m, inputs = policy(model, 800, 1, 20, 50)
+    ctx = m._engine.ctx
+    want = m.forward(*inputs).clone()
+    ctx.flow_limits(0, 0)
+    assert torch.equal(m.forward(*inputs), want)                             # (alone; the host knows when it has ended)
+    torch.cuda.synchronize()
+    assert ctx.flow_status() == (True, 1)
+    ctx.flow_limits()
+    close = []
+    for _ in range(64):
+        out = m.forward(*inputs).float()
+        close.append((out - want.float()).abs().mean())
+        assert ctx.flow_status() == (False, 1)
+    assert torch.stack(close).max().item() <= 2e-2                           # (as in the comparison of the two routes above)
+    assert torch.equal(m.forward(*inputs), want) and ctx.flow_status() == (True, 1)
+    ctx.set_flow_route(capi.FLOW_LAUNCHES)
+    assert (m.forward(*inputs).float() - want.float()).abs().mean().item() <= 2e-2 and ctx.flow_status() == (False, 1)
+
+
+def hip_runtime():
+    """the HIP runtime of this process"""
+    for line in open("/proc/self/maps"):
+        if "libamdhip64.so" in line:
+            return ctypes.CDLL(line.split()[-1])
+    raise RuntimeError("no HIP runtime loaded")
+
+
+@pytest.mark.parametrize("model", ["pi0", "dm0"])
+def test_a_stream_that_may_not_use_every_compute_unit(model):
+    """The resident kernel could not begin there: eager forwards and graph launches take the launches, on that stream only."""
+    m, inputs = policy(model, 900, 1, 20, 50)
+    e = m._engine
+    want = m.forward(*inputs).clone()
+    torch.cuda.synchronize()
+    hip, handle = hip_runtime(), ctypes.c_void_p()
+    mask = (ctypes.c_uint32 * 8)(*[0x0fffffff] * 8)                          # 28 of every 32
+    assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(handle), 8, mask) == 0
+    masked = torch.cuda.ExternalStream(handle.value)
+    with torch.cuda.stream(masked):
+        for eager in (True, False, False):
+            e.buffers["diffusion_noise"].copy_(inputs[-1].reshape(e.buffers["diffusion_noise"].shape))
+            e.run_eager() if eager else e.replay()
+            got = e.buffers["diffusion_noise"].float().reshape(want.shape)
+            assert e.ctx.flow_status() == (False, 0)
+            assert (got - want.float()).abs().mean().item() <= 2e-2
+    masked.synchronize()
+    assert torch.equal(m.forward(*inputs), want) and e.ctx.flow_status() == (True, 0)
+    torch.cuda.synchronize()
+    assert hip.hipStreamDestroy(handle) == 0
 
 
 def test_policies_on_two_streams_and_threads():
@@ -134,7 +191,6 @@ def test_policies_on_two_streams_and_threads():
 
 def test_only_the_flow_loops_take_turns():
     """What comes before a loop does not wait for the loops of another stream."""
-    import rtvla_capi as capi
     (a, a_in), (b, b_in) = policy("pi0", 703, 1, 5, 50), policy("pi0", 704, 1, 5, 50)
     a.forward(*a_in)
     b.forward(*b_in)
