@@ -32,7 +32,6 @@
 #include "kernels.h"
 #include <algorithm>
 #include <atomic>
-#include <mutex>
 
 namespace {
 
@@ -1016,14 +1015,6 @@ __global__ __launch_bounds__(256) void flow_init_kernel(FlowSync* sync, uint4* p
     }
 }
 
-__global__ __launch_bounds__(FLOW_THREADS) void flow_check_kernel(FlowSync* sync) {
-    if (threadIdx.x != 0) return;
-    const int xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7;
-    int rank, gate;
-    flow_gate(sync, 0, xcc, 5000000u, &rank, &gate);                           // 50 ms
-    if (gate != GATE_OPEN) atomicOr(&sync->abort, 1u);
-}
-
 template <int MODEL, int RH>
 int launch_inst(const FlowP& p, hipStream_t s) {
     const size_t need = (size_t)FW * 4 * RH * 1024 + SQ_BYTES + 320 + (MODEL == FLOW_DM0 ? 2 * RH * 16 * ROPE_PITCH : 0);
@@ -1076,29 +1067,9 @@ int launch_flow(const FlowP& p, int model, hipStream_t s) {
     return 2;
 }
 
-// Whether the flow kernel's assumption holds here: 256 workgroups of its size are resident together, 32 on each of 8 XCDs (not so on
-// a partitioned device or under a CU mask).  Tried once per device with a kernel that does nothing else; every wait in it ends.
-bool flow_supported(FlowSync* sync, hipStream_t s) {
-    static std::atomic<int> known[64];                                         // 0: not tried, 1: yes, 2: no
-    static std::mutex trying;                                                  // two checks at once could close each other's gates
+// Whether the current device has the 256 CUs the flow kernel splits its work over (a partitioned one has fewer).  Whether this process and
+// stream may use them all, and whether they are free, the gate finds out at each launch.
+bool flow_supported() {
     int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
-    if (const int k = known[dev].load(std::memory_order_acquire)) return k == 1;
-    const std::lock_guard<std::mutex> lock(trying);
-    if (const int k = known[dev].load(std::memory_order_acquire)) return k == 1;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
-    bool ok = cus == 256;
-    if (ok) {
-        const size_t smem = 96 * 1024;
-        unsigned bad = 1;
-        ok = hipFuncSetAttribute((const void*)flow_check_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) == hipSuccess;
-        if (ok) {
-            launch_flow_init(sync, nullptr, 0, FlowStart{}, nullptr, nullptr, nullptr, nullptr, s);
-            hipLaunchKernelGGL(flow_check_kernel, dim3(256), dim3(FLOW_THREADS), smem, s, sync);
-            ok = hipGetLastError() == hipSuccess && hipMemcpyAsync(&bad, &sync->abort, sizeof bad, hipMemcpyDeviceToHost, s) == hipSuccess &&
-                 hipStreamSynchronize(s) == hipSuccess && bad == 0;
-        }
-    }
-    known[dev].store(ok ? 1 : 2, std::memory_order_release);
-    return ok;
+    return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus == 256;
 }

@@ -206,7 +206,7 @@ int flow_row_pairs(int rows);                  // the kernel's row-tile pairs (t
 size_t flow_layout(FlowP* p, int qtiles, int blocks, int hidden);
 void launch_flow_init(FlowSync* sync, float* part, unsigned part_bytes, const FlowStart& start, const bf16_t* state, const bf16_t* w, const bf16_t* b, bf16_t* out, hipStream_t s);
 int launch_flow(const FlowP& p, int model, hipStream_t s);
-bool flow_supported(FlowSync* sync, hipStream_t s);      // whether the current device can run it (tried once per device; synchronises then)
+bool flow_supported();                         // whether the current device can run it
 
 // Row-major q [tokens][kv_heads][group][hd], k / v [keys][kv_heads][hd] -> the kernels' layouts per K/V head b: Q fragment-tiled
 // [row = local token * group + head][hd_pad] at qt + b' * q_bstride, K fragment-tiled [key][hd_pad], V^T tiled [hd][keys_pad];

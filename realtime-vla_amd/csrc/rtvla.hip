@@ -76,7 +76,7 @@ struct rtvla_ctx {
     size_t act_begin = 0;          // activations start here (cleared at prepare)
     char* ws = nullptr;
     bool prepared = false;
-    bool flow_able = false;        // the device can run the flow loop as one resident kernel (csrc/flow.hip), see flow_supported()
+    bool flow_able = false;        // the device can run the flow loop as one resident kernel (csrc/flow.hip)
     bool flow = false;             // the call being enqueued does; false: as launches (choose_route)
     int flow_route = RTVLA_FLOW_AUTO;
     unsigned flow_alone_seen = 0;  // of *flow_alone
@@ -1299,7 +1299,8 @@ int rtvla_buffer_info(const rtvla_ctx* c, int index, const char** name, size_t* 
 static int prepare_impl(rtvla_ctx* c, void* stream, bool tiles_loaded) {
     if (int rc = check_ready(c, false)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;
-    c->flow_able = !capturing((hipStream_t)stream) && flow_supported((FlowSync*)c->B<float>("flow_sync"), (hipStream_t)stream);      // (it waits for its answer)
+    c->flow_able = flow_supported();
+    if (c->flow_able && !c->flow_alone && !capturing((hipStream_t)stream)) c->flow_alone = host_words.take();
     Sched(c, (hipStream_t)stream).prepare(tiles_loaded);
     if (c->status) return c->status;
     hipError_t e = hipGetLastError();

@@ -162,6 +162,28 @@ def test_a_stream_that_may_not_use_every_compute_unit(model):
     assert hip.hipStreamDestroy(handle) == 0
 
 
+def test_prepare_neither_waits_nor_judges_the_device_by_its_stream():
+    """rtvla_prepare is enqueued, and a device that is busy or a stream that is masked during it decides nothing about later forwards."""
+    m, inputs = policy("pi0", 910, 1, 20, 50)
+    e = m._engine
+    want = m.forward(*inputs).clone()
+    torch.cuda.synchronize()
+    hip, handle = hip_runtime(), ctypes.c_void_p()
+    mask = (ctypes.c_uint32 * 8)(*[0x0fffffff] * 8)
+    assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(handle), 8, mask) == 0
+    masked = torch.cuda.ExternalStream(handle.value)
+    with torch.cuda.stream(masked):
+        for _ in range(100):
+            e.replay()
+        e.ctx.prepare(masked.cuda_stream)
+        assert not masked.query()
+    masked.synchronize()
+    e.capture()
+    assert torch.equal(m.forward(*inputs), want) and e.ctx.flow_status() == (True, 0)
+    torch.cuda.synchronize()
+    assert hip.hipStreamDestroy(handle) == 0
+
+
 def test_policies_on_two_streams_and_threads():
     """The loops of one process take turns, whatever streams and threads they come from; each policy's actions are those it gives alone."""
     pairs = [policy(*args) for args in (("pi0", 701, 2, 20, 50), ("dm0", 702, 1, 24, 50))]
