@@ -640,6 +640,16 @@ void flow_kernel(FlowP kernel_args) {
                     const bool in = b0 + w + FW * i < KB;
                     const float f0 = in ? __builtin_amdgcn_exp2f(mo[i][0] - M) : 0.f, f1 = in ? __builtin_amdgcn_exp2f(mo[i][2] - M) : 0.f;
                     L += f0 * mo[i][1] + f1 * mo[i][3];
+                    if constexpr (ALONE) {
+                        // the cache's rows behind the prefix, where a launch that gave up may have left anything: their probabilities are
+                        // zero, but 0 x NaN is NaN (blocks past the last one hold the prefix's last one)
+                        if (const int kb = b0 + w + FW * i, key0 = min(kb, KBp - 1) * 32 + 4 * g; kb < KBp || !in)
+#pragma unroll
+                            for (int d = 0; d < NDT; ++d)
+#pragma unroll
+                                for (int j = 0; j < 8; ++j)
+                                    if (key0 + (j & 3) + 16 * (j >> 2) >= kernel_args.prefix) vf[i][d][j] = f2bf(0.f);
+                    }
 #pragma unroll
                     for (int d = 0; d < NDT; ++d) o[d] += f0 * mfma16k16(vf[i][d], pf[i], 0) + f1 * mfma16k16(vf[i][d], pf[i], 1);
                 }

@@ -222,6 +222,8 @@ void launch_prompt_stage(const bf16_t* emb, int vocab, const int* ids, const int
 void launch_store_ids(const int64_t* ids_host, int n, int* ids, int valid_len, int* valid_len_dst, hipStream_t s);
 void launch_im2col(const bf16_t* images, bf16_t* patches, int ldp, int views, hipStream_t s);
 void launch_copy_rows(const bf16_t* src, int lds, bf16_t* dst, int ldd, int rows, int cols, hipStream_t s);
+// zeroes the tile kt of each of `tiles` rows of V^T tiles (keys32 long) and, with valid_len, the rows [max(row0, *valid_len), row1) of x
+void launch_clear_unseen(bf16_t* vt, int tiles, int keys32, int kt, bf16_t* x, int ldx, int row0, int row1, const int* valid_len, hipStream_t s);
 void launch_fill_zero(void* p, size_t bytes, hipStream_t s);
 void launch_fill_bf16(bf16_t* p, size_t n, float v, hipStream_t s);
 void launch_fill_f32(float* p, size_t n, float v, hipStream_t s);

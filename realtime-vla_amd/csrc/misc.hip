@@ -176,6 +176,23 @@ RTVLA_DEVICE void small_linear_one(const SmallLinearJob& j, int idx) {
     if (j.out_tiled) j.out[ft_index(m + j.out_row0, n, j.ldo >> 5)] = f2bf(acc);
     else j.out[(size_t)m * j.ldo + n] = f2bf(acc);
 }
+// Rows that a forward reads and no forward writes before it: the last 32-key tile of every layer's V^T (the keys behind the prefix hold
+// what the last suffix left there) and, of a prompt shorter than its allocation, the prompt rows behind it (the residual stream is updated in
+// place).  Nobody sees these keys, but they are multiplied with their probability of zero, and once there is a NaN or an infinity among them
+// (one bad input is enough) every later forward would be NaN.  One launch of 2 - 3 us; masking V in the attention kernels instead costs
+// 1.2 us per prefix layer and 0.2 - 0.3 us per layer and step of the action expert.
+__global__ __launch_bounds__(256) void clear_unseen_kernel(uint4* vt, int tiles, int keys32, int kt, uint4* x, int x16, int row0, int row1, const int* valid_len) {
+    const int b = blockIdx.x, vb = (tiles + 3) / 4;
+    if (b < vb) {
+        const int tile = b * 4 + (threadIdx.x >> 6);
+        if (tile < tiles) vt[((size_t)tile * keys32 + kt) * 64 + (threadIdx.x & 63)] = uint4{0, 0, 0, 0};
+        return;
+    }
+    const int row = row0 + b - vb;
+    if (row >= row1 || row < *valid_len) return;
+    for (int i = threadIdx.x; i < x16; i += 256) x[(size_t)row * x16 + i] = uint4{0, 0, 0, 0};
+}
+
 // one launch for up to two independent tiny linears (the state-token and the action input projections of a flow step)
 __global__ void small_linear_kernel(SmallLinearJob a, SmallLinearJob b) {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
@@ -340,6 +357,11 @@ void launch_store_ids(const int64_t* ids_host, int n, int* ids, int valid_len, i
         hipLaunchKernelGGL(store_ids_kernel, dim3(1), dim3(STORE_IDS), 0, s, b, m, ids + at, valid_len, valid_len_dst);
         at += m;
     } while (at < n);
+}
+
+void launch_clear_unseen(bf16_t* vt, int tiles, int keys32, int kt, bf16_t* x, int ldx, int row0, int row1, const int* valid_len, hipStream_t s) {
+    const int blocks = (tiles + 3) / 4 + (valid_len ? row1 - row0 : 0);
+    if (blocks > 0) hipLaunchKernelGGL(clear_unseen_kernel, dim3(blocks), dim3(256), 0, s, (uint4*)vt, tiles, keys32, kt, (uint4*)x, ldx / 8, row0, row1, valid_len);
 }
 
 void launch_fill_zero(void* p, size_t bytes, hipStream_t s) {

@@ -622,8 +622,19 @@ struct Sched {
                NORM_LAYER, nw, nb, 1e-5f, last_split, "vision down reduce");
     }
 
+    // before the prefix layers fill the cache (misc.hip); tiles: of one d tile each, of all layers and K / V heads
+    void clear_unseen(bf16_t* vt, int tiles) {
+        const bool prompt = pi05 && d.prompt_len > 0;
+        if (!(c->S_e & 31) && !prompt) return;
+        if (c->want("clear unseen rows")) {
+            launch_clear_unseen(vt, c->S_e & 31 ? tiles : 0, c->keys_pad >> 5, c->S_e >> 5, prompt ? c->B("encoder_x") : nullptr, 2048, c->S_v, c->S_e, prompt ? valid_len() : nullptr, s);
+            c->note(0, "clear unseen rows");
+        }
+    }
+
     void project() {
         const int S_v = c->S_v, S_e = c->S_e;
+        clear_unseen(Vt(0), d.llm_layers * 16);
         GemmP e{}; e.out = c->B("encoder_x"); e.ldo = 2048; e.bias = c->W("encoder_multi_modal_projector_b");
         gemm(c->B("vision_x_norm"), 1152, S_v, S_v, c->TW("t_encoder_multi_modal_projector_w"), nullptr, 1152, 2048, EPI_BIAS, e, "projector");
         if (pi05 && d.prompt_len > 0 && c->T("embedding_weight").bound && c->T("prompt_token_ids").bound && c->T("rope_table").bound) {
@@ -846,6 +857,7 @@ struct Sched {
     // factor of the first prefix layer
     void dm0_project() {
         const int n = d.num_views, P = c->S_e, T = n * DM0_TOK;
+        clear_unseen(dVt(0), d.llm_layers * 8 * 8);
         if (c->want("im2col ds1")) { launch_dm0_im2col3x3(c->B("vision_x_2d"), DM0_SEQ_PAD, 1, 52, 52, 1024, c->B("vision_col1"), n, s); c->note(0, "im2col ds1"); }
         GemmP e{}; e.out = c->B("vision_mm1"); e.ldo = 2048; e.bias = c->W("vision_ds1_b");
         gemm(c->B("vision_col1"), 9216, n * 676, n * 676, c->TW("t_vision_ds1_w"), nullptr, 9216, 2048, EPI_BIAS, e, "ds1");

@@ -108,6 +108,20 @@ def test_one_workgroup_gives_the_same_layer(model):
     assert e.ctx.flow_status() == (True, 6)
 
 
+# prefixes that end inside a 32-key block: its rows behind the prefix hold what the last forward's suffix left there
+@pytest.mark.parametrize("route", [capi.FLOW_RESIDENT, capi.FLOW_LAUNCHES], ids=["resident", "launches"])
+@pytest.mark.parametrize("model,views,prompt,chunk", [("pi0", 1, 20, 50), ("pi05", 1, 9, 33), ("dm0", 1, 24, 50), ("pi0", 1, 31, 9)])
+@pytest.mark.parametrize("bad,which", [(float("nan"), -1), (float("inf"), -1), (float("nan"), 0)], ids=["nan noise", "inf noise", "nan images"])
+def test_a_forward_on_bad_inputs_leaves_nothing_behind(model, views, prompt, chunk, route, bad, which):
+    m, inputs = policy(model, 850, views, prompt, chunk)
+    m._engine.ctx.set_flow_route(route)
+    want = m.forward(*inputs).clone()
+    spoiled = list(inputs)
+    spoiled[which] = torch.full_like(inputs[which], bad)
+    assert not torch.isfinite(m.forward(*spoiled).float()).any()
+    assert torch.equal(m.forward(*inputs), want) and torch.isfinite(want.float()).all()
+
+
 @pytest.mark.parametrize("model", ["pi0", "pi05", "dm0"])
 def test_launches_after_a_loop_in_one_workgroup(model):
     """Whatever held the CUs may go on doing so: the next 64 forwards take the launches, then the resident kernel is tried again."""
