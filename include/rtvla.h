@@ -130,7 +130,10 @@ int rtvla_bind_workspace(rtvla_ctx* ctx, void* device_ptr, size_t bytes);
 /* Location of a named internal activation inside the workspace, for taps and for the
  * `buffers` views of the Python object: byte offset, rows, cols, leading dimension (elements),
  * element size.  Names follow the reference's buffer keys where one exists (vision_x, encoder_x,
- * encoder_K, decoder_x, ...); encoder_Vt is the transposed V cache. */
+ * encoder_K, decoder_x, ...); encoder_Vt is the transposed V cache.  After a forward decoder_x_buf (Pi0, DM0), decoder_q_buf (Pi0, Pi05),
+ * decoder_attn and decoder_hidden hold those of the last layer and flow step on either route of the flow loop, and encoder_K / encoder_Vt the
+ * suffix rows behind the prefix.  Working memory, with whatever the route that ran left there: attn_partial, decoder_qkv, decoder_Q, flow_* and the
+ * rows behind the prefix in DM0's kv_K / kv_Vt (writing them in the resident kernel took 0.5 us per layer and step). */
 int rtvla_buffer_count(const rtvla_ctx* ctx);
 int rtvla_buffer_info(const rtvla_ctx* ctx, int index, const char** name, size_t* offset,
                       int64_t* rows, int64_t* cols, int64_t* ld, int32_t* elem_bytes);

@@ -9,6 +9,8 @@ import rtvla_capi as capi
 from tile_cache import TileCache, UNTILED_WEIGHTS, fingerprint
 
 _DTYPES = {2: torch.bfloat16, 4: torch.int32}
+# working memory of one route of the flow loop: which forwards write it, and what it holds afterwards, is the library's business
+_SCRATCH = ("attn_partial", "decoder_qkv", "decoder_Q", "flow_priv", "flow_part", "flow_sync", "flow_state_x", "flow_noise", "flow_x")
 _ANY_ROWS = ("vision_embed_tokens_w",)          # tables whose row count is whatever the checkpoint holds
 
 
@@ -68,7 +70,7 @@ class Engine:
         self.ctx.bind_workspace(self.workspace.data_ptr(), nbytes)
         # views of the library's internal activations, under the reference's buffer names where one exists
         for name, off, rows, cols, ld, elem in self.ctx.buffers():
-            if name.startswith("t_"):
+            if name.startswith("t_") or name in _SCRATCH:
                 continue
             flat = self.workspace[off:off + rows * ld * elem].view(torch.bfloat16 if elem == 2 else torch.float32)
             self.buffers.setdefault(name, flat.view(rows, ld)[:, :cols])
@@ -108,7 +110,8 @@ class Engine:
         (/root/reference/pi0_infer.py:1291-1317, pi05_infer.py:690-730): the MFMA kernels hold these tensors fragment-tiled,
         so `buffers[name]` has other bytes than the reference's tensor of that name.  Pi0 / Pi05 names: encoder_K, encoder_V
         ([layers][prefix + suffix rows][256]), encoder_Q ([prefix rows * 8][256]), vision_QKV ([views][256][3 * 1152]),
-        decoder_x, decoder_x_buf, decoder_q_buf, decoder_hidden.  Row-major buffers are returned as they are."""
+        decoder_x, decoder_x_buf (Pi0), decoder_q_buf, decoder_attn, decoder_hidden (of the last layer and flow step).  Row-major buffers
+        are returned as they are."""
         B, L = self.buffers, self.llm_layers
         if self.model == capi.DM0:
             raise KeyError("reference_buffer covers the Pi0 / Pi05 buffers")
@@ -118,10 +121,9 @@ class Engine:
         if name == "encoder_V":
             kp = B["encoder_Vt"].numel() // (L * 256)
             return torch.stack([untile_vt(B["encoder_Vt"].reshape(L, -1)[i], 256, kp).t() for i in range(L)])[:, : self.prefix_rows + self.suffix_rows].contiguous()
-        if name in ("encoder_Q", "decoder_q_buf", "decoder_x", "decoder_x_buf", "decoder_hidden"):
+        if name in ("encoder_Q", "decoder_q_buf", "decoder_x", "decoder_x_buf", "decoder_attn", "decoder_hidden"):
             t = B[name]
-            rows = {"encoder_Q": 8 * self.prefix_rows, "decoder_q_buf": 8 * self.suffix_rows, "decoder_x": self.suffix_rows,
-                    "decoder_x_buf": self.suffix_rows, "decoder_hidden": self.suffix_rows}[name]
+            rows = {"encoder_Q": 8 * self.prefix_rows, "decoder_q_buf": 8 * self.suffix_rows}.get(name, self.suffix_rows)
             cols = t.shape[1]
             return untile_ft(t, t.numel() // cols, cols)[:rows]
         if name == "vision_QKV":

@@ -137,7 +137,8 @@ template <> struct Cfg<FLOW_DM0> {
     static constexpr int HD = 128, HEADS = 2, AT = 2, ET = 1, EGRP = 12, FK = 1, FWAVES = 6, HID = 192, WD_K32 = 64;
 };
 
-// ALONE: the last launch, one workgroup of the compute waves only
+// ALONE: the last launch, of compute waves only: if the program has not run, one workgroup runs it; then the activations of the last layer
+// and step, which a user's program may look at, go from the XCDs' memory to where the loop as launches leaves them.
 template <int MODEL, int RH, bool ALONE>
 __global__ __launch_bounds__(ALONE ? FW * 64 : FLOW_THREADS)
 void flow_kernel(FlowP kernel_args) {
@@ -170,17 +171,21 @@ void flow_kernel(FlowP kernel_args) {
     const int w_ = __builtin_amdgcn_readfirstlane(tid >> 6);
     // the XCD this workgroup runs on and its number among the XCD's workgroups (ALONE: both are walked through below)
     if constexpr (ALONE) {
-        if (tid == 0) sh[2] = flow_ran(kernel_args.sync) ? GATE_DONE : GATE_OPEN;
+        if (tid == 0) sh[2] = flow_ran(kernel_args.sync) ? GATE_DONE : blockIdx.x == 0 ? GATE_OPEN : GATE_CLOSED;
     } else if (tid == 0) {
         const int xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7;         // HW_REG_XCC_ID
         sh[0] = xcc;
         flow_gate(kernel_args.sync, kernel_args.attempt, xcc, kernel_args.gate_ticks, &sh[1], &sh[2]);
     }
-    if constexpr (DM0)
-        for (int i = tid; i < RTP * 16 * 16; i += ALONE ? FW * 64 : FLOW_THREADS)
-            *(uint4*)(rope_lds + (i >> 4) * ROPE_PITCH + (i & 15) * 16) = *(const uint4*)(kernel_args.rope + (size_t)min(i >> 4, kernel_args.rows - 1) * 128 + (i & 15) * 8);
+    auto load_rope = [&]() __attribute__((always_inline)) {
+        if constexpr (DM0)
+            for (int i = tid; i < RTP * 16 * 16; i += ALONE ? FW * 64 : FLOW_THREADS)
+                *(uint4*)(rope_lds + (i >> 4) * ROPE_PITCH + (i & 15) * 16) = *(const uint4*)(kernel_args.rope + (size_t)min(i >> 4, kernel_args.rows - 1) * 128 + (i & 15) * 8);
+    };
+    if constexpr (!ALONE) load_rope();                                         // (while others arrive)
     __syncthreads();
-    if (__builtin_amdgcn_readfirstlane(sh[2]) != GATE_OPEN) return;
+    const int gate = __builtin_amdgcn_readfirstlane(sh[2]);
+    if (gate != GATE_OPEN && !(ALONE && gate == GATE_DONE)) return;
     int x_ = ALONE ? 0 : __builtin_amdgcn_readfirstlane(sh[0]), r_ = ALONE ? 0 : __builtin_amdgcn_readfirstlane(sh[1]);
     const int step0 = kernel_args.step0, step1 = kernel_args.step1, layer0 = kernel_args.layer0, layer1 = kernel_args.layer1;
     const bool begin = kernel_args.begin != 0, end = kernel_args.end != 0;
@@ -902,6 +907,28 @@ void flow_kernel(FlowP kernel_args) {
                 }
             }
         };
+        // pieces of 8 columns of a row; XCD x holds query head x (DM0: heads 2 x, 2 x + 1), their output, and its share of the hidden columns
+        auto publish = [&](int i0, int n) __attribute__((always_inline)) {
+            cFlowP& p = prm();
+            if (layer0 < layer1) {
+                for (int i = i0; i < rows * 256; i += n) {
+                    const int c = (i & 31) * 8, y = (i >> 5) & 7, row = i >> 8;
+                    const char* src = p.priv + (size_t)y * p.priv_stride;
+                    *(bf16x8*)(p.out_attn + ft_index(row, y * 256 + c, 64)) = *(const bf16x8*)(src + p.off_o + ft_off(row, c, 8));
+                    if (!DM0) *(bf16x8*)(p.out_q + ft_index(row * 8 + y, c, 8)) = *(const bf16x8*)(src + p.off_q + ft_off(row, c, 8));
+                }
+                for (int i = i0; i < rows * C::HID; i += n) {
+                    const int c = i % (C::HID / 8) * 8, y = i / (C::HID / 8) % 8, row = i / C::HID;
+                    *(bf16x8*)(p.out_hidden + ft_index(row, y * C::HID + c, p.hidden_cols32)) = *(const bf16x8*)(p.priv + (size_t)y * p.priv_stride + p.off_h + ft_off(row, c, HID32));
+                }
+            }
+            if (begin && !PI05)
+                for (int i = i0; i < (rows - s0) * 128; i += n)
+                    *(bf16x8*)(p.out_xin + ft_index(i >> 7, (i & 127) * 8, 32)) = *(const bf16x8*)(p.priv + p.off_xin + ft_off((i >> 7) + s0, (i & 127) * 8, 32));
+        };
+        if (gate == GATE_DONE) { publish(blockIdx.x * (FW * 64) + tid, gridDim.x * (FW * 64)); return; }
+        load_rope();
+        __syncthreads();
         f32x4 own[SK];                                                         // (read back from memory like those of the others)
         if (!begin) each([&]() __attribute__((always_inline)) { copy_x(true); });
         for (int t = step0; t < step1; ++t) {
@@ -935,6 +962,7 @@ void flow_kernel(FlowP kernel_args) {
             }
             if (end) each([&]() __attribute__((always_inline)) { euler(prm(), t); });
         }
+        publish(tid, FW * 64);
         if (tid == 0 && kernel_args.alone) __hip_atomic_store(kernel_args.alone, __hip_atomic_load(kernel_args.alone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         return;
     }
@@ -1040,7 +1068,7 @@ int launch_inst(const FlowP& p, hipStream_t s) {
         hipLaunchKernelGGL(kern, dim3(256), dim3(FLOW_THREADS), smem, s, q);
         if (hipGetLastError() != hipSuccess) return 5;
     }
-    hipLaunchKernelGGL(alone, dim3(1), dim3(FW * 64), need, s, q);
+    hipLaunchKernelGGL(alone, dim3(64), dim3(FW * 64), need, s, q);
     return hipGetLastError() == hipSuccess ? 0 : 5;
 }
 

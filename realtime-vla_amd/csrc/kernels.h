@@ -195,6 +195,9 @@ struct FlowP {
     bf16_t *kcache, *vcache; size_t kv_stride; int ldvt;
     const bf16_t* noise; bf16_t* noise_out;    // [chunk][32]
     const bf16_t* x_in; bf16_t* x;             // residual stream, fragment-tiled: where programs without `begin` start, where all end
+    // where the activations of the last layer and step go for those who look at them, fragment-tiled as the loop as launches leaves them (or
+    // null): rotated queries [8 rows][256] (not DM0), attention output [rows][2048], hidden [rows][hidden_cols32 * 32], input MLP's input [rows][1024]
+    bf16_t *out_q, *out_attn, *out_hidden, *out_xin; int hidden_cols32;
     char* priv; size_t priv_stride;            // memory of one XCD's own, 8 of them
     int off_x, off_xin, off_q, off_k, off_v, off_o, off_h, off_n, off_f, off_m, off_p;
     float* part; unsigned part_bytes;          // fp32 partial sums exchanged between the XCDs

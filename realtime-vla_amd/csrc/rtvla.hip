@@ -716,6 +716,9 @@ struct Sched {
         }
         p.noise = c->B("flow_noise"); p.noise_out = c->W("diffusion_noise"); p.x_in = c->B("flow_x"); p.x = c->B("decoder_x");
         p.alone = c->flow_alone;
+        p.out_q = dm0 ? nullptr : c->B("decoder_q_buf"); p.out_attn = c->B("decoder_attn");
+        p.out_hidden = c->B("decoder_hidden"); p.hidden_cols32 = (int)c->BI("decoder_hidden").cols / 32;
+        p.out_xin = pi05 ? nullptr : c->B("decoder_x_buf");
         const FlowStart start{(const uint4*)p.noise_out, (const uint4*)p.x, (uint4*)c->B("flow_noise"), (uint4*)c->B("flow_x"), d.chunk_size * 4,
                               begin ? 0 : flow_row_pairs(c->S_d) * 32 * 1024 / 8};
         p.priv = (char*)c->B<float>("flow_priv"); p.part = c->B<float>("flow_part"); p.sync = (FlowSync*)c->B<float>("flow_sync");

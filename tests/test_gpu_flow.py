@@ -11,6 +11,7 @@ import torch
 
 import rtvla_capi as capi
 import synthetic as syn
+from _engine import tile_ft, tile_vt, untile_ft, untile_vt
 
 pytestmark = pytest.mark.gpu
 
@@ -142,6 +143,56 @@ def test_launches_after_a_loop_in_one_workgroup(model):
     assert torch.equal(m.forward(*inputs), want) and ctx.flow_status() == (True, 1)
     ctx.set_flow_route(capi.FLOW_LAUNCHES)
     assert (m.forward(*inputs).float() - want.float()).abs().mean().item() <= 2e-2 and ctx.flow_status() == (False, 1)
+
+
+@pytest.mark.parametrize("model,views,prompt,chunk", [("pi0", 1, 20, 50), ("pi0", 1, 3, 31), ("pi0", 2, 8, 127), ("pi05", 1, 32, 33), ("pi05", 1, 9, 128),
+                                                      ("dm0", 1, 24, 50), ("dm0", 1, 23, 50)])
+@pytest.mark.parametrize("limits", [(-1, -1), (0, 0)], ids=["resident", "one workgroup"])
+def test_the_activations_are_left_where_the_launches_leave_them(model, views, prompt, chunk, limits):
+    """One input projection and one layer from the same stream and noise by either route: what `buffers` and `reference_buffer` show of them."""
+    m, inputs = policy(model, 950, views, prompt, chunk)
+    e = m._engine
+    m.forward(*inputs)
+    names = ["decoder_attn", "decoder_hidden"] + (["decoder_x_buf"] if model != "pi05" else []) + (["decoder_q_buf"] if model != "dm0" else [])
+    caches = ["encoder_K", "encoder_Vt"] if model != "dm0" else []           # (behind the prefix DM0's are working memory)
+    keep = {n: e.buffers[n].clone() for n in ["decoder_x", "diffusion_noise"] + caches}
+    e.ctx.flow_limits(*limits)
+    seen = {}
+    for route in (capi.FLOW_RESIDENT, capi.FLOW_LAUNCHES):
+        e.ctx.set_flow_route(route)
+        for n in names:
+            e.buffers[n].zero_()
+        for n, t in keep.items():
+            e.buffers[n].copy_(t)
+        for c in caches:                                                     # rows behind the prefix: gone
+            for part in e.buffers[c].view(2, -1):
+                if c == "encoder_K":
+                    cleared = untile_ft(part, part.numel() // 256, 256)
+                    cleared[e.prefix_rows:] = 0
+                    part.copy_(tile_ft(cleared))
+                else:
+                    cleared = untile_vt(part, 256, part.numel() // 256)
+                    cleared[:, e.prefix_rows:] = 0
+                    part.copy_(tile_vt(cleared))
+        e.run_stage(capi.STAGE_SUFFIX_STEP_BEGIN, 0, 4)
+        e.buffers["decoder_x"].copy_(keep["decoder_x"])
+        e.run_stage(capi.STAGE_SUFFIX_LAYER, 1, 4)
+        torch.cuda.synchronize()
+        assert e.ctx.flow_status()[0] == (route == capi.FLOW_RESIDENT)
+        seen[route] = {n: e.buffers[n].float().clone() for n in names + caches}
+        if model != "dm0":
+            seen[route].update({"untiled " + n: e.reference_buffer(n).float().clone() for n in names + ["encoder_K", "encoder_V"]})
+    for n, want in seen[capi.FLOW_LAUNCHES].items():
+        got = seen[capi.FLOW_RESIDENT][n]
+        if "encoder_" not in n:
+            assert want.norm() > 0
+            rows = {"decoder_q_buf": 8}.get(n.split()[-1], 1) * (chunk + (model == "pi0") - (model == "pi0" and "x_buf" in n))
+            if not n.startswith("untiled"):                                  # (rows past the suffix are the kernels' padding)
+                got, want = (untile_ft(t, t.numel() // t.shape[1], t.shape[1])[:rows] for t in (got, want))
+            else:
+                got, want = got[:rows], want[:rows]
+        # sums of up to 4 096 products in another order, each stage rounded to bf16 (2^-9) as often as on the other route: a few roundings that fall to the other side
+        assert ((got - want).norm() / want.norm()).item() < 5e-3, n
 
 
 def hip_runtime():
