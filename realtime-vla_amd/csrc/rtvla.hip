@@ -1638,12 +1638,12 @@ struct ActPlan { size_t a_off, w0_off, w1_off, bias_off, scale_off, total; int K
 
 int plan_linear_act(int M, int K, int N, int act, int tile, ActPlan* out) {
     if (M <= 0 || K <= 0 || N <= 0 || (K & 7) || (N & 15)) return RTVLA_ERR_ARG;
-    if (act != RTVLA_ACT_BIAS_GELU && act != RTVLA_ACT_GEGLU && act != RTVLA_ACT_SWIGLU) return RTVLA_ERR_ARG;
+    if (act < RTVLA_ACT_BIAS_GELU || act > RTVLA_ACT_RESIDUAL) return RTVLA_ERR_ARG;
     if (tile < -1 || tile >= (int)TILE_COUNT) return RTVLA_ERR_ARG;
     ActPlan p{};
-    p.dual = act != RTVLA_ACT_BIAS_GELU;
+    p.dual = act == RTVLA_ACT_GEGLU || act == RTVLA_ACT_SWIGLU;
     p.K128 = k32_padded(K) * 32;
-    p.tile = tile >= 0 ? tile : choose_tile(M, n16_tiles(N), k32_padded(K) / 2, p.dual, false, "linear act", !p.dual).tile;
+    p.tile = tile >= 0 ? tile : choose_tile(M, n16_tiles(N), k32_padded(K) / 2, p.dual, false, "linear act", act == RTVLA_ACT_BIAS_GELU).tile;
     if (p.dual && (gemm_tile_bn(p.tile) != 256 || gemm_tile_eight_waves(p.tile))) return RTVLA_ERR_LIMIT;      // gate and up share a 256-column workgroup tile
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const int G = p.dual ? 4 : 8;
@@ -1685,6 +1685,7 @@ int rtvla_linear_act(const void* x, int M, int K, const void* w, const void* w_u
     p.bgroup = G; p.N16 = n16_tiles(N); p.K32p = k32_padded(K); p.nsplit = 1;
     p.out = (bf16_t*)out; p.ldo = N; p.bias = bias ? (const bf16_t*)bias : zbias;
     int epi = EPI_BIAS_GELU;
+    if (act == RTVLA_ACT_RESIDUAL) { epi = EPI_RESIDUAL; p.res = p.out; p.ldr = N; }
     if (act == RTVLA_ACT_GEGLU) epi = EPI_GEGLU;
     if (act == RTVLA_ACT_SWIGLU) {
         epi = EPI_SWIGLU;

@@ -188,6 +188,15 @@ def test_dm0_two_images_odd_prompt():
     check_case(Case(62, 2, 37, 1, 2), "dm0_2img")
 
 
+@pytest.mark.parametrize("images,lang", [(1, 6), (2, 37)])
+def test_dm0_flow_loop_as_launches(images, lang):
+    """The route of a caller's own graph and of a stream that may not use the whole device: the same checks, layer by layer."""
+    case = Case(64, images, lang, 1, 2)
+    case.e.ctx.set_flow_route(case.capi.FLOW_LAUNCHES)
+    check_case(case, "dm0 launches")
+    assert not case.e.ctx.flow_status()[0]
+
+
 def test_dm0_full_size_three_images():
     """The reference benchmark's shape: 3 images, 100 language tokens, 23 + 28 + 28 layers (benchmark.py:61-62)."""
     case = Case(1234, 3, 100, 23, 28, vocab=4096, fp32_taps=False)

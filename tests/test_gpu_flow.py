@@ -86,6 +86,17 @@ def test_one_workgroup_gives_the_same_actions(model, views, prompt, chunk, limit
     assert torch.equal(again, want) and ctx.flow_status() == (True, before + 2)
 
 
+@pytest.mark.parametrize("model,views,prompt,chunk", SHAPES)
+def test_the_second_launch_runs_where_the_first_gave_way(model, views, prompt, chunk):
+    m, inputs = policy(model, 550 + chunk, views, prompt, chunk)
+    want = m.forward(*inputs).clone()
+    m._engine.ctx.flow_limits(0)
+    for _ in range(3):
+        assert torch.equal(m.forward(*inputs), want)
+    torch.cuda.synchronize()
+    assert torch.isfinite(want.float()).all() and m._engine.ctx.flow_status() == (True, 0)
+
+
 @pytest.mark.parametrize("model", ["pi0", "pi05", "dm0"])
 def test_one_workgroup_gives_the_same_layer(model):
     """The stages start from the caller's stream and noise; a loop that gave up half way has spoiled neither."""

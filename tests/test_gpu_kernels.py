@@ -188,6 +188,54 @@ def test_fused_activation_epilogues_against_fp32(M, K, N, act):
     assert ran >= 3
 
 
+# the eight-wave tiles deal the row tiles over more blocks than the least number where the last round of workgroups has room for them (56 row
+# tiles: 8, 9 and 11 blocks instead of 7, 8 and 10 at 256 .. 272 columns); at 9 216 columns it has none
+@pytest.mark.parametrize("M,K,N", [(1777, 264, 272), (1792, 136, 256), (1761, 136, 9216), (2720, 136, 3072)])
+def test_eight_wave_tiles_with_more_row_blocks_than_the_least(M, K, N):
+    import rtvla_capi as capi
+    lib = capi.load()
+    ran = 0
+    for tile, rows, cols in _tiles(lib)[7:11]:
+        assert rows in (256, 224, 192, 128) and cols == 256
+        res = _run(lib, capi, M, K, N, tile, 1)
+        if res is None:
+            continue
+        ran += 1
+        assert res[0] <= REL_TOL and res[1] <= 1.01, ("tile %dx%d" % (rows, cols), res)
+    assert ran >= 3
+
+
+# every tile that takes the epilogue, at whole and ragged tiles; the stream is read and written in place, rows behind it stay as they are
+@pytest.mark.parametrize("M,K,N", [(2720, 1024, 1024), (2720, 4096, 1024), (224, 128, 256), (225, 264, 272), (37, 136, 48), (1, 64, 16), (97, 192, 144)])
+def test_residual_epilogue_in_place_against_fp32(M, K, N):
+    import rtvla_capi as capi
+    lib = capi.load()
+    g = torch.Generator(device="cuda:0").manual_seed(M + K + N)
+    x = torch.randn(M, K, device="cuda:0", generator=g).to(torch.bfloat16)
+    w = (torch.randn(K, N, device="cuda:0", generator=g) * 0.05).to(torch.bfloat16)
+    b = torch.randn(N, device="cuda:0", generator=g).to(torch.bfloat16)
+    stream = (torch.randn(M + 1, N, device="cuda:0", generator=g) * 3).to(torch.bfloat16)
+    ref = x.float() @ w.float() + b.float() + stream[:M].float()
+    ran = 0
+    for tile, rows, cols in [(capi.TILE_AUTO, 0, 0)] + _tiles(lib):
+        need = lib.rtvla_linear_act_workspace_bytes(M, K, N, capi.ACT_RESIDUAL, tile)
+        ws = torch.empty(need, dtype=torch.uint8, device="cuda:0")
+        out = stream.clone()
+        rc = lib.rtvla_linear_act(_P(x.data_ptr()), M, K, _P(w.data_ptr()), None, N, _P(b.data_ptr()), capi.ACT_RESIDUAL, _P(out.data_ptr()),
+                                  _P(ws.data_ptr()), need, tile, _P(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        if rc == capi.ERR_LIMIT:
+            continue                                        # the eight-wave tiles, and the large ones at an odd number of stages
+        assert rc == 0
+        ran += 1
+        got = out[:M].float()
+        excess = (got - ref).abs() / (ref.abs() * 2.0 ** -7 + 1e-3 * ref.pow(2).mean().sqrt())
+        assert ((got - ref).norm() / ref.norm()).item() <= REL_TOL and excess.max().item() <= 1.01, (tile, rows, cols)
+        assert torch.equal(out[M], stream[M])
+    assert ran >= 5
+    assert lib.rtvla_linear_act_workspace_bytes(M, K, N, 5, -1) == 0
+
+
 @pytest.mark.parametrize("M", [1, 3, 5, 2720])
 def test_layer_norm_of_1024_wide_rows_alone(M):
     """Four rows a workgroup, so row counts off by one; against float64: half a bf16 step of the result, and of the sum's terms fp32 errors."""

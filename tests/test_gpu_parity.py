@@ -280,6 +280,18 @@ def test_shape_sweep_against_the_oracle(model, views, prompt, chunk, state_token
     check_case(Case(model, 100 + views * 7 + prompt, views, prompt, chunk, 1, 2, state_tokens=state_tokens))
 
 
+@pytest.mark.parametrize("model,views,prompt,chunk,state_tokens,max_prompt", [
+    ("pi0", 1, 4, 10, 0, None), ("pi0", 1, 3, 100, 0, None), ("pi0", 1, 2000, 20, 0, None), ("pi0", 2, 20, 50, 0, None),
+    ("pi05", 1, 4, 10, 3, 12), ("pi05", 1, 5, 128, 4, None),
+])
+def test_the_flow_loop_as_launches_against_the_oracle(model, views, prompt, chunk, state_tokens, max_prompt):
+    """The route of a caller's own graph and of a stream that may not use the whole device: the same checks, layer by layer."""
+    case = Case(model, 700 + prompt + chunk, views, prompt, chunk, 1, 2, state_tokens=state_tokens, max_prompt=max_prompt)
+    case.e.ctx.set_flow_route(case.capi.FLOW_LAUNCHES)
+    check_case(case)
+    assert not case.e.ctx.flow_status()[0]
+
+
 @pytest.mark.parametrize("name,spec", [
     ("c1", ("pi0", 1234, 1, 0, 50)),
     ("c2", ("pi0", 1234, 2, 20, 50)),
