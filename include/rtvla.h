@@ -256,7 +256,7 @@ int rtvla_time_linear(const void* x, int M, int K, const void* w, int N, void* o
  * LayerNorm, :648-663 RMSNorm): x_out[M][N] = sum of the nsplit fp32 partials [split][M][N] (nsplit 0..4, 6, 8) + bias + residual, all optional
  * but one; xn_out = its LayerNorm with norm_w / norm_b (norm = RTVLA_NORM_LAYER) or x_out * rsqrt(mean x^2 + eps) (RTVLA_NORM_RMS),
  * computed from the bf16-rounded x_out as the forward does; N a multiple of 4, at most 2048; x_out or xn_out may be null. */
-enum rtvla_act { RTVLA_ACT_BIAS_GELU = 1, RTVLA_ACT_GEGLU = 2, RTVLA_ACT_SWIGLU = 3, RTVLA_ACT_RESIDUAL = 4 };
+enum rtvla_act { RTVLA_ACT_BIAS_GELU = 1, RTVLA_ACT_GEGLU = 2, RTVLA_ACT_SWIGLU = 3, RTVLA_ACT_RESIDUAL = 8 };
 enum rtvla_norm { RTVLA_NORM_NONE = 0, RTVLA_NORM_RMS = 1, RTVLA_NORM_LAYER = 2 };
 size_t rtvla_linear_act_workspace_bytes(int M, int K, int N, int act, int tile);
 int rtvla_linear_act(const void* x, int M, int K, const void* w, const void* w_up, int N, const void* bias, int act, void* out,

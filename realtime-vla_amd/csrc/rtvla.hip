@@ -1638,7 +1638,7 @@ struct ActPlan { size_t a_off, w0_off, w1_off, bias_off, scale_off, total; int K
 
 int plan_linear_act(int M, int K, int N, int act, int tile, ActPlan* out) {
     if (M <= 0 || K <= 0 || N <= 0 || (K & 7) || (N & 15)) return RTVLA_ERR_ARG;
-    if (act < RTVLA_ACT_BIAS_GELU || act > RTVLA_ACT_RESIDUAL) return RTVLA_ERR_ARG;
+    if (act != RTVLA_ACT_BIAS_GELU && act != RTVLA_ACT_GEGLU && act != RTVLA_ACT_SWIGLU && act != RTVLA_ACT_RESIDUAL) return RTVLA_ERR_ARG;
     if (tile < -1 || tile >= (int)TILE_COUNT) return RTVLA_ERR_ARG;
     ActPlan p{};
     p.dual = act == RTVLA_ACT_GEGLU || act == RTVLA_ACT_SWIGLU;
