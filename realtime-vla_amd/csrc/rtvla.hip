@@ -145,15 +145,18 @@ constexpr int XN_LD = 2048 + 64;   // row strides that are a large power of two 
 constexpr int EHID_LD = 16384 + 64;
 constexpr int64_t ATTN_PARTIAL_FLOATS = 64 * 16 * (16 * 64 * 4 + 32);   // 64 row blocks (128 suffix rows x 8 heads) x 16 key splits of the suffix attention
 
-// Pick block tile and split-K factor from a cost model fitted to measurements on MI355X (every tile and split on 73 shapes: the GEMMs of
-// a SigLIP, Gemma, DM0 ViT and DM0 prefix layer at one to four views, weights cold).  One K stage of a workgroup takes the larger of its
-// MFMA time (32 cycles per 32x32x16 MFMA at 2.05 GHz and 48 % issue efficiency) and a latency-bound load time (0.11 us + 10.4 us per MB
-// of operands pulled by the workgroup); tiles of 64 rows run two workgroups per CU, which then share the MFMA pipe but overlap their load
-// latency; all workgroups together cannot pull more than 17 TB/s out of L2; every launch pays a fixed ramp and an epilogue that grows
-// with the tile; split-K adds the reduce pass over the fp32 partials.  Over those shapes, weighted by the launches per forward, the choice
-// is 0.46 ms off the best one in sum (1.48 ms before the fit, with a table of exceptions and without the 96-row tile): SigLIP
-// up-projection at 768 rows 128x128 15.8 -> 64x128 14.0 us, DM0 ViT output projection at 2 720 rows 64x128 17.0 -> 96x128 13.4 us.
-TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittable, const char* what, bool eight = false) {
+// Pick block tile and split-K factor from a cost model fitted to measurements on MI355X: every tile and split in place of the chosen one in
+// a whole layer (114 GEMMs of a SigLIP, Gemma, DM0 ViT or DM0 prefix layer at one to four views and prompts of 0 to 200 tokens, all layers in
+// turn, so weights and activations are where a forward has them).  One K stage of a workgroup takes the larger of its MFMA time (32 cycles
+// per 32x32x16 MFMA at 2.05 GHz and 88 % issue efficiency) and its load time (0.143 us + 10.1 us per MB of operands pulled by the workgroup);
+// tiles of 64 rows run two workgroups per CU, which share the MFMA pipe and the CU's load path; all workgroups together cannot pull more
+// than 18.7 TB/s out of L2; every launch pays a ramp and an epilogue per 32 x 128 outputs of a workgroup, 2.7 times as long where Q, K and
+// V^T are scattered into fragment order; split-K adds the fp32 partials, written and read.  Over those layers, weighted by their number per
+// forward, the choice is 0.46 ms off the best one in sum.  It was 2.7 ms as long as two workgroups of a CU were taken to load twice as fast as
+// one, and needed a table for two shapes (SigLIP down-projection at 768 rows, output projection at 1 024) whose choices now follow.  Layer
+// times: SigLIP down-projection at 512 rows 64x128/6 -> 96x128/4 69.4 -> 65.8 us, at 1 024 rows 64x128/2 -> 128x128/3 93.7 -> 89.5; Gemma
+// down-projection at 868 rows 128x128/2 -> 128x256/4 247.7 -> 236.1, output projection at 649 rows 64x128/2 -> 96x128/2 205.2 -> 200.7.
+TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittable, const char* what, bool eight = false, bool scattered = false) {
     static const int tiles[] = {TILE_224x256, TILE_192x256, TILE_160x256, TILE_128x256, TILE_64x256, TILE_128x128, TILE_96x128, TILE_64x128};
     static const int splits[] = {1, 2, 3, 4, 6, 8};
     { TileChoice forced; if (tuning_forced_tile(what, splittable, &forced.tile, &forced.nsplit)) return forced; }
@@ -172,14 +175,6 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
         }
         return c8;
     }
-    // row counts where a launch by itself (its weights of a few layers stay in the last-level cache) disagrees with the whole forward, which
-    // was timed with either choice: SigLIP down-projection at 768 rows 128x128 against the model's 64x128, four splits each: 60 us less a
-    // forward; SigLIP output projection at 1 024 rows, two splits against the model's three: 95 us less
-    struct Measured { int ncols16, stages, m_lo, m_hi, tile, nsplit; };
-    static const Measured measured[] = {{72, 68, 513, 768, TILE_128x128, 4}, {72, 18, 769, 1024, TILE_64x128, 2}};
-    if (splittable)
-        for (const Measured& e : measured)
-            if (e.ncols16 == ncols16 && e.stages == stages && M >= e.m_lo && M <= e.m_hi) return TileChoice{e.tile, e.nsplit};
     double best = 1e30; TileChoice bc{TILE_128x256, 1};
     for (int tile : tiles) {
         const int bm = gemm_tile_bm(tile);
@@ -201,12 +196,12 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
             if (bm > 128 && ((sps & 1) || (tail & 1))) continue;          // the large tiles consume K stages in pairs
             const int blocks = mb * nb * sp;
             const int per_cu = (blocks + 255) / 256;
-            const double mfma_us = mt * nt * 4 * 32 / 2050.0 / 0.48;
+            const double mfma_us = mt * nt * 4 * 32 / 2050.0 / 0.88;
             const double stage_bytes = (double)(bm + bn) * 64 * 2;
-            const double alone_us = std::max(mfma_us, 0.11 + stage_bytes / 9.6e4), pair_us = std::max(occ * mfma_us, 0.11 + stage_bytes / 9.6e4);
-            double t = std::max((per_cu / occ * pair_us + per_cu % occ * alone_us) * sps, blocks * (double)sps * stage_bytes / 17.2e6);
-            t += 5.9 + 1.2 * mt * (splittable ? 1.5 : 1.0);
-            if (splittable) t += 2.2 + (double)sp * M * ncols16 * 16 * 4.0 / 7.5e6;    // the reduce pass over the partials
+            const double alone_us = std::max(mfma_us, 0.143 + stage_bytes / 9.9e4), pair_us = std::max(occ * mfma_us, 0.143 + occ * stage_bytes / 9.9e4);
+            double t = std::max((per_cu / occ * pair_us + per_cu % occ * alone_us) * sps, blocks * (double)sps * stage_bytes / 18.7e6);
+            t += 5.9 + (scattered ? 2.3 : 0.85) * mt * nt;
+            if (splittable) t += 2.2 + (double)sp * M * ncols16 * 16 * 4.0 / 3e6;    // the partials, written and read
             if (t <= best) { best = t; bc = TileChoice{tile, sp}; }      // (of equals the smaller tile)
         }
     }
@@ -557,7 +552,8 @@ struct Sched {
         GemmP p = extra;
         p.A = A; p.lda = lda; p.a_rows = a_rows; p.M = M; p.B0 = B0; p.B1 = B1;
         p.N16 = n16_tiles(N); p.K32p = k32_padded(K); p.bgroup = bgroup;
-        const TileChoice tc = choose_tile(M, p.N16, p.K32p / 2, epi == EPI_GEGLU || epi == EPI_SWIGLU, epi == EPI_PARTIAL, what, epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_VIT_QKV_ROPE);
+        const TileChoice tc = choose_tile(M, p.N16, p.K32p / 2, epi == EPI_GEGLU || epi == EPI_SWIGLU, epi == EPI_PARTIAL, what, epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_VIT_QKV_ROPE,
+                                          epi == EPI_QKV_ROPE || epi == EPI_VIS_QKV || epi == EPI_VIT_QKV_ROPE);
         p.nsplit = tc.nsplit;
         if (epi == EPI_PARTIAL) {
             p.partial = c->B<float>("splitk_partial"); p.ldp = N; p.pstride = (size_t)M * N;
