@@ -89,11 +89,11 @@ def bench_transforms(args, dev):
             tr.resize_pad_normalize_into(dframes[v], out[v])
     e1.record(); torch.cuda.synchronize()
     img_us = e0.elapsed_time(e1) * 1e3 / 20
-    alg_bytes = 3 * (480 * 640 * 3 + 2 * 480 * 224 * 3 + 224 * 224 * 3 * 2)        # frame read, 8-bit intermediate write+read, bf16 write
+    alg_bytes = 3 * (480 * 640 * 3 + 224 * 224 * 3 * 2)        # frame read, bf16 written (the 8-bit intermediate stays in LDS)
     result = {"metric": "us per observation pre+post-processing (3 frames 480x640 -> 224x224 bf16, state, 50x7 actions)",
               "value": round(times[len(times) // 2], 1), "unit": "us", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
               "higher_is_better": False, "dtype": "u8/f64", "data": "synthetic",
-              "roofline": {"bound": "hbm", "kernel": "resample_h_kernel + resample_v_pad_norm_kernel x 3 frames", "achieved": round(alg_bytes / img_us / 1e3, 2),
+              "roofline": {"bound": "hbm", "kernel": "resize_kernel x 3 frames", "achieved": round(alg_bytes / img_us / 1e3, 2),
                            "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(alg_bytes / img_us / 1e3 / HBM_PEAK_GBS, 5), "launch_ms": round(img_us / 1e3, 4),
                            "traffic": None}}
     if not args.no_cpu:
@@ -375,16 +375,17 @@ def main():
                 "algorithmic_bytes": 2.0 * (S_e * 2048 + 2 * 2048 * 16384 + S_e * 16384),
                 # informational: the rate at which the launch draws its operand tiles from L2 (the kernels here top out near 10 TB/s)
                 "l2_to_cu": {"bytes": l2_bytes, "tb_per_s": round(l2_bytes / (geglu_ms * 1e-3) / 1e12, 2)}}
-    # the action-expert side: one suffix layer (5 launches) streams 18 D_L-sized weight sets per step
+    # the action-expert side: the layers of one flow step in one launch of the resident kernel, divided by their number
     layer_ms = ctx.time_stage(capi.STAGE_SUFFIX_LAYER, -1, 0, 5, stream)          # all 18 layers in turn: weights cold, as in the forward
-    layer_warm_ms = ctx.time_stage(capi.STAGE_SUFFIX_LAYER, 3, 0, 20, stream)
+    # (a layer as a program of its own, as the stage calls run it, is that plus the program's four launches and copies of the stream)
+    layer_program_ms = ctx.time_stage(capi.STAGE_SUFFIX_LAYER, 3, 0, 20, stream)
     d_l = 1024 * 2560 + 2048 * 1024 + 3 * 1024 * 4096
     layer_bytes = 2.0 * d_l + 2.0 * keys * 256 * 2
     hbm = layer_bytes / (layer_ms * 1e-3) / 1e9
-    roofline_hbm = {"bound": "hbm", "kernel": "one action-expert layer (qkv, attention, o, geglu, down)",
+    roofline_hbm = {"bound": "hbm", "kernel": "one action-expert layer of the resident flow loop (flow_kernel)",
                     "achieved": round(hbm, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(hbm / HBM_PEAK_GBS, 4),
-                    "launch_ms": round(layer_ms, 4), "launch_ms_cache_warm": round(layer_warm_ms, 4),
-                    # HBM bytes per layer from rocprofv3 FETCH_SIZE + WRITE_SIZE summed over the layer's kernels (profiles/)
+                    "launch_ms": round(layer_ms, 4), "one_layer_program_ms": round(layer_program_ms, 4),
+                    # HBM bytes per layer from rocprofv3 FETCH_SIZE + WRITE_SIZE of a launch over all layers (profiles/)
                     "traffic": profiled_traffic("action_expert_layer_%s_hbm_traffic.md" % PROFILE_TAGS.get(args.config), "action-expert layer", args.config, lib_version),
                     "algorithmic_bytes": layer_bytes}
     # whole-forward roofline fraction: (F_vis + F_pre) / P_mfma + B_dec / BW  over the measured p50
