@@ -13,18 +13,20 @@
 // for the CUs r of the other seven (8 flags), then sums the tiles those eight produced in a fixed order.  A layer is
 //   qkv | logits + exp | P V | O partial || sum + residual | gate, up | down partial || sum + residual |      (| XCD barrier, || 8-CU barrier)
 // Measured on MI355X: XCD barrier 0.35 us (1.02 us with 1 KB stored per workgroup before it and 32 KB read after it, 1.43 us with
-// 64 KB), a barrier over all CUs 1.6 us, a dependent launch 2.3 us empty and 4.4-5.0 us as part of a layer.
+// 64 KB), a barrier over all CUs 1.6 us, a dependent launch 2.3 us empty and 4.4-5.0 us as part of a layer.  Of a layer's 25.7 us
+// (Pi0, one view, chunk 50) 14 are barriers, exchanges and the waits behind them.
 //
 // A CU holds RH of the 2 RH row tiles (CU parity) and the columns of one of 16 groups, so the activations of a phase are read once
 // into half the CUs each and the weights twice per XCD (once from memory).  The eight compute waves split K and reduce through LDS; a
-// ninth wave does the waiting, so that the compute waves can have the next phase's weights on the way while it polls.
+// ninth wave does the waiting, so that the compute waves can have the next phase's weights on the way while it polls, and a tenth pulls the
+// weights of the phases after that into the XCD's L2.
 //
 // All workgroups have to be resident at once.  A process keeps one flow kernel per device in flight (rtvla.hip), but another process's
 // may be placed on half of the CUs at the same moment.  So no workgroup starts before all 256 have reported: the last one opens the
 // gate, and one that has waited too long closes it, after which all of them leave and the CUs are free.  The kernel is therefore
-// launched twice; the second launch ends at once if the first one ran, and the limits differ from process to process.  Past the gate
-// every wait still ends after wait_ticks: the wave notes it in `abort` and the kernel runs to its end without waiting, so the grid always
-// drains.  Nothing makes the two launches succeed: kernels of others may hold the CUs for as long as they like.  The last launch
+// launched twice; the second launch ends at once if the first one ran, and the limits differ from process to process and from loop to
+// loop.  Past the gate every wait still ends after wait_ticks: the wave notes it in `abort` and the kernel runs to its end without
+// waiting, so the grid always drains.  Nothing makes the two launches succeed: kernels of others may hold the CUs for as long as they like.  The last launch
 // (flow_kernel<.., ALONE>) therefore runs the same program in ONE workgroup, which waits for nobody, if neither finished: the phases one
 // after another for the 256 (XCD, number) pairs, with the same sums in the same order, hence the same bits.  That takes 0.7 - 1.0 s
 // instead of 5 - 7 ms; otherwise it ends at once (a forward of 8.33, 10.72 or 13.43 ms takes the same with and without it).  The input noise and

@@ -332,3 +332,21 @@ def test_two_processes_on_one_gpu():
         for w in workers:
             w.stdin.close()
             w.wait(timeout=60)
+
+
+def test_three_processes_on_one_gpu():
+    """The CUs that one of three leaves may be shared by the other two, so that all of them get to the last launch, of one workgroup: no forward
+    is lost there either, and with the route held to the resident kernel all of them are the same bits."""
+    paths = [os.path.dirname(os.path.abspath(__file__)), os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "realtime-vla_amd")]
+    code = (WORKER % paths).replace("first = ", "m._engine.ctx.set_flow_route(1)\nfirst = ").replace("range(500)", "range(100)")
+    workers = [subprocess.Popen([sys.executable, "-u", "-c", code], stdin=subprocess.PIPE, stdout=subprocess.PIPE, text=True) for _ in range(3)]
+    try:
+        assert [w.stdout.readline().split() for w in workers] == [["ready"]] * 3
+        for w in workers:
+            w.stdin.write("go\n")
+            w.stdin.flush()
+        assert [w.stdout.readline().split() for w in workers] == [["same", "100", "True"]] * 3
+    finally:
+        for w in workers:
+            w.stdin.close()
+            w.wait(timeout=60)
