@@ -103,7 +103,7 @@ class Engine:
         side.wait_stream(torch.cuda.current_stream(self.device))
         self.ctx.graph_capture(side.cuda_stream)
         side.synchronize()
-        self.graph_launches = self.ctx.launch_count()      # kernel nodes in the captured graph
+        self.graph_launches = self.ctx.launch_count()      # kernels of one replay: the captured graph's and the flow loop's
 
     def reference_buffer(self, name):
         """Row-major copy of an internal activation in the shape the reference keeps it in

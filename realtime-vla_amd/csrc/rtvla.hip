@@ -153,7 +153,7 @@ constexpr int64_t ATTN_PARTIAL_FLOATS = 64 * 16 * (16 * 64 * 4 + 32);   // 64 ro
 // than 18.7 TB/s out of L2; every launch pays a ramp and an epilogue per 32 x 128 outputs of a workgroup, 2.7 times as long where Q, K and
 // V^T are scattered into fragment order; split-K adds the fp32 partials, written and read.  Over those layers, weighted by their number per
 // forward, the choice is 0.46 ms off the best one in sum.  It was 2.7 ms as long as two workgroups of a CU were taken to load twice as fast as
-// one, and needed a table for two shapes (SigLIP down-projection at 768 rows, output projection at 1 024) whose choices now follow.  Layer
+// one, and needed a table for two shapes (SigLIP down-projection at 768 rows, output projection at 1 024) that are within 0.7 us of the best now.  Layer
 // times: SigLIP down-projection at 512 rows 64x128/6 -> 96x128/4 69.4 -> 65.8 us, at 1 024 rows 64x128/2 -> 128x128/3 93.7 -> 89.5; Gemma
 // down-projection at 868 rows 128x128/2 -> 128x256/4 247.7 -> 236.1, output projection at 649 rows 64x128/2 -> 96x128/2 205.2 -> 200.7.
 TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittable, const char* what, bool eight = false, bool scattered = false) {
