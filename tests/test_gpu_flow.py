@@ -134,6 +134,31 @@ def test_a_forward_on_bad_inputs_leaves_nothing_behind(model, views, prompt, chu
     assert torch.equal(m.forward(*inputs), want) and torch.isfinite(want.float()).all()
 
 
+@pytest.mark.parametrize("route", [capi.FLOW_RESIDENT, capi.FLOW_LAUNCHES], ids=["resident", "launches"])
+@pytest.mark.parametrize("staged_on", ["device", "host"])
+def test_rows_behind_a_short_prompt_are_not_those_of_a_bad_forward(staged_on, route):
+    """Pi05 with 40 rows for its prompt: the rows behind a shorter one keep their residual stream from call to call, and nobody may see them."""
+    from pi05_infer import Pi05Inference
+    rows, vocab = 40, 640
+    ck = syn.pi05_checkpoint(860, 0, "cuda:0", 1, 2, state_tokens=0, norms="random")
+    del ck["language_embeds"]
+    table = syn.normal_bf16(860, "embedding_weight_small", (vocab, 2048), 0.02, "cuda:0")
+    images, _, noise = syn.observation(860, 1, 33, "cuda:0")
+    if staged_on == "device":
+        m = Pi05Inference(dict(ck, embedding_weight=table), 1, 33, max_tokenize_len=rows, discrete_state_input=False)
+        forward = lambda img, n: m.forward_ids(img, noise, syn.randint(860, "ids%d" % n, n, vocab)).clone()
+    else:
+        m = Pi05Inference(dict(ck, language_embeds=torch.zeros(rows, 2048, dtype=torch.bfloat16, device="cuda:0")), 1, 33, discrete_state_input=False)
+
+        def forward(img, n):
+            m.weights["language_embeds"] = (table[syn.randint(860, "ids%d" % n, n, vocab).to("cuda:0")].float() * (2048.0 ** 0.5)).to(torch.bfloat16)
+            return m.forward(img, noise).clone()
+    m._engine.ctx.set_flow_route(route)
+    want = forward(images, 4)
+    assert not torch.isfinite(forward(torch.full_like(images, float("nan")), 37).float()).any()
+    assert torch.equal(forward(images, 4), want) and torch.isfinite(want.float()).all()
+
+
 @pytest.mark.parametrize("model", ["pi0", "pi05", "dm0"])
 def test_launches_after_a_loop_in_one_workgroup(model):
     """Whatever held the CUs may go on doing so: the next 64 forwards take the launches, then the resident kernel is tried again."""
