@@ -18,8 +18,16 @@
 //
 // A CU holds RH of the 2 RH row tiles (CU parity) and the columns of one of 16 groups, so the activations of a phase are read once
 // into half the CUs each and the weights twice per XCD (once from memory).  The eight compute waves split K and reduce through LDS; a
-// ninth wave does the waiting, so that the compute waves can have the next phase's weights on the way while it polls, and a tenth pulls the
-// weights of the phases after that into the XCD's L2.
+// ninth wave does the waiting, so that the compute waves can have the next phase's weights on the way while it polls.
+//
+// When the weights are asked for decides a layer's time more than anything else.  A CU's vector cache returns its loads in the order it
+// got them, whichever wave asked: a line that comes from HBM holds up the flags, activations and partial sums behind it by its 1 - 2 us.
+// A tenth wave that pulled all of the coming phases' weights into L2 (one word per line, spread over the phases) made a layer 2.2 us
+// slower than none (Pi0, 1 view, chunk 50: forward of one vision layer 6 735 us with it, 6 340 us without); so did weights requested ahead
+// of an exchange (+0.7 us for the up tiles, +0.6 us for qkv), or K / V^T behind the qkv products (+0.1 us).  What pays: the weights of a
+// phase behind the flag of the one before, while the others are waited for; those of the output projection already behind the P V
+// products (-0.3 us), and the down projection's lines touched by the waiting wave during the output projection (-0.2 us), whose exchange
+// takes longer than they do.
 //
 // All workgroups have to be resident at once.  A process keeps one flow kernel per device in flight (rtvla.hip), but another process's
 // may be placed on half of the CUs at the same moment.  So no workgroup starts before all 256 have reported: the last one opens the
@@ -38,7 +46,7 @@
 namespace {
 
 constexpr int FW = 8;                                    // compute waves
-constexpr int FLOW_THREADS = (FW + 2) * 64;              // + the wave that posts and polls flags, + the wave that fetches ahead
+constexpr int FLOW_THREADS = (FW + 1) * 64;              // + the wave that polls flags
 constexpr float NEG_BIG = -1.0e30f;
 constexpr int SQ_BYTES = FW * 4 * 64;
 constexpr int ROPE_PITCH = 272;                                       // 256 bytes of a row, and 16 that move the next one to other banks
@@ -194,9 +202,8 @@ void flow_kernel(FlowP kernel_args) {
     const bool keep_in = layer0 == layer1;                                     // (a single stage: the new stream goes back to the caller's buffer)
     auto bar = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
-    // ============ the waiting wave posts and polls the flags, the fetching wave pulls what comes up into the XCD's L2; both meet the
-    // ============ compute waves at every barrier
-    [[maybe_unused]] auto walk = [&](auto&& local, auto&& slot) __attribute__((always_inline)) {
+    // ============ the waiting wave polls the flags and meets the compute waves at every barrier
+    [[maybe_unused]] auto walk = [&](auto&& local, auto&& ahead) __attribute__((always_inline)) {
         if (!begin) local();
         for (int t = step0; t < step1; ++t) {
             if (begin) {
@@ -204,12 +211,12 @@ void flow_kernel(FlowP kernel_args) {
                 if (!PI05) { bar(); if (!keep_in) local(); }
             }
             for (int l = layer0; l < layer1; ++l) {
-                slot(0, t, l); bar(); local();                                 // qkv
-                slot(1, t, l); local();                                        // logits
-                slot(2, t, l); bar(); local();                                 // P V
-                slot(3, t, l); bar(); slot(4, t, l); local();                  // output projection, exchange, sum
-                slot(5, t, l); bar(); local();                                 // gate, up
-                slot(6, t, l); bar(); slot(7, t, l); local();                  // down projection, exchange, sum
+                bar(); local();                                                // qkv
+                local();                                                       // logits
+                bar(); local();                                                // P V
+                ahead(l); bar(); local();                                      // output projection, exchange, sum
+                bar(); local();                                                // gate, up
+                bar(); local();                                                // down projection, exchange, sum
             }
             if (end) {
                 bar(); bar();
@@ -220,6 +227,10 @@ void flow_kernel(FlowP kernel_args) {
     if constexpr (!ALONE) if (w_ == FW) {
         const int lane = lane_, x = x_;
         const unsigned* const flags = kernel_args.sync->lflag + x * 256 + lane * 4;      // 32 workgroups x 8 compute waves, 4 flags per lane
+        // One word of every 128-byte line is loaded into a scrap of LDS: the line is then in this XCD's L2 when the compute waves ask for it.
+        const unsigned scrap = (unsigned)(FW * 4 * RH * 1024 + SQ_BYTES + 64);
+        typedef const __attribute__((address_space(1))) void* gptr_t;
+        typedef __attribute__((address_space(3))) void* lptr_t;
         unsigned ep = 0;
         Patience patience;
         if (kernel_args.wait_ticks == 0) {
@@ -237,71 +248,19 @@ void flow_kernel(FlowP kernel_args) {
                  patience.n = 0;
                  bar();
              },
-             [](int, int, int) __attribute__((always_inline)) {});
-        return;
-    }
-    if constexpr (!ALONE) if (w_ == FW + 1) {
-        // One word of every 128-byte line is loaded into a scrap of LDS: the line is then in this XCD's L2 when the compute waves ask for
-        // it, two to five phases later.  The 32 workgroups of an XCD share the lines out; a slot is 0.5 - 1 MB per XCD.
-        const unsigned scrap = (unsigned)(FW * 4 * RH * 1024 + SQ_BYTES + 64);
-        typedef const __attribute__((address_space(1))) void* gptr_t;
-        typedef __attribute__((address_space(3))) void* lptr_t;
-        auto touch = [&](const void* base, int first, int bytes, int lines64) __attribute__((always_inline)) {      // lines64 x 64 lines from byte `first` of `bytes`
-            for (int i = 0; i < lines64; ++i) {
-                const int off = min(first + (i * 64 + lane_) * 128, bytes - 128);
-                __builtin_amdgcn_global_load_lds((gptr_t)((const char*)base + off), (lptr_t)(smem + scrap), 4, 0, 0);
-            }
-        };
-        const int KBp = (kernel_args.prefix + 31) >> 5;
-        walk(bar, [&](int k, int t, int l) __attribute__((always_inline)) {
-            cFlowP& p = prm();
-            const int x = x_, r = r_;
-            int tn = t, ln = l + 1;                                            // the layer after this one
-            if (ln == layer1) { ln = layer0; tn = t + 1 < step1 ? t + 1 : t; }
-            // what a phase reads of a few kilobytes that nothing else has touched: norm weights (DM0), biases and gates (Pi05)
-            if constexpr (DM0) {
-                if (k == 4 && r < 2) touch((r ? p.knorm : p.qnorm) + (size_t)ln * 128, 0, 256, 1);
-            } else if constexpr (PI05) {
-                const size_t tl = (size_t)t * p.layers + l;
-                if (k == 4 && r < 2) touch(p.bias_qkv + ((size_t)tn * p.layers + ln) * 2560 + (r ? 2048 : x * 256), 0, r ? 2048 : 1024, 1);
-                if (k == 0 && r < 4) touch(r == 0 ? (const void*)(p.style_attn + tl * 3072 + 2048) : r == 1 ? (const void*)(p.style_ffn + tl * 3072 + 2048) : (const void*)((r == 2 ? p.bias_gate : p.bias_up) + tl * 4096 + x * C::HID), 0, 2048, 1);
-            }
-            if (k <= 2) {                                                      // gate and up tiles of this layer: 2 x 32 KB of every workgroup, in thirds
-                if (r < C::HID / 16) {
-                    const size_t o = (size_t)(PI05 ? t * p.layers + l : l) * p.wg_stride + (size_t)(x * (C::HID / 16) + r) * 32 * 512;
-                    if (k == 0) touch(p.wg + o, 0, 32768, 3);
-                    if (k == 1) { touch(p.wg + o, 3 * 8192, 32768, 1); touch(p.wu + o, 0, 32768, 2); }
-                    if (k == 2) touch(p.wu + o, 2 * 8192, 32768, 2);
-                }
-            } else if (k == 3) {                                               // down projection of this layer: this XCD's K slice of two column tiles
+             [&](int l) __attribute__((always_inline)) {                       // down projection of this layer: this XCD's K slice of two column tiles
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    touch(p.wd + (size_t)l * p.wd_stride + ((size_t)(2 * r + j) * C::WD_K32 + x * HID32) * 512, 0, HID32 * 1024, (HID32 + 7) / 8);
-            } else if (k == 4 || k == 5) {                                     // qkv of the next layer: AT * 16 tiles of 32 KB
-                const bf16_t* base = p.wqkv + (size_t)(PI05 ? tn * p.layers + ln : ln) * p.wqkv_stride;
-                const int hf = r * C::AT + (k == 4 ? 0 : 1);                   // half tiles of 16 KB, AT per workgroup
-                auto half_tile = [&](int h) __attribute__((always_inline)) {
-                    const int grp = (h >> 1) & 15, j = (h >> 1) >> 4;
-                    const int nb = DM0 ? (j == 0 ? x * 16 + grp : (grp < 8 ? 128 + x * 8 + grp : 192 + x * 8 + grp - 8)) : (j == 0 ? x * 16 + grp : j == 1 ? 128 + grp : 144 + grp);
-                    touch(base + (size_t)nb * 32 * 512, (h & 1) * 16384, 32768, 2);
-                };
-                half_tile(hf);
-                if (k == 5 && C::AT == 3) half_tile(hf + 1);
-            } else if (k == 6) {                                               // cached K and V^T of the next layer
-                const size_t o = (size_t)(DM0 ? ln * 8 + x : ln) * p.kv_stride;
-                for (int kb = r; kb < KBp; kb += 32) touch(p.kcache + o + (size_t)kb * 2 * KD * 512, 0, 2 * KD * 1024, 2 * KD / 8);
-                constexpr int SH = 32 / DT;                                    // workgroups per 16-wide d tile
-                const int vb = KBp * 1024 / SH;
-                touch(p.vcache + o + (size_t)(r / SH) * (p.ldvt >> 5) * 512, (r % SH) * vb, KBp * 1024, (vb + 8191) >> 13);
-            } else {                                                           // output projection of the next layer
+                 for (int j = 0; j < 2; ++j) {
+                     cFlowP& p = prm();
+                     const bf16_t* const base = p.wd + (size_t)l * p.wd_stride + ((size_t)(2 * r_ + j) * C::WD_K32 + x * HID32) * 512;
 #pragma unroll
-                for (int j = 0; j < 2; ++j) touch(p.wo + (size_t)ln * p.wo_stride + ((size_t)(2 * r + j) * 64 + x * 8) * 512, 0, 8192, 1);
-            }
-        });
+                     for (int i = 0; i < (HID32 + 7) / 8; ++i)
+                         __builtin_amdgcn_global_load_lds((gptr_t)((const char*)base + min((i * 64 + lane) * 128, HID32 * 1024 - 128)), (lptr_t)(smem + scrap), 4, 0, 0);
+                 }
+             });
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                       // nothing may land in LDS after the workgroup has ended
         return;
     }
-
     // ================================================= the compute waves =================================================
     rsrc_t priv = make_rsrc(kernel_args.priv + (size_t)x_ * kernel_args.priv_stride, (unsigned)kernel_args.priv_stride);
     const rsrc_t part = make_rsrc(kernel_args.part, kernel_args.part_bytes);
@@ -464,8 +423,8 @@ void flow_kernel(FlowP kernel_args) {
                     const bf16x4 o = pack4(v[0] * c0 - v[1] * s0, v[1] * c0 + v[0] * s0, v[2] * c1 - v[3] * s1, v[3] * c1 + v[2] * s1);
                     const int row = row0 + lr;
                     st8(priv, (j == 0 ? p.off_q : p.off_k) + ft_off(row, n0, 8), o);
-                    // the cache rows behind the prefix, as the reference keeps them (nothing here reads them back)
-                    if (j == 1 && x == 0 && row < rows) store4(p.kcache + (size_t)l * p.kv_stride + ft_index(p.prefix + row, n0, 8), o);
+                    // the cache rows behind the prefix, as the reference keeps them after the last step (nothing here reads them back)
+                    if (j == 1 && x == 0 && row < rows && t == step1 - 1) store4(p.kcache + (size_t)l * p.kv_stride + ft_index(p.prefix + row, n0, 8), o);
                 } else {                                                       // V: lane holds 4 keys of one column
                     const int d = grp * 16 + lr, key = row0 + 4 * g;
                     float b = 0.f;
@@ -475,7 +434,7 @@ void flow_kernel(FlowP kernel_args) {
                     for (int e = 0; e < 4; ++e) o[e] = v[e] * row_factor(m * 16 + 4 * g + e) + b;
                     const bf16x4 pk = pack4(o);
                     st8(priv, p.off_v + (((d >> 4) * 4 + (key >> 5)) * 64 + (d & 15) + 16 * ((key & 15) >> 2)) * 16 + 8 * ((key & 31) >> 4), pk);
-                    if (x == 0) {
+                    if (x == 0 && t == step1 - 1) {
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
                             if (key + e < rows) p.vcache[(size_t)l * p.kv_stride + vt_index(d, p.prefix + key + e, p.ldvt >> 5)] = pk[e];
@@ -595,18 +554,20 @@ void flow_kernel(FlowP kernel_args) {
 
     // ---- O = P V for one query row tile and NDT 16-wide column tiles; the waves split the key blocks, every 16 keys with their own factor ----
     constexpr int VB = 4;                                                      // blocks of a wave per trip (32 key blocks per workgroup)
+    // (a block past the prefix is requested behind the end of the buffer: the hardware returns zero and reads nothing)
     auto load_v = [&](cFlowP& p, int lane, int x, int pdg, int l, int kb, bf16x8 (&v)[NDT]) __attribute__((always_inline)) {
-        const bf16_t* base = p.vcache + (size_t)(DM0 ? l * 8 + x : l) * p.kv_stride;
+        const rsrc_t rs = make_rsrc(p.vcache + (size_t)(DM0 ? l * 8 + x : l) * p.kv_stride, (unsigned)p.kv_stride * 2u);
 #pragma unroll
-        for (int d = 0; d < NDT; ++d) v[d] = *(const bf16x8*)(base + ((size_t)((pdg * NDT + d) * (p.ldvt >> 5) + kb) * 64 + lane) * 8);
+        for (int d = 0; d < NDT; ++d)
+            v[d] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rs, kb < KBp ? (((pdg * NDT + d) * (p.ldvt >> 5) + kb) * 64 + lane) * 16 : 0x7fffff00, 0, 0));
     };
     auto pre_pv = [&](cFlowP& p, int l, bf16x8 (&vf)[VB][NDT]) __attribute__((always_inline)) {
         FLOW_IDS;
         const int pdg = r / QRTP;
 #pragma unroll
-        for (int i = 0; i < VB; ++i) load_v(p, lane, x, pdg, l, min(w + FW * i, KBp - 1), vf[i]);
+        for (int i = 0; i < VB; ++i) load_v(p, lane, x, pdg, l, w + FW * i, vf[i]);
     };
-    auto pv = [&](cFlowP& p, int l, bf16x8 (&vf)[VB][NDT]) __attribute__((always_inline)) {
+    auto pv = [&](cFlowP& p, int l, bf16x8 (&vf)[VB][NDT], auto&& next) __attribute__((always_inline)) {
         FLOW_IDS;
         const int prt = r % QRTP, pdg = r / QRTP;
         if (QRT == QRTP || prt < QRT) {
@@ -629,7 +590,7 @@ void flow_kernel(FlowP kernel_args) {
                     if (kb >= KBp && kb < KB)
 #pragma unroll
                         for (int d = 0; d < NDT; ++d) vf[i][d] = ld16(priv, p.off_v + (((pdg * NDT + d) * 4 + kb - KBp) * 64 + lane) * 16);
-                    else if (b0 > 0) load_v(p, lane, x, pdg, l, min(kb, KBp - 1), vf[i]);
+                    else if (b0 > 0) load_v(p, lane, x, pdg, l, kb, vf[i]);
                 }
                 float m = M;
 #pragma unroll
@@ -649,8 +610,8 @@ void flow_kernel(FlowP kernel_args) {
                     L += f0 * mo[i][1] + f1 * mo[i][3];
                     if constexpr (ALONE) {
                         // the cache's rows behind the prefix, where a launch that gave up may have left anything: their probabilities are
-                        // zero, but 0 x NaN is NaN (blocks past the last one hold the prefix's last one)
-                        if (const int kb = b0 + w + FW * i, key0 = min(kb, KBp - 1) * 32 + 4 * g; kb < KBp || !in)
+                        // zero, but 0 x NaN is NaN
+                        if (const int kb = b0 + w + FW * i, key0 = kb * 32 + 4 * g; kb < KBp)
 #pragma unroll
                             for (int d = 0; d < NDT; ++d)
 #pragma unroll
@@ -665,6 +626,7 @@ void flow_kernel(FlowP kernel_args) {
             for (int d = 0; d < NDT; ++d) red[((size_t)w * NDT + d) * 64 + lane] = o[d];
             if (g == 0) { sq[w * 16 + lr] = M; sq[FW * 16 + w * 16 + lr] = L; }
         }
+        next();
         bar();
         if (w < NDT && (QRT == QRTP || prt < QRT)) {
             float mw[FW], M = NEG_BIG, L = 0.f;
@@ -943,7 +905,7 @@ void flow_kernel(FlowP kernel_args) {
                 const size_t tl = (size_t)t * kernel_args.layers + l;
                 each([&]() __attribute__((always_inline)) { bf16x8 wA[C::AT][4]; bf16x4 cs[AK]; pre_qkv(prm(), t, l, wA, cs); qkv(prm(), t, l, wA, cs); });
                 each([&]() __attribute__((always_inline)) { bf16x8 kf[KD]; pre_logits(prm(), l, kf); logits(prm(), l, kf); });
-                each([&]() __attribute__((always_inline)) { bf16x8 vf[VB][NDT]; pre_pv(prm(), l, vf); pv(prm(), l, vf); });
+                each([&]() __attribute__((always_inline)) { bf16x8 vf[VB][NDT]; pre_pv(prm(), l, vf); pv(prm(), l, vf, nothing); });
                 each([&]() __attribute__((always_inline)) {
                     bf16x8 wC[4][1];
                     load_c(prm(), l, wC);
@@ -995,19 +957,17 @@ void flow_kernel(FlowP kernel_args) {
                 sync([&]() __attribute__((always_inline)) { pre_logits(prm(), l, kf); });
                 logits(prm(), l, kf);
             }
+            bf16x8 wC[4][1];
             {
                 bf16x8 vf[VB][NDT];
                 sync([&]() __attribute__((always_inline)) { pre_pv(prm(), l, vf); });
-                pv(prm(), l, vf);
+                pv(prm(), l, vf, [&]() __attribute__((always_inline)) { load_c(prm(), l, wC); });
             }
             {
                 bf16x8 wE[2 * C::ET][4];
                 f32x4 own[SK];
-                {
-                    bf16x8 wC[4][1];
-                    sync([&]() __attribute__((always_inline)) { load_c(prm(), l, wC); load_e(prm(), t, l, 0, wE); });
-                    gemm.template operator()<4, 1>(wC, prm().off_o, 8, w_, false, 9);
-                }
+                sync([&]() __attribute__((always_inline)) { load_e(prm(), t, l, 0, wE); });
+                gemm.template operator()<4, 1>(wC, prm().off_o, 8, w_, false, 9);
                 bar();
                 store_part(FW, own);
                 cFlowP& p = prm();
