@@ -382,7 +382,10 @@ void flow_kernel(FlowP kernel_args) {
     auto pre_qkv = [&](cFlowP& p, int t, int l, bf16x8 (&wA)[C::AT][4], bf16x4 (&pre_cs)[AK]) __attribute__((always_inline)) {
         FLOW_IDS;
         load_a(p, t, l, wA);
-        if constexpr (!DM0) {
+        if constexpr (DM0) {                                                   // norm weights instead (the rotary table is in LDS)
+#pragma unroll
+            for (int k = 0; k < AK; ++k) pre_cs[k] = load4(((w + 8 * k) / RH == 0 ? p.qnorm : p.knorm) + (size_t)l * 128 + (grp & 7) * 16 + 4 * g);
+        } else {
 #pragma unroll
             for (int k = 0; k < AK; ++k) {
                 const int u = w + 8 * k;
@@ -404,9 +407,21 @@ void flow_kernel(FlowP kernel_args) {
                 f32x4 v = tile_sum(lane, NT * RH, u, FW);
                 const int row0 = (half * RH + m) * 16;
                 if constexpr (DM0) {
-                    // raw products, rounded as the reference's QKV buffer; V carries the row's RMS factor, Q and K get it with their norm
-                    if (j == 0) st8(priv, p.off_q + ft_off(((grp >> 3) * RTP) * 16 + row0 + lr, (grp & 7) * 16 + 4 * g, KD), pack4(v));
-                    else if (grp < 8) st8(priv, p.off_k + ft_off(row0 + lr, grp * 16 + 4 * g, KD), pack4(v));
+                    // products rounded as the reference's QKV buffer; V carries the row's RMS factor.  Q and K leave with norm weight and
+                    // rotary embedding but without the row's factors (RMS factor, norm over the head's 128 features), which are scalars
+                    // of the logits: for those goes the sum of squares of the tile's 16 features.
+                    if (j == 0 || grp < 8) {
+                        const int col = (grp & 7) * 16 + 4 * g, row = row0 + lr;
+                        const bf16x4 cs = *(const bf16x4*)(rope_lds + row * ROPE_PITCH + col * 2);
+                        float ss = 0.f;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) { v[e] = round_bf16(v[e]); ss += v[e] * v[e]; v[e] *= bf2f(pre_cs[k][e]); }
+                        ss = rows_sum(ss);
+                        const float c0 = bf2f(cs[0]), s0 = bf2f(cs[1]), c1 = bf2f(cs[2]), s1 = bf2f(cs[3]);
+                        const bf16x4 o = pack4(v[0] * c0 - v[1] * s0, v[1] * c0 + v[0] * s0, v[2] * c1 - v[3] * s1, v[3] * c1 + v[2] * s1);
+                        st8(priv, j == 0 ? p.off_q + ft_off((grp >> 3) * RTP * 16 + row, col, KD) : p.off_k + ft_off(row, col, KD), o);
+                        if (g == 0) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ss), priv, p.off_s + (((j == 0 ? grp >> 3 : 2) * RTP * 16 + row) * 8 + (grp & 7)) * 4, 0, 0);
+                    }
                     else {
                         const int d = (grp - 8) * 16 + lr, key = row0 + 4 * g;
                         f32x4 o;
@@ -450,26 +465,14 @@ void flow_kernel(FlowP kernel_args) {
         }
     };
 
-    // DM0: factor, RMS norm over the head's 128 features, norm weight, rotary embedding on adjacent pairs; lane holds 8 features per block
-    // The rotary table comes from LDS: from memory it would be 4 KB per wave and row tile, more than the queries.
-    auto dm0_qk = [&](int g, bf16x8 (&v)[KD], float f, int tok, const bf16_t* nw) __attribute__((always_inline)) {
-        bf16x8 cs[KD], ww[KD];
+    // DM0: what a row of raw queries (head 0, 1) or keys (2) is scaled by: its RMS factor f, then the RMS norm over the head's 128 features
+    auto dm0_scale = [&](cFlowP& p, int which, int row) __attribute__((always_inline)) {
+        f32x4 s[2];
 #pragma unroll
-        for (int kd = 0; kd < KD; ++kd) { cs[kd] = *(const bf16x8*)(rope_lds + tok * ROPE_PITCH + kd * 64 + 16 * g); ww[kd] = *(const bf16x8*)(nw + kd * 32 + 8 * g); }
-        float y[KD][8], s = 0.f;
-#pragma unroll
-        for (int kd = 0; kd < KD; ++kd)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) { y[kd][j] = bf2f(v[kd][j]) * f; s += y[kd][j] * y[kd][j]; }
-        const float inv = rsqrtf(rows_sum(s) * (1.0f / 128.0f) + 1e-6f);
-#pragma unroll
-        for (int kd = 0; kd < KD; ++kd)
-#pragma unroll
-            for (int j = 0; j < 8; j += 2) {
-                const float a = y[kd][j] * inv * bf2f(ww[kd][j]), b = y[kd][j + 1] * inv * bf2f(ww[kd][j + 1]);
-                const float c = bf2f(cs[kd][j]), sn = bf2f(cs[kd][j + 1]);
-                v[kd][j] = f2bf(a * c - b * sn); v[kd][j + 1] = f2bf(b * c + a * sn);
-            }
+        for (int i = 0; i < 2; ++i) s[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(priv, p.off_s + ((which * RTP * 16 + row) * 8 + 4 * i) * 4, 0, SC1));
+        const float f = ld4(priv, p.off_f + row * 4);
+        s[0] += s[1];
+        return f * rsqrtf(f * f * (s[0][0] + s[0][1] + s[0][2] + s[0][3]) * (1.0f / 128.0f) + 1e-6f);
     };
 
     // ---- logits of (query row tile, 16 keys) per wave and their exponentials relative to the row maximum over those 16 keys ----
@@ -499,26 +502,29 @@ void flow_kernel(FlowP kernel_args) {
         for (int i = 0; i < NQ; ++i)
 #pragma unroll
             for (int kd = 0; kd < KD; ++kd) qf[i][kd] = ld16(priv, p.off_q + frag_off(min((w >> 1) + 4 * i, QRT - 1), kd, KD, lane));
-        float fq = 0.f, fk = 0.f;
-        const int tok0 = ((w >> 1) % RTP) * 16 + lr;
-        if constexpr (DM0) fq = ld4(priv, p.off_f + tok0 * 4);                         // (both row tiles of a wave are of the same tokens)
+        float fq[NQ] = {}, fk = 0.f;
+        if constexpr (DM0)
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) {
+                const int rt = min((w >> 1) + 4 * i, QRT - 1);
+                fq[i] = dm0_scale(p, rt / RTP, rt % RTP * 16 + lr);
+            }
         if (r >= KBp) {
             new_k(r);
-            if constexpr (DM0) fk = ld4(priv, p.off_f + key_row(r) * 4);
-        }
-        if constexpr (DM0) {
-            static_assert(NQ == 1 || RTP == 4, "row tiles four apart are of the same tokens");
-#pragma unroll
-            for (int i = 0; i < NQ; ++i) dm0_qk(g, qf[i], fq, tok0, p.qnorm + (size_t)l * 128);
+            if constexpr (DM0) fk = dm0_scale(p, 2, key_row(r));
         }
         for (int kb = r; kb < KB; kb += 32) {
             if (kb >= KBp) {
                 if (kb >= 32) {
                     new_k(kb);
-                    if constexpr (DM0) fk = ld4(priv, p.off_f + key_row(kb) * 4);
+                    if constexpr (DM0) fk = dm0_scale(p, 2, key_row(kb));
                 }
-                if constexpr (DM0) dm0_qk(g, kf, fk, key_row(kb), p.knorm + (size_t)l * 128);
             } else if (kb >= 32) load_k(p, lane, x, l, nt, kb, kf);
+            f32x4 sc = {sc2, sc2, sc2, sc2};
+            if constexpr (DM0)
+                if (kb >= KBp)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sc[e] *= __shfl(fk, 4 * g + e, 64);            // (lane lr has the factor of key lr)
             // the keys of this lane: 4 g .. 4 g + 3 of the 16; visible are those below `lim` (of the state row, among the new keys, only the first)
             const int key = nt * 16 + 4 * g;
             const int lim = kb < KBp ? vl - kb * 32 : rows - (kb - KBp) * 32;
@@ -534,7 +540,7 @@ void flow_kernel(FlowP kernel_args) {
                 float mx = NEG_BIG;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    st[e] = key + e < lm ? st[e] * sc2 : NEG_BIG;
+                    st[e] = key + e < lm ? st[e] * (DM0 ? sc[e] * fq[i] : sc2) : NEG_BIG;
                     mx = fmaxf(mx, st[e]);
                 }
                 mx = rows_max(mx);
@@ -1043,7 +1049,7 @@ size_t flow_layout(FlowP* p, int qtiles, int blocks, int hidden) {
     auto take = [&](size_t bytes) { const int o = (int)at; at += (bytes + 255) & ~(size_t)255; return o; };
     p->off_x = take(128 * 1024 * 2); p->off_xin = take(128 * 1024 * 2);
     p->off_q = take((size_t)std::max(qtiles, 8) * 16 * 256 * 2); p->off_k = take(128 * 256 * 2); p->off_v = take(256 * 128 * 2);
-    p->off_o = take(128 * 256 * 2); p->off_h = take((size_t)128 * hidden * 2); p->off_n = take(128 * 32 * 2); p->off_f = take(128 * 4);
+    p->off_o = take(128 * 256 * 2); p->off_h = take((size_t)128 * hidden * 2); p->off_n = take(128 * 32 * 2); p->off_f = take(128 * 4); p->off_s = take(3 * 128 * 8 * 4);
     p->off_m = take((size_t)qtiles * blocks * 16 * 16); p->off_p = take((size_t)qtiles * blocks * 1024);
     return (at + 4095) & ~(size_t)4095;
 }

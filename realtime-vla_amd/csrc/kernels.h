@@ -199,7 +199,7 @@ struct FlowP {
     // null): rotated queries [8 rows][256] (not DM0), attention output [rows][2048], hidden [rows][hidden_cols32 * 32], input MLP's input [rows][1024]
     bf16_t *out_q, *out_attn, *out_hidden, *out_xin; int hidden_cols32;
     char* priv; size_t priv_stride;            // memory of one XCD's own, 8 of them
-    int off_x, off_xin, off_q, off_k, off_v, off_o, off_h, off_n, off_f, off_m, off_p;
+    int off_x, off_xin, off_q, off_k, off_v, off_o, off_h, off_n, off_f, off_s, off_m, off_p;
     float* part; unsigned part_bytes;          // fp32 partial sums exchanged between the XCDs
     FlowSync* sync;
 };
