@@ -26,8 +26,11 @@
 // slower than none (Pi0, 1 view, chunk 50: forward of one vision layer 6 735 us with it, 6 340 us without); so did weights requested ahead
 // of an exchange (+0.7 us for the up tiles, +0.6 us for qkv), or K / V^T behind the qkv products (+0.1 us).  What pays: the weights of a
 // phase behind the flag of the one before, while the others are waited for; those of the output projection already behind the P V
-// products (-0.3 us), and the down projection's lines touched by the waiting wave during the output projection (-0.2 us), whose exchange
-// takes longer than they do.
+// products (-0.3 us), and lines touched by the waiting wave where nobody waits for the CU's loads: the down projection's during the
+// output projection (-0.2 us), whose exchange takes longer than they do, and the gate tiles' in the qkv phase once its operands have
+// arrived and the products run (Cfg::AHEAD naps of 64 cycles; Pi0 3 views: 8 578 us without, 8 464 us with; half the naps: no gain).  With more
+// than two row tiles per CU the operands come in two passes and the touches cost 0.1 - 0.3 us instead.  DM0's smaller tiles leave room for
+// the up tiles in the P V phase too (gate and up: 1 image 8 787 -> 8 600 us; in Pi0's longer P V phase 0.4 us slower).
 //
 // All workgroups have to be resident at once.  A process keeps one flow kernel per device in flight (rtvla.hip), but another process's
 // may be placed on half of the CUs at the same moment.  So no workgroup starts before all 256 have reported: the last one opens the
@@ -140,11 +143,11 @@ RTVLA_DEVICE f32x4 mfma16k16(bf16x8 a, bf16x8 b, int hi) {
 // what differs between the models' action experts
 template <int MODEL> struct Cfg;
 template <> struct Cfg<FLOW_PI0> {
-    static constexpr int HD = 256, HEADS = 1, AT = 3, ET = 2, EGRP = 16, FK = 2, FWAVES = 8, HID = 512, WD_K32 = 128;
+    static constexpr int HD = 256, HEADS = 1, AT = 3, ET = 2, EGRP = 16, FK = 2, FWAVES = 8, HID = 512, WD_K32 = 128, AHEAD = 13; static constexpr bool UP_AHEAD = false;
 };
 template <> struct Cfg<FLOW_PI05> : Cfg<FLOW_PI0> {};
 template <> struct Cfg<FLOW_DM0> {
-    static constexpr int HD = 128, HEADS = 2, AT = 2, ET = 1, EGRP = 12, FK = 1, FWAVES = 6, HID = 192, WD_K32 = 64;
+    static constexpr int HD = 128, HEADS = 2, AT = 2, ET = 1, EGRP = 12, FK = 1, FWAVES = 6, HID = 192, WD_K32 = 64, AHEAD = 7; static constexpr bool UP_AHEAD = true;
 };
 
 // ALONE: the last launch, of compute waves only: if the program has not run, one workgroup runs it; then the activations of the last layer
@@ -211,10 +214,10 @@ void flow_kernel(FlowP kernel_args) {
                 if (!PI05) { bar(); if (!keep_in) local(); }
             }
             for (int l = layer0; l < layer1; ++l) {
-                bar(); local();                                                // qkv
+                ahead(0, t, l); bar(); local();                                // qkv
                 local();                                                       // logits
-                bar(); local();                                                // P V
-                ahead(l); bar(); local();                                      // output projection, exchange, sum
+                ahead(1, t, l); bar(); local();                                // P V
+                ahead(2, t, l); bar(); local();                                // output projection, exchange, sum
                 bar(); local();                                                // gate, up
                 bar(); local();                                                // down projection, exchange, sum
             }
@@ -248,14 +251,18 @@ void flow_kernel(FlowP kernel_args) {
                  patience.n = 0;
                  bar();
              },
-             [&](int l) __attribute__((always_inline)) {                       // down projection of this layer: this XCD's K slice of two column tiles
+             [&](int k, int t, int l) __attribute__((always_inline)) {
+                 cFlowP& p = prm();
+                 auto touch = [&](const bf16_t* base, int kb) __attribute__((always_inline)) {     // kb KB from base
+                     for (int i = 0; i < (kb + 7) / 8; ++i)
+                         __builtin_amdgcn_global_load_lds((gptr_t)((const char*)base + min((i * 64 + lane) * 128, kb * 1024 - 128)), (lptr_t)(smem + scrap), 4, 0, 0);
+                 };
+                 if (k == 2) {                                                 // down projection of this layer: this XCD's K slice of two column tiles
 #pragma unroll
-                 for (int j = 0; j < 2; ++j) {
-                     cFlowP& p = prm();
-                     const bf16_t* const base = p.wd + (size_t)l * p.wd_stride + ((size_t)(2 * r_ + j) * C::WD_K32 + x * HID32) * 512;
-#pragma unroll
-                     for (int i = 0; i < (HID32 + 7) / 8; ++i)
-                         __builtin_amdgcn_global_load_lds((gptr_t)((const char*)base + min((i * 64 + lane) * 128, HID32 * 1024 - 128)), (lptr_t)(smem + scrap), 4, 0, 0);
+                     for (int j = 0; j < 2; ++j) touch(p.wd + (size_t)l * p.wd_stride + ((size_t)(2 * r_ + j) * C::WD_K32 + x * HID32) * 512, HID32);
+                 } else if (RH <= 2 && (k == 0 || C::UP_AHEAD)) {              // gate, up: one tile of every workgroup, behind the phase's operands
+                     for (int i = 0; i < C::AHEAD * RH; ++i) __builtin_amdgcn_s_sleep(1);
+                     if (r_ < C::HID / 16) touch((k == 0 ? p.wg : p.wu) + (size_t)(PI05 ? t * p.layers + l : l) * p.wg_stride + (size_t)(x * (C::HID / 16) + r_) * 32 * 512, 32);
                  }
              });
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                       // nothing may land in LDS after the workgroup has ended
