@@ -161,7 +161,9 @@ void flow_kernel(FlowP kernel_args) {
     constexpr int QRT = RTP * C::HEADS;                  // row tiles of the queries of one XCD
     constexpr int QRTP = QRT <= 2 ? 2 : QRT <= 4 ? 4 : 8;
     constexpr int KD = C::HD / 32, DT = C::HD / 16, NDT = DT * QRTP / 32;      // d tiles per CU of the P V phase
-    constexpr int MC = RH < 2 ? RH : 2;                  // row tiles per pass of a GEMM phase (registers)
+    // row tiles per pass of a GEMM phase: both of two; of three or four one at a time, which leaves the registers for the pass's loads to be
+    // in flight together (two at a time spill; layer of 1 view, chunk 80: 31.6 -> 28.5 us, Pi05 32.0 -> 28.2; chunk 120: 33.8 -> 33.3)
+    constexpr int MC = RH == 2 ? 2 : 1;
     constexpr int HID32 = C::HID / 32;
     constexpr int AK = (C::AT * RH + 7) / 8, SK = (4 * RH + 7) / 8;            // finished tiles per wave of the qkv and of the 4-column-tile phases
     static_assert(QRT <= 8 && NDT >= 1, "row tiles of one XCD");

@@ -134,6 +134,18 @@ def test_a_forward_on_bad_inputs_leaves_nothing_behind(model, views, prompt, chu
     assert torch.equal(m.forward(*inputs), want) and torch.isfinite(want.float()).all()
 
 
+@pytest.mark.parametrize("model,views,prompt,chunk", [("pi0", 1, 20, 50), ("pi0", 1, 8, 90), ("pi05", 1, 9, 33), ("dm0", 1, 24, 50)])
+def test_values_that_look_like_values_not_there_yet(model, views, prompt, chunk):
+    """The workgroups wait for words that are not all ones: NaNs with every bit set, in the noise, must not be waited for."""
+    m, inputs = policy(model, 870, views, prompt, chunk)
+    want = m.forward(*inputs).clone()
+    ones = torch.full(inputs[-1].shape, -1, dtype=torch.int16, device=inputs[-1].device).view(torch.bfloat16)
+    assert not torch.isfinite(m.forward(*inputs[:-1], ones).float()).any()
+    assert torch.equal(m.forward(*inputs), want)
+    torch.cuda.synchronize()
+    assert m._engine.ctx.flow_status() == (True, 0)
+
+
 @pytest.mark.parametrize("route", [capi.FLOW_RESIDENT, capi.FLOW_LAUNCHES], ids=["resident", "launches"])
 @pytest.mark.parametrize("staged_on", ["device", "host"])
 def test_rows_behind_a_short_prompt_are_not_those_of_a_bad_forward(staged_on, route):
