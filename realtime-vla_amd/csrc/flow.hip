@@ -11,7 +11,8 @@
 // only this XCD touches and is exchanged through its L2: plain stores, loads that pass the L1 (sc1), a barrier of 32 flags.  Only the
 // output and down projections produce sums over XCDs: each XCD writes its fp32 partial through to memory and CU r of every XCD waits
 // for the CUs r of the other seven (8 flags), then sums the tiles those eight produced in a fixed order.  A layer is
-//   qkv | logits + exp | P V | O partial || sum + residual | gate, up | down partial || sum + residual |      (| XCD barrier, || 8-CU barrier)
+//   qkv | logits + exp | P V : O partial || sum + residual | gate, up : down partial || sum + residual |      (| XCD barrier, : values that are
+// their own flags, || exchange between the 8 CUs of one number)
 // Measured on MI355X: XCD barrier 0.35 us (1.02 us with 1 KB stored per workgroup before it and 32 KB read after it, 1.43 us with
 // 64 KB), a barrier over all CUs 1.6 us, a dependent launch 2.3 us empty and 4.4-5.0 us as part of a layer.  Of a layer's 25.7 us
 // (Pi0, one view, chunk 50) 14 are barriers, exchanges and the waits behind them.
@@ -66,6 +67,12 @@ RTVLA_DEVICE bf16x4 ld8(rsrc_t r, int off) { return __builtin_bit_cast(bf16x4, _
 RTVLA_DEVICE float ld4(rsrc_t r, int off) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, SC1)); }
 RTVLA_DEVICE void st8(rsrc_t r, int off, bf16x4 v) { __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, off, 0, 0); }
 RTVLA_DEVICE void st16(rsrc_t r, int off, bf16x8 v) { __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, off, 0, 0); }
+// A value that is its own flag: a word of ones means "not there yet", so a pair of NaNs with this pattern loses a bit of its payload.
+RTVLA_DEVICE void st8_flag(rsrc_t r, int off, bf16x4 v) {
+    u32x2 b = __builtin_bit_cast(u32x2, v);
+    b[0] = min(b[0], ~1u); b[1] = min(b[1], ~1u);
+    __builtin_amdgcn_raw_buffer_store_b64(b, r, off, 0, 0);
+}
 RTVLA_DEVICE int ft_off(int row, int col, int cols32) { return (((row >> 4) * cols32 + (col >> 5)) * 64 + (row & 15) + 16 * ((col & 31) >> 3)) * 16 + (col & 7) * 2; }
 RTVLA_DEVICE int frag_off(int rt, int kb, int cols32, int lane) { return ((rt * cols32 + kb) * 64 + lane) * 16; }
 RTVLA_DEVICE bf16x8 ldw(const bf16_t* tiles, int nb, int kb, int K32p, int lane) { return *(const bf16x8*)(tiles + ((size_t)nb * K32p + kb) * 512 + lane * 8); }
@@ -218,9 +225,9 @@ void flow_kernel(FlowP kernel_args) {
             for (int l = layer0; l < layer1; ++l) {
                 ahead(0, t, l); bar(); local();                                // qkv
                 local();                                                       // logits
-                ahead(1, t, l); bar(); local();                                // P V
+                ahead(1, t, l); bar(); bar();                                  // P V
                 ahead(2, t, l); bar(); local();                                // output projection, exchange, sum
-                bar(); local();                                                // gate, up
+                bar(); bar();                                                  // gate, up
                 bar(); local();                                                // down projection, exchange, sum
             }
             if (end) {
@@ -288,9 +295,12 @@ void flow_kernel(FlowP kernel_args) {
         bar();
     };
 
+    Patience patience;
+    patience.lost = !ALONE && kernel_args.wait_ticks == 0;
+
     // ---- one GEMM phase: NT column tiles x RH row tiles, K of this wave = NK blocks; partial sums to LDS ----
-    // `swap`: tile index from which on the product is taken as rows x columns instead of columns x rows
-    auto gemm = [&]<int NT, int NK>(const bf16x8 (&wt)[NT][NK], int a_base, int a_cols32, int kb0, bool with_sq, int swap) __attribute__((always_inline)) {
+    // `swap`: tile index from which on the product is taken as rows x columns instead of columns x rows; `polled`: the values are their own flags
+    auto gemm = [&]<int NT, int NK>(const bf16x8 (&wt)[NT][NK], int a_base, int a_cols32, int kb0, bool with_sq, int swap, bool polled) __attribute__((always_inline)) {
         FLOW_IDS;
 #pragma unroll
         for (int m0 = 0; m0 < RH; m0 += MC) {
@@ -300,6 +310,22 @@ void flow_kernel(FlowP kernel_args) {
 #pragma unroll
                 for (int i = 0; i < NK; ++i)
                     if (m0 + m < RH) a[m][i] = ld16(priv, a_base + frag_off(half * RH + m0 + m, kb0 + i, a_cols32, lane));
+            if (polled && !ALONE) {                                            // what had not arrived is asked for again
+                for (;;) {
+                    bool missing = false;
+#pragma unroll
+                    for (int m = 0; m < MC; ++m)
+#pragma unroll
+                        for (int i = 0; i < NK; ++i) {
+                            if (m0 + m >= RH) continue;
+                            const u32x4 v = __builtin_bit_cast(u32x4, a[m][i]);
+                            if (__any(max(max(v[0], v[1]), max(v[2], v[3])) == ~0u)) { a[m][i] = ld16(priv, a_base + frag_off(half * RH + m0 + m, kb0 + i, a_cols32, lane)); missing = true; }
+                        }
+                    if (!missing || patience.lost) break;
+                    patience.spin(kernel_args.sync, kernel_args.wait_ticks, lane);
+                }
+                patience.n = 0;
+            }
             f32x4 acc[MC][NT];
 #pragma unroll
             for (int m = 0; m < MC; ++m)
@@ -405,7 +431,7 @@ void flow_kernel(FlowP kernel_args) {
     auto qkv = [&](cFlowP& p, int t, int l, const bf16x8 (&wA)[C::AT][4], const bf16x4 (&pre_cs)[AK]) __attribute__((always_inline)) {
         FLOW_IDS;
         constexpr int NT = C::AT;
-        gemm.template operator()<NT, 4>(wA, p.off_x, 32, w * 4, true, DM0 ? (grp >= 8 ? 1 : 9) : 2);
+        gemm.template operator()<NT, 4>(wA, p.off_x, 32, w * 4, true, DM0 ? (grp >= 8 ? 1 : 9) : 2, false);
         bar();
         if (w < FW) {
 #pragma unroll
@@ -656,7 +682,7 @@ void flow_kernel(FlowP kernel_args) {
             }
             v *= L > 0.f ? 1.0f / L : 0.f;
             const int tok = (prt % RTP) * 16 + lr, col = (prt / RTP) * C::HD + (pdg * NDT + w) * 16 + 4 * g;
-            st8(priv, p.off_o + ft_off(tok, col, 8), pack4(v));
+            st8_flag(priv, p.off_o + ft_off(tok, col, 8), pack4(v));
         }
     };
 
@@ -667,8 +693,6 @@ void flow_kernel(FlowP kernel_args) {
     // e + 2, which a peer only looks at after it has received this workgroup's exchange e + 1, sent behind a wait for those ones.
     // Tile layout: 64 bytes per row, so that the rows past the last one are neither written nor read.
     int ex = 0;                                                                // exchange number modulo 3
-    Patience patience;
-    patience.lost = !ALONE && kernel_args.wait_ticks == 0;
     auto part_off = [&](int buf, int y, int r, int u, int lane) __attribute__((always_inline)) {
         return (((buf * 8 + y) * 32 + r) * (4 * RH) + u) * 1024 + ((lane & 15) * 4 + (lane >> 4)) * 16;
     };
@@ -740,7 +764,7 @@ void flow_kernel(FlowP kernel_args) {
     auto mlp_up = [&](cFlowP& p, int t, int l, const bf16x8 (&wE)[2 * C::ET][4]) __attribute__((always_inline)) {
         FLOW_IDS;
         constexpr int NT = 2 * C::ET;
-        if (C::EGRP == 16 || grp < C::EGRP) gemm.template operator()<NT, 4>(wE, p.off_x, 32, w * 4, true, 9);
+        if (C::EGRP == 16 || grp < C::EGRP) gemm.template operator()<NT, 4>(wE, p.off_x, 32, w * 4, true, 9, false);
         bar();
         if (w < C::ET * RH && (C::EGRP == 16 || grp < C::EGRP)) {
             const int j = w / RH, m = w % RH;
@@ -755,8 +779,21 @@ void flow_kernel(FlowP kernel_args) {
             f32x4 h;
 #pragma unroll
             for (int e = 0; e < 4; ++e) h[e] = (DM0 ? siluf(gv[e]) : gelu_tanh(gv[e])) * uv[e];
-            st8(priv, p.off_h + ft_off((half * RH + m) * 16 + lr, hc, HID32), pack4(h));
+            st8_flag(priv, p.off_h + ft_off((half * RH + m) * 16 + lr, hc, HID32), pack4(h));
         }
+    };
+
+    // The attention output and the hidden activations are their own flags: the GEMM that reads them asks until no word is all ones, which
+    // saves the acknowledgement of the stores, the flag and the second look (forward of Pi0, 1 view, 6 355 -> 6 273 us, DM0, 3 images, 10 060 ->
+    // 9 780; with the residual stream exchanged in the same way, which more CUs look for longer, 6 490).  Behind the flag of the qkv phase everybody has read those
+    // of the layer before (the flags of the exchanges lie between), and they are set to ones again, 1 KB pieces dealt over the XCD's waves;
+    // the flag of the logits phase, which everybody awaits before looking again, is sent behind a wait for these stores.
+    auto reset_values = [&](cFlowP& p) __attribute__((always_inline)) {
+        FLOW_IDS;
+        constexpr int NO = RTP * 8, N = NO + RTP * HID32;
+        static_assert(N <= 256, "one piece per wave");
+        const int i = r * FW + w;
+        if (i < N) __builtin_amdgcn_raw_buffer_store_b128(u32x4{~0u, ~0u, ~0u, ~0u}, priv, (i < NO ? p.off_o + i * 1024 : p.off_h + (i - NO) * 1024) + lane * 16, 0, 0);
     };
 
     // ---- start of a flow step: noise -> input projection (+ SiLU, MLP) -> residual stream ----
@@ -788,7 +825,7 @@ void flow_kernel(FlowP kernel_args) {
     };
     auto mlp_in = [&](cFlowP& p, bool keep, const bf16x8 (&wM)[4][4]) __attribute__((always_inline)) {
         FLOW_IDS;
-        gemm.template operator()<4, 4>(wM, p.off_xin, 32, w * 4, false, 9);
+        gemm.template operator()<4, 4>(wM, p.off_xin, 32, w * 4, false, 9, false);
         bar();
         {
 #pragma unroll
@@ -924,7 +961,7 @@ void flow_kernel(FlowP kernel_args) {
                 each([&]() __attribute__((always_inline)) {
                     bf16x8 wC[4][1];
                     load_c(prm(), l, wC);
-                    gemm.template operator()<4, 1>(wC, prm().off_o, 8, w_, false, 9);
+                    gemm.template operator()<4, 1>(wC, prm().off_o, 8, w_, false, 9, true);
                     bar();
                     store_part(FW, own);
                 });
@@ -933,7 +970,7 @@ void flow_kernel(FlowP kernel_args) {
                 each([&]() __attribute__((always_inline)) {
                     bf16x8 wF[4][C::FK];
                     load_f(prm(), l, wF);
-                    if (C::FWAVES == FW || w_ < C::FWAVES) gemm.template operator()<4, C::FK>(wF, prm().off_h, HID32, w_ * C::FK, false, 9);
+                    if (C::FWAVES == FW || w_ < C::FWAVES) gemm.template operator()<4, C::FK>(wF, prm().off_h, HID32, w_ * C::FK, false, 9, true);
                     bar();
                     store_part(C::FWAVES, own);
                 });
@@ -969,7 +1006,7 @@ void flow_kernel(FlowP kernel_args) {
             qkv(prm(), t, l, wA, cs);
             {
                 bf16x8 kf[KD];
-                sync([&]() __attribute__((always_inline)) { pre_logits(prm(), l, kf); });
+                sync([&]() __attribute__((always_inline)) { pre_logits(prm(), l, kf); reset_values(prm()); });
                 logits(prm(), l, kf);
             }
             bf16x8 wC[4][1];
@@ -981,8 +1018,9 @@ void flow_kernel(FlowP kernel_args) {
             {
                 bf16x8 wE[2 * C::ET][4];
                 f32x4 own[SK];
-                sync([&]() __attribute__((always_inline)) { load_e(prm(), t, l, 0, wE); });
-                gemm.template operator()<4, 1>(wC, prm().off_o, 8, w_, false, 9);
+                load_e(prm(), t, l, 0, wE);
+                bar();                                                         // (LDS: the sums of P V have been read)
+                gemm.template operator()<4, 1>(wC, prm().off_o, 8, w_, false, 9, true);
                 bar();
                 store_part(FW, own);
                 cFlowP& p = prm();
@@ -994,8 +1032,9 @@ void flow_kernel(FlowP kernel_args) {
                 f32x4 own[SK];
                 {
                     bf16x8 wF[4][C::FK];
-                    sync([&]() __attribute__((always_inline)) { load_f(prm(), l, wF); });
-                    if (C::FWAVES == FW || w_ < C::FWAVES) gemm.template operator()<4, C::FK>(wF, prm().off_h, HID32, w_ * C::FK, false, 9);
+                    load_f(prm(), l, wF);
+                    bar();
+                    if (C::FWAVES == FW || w_ < C::FWAVES) gemm.template operator()<4, C::FK>(wF, prm().off_h, HID32, w_ * C::FK, false, 9, true);
                 }
                 bar();
                 store_part(C::FWAVES, own);
