@@ -14,24 +14,24 @@
 //   qkv | logits + exp | P V : O partial || sum + residual | gate, up : down partial || sum + residual |      (| XCD barrier, : values that are
 // their own flags, || exchange between the 8 CUs of one number)
 // Measured on MI355X: XCD barrier 0.35 us (1.02 us with 1 KB stored per workgroup before it and 32 KB read after it, 1.43 us with
-// 64 KB), a barrier over all CUs 1.6 us, a dependent launch 2.3 us empty and 4.4-5.0 us as part of a layer.  Of a layer's 25.7 us
-// (Pi0, one view, chunk 50) 14 are barriers, exchanges and the waits behind them.
+// 64 KB), a barrier over all CUs 1.6 us, a dependent launch 2.3 us empty and 4.4-5.0 us as part of a layer.  About half of a layer's 21.8 us
+// (Pi0, one view, chunk 50) are barriers, exchanges and the waits behind them.
 //
 // A CU holds RH of the 2 RH row tiles (CU parity) and the columns of one of 16 groups, so the activations of a phase are read once
 // into half the CUs each and the weights twice per XCD (once from memory).  The eight compute waves split K and reduce through LDS; a
 // ninth wave does the waiting, so that the compute waves can have the next phase's weights on the way while it polls.
 //
-// When the weights are asked for decides a layer's time more than anything else.  A CU's vector cache returns its loads in the order it
-// got them, whichever wave asked: a line that comes from HBM holds up the flags, activations and partial sums behind it by its 1 - 2 us.
-// A tenth wave that pulled all of the coming phases' weights into L2 (one word per line, spread over the phases) made a layer 2.2 us
-// slower than none (Pi0, 1 view, chunk 50: forward of one vision layer 6 735 us with it, 6 340 us without); so did weights requested ahead
-// of an exchange (+0.7 us for the up tiles, +0.6 us for qkv), or K / V^T behind the qkv products (+0.1 us).  What pays: the weights of a
-// phase behind the flag of the one before, while the others are waited for; those of the output projection already behind the P V
-// products (-0.3 us), and lines touched by the waiting wave where nobody waits for the CU's loads: the down projection's during the
-// output projection (-0.2 us), whose exchange takes longer than they do, and the gate tiles' in the qkv phase once its operands have
-// arrived and the products run (Cfg::AHEAD naps of 64 cycles; Pi0 3 views: 8 578 us without, 8 464 us with; half the naps: no gain).  With more
-// than two row tiles per CU the operands come in two passes and the touches cost 0.1 - 0.3 us instead.  DM0's smaller tiles leave room for
-// the up tiles in the P V phase too (gate and up: 1 image 8 787 -> 8 600 us; in Pi0's longer P V phase 0.4 us slower).
+// When the weights are asked for decides a layer's time more than anything else: a CU has one path to its vector cache, and what is in
+// it goes before the flags, activations and partial sums asked for later.  Loads of whole lines hardly show (a hot line that takes 0.10 us
+// takes 0.15 us beside a wave that streams from HBM), but touching one word of 64 lines holds the path up for all 8 KB of them (0.38 us).
+// A tenth wave that touched all weights of the coming phases, spread over the phases, made a layer 2.2 us slower than none at all (Pi0, 1
+// view, chunk 50: forward with one vision layer 6 735 us with it, 6 340 us without); so did weights requested ahead of an exchange (+0.7 us
+// for the up tiles, +0.6 us for qkv), or K / V^T behind the qkv products (+0.1 us).  What pays: the weights of a phase behind the flag of the
+// one before, while the others are waited for; those of the output projection already behind the P V products (-0.3 us); and touches
+// by the waiting wave, 8 - 32 KB a phase, where nobody waits for the CU's loads: once the phase's operands have arrived and the products run
+// (Cfg::NAP naps of 64 cycles; with half of them half of the gain is gone).  Those are a half of the gate tiles in the qkv phase (DM0: all),
+// the other half in P V (DM0: the up tiles), the down projection's lines during the output projection, and the next layer's query columns during
+// the down projection: 6 340 -> 6 127 us together.  Twice as much in a phase, or the K / V columns too, is slower again.
 //
 // All workgroups have to be resident at once.  A process keeps one flow kernel per device in flight (rtvla.hip), but another process's
 // may be placed on half of the CUs at the same moment.  So no workgroup starts before all 256 have reported: the last one opens the
@@ -150,11 +150,11 @@ RTVLA_DEVICE f32x4 mfma16k16(bf16x8 a, bf16x8 b, int hi) {
 // what differs between the models' action experts
 template <int MODEL> struct Cfg;
 template <> struct Cfg<FLOW_PI0> {
-    static constexpr int HD = 256, HEADS = 1, AT = 3, ET = 2, EGRP = 16, FK = 2, FWAVES = 8, HID = 512, WD_K32 = 128, AHEAD = 13; static constexpr bool UP_AHEAD = false;
+    static constexpr int HD = 256, HEADS = 1, AT = 3, ET = 2, EGRP = 16, FK = 2, FWAVES = 8, HID = 512, WD_K32 = 128, NAP_QKV = 13, NAP = 10;
 };
 template <> struct Cfg<FLOW_PI05> : Cfg<FLOW_PI0> {};
 template <> struct Cfg<FLOW_DM0> {
-    static constexpr int HD = 128, HEADS = 2, AT = 2, ET = 1, EGRP = 12, FK = 1, FWAVES = 6, HID = 192, WD_K32 = 64, AHEAD = 7; static constexpr bool UP_AHEAD = true;
+    static constexpr int HD = 128, HEADS = 2, AT = 2, ET = 1, EGRP = 12, FK = 1, FWAVES = 6, HID = 192, WD_K32 = 64, NAP_QKV = 7, NAP = 7;
 };
 
 // ALONE: the last launch, of compute waves only: if the program has not run, one workgroup runs it; then the activations of the last layer
@@ -228,7 +228,7 @@ void flow_kernel(FlowP kernel_args) {
                 ahead(1, t, l); bar(); bar();                                  // P V
                 ahead(2, t, l); bar(); local();                                // output projection, exchange, sum
                 bar(); bar();                                                  // gate, up
-                bar(); local();                                                // down projection, exchange, sum
+                ahead(3, t, l); bar(); local();                                // down projection, exchange, sum
             }
             if (end) {
                 bar(); bar();
@@ -269,9 +269,15 @@ void flow_kernel(FlowP kernel_args) {
                  if (k == 2) {                                                 // down projection of this layer: this XCD's K slice of two column tiles
 #pragma unroll
                      for (int j = 0; j < 2; ++j) touch(p.wd + (size_t)l * p.wd_stride + ((size_t)(2 * r_ + j) * C::WD_K32 + x * HID32) * 512, HID32);
-                 } else if (RH <= 2 && (k == 0 || C::UP_AHEAD)) {              // gate, up: one tile of every workgroup, behind the phase's operands
-                     for (int i = 0; i < C::AHEAD * RH; ++i) __builtin_amdgcn_s_sleep(1);
-                     if (r_ < C::HID / 16) touch((k == 0 ? p.wg : p.wu) + (size_t)(PI05 ? t * p.layers + l : l) * p.wg_stride + (size_t)(x * (C::HID / 16) + r_) * 32 * 512, 32);
+                 } else {                                                      // behind the phase's operands
+                     for (int i = 0; i < (k == 0 ? C::NAP_QKV : C::NAP) * min(RH, 2); ++i) __builtin_amdgcn_s_sleep(1);
+                     if (k == 3) {                                             // the next layer's query columns: half a tile of every workgroup
+                         const int ln = l + 1 < layer1 ? l + 1 : layer0, tn = l + 1 < layer1 || t + 1 == step1 ? t : t + 1;
+                         touch(p.wqkv + (size_t)(PI05 ? tn * p.layers + ln : ln) * p.wqkv_stride + (size_t)(x * 32 + r_) * 16 * 512, 16);
+                     } else if (r_ < C::HID / 16) {                            // qkv: the gate tiles or their first halves, P V: the others or the up tiles
+                         const size_t o = (size_t)(PI05 ? t * p.layers + l : l) * p.wg_stride + (size_t)(x * (C::HID / 16) + r_) * 32 * 512;
+                         touch((DM0 && k == 1 ? p.wu : p.wg) + o + (DM0 || k == 0 ? 0 : 16 * 512), DM0 ? 32 : 16);
+                     }
                  }
              });
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                       // nothing may land in LDS after the workgroup has ended
