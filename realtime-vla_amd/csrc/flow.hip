@@ -1043,6 +1043,7 @@ void flow_kernel(FlowP kernel_args) {
                     if (C::FWAVES == FW || w_ < C::FWAVES) gemm.template operator()<4, C::FK>(wF, prm().off_h, HID32, w_ * C::FK, false, 9, true);
                 }
                 bar();
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");               // (the ones of reset_part have arrived; nothing else is under way)
                 store_part(C::FWAVES, own);
                 cFlowP& p = prm();
                 sum_residual(p, lastl, own, PI05 ? p.style_ffn + ((size_t)t * p.layers + l) * 3072 + 2048 : nullptr);
