@@ -517,8 +517,22 @@ void flow_kernel(FlowP kernel_args) {
     };
 
     // ---- logits of (query row tile, 16 keys) per wave and their exponentials relative to the row maximum over those 16 keys ----
-    // Workgroup: the 32-key blocks r, r + 32, ...; wave: one half of the block (w & 1), row tiles (w >> 1), + 4
+    // A workgroup takes a 32-key block, a wave one half of it (w & 1) and the row tiles (w >> 1), + 4.  The phase lasts as long as the slowest
+    // workgroup: one with keys that this layer made, which it loads behind the barrier beside the queries.  So where workgroups are left over, two of
+    // them share a block, half of the row tiles each: all blocks if there are at most 16, else those of the new keys.  Blocks past the 32nd are
+    // dealt over the pairs of waves by row tiles, as a second pass.  (Forward with one vision layer, before and after: Pi0 1 view 6 130 ->
+    // 6 056 us, 3 views 8 100 -> 8 042, DM0 1 image 8 299 -> 8 165; 33 blocks 9 112 -> 9 104.)
     constexpr int NQ = (QRT + 3) / 4;
+    auto first_block = [&](int r, int& tb, int& tc) __attribute__((always_inline)) {           // the block (KB: none) and its row tiles
+        tb = 0; tc = QRT;
+        int kb = min(r, KB);
+        const int whole = 2 * KB <= 32 ? 0 : KBp;                              // blocks that are not shared
+        if (whole + 2 * (KB - whole) <= 32 && r >= whole) {
+            kb = min(whole + (r - whole) / 2, KB);
+            tc = QRT / 2; tb = (r - whole) % 2 * tc;
+        }
+        return kb;
+    };
     auto load_k = [&](cFlowP& p, int lane, int x, int l, int nt, int kb, bf16x8 (&kf)[KD]) __attribute__((always_inline)) {
         const bf16_t* base = p.kcache + (size_t)(DM0 ? l * 8 + x : l) * p.kv_stride;
 #pragma unroll
@@ -526,76 +540,81 @@ void flow_kernel(FlowP kernel_args) {
     };
     auto pre_logits = [&](cFlowP& p, int l, bf16x8 (&kf)[KD]) __attribute__((always_inline)) {
         FLOW_IDS;
-        load_k(p, lane, x, l, w & 1, min(r, KBp - 1), kf);
+        int tb, tc;
+        const int kb = first_block(r, tb, tc);
+        load_k(p, lane, x, l, w & 1, min(kb, KBp - 1), kf);
     };
     auto logits = [&](cFlowP& p, int l, bf16x8 (&kf)[KD]) __attribute__((always_inline)) {
         FLOW_IDS;
         const int nt = w & 1;
-        if (r >= KB) return;
+        int tb, tc;
+        const int kb0 = first_block(r, tb, tc);
+        if (kb0 >= KB) return;
         auto new_k = [&](int kb) __attribute__((always_inline)) {
 #pragma unroll
             for (int kd = 0; kd < KD; ++kd) kf[kd] = ld16(priv, p.off_k + frag_off((kb - KBp) * 2 + nt, kd, KD, lane));
         };
-        auto key_row = [&](int kb) __attribute__((always_inline)) { return min(((kb - KBp) * 2 + nt) * 16 + lr, RTP * 16 - 1); };
-        // all that the first block needs is requested before any of it is used
-        bf16x8 qf[NQ][KD];
+        auto key_factor = [&](int kb) __attribute__((always_inline)) { return dm0_scale(p, 2, min(((kb - KBp) * 2 + nt) * 16 + lr, RTP * 16 - 1)); };
+        auto load_q = [&](int rt, bf16x8 (&q)[KD], float& f) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < NQ; ++i)
-#pragma unroll
-            for (int kd = 0; kd < KD; ++kd) qf[i][kd] = ld16(priv, p.off_q + frag_off(min((w >> 1) + 4 * i, QRT - 1), kd, KD, lane));
-        float fq[NQ] = {}, fk = 0.f;
-        if constexpr (DM0)
-#pragma unroll
-            for (int i = 0; i < NQ; ++i) {
-                const int rt = min((w >> 1) + 4 * i, QRT - 1);
-                fq[i] = dm0_scale(p, rt / RTP, rt % RTP * 16 + lr);
-            }
-        if (r >= KBp) {
-            new_k(r);
-            if constexpr (DM0) fk = dm0_scale(p, 2, key_row(r));
-        }
-        for (int kb = r; kb < KB; kb += 32) {
-            if (kb >= KBp) {
-                if (kb >= 32) {
-                    new_k(kb);
-                    if constexpr (DM0) fk = dm0_scale(p, 2, key_row(kb));
-                }
-            } else if (kb >= 32) load_k(p, lane, x, l, nt, kb, kf);
-            f32x4 sc = {sc2, sc2, sc2, sc2};
-            if constexpr (DM0)
-                if (kb >= KBp)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) sc[e] *= __shfl(fk, 4 * g + e, 64);            // (lane lr has the factor of key lr)
+            for (int kd = 0; kd < KD; ++kd) q[kd] = ld16(priv, p.off_q + frag_off(rt, kd, KD, lane));
+            if constexpr (DM0) f = dm0_scale(p, rt / RTP, rt % RTP * 16 + lr);
+        };
+        auto tile = [&](int kb, int rt, const bf16x8 (&q)[KD], float fq, float fk) __attribute__((always_inline)) {
             // the keys of this lane: 4 g .. 4 g + 3 of the 16; visible are those below `lim` (of the state row, among the new keys, only the first)
             const int key = nt * 16 + 4 * g;
             const int lim = kb < KBp ? vl - kb * 32 : rows - (kb - KBp) * 32;
             const int lim_state = kb < KBp ? lim : KBp == kb ? 1 : 0;
+            const int lm = (MODEL == FLOW_PI0 && rt % RTP == 0 && lr == 0) ? lim_state : lim;      // the state token sees the prefix and itself
+            f32x4 st = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < NQ; ++i) {
-                const int rt = (w >> 1) + 4 * i;
-                if (QRT % 4 != 0 && rt >= QRT) continue;
-                const int lm = (MODEL == FLOW_PI0 && rt % RTP == 0 && lr == 0) ? lim_state : lim;      // the state token sees the prefix and itself
-                f32x4 st = {0.f, 0.f, 0.f, 0.f};
+            for (int kd = 0; kd < KD; ++kd) st = mfma16(kf[kd], q[kd], st);
+            f32x4 sc = {sc2, sc2, sc2, sc2};
+            if constexpr (DM0) {
+                if (kb >= KBp)
 #pragma unroll
-                for (int kd = 0; kd < KD; ++kd) st = mfma16(kf[kd], qf[i][kd], st);
-                float mx = NEG_BIG;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    st[e] = key + e < lm ? st[e] * (DM0 ? sc[e] * fq[i] : sc2) : NEG_BIG;
-                    mx = fmaxf(mx, st[e]);
-                }
-                mx = rows_max(mx);
-                float sum = 0.f;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    st[e] = key + e < lm ? __builtin_amdgcn_exp2f(st[e] - mx) : 0.f;
-                    sum += st[e];
-                }
-                sum = rows_sum(sum);
-                // this half's four probabilities of the lane's 16-byte piece of the P^T fragment
-                st8(priv, p.off_p + ((rt * KB + kb) * 64 + lane) * 16 + nt * 8, pack4(st));
-                if (g == 0) __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(mx), __float_as_uint(sum)}, priv, p.off_m + ((rt * KB + kb) * 16 + lr) * 16 + nt * 8, 0, 0);
+                    for (int e = 0; e < 4; ++e) sc[e] *= __shfl(fk, 4 * g + e, 64);                // (lane lr has the factor of key lr)
+                sc *= fq;
             }
+            float mx = NEG_BIG;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                st[e] = key + e < lm ? st[e] * sc[e] : NEG_BIG;
+                mx = fmaxf(mx, st[e]);
+            }
+            mx = rows_max(mx);
+            float sum = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                st[e] = key + e < lm ? __builtin_amdgcn_exp2f(st[e] - mx) : 0.f;
+                sum += st[e];
+            }
+            sum = rows_sum(sum);
+            // this half's four probabilities of the lane's 16-byte piece of the P^T fragment
+            st8(priv, p.off_p + ((rt * KB + kb) * 64 + lane) * 16 + nt * 8, pack4(st));
+            if (g == 0) __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(mx), __float_as_uint(sum)}, priv, p.off_m + ((rt * KB + kb) * 16 + lr) * 16 + nt * 8, 0, 0);
+        };
+        // all that the block needs is requested before any of it is used
+        bf16x8 qf[NQ][KD];
+        float fq[NQ] = {}, fk = 0.f;
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) load_q(tb + min((w >> 1) + 4 * i, tc - 1), qf[i], fq[i]);     // (by every wave: a branch around the loads costs 1 % of a forward)
+        if (kb0 >= KBp) {
+            new_k(kb0);
+            if constexpr (DM0) fk = key_factor(kb0);
+        }
+#pragma unroll
+        for (int i = 0; i < NQ; ++i)
+            if ((w >> 1) + 4 * i < tc) tile(kb0, tb + (w >> 1) + 4 * i, qf[i], fq[i], fk);
+        for (int u = r + 32 * (w >> 1); u < (KB - 32) * QRT; u += 128) {
+            const int kb = 32 + u / QRT, rt = u % QRT;
+            load_q(rt, qf[0], fq[0]);
+            if (kb < KBp) load_k(p, lane, x, l, nt, kb, kf);
+            else {
+                new_k(kb);
+                if constexpr (DM0) fk = key_factor(kb);
+            }
+            tile(kb, rt, qf[0], fq[0], fk);
         }
     };
 

@@ -59,6 +59,14 @@ def test_resident_loop_equals_the_loop_as_launches(model, views, prompt, chunk):
 
 # suffix rows at the ends of every instance's range, a prefix that ends inside a 32-key block, past one round of the attention phases, and
 # a prompt that is shorter than its allocation (Pi05)
+# 32-key blocks of the prefix and of the suffix: 14 + 2 (all shared by two workgroups), 15 + 2, 28 + 2 and 24 + 4 (the suffix's shared), 30 + 2 (none),
+# 31 + 2 and 39 + 4 (blocks past the 32nd), 33 + 2 with two query heads
+@pytest.mark.parametrize("model,views,prompt,chunk", [("pi0", 1, 190, 50), ("pi0", 1, 200, 50), ("pi0", 3, 128, 50), ("pi0", 3, 0, 127), ("pi0", 3, 192, 50), ("pi0", 3, 200, 50),
+                                                      ("pi0", 4, 200, 127), ("pi05", 3, 200, 33), ("dm0", 2, 700, 50)])
+def test_key_blocks_dealt_in_every_way(model, views, prompt, chunk):
+    test_resident_loop_equals_the_loop_as_launches(model, views, prompt, chunk)
+
+
 SHAPES = [("pi0", 1, 5, 9), ("pi0", 1, 31, 50), ("pi0", 1, 7, 95), ("pi0", 4, 40, 127), ("pi05", 1, 9, 32), ("pi05", 1, 32, 64), ("pi05", 2, 21, 96),
           ("pi05", 1, 5, 128), ("dm0", 1, 23, 50), ("dm0", 2, 24, 50)]
 
