@@ -69,6 +69,13 @@ def test_gemma_prefix_pass(tokens):
     run(capi.ATTN_GEMMA_PREFIX, tokens, tokens, 1, seed=tokens)
 
 
+@pytest.mark.parametrize("tokens", [767, 768, 769, 1023, 1024, 1025, 1224])
+def test_gemma_prefix_pass_around_the_row_tiles_of_a_workgroup(tokens):
+    """Half a 16-row tile per token: 384 tiles are the last with one tile per workgroup, 385 (769 tokens: an odd number of tiles
+    for workgroups of two) to 512 take two, 513 one again."""
+    run(capi.ATTN_GEMMA_PREFIX, tokens, tokens, 1, seed=tokens)
+
+
 @pytest.mark.parametrize("tokens,valid", [(820, 789), (820, 1), (300, 288), (64, 64)])
 def test_gemma_prefix_pass_with_a_valid_length_below_the_allocated_prefix(tokens, valid):
     """Pi05: prompt rows past valid_encoder_len are allocated but masked as keys (their own outputs are never read)."""
