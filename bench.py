@@ -7,8 +7,10 @@ already resident in HBM.  Prints ONE JSON line: p50 latency (ms) as `value`, the
 dominant kernel, and the CPU oracle timed on the host cores as a reported baseline.
 """
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -33,10 +35,27 @@ PROFILES = os.path.join(ROOT, "profiles")
 PROFILE_TAGS = {"headline": "pi0_3view_p20_c50"}      # workloads that have counter summaries under profiles/
 
 
-def profiled_traffic(file_name, kernel_desc, workload, lib_version):
+# what each counter summary was recorded of: the files that hold its kernels (csrc/)
+GEGLU_SOURCES = ("gemm.hip", "common.h", "kernels.h")
+FLOW_SOURCES = ("flow.hip", "common.h", "kernels.h")
+
+
+def kernel_digest(sources, csrc=os.path.join(ROOT, "realtime-vla_amd", "csrc")):
+    """A digest of the code in `sources` and of the flags they are built with, comments and white space left out: another kernel has
+    another one, whether or not the library's version was raised with it."""
+    import build
+    h = hashlib.sha256(repr(build.FLAGS).encode())
+    for name in sources:
+        with open(os.path.join(csrc, name)) as f:
+            code = re.sub(r'("(?:\\.|[^"\\])*")|//[^\n]*|/\*.*?\*/', lambda m: m.group(1) or " ", f.read(), flags=re.S)
+        h.update(repr((name, build.EXTRA.get(name), " ".join(code.split()))).encode())
+    return h.hexdigest()[:16]
+
+
+def profiled_traffic(file_name, kernel_desc, workload, lib_version, digest):
     """HBM bytes per launch as recorded in a rocprofv3 counter summary under profiles/ (a line `facts: {json}`), or None
-    when no summary exists for exactly this kernel variant (tile and split as the library reports them), workload and
-    library version: a counter reading of an older kernel says nothing about the current one."""
+    when no summary exists for exactly this kernel variant (tile and split as the library reports them), workload, library version and
+    code (`kernel_digest`): a counter reading of an older kernel says nothing about the current one."""
     path = os.path.join(PROFILES, file_name)
     if not os.path.exists(path):
         return None
@@ -46,7 +65,7 @@ def profiled_traffic(file_name, kernel_desc, workload, lib_version):
                 f = json.loads(line[len("facts:"):])
             except ValueError:
                 return None
-            if f.get("kernel") == kernel_desc and f.get("workload") == workload and f.get("rtvla_version") == lib_version:
+            if (f.get("kernel"), f.get("workload"), f.get("rtvla_version"), f.get("digest")) == (kernel_desc, workload, lib_version, digest):
                 return f.get("traffic_bytes_per_launch")
     return None
 
@@ -325,7 +344,7 @@ def main():
             dst.copy_(src)
         torch.cuda.synchronize()
         print(json.dumps({"probe": name, "launch_ms": ms, "copy_bytes": COPY_PROBE_BYTES, "rtvla_version": lib_version,
-                          "workload": args.config}))
+                          "workload": args.config, "digests": {"prefix geglu": kernel_digest(GEGLU_SOURCES), "action-expert layer": kernel_digest(FLOW_SOURCES)}}))
         return
     # fresh noise every iteration; drawn up front so the timed region holds only forward()
     draws = [syn.observation(seed, views, chunk, device=dev, draw=i % 16)[2] for i in range(16)]
@@ -361,7 +380,6 @@ def main():
     mfma = geglu_flop / (geglu_ms * 1e-3) / 1e12
     # bytes the launch pulls from L2 into the CUs, fixed by its block tile (no operand is reused out of L1): every column block
     # reads the (32-row padded) activations once, every row block the gate and up weights once
-    import re
     bm, bn = (int(v) for v in re.search(r"\[(\d+)x(\d+)", geglu_name).groups())
     m_pad = 32 * ((S_e + 31) // 32)
     l2_bytes = 2.0 * 2048 * ((2 * 16384 // bn) * m_pad + ((m_pad + bm - 1) // bm) * 2 * 16384)
@@ -369,8 +387,9 @@ def main():
                 "achieved": round(mfma, 1), "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(mfma / MFMA_PEAK_TFLOPS, 4),
                 "launch_ms": round(geglu_ms, 4), "launch_ms_cache_warm": round(geglu_warm_ms, 4),
                 # HBM bytes per launch from rocprofv3 FETCH_SIZE + WRITE_SIZE, each calibrated on a 256 MiB copy, as recorded in
-                # profiles/ for exactly this kernel variant and library version (null otherwise)
-                "traffic": profiled_traffic("gemm_geglu_%s_hbm_traffic.md" % PROFILE_TAGS.get(args.config), geglu_name, args.config, lib_version),
+                # profiles/ for exactly this kernel: variant, library version and code (null otherwise)
+                "traffic": profiled_traffic("gemm_geglu_%s_hbm_traffic.md" % PROFILE_TAGS.get(args.config), geglu_name, args.config, lib_version,
+                                            kernel_digest(GEGLU_SOURCES)),
                 "kernel_variant": geglu_name,
                 "algorithmic_bytes": 2.0 * (S_e * 2048 + 2 * 2048 * 16384 + S_e * 16384),
                 # informational: the rate at which the launch draws its operand tiles from L2 (the kernels here top out near 10 TB/s)
@@ -386,7 +405,8 @@ def main():
                     "achieved": round(hbm, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(hbm / HBM_PEAK_GBS, 4),
                     "launch_ms": round(layer_ms, 4), "one_layer_program_ms": round(layer_program_ms, 4),
                     # HBM bytes per layer from rocprofv3 FETCH_SIZE + WRITE_SIZE of a launch over all layers (profiles/)
-                    "traffic": profiled_traffic("action_expert_layer_%s_hbm_traffic.md" % PROFILE_TAGS.get(args.config), "action-expert layer", args.config, lib_version),
+                    "traffic": profiled_traffic("action_expert_layer_%s_hbm_traffic.md" % PROFILE_TAGS.get(args.config), "action-expert layer", args.config, lib_version,
+                                                kernel_digest(FLOW_SOURCES)),
                     "algorithmic_bytes": layer_bytes}
     # whole-forward roofline fraction: (F_vis + F_pre) / P_mfma + B_dec / BW  over the measured p50
     v_l = 1152 * 3456 + 1152 * 1152 + 2 * 1152 * 4304
