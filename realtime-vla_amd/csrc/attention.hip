@@ -606,17 +606,11 @@ int launch_mqa_attention(const AttnP& p0, int variant, hipStream_t s, int* nk) {
     if (p.batch < 1) p.batch = 1;
     if (p.batch_inner < 1) p.batch_inner = 1;
     if (p.group < 1) return 1;
-    // Every workgroup reads all keys, so two row tiles per workgroup halve what the chip reads from L2, and one row tile halves
-    // what a workgroup does between two waits.  One row tile where these blocks lie at most three to two CUs, and again where two
-    // row tiles no longer fit the CUs in one go; two in between, where a second resident workgroup only adds reads.  us with
-    // one / two row tiles, Gemma prefix pass on 256 CUs: 256 tokens (128 / 64 workgroups) 6.5 / 9.2, 532 (266 / 133) 14.0 / 14.7,
-    // 788 (394 / 197) 18.9 / 18.8, 968 (484 / 242) 22.8 / 20.7, 1224 (612 / 306) 37.0 / 42.6.
-    const int tiles = (p.rows + 15) / 16 * p.batch;
-    const bool two = tiles > 384 && (tiles + 1) / 2 <= 256;
+    const bool two = attn_two_row_tiles(variant, p.rows, p.batch);
     switch (variant) {                                          // template: waves, row tiles per workgroup, 16-key tiles per wave round, head width
         case ATTN_PREFIX: return two ? launch_mqa_inst<4, 2, 2, 256>(p, s, nk) : launch_mqa_inst<4, 1, 2, 256>(p, s, nk);
         case ATTN_SUFFIX: return launch_mqa_inst<4, 1, 2, 256>(p, s, nk);
-        case ATTN_GQA128_PREFIX: return launch_mqa_inst<4, 1, 2, 128, true>(p, s, nk);       // causal: blocks of unlike length, small ones fill the CUs better (206 / 607 tokens: 5.6 / 11.1 us; two row tiles: 7.5 / 13.3)
+        case ATTN_GQA128_PREFIX: return two ? launch_mqa_inst<4, 2, 2, 128, true>(p, s, nk) : launch_mqa_inst<4, 1, 2, 128, true>(p, s, nk);
         case ATTN_GQA128_SUFFIX: return launch_mqa_inst<4, 1, 2, 128>(p, s, nk);
     }
     return 2;

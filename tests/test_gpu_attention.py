@@ -69,11 +69,37 @@ def test_gemma_prefix_pass(tokens):
     run(capi.ATTN_GEMMA_PREFIX, tokens, tokens, 1, seed=tokens)
 
 
-@pytest.mark.parametrize("tokens", [767, 768, 769, 1023, 1024, 1025, 1224])
+@pytest.mark.parametrize("tokens", [681, 682, 683, 767, 768, 769, 1023, 1024, 1025, 1224, 1536, 1537])
 def test_gemma_prefix_pass_around_the_row_tiles_of_a_workgroup(tokens):
-    """Half a 16-row tile per token: 384 tiles are the last with one tile per workgroup, 385 (769 tokens: an odd number of tiles
-    for workgroups of two) to 512 take two, 513 one again."""
+    """Half a 16-row tile per token: 341 tiles are the last with one tile per workgroup, 342 (683 tokens) to 512 take two (an odd number
+    of tiles among them), 513 to 768 one again, 769 two."""
     run(capi.ATTN_GEMMA_PREFIX, tokens, tokens, 1, seed=tokens)
+
+
+@pytest.mark.parametrize("tokens", [848, 849, 864, 1201])
+def test_causal_prefix_pass_around_the_row_tiles_of_a_workgroup(tokens):
+    """Eight heads of an eighth of a 16-row tile per token: 848 tiles are the last with one tile per workgroup, 849 tokens give 107 tiles a head."""
+    run(capi.ATTN_GQA128_PREFIX, tokens, tokens, 8, seed=tokens)
+
+
+# (tokens, row tiles per workgroup): one where that was the faster, which it was not for long passes
+@pytest.mark.parametrize("model,views,sizes", [("pi0", 1, [(256, 1), (682, 1), (683, 2)]), ("pi0", 4, [(1024, 2), (1025, 1), (1536, 1), (1537, 2), (2048, 2)]),
+                                               ("dm0", 1, [(177, 1), (848, 1), (849, 2), (2107, 2)])])
+def test_long_prefix_passes_take_two_row_tiles(model, views, sizes):
+    """A workgroup with one row tile reads all keys for 16 rows: past about 1 600 (DM0: 850) tokens that is 10 - 30 % slower than for 32."""
+    import synthetic as syn
+    for tokens, tiles in sizes:
+        if model == "pi0":
+            from pi0_infer import Pi0Inference
+            prompt = tokens - 256 * views
+            m = Pi0Inference(syn.pi0_checkpoint(11, prompt, "cuda:0", vision_layers=1, llm_layers=2), views, 8)
+        else:
+            from dm0_infer import DM0Inference
+            m = DM0Inference(syn.dm0_checkpoint(11, "cuda:0", 1, 2, vocab=64), num_images=views, max_lang_len=tokens - 169 * views)
+        stream, names = torch.cuda.current_stream().cuda_stream, []
+        while (r := m._engine.ctx.time_launch(capi.STAGE_PREFIX_LAYER, 0, 0, len(names), 1, stream)) is not None:
+            names.append(r[1])
+        assert "prefix attn [%d rows]" % (16 * tiles) in names, (tokens, names)
 
 
 @pytest.mark.parametrize("tokens,valid", [(820, 789), (820, 1), (300, 288), (64, 64)])
