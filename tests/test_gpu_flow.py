@@ -16,18 +16,22 @@ from _engine import tile_ft, tile_vt, untile_ft, untile_vt
 pytestmark = pytest.mark.gpu
 
 
-def policy(model, seed, views, prompt, chunk):
-    """(policy, arguments of its forward) at one ViT layer and two decoder layers"""
+def policy(model, seed, views, prompt, chunk, change=lambda checkpoint: None):
+    """(policy, arguments of its forward) at one ViT layer and two decoder layers, of the seeded checkpoint after `change`"""
     if model == "dm0":
         from dm0_infer import DM0Inference
         ck = syn.dm0_checkpoint(seed, "cuda:0", 1, 2, vocab=300)
+        change(ck)
         return DM0Inference(ck, num_images=views, max_lang_len=prompt), syn.dm0_observation(seed, views, "cuda:0", max_lang_len=prompt, vocab=300)
     images, state, noise = syn.observation(seed, views, chunk, "cuda:0")
     if model == "pi0":
         from pi0_infer import Pi0Inference
-        return Pi0Inference(syn.pi0_checkpoint(seed, prompt, "cuda:0", vision_layers=1, llm_layers=2, norms="random"), views, chunk), (images, state, noise)
+        ck = syn.pi0_checkpoint(seed, prompt, "cuda:0", vision_layers=1, llm_layers=2, norms="random")
+        change(ck)
+        return Pi0Inference(ck, views, chunk), (images, state, noise)
     from pi05_infer import Pi05Inference
     ck = syn.pi05_checkpoint(seed, prompt - 3, "cuda:0", state_tokens=3, vision_layers=1, llm_layers=2, norms="random")
+    change(ck)
     return Pi05Inference(ck, views, chunk, discrete_state_input=False), (images, noise)
 
 
@@ -57,16 +61,68 @@ def test_resident_loop_equals_the_loop_as_launches(model, views, prompt, chunk):
     assert torch.equal(m.forward(*inputs).float().cpu(), resident)
 
 
-# suffix rows at the ends of every instance's range, a prefix that ends inside a 32-key block, past one round of the attention phases, and
-# a prompt that is shorter than its allocation (Pi05)
 # 32-key blocks of the prefix and of the suffix: 14 + 2 (all shared by two workgroups), 15 + 2, 28 + 2 and 24 + 4 (the suffix's shared), 30 + 2 (none),
-# 31 + 2 and 39 + 4 (blocks past the 32nd), 33 + 2 with two query heads
-@pytest.mark.parametrize("model,views,prompt,chunk", [("pi0", 1, 190, 50), ("pi0", 1, 200, 50), ("pi0", 3, 128, 50), ("pi0", 3, 0, 127), ("pi0", 3, 192, 50), ("pi0", 3, 200, 50),
-                                                      ("pi0", 4, 200, 127), ("pi05", 3, 200, 33), ("dm0", 2, 700, 50)])
+# 31 + 2 and 39 + 4 (blocks past the 32nd), 31 + 2 with adaptive norms, 33 + 2 with two query heads
+BLOCKS = [("pi0", 1, 190, 50), ("pi0", 1, 200, 50), ("pi0", 3, 128, 50), ("pi0", 3, 0, 127), ("pi0", 3, 192, 50), ("pi0", 3, 200, 50),
+          ("pi0", 4, 200, 127), ("pi05", 3, 200, 50), ("dm0", 2, 700, 50)]
+
+
+@pytest.mark.parametrize("model,views,prompt,chunk", BLOCKS + [("pi05", 3, 200, 33)])
 def test_key_blocks_dealt_in_every_way(model, views, prompt, chunk):
     test_resident_loop_equals_the_loop_as_launches(model, views, prompt, chunk)
 
 
+@pytest.mark.parametrize("model,views,prompt,chunk", BLOCKS)
+@pytest.mark.parametrize("limits", [(-1, -1), (0, 0)], ids=["resident", "one workgroup"])
+def test_every_key_block_counts_once(model, views, prompt, chunk, limits):
+    """One layer whose values tell the keys apart: V of prefix key k is the (k / 16)th unit vector and V of the suffix zero, so that the attention output
+    is the probability of every 16 prefix keys."""
+    heads, width = (16, 128) if model == "dm0" else (8, 256)                 # query heads; columns of one
+    new_v = slice(3072, 4096) if model == "dm0" else slice(2304, 2560)
+    m, inputs = policy(model, 970, views, prompt, chunk, lambda ck: ck["decoder_attn_qkv_w"][:, :, new_v].zero_())
+    e = m._engine
+    m.forward(*inputs)
+    prefix, rows = views * (169 if model == "dm0" else 256) + prompt, chunk + (model == "pi0")
+    x, cache = e.buffers["decoder_x"].clone(), e.buffers["kv_Vt" if model == "dm0" else "encoder_Vt"]
+    keys_pad = cache.numel() // (2 * width * (8 if model == "dm0" else 1))   # (two layers)
+    key = torch.arange(keys_pad, device="cuda:0")
+    marked = tile_vt(((key // 16 == torch.arange(width, device="cuda:0")[:, None]) & (key < prefix)).to(torch.bfloat16))
+    e.ctx.flow_limits(*limits)
+
+    def probabilities(route):
+        e.ctx.set_flow_route(route)
+        cache.view(-1, marked.numel()).copy_(marked)
+        e.buffers["decoder_x"].copy_(x)
+        e.buffers["decoder_attn"].zero_()
+        e.run_stage(capi.STAGE_SUFFIX_LAYER, 1, 4)
+        torch.cuda.synchronize()
+        assert e.ctx.flow_status()[0] == (route == capi.FLOW_RESIDENT)
+        attn = e.buffers["decoder_attn"]
+        return untile_ft(attn, attn.numel() // 2048, 2048)[:rows].double().cpu().view(rows, heads, width)
+
+    # of 16 keys for a head, over the rows, relative: either route rounds it to bf16 (2^-9 at most, twice 2^-9 between two) after adding up 16
+    # probabilities rounded to bf16 (2^-9 each, independent: a quarter of that)
+    def differ(got, want):
+        return ((got - want).norm(dim=0) / want.norm(dim=0).clamp_min(1e-30)).max().item() > 5e-3
+
+    got, want = probabilities(capi.FLOW_RESIDENT), probabilities(capi.FLOW_LAUNCHES)
+    halves = (prefix + 15) // 16
+    assert (want[:, :, :halves].norm(dim=0) > 0).all() and not want[:, :, halves:].any() and not got[:, :, halves:].any()
+    assert not differ(got, want)
+    # what a mistake would look like: 16 keys, all 32 of a block or the smallest block of the suffix left out or counted twice
+    of_suffix = 1 - want.sum(dim=2, keepdim=True)
+    smallest = of_suffix * min(32, (rows - 1) % 32 + 1) / rows
+    for times in (-1, 1):
+        assert differ(want / (1 + times * smallest), want)
+        for size in (1, 2):
+            for j in range(0, halves, size):
+                wrong = want.clone()
+                wrong[:, :, j:j + size] *= 1 + times
+                assert differ(wrong / (1 + times * want[:, :, j:j + size].sum(dim=2, keepdim=True)), want)
+
+
+# suffix rows at the ends of every instance's range, a prefix that ends inside a 32-key block, past one round of the attention phases, and
+# a prompt that is shorter than its allocation (Pi05)
 SHAPES = [("pi0", 1, 5, 9), ("pi0", 1, 31, 50), ("pi0", 1, 7, 95), ("pi0", 4, 40, 127), ("pi05", 1, 9, 32), ("pi05", 1, 32, 64), ("pi05", 2, 21, 96),
           ("pi05", 1, 5, 128), ("dm0", 1, 23, 50), ("dm0", 2, 24, 50)]
 
@@ -202,7 +258,7 @@ def test_launches_after_a_loop_in_one_workgroup(model):
 
 
 @pytest.mark.parametrize("model,views,prompt,chunk", [("pi0", 1, 20, 50), ("pi0", 1, 3, 31), ("pi0", 2, 8, 127), ("pi05", 1, 32, 33), ("pi05", 1, 9, 128),
-                                                      ("dm0", 1, 24, 50), ("dm0", 1, 23, 50)])
+                                                      ("dm0", 1, 24, 50), ("dm0", 1, 23, 50)] + BLOCKS[1:])
 @pytest.mark.parametrize("limits", [(-1, -1), (0, 0)], ids=["resident", "one workgroup"])
 def test_the_activations_are_left_where_the_launches_leave_them(model, views, prompt, chunk, limits):
     """One input projection and one layer from the same stream and noise by either route: what `buffers` and `reference_buffer` show of them."""
