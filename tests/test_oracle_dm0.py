@@ -128,6 +128,37 @@ def test_llm_rope_table_and_qknorm_split_against_loops(ck):
             assert torch.allclose(got, out, atol=1e-5)
 
 
+@pytest.mark.parametrize("scale,factor,outliers", [(1.0, 1.0, 1.0), (5.0, 0.3, 1.0), (0.05, 12.0, 1.0), (1e-3, 1.0, 1.0), (1.0, 0.5, 30.0)],
+                         ids=["one", "large", "small", "near epsilon", "outlier features"])
+def test_norm_of_queries_and_keys_as_a_scalar_of_the_logit(scale, factor, outliers):
+    """The resident flow kernel rounds queries and keys to bf16 with norm weight and rotary embedding but without the row's RMS factor and head norm,
+    which it applies to the logit in fp32; the launches (and this oracle) round the finished rows.  The same roundings in number, each
+    relative to the value: against 64 bits the logits are no further off, though their bits differ."""
+    rows = 256
+    g = torch.Generator().manual_seed(int(scale * 1000))
+    bf16 = lambda x: x.bfloat16().double()
+    qkv = torch.randn(rows, 32, 128, generator=g) * scale
+    qkv[:, :, 5::16] *= outliers
+    qkv, factor = bf16(qkv).reshape(rows, 4096), torch.rand(rows, 1, generator=g).double() + factor
+    qw, kw = (bf16(1 + 0.1 * torch.randn(128, generator=g)) for _ in range(2))
+    table = dm0.rope_table(300, rows).bfloat16().double()
+    logits = lambda q, k: torch.einsum("qhgd,khd->hgqk", q.view(rows, 8, 2, 128), k)
+    q, k, _ = dm0.qknorm_rope_split(qkv, factor, qw, kw, table, lambda x: x)
+    exact = logits(q, k)
+    q, k, _ = dm0.qknorm_rope_split(qkv, factor, qw, kw, table, bf16)
+    before = logits(q, k)
+
+    def scaled(rnd):
+        raw = [(t, w) for t, w in ((qkv[:, :2048].view(rows, 16, 128), qw), (qkv[:, 2048:3072].view(rows, 8, 128), kw))]
+        (q, k), (fq, fk) = zip(*((rnd(dm0._rope_heads(t * w, table)), factor * torch.rsqrt(factor ** 2 * (t * t).mean(-1) + 1e-6)) for t, w in raw))
+        return logits(q, k) * fq.view(rows, 8, 2).permute(1, 2, 0)[..., None] * fk.t()[:, None, None, :]
+    off = lambda got: ((got - exact).norm() / exact.norm()).item()
+    assert off(scaled(lambda x: x)) < 1e-12
+    # (measured 0.995 - 1.004 of each other; the bound: two factors, each off by 2^-9 at most)
+    assert off(scaled(bf16)) <= 1.02 * off(before) and off(before) < 4e-3
+    assert not torch.equal(scaled(bf16), before)
+
+
 def test_grouped_query_attention_against_sdpa():
     rows = 9
     q, k, v = torch.randn(rows, 16, 128), torch.randn(rows, 8, 128), torch.randn(rows, 8, 128)
