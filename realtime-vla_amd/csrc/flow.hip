@@ -29,9 +29,9 @@
 // for the up tiles, +0.6 us for qkv), or K / V^T behind the qkv products (+0.1 us).  What pays: the weights of a phase behind the flag of the
 // one before, while the others are waited for; those of the output projection already behind the P V products (-0.3 us); and touches
 // by the waiting wave, 8 - 32 KB a phase, where nobody waits for the CU's loads: once the phase's operands have arrived and the products run
-// (Cfg::NAP naps of 64 cycles; with half of them half of the gain is gone).  Those are a half of the gate tiles in the qkv phase (DM0: all),
-// the other half in P V (DM0: the up tiles), the down projection's lines during the output projection, and the next layer's query columns during
-// the down projection: 6 340 -> 6 127 us together.  Twice as much in a phase, or the K / V columns too, is slower again.
+// (Cfg::NAP).  Those are a half of the gate tiles in the qkv phase (DM0: all), the other half in P V (DM0: the up tiles), the down projection's
+// lines during the output projection, and the next layer's query columns during the down projection: 6 340 -> 6 127 us together.  Twice as much in a
+// phase, or the K / V columns too, is slower again.
 //
 // All workgroups have to be resident at once.  A process keeps one flow kernel per device in flight (rtvla.hip), but another process's
 // may be placed on half of the CUs at the same moment.  So no workgroup starts before all 256 have reported: the last one opens the
@@ -147,14 +147,17 @@ RTVLA_DEVICE f32x4 mfma16k16(bf16x8 a, bf16x8 b, int hi) {
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a4), __builtin_bit_cast(s16x4, b4), f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 }
 
-// what differs between the models' action experts
+// What differs between the models' action experts.  NAP: naps of 64 cycles before the touches of a phase, whatever the number of rows.  Forward
+// with one vision layer, us, without naps / a half / as they are / twice as many: Pi0, 1 view, chunk 20 5 549 / 5 477 / 5 431 / 5 644, chunk 50 6 181 /
+// 6 154 / 6 028 / 6 193, Pi05, 2 views, chunk 25 6 659 / 6 592 / 6 534 / 6 757, DM0, 1 image 8 308 / 8 292 / 8 100 / 8 343; with three and
+// four row tiles per CU they make next to no difference (Pi0, 1 view, chunk 80 7 348 / 7 347 / 7 366 / 7 272, chunk 120 8 290 / 8 305 / 8 299 / 8 284).
 template <int MODEL> struct Cfg;
 template <> struct Cfg<FLOW_PI0> {
-    static constexpr int HD = 256, HEADS = 1, AT = 3, ET = 2, EGRP = 16, FK = 2, FWAVES = 8, HID = 512, WD_K32 = 128, NAP_QKV = 13, NAP = 10;
+    static constexpr int HD = 256, HEADS = 1, AT = 3, ET = 2, EGRP = 16, FK = 2, FWAVES = 8, HID = 512, WD_K32 = 128, NAP_QKV = 26, NAP = 20;
 };
 template <> struct Cfg<FLOW_PI05> : Cfg<FLOW_PI0> {};
 template <> struct Cfg<FLOW_DM0> {
-    static constexpr int HD = 128, HEADS = 2, AT = 2, ET = 1, EGRP = 12, FK = 1, FWAVES = 6, HID = 192, WD_K32 = 64, NAP_QKV = 7, NAP = 7;
+    static constexpr int HD = 128, HEADS = 2, AT = 2, ET = 1, EGRP = 12, FK = 1, FWAVES = 6, HID = 192, WD_K32 = 64, NAP_QKV = 14, NAP = 14;
 };
 
 // ALONE: the last launch, of compute waves only: if the program has not run, one workgroup runs it; then the activations of the last layer
@@ -169,7 +172,8 @@ void flow_kernel(FlowP kernel_args) {
     constexpr int QRTP = QRT <= 2 ? 2 : QRT <= 4 ? 4 : 8;
     constexpr int KD = C::HD / 32, DT = C::HD / 16, NDT = DT * QRTP / 32;      // d tiles per CU of the P V phase
     // row tiles per pass of a GEMM phase: both of two; of three or four one at a time, which leaves the registers for the pass's loads to be
-    // in flight together (two at a time spill; layer of 1 view, chunk 80: 31.6 -> 28.5 us, Pi05 32.0 -> 28.2; chunk 120: 33.8 -> 33.3)
+    // in flight together (layer of 1 view, chunk 80: 31.6 -> 28.5 us, Pi05 32.0 -> 28.2; chunk 120: 33.8 -> 33.3).  Vector registers spilled
+    // with two / one at a time: Pi0 with three row tiles 48 / 26, with four 18 / 0, Pi05 12 / 0 and 0 / 0; all other instances none.
     constexpr int MC = RH == 2 ? 2 : 1;
     constexpr int HID32 = C::HID / 32;
     constexpr int AK = (C::AT * RH + 7) / 8, SK = (4 * RH + 7) / 8;            // finished tiles per wave of the qkv and of the 4-column-tile phases
@@ -270,7 +274,7 @@ void flow_kernel(FlowP kernel_args) {
 #pragma unroll
                      for (int j = 0; j < 2; ++j) touch(p.wd + (size_t)l * p.wd_stride + ((size_t)(2 * r_ + j) * C::WD_K32 + x * HID32) * 512, HID32);
                  } else {                                                      // behind the phase's operands
-                     for (int i = 0; i < (k == 0 ? C::NAP_QKV : C::NAP) * min(RH, 2); ++i) __builtin_amdgcn_s_sleep(1);
+                     for (int i = 0; i < (k == 0 ? C::NAP_QKV : C::NAP); ++i) __builtin_amdgcn_s_sleep(1);
                      if (k == 3) {                                             // the next layer's query columns: half a tile of every workgroup
                          const int ln = l + 1 < layer1 ? l + 1 : layer0, tn = l + 1 < layer1 || t + 1 == step1 ? t : t + 1;
                          touch(p.wqkv + (size_t)(PI05 ? tn * p.layers + ln : ln) * p.wqkv_stride + (size_t)(x * 32 + r_) * 16 * 512, 16);
