@@ -392,7 +392,7 @@ def main():
                                             kernel_digest(GEGLU_SOURCES)),
                 "kernel_variant": geglu_name,
                 "algorithmic_bytes": 2.0 * (S_e * 2048 + 2 * 2048 * 16384 + S_e * 16384),
-                # informational: the rate at which the launch draws its operand tiles from L2 (the kernels here top out near 10 TB/s)
+                # informational: the rate at which the launch draws its operand tiles from L2
                 "l2_to_cu": {"bytes": l2_bytes, "tb_per_s": round(l2_bytes / (geglu_ms * 1e-3) / 1e12, 2)}}
     # the action-expert side: the layers of one flow step in one launch of the resident kernel, divided by their number
     layer_ms = ctx.time_stage(capi.STAGE_SUFFIX_LAYER, -1, 0, 5, stream)          # all 18 layers in turn: weights cold, as in the forward

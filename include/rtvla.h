@@ -181,9 +181,9 @@ int rtvla_graph_launch(rtvla_ctx* ctx, void* hip_stream);
  * the device at the same moment.  While kernels of other processes or streams hold some, its first launch waits `first_ms` (default 5 - 20)
  * and its second `second_ms` (200 - 350) for all of its workgroups to be placed; a loop that has begun waits `wait_ms` (2000) for a
  * workgroup that does not answer.  If none of them finishes, one workgroup runs the whole loop by itself: the same actions bit for bit, in
- * about a second instead of 5 - 7 ms.  No forward is lost.  0: does not wait at all, negative: the default. */
+ * about a second instead of 4 - 6 ms.  No forward is lost.  0: does not wait at all, negative: the default. */
 int rtvla_flow_limits(rtvla_ctx* ctx, float first_ms, float second_ms, float wait_ms);
-/* The flow loop exists as launches too: a quarter longer (Pi0 5.8 ms instead of 4.7), but any number of compute units will do.  RTVLA_FLOW_AUTO takes them under a
+/* The flow loop exists as launches too: half as long again (Pi0 5.5 ms instead of 3.9, DM0 8.8 instead of 5.5), but any number of compute units will do.  RTVLA_FLOW_AUTO takes them under a
  * caller's own capture, on a stream whose CU mask leaves out part of the device, and for the forwards after one whose loop had to run in one
  * workgroup (64 of them, more if that happens again).  RTVLA_FLOW_RESIDENT leaves out the last of these, RTVLA_FLOW_LAUNCHES takes nothing
  * else.  The two differ by roundings of the bf16 stream.  Applies to what is enqueued from here on. */

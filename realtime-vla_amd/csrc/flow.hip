@@ -14,8 +14,8 @@
 //   qkv | logits + exp | P V : O partial || sum + residual | gate, up : down partial || sum + residual |      (| XCD barrier, : values that are
 // their own flags, || exchange between the 8 CUs of one number)
 // Measured on MI355X: XCD barrier 0.35 us (1.02 us with 1 KB stored per workgroup before it and 32 KB read after it, 1.43 us with
-// 64 KB), a barrier over all CUs 1.6 us, a dependent launch 2.3 us empty and 4.4-5.0 us as part of a layer.  About half of a layer's 21.8 us
-// (Pi0, one view, chunk 50) are barriers, exchanges and the waits behind them.
+// 64 KB), a barrier over all CUs 1.6 us, a dependent launch 2.3 us empty and 4.4-5.0 us as part of a layer.  Of a layer's 21 us
+// (Pi0, one view, chunk 50) 6.4 are waits for flags and 5.0 the two exchanges.
 //
 // A CU holds RH of the 2 RH row tiles (CU parity) and the columns of one of 16 groups, so the activations of a phase are read once
 // into half the CUs each and the weights twice per XCD (once from memory).  The eight compute waves split K and reduce through LDS; a
@@ -41,7 +41,7 @@
 // waiting, so the grid always drains.  Nothing makes the two launches succeed: kernels of others may hold the CUs for as long as they like.  The last launch
 // (flow_kernel<.., ALONE>) therefore runs the same program in ONE workgroup, which waits for nobody, if neither finished: the phases one
 // after another for the 256 (XCD, number) pairs, with the same sums in the same order, hence the same bits.  That takes 0.7 - 1.0 s
-// instead of 5 - 7 ms; otherwise it ends at once (a forward of 8.33, 10.72 or 13.43 ms takes the same with and without it).  The input noise and
+// instead of 4 - 6 ms; otherwise it ends at once (a forward of 8.33, 10.72 or 13.43 ms takes the same with and without it).  The input noise and
 // the stream a program starts from are copies that flow_init_kernel made, so that an unfinished launch cannot spoil them.
 #include "kernels.h"
 #include <algorithm>
