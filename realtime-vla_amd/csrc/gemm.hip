@@ -480,7 +480,7 @@ int launch_epi(const GemmP& p, int tile, hipStream_t s) {
 
 }  // namespace
 
-int gemm_tile_bm(int tile) { static const int v[TILE_COUNT] = {224, 192, 160, 128, 64, 64, 128, 256, 224, 192, 128, 96}; return v[tile]; }
+int gemm_tile_bm(int tile) { static const int v[TILE_COUNT + 1] = {224, 192, 160, 128, 64, 64, 128, 256, 224, 192, 128, 96, 160}; return v[tile]; }
 int gemm_tile_bn(int tile) { return (tile == TILE_64x128 || tile == TILE_128x128 || tile == TILE_96x128) ? 128 : 256; }
 
 int launch_gemm(const GemmP& p, int epi, int tile, hipStream_t s) {

@@ -156,24 +156,30 @@ constexpr int64_t ATTN_PARTIAL_FLOATS = 64 * 16 * (16 * 64 * 4 + 32);   // 64 ro
 // one, and needed a table for two shapes (SigLIP down-projection at 768 rows, output projection at 1 024) that are within 0.7 us of the best now.  Layer
 // times: SigLIP down-projection at 512 rows 64x128/6 -> 96x128/4 69.4 -> 65.8 us, at 1 024 rows 64x128/2 -> 128x128/3 93.7 -> 89.5; Gemma
 // down-projection at 868 rows 128x128/2 -> 128x256/4 247.7 -> 236.1, output projection at 649 rows 64x128/2 -> 96x128/2 205.2 -> 200.7.
-TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittable, const char* what, bool eight = false, bool scattered = false) {
+TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittable, const char* what, bool eight = false, bool scattered = false, bool activation = false) {
     static const int tiles[] = {TILE_224x256, TILE_192x256, TILE_160x256, TILE_128x256, TILE_64x256, TILE_128x128, TILE_96x128, TILE_64x128};
     static const int splits[] = {1, 2, 3, 4, 6, 8};
     { TileChoice forced; if (tuning_forced_tile(what, splittable, &forced.tile, &forced.nsplit)) return forced; }
-    // measured (M = 8115, K = 1024, N = 4096, bias + GELU): the eight-wave 256 x 256 tile takes 84-89 us where the best four-wave
-    // tile takes 93-101 us, N = 3072 with the ViT QKV epilogue 77 us against 79-93 us; with 788 rows, with the gated epilogues and with fp32
-    // split-K partials the four-wave tiles win.  Of the eight-wave tiles the one whose rounds of 256 workgroups cost the fewest row tiles,
-    // one more per round for its ramp (5 440 rows: N = 4096 256 rows 66.3 -> 192 rows 59.4 us, N = 3072 128 rows 66.8 -> 192 rows 60.2 us)
-    if (eight && M >= 4096 && stages <= 32 && ncols16 >= 128) {
-        TileChoice c8{TILE8_256x256, 1};
-        int least = 1 << 30;
-        for (int tile : {TILE8_256x256, TILE8_224x256, TILE8_192x256}) {
-            const int cols = (ncols16 + 15) / 16, row_tiles = (M + 31) / 32;
-            const int m_blocks = gemm8_row_blocks(row_tiles, gemm_tile_bm(tile) / 32, cols);
-            const int cost = (m_blocks * cols + 255) / 256 * ((row_tiles + m_blocks - 1) / m_blocks + 1);
-            if (cost < least) { least = cost; c8.tile = tile; }
+    // The eight-wave tiles (csrc/gemm8.hip) win where their workgroups fill the chip and the weights are read for many rows.  us, four / eight waves,
+    // weights cold: 8 160 x 1 024 x 1 024 23.6 / 18.7, 2 720 x 1 024 x 3 072 35 / 21, but 2 720 x 1 024 x 1 024 (88 workgroups of 128 rows) 11.5 / 14.5 and 2 028 x 9 216 x 2 048
+    // (128) 89 / 134.  The gated GEMMs are held by the clock that their MFMAs leave (GeGLU with K = 2 048, N = 16 384, by itself: 532 rows 81.4 / 83.2, 788 109 / 102;
+    // a forward with 788 takes the same with both, 10 053 / 10 057 us), unless 256 rows to a workgroup save a round that 224 need (968 rows: 131 / 116, forward 11 150 / 10 954).
+    // Among them the one whose rounds of 256 workgroups cost least: a K stage of 32 takes 0.36 us + 0.0155 us per row tile (8 160 x 4 096 x 1 024 against
+    // K = 1 024), first loads and epilogue 1.6 us per row tile - 1.8 us, 2.4 us - 2 us with an activation.
+    if (eight && M >= 640) {
+        const int cols = (ncols16 + (dual ? 7 : 15)) / (dual ? 8 : 16), row_tiles = (M + 31) / 32;
+        auto rounds = [&](int mt) { return ((row_tiles + mt - 1) / mt * cols + 255) / 256; };
+        if (dual ? rounds(8) < rounds(7) : (row_tiles + 3) / 4 * cols >= 172) {
+            TileChoice c8{TILE8_256x256, 1};
+            double least = 1e30;
+            for (int tile : {TILE8_128x256, TILE8_160x256, TILE8_192x256, TILE8_224x256, TILE8_256x256}) {
+                const int m_blocks = gemm8_row_blocks(row_tiles, gemm_tile_bm(tile) / 32, cols);
+                const int mt = (row_tiles + m_blocks - 1) / m_blocks;
+                const double cost = (m_blocks * cols + 255) / 256 * (2 * stages * (0.36 + 0.0155 * mt) + (activation ? 2.4 * mt - 2.0 : 1.6 * mt - 1.8));
+                if (cost < least) { least = cost; c8.tile = tile; }
+            }
+            return c8;
         }
-        return c8;
     }
     double best = 1e30; TileChoice bc{TILE_128x256, 1};
     for (int tile : tiles) {
@@ -552,8 +558,9 @@ struct Sched {
         GemmP p = extra;
         p.A = A; p.lda = lda; p.a_rows = a_rows; p.M = M; p.B0 = B0; p.B1 = B1;
         p.N16 = n16_tiles(N); p.K32p = k32_padded(K); p.bgroup = bgroup;
-        const TileChoice tc = choose_tile(M, p.N16, p.K32p / 2, epi == EPI_GEGLU || epi == EPI_SWIGLU, epi == EPI_PARTIAL, what, epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_VIT_QKV_ROPE,
-                                          epi == EPI_QKV_ROPE || epi == EPI_VIS_QKV || epi == EPI_VIT_QKV_ROPE);
+        const bool dual = epi == EPI_GEGLU || epi == EPI_SWIGLU;
+        const TileChoice tc = choose_tile(M, p.N16, p.K32p / 2, dual, epi == EPI_PARTIAL, what, dual || epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_RESIDUAL || epi == EPI_VIT_QKV_ROPE,
+                                          epi == EPI_QKV_ROPE || epi == EPI_VIS_QKV || epi == EPI_VIT_QKV_ROPE, dual || epi == EPI_BIAS_GELU);
         p.nsplit = tc.nsplit;
         if (epi == EPI_PARTIAL) {
             p.partial = c->B<float>("splitk_partial"); p.ldp = N; p.pstride = (size_t)M * N;
@@ -1639,8 +1646,8 @@ int plan_linear_act(int M, int K, int N, int act, int tile, ActPlan* out) {
     ActPlan p{};
     p.dual = act == RTVLA_ACT_GEGLU || act == RTVLA_ACT_SWIGLU;
     p.K128 = k32_padded(K) * 32;
-    p.tile = tile >= 0 ? tile : choose_tile(M, n16_tiles(N), k32_padded(K) / 2, p.dual, false, "linear act", act == RTVLA_ACT_BIAS_GELU).tile;
-    if (p.dual && (gemm_tile_bn(p.tile) != 256 || gemm_tile_eight_waves(p.tile))) return RTVLA_ERR_LIMIT;      // gate and up share a 256-column workgroup tile
+    p.tile = tile >= 0 ? tile : choose_tile(M, n16_tiles(N), k32_padded(K) / 2, p.dual, false, "linear act", true, false, act != RTVLA_ACT_RESIDUAL).tile;
+    if (p.dual && tile >= 0 && (gemm_tile_bn(tile) != 256 || gemm_tile_eight_waves(tile))) return RTVLA_ERR_LIMIT;      // gate and up share a 256-column workgroup tile
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const int G = p.dual ? 4 : 8;
     p.a_off = 0;
@@ -1666,6 +1673,7 @@ int rtvla_linear_act(const void* x, int M, int K, const void* w, const void* w_u
     if (int rc = plan_linear_act(M, K, N, act, tile, &pl)) return rc;
     if (pl.dual != (w_up != nullptr)) return RTVLA_ERR_ARG;
     if (workspace_bytes < pl.total) return RTVLA_ERR_SIZE;
+    if (act == RTVLA_ACT_RESIDUAL && tile >= 0 && gemm_tile_eight_waves(tile)) return RTVLA_ERR_LIMIT;
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
     bf16_t* a = (bf16_t*)(ws + pl.a_off);

@@ -205,6 +205,41 @@ def test_eight_wave_tiles_with_more_row_blocks_than_the_least(M, K, N):
     assert ran >= 3
 
 
+# what the cost model gives to the eight-wave tiles that a caller cannot name: 160 rows (85 row tiles by 12 blocks of columns), the residual epilogue
+# (171 row tiles by 4) and a gated one (32 row tiles: 256 rows save a round); one row past a tile, K past a pair of stages, columns past a block
+@pytest.mark.parametrize("M,K,N,act", [(2705, 136, 3072, 1), (2689, 72, 3056, 1), (5441, 72, 1008, 8), (5473, 264, 1024, 8), (1000, 264, 16384, 2), (993, 136, 16368, 3)])
+def test_eight_wave_tiles_of_the_cost_model_against_fp32(M, K, N, act):
+    import rtvla_capi as capi
+    lib = capi.load()
+    if act != capi.ACT_RESIDUAL:
+        res = _run_act(lib, capi, M, K, N, act, capi.TILE_AUTO)
+        assert res is not None and res[0] <= REL_TOL and res[1] <= 1.01, res
+        return
+    g = torch.Generator(device="cuda:0").manual_seed(M + K + N)
+    x = torch.randn(M, K, device="cuda:0", generator=g).to(torch.bfloat16)
+    w = (torch.randn(K, N, device="cuda:0", generator=g) * 0.05).to(torch.bfloat16)
+    b = torch.randn(N, device="cuda:0", generator=g).to(torch.bfloat16)
+    stream = (torch.randn(M + 1, N, device="cuda:0", generator=g) * 3).to(torch.bfloat16)
+    out = stream.clone()
+    need = lib.rtvla_linear_act_workspace_bytes(M, K, N, act, capi.TILE_AUTO)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda:0")
+    assert lib.rtvla_linear_act(_P(x.data_ptr()), M, K, _P(w.data_ptr()), None, N, _P(b.data_ptr()), act, _P(out.data_ptr()), _P(ws.data_ptr()), need,
+                                capi.TILE_AUTO, _P(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    ref = x.float() @ w.float() + b.float() + stream[:M].float()
+    got = out[:M].float()
+    excess = (got - ref).abs() / (ref.abs() * 2.0 ** -7 + 1e-3 * ref.pow(2).mean().sqrt())
+    assert ((got - ref).norm() / ref.norm()).item() <= REL_TOL and excess.max().item() <= 1.01
+    assert torch.equal(out[M], stream[M])
+
+
+def test_eight_wave_tiles_give_what_their_offsets_cannot_reach_to_the_four_wave_kernel():
+    import rtvla_capi as capi
+    lib = capi.load()
+    res = _run(lib, capi, 3, (1 << 21) + 8, 16, 7, 1)           # one 16-byte piece of K past what 32-bit offsets reach
+    assert res is not None and res[0] <= REL_TOL and res[1] <= 1.01, res
+
+
 # every tile that takes the epilogue, at whole and ragged tiles; the stream is read and written in place, rows behind it stay as they are
 @pytest.mark.parametrize("M,K,N", [(2720, 1024, 1024), (2720, 4096, 1024), (224, 128, 256), (225, 264, 272), (37, 136, 48), (1, 64, 16), (97, 192, 144)])
 def test_residual_epilogue_in_place_against_fp32(M, K, N):
