@@ -11,6 +11,7 @@
 // every lane ends up with 4 groups of 4 consecutive output columns of one row: 8-byte packed stores,
 // and RoPE pairs / GeGLU partners sit in the same lane.
 #include "kernels.h"
+#include "gemm_scatter.h"
 #include <algorithm>
 
 namespace {
@@ -22,7 +23,8 @@ RTVLA_DEVICE f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdg
 // MT, NT: 32-row tiles per workgroup and 32-column tiles per wave.  Small tiles are compiled to fit two
 // workgroups per CU so that one workgroup's MFMAs run under the other's memory latency.
 // One block tile of MT 32-row tiles starting at row m0: K loop and epilogue.
-template <int WN, int MT, int NT, int EPI>
+// V: a tile of V columns, whose product is taken as activations x weights (gemm_scatter.h)
+template <int WN, int MT, int NT, int EPI, bool V = false>
 RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, int n_blk, int split, int stages_total, int stages_per_split) {
     constexpr int NTH = WN * 64;
     constexpr int BM = MT * 32;
@@ -127,7 +129,7 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
 #pragma unroll
         for (int f = 0; f < HR; ++f)
 #pragma unroll
-            for (int j = 0; j < NT; ++j) acc[f % MT][j] = mfma32(br[j][f / MT], af[f], acc[f % MT][j]);
+            for (int j = 0; j < NT; ++j) acc[f % MT][j] = V ? mfma32(af[f], br[j][f / MT], acc[f % MT][j]) : mfma32(br[j][f / MT], af[f], acc[f % MT][j]);
         store_a(wr, ar_store);
 #pragma unroll
         for (int t = 0; t < HR; ++t) {
@@ -148,7 +150,7 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
 #pragma unroll
         for (int f = HR; f < 2 * HR; ++f)
 #pragma unroll
-            for (int j = 0; j < NT; ++j) acc[f % MT][j] = mfma32(br[j][f / MT], af[f], acc[f % MT][j]);
+            for (int j = 0; j < NT; ++j) acc[f % MT][j] = V ? mfma32(af[f], br[j][f / MT], acc[f % MT][j]) : mfma32(br[j][f / MT], af[f], acc[f % MT][j]);
         load_b_half(s_next, br, 1);
 #pragma unroll
         for (int t = 0; t < HR; ++t) {
@@ -292,123 +294,14 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
           }
           if (g0 + GROUP < MT) __syncthreads();
         }
-        return;
-    }
+    } else {
+        static_assert(epi_scatters(EPI), "every epilogue is one of the two kinds");
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-        const int m = m0 + i * 32 + r;
-        if (m >= p.M) continue;
+        for (int i = 0; i < MT; ++i) {
+            if (m0 + i * 32 >= p.M) continue;
 #pragma unroll
-        for (int j = 0; j < HALF; ++j) {
-          uint2 qk[4];                                                  // (EPI_VIT_QKV_ROPE: the rotated values of the four groups)
-#pragma unroll
-          for (int grp = 0; grp < 4; ++grp) {
-            const int n0 = tile_of[j] * 32 + 8 * grp + 4 * h;
-            if (n0 >= p.N16 * 16) continue;
-            f32x4 v = {acc[i][j][4 * grp], acc[i][j][4 * grp + 1], acc[i][j][4 * grp + 2], acc[i][j][4 * grp + 3]};
-            if constexpr (EPI == EPI_PARTIAL) {
-                *(f32x4*)(p.partial + (size_t)split * p.pstride + (size_t)m * p.ldp + n0) = v;
-            } else if constexpr (EPI == EPI_GEGLU) {
-                const f32x4 u = {acc[i][j + HALF][4 * grp], acc[i][j + HALF][4 * grp + 1], acc[i][j + HALF][4 * grp + 2], acc[i][j + HALF][4 * grp + 3]};
-                store4(p.out + (size_t)m * p.ldo + n0,
-                       pack4(gelu_tanh(v[0]) * u[0], gelu_tanh(v[1]) * u[1], gelu_tanh(v[2]) * u[2], gelu_tanh(v[3]) * u[3]));
-            } else if constexpr (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU || EPI == EPI_PATCH) {
-                const bf16x4 b = load4(p.bias + n0);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] += bf2f(b[e]);
-                if constexpr (EPI == EPI_PATCH) {
-                    const bf16x4 rs = load4(p.res + (size_t)(m % p.res_mod) * p.ldr + n0);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] += bf2f(rs[e]);
-                }
-                if constexpr (EPI == EPI_BIAS_GELU) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
-                }
-                store4(p.out + (size_t)m * p.ldo + n0, pack4(v));
-            } else if constexpr (EPI == EPI_QKV_ROPE) {
-                // the reference rounds the accumulator to bf16 before the rotation (pi0_infer.py:793)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = round_bf16(v[e]);
-                if (n0 < 2304) {
-                    const bf16x4 cs = load4(p.rope + (size_t)m * 256 + (n0 & 255));
-                    const float c0 = bf2f(cs[0]), s0 = bf2f(cs[1]), c1 = bf2f(cs[2]), s1 = bf2f(cs[3]);
-                    const f32x4 w = v;
-                    v[0] = w[0] * c0 - w[1] * s0; v[1] = w[1] * c0 + w[0] * s0;
-                    v[2] = w[2] * c1 - w[3] * s1; v[3] = w[3] * c1 + w[2] * s1;
-                    // Q rows are token*8 + head; Q and K are kept fragment-tiled for the attention kernel
-                    if (n0 < 2048) store4(p.q + ft_index(m * 8 + (n0 >> 8), n0 & 255, 8), pack4(v));
-                    else store4(p.k + ft_index(m, n0 - 2048, 8), pack4(v));
-                } else {
-                    const int d = n0 - 2304;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) p.vt[vt_index(d + e, m, p.ldvt >> 5)] = f2bf(v[e]);
-                }
-            } else if constexpr (EPI == EPI_VIT_QKV_ROPE) {
-                // DM0 ViT (dm0_infer.py:589-598): + fp32 bias, rounded to bf16 as the reference's QKV buffer is, then the 2-D rotary
-                // embedding on Q and K; per (image, head) Q and K as fragment-tiled [seq_pad][64], V^T as [64][seq_pad].  The rows
-                // are laid out as seq_pad (a multiple of 32) per image, so a 32-row tile is one 32-key block of one image.
-                v += *(const f32x4*)(p.bias_f32 + n0);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = round_bf16(v[e]);
-                const int which = n0 >> 10, cc = n0 & 1023, head = cc >> 6, d = cc & 63;
-                const int img = m / p.seq_pad, tok = m - img * p.seq_pad;
-                const size_t vh = (size_t)(img * 16 + head);
-                if (which < 2) {
-                    const bf16x4 cs = load4(p.rope + (size_t)min(tok, p.seq - 1) * 64 + d);
-                    const float c0 = bf2f(cs[0]), s0 = bf2f(cs[1]), c1 = bf2f(cs[2]), s1 = bf2f(cs[3]);
-                    const f32x4 w = v;
-                    v[0] = w[0] * c0 - w[1] * s0; v[1] = w[1] * c0 + w[0] * s0;
-                    v[2] = w[2] * c1 - w[3] * s1; v[3] = w[3] * c1 + w[2] * s1;
-                    // lanes h = 0 / 1 of a row hold the two halves of every 8-wide chunk: swap halves so that each lane owns two
-                    // whole 16-byte pieces of the fragment-tiled Q / K
-                    const bf16x4 pk = pack4(v);
-                    qk[grp] = *(const uint2*)&pk;
-                    if (grp == 3) {
-                        bf16_t* const dst = (which == 0 ? p.q : p.k) + vh * ((size_t)p.seq_pad * 64);
-                        const int d0 = (tile_of[j] * 32) & 63;
-#pragma unroll
-                        for (int pr = 0; pr < 2; ++pr) {
-                            const uint2 keep = h ? qk[2 * pr + 1] : qk[2 * pr], send = h ? qk[2 * pr] : qk[2 * pr + 1];
-                            const uint2 recv = {(unsigned)__shfl_xor((int)send.x, 32, 64), (unsigned)__shfl_xor((int)send.y, 32, 64)};
-                            *(uint4*)(dst + ft_index(tok, d0 + 8 * (2 * pr + h), 2)) = h ? uint4{recv.x, recv.y, keep.x, keep.y} : uint4{keep.x, keep.y, recv.x, recv.y};
-                        }
-                    }
-                } else {
-                    // V^T: the wave's 32 keys x 32 d tile is transposed through a private 2.3 KB of LDS ([d][key], 72-byte pitch)
-                    // so that it leaves as whole 16-byte pieces of the permuted-key fragments instead of 2-byte stores
-                    volatile bf16_t* tb = (volatile bf16_t*)(smem_raw + wn * 2304);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) tb[(8 * grp + 4 * h + e) * 36 + r] = f2bf(v[e]);
-                    if (grp == 3) {
-                        const int tok0 = tok - r;                                   // first key of the tile: a multiple of 32
-                        const int d0 = (tile_of[j] * 32) & 63;                      // head-local d of the tile's first column
-                        const int gq = lane >> 4, rq = lane & 15;
-#pragma unroll
-                        for (int dt = 0; dt < 2; ++dt) {
-                            const volatile uint2* src = (const volatile uint2*)(smem_raw + wn * 2304 + (16 * dt + rq) * 72 + gq * 8);
-                            const uint2 lo = {src[0].x, src[0].y}, hi = {src[4].x, src[4].y};       // keys 4 gq .. +3 and 16 + 4 gq .. +3
-                            const size_t frag = (size_t)(((d0 >> 4) + dt) * (p.seq_pad >> 5) + (tok0 >> 5)) * 64 + lane;
-                            *(uint4*)(p.vt + vh * ((size_t)64 * p.seq_pad) + frag * 8) = uint4{lo.x, lo.y, hi.x, hi.y};
-                        }
-                    }
-                }
-            } else if constexpr (EPI == EPI_VIS_QKV) {
-                const bf16x4 b = load4(p.bias + n0);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] += bf2f(b[e]);
-                // per (view, head): Q and K as fragment-tiled [256 tokens][96] (72 padded), V^T as [80][256]
-                const int which = n0 / 1152, c = n0 - which * 1152, head = c / 72, d = c - head * 72;
-                const int view = m >> 8, tok = m & 255;
-                const size_t vh = (size_t)(view * 16 + head);
-                if (which == 0) store4(p.q + vh * (256 * 96) + ft_index(tok, d, 3), pack4(v));
-                else if (which == 1) store4(p.k + vh * (256 * 96) + ft_index(tok, d, 3), pack4(v));
-                else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) p.vt[vh * (80 * 256) + vt_index(d + e, tok, 8)] = f2bf(v[e]);
-                }
-            }
-          }
+            for (int j = 0; j < NT; ++j)
+                if (tile_of[j] * 32 < p.N16 * 16) scatter_tile<EPI, V>(p, acc[i][j], m0 + i * 32, tile_of[j] * 32, lane);
         }
     }
 }
@@ -426,12 +319,18 @@ void gemm_mfma_kernel(GemmP p, int m_blocks, int n_blocks, int stages_total, int
     const int rem = lid - split * (m_blocks * n_blocks);
     const int n_blk = rem / m_blocks;
     const int m_blk = rem - n_blk * m_blocks;
-    if constexpr (MIXED) {
-        if (m_blk < n_big) gemm_block<WN, MT, NT, EPI>(p, smem_raw, m_blk * (MT * 32), n_blk, split, stages_total, stages_per_split);
-        else gemm_block<WN, MT - 1, NT, EPI>(p, smem_raw, n_big * (MT * 32) + (m_blk - n_big) * ((MT - 1) * 32), n_blk, split, stages_total, stages_per_split);
-    } else {
-        gemm_block<WN, MT, NT, EPI>(p, smem_raw, m_blk * (MT * 32), n_blk, split, stages_total, stages_per_split);
+    auto block = [&](auto v) __attribute__((always_inline)) {
+        if constexpr (MIXED) {
+            if (m_blk < n_big) gemm_block<WN, MT, NT, EPI, v.value>(p, smem_raw, m_blk * (MT * 32), n_blk, split, stages_total, stages_per_split);
+            else gemm_block<WN, MT - 1, NT, EPI, v.value>(p, smem_raw, n_big * (MT * 32) + (m_blk - n_big) * ((MT - 1) * 32), n_blk, split, stages_total, stages_per_split);
+        } else {
+            gemm_block<WN, MT, NT, EPI, v.value>(p, smem_raw, m_blk * (MT * 32), n_blk, split, stages_total, stages_per_split);
+        }
+    };
+    if constexpr (epi_scatters(EPI)) {
+        if (n_blk * (WN * NT * 32) >= epi_first_v(EPI)) { block(std::true_type{}); return; }
     }
+    block(std::false_type{});
 }
 
 template <int WN, int MT, int NT, int EPI, bool MIXED>
@@ -497,7 +396,6 @@ int launch_gemm(const GemmP& p, int epi, int tile, hipStream_t s) {
         case EPI_QKV_ROPE:  return launch_epi<EPI_QKV_ROPE>(p, tile, s);
         case EPI_VIS_QKV:   return launch_epi<EPI_VIS_QKV>(p, tile, s);
         case EPI_SWIGLU:    return launch_epi<EPI_SWIGLU>(p, tile, s);
-        case EPI_VIT_QKV_ROPE: return launch_epi<EPI_VIT_QKV_ROPE>(p, tile, s);
     }
     return 2;
 }

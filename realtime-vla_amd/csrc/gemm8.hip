@@ -19,6 +19,7 @@
 // loads of stage s + RING - 1 may overwrite, half of them issued in the second half of stage s, the rest in the first half of s + 1: issued together they
 // hold up the wave's MFMAs while the load path takes them in (8 160 x 4 096 x 1 024 with 128 rows: 61 -> 59 us).  And in front of it every wave has waited for its own loads of stage s + 1.
 #include "kernels.h"
+#include "gemm_scatter.h"
 #include <algorithm>
 
 namespace {
@@ -44,7 +45,7 @@ template <int N> RTVLA_DEVICE void wait_and_meet() {
 }
 
 // The K loop of one wave: MTW of the workgroup's MT row tiles, from i0 on, and its 64 columns (two column tiles; DUAL: one of each weight).
-template <int MT, int MTW, int RING, bool DUAL, int MTA>
+template <int MT, int MTW, int RING, bool DUAL, bool V, int MTA>
 RTVLA_DEVICE void gemm8_loop(const GemmP& p, unsigned char* smem, int m0, int n_blk, int i0, int s_begin, int s_end, f32x16 (&acc)[MTA][2]) {
 #ifdef __HIP_DEVICE_COMPILE__                                                          // (the host pass knows neither the LDS load's size nor the waits)
     constexpr int NT = 2, A_B = MT * 2048, STAGE_B = stage_bytes(MT);
@@ -92,7 +93,7 @@ RTVLA_DEVICE void gemm8_loop(const GemmP& p, unsigned char* smem, int m0, int n_
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
                 const int at = i * NT + j;
-                acc[i][j] = mfma32(bf[ks][j], af[ks][i], acc[i][j]);
+                acc[i][j] = V ? mfma32(af[ks][i], bf[ks][j], acc[i][j]) : mfma32(bf[ks][j], af[ks][i], acc[i][j]);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int q = 0; q < NR; ++q)
@@ -126,7 +127,7 @@ RTVLA_DEVICE void gemm8_loop(const GemmP& p, unsigned char* smem, int m0, int n_
 #endif
 }
 
-template <int MT, int RING, int EPI>
+template <int MT, int RING, int EPI, bool V>
 RTVLA_DEVICE void gemm8_block(const GemmP& p, unsigned char* smem_raw, int m0, int n_blk, int split, int s_begin, int s_end) {
     constexpr int WN = 4, NT = 2, NTH = 512;
     constexpr int MTW = (MT + 1) / 2;                      // row tiles of the upper wave; the lower one has MT / 2
@@ -149,66 +150,17 @@ RTVLA_DEVICE void gemm8_block(const GemmP& p, unsigned char* smem_raw, int m0, i
         for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    if (MT % 2 == 0 || wm == 0) gemm8_loop<MT, MTW, RING, DUAL>(p, smem_raw, m0, n_blk, i0, s_begin, s_end, acc);
-    else gemm8_loop<MT, MT / 2, RING, DUAL>(p, smem_raw, m0, n_blk, i0, s_begin, s_end, acc);
+    if (MT % 2 == 0 || wm == 0) gemm8_loop<MT, MTW, RING, DUAL, V>(p, smem_raw, m0, n_blk, i0, s_begin, s_end, acc);
+    else gemm8_loop<MT, MT / 2, RING, DUAL, V>(p, smem_raw, m0, n_blk, i0, s_begin, s_end, acc);
 
-    if constexpr (EPI == EPI_VIT_QKV_ROPE) {
-        // DM0 ViT (dm0_infer.py:589-598), as in the four-wave kernel: + fp32 bias, rounded to bf16, 2-D rotary embedding on Q and
-        // K, per (image, head) Q and K as fragment-tiled [seq_pad][64] (16-byte pieces after a half swap between lane pairs),
-        // V^T transposed through a wave-private 2.3 KB of LDS into whole pieces of the permuted-key fragments
+    if constexpr (epi_scatters(EPI)) {
 #pragma unroll
         for (int k = 0; k < MTW; ++k) {
-            const int m = m0 + (i0 + k) * 32 + r;
-            if (k >= mtw || m0 + (i0 + k) * 32 >= p.M) continue;
-            const int img = m / p.seq_pad, tok = m - img * p.seq_pad;
+            const int mt0 = m0 + (i0 + k) * 32;
+            if (k >= mtw || mt0 >= p.M) continue;
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                const int nt0 = tile_of[j] * 32;
-                if (nt0 >= p.N16 * 16) continue;
-                const int which = nt0 >> 10, head = (nt0 & 1023) >> 6, d0 = nt0 & 63;
-                const size_t vh = (size_t)(img * 16 + head);
-                uint2 qk[4];
-#pragma unroll
-                for (int grp = 0; grp < 4; ++grp) {
-                    const int n0 = nt0 + 8 * grp + 4 * h;
-                    f32x4 v = {acc[k][j][4 * grp], acc[k][j][4 * grp + 1], acc[k][j][4 * grp + 2], acc[k][j][4 * grp + 3]};
-                    v += *(const f32x4*)(p.bias_f32 + n0);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = round_bf16(v[e]);
-                    if (which < 2) {
-                        const bf16x4 cs = load4(p.rope + (size_t)min(tok, p.seq - 1) * 64 + d0 + 8 * grp + 4 * h);
-                        const float c0 = bf2f(cs[0]), s0 = bf2f(cs[1]), c1 = bf2f(cs[2]), s1 = bf2f(cs[3]);
-                        const f32x4 w = v;
-                        v[0] = w[0] * c0 - w[1] * s0; v[1] = w[1] * c0 + w[0] * s0;
-                        v[2] = w[2] * c1 - w[3] * s1; v[3] = w[3] * c1 + w[2] * s1;
-                        const bf16x4 pk = pack4(v);
-                        qk[grp] = *(const uint2*)&pk;
-                    } else {
-                        volatile bf16_t* tb = (volatile bf16_t*)(smem_raw + wave * 2304);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) tb[(8 * grp + 4 * h + e) * 36 + r] = f2bf(v[e]);
-                    }
-                }
-                if (which < 2) {
-                    bf16_t* const dst = (which == 0 ? p.q : p.k) + vh * ((size_t)p.seq_pad * 64);
-#pragma unroll
-                    for (int pr = 0; pr < 2; ++pr) {
-                        const uint2 keep = h ? qk[2 * pr + 1] : qk[2 * pr], send = h ? qk[2 * pr] : qk[2 * pr + 1];
-                        const uint2 recv = {(unsigned)__shfl_xor((int)send.x, 32, 64), (unsigned)__shfl_xor((int)send.y, 32, 64)};
-                        *(uint4*)(dst + ft_index(tok, d0 + 8 * (2 * pr + h), 2)) = h ? uint4{recv.x, recv.y, keep.x, keep.y} : uint4{keep.x, keep.y, recv.x, recv.y};
-                    }
-                } else {
-                    const int tok0 = tok - r;
-                    const int gq = lane >> 4, rq = lane & 15;
-#pragma unroll
-                    for (int dt = 0; dt < 2; ++dt) {
-                        const volatile uint2* src = (const volatile uint2*)(smem_raw + wave * 2304 + (16 * dt + rq) * 72 + gq * 8);
-                        const uint2 lo = {src[0].x, src[0].y}, hi = {src[4].x, src[4].y};
-                        const size_t frag = (size_t)(((d0 >> 4) + dt) * (p.seq_pad >> 5) + (tok0 >> 5)) * 64 + lane;
-                        *(uint4*)(p.vt + vh * ((size_t)64 * p.seq_pad) + frag * 8) = uint4{lo.x, lo.y, hi.x, hi.y};
-                    }
-                }
-            }
+            for (int j = 0; j < NT; ++j)
+                if (tile_of[j] * 32 < p.N16 * 16) scatter_tile<EPI, V>(p, acc[k][j], mt0, tile_of[j] * 32, lane);
         }
         return;
     }
@@ -326,8 +278,14 @@ void gemm8_kernel(GemmP p, int m_blocks, int n_blocks, int stages_total, int sta
     const int rows = min(ROWS, m_blocks - group * ROWS);
     const int n_blk = in_group / rows, m_blk = group * ROWS + in_group % rows;
     const int s_begin = split * stages_per_split, s_end = min(s_begin + stages_per_split, stages_total);
-    if (m_blk < n_big) gemm8_block<MT, RING, EPI>(p, smem_raw, m_blk * (MT * 32), n_blk, split, s_begin, s_end);
-    else gemm8_block<MT - 1, RING, EPI>(p, smem_raw, n_big * (MT * 32) + (m_blk - n_big) * ((MT - 1) * 32), n_blk, split, s_begin, s_end);
+    auto block = [&](auto v) __attribute__((always_inline)) {
+        if (m_blk < n_big) gemm8_block<MT, RING, EPI, v.value>(p, smem_raw, m_blk * (MT * 32), n_blk, split, s_begin, s_end);
+        else gemm8_block<MT - 1, RING, EPI, v.value>(p, smem_raw, n_big * (MT * 32) + (m_blk - n_big) * ((MT - 1) * 32), n_blk, split, s_begin, s_end);
+    };
+    if constexpr (epi_scatters(EPI)) {
+        if (n_blk * 256 >= epi_first_v(EPI)) { block(std::true_type{}); return; }
+    }
+    block(std::false_type{});
 }
 
 template <int MT, int EPI>

@@ -1,0 +1,112 @@
+// Epilogue of the QKV GEMMs: one 32 x 32 tile of accumulators into the fragment order the attention kernels read.  Everything leaves as whole 16-byte
+// pieces.  A Q / K tile is the product weights x activations: lanes h = 0 / 1 of a row hold the two halves of every 8 columns and swap registers, which
+// goes for the rotary table as well.  A V tile is taken the other way round, activations x weights, so that a lane holds four consecutive keys of one
+// column: two 16-byte pieces of V^T as they are.  What it replaces stored Q / K in 8-byte and V^T in 2-byte pieces (DM0: through LDS) and read the
+// tables 8 bytes at a time; us, before and after: SigLIP 256 rows x 3 456 10.4 and 8.7, 768 14.0 and 11.7, Gemma 256 x 2 560 14.8 and 13.3, 788 20.2 and 18.4.
+#pragma once
+#include "kernels.h"
+
+constexpr bool epi_scatters(int epi) { return epi == EPI_QKV_ROPE || epi == EPI_VIS_QKV || epi == EPI_VIT_QKV_ROPE; }
+// first V column: a multiple of 256, so no workgroup tile holds both kinds
+constexpr int epi_first_v(int epi) { return epi == EPI_VIT_QKV_ROPE ? 2048 : 2304; }
+
+// lanes h = 0 / 1: {x0 (h = 0), x0 (h = 1)} / {x1 (h = 0), x1 (h = 1)}
+RTVLA_DEVICE uint4 swap_halves(uint2 x0, uint2 x1) {
+    const rtvla_u2 a = __builtin_amdgcn_permlane32_swap(x0.x, x1.x, false, false), b = __builtin_amdgcn_permlane32_swap(x0.y, x1.y, false, false);
+    return uint4{a[0], b[0], a[1], b[1]};
+}
+
+// rows mt0 .. mt0 + 31, columns nt0 .. nt0 + 31 (multiples of 32), mt0 < p.M
+template <int EPI, bool V>
+RTVLA_DEVICE void scatter_tile(const GemmP& p, const f32x16& acc, int mt0, int nt0, int lane) {
+    const int h = lane >> 5, r = lane & 31;
+    if constexpr (V) {
+        const int n = nt0 + r;                             // rows mt0 + 8 grp + 4 h + e
+        float b = 0.f;
+        if constexpr (EPI == EPI_VIS_QKV) b = bf2f(p.bias[n]);
+        if constexpr (EPI == EPI_VIT_QKV_ROPE) b = p.bias_f32[n];
+        bf16x4 pk[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) pk[g] = pack4(acc[4 * g] + b, acc[4 * g + 1] + b, acc[4 * g + 2] + b, acc[4 * g + 3] + b);
+        bf16_t* base;
+        int d, key0, keys32;
+        if constexpr (EPI == EPI_QKV_ROPE) { base = p.vt; d = n - 2304; key0 = mt0; keys32 = p.ldvt >> 5; }
+        else if constexpr (EPI == EPI_VIS_QKV) {
+            const int c = n - 2304, head = c / 72;
+            base = p.vt + (size_t)((mt0 >> 8) * 16 + head) * (80 * 256); d = c - head * 72; key0 = mt0 & 255; keys32 = 8;
+        } else {
+            const int c = n - 2048, img = mt0 / p.seq_pad;
+            base = p.vt + (size_t)(img * 16 + (c >> 6)) * ((size_t)64 * p.seq_pad); d = c & 63; key0 = mt0 - img * p.seq_pad; keys32 = p.seq_pad >> 5;
+        }
+        if (EPI != EPI_QKV_ROPE || mt0 + 32 <= p.M) {      // (the others' rows are whole tiles)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {                  // keys 8 q + 4 h + e and 16 more
+                const uint2 lo = *(const uint2*)&pk[q], hi = *(const uint2*)&pk[q + 2];
+                *(uint4*)(base + vt_index(d, key0 + 8 * q + 4 * h, keys32)) = uint4{lo.x, lo.y, hi.x, hi.y};
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (mt0 + 8 * g + 4 * h + e < p.M) base[vt_index(d, key0 + 8 * g + 4 * h + e, keys32)] = pk[g][e];
+        }
+    } else {
+        const int m = mt0 + r, mc = min(m, p.M - 1);       // columns nt0 + 8 grp + 4 h + e
+        int tok = mc, img = 0;
+        if constexpr (EPI == EPI_VIS_QKV) { img = mc >> 8; tok = mc & 255; }
+        if constexpr (EPI == EPI_VIT_QKV_ROPE) { img = mt0 / p.seq_pad; tok = mc - img * p.seq_pad; }
+        uint4 table[2] = {};
+        if constexpr (EPI == EPI_QKV_ROPE) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) table[q] = *(const uint4*)(p.rope + (size_t)mc * 256 + (nt0 & 255) + 16 * q + 8 * h);
+        }
+        if constexpr (EPI == EPI_VIT_QKV_ROPE) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) table[q] = *(const uint4*)(p.rope + (size_t)min(tok, p.seq - 1) * 64 + (nt0 & 63) + 16 * q + 8 * h);
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            bf16x4 pk[2];
+            uint4 cs4 = {};
+            if constexpr (EPI != EPI_VIS_QKV) cs4 = swap_halves(uint2{table[q].x, table[q].y}, uint2{table[q].z, table[q].w});       // this lane's halves of the two groups
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int g = 2 * q + k, n0 = nt0 + 8 * g + 4 * h;
+                f32x4 v = {acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+                if constexpr (EPI == EPI_VIS_QKV) {
+                    const bf16x4 b = load4(p.bias + n0);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] += bf2f(b[e]);
+                } else {
+                    // rounded to bf16 before the rotation, as the reference's QKV buffers are (pi0_infer.py:793; dm0_infer.py:589-598)
+                    if constexpr (EPI == EPI_VIT_QKV_ROPE) v += *(const f32x4*)(p.bias_f32 + n0);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = round_bf16(v[e]);
+                    const uint2 raw = k ? uint2{cs4.z, cs4.w} : uint2{cs4.x, cs4.y};
+                    const bf16x4 cs = *(const bf16x4*)&raw;
+                    const float c0 = bf2f(cs[0]), s0 = bf2f(cs[1]), c1 = bf2f(cs[2]), s1 = bf2f(cs[3]);
+                    const f32x4 w = v;
+                    v[0] = w[0] * c0 - w[1] * s0; v[1] = w[1] * c0 + w[0] * s0;
+                    v[2] = w[2] * c1 - w[3] * s1; v[3] = w[3] * c1 + w[2] * s1;
+                }
+                pk[k] = pack4(v);
+            }
+            const uint4 piece = swap_halves(*(const uint2*)&pk[0], *(const uint2*)&pk[1]);
+            const int n8 = nt0 + 16 * q + 8 * h;           // whole 8 columns now
+            if (m >= p.M) continue;
+            if constexpr (EPI == EPI_QKV_ROPE) {
+                // Q rows are token * 8 + head
+                if (n8 < 2048) *(uint4*)(p.q + ft_index(m * 8 + (n8 >> 8), n8 & 255, 8)) = piece;
+                else *(uint4*)(p.k + ft_index(m, n8 - 2048, 8)) = piece;
+            } else if constexpr (EPI == EPI_VIS_QKV) {
+                // per (view, head): [256 tokens][96], 72 of them used
+                const int which = n8 >= 1152, c = n8 - which * 1152, head = c / 72;
+                *(uint4*)((which ? p.k : p.q) + (size_t)(img * 16 + head) * (256 * 96) + ft_index(tok, c - head * 72, 3)) = piece;
+            } else {
+                const int which = n8 >> 10, head = (n8 & 1023) >> 6;
+                *(uint4*)((which ? p.k : p.q) + (size_t)(img * 16 + head) * ((size_t)p.seq_pad * 64) + ft_index(tok, n8 & 63, 2)) = piece;
+            }
+        }
+    }
+}

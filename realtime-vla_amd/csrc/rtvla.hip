@@ -150,7 +150,7 @@ constexpr int64_t ATTN_PARTIAL_FLOATS = 64 * 16 * (16 * 64 * 4 + 32);   // 64 ro
 // turn, so weights and activations are where a forward has them).  One K stage of a workgroup takes the larger of its MFMA time (32 cycles
 // per 32x32x16 MFMA at 2.05 GHz and 88 % issue efficiency) and its load time (0.143 us + 10.1 us per MB of operands pulled by the workgroup);
 // tiles of 64 rows run two workgroups per CU, which share the MFMA pipe and the CU's load path; all workgroups together cannot pull more
-// than 18.7 TB/s out of L2; every launch pays a ramp and an epilogue per 32 x 128 outputs of a workgroup, 2.7 times as long where Q, K and
+// than 18.7 TB/s out of L2; every launch pays a ramp and an epilogue per 32 x 128 outputs of a workgroup, 1.3 times as long where Q, K and
 // V^T are scattered into fragment order; split-K adds the fp32 partials, written and read.  Over those layers, weighted by their number per
 // forward, the choice is 0.46 ms off the best one in sum.  It was 2.7 ms as long as two workgroups of a CU were taken to load twice as fast as
 // one, and needed a table for two shapes (SigLIP down-projection at 768 rows, output projection at 1 024) that are within 0.7 us of the best now.  Layer
@@ -206,7 +206,7 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
             const double stage_bytes = (double)(bm + bn) * 64 * 2;
             const double alone_us = std::max(mfma_us, 0.143 + stage_bytes / 9.9e4), pair_us = std::max(occ * mfma_us, 0.143 + occ * stage_bytes / 9.9e4);
             double t = std::max((per_cu / occ * pair_us + per_cu % occ * alone_us) * sps, blocks * (double)sps * stage_bytes / 18.7e6);
-            t += 5.9 + (scattered ? 2.3 : 0.85) * mt * nt;
+            t += 5.9 + (scattered ? 1.1 : 0.85) * mt * nt;
             if (splittable) t += 2.2 + (double)sp * M * ncols16 * 16 * 4.0 / 3e6;    // the partials, written and read
             if (t <= best) { best = t; bc = TileChoice{tile, sp}; }      // (of equals the smaller tile)
         }

@@ -292,6 +292,29 @@ def test_the_flow_loop_as_launches_against_the_oracle(model, views, prompt, chun
     assert not case.e.ctx.flow_status()[0]
 
 
+# the QKV epilogue stores whole 16-byte pieces: the last 32-key tile of V^T holds 1, 17, 31 or 32 of this pass's keys, the rest is not its own
+@pytest.mark.parametrize("prompt", [1, 17, 31, 32])
+def test_prefix_cache_rows_at_the_end_of_a_key_tile(prompt):
+    from _engine import tile_vt
+    t = Case("pi0", 23, 1, prompt, 9, vision_layers=1, llm_layers=2)
+    c = t.capi
+    t.stage_inputs()
+    t.run(c.STAGE_VISION_EMBED)
+    t.run(c.STAGE_VISION_LAYER, 0)
+    t.run(c.STAGE_PROJECT)
+    V = t.cache(0)[1].clone()
+    V[t.S_e:] = 5.0
+    t.B["encoder_Vt"].reshape(t.LL, -1)[0].copy_(tile_vt(V.t().contiguous()))
+    t.run(c.STAGE_PREFIX_LAYER, 0)
+    K, V = t.cache(0)
+    assert rel(K[: t.S_e], t.taps["encoder_K/0"][: t.S_e]) <= LAYER_TOL
+    assert rel(V[: t.S_e], t.taps["encoder_V/0"][: t.S_e]) <= LAYER_TOL
+    last = t.S_e // 32 * 32                                  # (the rows of the last tile on their own, where there are any)
+    if last < t.S_e:
+        assert rel(V[last: t.S_e], t.taps["encoder_V/0"][last: t.S_e]) <= LAYER_TOL
+    assert (V[t.S_e: (t.S_e + 31) // 32 * 32] == 5.0).all()
+
+
 @pytest.mark.parametrize("name,spec", [
     ("c1", ("pi0", 1234, 1, 0, 50)),
     ("c2", ("pi0", 1234, 2, 20, 50)),
