@@ -54,7 +54,10 @@ constexpr int FLASH_STAGES = 3;
 // A block needs 8 MFMAs (256 cycles) and ~65 VALU instructions of one wave; issued back to back by one wave, or by
 // several waves in turn, the two streams mostly add up on a SIMD, interleaved one MFMA to a handful of VALU
 // instructions they overlap.  Three LDS stages: tile T+2 is requested when tile T-1 has been read by every wave.
-template <int HD>
+// SCALED: the queries carry scale * log2(e), and S^T starts from minus the running maximum instead of zero, so that the logits leave the MFMAs
+// as exponents of 2: 16 multiply-adds per block less, of about 70 vector instructions beside 8 MFMAs that hardly overlap them (busy 59 + 37 % of
+// the time).  The rows' maxima are exchanged between the lane halves only where one has grown.  48 x 2 705 tokens: see launch_flash_attention.
+template <int HD, bool SCALED>
 __global__ __launch_bounds__(256, 3)
 void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
     static_assert(HD == 64, "fragment bookkeeping below is written out for a head width of 64");
@@ -92,8 +95,11 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
     float m = NEG_BIG, l = 0.f;
-    const float c = p.scale * 1.4426950408889634f;
+    const float c = SCALED ? 1.0f : p.scale * 1.4426950408889634f;
     const float slack = RESCALE_BITS / c;               // the same threshold in units of the raw logits
+    f32x16 start;                                       // what S^T starts from: - m (SCALED), 0
+#pragma unroll
+    for (int e = 0; e < 16; ++e) start[e] = 0.f;
 
     const int keys32 = (p.keys + 31) >> 5, ldvt32 = p.ldvt >> 5;
     int ntiles = (p.keys + 63) >> 6;
@@ -163,27 +169,35 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
             for (int t = 0; t < DT2; ++t) vf[q][t] = *(const bf16x8*)(vt + ((2 * t * 2 + b) * 64 + 2 * q * 16) * 16);
     };
     const bf16x2 ones = {(bf16_t)1.0f, (bf16_t)1.0f};
+    // masks of block g: keys past the end, and (causal) keys after the row's own token
+    auto mask = [&](int g, f32x16& st) __attribute__((always_inline)) {
+        const int last = p.causal ? min(p.keys - 1, (row0 + n) / p.group) : p.keys - 1;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            if (g * 32 + 8 * (e >> 2) + 4 * h + (e & 3) > last) st[e] = NEG_BIG;
+    };
+    auto lane_max = [&](const f32x16& st) __attribute__((always_inline)) {
+        float mx0 = st[0], mx1 = st[8];
+#pragma unroll
+        for (int e = 1; e < 8; ++e) { mx0 = fmaxf(mx0, st[e]); mx1 = fmaxf(mx1, st[8 + e]); }
+        return fmaxf(mx0, mx1);
+    };
     // One pipeline step for block g = 2 T + b.  On entry: s_cur = S^T(g), kf = K fragments of block g+1, vf = V^T fragments and
     // p_prev = probabilities of block g-1.  On exit: s_next = S^T(g+1), kf = K fragments of g+2, vf / p_cur those of block g.
     // `off_v` is the stage of tile T, `off_k` that of the tile block g+2 lies in (T+1).
     auto step = [&](auto edge_tag, int g, int b, unsigned off_v, unsigned off_k, f32x16& s_cur, f32x16& s_next, bf16x8 (&kf)[DS],
                     bf16x8 (&vf)[2][DT2], bf16x8 (&p_prev)[2], bf16x8 (&p_cur)[2]) __attribute__((always_inline)) {
         constexpr bool EDGE = decltype(edge_tag)::value;
-        if (EDGE) {      // masks: keys past the end, and (causal) keys after the row's own token
-            const int key0 = g * 32;
-            const int last = p.causal ? min(p.keys - 1, (row0 + n) / p.group) : p.keys - 1;
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                if (key0 + 8 * (e >> 2) + 4 * h + (e & 3) > last) s_cur[e] = NEG_BIG;
-        }
-        float mx0 = s_cur[0], mx1 = s_cur[8];
-#pragma unroll
-        for (int e = 1; e < 8; ++e) { mx0 = fmaxf(mx0, s_cur[e]); mx1 = fmaxf(mx1, s_cur[8 + e]); }
-        const float mx = halves_max(fmaxf(mx0, mx1));
-        if (__any(mx > m + slack)) {
+        if (EDGE) mask(g, s_cur);
+        const float mx = SCALED ? lane_max(s_cur) : halves_max(lane_max(s_cur));
+        if (__any(mx > (SCALED ? slack : m + slack))) {
             // rare: the accumulator and the pending probabilities of block g-1 (still in the old scale) move to the new one
-            const float mnew = fmaxf(m, mx);
+            const float mnew = SCALED ? m + fmaxf(halves_max(mx), 0.f) : fmaxf(m, mx);
             const float alpha = __builtin_amdgcn_exp2f((m - mnew) * c);
+            if constexpr (SCALED) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) { s_cur[e] += m - mnew; start[e] += m - mnew; }
+            }
             l *= alpha;
 #pragma unroll
             for (int t = 0; t < DT2; ++t)
@@ -201,14 +215,13 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
 #pragma unroll
             for (int t = 0; t < DT2; ++t) o[t] = mfma32(vf[q][t], p_prev[q], o[t]);
         read_v(off_v, b, vf);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) s_next[e] = 0.f;
+        s_next = start;
 #pragma unroll
         for (int s4 = 0; s4 < DS; ++s4) s_next = mfma32(kf[s4], qf[s4], s_next);
         read_k(off_k, b, kf);
         const float mc = m * c;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) s_cur[e] = __builtin_amdgcn_exp2f(s_cur[e] * c - mc);
+        for (int e = 0; e < 16; ++e) s_cur[e] = __builtin_amdgcn_exp2f(SCALED ? s_cur[e] : s_cur[e] * c - mc);
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             p_cur[q] = pack8(s_cur, q, q + 2);
@@ -216,18 +229,19 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
 #pragma unroll
             for (int j = 0; j < 8; j += 2) l = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{p_cur[q][j], p_cur[q][j + 1]}, ones, l, false);
         }
-        // issue order: one MFMA to every six VALU instructions of the softmax; the fragment reads of the next step go into
+        // issue order: one MFMA to every six (SCALED: four) VALU instructions of the softmax; the fragment reads of the next step go into
         // the registers the MFMAs before them have consumed
+        constexpr int PER = SCALED ? 4 : 6;
 #pragma unroll
         for (int i = 0; i < 2 * DT2; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x402, 6, 0);
+            __builtin_amdgcn_sched_group_barrier(0x402, PER, 0);
         }
         __builtin_amdgcn_sched_group_barrier(0x100, 2 * DT2, 0);
 #pragma unroll
         for (int i = 0; i < DS; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x402, 6, 0);
+            __builtin_amdgcn_sched_group_barrier(0x402, PER, 0);
         }
         __builtin_amdgcn_sched_group_barrier(0x100, DS, 0);
         __builtin_amdgcn_sched_barrier(0);
@@ -244,6 +258,12 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
     for (int e = 0; e < 16; ++e) sA[e] = 0.f;
 #pragma unroll
     for (int s4 = 0; s4 < DS; ++s4) sA = mfma32(kf[s4], qf[s4], sA);
+    if constexpr (SCALED) {                             // the first block's maxima
+        mask(0, sA);
+        m = halves_max(lane_max(sA));
+#pragma unroll
+        for (int e = 0; e < 16; ++e) { sA[e] -= m; start[e] = -m; }
+    }
     read_k(0, 1, kf);
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
@@ -296,6 +316,7 @@ int launch_flash_attention(const AttnP& p0, int hd, hipStream_t s) {
     const int items = (p.rows + 127) / 128;
     const int bpx = (p.batch % 8 == 0) ? p.batch / 8 : 0;
     if (hd != 64) return 2;
-    hipLaunchKernelGGL((flash_kernel<64>), dim3(items * p.batch), dim3(256), FLASH_STAGES * 2 * 64 * 64 * 2, s, p, items, bpx);
+    if (p.q_scaled) hipLaunchKernelGGL((flash_kernel<64, true>), dim3(items * p.batch), dim3(256), FLASH_STAGES * 2 * 64 * 64 * 2, s, p, items, bpx);
+    else hipLaunchKernelGGL((flash_kernel<64, false>), dim3(items * p.batch), dim3(256), FLASH_STAGES * 2 * 64 * 64 * 2, s, p, items, bpx);
     return hipGetLastError() == hipSuccess ? 0 : 5;
 }

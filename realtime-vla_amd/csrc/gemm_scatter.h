@@ -89,6 +89,7 @@ RTVLA_DEVICE void scatter_tile(const GemmP& p, const f32x16& acc, int mt0, int n
                     const f32x4 w = v;
                     v[0] = w[0] * c0 - w[1] * s0; v[1] = w[1] * c0 + w[0] * s0;
                     v[2] = w[2] * c1 - w[3] * s1; v[3] = w[3] * c1 + w[2] * s1;
+                    if constexpr (EPI == EPI_VIT_QKV_ROPE) v *= nt0 < 1024 ? p.qscale : 1.0f;
                 }
                 pk[k] = pack4(v);
             }

@@ -67,6 +67,7 @@ struct GemmP {
     const float* bias_f32;                     // fp32 bias instead of `bias` (DM0's folded LayerNorm biases)
     const float* rowscale;                     // per-row factor applied to the accumulators (EPI_SWIGLU)
     int seq, seq_pad;                          // EPI_VIT_QKV_ROPE: tokens per image and their padded count in the Q / K / V^T tiles
+    float qscale;                              // EPI_VIT_QKV_ROPE: factor of the rotated queries, before they are rounded
     const bf16_t* res; int ldr; int res_mod;
     float* partial; int ldp; size_t pstride;   // [split][row][ldp]
     const bf16_t* rope;                        // [row][256] = cos0 sin0 cos1 sin1 ...
@@ -149,6 +150,7 @@ struct AttnP {
     int out_tiled, out_bcol, out_cols32;
     int rows, keys;
     float scale;
+    int q_scaled;                    // launch_flash_attention: the queries carry scale * log2(e) already (rounded to bf16 behind it)
     int causal;                      // key j visible to row r only if j <= r / group (keys and tokens count from the same origin)
     // masking: key j is visible to row r iff
     //   j < prefix_alloc ? j < *valid_len (or prefix_alloc if valid_len == null)

@@ -841,12 +841,12 @@ struct Sched {
     void dm0_vision_layer(int i) {
         const int n = d.num_views, M = n * DM0_SEQ_PAD;
         GemmP e{}; e.bias_f32 = WF("vision_fused_qkv_b", 3072, i); e.rope = c->W("vision_rope"); e.seq = DM0_SEQ; e.seq_pad = DM0_SEQ_PAD;
-        e.q = c->B("vision_Q"); e.k = c->B("vision_K"); e.vt = c->B("vision_Vt");
+        e.q = c->B("vision_Q"); e.k = c->B("vision_K"); e.vt = c->B("vision_Vt"); e.qscale = 0.125f * 1.4426950408889634f;      // (flash.hip: logits as exponents of 2)
         gemm(c->B("vision_x_norm"), 1024, M, M, c->TW("t_vision_fused_qkv_w", i), nullptr, 1024, 3072, EPI_VIT_QKV_ROPE, e, "vit qkv");
         AttnP a{};
         a.q = c->B("vision_Q"); a.k = c->B("vision_K"); a.vt = c->B("vision_Vt"); a.ldvt = DM0_SEQ_PAD;
         a.batch = n * 16; a.q_bstride = a.k_bstride = (size_t)DM0_SEQ_PAD * 64; a.vt_bstride = (size_t)64 * DM0_SEQ_PAD;
-        a.group = 1; a.rows = DM0_SEQ; a.keys = DM0_SEQ; a.scale = 0.125f; a.prefix_alloc = DM0_SEQ;
+        a.group = 1; a.rows = DM0_SEQ; a.keys = DM0_SEQ; a.q_scaled = 1; a.prefix_alloc = DM0_SEQ;
         a.out = c->B("vision_attn"); a.ld_tok = 1024; a.batch_inner = 16; a.out_ostride = (size_t)DM0_SEQ_PAD * 1024; a.out_istride = 64;
         if (c->want("vit attn")) c->note(launch_flash_attention(a, 64, s), "vit attn");
         gemm_residual(c->B("vision_attn"), 1024, M, c->TW("t_vision_out_proj_w", i), 1024, 1024, c->W("vision_out_proj_b", 1024, i), c->B("vision_x_2d"),

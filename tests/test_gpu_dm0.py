@@ -179,6 +179,33 @@ def check_case(case, tag):
     assert layer[worst] <= LAYER_TOL, (worst, layer[worst])
     assert all(v <= MAE_TOL for k, v in errs.items() if k.startswith("euler"))
 
+# The ViT attention on its own: queries that carry scale * log2(e), S^T started from minus the running maximum.  From the operands that the layer left,
+# in fp32; plain rows, logits several times as sharp, and keys that grow along the sequence, so that maxima grow all the way through the key loop.
+@pytest.mark.parametrize("first,last", [(1.0, 1.0), (6.0, 6.0), (0.2, 9.0)])
+def test_vit_attention_from_the_operands_of_its_layer(first, last):
+    from _engine import untile_ft, untile_vt
+    import rtvla_capi as capi
+    from dm0_infer import DM0Inference
+    ck = syn.dm0_checkpoint(31, "cuda:0", 1, 1, vocab=300)
+    m = DM0Inference(ck, num_images=1, max_lang_len=8)
+    B = m.buffers
+    g = torch.Generator(device="cuda:0").manual_seed(5)
+    x = torch.randn(2720, 1024, device="cuda:0", generator=g) * torch.linspace(first, last, 2720, device="cuda:0")[:, None]
+    B["vision_x_norm"][:2720].copy_(x)
+    m._engine.run_stage(capi.STAGE_VISION_LAYER, 0, 0)
+    torch.cuda.synchronize()
+    worst = 0.0
+    for h in range(16):
+        q, k = (untile_ft(B[n][h], 2720, 64)[:2705].float() for n in ("vision_Q", "vision_K"))
+        v = untile_vt(B["vision_Vt"][h], 64, 2720).t()[:2705].float()
+        ref = torch.softmax((q @ k.t()) * 0.6931471805599453, -1) @ v                    # exponents of 2
+        got = B["vision_attn"].view(-1, 1024)[:2705, 64 * h: 64 * h + 64].float()
+        assert torch.isfinite(got).all()
+        worst = max(worst, ((got - ref).norm() / ref.norm()).item())
+    # probabilities and result rounded to bf16 (2^-9 each), the row sum from the rounded probabilities
+    assert worst <= 1e-2, worst
+
+
 
 def test_dm0_reduced_depth_staged_and_graph():
     check_case(Case(61, 1, 6, 2, 2), "dm0_small")

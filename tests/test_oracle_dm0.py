@@ -159,6 +159,23 @@ def test_norm_of_queries_and_keys_as_a_scalar_of_the_logit(scale, factor, outlie
     assert not torch.equal(scaled(bf16), before)
 
 
+@pytest.mark.parametrize("spread", [0.1, 1.0, 3.0, 8.0])
+def test_vit_queries_rounded_behind_the_softmax_scale(spread):
+    """The HIP path rounds the ViT's rotated queries to bf16 times scale * log2(e), the reference without it and scales the logits: one rounding either
+    way, so the attention output is no further off 64 bits."""
+    g = torch.Generator().manual_seed(int(spread * 10))
+    q, k, v = (torch.randn(8, 400, 64, generator=g).double() for _ in range(3))
+    q, k, v = q * spread, k.bfloat16().double(), v.bfloat16().double()
+    out = lambda logits: torch.softmax(logits, -1) @ v
+    exact = out(q @ k.transpose(1, 2) * 0.125)
+    c = 0.125 * 1.4426950408889634
+    before = out(q.bfloat16().double() @ k.transpose(1, 2) * 0.125)
+    now = out((q * c).bfloat16().double() @ k.transpose(1, 2) * 0.6931471805599453)
+    off = lambda got: ((got - exact).norm() / exact.norm()).item()
+    # (measured 0.994 - 1.012 of each other)
+    assert off(now) <= 1.05 * off(before) + 1e-12 and off(before) < 0.05
+
+
 def test_grouped_query_attention_against_sdpa():
     rows = 9
     q, k, v = torch.randn(rows, 16, 128), torch.randn(rows, 8, 128), torch.randn(rows, 8, 128)
