@@ -75,32 +75,28 @@ __global__ void dm0_gather_rows_kernel(const bf16_t* __restrict__ table, int tab
     *(uint4*)(dst + (size_t)blockIdx.x * 2048 + threadIdx.x * 8) = *(const uint4*)(table + (size_t)id * 2048 + threadIdx.x * 8);
 }
 
-// dm0_infer.py:236-306.  One wave per (row, head) of the bf16 QKV rows [rows][32 heads x 128]: value * RMS factor of the row;
+// dm0_infer.py:236-306, the action expert's rows (the prefix has this in the epilogue of its GEMM: csrc/gemm_scatter.h).  One wave per (row, head) of the
+// bf16 QKV rows [rows][32 heads x 128]: value * RMS factor of the row, computed from the row of the fragment-tiled activation matrix x [64][1024];
 // Q and K heads are RMS-normalised over their 128 features (eps 1e-6), scaled by the norm weight and rotated on adjacent
 // pairs by the row's (cos, sin) table; V heads are only scaled.  Lane l holds features 2l, 2l+1 (one rotation pair).
 // Q head h goes to the fragment-tiled [rows*2][128] matrix of K/V head h/2 at row token*2 + h%2, K to cache row
-// key_row0 + token, V transposed to cache column key_row0 + token.  The factor is read from `factor` or, when that is
-// null, computed from the row of the fragment-tiled activation matrix x [64][1024].
+// key_row0 + token, V transposed to cache column key_row0 + token.
 __global__ __launch_bounds__(256)
-void dm0_qknorm_rope_kernel(const bf16_t* __restrict__ qkv, int ld, const float* __restrict__ factor, const bf16_t* __restrict__ x_tiled,
+void dm0_qknorm_rope_kernel(const bf16_t* __restrict__ qkv, int ld, const bf16_t* __restrict__ x_tiled,
                             const bf16_t* __restrict__ qw, const bf16_t* __restrict__ kw, const bf16_t* __restrict__ rope,
                             bf16_t* __restrict__ q, size_t q_bstride, bf16_t* __restrict__ k, size_t k_bstride,
                             bf16_t* __restrict__ vt, size_t vt_bstride, int keys32, int key_row0, int rows) {
     const int wave = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (wave >= rows * 32) return;
     const int row = wave >> 5, head = wave & 31;
-    float f;
-    if (factor) f = factor[row];
-    else {
-        float ss = 0.f;
+    float ss = 0.f;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const bf16x8 v = *(const bf16x8*)(x_tiled + ft_index(row, (lane * 2 + i) * 8, 32));
+    for (int i = 0; i < 2; ++i) {
+        const bf16x8 v = *(const bf16x8*)(x_tiled + ft_index(row, (lane * 2 + i) * 8, 32));
 #pragma unroll
-            for (int j = 0; j < 8; ++j) ss += bf2f(v[j]) * bf2f(v[j]);
-        }
-        f = rsqrtf(wave_sum(ss) * (1.0f / 1024.0f) + 1e-6f);
+        for (int j = 0; j < 8; ++j) ss += bf2f(v[j]) * bf2f(v[j]);
     }
+    const float f = rsqrtf(wave_sum(ss) * (1.0f / 1024.0f) + 1e-6f);
     const bf16_t* src = qkv + (size_t)row * ld + head * 128 + lane * 2;
     float v0 = bf2f(src[0]) * f, v1 = bf2f(src[1]) * f;
     if (head < 24) {
@@ -149,10 +145,10 @@ void launch_dm0_gather_rows(const bf16_t* table, int table_rows, const int* ids,
     if (rows > 0) hipLaunchKernelGGL(dm0_gather_rows_kernel, dim3(rows), dim3(256), 0, s, table, table_rows, ids, dst);
 }
 
-void launch_dm0_qknorm_rope(const bf16_t* qkv, int ld, const float* factor, const bf16_t* x_tiled, const bf16_t* qw, const bf16_t* kw, const bf16_t* rope,
+void launch_dm0_qknorm_rope(const bf16_t* qkv, int ld, const bf16_t* x_tiled, const bf16_t* qw, const bf16_t* kw, const bf16_t* rope,
                             bf16_t* q, size_t q_bstride, bf16_t* k, size_t k_bstride, bf16_t* vt, size_t vt_bstride, int keys32, int key_row0, int rows,
                             hipStream_t s) {
-    hipLaunchKernelGGL(dm0_qknorm_rope_kernel, dim3((rows * 32 + 3) / 4), dim3(256), 0, s, qkv, ld, factor, x_tiled, qw, kw, rope, q, q_bstride, k, k_bstride,
+    hipLaunchKernelGGL(dm0_qknorm_rope_kernel, dim3((rows * 32 + 3) / 4), dim3(256), 0, s, qkv, ld, x_tiled, qw, kw, rope, q, q_bstride, k, k_bstride,
                        vt, vt_bstride, keys32, key_row0, rows);
 }
 

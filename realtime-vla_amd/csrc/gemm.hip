@@ -296,6 +296,12 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
         }
     } else {
         static_assert(epi_scatters(EPI), "every epilogue is one of the two kinds");
+        if constexpr (EPI == EPI_GQA_QKV) {
+            static_assert(WN == 4 && NT == 1, "a head is 128 columns");
+            scatter_head<MT, V>(p, acc, (float*)smem_raw, m0, tile_of[0] * 32, wn, lane);
+            return;
+        }
+        else
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
             if (m0 + i * 32 >= p.M) continue;
@@ -365,11 +371,11 @@ int launch_cfg(const GemmP& p, hipStream_t s) {
 template <int EPI>
 int launch_epi(const GemmP& p, int tile, hipStream_t s) {
     switch (tile) {
-        case TILE_224x256: return launch_cfg<4, 7, 2, EPI, true>(p, s);
-        case TILE_192x256: return launch_cfg<4, 6, 2, EPI, true>(p, s);
-        case TILE_160x256: return launch_cfg<4, 5, 2, EPI, true>(p, s);
-        case TILE_128x256: return launch_cfg<4, 4, 2, EPI, true>(p, s);
-        case TILE_64x256:  return launch_cfg<4, 2, 2, EPI, false>(p, s);
+        case TILE_224x256: if constexpr (EPI != EPI_GQA_QKV) return launch_cfg<4, 7, 2, EPI, true>(p, s); else return 2;
+        case TILE_192x256: if constexpr (EPI != EPI_GQA_QKV) return launch_cfg<4, 6, 2, EPI, true>(p, s); else return 2;
+        case TILE_160x256: if constexpr (EPI != EPI_GQA_QKV) return launch_cfg<4, 5, 2, EPI, true>(p, s); else return 2;
+        case TILE_128x256: if constexpr (EPI != EPI_GQA_QKV) return launch_cfg<4, 4, 2, EPI, true>(p, s); else return 2;
+        case TILE_64x256:  if constexpr (EPI != EPI_GQA_QKV) return launch_cfg<4, 2, 2, EPI, false>(p, s); else return 2;
         case TILE_64x128:  if constexpr (!EpiTraits<EPI>::dual) return launch_cfg<4, 2, 1, EPI, false>(p, s); else return 2;
         case TILE_128x128: if constexpr (!EpiTraits<EPI>::dual) return launch_cfg<4, 4, 1, EPI, false>(p, s); else return 2;
         case TILE_96x128:  if constexpr (!EpiTraits<EPI>::dual) return launch_cfg<4, 3, 1, EPI, false>(p, s); else return 2;
@@ -396,6 +402,7 @@ int launch_gemm(const GemmP& p, int epi, int tile, hipStream_t s) {
         case EPI_QKV_ROPE:  return launch_epi<EPI_QKV_ROPE>(p, tile, s);
         case EPI_VIS_QKV:   return launch_epi<EPI_VIS_QKV>(p, tile, s);
         case EPI_SWIGLU:    return launch_epi<EPI_SWIGLU>(p, tile, s);
+        case EPI_GQA_QKV:   return launch_epi<EPI_GQA_QKV>(p, tile, s);
     }
     return 2;
 }

@@ -53,6 +53,7 @@ enum GemmEpilogue {
     EPI_QKV_ROPE,      // Gemma prefix: bf16 -> interleaved RoPE on Q,K -> Q / K cache / transposed V cache
     EPI_VIS_QKV,       // SigLIP: +bias, Q|K row-major, V transposed per (view, head)
     EPI_SWIGLU,        // out = silu(acc(B0) * rowscale[row]) * (acc(B1) * rowscale[row])   (DM0 prefix MLP)
+    EPI_GQA_QKV,       // DM0 prefix: bf16, times rowscale, norm over the head and interleaved RoPE on Q, K -> Q / K cache / V^T cache per K/V head
     EPI_VIT_QKV_ROPE,  // DM0 ViT: +bias, bf16, 2-D rotary on Q and K (16 heads x 64), Q / K / V^T per (image, head)
 };
 
@@ -65,12 +66,13 @@ struct GemmP {
     bf16_t* out; int ldo;
     const bf16_t* bias;
     const float* bias_f32;                     // fp32 bias instead of `bias` (DM0's folded LayerNorm biases)
-    const float* rowscale;                     // per-row factor applied to the accumulators (EPI_SWIGLU)
+    const float* rowscale;                     // per-row factor applied to the accumulators (EPI_SWIGLU, EPI_GQA_QKV)
+    const bf16_t *qnorm, *knorm; size_t q_bstride, k_bstride, vt_bstride;      // EPI_GQA_QKV: norm weights [128], elements from one K/V head to the next
     int seq, seq_pad;                          // EPI_VIT_QKV_ROPE: tokens per image and their padded count in the Q / K / V^T tiles
     float qscale;                              // EPI_VIT_QKV_ROPE: factor of the rotated queries, before they are rounded
     const bf16_t* res; int ldr; int res_mod;
     float* partial; int ldp; size_t pstride;   // [split][row][ldp]
-    const bf16_t* rope;                        // [row][256] = cos0 sin0 cos1 sin1 ...
+    const bf16_t* rope;                        // [row][256] = cos0 sin0 cos1 sin1 ... (EPI_GQA_QKV: 128)
     bf16_t* q; bf16_t* k; bf16_t* vt; int ldvt;
 };
 // workgroup tile (rows x columns), 4 waves each owning 64 columns (two 32-column MFMA tiles).  The tiles of 128 rows and
@@ -254,7 +256,7 @@ void launch_dm0_im2col_nchw(const bf16_t* images, bf16_t* patches, int ldp, int 
 void launch_dm0_embed_ln(const bf16_t* conv, const bf16_t* cls, const bf16_t* pos, const bf16_t* w, const bf16_t* b, bf16_t* x, int x_img_rows, int n_images, hipStream_t s);
 void launch_dm0_im2col3x3(const bf16_t* in, int img_rows, int row0, int in_h, int in_w, int C, bf16_t* col, int n_images, hipStream_t s);
 void launch_dm0_gather_rows(const bf16_t* table, int table_rows, const int* ids, bf16_t* dst, int rows, hipStream_t s);
-void launch_dm0_qknorm_rope(const bf16_t* qkv, int ld, const float* factor, const bf16_t* x_tiled, const bf16_t* qw, const bf16_t* kw, const bf16_t* rope,
+void launch_dm0_qknorm_rope(const bf16_t* qkv, int ld, const bf16_t* x_tiled, const bf16_t* qw, const bf16_t* kw, const bf16_t* rope,
                             bf16_t* q, size_t q_bstride, bf16_t* k, size_t k_bstride, bf16_t* vt, size_t vt_bstride, int keys32, int key_row0, int rows,
                             hipStream_t s);
 void launch_scale_inplace(bf16_t* p, size_t n, float f, hipStream_t s);

@@ -156,7 +156,8 @@ constexpr int64_t ATTN_PARTIAL_FLOATS = 64 * 16 * (16 * 64 * 4 + 32);   // 64 ro
 // one, and needed a table for two shapes (SigLIP down-projection at 768 rows, output projection at 1 024) that are within 0.7 us of the best now.  Layer
 // times: SigLIP down-projection at 512 rows 64x128/6 -> 96x128/4 69.4 -> 65.8 us, at 1 024 rows 64x128/2 -> 128x128/3 93.7 -> 89.5; Gemma
 // down-projection at 868 rows 128x128/2 -> 128x256/4 247.7 -> 236.1, output projection at 649 rows 64x128/2 -> 96x128/2 205.2 -> 200.7.
-TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittable, const char* what, bool eight = false, bool scattered = false, bool activation = false) {
+struct TileNeeds { bool eight = false, scattered = false, activation = false, head = false; };      // may take eight waves; the kind of epilogue; 128 columns
+TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittable, const char* what, TileNeeds need = {}) {
     static const int tiles[] = {TILE_224x256, TILE_192x256, TILE_160x256, TILE_128x256, TILE_64x256, TILE_128x128, TILE_96x128, TILE_64x128};
     static const int splits[] = {1, 2, 3, 4, 6, 8};
     { TileChoice forced; if (tuning_forced_tile(what, splittable, &forced.tile, &forced.nsplit)) return forced; }
@@ -166,7 +167,7 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
     // a forward with 788 takes the same with both, 10 053 / 10 057 us), unless 256 rows to a workgroup save a round that 224 need (968 rows: 131 / 116, forward 11 150 / 10 954).
     // Among them the one whose rounds of 256 workgroups cost least: a K stage of 32 takes 0.36 us + 0.0155 us per row tile (8 160 x 4 096 x 1 024 against
     // K = 1 024), first loads and epilogue 1.6 us per row tile - 1.8 us, 2.4 us - 2 us with an activation.
-    if (eight && M >= 640) {
+    if (need.eight && M >= 640) {
         const int cols = (ncols16 + (dual ? 7 : 15)) / (dual ? 8 : 16), row_tiles = (M + 31) / 32;
         auto rounds = [&](int mt) { return ((row_tiles + mt - 1) / mt * cols + 255) / 256; };
         if (dual ? rounds(8) < rounds(7) : (row_tiles + 3) / 4 * cols >= 172) {
@@ -175,17 +176,17 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
             for (int tile : {TILE8_128x256, TILE8_160x256, TILE8_192x256, TILE8_224x256, TILE8_256x256}) {
                 const int m_blocks = gemm8_row_blocks(row_tiles, gemm_tile_bm(tile) / 32, cols);
                 const int mt = (row_tiles + m_blocks - 1) / m_blocks;
-                const double cost = (m_blocks * cols + 255) / 256 * (2 * stages * (0.36 + 0.0155 * mt) + (activation ? 2.4 * mt - 2.0 : 1.6 * mt - 1.8));
+                const double cost = (m_blocks * cols + 255) / 256 * (2 * stages * (0.36 + 0.0155 * mt) + (need.activation ? 2.4 * mt - 2.0 : 1.6 * mt - 1.8));
                 if (cost < least) { least = cost; c8.tile = tile; }
             }
             return c8;
         }
     }
-    double best = 1e30; TileChoice bc{TILE_128x256, 1};
+    double best = 1e30; TileChoice bc{need.head ? TILE_128x128 : TILE_128x256, 1};
     for (int tile : tiles) {
         const int bm = gemm_tile_bm(tile);
         const int bn = gemm_tile_bn(tile);
-        if (dual && bn < 256) continue;
+        if ((dual && bn < 256) || (need.head && bn != 128)) continue;
         const int bn16 = bn / 16 / (dual ? 2 : 1);
         const int mb = (M + bm - 1) / bm, nb = (ncols16 + bn16 - 1) / bn16;
         const int nt = bn / 128;
@@ -206,7 +207,7 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
             const double stage_bytes = (double)(bm + bn) * 64 * 2;
             const double alone_us = std::max(mfma_us, 0.143 + stage_bytes / 9.9e4), pair_us = std::max(occ * mfma_us, 0.143 + occ * stage_bytes / 9.9e4);
             double t = std::max((per_cu / occ * pair_us + per_cu % occ * alone_us) * sps, blocks * (double)sps * stage_bytes / 18.7e6);
-            t += 5.9 + (scattered ? 1.1 : 0.85) * mt * nt;
+            t += 5.9 + (need.scattered ? 1.1 : 0.85) * mt * nt;
             if (splittable) t += 2.2 + (double)sp * M * ncols16 * 16 * 4.0 / 3e6;    // the partials, written and read
             if (t <= best) { best = t; bc = TileChoice{tile, sp}; }      // (of equals the smaller tile)
         }
@@ -488,7 +489,6 @@ int build_tables_dm0(rtvla_ctx* c) {
     c->add_buf("vision_col2", n * DM0_TOK, 18432, 18432);
     c->add_buf("vision_mm2", n * DM0_TOK, 4096, 4096);
     c->add_buf("prefix_x", P, 2048, 2048);
-    c->add_buf("prefix_qkv", P, 4096, 4096);
     c->add_buf("prefix_Q", 8, ((2 * P + 31) / 32) * 32 * 128, ((2 * P + 31) / 32) * 32 * 128);     // per K/V head: fragment-tiled [token*2 + head][128]
     c->add_buf("prefix_attn", P, 2048, 2048);
     c->add_buf("prefix_hidden", P, 6144, 6144);
@@ -558,9 +558,10 @@ struct Sched {
         GemmP p = extra;
         p.A = A; p.lda = lda; p.a_rows = a_rows; p.M = M; p.B0 = B0; p.B1 = B1;
         p.N16 = n16_tiles(N); p.K32p = k32_padded(K); p.bgroup = bgroup;
-        const bool dual = epi == EPI_GEGLU || epi == EPI_SWIGLU;
-        const TileChoice tc = choose_tile(M, p.N16, p.K32p / 2, dual, epi == EPI_PARTIAL, what, dual || epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_RESIDUAL || epi == EPI_VIT_QKV_ROPE,
-                                          epi == EPI_QKV_ROPE || epi == EPI_VIS_QKV || epi == EPI_VIT_QKV_ROPE, dual || epi == EPI_BIAS_GELU);
+        const bool dual = epi == EPI_GEGLU || epi == EPI_SWIGLU, vit_qkv = epi == EPI_VIT_QKV_ROPE, gqa_qkv = epi == EPI_GQA_QKV;
+        const TileNeeds need{dual || epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_RESIDUAL || vit_qkv,
+                             epi == EPI_QKV_ROPE || epi == EPI_VIS_QKV || vit_qkv || gqa_qkv, dual || epi == EPI_BIAS_GELU, gqa_qkv};
+        const TileChoice tc = choose_tile(M, p.N16, p.K32p / 2, dual, epi == EPI_PARTIAL, what, need);
         p.nsplit = tc.nsplit;
         if (epi == EPI_PARTIAL) {
             p.partial = c->B<float>("splitk_partial"); p.ldp = N; p.pstride = (size_t)M * N;
@@ -884,13 +885,10 @@ struct Sched {
     void dm0_prefix_layer(int i) {
         const int P = c->S_e, kp = c->keys_pad;
         const size_t qstride = (size_t)((2 * P + 31) / 32) * 32 * 128;
-        GemmP e{}; e.out = c->B("prefix_qkv"); e.ldo = 4096; e.bias = c->B("const_zeros");
-        gemm(c->B("prefix_x"), 2048, P, P, c->TW("t_llm_attn_qkv_w", i), nullptr, 2048, 4096, EPI_BIAS, e, "prefix qkv");
-        if (c->want("prefix qk-norm rope")) {
-            launch_dm0_qknorm_rope(c->B("prefix_qkv"), 4096, c->B<float>("prefix_norm_factor"), nullptr, c->W("llm_q_norm_w", 128, i), c->W("llm_k_norm_w", 128, i),
-                                   c->W("prefix_rope_weights"), c->B("prefix_Q"), qstride, dK(i), (size_t)kp * 128, dVt(i), (size_t)128 * kp, kp >> 5, 0, P, s);
-            c->note(0, "prefix qk-norm rope");
-        }
+        GemmP e{}; e.rowscale = c->B<float>("prefix_norm_factor"); e.qnorm = c->W("llm_q_norm_w", 128, i); e.knorm = c->W("llm_k_norm_w", 128, i);
+        e.rope = c->W("prefix_rope_weights"); e.q = c->B("prefix_Q"); e.k = dK(i); e.vt = dVt(i); e.ldvt = kp;
+        e.q_bstride = qstride; e.k_bstride = (size_t)kp * 128; e.vt_bstride = (size_t)128 * kp;
+        gemm(c->B("prefix_x"), 2048, P, P, c->TW("t_llm_attn_qkv_w", i), nullptr, 2048, 4096, EPI_GQA_QKV, e, "prefix qkv");
         if (i == d.llm_layers - 1) return;           // the action expert reads only the K / V cache of the last prefix layer
         AttnP a{};
         a.q = c->B("prefix_Q"); a.k = dK(i); a.vt = dVt(i); a.ldvt = kp;
@@ -928,7 +926,7 @@ struct Sched {
         SkinnyP q{}; q.a_tiled = 1; q.out = c->B("decoder_qkv"); q.ldo = 4096; q.bias = c->B("const_zeros");
         skinny(c->B("decoder_x"), 1024, ch, c->TW("t_decoder_attn_qkv_w", i), nullptr, 1024, 4096, SN_NONE, nullptr, SK_BIAS, q, "suffix qkv");
         if (c->want("suffix qk-norm rope")) {
-            launch_dm0_qknorm_rope(c->B("decoder_qkv"), 4096, nullptr, c->B("decoder_x"), c->W("decoder_q_norm_w", 128, i), c->W("decoder_k_norm_w", 128, i),
+            launch_dm0_qknorm_rope(c->B("decoder_qkv"), 4096, c->B("decoder_x"), c->W("decoder_q_norm_w", 128, i), c->W("decoder_k_norm_w", 128, i),
                                    c->W("decoder_rope_weights"), c->B("decoder_Q"), (size_t)128 * 128, dK(i), (size_t)kp * 128, dVt(i), (size_t)128 * kp, kp >> 5, P, ch, s);
             c->note(0, "suffix qk-norm rope");
         }
@@ -1646,7 +1644,7 @@ int plan_linear_act(int M, int K, int N, int act, int tile, ActPlan* out) {
     ActPlan p{};
     p.dual = act == RTVLA_ACT_GEGLU || act == RTVLA_ACT_SWIGLU;
     p.K128 = k32_padded(K) * 32;
-    p.tile = tile >= 0 ? tile : choose_tile(M, n16_tiles(N), k32_padded(K) / 2, p.dual, false, "linear act", true, false, act != RTVLA_ACT_RESIDUAL).tile;
+    p.tile = tile >= 0 ? tile : choose_tile(M, n16_tiles(N), k32_padded(K) / 2, p.dual, false, "linear act", {true, false, act != RTVLA_ACT_RESIDUAL, false}).tile;
     if (p.dual && tile >= 0 && (gemm_tile_bn(tile) != 256 || gemm_tile_eight_waves(tile))) return RTVLA_ERR_LIMIT;      // gate and up share a 256-column workgroup tile
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const int G = p.dual ? 4 : 8;

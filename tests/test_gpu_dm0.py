@@ -206,6 +206,43 @@ def test_vit_attention_from_the_operands_of_its_layer(first, last):
     assert worst <= 1e-2, worst
 
 
+# The prefix QKV GEMM normalises and rotates its heads itself: prompts that end inside, at and one past a 32-row tile, a row tile of the workgroup and a key
+# tile; heads and rows of different sizes, which their norms have to undo; the cache behind the prompt stays as it is.
+@pytest.mark.parametrize("images,lang", [(1, 7), (1, 23), (1, 24), (1, 88), (2, 100), (3, 100), (3, 300)])
+def test_prefix_heads_are_normalised_by_their_gemm(images, lang):
+    from _engine import untile_ft, untile_vt
+    import rtvla_capi as capi
+    from dm0_infer import DM0Inference
+    from oracle import dm0 as o, ops
+    ck = syn.dm0_checkpoint(33, "cuda:0", 1, 1, vocab=64)
+    g = torch.Generator(device="cuda:0").manual_seed(6)
+    ck["llm_attn_qkv_w"] *= torch.linspace(0.2, 5.0, 32, device="cuda:0").to(torch.bfloat16).repeat_interleave(128)
+    for n in ("llm_q_norm_w", "llm_k_norm_w"):
+        ck[n].copy_(1 + 0.2 * torch.randn(ck[n].shape, device="cuda:0", generator=g))
+    m = DM0Inference(ck, num_images=images, max_lang_len=lang)
+    B, P = m.buffers, m.prefix_len
+    x = torch.randn(P, 2048, device="cuda:0", generator=g) * torch.logspace(-1, 1, P, device="cuda:0")[:, None]
+    B["prefix_x"].copy_(x)
+    xc = B["prefix_x"].float().cpu()
+    factor = ops.rms_factor(xc)
+    B["prefix_norm_factor"].reshape(-1).copy_(factor[:, 0].to("cuda"))
+    B["kv_K"].fill_(3); B["kv_Vt"].fill_(3)
+    m._engine.run_stage(capi.STAGE_PREFIX_LAYER, 0, 0)
+    torch.cuda.synchronize()
+    kp = B["kv_K"].shape[1] // 128
+    Q = torch.stack([untile_ft(B["prefix_Q"][h], B["prefix_Q"].shape[1] // 128, 128)[: 2 * P].reshape(P, 2, 128) for h in range(8)], 1).reshape(P, 16, 128)
+    K = torch.stack([untile_ft(B["kv_K"][h], kp, 128) for h in range(8)], 1)
+    V = torch.stack([untile_vt(B["kv_Vt"][h], 128, kp).t() for h in range(8)], 1)
+    assert bool((K[P:] == 3).all()) and bool((V[P:] == 3).all())
+    ref = o.qknorm_rope_split(xc @ ck["llm_attn_qkv_w"][0].float().cpu(), factor, ck["llm_q_norm_w"][0].cpu(), ck["llm_k_norm_w"][0].cpu(),
+                              o.rope_table(0, P), lambda t: t)
+    # each element rounded twice to bf16 (the product, the result), at most 2^-9 of itself each; the product's rounding moves a pair's partner as well and
+    # the table is bf16 too: 2^-9 (1 + 2 sqrt(2)) at worst over a whole head, and errors of a head average to about 1 / sqrt(3) of that
+    for name, got, want in (("Q", Q, ref[0]), ("K", K[:P], ref[1]), ("V", V[:P], ref[2])):
+        got, want = got.float().cpu(), want.reshape(got.shape).float()
+        err = (got - want).norm(dim=-1) / want.norm(dim=-1)
+        assert err.max().item() <= 2 ** -9 * 3.83, (name, err.max().item())
+
 
 def test_dm0_reduced_depth_staged_and_graph():
     check_case(Case(61, 1, 6, 2, 2), "dm0_small")
