@@ -94,11 +94,13 @@ RTVLA_DEVICE float halves_sum(float v) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// the 16 lanes of a row: quads by lane permutes, then mirrors of half a row and of a row, all inside the VALU
 RTVLA_DEVICE float wave_sum(float v) {
-    v = rows_sum(v);
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0xB1, 0xf, 0xf, true));       // quad_perm [1 0 3 2]
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x4E, 0xf, 0xf, true));       // quad_perm [2 3 0 1]
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x141, 0xf, 0xf, true));      // row_half_mirror
+    v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x140, 0xf, 0xf, true));      // row_mirror
+    return rows_sum(v);
 }
 
 // Pulling weight tiles that a LATER launch of the same graph will stream towards the caches: every thread reads one word of

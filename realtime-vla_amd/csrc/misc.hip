@@ -31,54 +31,69 @@ __global__ void pretile_kernel(const bf16_t* __restrict__ W, int K, int N, bf16_
 // One workgroup per row: x = bf16(res + bias + sum_s partial[s]); optional normalised copy.
 // Replaces merge_split_k_bias_res + layer_norm_small_kernel / rms_norm_kernel
 // (/root/reference/pi0_infer.py:325-346, :366-382, :648-663).
+// Bound by latency at 256 rows and by the partials it reads at 788 x 2 048 x 4: everything that the row needs is requested before the first use, so that
+// it pays one trip to memory, not one per operand and group, and a sum over the row crosses its waves behind one barrier.  us per launch, one trip
+// per operand / this: 768 x 1 152 rows of 3 splits with LayerNorm 6.7 / 5.75, of 2 6.25 / 5.3, 788 x 2 048 of 4 with RMSNorm 8.7 / 8.3 (a launch that
+// does nothing is 4.6 in the same trace).  Two waves to a row instead of four: the same within 0.1 at 768 rows, 0.1 - 0.6 more at 256.
 template <int NORM, int NSPLIT>
 __global__ __launch_bounds__(256)
 void reduce_kernel(ReduceP p) {
-    __shared__ float red[8];
+    constexpr int NG = 2;                      // N <= 2048; a group past the row reads the last one again and is dropped
+    __shared__ float red[2][4];
     const int m = blockIdx.x;
     const int tid = threadIdx.x;
-    const int nq = p.N >> 2;                   // float4 groups per row (N <= 2048 -> at most 2 per thread)
-    f32x4 v[2];
+    const int nq = p.N >> 2;                   // groups of four columns
+    f32x4 part[NG][NSPLIT > 0 ? NSPLIT : 1], v[NG];
+    bf16x4 b[NG], rr[NG], w[NG], nb[NG];
+#pragma unroll
+    for (int it = 0; it < NG; ++it) {
+        const int n0 = min(tid + it * 256, nq - 1) * 4;
+#pragma unroll
+        for (int sp = 0; sp < NSPLIT; ++sp) part[it][sp] = *(const f32x4*)(p.partial + (size_t)sp * p.pstride + (size_t)m * p.ldp + n0);
+    }
+    if (p.res)
+#pragma unroll
+        for (int it = 0; it < NG; ++it) rr[it] = load4(p.res + (size_t)m * p.ldr + min(tid + it * 256, nq - 1) * 4);
+    if (p.bias)
+#pragma unroll
+        for (int it = 0; it < NG; ++it) b[it] = load4(p.bias + min(tid + it * 256, nq - 1) * 4);
+    if constexpr (NORM == NORM_LAYER)
+#pragma unroll
+        for (int it = 0; it < NG; ++it) {
+            const int n0 = min(tid + it * 256, nq - 1) * 4;
+            w[it] = load4(p.nw + n0); nb[it] = load4(p.nb + n0);
+        }
     float s = 0.f;
 #pragma unroll
-    for (int it = 0; it < 2; ++it) {
+    for (int it = 0; it < NG; ++it) {
         const int c = tid + it * 256;
-        v[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (c < nq) {
-            const int n0 = c * 4;
-            // the split count is a template argument so that every partial is requested before the first add
-            f32x4 part[NSPLIT > 0 ? NSPLIT : 1];
+        f32x4 a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int sp = 0; sp < NSPLIT; ++sp) part[sp] = *(const f32x4*)(p.partial + (size_t)sp * p.pstride + (size_t)m * p.ldp + n0);
-            f32x4 a = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int sp = 0; sp < NSPLIT; ++sp) a += part[sp];
-            if (p.bias) { const bf16x4 b = load4(p.bias + n0); for (int e = 0; e < 4; ++e) a[e] += bf2f(b[e]); }
-            if (p.res) { const bf16x4 rr = load4(p.res + (size_t)m * p.ldr + n0); for (int e = 0; e < 4; ++e) a[e] += bf2f(rr[e]); }
-            const bf16x4 xb = pack4(a);
-            if (p.x) store4(p.x + (size_t)m * p.ldx + n0, xb);
-            for (int e = 0; e < 4; ++e) a[e] = bf2f(xb[e]);       // the norm reads the bf16 stream
-            v[it] = a;
-            if (NORM == NORM_RMS) s += a[0] * a[0] + a[1] * a[1] + a[2] * a[2] + a[3] * a[3];
-            else s += a[0] + a[1] + a[2] + a[3];
-        }
+        for (int sp = 0; sp < NSPLIT; ++sp) a += part[it][sp];
+        if (p.bias) { for (int e = 0; e < 4; ++e) a[e] += bf2f(b[it][e]); }
+        if (p.res) { for (int e = 0; e < 4; ++e) a[e] += bf2f(rr[it][e]); }
+        const bf16x4 xb = pack4(a);
+        if (p.x && c < nq) store4(p.x + (size_t)m * p.ldx + c * 4, xb);
+        for (int e = 0; e < 4; ++e) a[e] = c < nq ? bf2f(xb[e]) : 0.f;       // the norm reads the bf16 stream
+        v[it] = a;
+        if (NORM == NORM_RMS) s += a[0] * a[0] + a[1] * a[1] + a[2] * a[2] + a[3] * a[3];
+        else s += a[0] + a[1] + a[2] + a[3];
     }
     if (NORM == NORM_NONE) return;
-    auto block_sum = [&](float x) {
+    auto block_sum = [&](float x, int k) {
         x = wave_sum(x);
+        if ((tid & 63) == 0) red[k][tid >> 6] = x;
         __syncthreads();
-        if ((tid & 63) == 0) red[tid >> 6] = x;
-        __syncthreads();
-        return red[0] + red[1] + red[2] + red[3];
+        return red[k][0] + red[k][1] + red[k][2] + red[k][3];
     };
-    const float tot = block_sum(s);
+    const float tot = block_sum(s, 0);
     const float inv_n = 1.0f / (float)p.N;
     if (NORM == NORM_RMS) {
         const float f = rsqrtf(tot * inv_n + p.eps);
         if (p.factor && tid == 0) p.factor[m] = f;
         if (p.xn) {
 #pragma unroll
-            for (int it = 0; it < 2; ++it) {
+            for (int it = 0; it < NG; ++it) {
                 const int c = tid + it * 256;
                 if (c < nq) store4(p.xn + (size_t)m * p.ldxn + c * 4, pack4(v[it] * f));
             }
@@ -87,41 +102,38 @@ void reduce_kernel(ReduceP p) {
         const float mean = tot * inv_n;
         float q = 0.f;
 #pragma unroll
-        for (int it = 0; it < 2; ++it) {
+        for (int it = 0; it < NG; ++it) {
             const int c = tid + it * 256;
-            if (c < nq) for (int e = 0; e < 4; ++e) { const float d = v[it][e] - mean; q += d * d; }
+            for (int e = 0; e < 4; ++e) { const float d = c < nq ? v[it][e] - mean : 0.f; q += d * d; }
         }
-        const float var = block_sum(q) * inv_n;
+        const float var = block_sum(q, 1) * inv_n;
         const float inv_std = 1.0f / sqrtf(var + p.eps);
 #pragma unroll
-        for (int it = 0; it < 2; ++it) {
+        for (int it = 0; it < NG; ++it) {
             const int c = tid + it * 256;
-            if (c < nq) {
-                const int n0 = c * 4;
-                const bf16x4 w = load4(p.nw + n0), b = load4(p.nb + n0);
-                f32x4 o;
-                for (int e = 0; e < 4; ++e) o[e] = (v[it][e] - mean) * inv_std * bf2f(w[e]) + bf2f(b[e]);
-                store4(p.xn + (size_t)m * p.ldxn + n0, pack4(o));
-            }
+            f32x4 o;
+            for (int e = 0; e < 4; ++e) o[e] = (v[it][e] - mean) * inv_std * bf2f(w[it][e]) + bf2f(nb[it][e]);
+            if (c < nq) store4(p.xn + (size_t)m * p.ldxn + c * 4, pack4(o));
         }
     }
 }
 
 // LayerNorm of bf16 rows of 1024, four rows per workgroup: with nothing to sum, a row is one 32-byte piece per lane, so one wave holds
-// it and no barrier is needed.  Bound by memory (2 + 2 bytes per element): 8 160 rows in
-// 6.5 us = 5.1 TB/s.
+// it and no barrier is needed.  Bound by memory (2 + 2 bytes per element): 8 160 rows in 7.5 us with the norm's weights requested behind the sums and
+// these taken by LDS permutes, 6.7 as it stands (5.0 TB/s).
 __global__ __launch_bounds__(256)
 void layer_norm_1024_kernel(ReduceP p) {
     const int m = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (m >= p.M) return;
+    bf16x8 a[2], w[2], b[2];                               // all requested before the first use
+#pragma unroll
+    for (int k = 0; k < 2; ++k) a[k] = *(const bf16x8*)(p.res + (size_t)m * p.ldr + k * 512 + lane * 8);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) { w[k] = *(const bf16x8*)(p.nw + k * 512 + lane * 8); b[k] = *(const bf16x8*)(p.nb + k * 512 + lane * 8); }
     float v[16];
     float s = 0.f;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const bf16x8 a = *(const bf16x8*)(p.res + (size_t)m * p.ldr + k * 512 + lane * 8);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) { v[8 * k + e] = bf2f(a[e]); s += v[8 * k + e]; }
-    }
+    for (int e = 0; e < 16; ++e) { v[e] = bf2f(a[e >> 3][e & 7]); s += v[e]; }
     const float mean = wave_sum(s) * (1.0f / 1024.0f);
     float q = 0.f;
 #pragma unroll
@@ -129,12 +141,10 @@ void layer_norm_1024_kernel(ReduceP p) {
     const float inv_std = 1.0f / sqrtf(wave_sum(q) * (1.0f / 1024.0f) + p.eps);
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-        const int n0 = k * 512 + lane * 8;
-        const bf16x8 w = *(const bf16x8*)(p.nw + n0), b = *(const bf16x8*)(p.nb + n0);
         bf16x8 o;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = f2bf((v[8 * k + e] - mean) * inv_std * bf2f(w[e]) + bf2f(b[e]));
-        *(bf16x8*)(p.xn + (size_t)m * p.ldxn + n0) = o;
+        for (int e = 0; e < 8; ++e) o[e] = f2bf((v[8 * k + e] - mean) * inv_std * bf2f(w[k][e]) + bf2f(b[k][e]));
+        *(bf16x8*)(p.xn + (size_t)m * p.ldxn + k * 512 + lane * 8) = o;
     }
 }
 

@@ -289,6 +289,36 @@ def test_layer_norm_of_1024_wide_rows_alone(M):
     assert (out[M] == 9.0).all()
 
 
+# Groups of four columns past the row read the last one again: rows that end inside, at and just behind a pass of 256 groups, in place, next row untouched;
+# against float64: half a bf16 step of the sum and of the result, and of the sum's terms fp32 errors.
+@pytest.mark.parametrize("N", [4, 252, 1020, 1024, 1028, 2044, 2048])
+@pytest.mark.parametrize("nsplit,norm", [(2, 2), (3, 1), (8, 0), (0, 2)])
+def test_reduce_rows_that_end_around_a_pass(N, nsplit, norm):
+    import rtvla_capi as capi
+    lib = capi.load()
+    g = torch.Generator(device="cuda:0").manual_seed(N + nsplit)
+    M = 3
+    parts = torch.randn(max(nsplit, 1), M, N, device="cuda:0", generator=g)
+    bias, nw, nb = (torch.randn(N, device="cuda:0", generator=g).bfloat16() for _ in range(3))
+    x = torch.full((M + 1, N), 9.0, dtype=torch.bfloat16, device="cuda:0")
+    x[:M] = torch.randn(M, N, device="cuda:0", generator=g)
+    res = x[:M].clone()
+    xn = torch.full((M + 1, N), 9.0, dtype=torch.bfloat16, device="cuda:0")
+    assert lib.rtvla_reduce_norm(_P(parts.data_ptr()) if nsplit else None, nsplit, M, N, _P(bias.data_ptr()), _P(x.data_ptr()), norm, _P(nw.data_ptr()),
+                                 _P(nb.data_ptr()), ctypes.c_float(1e-5), _P(x.data_ptr()), _P(xn.data_ptr()) if norm else None,
+                                 _P(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    terms = [bias.double().expand(M, N), res.double()] + [parts[i].double() for i in range(nsplit)]
+    want, size = sum(terms), sum(t.abs() for t in terms)
+    assert ((x[:M].double() - want).abs() <= want.abs() * 2.0 ** -8 + size * 2.0 ** -20).all()
+    xb = x[:M].double()
+    if norm:
+        ref = torch.nn.functional.layer_norm(xb, (N,), nw.double(), nb.double(), 1e-5) if norm == 2 else xb * torch.rsqrt(xb.pow(2).mean(-1, keepdim=True) + 1e-5)
+        assert ((xn[:M].double() - ref).abs() <= ref.abs() * 2.0 ** -8 + 1e-4).all()
+        assert (xn[M] == 9.0).all()
+    assert (x[M] == 9.0).all()
+
+
 @pytest.mark.parametrize("M,N,nsplit,norm,has_bias,has_res", [
     (768, 1152, 2, 2, True, True),        # SigLIP O projection: split 2 + bias + residual + LayerNorm
     (768, 1152, 4, 2, True, True),        # SigLIP down projection
