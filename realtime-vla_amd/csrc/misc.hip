@@ -38,25 +38,26 @@ __global__ void pretile_kernel(const bf16_t* __restrict__ W, int K, int N, bf16_
 template <int NORM, int NSPLIT>
 __global__ __launch_bounds__(256)
 void reduce_kernel(ReduceP p) {
-    constexpr int NG = 2;                      // N <= 2048; a group past the row reads the last one again and is dropped
+    constexpr int NG = 2;                      // 2 048 columns; a group past the row reads the last one again and is dropped
     __shared__ float red[2][4];
     const int m = blockIdx.x;
     const int tid = threadIdx.x;
-    const int nq = p.N >> 2;                   // groups of four columns
+    const int col0 = NORM == NORM_NONE ? blockIdx.y * 2048 : 0;       // (sums alone: wider rows in blocks)
+    const int nq = min(p.N - col0, 2048) >> 2; // groups of four columns
     f32x4 part[NG][NSPLIT > 0 ? NSPLIT : 1], v[NG];
     bf16x4 b[NG], rr[NG], w[NG], nb[NG];
 #pragma unroll
     for (int it = 0; it < NG; ++it) {
-        const int n0 = min(tid + it * 256, nq - 1) * 4;
+        const int n0 = col0 + min(tid + it * 256, nq - 1) * 4;
 #pragma unroll
         for (int sp = 0; sp < NSPLIT; ++sp) part[it][sp] = *(const f32x4*)(p.partial + (size_t)sp * p.pstride + (size_t)m * p.ldp + n0);
     }
     if (p.res)
 #pragma unroll
-        for (int it = 0; it < NG; ++it) rr[it] = load4(p.res + (size_t)m * p.ldr + min(tid + it * 256, nq - 1) * 4);
+        for (int it = 0; it < NG; ++it) rr[it] = load4(p.res + (size_t)m * p.ldr + col0 + min(tid + it * 256, nq - 1) * 4);
     if (p.bias)
 #pragma unroll
-        for (int it = 0; it < NG; ++it) b[it] = load4(p.bias + min(tid + it * 256, nq - 1) * 4);
+        for (int it = 0; it < NG; ++it) b[it] = load4(p.bias + col0 + min(tid + it * 256, nq - 1) * 4);
     if constexpr (NORM == NORM_LAYER)
 #pragma unroll
         for (int it = 0; it < NG; ++it) {
@@ -73,7 +74,7 @@ void reduce_kernel(ReduceP p) {
         if (p.bias) { for (int e = 0; e < 4; ++e) a[e] += bf2f(b[it][e]); }
         if (p.res) { for (int e = 0; e < 4; ++e) a[e] += bf2f(rr[it][e]); }
         const bf16x4 xb = pack4(a);
-        if (p.x && c < nq) store4(p.x + (size_t)m * p.ldx + c * 4, xb);
+        if (p.x && c < nq) store4(p.x + (size_t)m * p.ldx + col0 + c * 4, xb);
         for (int e = 0; e < 4; ++e) a[e] = c < nq ? bf2f(xb[e]) : 0.f;       // the norm reads the bf16 stream
         v[it] = a;
         if (NORM == NORM_RMS) s += a[0] * a[0] + a[1] * a[1] + a[2] * a[2] + a[3] * a[3];
@@ -294,7 +295,7 @@ void launch_pretile_padded(const bf16_t* W, int K, int K_pad, int N, bf16_t* out
 
 template <int NORM>
 static int launch_reduce_norm(const ReduceP& p, hipStream_t s) {
-    const dim3 grid(p.M), block(256);
+    const dim3 grid(p.M, NORM == NORM_NONE ? (p.N + 2047) / 2048 : 1), block(256);
     switch (p.nsplit) {
         case 0: hipLaunchKernelGGL((reduce_kernel<NORM, 0>), grid, block, 0, s, p); break;
         case 1: hipLaunchKernelGGL((reduce_kernel<NORM, 1>), grid, block, 0, s, p); break;
@@ -309,7 +310,7 @@ static int launch_reduce_norm(const ReduceP& p, hipStream_t s) {
 }
 
 int launch_reduce(const ReduceP& p, hipStream_t s) {
-    if (p.M <= 0 || p.N <= 0 || (p.N & 3) || p.N > 2048) return 1;
+    if (p.M <= 0 || p.N <= 0 || (p.N & 3) || (p.N > 2048 && p.norm != NORM_NONE)) return 1;
     if (p.norm == NORM_LAYER && !p.xn) return 1;
     if (p.norm == NORM_RMS && !p.xn && !p.factor) return 1;
     if (p.norm == NORM_LAYER && (!p.nw || !p.nb)) return 1;

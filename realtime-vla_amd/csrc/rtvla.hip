@@ -598,6 +598,20 @@ struct Sched {
         if (xn) reduce(M, N, nullptr, x, N, nullptr, 0, xn, N, NORM_LAYER, nw, nb, eps, 0, what_norm);
     }
 
+    // out = A B + bias for few rows and a long K (DM0's convolutions and projector): one workgroup per tile leaves most of the chip idle, so K is split where
+    // choose_tile finds that to pay, for a pass that sums.  us, whole K / split and summed: 169 x 18 432 x 4 096 128 / 46 + 5, 676 x 9 216 x 2 048 63 / 36 + 8,
+    // 169 x 4 096 x 2 048 31 / 11 + 5; 507 x 18 432 x 4 096 136 / 78 + 9, 2 028 x 9 216 x 2 048 92 / 78 + 6.  Forward with 1, 2, 3, 4 images
+    // 11 950 / 11 815, 15 380 / 15 290, 17 920 / 17 870, 21 610 / 21 545.
+    void gemm_bias_split(const bf16_t* A, int M, const bf16_t* B0, int K, int N, const bf16_t* bias, bf16_t* out, const char* what, const char* what_sum) {
+        if (choose_tile(M, n16_tiles(N), k32_padded(K) / 2, false, true, what).nsplit > 1) {
+            gemm(A, K, M, M, B0, nullptr, K, N, EPI_PARTIAL, GemmP{}, what);
+            reduce(M, N, bias, nullptr, 0, out, N, nullptr, 0, NORM_NONE, nullptr, nullptr, 0.f, last_split, what_sum);
+        } else {
+            GemmP e{}; e.out = out; e.ldo = N; e.bias = bias;
+            gemm(A, K, M, M, B0, nullptr, K, N, EPI_BIAS, e, what);
+        }
+    }
+
     void vision_embed() {
         const int S_v = c->S_v;
         if (c->want("im2col")) { launch_im2col(c->W("observation_images_normalized"), c->B("vision_patches"), PATCH_LD, d.num_views, s); c->note(0, "im2col"); }
@@ -866,13 +880,10 @@ struct Sched {
         const int n = d.num_views, P = c->S_e, T = n * DM0_TOK;
         clear_unseen(dVt(0), d.llm_layers * 8 * 8);
         if (c->want("im2col ds1")) { launch_dm0_im2col3x3(c->B("vision_x_2d"), DM0_SEQ_PAD, 1, 52, 52, 1024, c->B("vision_col1"), n, s); c->note(0, "im2col ds1"); }
-        GemmP e{}; e.out = c->B("vision_mm1"); e.ldo = 2048; e.bias = c->W("vision_ds1_b");
-        gemm(c->B("vision_col1"), 9216, n * 676, n * 676, c->TW("t_vision_ds1_w"), nullptr, 9216, 2048, EPI_BIAS, e, "ds1");
+        gemm_bias_split(c->B("vision_col1"), n * 676, c->TW("t_vision_ds1_w"), 9216, 2048, c->W("vision_ds1_b"), c->B("vision_mm1"), "ds1", "ds1 sum");
         if (c->want("im2col ds2")) { launch_dm0_im2col3x3(c->B("vision_mm1"), 676, 0, 26, 26, 2048, c->B("vision_col2"), n, s); c->note(0, "im2col ds2"); }
-        GemmP f{}; f.out = c->B("vision_mm2"); f.ldo = 4096; f.bias = c->W("vision_ds2_b");
-        gemm(c->B("vision_col2"), 18432, T, T, c->TW("t_vision_ds2_w"), nullptr, 18432, 4096, EPI_BIAS, f, "ds2");
-        GemmP g{}; g.out = c->B("prefix_x"); g.ldo = 2048; g.bias = c->B("const_zeros");
-        gemm(c->B("vision_mm2"), 4096, T, T, c->TW("t_vision_projector_w_t"), nullptr, 4096, 2048, EPI_BIAS, g, "projector");
+        gemm_bias_split(c->B("vision_col2"), T, c->TW("t_vision_ds2_w"), 18432, 4096, c->W("vision_ds2_b"), c->B("vision_mm2"), "ds2", "ds2 sum");
+        gemm_bias_split(c->B("vision_mm2"), T, c->TW("t_vision_projector_w_t"), 4096, 2048, c->B("const_zeros"), c->B("prefix_x"), "projector", "projector sum");
         if (d.prompt_len > 0 && c->want("token embeddings")) {
             launch_dm0_gather_rows(c->W("vision_embed_tokens_w"), (int)c->T("vision_embed_tokens_w").shape[0], (const int*)c->T("input_ids").ptr,
                                    c->B("prefix_x") + (size_t)T * 2048, d.prompt_len, s);

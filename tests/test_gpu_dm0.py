@@ -244,6 +244,28 @@ def test_prefix_heads_are_normalised_by_their_gemm(images, lang):
         assert err.max().item() <= 2 ** -9 * 3.83, (name, err.max().item())
 
 
+# Convolutions and projector split K and sum partials, 4 096 columns wide in two blocks; against fp32 from the operands they left in memory
+@pytest.mark.parametrize("images", [1, 2, 3, 4])
+def test_convolutions_sum_their_splits(images):
+    import rtvla_capi as capi
+    from dm0_infer import DM0Inference
+    ck = syn.dm0_checkpoint(35, "cuda:0", 1, 1, vocab=64)
+    m = DM0Inference(ck, num_images=images, max_lang_len=3)
+    B, T = m.buffers, images * 169
+    x = torch.randn(B["vision_x_2d"].shape, device="cuda:0", generator=torch.Generator(device="cuda:0").manual_seed(7))
+    B["vision_x_2d"].copy_(x)
+    B["splitk_partial"].fill_(float("nan"))
+    m._engine.run_stage(capi.STAGE_PROJECT, 0, 0)
+    torch.cuda.synchronize()
+    for a, w, b, out in (("vision_col1", "vision_ds1_w", "vision_ds1_b", B["vision_mm1"]), ("vision_col2", "vision_ds2_w", "vision_ds2_b", B["vision_mm2"]),
+                         ("vision_mm2", "vision_projector_w_t", None, B["prefix_x"][:T])):
+        w = ck[w].float().reshape(-1, out.shape[1])
+        want = B[a].float().reshape(-1, w.shape[0]) @ w + (ck[b].float() if b else 0.0)
+        err = (out.float() - want).norm(dim=1) / want.norm(dim=1)
+        # rounded once to bf16, at most 2^-9 of each element; fp32 sums of 18 432 products differ by less than a tenth of that
+        assert err.max().item() <= 2.0 ** -9 * 1.1, (a, err.max().item())
+
+
 def test_dm0_reduced_depth_staged_and_graph():
     check_case(Case(61, 1, 6, 2, 2), "dm0_small")
 
