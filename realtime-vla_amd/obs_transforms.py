@@ -32,6 +32,9 @@ class ObservationTransforms:
                 self._stats[group] = (a, b, int(a.numel()))
         self._index = self.device.index if self.device.index is not None else torch.cuda.current_device()
         self.device = torch.device("cuda", self._index)
+        # what results are allocated like: cheaper than naming a type and a device in each call
+        self._row = torch.empty(32, dtype=torch.float64, device=self.device)
+        self._bin_row = torch.empty(32, dtype=torch.int32, device=self.device)
 
     def _stream(self):
         return torch._C._cuda_getCurrentRawStream(self._index)      # the bare handle: the Stream object costs more than a launch
@@ -101,9 +104,9 @@ class ObservationTransforms:
             return None, None
         a, b, n_stats = self._stats["state"]
         st = np.ascontiguousarray(state, dtype=np.float64)         # travels with the launch
-        z = torch.empty(32, dtype=torch.float64, device=self.device)
-        bins = torch.empty(32, dtype=torch.int32, device=self.device) if want_bins else None
-        rc = self.lib.rtvla_preprocess_state_host(st.__array_interface__["data"][0], st.size, a.data_ptr(), b.data_ptr(), n_stats, self.mode,
+        z = torch.empty_like(self._row)
+        bins = torch.empty_like(self._bin_row) if want_bins else None
+        rc = self.lib.rtvla_preprocess_state_host(st.tobytes(), st.size, a.data_ptr(), b.data_ptr(), n_stats, self.mode,
                                                   out_bf16.data_ptr() if out_bf16 is not None else None, z.data_ptr(),
                                                   bins.data_ptr() if bins is not None else None, self._stream())
         if rc:
@@ -122,7 +125,7 @@ class ObservationTransforms:
         st = np.ascontiguousarray(ori_state, dtype=np.float64)
         out = torch.empty((chunk, self.action_dim), dtype=torch.float64, device=self.device)
         rc = self.lib.rtvla_postprocess_actions_host(actions_bf16.data_ptr(), chunk, a.data_ptr(), b.data_ptr(), n_stats, self.mode,
-                                                     st.__array_interface__["data"][0], st.size, self.action_dim, out.data_ptr(), self._stream())
+                                                     st.tobytes(), st.size, self.action_dim, out.data_ptr(), self._stream())
         if rc:
             self._check(rc, "rtvla_postprocess_actions_host")
         return out
