@@ -48,6 +48,26 @@ def test_frame_formats_at_the_edges_of_the_tiles(h, w, fmt):
     assert torch.equal(out.cpu(), want)
 
 
+@pytest.mark.parametrize("h,w", [(224, 224), (225, 224), (226, 301), (1080, 1920), (1920, 1079), (2065, 2065), (2066, 2066)])
+@pytest.mark.parametrize("chw", [False, True])
+def test_float_frames_staged_and_not(h, w, chw):
+    """Either side of the rule that stages float frames in LDS (more than 4 taps, 76 KB); frames that start between two 16-byte pieces; values
+    whose low byte counts."""
+    from oracle import transforms as T
+    from obs_transforms import ObservationTransforms
+    tr = ObservationTransforms("pi0")
+    x = (np.random.RandomState(h + w).rand(h, w, 3) * 3 - 1).astype(np.float32)
+    if chw:
+        x = x.transpose(2, 0, 1).copy()
+    want = torch.from_numpy(T.normalize_image(T.resize_with_pad((255 * (x.transpose(1, 2, 0) if chw else x)).astype(np.int32).astype(np.uint8)))).to(torch.bfloat16)
+    room = torch.empty(x.size + 1, dtype=torch.float32, device="cuda:0")
+    frame = room[1:].view(x.shape)
+    frame.copy_(torch.from_numpy(x))
+    out = torch.full((224, 224, 3), 7.0, dtype=torch.bfloat16, device="cuda:0")
+    tr.resize_pad_normalize_into(frame, out)
+    assert torch.equal(out.cpu(), want)
+
+
 def test_image_inputs_float_and_chw_and_errors():
     from oracle import transforms as T
     from obs_transforms import ObservationTransforms
