@@ -188,6 +188,30 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
             if (s < s_end) stage(b0, b1, last, breg0, areg0, areg1);
         }
     }
+    // the bias of this wave's columns, asked for as one: a load per group of four columns is a branch and a trip to the cache for each
+    constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU || EPI == EPI_PATCH || EPI == EPI_RESIDUAL;
+    f32x4 bias[BIAS ? HALF : 1][4];
+    if constexpr (BIAS) {
+        auto col = [&](int j, int grp) { return min((n_blk * (WN * HALF) + wn * HALF + j) * 32 + 8 * grp + 4 * h, p.N16 * 16 - 4); };      // clamped: columns past the end are never copied out
+        if (p.bias_f32) {
+#pragma unroll
+            for (int j = 0; j < HALF; ++j)
+#pragma unroll
+                for (int grp = 0; grp < 4; ++grp) bias[j][grp] = *(const f32x4*)(p.bias_f32 + col(j, grp));
+        } else {
+            bf16x4 b[HALF][4];
+#pragma unroll
+            for (int j = 0; j < HALF; ++j)
+#pragma unroll
+                for (int grp = 0; grp < 4; ++grp) b[j][grp] = load4(p.bias + col(j, grp));
+#pragma unroll
+            for (int j = 0; j < HALF; ++j)
+#pragma unroll
+                for (int grp = 0; grp < 4; ++grp)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) bias[j][grp][e] = bf2f(b[j][grp][e]);
+        }
+    }
     __syncthreads();                                        // the epilogue reuses the stage buffers
 
     // ---- epilogue: lane (h, r) holds rows m = m0 + 32 i + r, columns n = 32 tile + 8 grp + 4 h + e ----
@@ -245,12 +269,7 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
                         v *= f; u *= f;
                         *(bf16x4*)dst = pack4(siluf(v[0]) * u[0], siluf(v[1]) * u[1], siluf(v[2]) * u[2], siluf(v[3]) * u[3]);
                     } else {
-                        if (p.bias_f32) v += *(const f32x4*)(p.bias_f32 + n0);
-                        else {
-                            const bf16x4 b = load4(p.bias + n0);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) v[e] += bf2f(b[e]);
-                        }
+                        v += bias[j][grp];
                         if constexpr (EPI == EPI_PATCH) {
                             const bf16x4 rs = load4(p.res + (size_t)(min(m, p.M - 1) % p.res_mod) * p.ldr + n0);
 #pragma unroll

@@ -150,9 +150,33 @@ RTVLA_DEVICE void gemm8_block(const GemmP& p, unsigned char* smem_raw, int m0, i
         for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    // the bias of this wave's columns, asked for ahead of the loop (bf16: in the lower half of the registers until the loop has ended)
+    constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU || EPI == EPI_PATCH || EPI == EPI_RESIDUAL;
+    f32x4 bias[BIAS ? HALF : 1][4];
+    if constexpr (BIAS) {
+#pragma unroll
+        for (int j = 0; j < HALF; ++j)
+#pragma unroll
+            for (int grp = 0; grp < 4; ++grp) {
+                const int n0 = min(tile_of[j] * 32 + 8 * grp + 4 * h, p.N16 * 16 - 4);        // clamped: columns past the end are never copied out
+                if (p.bias_f32) bias[j][grp] = *(const f32x4*)(p.bias_f32 + n0);
+                else *(bf16x4*)&bias[j][grp] = load4(p.bias + n0);
+            }
+    }
     if (MT % 2 == 0 || wm == 0) gemm8_loop<MT, MTW, RING, DUAL, V>(p, smem_raw, m0, n_blk, i0, s_begin, s_end, acc);
     else gemm8_loop<MT, MT / 2, RING, DUAL, V>(p, smem_raw, m0, n_blk, i0, s_begin, s_end, acc);
 
+    if constexpr (BIAS) {
+        if (!p.bias_f32)
+#pragma unroll
+            for (int j = 0; j < HALF; ++j)
+#pragma unroll
+                for (int grp = 0; grp < 4; ++grp) {
+                    const bf16x4 b = *(const bf16x4*)&bias[j][grp];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) bias[j][grp][e] = bf2f(b[e]);
+                }
+    }
     if constexpr (epi_scatters(EPI)) {
 #pragma unroll
         for (int k = 0; k < MTW; ++k) {
@@ -212,12 +236,7 @@ RTVLA_DEVICE void gemm8_block(const GemmP& p, unsigned char* smem_raw, int m0, i
                         v *= f; u *= f;
                         *(bf16x4*)dst = pack4(siluf(v[0]) * u[0], siluf(v[1]) * u[1], siluf(v[2]) * u[2], siluf(v[3]) * u[3]);
                     } else {
-                        if (p.bias_f32) v += *(const f32x4*)(p.bias_f32 + n0);
-                        else {
-                            const bf16x4 b = load4(p.bias + n0);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) v[e] += bf2f(b[e]);
-                        }
+                        v += bias[j][grp];
                         if constexpr (EPI == EPI_PATCH) {
                             const bf16x4 rs = load4(p.res + (size_t)(min(m, p.M - 1) % p.res_mod) * p.ldr + n0);
 #pragma unroll
