@@ -212,6 +212,10 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
                     for (int e = 0; e < 4; ++e) bias[j][grp][e] = bf2f(b[j][grp][e]);
         }
     }
+    float factor[EPI == EPI_SWIGLU ? MT : 1];
+    if constexpr (EPI == EPI_SWIGLU)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) factor[i] = p.rowscale[min(m0 + i * 32 + r, p.M - 1)];
     __syncthreads();                                        // the epilogue reuses the stage buffers
 
     // ---- epilogue: lane (h, r) holds rows m = m0 + 32 i + r, columns n = 32 tile + 8 grp + 4 h + e ----
@@ -264,7 +268,7 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
                         const f32x4 u = {acc[i][j + HALF][4 * grp], acc[i][j + HALF][4 * grp + 1], acc[i][j + HALF][4 * grp + 2], acc[i][j + HALF][4 * grp + 3]};
                         *(bf16x4*)dst = pack4(gelu_tanh(v[0]) * u[0], gelu_tanh(v[1]) * u[1], gelu_tanh(v[2]) * u[2], gelu_tanh(v[3]) * u[3]);
                     } else if constexpr (EPI == EPI_SWIGLU) {
-                        const float f = p.rowscale[min(m, p.M - 1)];
+                        const float f = factor[i];
                         f32x4 u = {acc[i][j + HALF][4 * grp], acc[i][j + HALF][4 * grp + 1], acc[i][j + HALF][4 * grp + 2], acc[i][j + HALF][4 * grp + 3]};
                         v *= f; u *= f;
                         *(bf16x4*)dst = pack4(siluf(v[0]) * u[0], siluf(v[1]) * u[1], siluf(v[2]) * u[2], siluf(v[3]) * u[3]);
@@ -320,14 +324,7 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
             scatter_head<MT, V>(p, acc, (float*)smem_raw, m0, tile_of[0] * 32, wn, lane);
             return;
         }
-        else
-#pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            if (m0 + i * 32 >= p.M) continue;
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-                if (tile_of[j] * 32 < p.N16 * 16) scatter_tile<EPI, V>(p, acc[i][j], m0 + i * 32, tile_of[j] * 32, lane);
-        }
+        else scatter_tiles<EPI, V>(p, acc, MT, m0, tile_of, lane);
     }
 }
 

@@ -163,6 +163,10 @@ RTVLA_DEVICE void gemm8_block(const GemmP& p, unsigned char* smem_raw, int m0, i
                 else *(bf16x4*)&bias[j][grp] = load4(p.bias + n0);
             }
     }
+    float factor[EPI == EPI_SWIGLU ? MTW : 1];
+    if constexpr (EPI == EPI_SWIGLU)
+#pragma unroll
+        for (int k = 0; k < MTW; ++k) factor[k] = p.rowscale[min(m0 + (i0 + k) * 32 + r, p.M - 1)];
     if (MT % 2 == 0 || wm == 0) gemm8_loop<MT, MTW, RING, DUAL, V>(p, smem_raw, m0, n_blk, i0, s_begin, s_end, acc);
     else gemm8_loop<MT, MT / 2, RING, DUAL, V>(p, smem_raw, m0, n_blk, i0, s_begin, s_end, acc);
 
@@ -178,14 +182,7 @@ RTVLA_DEVICE void gemm8_block(const GemmP& p, unsigned char* smem_raw, int m0, i
                 }
     }
     if constexpr (epi_scatters(EPI)) {
-#pragma unroll
-        for (int k = 0; k < MTW; ++k) {
-            const int mt0 = m0 + (i0 + k) * 32;
-            if (k >= mtw || mt0 >= p.M) continue;
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-                if (tile_of[j] * 32 < p.N16 * 16) scatter_tile<EPI, V>(p, acc[k][j], mt0, tile_of[j] * 32, lane);
-        }
+        scatter_tiles<EPI, V>(p, acc, mtw, m0 + 32 * i0, tile_of, lane);
         return;
     }
     // ---- epilogue: lane (h, r) holds rows m0 + 32 (i0 + i) + r, columns 32 tile + 8 grp + 4 h + e.  The k-th row tiles of
@@ -231,7 +228,7 @@ RTVLA_DEVICE void gemm8_block(const GemmP& p, unsigned char* smem_raw, int m0, i
                         const f32x4 u = {acc[k][j + HALF][4 * grp], acc[k][j + HALF][4 * grp + 1], acc[k][j + HALF][4 * grp + 2], acc[k][j + HALF][4 * grp + 3]};
                         *(bf16x4*)dst = pack4(gelu_tanh(v[0]) * u[0], gelu_tanh(v[1]) * u[1], gelu_tanh(v[2]) * u[2], gelu_tanh(v[3]) * u[3]);
                     } else if constexpr (EPI == EPI_SWIGLU) {
-                        const float f = p.rowscale[min(m, p.M - 1)];
+                        const float f = factor[k];
                         f32x4 u = {acc[k][j + HALF][4 * grp], acc[k][j + HALF][4 * grp + 1], acc[k][j + HALF][4 * grp + 2], acc[k][j + HALF][4 * grp + 3]};
                         v *= f; u *= f;
                         *(bf16x4*)dst = pack4(siluf(v[0]) * u[0], siluf(v[1]) * u[1], siluf(v[2]) * u[2], siluf(v[3]) * u[3]);

@@ -16,15 +16,54 @@ RTVLA_DEVICE uint4 swap_halves(uint2 x0, uint2 x1) {
     return uint4{a[0], b[0], a[1], b[1]};
 }
 
-// rows mt0 .. mt0 + 31, columns nt0 .. nt0 + 31 (multiples of 32), mt0 < p.M
+// What a tile needs besides its accumulators.  Asked for ahead where scatter_tiles says so: behind the stores of the tile before, which the compiler may not
+// move loads across, each is a trip to the cache of its own.  us: SigLIP 768 rows x 3 456 13.9 -> 12.9, Gemma 788 x 2 560 22.2 -> 21.6, DM0's prefix 607 x 4 096
+// 22.0 -> 21.0.
+struct ScatterBias { f32x4 v[4]; float b; };               // Q, K: columns nt0 + 8 g + 4 h + e; V: column nt0 + r
+struct ScatterTable { uint4 v[2]; };
+
 template <int EPI, bool V>
-RTVLA_DEVICE void scatter_tile(const GemmP& p, const f32x16& acc, int mt0, int nt0, int lane) {
+RTVLA_DEVICE ScatterBias scatter_bias(const GemmP& p, int nt0, int lane) {
+    ScatterBias o = {};
+    const int h = lane >> 5, r = lane & 31, last = p.N16 * 16 - 4;                     // clamped: columns past the end are not stored
+    if constexpr (V) {
+        if constexpr (EPI == EPI_VIS_QKV) o.b = bf2f(p.bias[min(nt0 + r, last + 3)]);
+        if constexpr (EPI == EPI_VIT_QKV_ROPE) o.b = p.bias_f32[min(nt0 + r, last + 3)];
+    } else {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int n0 = min(nt0 + 8 * g + 4 * h, last);
+            if constexpr (EPI == EPI_VIT_QKV_ROPE) o.v[g] = *(const f32x4*)(p.bias_f32 + n0);
+            if constexpr (EPI == EPI_VIS_QKV) {
+                const bf16x4 b = load4(p.bias + n0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o.v[g][e] = bf2f(b[e]);
+            }
+        }
+    }
+    return o;
+}
+template <int EPI, bool V>
+RTVLA_DEVICE ScatterTable scatter_table(const GemmP& p, int mt0, int nt0, int lane) {
+    ScatterTable o = {};
+    if constexpr (!V) {
+        const int h = lane >> 5, mc = min(mt0 + (lane & 31), p.M - 1);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            if constexpr (EPI == EPI_QKV_ROPE) o.v[q] = *(const uint4*)(p.rope + (size_t)mc * 256 + (nt0 & 255) + 16 * q + 8 * h);
+            if constexpr (EPI == EPI_VIT_QKV_ROPE) o.v[q] = *(const uint4*)(p.rope + (size_t)min(mc - mt0 / p.seq_pad * p.seq_pad, p.seq - 1) * 64 + (nt0 & 63) + 16 * q + 8 * h);
+        }
+    }
+    return o;
+}
+
+// rows mt0 .. mt0 + 31, columns nt0 .. nt0 + 31 (multiples of 32), mt0 < p.M
+template <int EPI, bool V, bool AHEAD>
+RTVLA_DEVICE void scatter_tile(const GemmP& p, const f32x16& acc, const ScatterBias& bias, const ScatterTable& tab, int mt0, int nt0, int lane) {
     const int h = lane >> 5, r = lane & 31;
     if constexpr (V) {
         const int n = nt0 + r;                             // rows mt0 + 8 grp + 4 h + e
-        float b = 0.f;
-        if constexpr (EPI == EPI_VIS_QKV) b = bf2f(p.bias[n]);
-        if constexpr (EPI == EPI_VIT_QKV_ROPE) b = p.bias_f32[n];
+        const float b = bias.b;
         bf16x4 pk[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) pk[g] = pack4(acc[4 * g] + b, acc[4 * g + 1] + b, acc[4 * g + 2] + b, acc[4 * g + 3] + b);
@@ -56,31 +95,20 @@ RTVLA_DEVICE void scatter_tile(const GemmP& p, const f32x16& acc, int mt0, int n
         int tok = mc, img = 0;
         if constexpr (EPI == EPI_VIS_QKV) { img = mc >> 8; tok = mc & 255; }
         if constexpr (EPI == EPI_VIT_QKV_ROPE) { img = mt0 / p.seq_pad; tok = mc - img * p.seq_pad; }
-        uint4 table[2] = {};
-        if constexpr (EPI == EPI_QKV_ROPE) {
-#pragma unroll
-            for (int q = 0; q < 2; ++q) table[q] = *(const uint4*)(p.rope + (size_t)mc * 256 + (nt0 & 255) + 16 * q + 8 * h);
-        }
-        if constexpr (EPI == EPI_VIT_QKV_ROPE) {
-#pragma unroll
-            for (int q = 0; q < 2; ++q) table[q] = *(const uint4*)(p.rope + (size_t)min(tok, p.seq - 1) * 64 + (nt0 & 63) + 16 * q + 8 * h);
-        }
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             bf16x4 pk[2];
             uint4 cs4 = {};
-            if constexpr (EPI != EPI_VIS_QKV) cs4 = swap_halves(uint2{table[q].x, table[q].y}, uint2{table[q].z, table[q].w});       // this lane's halves of the two groups
+            if constexpr (EPI != EPI_VIS_QKV) cs4 = swap_halves(uint2{tab.v[q].x, tab.v[q].y}, uint2{tab.v[q].z, tab.v[q].w});       // this lane's halves of the two groups
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
-                const int g = 2 * q + k, n0 = nt0 + 8 * g + 4 * h;
+                const int g = 2 * q + k;
                 f32x4 v = {acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
                 if constexpr (EPI == EPI_VIS_QKV) {
-                    const bf16x4 b = load4(p.bias + n0);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] += bf2f(b[e]);
+                    v += bias.v[g];
                 } else {
                     // rounded to bf16 before the rotation, as the reference's QKV buffers are (pi0_infer.py:793; dm0_infer.py:589-598)
-                    if constexpr (EPI == EPI_VIT_QKV_ROPE) v += *(const f32x4*)(p.bias_f32 + n0);
+                    if constexpr (EPI == EPI_VIT_QKV_ROPE) v += AHEAD ? bias.v[g] : *(const f32x4*)(p.bias_f32 + nt0 + 8 * g + 4 * h);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[e] = round_bf16(v[e]);
                     const uint2 raw = k ? uint2{cs4.z, cs4.w} : uint2{cs4.x, cs4.y};
@@ -112,6 +140,34 @@ RTVLA_DEVICE void scatter_tile(const GemmP& p, const f32x16& acc, int mt0, int n
     }
 }
 
+// The first cnt of a wave's row tiles, from row mt0 on, and its NT column tiles.  One column tile (four waves a CU): four row tiles ahead.  Two column tiles are
+// those of the eight-wave kernel, whose other wave on the SIMD covers the loads of a tile (8 160 x 1 024 x 3 072: 63.5 us, 65.0 with all ahead, 64.4 with a
+// tile's).
+template <int EPI, bool V, int MT, int NT>
+RTVLA_DEVICE void scatter_tiles(const GemmP& p, const f32x16 (&acc)[MT][NT], int cnt, int mt0, const int (&tile_of)[NT], int lane) {
+    if constexpr (NT > 1) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            if (i >= cnt || mt0 + 32 * i >= p.M) continue;
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                if (tile_of[j] * 32 < p.N16 * 16)
+                    scatter_tile<EPI, V, false>(p, acc[i][j], scatter_bias<EPI, V>(p, tile_of[j] * 32, lane), scatter_table<EPI, V>(p, mt0 + 32 * i, tile_of[j] * 32, lane),
+                                                mt0 + 32 * i, tile_of[j] * 32, lane);
+        }
+    } else {
+        static_assert(MT <= 4, "the tables of a wave's rows are in registers at once");
+        if (tile_of[0] * 32 >= p.N16 * 16) return;
+        const ScatterBias bias = scatter_bias<EPI, V>(p, tile_of[0] * 32, lane);
+        ScatterTable tab[MT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) tab[i] = scatter_table<EPI, V>(p, min(mt0 + 32 * i, (p.M - 1) & ~31), tile_of[0] * 32, lane);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            if (i < cnt && mt0 + 32 * i < p.M) scatter_tile<EPI, V, true>(p, acc[i][0], bias, tab[i], mt0 + 32 * i, tile_of[0] * 32, lane);
+    }
+}
+
 // DM0's prefix (dm0_infer.py:853-878; EPI_GQA_QKV): the MT x 1 tiles of a wave whose workgroup's four waves hold the 128 columns of one head.  The product of the raw stream is
 // rounded to bf16 and takes its row's RMS factor; queries and keys are then normalised over their head's features and rotated (interleaved pairs).  As a
 // launch of its own behind the GEMM this read the products back and stored 2 and 4 bytes at a time, 8.3 us at 607 rows, 3.8 at 206; a forward
@@ -123,6 +179,13 @@ RTVLA_DEVICE void scatter_head(const GemmP& p, f32x16 (&acc)[MT][1], float* lds,
     if constexpr (V) {
         const int c = nt0 - 3072 + r;
         bf16_t* const base = p.vt + (size_t)(c >> 7) * p.vt_bstride;
+        f32x4 f[MT][4];
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) f[i][g][e] = p.rowscale[min(m0 + 32 * i + 8 * g + 4 * h + e, p.M - 1)];
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
             const int mt0 = m0 + 32 * i;                   // rows mt0 + 8 g + 4 h + e
@@ -132,7 +195,7 @@ RTVLA_DEVICE void scatter_head(const GemmP& p, f32x16 (&acc)[MT][1], float* lds,
             for (int g = 0; g < 4; ++g) {
                 f32x4 v;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = round_bf16(acc[i][0][4 * g + e]) * p.rowscale[min(mt0 + 8 * g + 4 * h + e, p.M - 1)];
+                for (int e = 0; e < 4; ++e) v[e] = round_bf16(acc[i][0][4 * g + e]) * f[i][g][e];
                 pk[g] = pack4(v);
             }
             if (mt0 + 32 <= p.M) {
@@ -151,33 +214,41 @@ RTVLA_DEVICE void scatter_head(const GemmP& p, f32x16 (&acc)[MT][1], float* lds,
         }
     } else {
         const int head = nt0 >> 7, d0 = nt0 & 127;         // 16 query heads, 8 of keys
+        float f[MT];
+        uint4 table[MT][2];
+        bf16x4 nw[4];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) f[i] = p.rowscale[min(m0 + 32 * i + r, p.M - 1)];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) nw[g] = load4((head < 16 ? p.qnorm : p.knorm) + d0 + 8 * g + 4 * h);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) table[i][q] = *(const uint4*)(p.rope + (size_t)min(m0 + 32 * i + r, p.M - 1) * 128 + d0 + 16 * q + 8 * h);
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-            const float f = p.rowscale[min(m0 + 32 * i + r, p.M - 1)];
             float ss = 0.f;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) { const float v = round_bf16(acc[i][0][e]) * f; acc[i][0][e] = v; ss += v * v; }
+            for (int e = 0; e < 16; ++e) { const float v = round_bf16(acc[i][0][e]) * f[i]; acc[i][0][e] = v; ss += v * v; }
             ss = halves_sum(ss);
             if (h == 0) lds[wn * (MT * 32) + 32 * i + r] = ss;
         }
         __syncthreads();
-        const bf16_t* const nw = (head < 16 ? p.qnorm : p.knorm) + d0;
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-            const int m = m0 + 32 * i + r, mc = min(m, p.M - 1);
+            const int m = m0 + 32 * i + r;
             float ss = 0.f;
 #pragma unroll
             for (int k = 0; k < 4; ++k) ss += lds[k * (MT * 32) + 32 * i + r];
             const float inv = rsqrtf(ss * (1.0f / 128.0f) + 1e-6f);
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
-                const uint4 table = *(const uint4*)(p.rope + (size_t)mc * 128 + d0 + 16 * q + 8 * h);
-                const uint4 cs4 = swap_halves(uint2{table.x, table.y}, uint2{table.z, table.w});
+                const uint4 cs4 = swap_halves(uint2{table[i][q].x, table[i][q].y}, uint2{table[i][q].z, table[i][q].w});
                 bf16x4 pk[2];
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
                     const int g = 2 * q + k;
-                    const bf16x4 w = load4(nw + 8 * g + 4 * h);
+                    const bf16x4 w = nw[g];
                     f32x4 v;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[e] = acc[i][0][4 * g + e] * inv * bf2f(w[e]);
