@@ -10,7 +10,8 @@
 // graph.  This file is compiled with floating-point contraction off: a fused
 // multiply-add would round the weights differently from the C code being matched.
 #include "../../include/rtvla.h"
-#include "common.h"
+#include "kernels.h"
+#include <atomic>
 #include <math.h>
 
 namespace {
@@ -360,6 +361,7 @@ int frame_plan(int height, int width, FrameP* p) {
     return RTVLA_OK;
 }
 
+constexpr size_t STAGED_LDS = 76 * 1024;     // two workgroups to a CU
 template <int FMT, int TH>
 void launch_resize(FrameP p, hipStream_t s) {
     const double sy = (double)p.h / p.rh;
@@ -369,7 +371,11 @@ void launch_resize(FrameP p, hipStream_t s) {
     p.pitch = ((int)((TW - 1) * ((double)p.w / p.rw)) + p.taps_x + 2 + 3) / 4 * 4 + 4;
     const size_t staged = smem + (size_t)p.max_rows * p.pitch * 4;
     if constexpr (FMT == FRAME_F32_HWC || FMT == FRAME_F32_CHW)
-        if (p.taps_x > 4 && staged <= 76 * 1024) { hipLaunchKernelGGL((resize_staged_kernel<FMT, TH>), dim3(224 / TW, 224 / TH), dim3(NT), staged, s, p); return; }
+        if (p.taps_x > 4 && staged <= STAGED_LDS) {
+            auto kern = resize_staged_kernel<FMT, TH>;
+            static std::atomic<uint64_t> done{0};
+            if (ensure_dynamic_lds((const void*)kern, STAGED_LDS, done) == 0) { hipLaunchKernelGGL(kern, dim3(224 / TW, 224 / TH), dim3(NT), staged, s, p); return; }
+        }
     hipLaunchKernelGGL((resize_kernel<FMT, TH>), dim3(224 / TW, 224 / TH), dim3(NT), smem, s, p);
 }
 template <int FMT>
