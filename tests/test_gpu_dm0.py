@@ -1,6 +1,8 @@
 """GPU parity of the DM0 path (through the C ABI) against the CPU oracle (oracle/dm0.py, pinned in
 tests/test_oracle_dm0.py).  Same tolerances as the Pi0 / Pi05 tests: action MAE <= 1e-2, layer-local relative L2 <= 2e-2
 with every layer fed the oracle's input, free-running drift bounded by 1.5 x the oracle's own bf16-vs-fp32 drift."""
+import functools
+
 import pytest
 import torch
 
@@ -206,20 +208,27 @@ def test_vit_attention_from_the_operands_of_its_layer(first, last):
     assert worst <= 1e-2, worst
 
 
-# The prefix QKV GEMM normalises and rotates its heads itself: prompts that end inside, at and one past a 32-row tile, a row tile of the workgroup and a key
-# tile; heads and rows of different sizes, which their norms have to undo; the cache behind the prompt stays as it is.
-@pytest.mark.parametrize("images,lang", [(1, 7), (1, 23), (1, 24), (1, 88), (2, 100), (3, 100), (3, 300)])
-def test_prefix_heads_are_normalised_by_their_gemm(images, lang):
-    from _engine import untile_ft, untile_vt
-    import rtvla_capi as capi
+@functools.lru_cache(maxsize=None)
+def one_layer_policy(images, lang):
+    """(policy, checkpoint) of one ViT and one prefix layer, heads of different sizes and norm weights around 1"""
     from dm0_infer import DM0Inference
-    from oracle import dm0 as o, ops
     ck = syn.dm0_checkpoint(33, "cuda:0", 1, 1, vocab=64)
     g = torch.Generator(device="cuda:0").manual_seed(6)
     ck["llm_attn_qkv_w"] *= torch.linspace(0.2, 5.0, 32, device="cuda:0").to(torch.bfloat16).repeat_interleave(128)
     for n in ("llm_q_norm_w", "llm_k_norm_w"):
         ck[n].copy_(1 + 0.2 * torch.randn(ck[n].shape, device="cuda:0", generator=g))
-    m = DM0Inference(ck, num_images=images, max_lang_len=lang)
+    return DM0Inference(ck, num_images=images, max_lang_len=lang), ck
+
+
+# The prefix QKV GEMM normalises and rotates its heads itself: prompts that end inside, at and one past a 32-row tile, a row tile of the workgroup and a key
+# tile; heads and rows of different sizes, which their norms have to undo; the cache behind the prompt stays as it is.
+@pytest.mark.parametrize("images,lang", [(1, 7), (1, 23), (1, 24), (1, 88), (2, 100), (3, 100), (4, 300)])
+def test_prefix_heads_are_normalised_by_their_gemm(images, lang):
+    from _engine import untile_ft, untile_vt
+    import rtvla_capi as capi
+    from oracle import dm0 as o, ops
+    m, ck = one_layer_policy(images, lang)
+    g = torch.Generator(device="cuda:0").manual_seed(6)
     B, P = m.buffers, m.prefix_len
     x = torch.randn(P, 2048, device="cuda:0", generator=g) * torch.logspace(-1, 1, P, device="cuda:0")[:, None]
     B["prefix_x"].copy_(x)
@@ -245,12 +254,10 @@ def test_prefix_heads_are_normalised_by_their_gemm(images, lang):
 
 
 # Convolutions and projector split K and sum partials, 4 096 columns wide in two blocks; against fp32 from the operands they left in memory
-@pytest.mark.parametrize("images", [1, 2, 3, 4])
-def test_convolutions_sum_their_splits(images):
+@pytest.mark.parametrize("images,lang", [(1, 7), (2, 100), (3, 100), (4, 300)])
+def test_convolutions_sum_their_splits(images, lang):
     import rtvla_capi as capi
-    from dm0_infer import DM0Inference
-    ck = syn.dm0_checkpoint(35, "cuda:0", 1, 1, vocab=64)
-    m = DM0Inference(ck, num_images=images, max_lang_len=3)
+    m, ck = one_layer_policy(images, lang)
     B, T = m.buffers, images * 169
     x = torch.randn(B["vision_x_2d"].shape, device="cuda:0", generator=torch.Generator(device="cuda:0").manual_seed(7))
     B["vision_x_2d"].copy_(x)
