@@ -36,7 +36,7 @@ PROFILE_TAGS = {"headline": "pi0_3view_p20_c50"}      # workloads that have coun
 
 
 # what each counter summary was recorded of: the files that hold its kernels (csrc/)
-GEGLU_SOURCES = ("gemm.hip", "common.h", "kernels.h")
+GEGLU_SOURCES = ("gemm.hip", "gemm_scatter.h", "common.h", "kernels.h")
 FLOW_SOURCES = ("flow.hip", "common.h", "kernels.h")
 
 

@@ -189,6 +189,7 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
         }
     }
     // the bias of this wave's columns, asked for as one: a load per group of four columns is a branch and a trip to the cache for each
+    // (768 x 1 152 x 4 304 with GELU, in a trace: 17.4 -> 15.9 us)
     constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU || EPI == EPI_PATCH || EPI == EPI_RESIDUAL;
     f32x4 bias[BIAS ? HALF : 1][4];
     if constexpr (BIAS) {

@@ -150,7 +150,8 @@ RTVLA_DEVICE void gemm8_block(const GemmP& p, unsigned char* smem_raw, int m0, i
         for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    // the bias of this wave's columns, asked for ahead of the loop (bf16: in the lower half of the registers until the loop has ended)
+    // the bias of this wave's columns, asked for ahead of the loop (bf16: in the lower half of the registers until the loop has ended).
+    // Per group of four columns in the epilogue: 8 160 x 1 024 x 4 096 with GELU 76.3 us in a trace, this 73.5
     constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU || EPI == EPI_PATCH || EPI == EPI_RESIDUAL;
     f32x4 bias[BIAS ? HALF : 1][4];
     if constexpr (BIAS) {

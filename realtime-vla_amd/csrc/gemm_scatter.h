@@ -17,7 +17,7 @@ RTVLA_DEVICE uint4 swap_halves(uint2 x0, uint2 x1) {
 }
 
 // What a tile needs besides its accumulators.  Asked for ahead where scatter_tiles says so: behind the stores of the tile before, which the compiler may not
-// move loads across, each is a trip to the cache of its own.  us: SigLIP 768 rows x 3 456 13.9 -> 12.9, Gemma 788 x 2 560 22.2 -> 21.6, DM0's prefix 607 x 4 096
+// move loads across, each is a trip to the cache of its own.  us in a trace: SigLIP 768 rows x 3 456 13.9 -> 12.9, Gemma 788 x 2 560 22.2 -> 21.6, DM0's prefix 607 x 4 096
 // 22.0 -> 21.0.
 struct ScatterBias { f32x4 v[4]; float b; };               // Q, K: columns nt0 + 8 g + 4 h + e; V: column nt0 + r
 struct ScatterTable { uint4 v[2]; };
