@@ -274,6 +274,7 @@ int rtvla_reduce_norm(const float* partials, int nsplit, int M, int N, const voi
  *     RTVLA_ATTN_GQA128_PREFIX (128, 2)  DM0 prefix, causal                  RTVLA_ATTN_GQA128_SUFFIX (128, 2)  DM0 action expert
  *     RTVLA_ATTN_VIT64         (64, 1)   DM0 ViT (keys == tokens)            RTVLA_ATTN_SIGLIP        (72, 1)   SigLIP: tokens == keys == 256 x
  *                                                                                                                 views, kv_heads == 16, every view apart
+ *     RTVLA_ATTN_VIT64_EXP2    (64, 1)   the DM0 ViT as its forward runs it: the queries carry their scale times log2(e), the logits are exponents of 2
  * Mask (the reference's predicate, pi0_infer.py:1089-1096, pi05_infer.py:294-299): key j is visible to query token t iff
  *     j < prefix_alloc ? j < valid_len : (t >= state_tokens || j == prefix_alloc)
  * and, for the causal kind, j <= t.  valid_len is read from device memory (`valid_len_dev`, int32) or is prefix_alloc when
@@ -281,10 +282,10 @@ int rtvla_reduce_norm(const float* partials, int nsplit, int M, int N, const voi
  * combine fp32 partials in a second launch, as in the forward.  `workspace`: rtvla_attention_workspace_bytes, 256-byte
  * aligned (operands re-laid out in the kernels' fragment order, partial records).  RTVLA_ERR_LIMIT for shapes outside a
  * kind's range (suffix kinds: at most 128 tokens; the vision kinds take no mask; the SigLIP kernel has scale = 72^-1/2 built in
- * and refuses another). */
+ * and RTVLA_ATTN_VIT64_EXP2 scale = ln 2, and refuse another). */
 enum rtvla_attention_kind {
     RTVLA_ATTN_GEMMA_PREFIX = 0, RTVLA_ATTN_GEMMA_SUFFIX = 1, RTVLA_ATTN_GQA128_PREFIX = 2, RTVLA_ATTN_GQA128_SUFFIX = 3,
-    RTVLA_ATTN_VIT64 = 4, RTVLA_ATTN_SIGLIP = 5
+    RTVLA_ATTN_VIT64 = 4, RTVLA_ATTN_SIGLIP = 5, RTVLA_ATTN_VIT64_EXP2 = 6
 };
 size_t rtvla_attention_workspace_bytes(int kind, int tokens, int keys, int kv_heads);
 int rtvla_attention(int kind, const void* q, const void* k, const void* v, void* out, int tokens, int keys, int kv_heads,

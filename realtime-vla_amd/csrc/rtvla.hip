@@ -1741,7 +1741,7 @@ int plan_attention(int kind, int tokens, int keys, int kv_heads, AttnPlan* out) 
     switch (kind) {
         case RTVLA_ATTN_GEMMA_PREFIX: case RTVLA_ATTN_GEMMA_SUFFIX: p.hd = p.hd_pad = p.vd_pad = 256; p.group = 8; if (kv_heads != 1) return RTVLA_ERR_LIMIT; break;
         case RTVLA_ATTN_GQA128_PREFIX: case RTVLA_ATTN_GQA128_SUFFIX: p.hd = p.hd_pad = p.vd_pad = 128; p.group = 2; break;
-        case RTVLA_ATTN_VIT64: p.hd = p.hd_pad = p.vd_pad = 64; p.group = 1; if (keys != tokens) return RTVLA_ERR_LIMIT; break;
+        case RTVLA_ATTN_VIT64: case RTVLA_ATTN_VIT64_EXP2: p.hd = p.hd_pad = p.vd_pad = 64; p.group = 1; if (keys != tokens) return RTVLA_ERR_LIMIT; break;
         case RTVLA_ATTN_SIGLIP:
             p.hd = 72; p.hd_pad = 96; p.vd_pad = 80; p.group = 1;
             if (kv_heads != 16 || keys != tokens || tokens % 256 || tokens > 4 * 256) return RTVLA_ERR_LIMIT;
@@ -1780,8 +1780,9 @@ int rtvla_attention(int kind, const void* q, const void* k, const void* v, void*
     if (workspace_bytes < pl.total) return RTVLA_ERR_SIZE;
     if (prefix_alloc < 0 || prefix_alloc > keys || state_tokens < 0 || state_tokens > tokens) return RTVLA_ERR_ARG;
     const bool masked = prefix_alloc < keys || valid_len_dev || state_tokens;
-    if (masked && (kind == RTVLA_ATTN_VIT64 || kind == RTVLA_ATTN_SIGLIP)) return RTVLA_ERR_LIMIT;      // the vision kernels take no masks
+    if (masked && (kind == RTVLA_ATTN_VIT64 || kind == RTVLA_ATTN_VIT64_EXP2 || kind == RTVLA_ATTN_SIGLIP)) return RTVLA_ERR_LIMIT;      // the vision kernels take no masks
     if (kind == RTVLA_ATTN_SIGLIP && fabsf(scale - 0.11785113019775792f) > 1e-6f) return RTVLA_ERR_LIMIT;   // 72^-1/2 is built into that kernel
+    if (kind == RTVLA_ATTN_VIT64_EXP2 && !(fabsf(scale - 0.69314718055994531f) <= 1e-6f)) return RTVLA_ERR_LIMIT;      // exponents of 2
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
     bf16_t* qt = (bf16_t*)(ws + pl.q_off); bf16_t* kt = (bf16_t*)(ws + pl.k_off); bf16_t* vtt = (bf16_t*)(ws + pl.vt_off);
@@ -1799,14 +1800,14 @@ int rtvla_attention(int kind, const void* q, const void* k, const void* v, void*
         a.group = pl.group; a.rows = pl.group * tokens; a.keys = keys; a.scale = scale;
         a.out = (bf16_t*)out; a.ld_tok = kv_heads * pl.group * pl.hd; a.batch_inner = kv_heads; a.out_istride = (size_t)pl.group * pl.hd;
         a.prefix_alloc = prefix_alloc; a.valid_len = valid_len_dev; a.state_rows = state_tokens * pl.group;
-        a.causal = kind == RTVLA_ATTN_GQA128_PREFIX;
+        a.causal = kind == RTVLA_ATTN_GQA128_PREFIX; a.q_scaled = kind == RTVLA_ATTN_VIT64_EXP2;
         a.nsplit = pl.nsplit; a.partial = (float*)(ws + pl.part_off); a.partial_floats = pl.part_floats;
         switch (kind) {
             case RTVLA_ATTN_GEMMA_PREFIX:  rc = launch_mqa_attention(a, ATTN_PREFIX, s); break;
             case RTVLA_ATTN_GEMMA_SUFFIX:  rc = launch_mqa_attention(a, ATTN_SUFFIX, s); break;
             case RTVLA_ATTN_GQA128_PREFIX: rc = launch_mqa_attention(a, ATTN_GQA128_PREFIX, s); break;
             case RTVLA_ATTN_GQA128_SUFFIX: rc = launch_mqa_attention(a, ATTN_GQA128_SUFFIX, s); break;
-            case RTVLA_ATTN_VIT64:         rc = launch_flash_attention(a, 64, s); break;
+            case RTVLA_ATTN_VIT64: case RTVLA_ATTN_VIT64_EXP2: rc = launch_flash_attention(a, 64, s); break;
         }
     }
     if (rc) return rc == 3 ? RTVLA_ERR_LIMIT : RTVLA_ERR_DEVICE;

@@ -13,9 +13,10 @@ pytestmark = pytest.mark.gpu
 _P = ctypes.c_void_p
 KINDS = {  # kind: (head_dim, group)
     capi.ATTN_GEMMA_PREFIX: (256, 8), capi.ATTN_GEMMA_SUFFIX: (256, 8), capi.ATTN_GQA128_PREFIX: (128, 2), capi.ATTN_GQA128_SUFFIX: (128, 2),
-    capi.ATTN_VIT64: (64, 1), capi.ATTN_SIGLIP: (72, 1)}
+    capi.ATTN_VIT64: (64, 1), capi.ATTN_SIGLIP: (72, 1), capi.ATTN_VIT64_EXP2: (64, 1)}
 REL_TOL = 1e-2      # relative L2 of the bf16 output against the fp32 result (probabilities and outputs are rounded to bf16 once each)
 ABS_TOL = 3e-2      # largest element error, outputs are O(1)
+LN2 = 0.6931471805599453
 
 
 def reference(kind, q, k, v, scale, prefix_alloc, valid_len, state_tokens):
@@ -44,8 +45,10 @@ def run(kind, tokens, keys, kv_heads, prefix_alloc=None, valid_len=None, state_t
     if ramp:            # logits that climb with the key index: the running maximum grows all the way through the key loop
         q = q.float(); q[..., 0] += 4.0; q = q.bfloat16()
         k = k.float(); k[..., 0] += ramp * torch.arange(keys, device="cuda:0")[:, None] / keys; k = k.bfloat16()
-    out = torch.full_like(q, 9.0)
     scale = D ** -0.5
+    if kind == capi.ATTN_VIT64_EXP2:
+        q, scale = (q.float() * (scale / LN2)).bfloat16(), LN2
+    out = torch.full_like(q, 9.0)
     prefix_alloc = keys if prefix_alloc is None else prefix_alloc
     vl = None if valid_len is None else torch.tensor([valid_len], dtype=torch.int32, device="cuda:0")
     need = lib.rtvla_attention_workspace_bytes(kind, tokens, keys, kv_heads)
@@ -161,6 +164,25 @@ def test_vit_flash_attention_with_a_maximum_that_keeps_growing(tokens):
     """The ViT kernel rescales its accumulator only when a row maximum grew by 2^8 and moves the probabilities of the block in
     flight to the new scale: logits that climb by ~90 bits over the keys take that path about a dozen times per row."""
     run(capi.ATTN_VIT64, tokens, tokens, 3, seed=tokens + 1, ramp=128.0)
+
+
+@pytest.mark.parametrize("tokens,heads,ramp,sharp", [(1, 16, 0.0, 1.0), (31, 8, 0.0, 1.0), (32, 1, 0.0, 1.0), (33, 8, 0.0, 1.0), (63, 3, 0.0, 1.0), (64, 8, 0.0, 1.0),
+                                                     (65, 3, 0.0, 1.0), (96, 2, 0.0, 1.0), (128, 4, 0.0, 1.0), (129, 16, 0.0, 1.0), (192, 3, 0.0, 1.0), (200, 2, 0.0, 1.0),
+                                                     (257, 5, 0.0, 1.0), (2705, 16, 0.0, 1.0), (96, 3, 128.0, 1.0), (700, 3, 128.0, 1.0), (2705, 3, 128.0, 1.0),
+                                                     (700, 3, -128.0, 1.0), (500, 4, 0.0, 6.0)])
+def test_vit_flash_attention_as_the_forward_runs_it(tokens, heads, ramp, sharp):
+    """Queries that carry their scale, S^T started from minus the running maximum: the edges of the instance without, a sequence that ends in its first
+    block, maxima that keep growing, that lie in the first block, and sharp rows."""
+    run(capi.ATTN_VIT64_EXP2, tokens, tokens, heads, seed=tokens + 2, ramp=ramp, sharp=sharp)
+
+
+def test_exponents_of_two_have_their_scale_built_in():
+    lib, p = capi.load(), _P(4096)
+    need = lib.rtvla_attention_workspace_bytes(capi.ATTN_VIT64_EXP2, 64, 64, 1)
+    assert need > 0 and lib.rtvla_attention_workspace_bytes(capi.ATTN_VIT64_EXP2, 64, 65, 1) == 0
+    for scale in (0.125, float("nan")):
+        assert lib.rtvla_attention(capi.ATTN_VIT64_EXP2, p, p, p, p, 64, 64, 1, ctypes.c_float(scale), 64, None, 0, p, need, None) == capi.ERR_LIMIT
+    assert lib.rtvla_attention(capi.ATTN_VIT64_EXP2, p, p, p, p, 64, 64, 1, ctypes.c_float(LN2), 63, None, 0, p, need, None) == capi.ERR_LIMIT
 
 
 @pytest.mark.parametrize("views", [1, 3])
