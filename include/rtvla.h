@@ -285,7 +285,7 @@ int rtvla_reduce_norm(const float* partials, int nsplit, int M, int N, const voi
  * and RTVLA_ATTN_VIT64_EXP2 scale = ln 2, and refuse another). */
 enum rtvla_attention_kind {
     RTVLA_ATTN_GEMMA_PREFIX = 0, RTVLA_ATTN_GEMMA_SUFFIX = 1, RTVLA_ATTN_GQA128_PREFIX = 2, RTVLA_ATTN_GQA128_SUFFIX = 3,
-    RTVLA_ATTN_VIT64 = 4, RTVLA_ATTN_SIGLIP = 5, RTVLA_ATTN_VIT64_EXP2 = 6
+    RTVLA_ATTN_VIT64 = 4, RTVLA_ATTN_SIGLIP = 5, RTVLA_ATTN_VIT64_EXP2 = 8
 };
 size_t rtvla_attention_workspace_bytes(int kind, int tokens, int keys, int kv_heads);
 int rtvla_attention(int kind, const void* q, const void* k, const void* v, void* out, int tokens, int keys, int kv_heads,

@@ -24,7 +24,8 @@ ERR_NAME, ERR_SIZE, ERR_STATE, ERR_LIMIT = 2, 3, 4, 7
 TILE_AUTO, TILE_SKINNY = -1, -2
 ACT_BIAS_GELU, ACT_GEGLU, ACT_SWIGLU, ACT_RESIDUAL = 1, 2, 3, 8
 NORM_NONE, NORM_RMS, NORM_LAYER = 0, 1, 2
-ATTN_GEMMA_PREFIX, ATTN_GEMMA_SUFFIX, ATTN_GQA128_PREFIX, ATTN_GQA128_SUFFIX, ATTN_VIT64, ATTN_SIGLIP, ATTN_VIT64_EXP2 = range(7)
+ATTN_GEMMA_PREFIX, ATTN_GEMMA_SUFFIX, ATTN_GQA128_PREFIX, ATTN_GQA128_SUFFIX, ATTN_VIT64, ATTN_SIGLIP = range(6)
+ATTN_VIT64_EXP2 = 8
 FLOW_AUTO, FLOW_RESIDENT, FLOW_LAUNCHES = range(3)
 FRAME_U8_HWC, FRAME_F32_HWC, FRAME_F32_CHW, FRAME_U8_CHW = range(4)
 STATIC_SCRATCH_BYTES = 2160 * 224 * 3          # RTVLA_STATIC_SCRATCH_BYTES
