@@ -152,7 +152,7 @@ RTVLA_DEVICE void gemm8_block(const GemmP& p, unsigned char* smem_raw, int m0, i
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
     // the bias of this wave's columns, asked for ahead of the loop (bf16: in the lower half of the registers until the loop has ended).
     // Per group of four columns in the epilogue: 8 160 x 1 024 x 4 096 with GELU 76.3 us in a trace, this 73.5
-    constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU || EPI == EPI_PATCH || EPI == EPI_RESIDUAL;
+    constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU || EPI == EPI_RESIDUAL;
     f32x4 bias[BIAS ? HALF : 1][4];
     if constexpr (BIAS) {
 #pragma unroll
@@ -213,14 +213,12 @@ RTVLA_DEVICE void gemm8_block(const GemmP& p, unsigned char* smem_raw, int m0, i
             }
         }
         if (k < mtw && m0 + i * 32 < p.M) {
-            const int m = m0 + i * 32 + r;
             unsigned char* const tbuf = obuf + wm * TILE_B;
 #pragma unroll
             for (int j = 0; j < HALF; ++j) {
 #pragma unroll
                 for (int grp = 0; grp < 4; ++grp) {
                     const int cl = (wn * HALF + j) * 32 + 8 * grp + 4 * h;
-                    const int n0 = min(nbase + cl, ncols - 4);
                     f32x4 v = {acc[k][j][4 * grp], acc[k][j][4 * grp + 1], acc[k][j][4 * grp + 2], acc[k][j][4 * grp + 3]};
                     unsigned char* dst = tbuf + r * ROWB + cl * ESZ;
                     if constexpr (EPI == EPI_PARTIAL) {
@@ -235,11 +233,6 @@ RTVLA_DEVICE void gemm8_block(const GemmP& p, unsigned char* smem_raw, int m0, i
                         *(bf16x4*)dst = pack4(siluf(v[0]) * u[0], siluf(v[1]) * u[1], siluf(v[2]) * u[2], siluf(v[3]) * u[3]);
                     } else {
                         v += bias[j][grp];
-                        if constexpr (EPI == EPI_PATCH) {
-                            const bf16x4 rs = load4(p.res + (size_t)(min(m, p.M - 1) % p.res_mod) * p.ldr + n0);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) v[e] += bf2f(rs[e]);
-                        }
                         if constexpr (EPI == EPI_BIAS_GELU) {
 #pragma unroll
                             for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
@@ -351,7 +344,8 @@ int gemm8_row_blocks(int row_tiles, int mt, int n_blocks) {
 int launch_gemm8(const GemmP& p, int epi, int tile, hipStream_t s) {
     if (p.M <= 0 || p.N16 <= 0 || p.K32p <= 0 || (p.K32p & 1) || p.a_rows <= 0 || p.bgroup < 1) return 1;
     if (epi != EPI_PARTIAL && p.nsplit > 1) return 1;
-    // the loads' offsets have 32 bits and count from the workgroup's first row and column: the four-wave kernel takes what they cannot reach
+    // the loads' offsets have 32 bits and count from the workgroup's first row and column: the four-wave kernel takes what they cannot reach (it has no
+    // EPI_VIT_QKV_ROPE, whose rows are 1 024 wide)
     if (p.a_rows < p.M || p.lda > 1 << 21 || p.K32p > 1 << 16 || p.bgroup != (epi == EPI_GEGLU || epi == EPI_SWIGLU ? 4 : 8)) return launch_gemm(p, epi, TILE_128x256, s);
     switch (epi) {
         case EPI_BIAS:      return launch8_epi<EPI_BIAS>(p, tile, s);

@@ -156,21 +156,22 @@ constexpr int64_t ATTN_PARTIAL_FLOATS = 64 * 16 * (16 * 64 * 4 + 32);   // 64 ro
 // one, and needed a table for two shapes (SigLIP down-projection at 768 rows, output projection at 1 024) that are within 0.7 us of the best now.  Layer
 // times: SigLIP down-projection at 512 rows 64x128/6 -> 96x128/4 69.4 -> 65.8 us, at 1 024 rows 64x128/2 -> 128x128/3 93.7 -> 89.5; Gemma
 // down-projection at 868 rows 128x128/2 -> 128x256/4 247.7 -> 236.1, output projection at 649 rows 64x128/2 -> 96x128/2 205.2 -> 200.7.
-struct TileNeeds { bool eight = false, scattered = false, activation = false, head = false; };      // may take eight waves; the kind of epilogue; 128 columns
+enum EightWaves { EIGHT_NEVER, EIGHT_MAY, EIGHT_MUST };      // which kernels have the epilogue: csrc/gemm.hip, both, csrc/gemm8.hip
+struct TileNeeds { EightWaves eight = EIGHT_NEVER; bool scattered = false, activation = false, head = false; };      // the kind of epilogue; 128 columns
 TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittable, const char* what, TileNeeds need = {}) {
     static const int tiles[] = {TILE_224x256, TILE_192x256, TILE_160x256, TILE_128x256, TILE_64x256, TILE_128x128, TILE_96x128, TILE_64x128};
     static const int splits[] = {1, 2, 3, 4, 6, 8};
-    { TileChoice forced; if (tuning_forced_tile(what, splittable, &forced.tile, &forced.nsplit)) return forced; }
+    { TileChoice forced; if (tuning_forced_tile(what, splittable, &forced.tile, &forced.nsplit) && (need.eight != EIGHT_MUST || gemm_tile_eight_waves(forced.tile))) return forced; }
     // The eight-wave tiles (csrc/gemm8.hip) win where their workgroups fill the chip and the weights are read for many rows.  us, four / eight waves,
     // weights cold: 8 160 x 1 024 x 1 024 23.6 / 18.7, 2 720 x 1 024 x 3 072 35 / 21, but 2 720 x 1 024 x 1 024 (88 workgroups of 128 rows) 11.5 / 14.5 and 2 028 x 9 216 x 2 048
     // (128) 89 / 134.  The gated GEMMs are held by the clock that their MFMAs leave (GeGLU with K = 2 048, N = 16 384, by itself: 532 rows 81.4 / 83.2, 788 109 / 102;
     // a forward with 788 takes the same with both, 10 053 / 10 057 us), unless 256 rows to a workgroup save a round that 224 need (968 rows: 131 / 116, forward 11 150 / 10 954).
     // Among them the one whose rounds of 256 workgroups cost least: a K stage of 32 takes 0.36 us + 0.0155 us per row tile (8 160 x 4 096 x 1 024 against
     // K = 1 024), first loads and epilogue 1.6 us per row tile - 1.8 us, 2.4 us - 2 us with an activation.
-    if (need.eight && M >= 640) {
+    if (need.eight == EIGHT_MUST || (need.eight == EIGHT_MAY && M >= 640)) {
         const int cols = (ncols16 + (dual ? 7 : 15)) / (dual ? 8 : 16), row_tiles = (M + 31) / 32;
         auto rounds = [&](int mt) { return ((row_tiles + mt - 1) / mt * cols + 255) / 256; };
-        if (dual ? rounds(8) < rounds(7) : (row_tiles + 3) / 4 * cols >= 172) {
+        if (need.eight == EIGHT_MUST || (dual ? rounds(8) < rounds(7) : (row_tiles + 3) / 4 * cols >= 172)) {
             TileChoice c8{TILE8_256x256, 1};
             double least = 1e30;
             for (int tile : {TILE8_128x256, TILE8_160x256, TILE8_192x256, TILE8_224x256, TILE8_256x256}) {
@@ -559,7 +560,7 @@ struct Sched {
         p.A = A; p.lda = lda; p.a_rows = a_rows; p.M = M; p.B0 = B0; p.B1 = B1;
         p.N16 = n16_tiles(N); p.K32p = k32_padded(K); p.bgroup = bgroup;
         const bool dual = epi == EPI_GEGLU || epi == EPI_SWIGLU, vit_qkv = epi == EPI_VIT_QKV_ROPE, gqa_qkv = epi == EPI_GQA_QKV;
-        const TileNeeds need{dual || epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_RESIDUAL || vit_qkv,
+        const TileNeeds need{vit_qkv ? EIGHT_MUST : dual || epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_RESIDUAL ? EIGHT_MAY : EIGHT_NEVER,
                              epi == EPI_QKV_ROPE || epi == EPI_VIS_QKV || vit_qkv || gqa_qkv, dual || epi == EPI_BIAS_GELU, gqa_qkv};
         const TileChoice tc = choose_tile(M, p.N16, p.K32p / 2, dual, epi == EPI_PARTIAL, what, need);
         p.nsplit = tc.nsplit;
@@ -1655,7 +1656,7 @@ int plan_linear_act(int M, int K, int N, int act, int tile, ActPlan* out) {
     ActPlan p{};
     p.dual = act == RTVLA_ACT_GEGLU || act == RTVLA_ACT_SWIGLU;
     p.K128 = k32_padded(K) * 32;
-    p.tile = tile >= 0 ? tile : choose_tile(M, n16_tiles(N), k32_padded(K) / 2, p.dual, false, "linear act", {true, false, act != RTVLA_ACT_RESIDUAL, false}).tile;
+    p.tile = tile >= 0 ? tile : choose_tile(M, n16_tiles(N), k32_padded(K) / 2, p.dual, false, "linear act", {EIGHT_MAY, false, act != RTVLA_ACT_RESIDUAL, false}).tile;
     if (p.dual && tile >= 0 && (gemm_tile_bn(tile) != 256 || gemm_tile_eight_waves(tile))) return RTVLA_ERR_LIMIT;      // gate and up share a 256-column workgroup tile
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const int G = p.dual ? 4 : 8;
