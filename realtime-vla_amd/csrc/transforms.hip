@@ -375,6 +375,7 @@ void launch_resize(FrameP p, hipStream_t s) {
             auto kern = resize_staged_kernel<FMT, TH>;
             static std::atomic<uint64_t> done{0};
             if (ensure_dynamic_lds((const void*)kern, STAGED_LDS, done) == 0) { hipLaunchKernelGGL(kern, dim3(224 / TW, 224 / TH), dim3(NT), staged, s, p); return; }
+            (void)hipGetLastError();                                           // (the refusal is not an error of the launch below, which needs no more than the default)
         }
     hipLaunchKernelGGL((resize_kernel<FMT, TH>), dim3(224 / TW, 224 / TH), dim3(NT), smem, s, p);
 }
