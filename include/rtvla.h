@@ -84,7 +84,7 @@ enum rtvla_stage {
 
 /* Library version (no reference counterpart): raised whenever a kernel or the schedule changes, so that a
  * measurement recorded for one version is not mistaken for the current kernels. */
-#define RTVLA_VERSION 13
+#define RTVLA_VERSION 14
 int rtvla_version(void);
 
 /* Create a context for one shape set.  Replaces the tensor allocation block of
@@ -131,8 +131,8 @@ int rtvla_bind_workspace(rtvla_ctx* ctx, void* device_ptr, size_t bytes);
  * `buffers` views of the Python object: byte offset, rows, cols, leading dimension (elements),
  * element size.  Names follow the reference's buffer keys where one exists (vision_x, encoder_x,
  * encoder_K, decoder_x, ...); encoder_Vt is the transposed V cache.  After a forward decoder_x_buf (Pi0, DM0), decoder_q_buf (Pi0, Pi05),
- * decoder_attn and decoder_hidden hold those of the last layer and flow step on either route of the flow loop, and encoder_K / encoder_Vt the
- * suffix rows behind the prefix.  Working memory, with whatever the route that ran left there: attn_partial, decoder_qkv, decoder_Q, flow_* and the
+ * decoder_attn and decoder_hidden hold those of the last layer and flow step on either route of the flow loop, encoder_K / encoder_Vt the
+ * suffix rows behind the prefix, and DM0's prefix_qkv the products of the last prefix layer (of rtvla_forward_stage: of its layer).  Working memory, with whatever the route that ran left there: attn_partial, decoder_qkv, decoder_Q, flow_* and the
  * rows behind the prefix in DM0's kv_K / kv_Vt (writing them in the resident kernel took 0.5 us per layer and step). */
 int rtvla_buffer_count(const rtvla_ctx* ctx);
 int rtvla_buffer_info(const rtvla_ctx* ctx, int index, const char** name, size_t* offset,

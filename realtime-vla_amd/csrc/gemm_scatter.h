@@ -172,10 +172,28 @@ RTVLA_DEVICE void scatter_tiles(const GemmP& p, const f32x16 (&acc)[MT][NT], int
 // rounded to bf16 and takes its row's RMS factor; queries and keys are then normalised over their head's features and rotated (interleaved pairs).  As a
 // launch of its own behind the GEMM this read the products back and stored 2 and 4 bytes at a time, 8.3 us at 607 rows, 3.8 at 206; a forward
 // with 3 images and 100 tokens took 17 991 us with it and takes 17 727, with 1 and 37 12 064 and 11 922.  Only 128-column tiles qualify (choose_tile): a head's
-// sum of squares then stays in the workgroup.
+// sum of squares then stays in the workgroup.  With p.out the products themselves are left there as well, row-major (callers that look at a layer: one
+// layer of a forward).
 template <int MT, bool V>
 RTVLA_DEVICE void scatter_head(const GemmP& p, f32x16 (&acc)[MT][1], float* lds, int m0, int nt0, int wn, int lane) {
     const int h = lane >> 5, r = lane & 31;
+    if (p.out) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const bf16x4 v = pack4(acc[i][0][4 * g], acc[i][0][4 * g + 1], acc[i][0][4 * g + 2], acc[i][0][4 * g + 3]);
+                if constexpr (V) {                         // rows m0 + 32 i + 8 g + 4 h + e, column nt0 + r
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int m = m0 + 32 * i + 8 * g + 4 * h + e;
+                        if (m < p.M) p.out[(size_t)m * p.ldo + nt0 + r] = v[e];
+                    }
+                } else if (m0 + 32 * i + r < p.M) {
+                    store4(p.out + (size_t)(m0 + 32 * i + r) * p.ldo + nt0 + 8 * g + 4 * h, v);
+                }
+            }
+    }
     if constexpr (V) {
         const int c = nt0 - 3072 + r;
         bf16_t* const base = p.vt + (size_t)(c >> 7) * p.vt_bstride;

@@ -53,7 +53,7 @@ enum GemmEpilogue {
     EPI_QKV_ROPE,      // Gemma prefix: bf16 -> interleaved RoPE on Q,K -> Q / K cache / transposed V cache
     EPI_VIS_QKV,       // SigLIP: +bias, Q|K row-major, V transposed per (view, head)
     EPI_SWIGLU,        // out = silu(acc(B0) * rowscale[row]) * (acc(B1) * rowscale[row])   (DM0 prefix MLP)
-    EPI_GQA_QKV,       // DM0 prefix: bf16, times rowscale, norm over the head and interleaved RoPE on Q, K -> Q / K cache / V^T cache per K/V head
+    EPI_GQA_QKV,       // DM0 prefix: bf16 (-> out, if not null), times rowscale, norm over the head and interleaved RoPE on Q, K -> Q / K cache / V^T cache per K/V head
     EPI_VIT_QKV_ROPE,  // DM0 ViT: +bias, bf16, 2-D rotary on Q and K (16 heads x 64), Q / K / V^T per (image, head)
 };
 

@@ -506,6 +506,9 @@ int build_tables_dm0(rtvla_ctx* c) {
     c->add_buf("splitk_partial", 1, pmax, pmax, 4);
     c->add_buf("attn_partial", 1, ATTN_PARTIAL_FLOATS, ATTN_PARTIAL_FLOATS, 4);
     add_flow_buffers(c, 2, 192);
+    // bf16 products of the last prefix layer, ahead of its norm factors, for callers.  Behind everything else: between prefix_x and prefix_Q it moves the buffers
+    // that follow, and a forward with 3 images takes 17 453 us instead of 17 415 (17 417 without the buffer)
+    c->add_buf("prefix_qkv", P, 4096, 4096);
     return 0;
 }
 
@@ -552,6 +555,7 @@ struct Sched {
     const rtvla_dims& d;
     bool pi05;
     bool have_turn = false;        // the caller holds the device's FlowTurn
+    bool every_layer = false;      // a stage by itself: its layer leaves what a forward leaves of the last one
     Sched(rtvla_ctx* c_, hipStream_t s_) : c(c_), s(s_), d(c_->d), pi05(c_->d.model == RTVLA_PI05) {}
 
     void gemm(const bf16_t* A, int lda, int a_rows, int M, const bf16_t* B0, const bf16_t* B1, int K, int N, int epi, GemmP extra, const char* what) {
@@ -900,6 +904,7 @@ struct Sched {
         GemmP e{}; e.rowscale = c->B<float>("prefix_norm_factor"); e.qnorm = c->W("llm_q_norm_w", 128, i); e.knorm = c->W("llm_k_norm_w", 128, i);
         e.rope = c->W("prefix_rope_weights"); e.q = c->B("prefix_Q"); e.k = dK(i); e.vt = dVt(i); e.ldvt = kp;
         e.q_bstride = qstride; e.k_bstride = (size_t)kp * 128; e.vt_bstride = (size_t)128 * kp;
+        if (every_layer || i == d.llm_layers - 1) { e.out = c->B("prefix_qkv"); e.ldo = 4096; }
         gemm(c->B("prefix_x"), 2048, P, P, c->TW("t_llm_attn_qkv_w", i), nullptr, 2048, 4096, EPI_GQA_QKV, e, "prefix qkv");
         if (i == d.llm_layers - 1) return;           // the action expert reads only the K / V cache of the last prefix layer
         AttnP a{};
@@ -1366,7 +1371,9 @@ int rtvla_forward_stage(rtvla_ctx* c, int stage, int layer, int step, void* stre
     if (int rc = check_ready(c, true)) return rc;
     c->status = 0; c->launches = 0; c->kernels = 0;
     choose_route(c, (hipStream_t)stream, false);
-    int rc = Sched(c, (hipStream_t)stream).stage(stage, layer, step);
+    Sched sc(c, (hipStream_t)stream);
+    sc.every_layer = true;
+    int rc = sc.stage(stage, layer, step);
     if (rc) return c->fail(rc, "bad stage / layer / step");
     return c->status;
 }

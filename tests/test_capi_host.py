@@ -119,6 +119,17 @@ def test_dm0_tensor_table(lib):
     c.close()
 
 
+def test_dm0_buffers_by_name(lib):
+    c = capi.Context(capi.DM0, 2, 30, 50, 10, 2, 3)
+    P, seq = 2 * 169 + 30, 2720
+    bufs = {n: (rows, cols, ld, e) for n, _, rows, cols, ld, e in c.buffers()}
+    for name, cols in (("prefix_x", 2048), ("prefix_qkv", 4096), ("prefix_attn", 2048), ("prefix_hidden", 6144)):
+        assert bufs[name] == (P, cols, cols, 2)
+    for name in ("vision_Q", "vision_K", "vision_Vt"):
+        assert bufs[name] == (32, seq * 64, seq * 64, 2)
+    c.close()
+
+
 def test_bind_errors_are_status_codes(lib):
     c = capi.Context(capi.PI0, 1, 0, 50)
     with pytest.raises(capi.RtvlaError) as e:

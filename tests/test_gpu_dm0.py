@@ -253,6 +253,27 @@ def test_prefix_heads_are_normalised_by_their_gemm(images, lang):
         assert err.max().item() <= 2 ** -9 * 3.83, (name, err.max().item())
 
 
+@pytest.mark.parametrize("images,lang", [(1, 7), (2, 30)])
+def test_prefix_products_of_a_layer_and_of_a_forward(images, lang):
+    """buffers["prefix_qkv"]: of the layer that run_stage was given, of the last one after a forward."""
+    import rtvla_capi as capi
+    from dm0_infer import DM0Inference
+    ck = syn.dm0_checkpoint(34, "cuda:0", 1, 2, vocab=64)
+    m = DM0Inference(ck, num_images=images, max_lang_len=lang)
+    B, P = m.buffers, m.prefix_len
+    B["prefix_qkv"].fill_(7)
+    m.forward(*syn.dm0_observation(34, images, "cuda:0", max_lang_len=lang, vocab=64))
+    got, x = B["prefix_qkv"].clone(), B["prefix_x"].clone()          # (the last layer leaves the stream as it is)
+    assert got.shape == (P, 4096)
+    for layer in (0, 1):
+        B["prefix_x"].copy_(x)
+        m._engine.run_stage(capi.STAGE_PREFIX_LAYER, layer, 0)
+        want = x.float() @ ck["llm_attn_qkv_w"][layer].float()
+        # rounded once to bf16, at most 2^-9 of each element; fp32 sums of 2 048 products differ by less than a tenth of that
+        assert ((B["prefix_qkv"].float() - want).norm(dim=1) / want.norm(dim=1)).max().item() <= 2.0 ** -9 * 1.1, layer
+    assert torch.equal(B["prefix_qkv"], got)
+
+
 # Convolutions and projector split K and sum partials, 4 096 columns wide in two blocks; against fp32 from the operands they left in memory
 @pytest.mark.parametrize("images,lang", [(1, 7), (2, 100), (3, 100), (4, 300)])
 def test_convolutions_sum_their_splits(images, lang):
