@@ -207,7 +207,14 @@ def test_eight_wave_tiles_with_more_row_blocks_than_the_least(M, K, N):
 
 # what the cost model gives to the eight-wave tiles that a caller cannot name: 160 rows (85 row tiles by 12 blocks of columns), the residual epilogue
 # (171 row tiles by 4) and a gated one (32 row tiles: 256 rows save a round); one row past a tile, K past a pair of stages, columns past a block
-@pytest.mark.parametrize("M,K,N,act", [(2705, 136, 3072, 1), (2689, 72, 3056, 1), (5441, 72, 1008, 8), (5473, 264, 1024, 8), (1000, 264, 16384, 2), (993, 136, 16368, 3)])
+@pytest.mark.parametrize("M,K,N,act", [
+    (2705, 136, 3072, 1), (2689, 72, 3056, 1), (5441, 72, 1008, 8), (5473, 264, 1024, 8), (1000, 264, 16384, 2), (993, 136, 16368, 3),
+    # every tile with each kind of epilogue, in launches that mix its row blocks with those of 32 rows fewer: 128, 160, 192, 224 and 256 rows
+    (1281, 136, 4096, 1), (2689, 136, 3056, 1), (3361, 136, 3056, 1), (4033, 136, 3056, 1), (4705, 136, 3056, 1),
+    (10881, 72, 272, 8), (8193, 72, 1008, 8), (10241, 136, 1008, 8), (4033, 72, 3072, 8), (4705, 136, 3072, 8),
+    (2689, 136, 16368, 2), (2241, 136, 6144, 3), (4737, 136, 6144, 2), (3841, 136, 16368, 3), (1121, 136, 6144, 2),
+    # row blocks of one size: 160, 192, 224 and 256 rows; the output projection of four ViT images (192 and 160 rows)
+    (3329, 72, 3072, 8), (4001, 136, 3072, 8), (4673, 72, 3072, 8), (5345, 136, 3072, 8), (10880, 1024, 1024, 8)])
 def test_eight_wave_tiles_of_the_cost_model_against_fp32(M, K, N, act):
     import rtvla_capi as capi
     lib = capi.load()
