@@ -389,20 +389,25 @@ def test_policies_on_two_streams_and_threads():
 
 
 def test_only_the_flow_loops_take_turns():
-    """What comes before a loop does not wait for the loops of another stream."""
+    """What comes before a loop does not wait for the loops of another stream.  Streams share a handful of hardware queues, and what is in one queue
+    does wait: one stream of several that gets past the other's loops shows it."""
     (a, a_in), (b, b_in) = policy("pi0", 703, 1, 5, 50), policy("pi0", 704, 1, 5, 50)
     a.forward(*a_in)
     b.forward(*b_in)
     torch.cuda.synchronize()
-    first, second = torch.cuda.Stream(), torch.cuda.Stream()
-    with torch.cuda.stream(first):
-        for _ in range(200):
-            a._engine.replay()
-    with torch.cuda.stream(second):
-        b._engine.run_stage(capi.STAGE_VISION_LAYER, 0)
-    second.synchronize()
-    assert not first.query()                                                 # 200 forwards against one layer
-    first.synchronize()
+    first, passed = torch.cuda.Stream(), False
+    for second in [torch.cuda.Stream() for _ in range(8)]:
+        with torch.cuda.stream(first):
+            for _ in range(200):
+                a._engine.replay()
+        with torch.cuda.stream(second):
+            b._engine.run_stage(capi.STAGE_VISION_LAYER, 0)
+        second.synchronize()
+        passed = not first.query()                                           # 200 forwards against one layer
+        first.synchronize()
+        if passed:
+            break
+    assert passed
 
 
 WORKER = """
