@@ -132,7 +132,8 @@ int rtvla_bind_workspace(rtvla_ctx* ctx, void* device_ptr, size_t bytes);
  * element size.  Names follow the reference's buffer keys where one exists (vision_x, encoder_x,
  * encoder_K, decoder_x, ...); encoder_Vt is the transposed V cache.  After a forward decoder_x_buf (Pi0, DM0), decoder_q_buf (Pi0, Pi05),
  * decoder_attn and decoder_hidden hold those of the last layer and flow step on either route of the flow loop, encoder_K / encoder_Vt the
- * suffix rows behind the prefix, and DM0's prefix_qkv the products of the last prefix layer (of rtvla_forward_stage: of its layer).  Working memory, with whatever the route that ran left there: attn_partial, decoder_qkv, decoder_Q, flow_* and the
+ * suffix rows behind the prefix, and DM0's prefix_qkv the products of the last prefix layer (of rtvla_forward_stage: of its layer).  DM0's vision_Q
+ * holds the ViT's queries rotated and times 0.125 log2(e) (its softmax takes exponents of 2), Pi0's and Pi05's without a factor.  Working memory, with whatever the route that ran left there: attn_partial, decoder_qkv, decoder_Q, flow_* and the
  * rows behind the prefix in DM0's kv_K / kv_Vt (writing them in the resident kernel took 0.5 us per layer and step). */
 int rtvla_buffer_count(const rtvla_ctx* ctx);
 int rtvla_buffer_info(const rtvla_ctx* ctx, int index, const char** name, size_t* offset,
