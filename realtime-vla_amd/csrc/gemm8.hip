@@ -7,8 +7,9 @@
 // for the 256 x 256 tile, 48 of the 64 bytes per clock that the path gives under full MFMAs; through LDS it is 64 KB, and nothing but LDS reads and
 // MFMAs waits.  us on MI355X, weights cold, registers -> LDS: 8 160 x 1 024 x 4 096 with bias + GELU 85 -> 73, 8 160 x 1 024 x 3 072 65 -> 54,
 // 2 720 x 1 024 x 4 096 43 (four waves, 128 rows) -> 28, 8 160 x 4 096 x 1 024 66 (four waves) -> 59, 788 x 2 048 x 2 * 16 384 with GeGLU 109 (four waves) -> 102.
-// At 1.16 PFLOP/s the longest of them is where the clock that MFMAs on such values leave takes it; two rounds of a 256 x 256 tile with K = 1 024 add
-// 2 x 10 us of first loads and epilogue to that.
+// The longest of them computes at 1.16 PFLOP/s by itself.  Counters inside a layer: 65 us, the matrix pipe busy in 60 % of the cycles (K = 1 024 with GELU 55, QKV 49 %) at
+// 1.65 GHz.  A loop of nothing but MFMAs on such values reaches 1.5 - 1.8 PFLOP/s, so the clock is a part of the distance and the cycles without products the rest: two
+// rounds of a 256 x 256 tile with K = 1 024 spend 2 x 10 us on first loads and epilogue.
 //
 // LDS of a stage: the activation rows at a pitch of 64 bytes, the 16-byte chunk c (8 of K) of row r in place c ^ ((r >> 2) & 3): 16 consecutive lanes of a
 // fragment read (16 rows, one chunk) touch each of the 64 banks once.  A DMA instruction writes 16 rows in lane order, so the permutation is

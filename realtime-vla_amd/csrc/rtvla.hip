@@ -146,26 +146,30 @@ constexpr int EHID_LD = 16384 + 64;
 constexpr int64_t ATTN_PARTIAL_FLOATS = 64 * 16 * (16 * 64 * 4 + 32);   // 64 row blocks (128 suffix rows x 8 heads) x 16 key splits of the suffix attention
 
 // Pick block tile and split-K factor from a cost model fitted to measurements on MI355X: every tile and split in place of the chosen one in
-// a whole layer (114 GEMMs of a SigLIP, Gemma, DM0 ViT or DM0 prefix layer at one to four views and prompts of 0 to 200 tokens, all layers in
+// a whole layer (SigLIP, Gemma, DM0 ViT and DM0 prefix layers at one to four views and prompts of 0 to 200 tokens, all layers in
 // turn, so weights and activations are where a forward has them).  One K stage of a workgroup takes the larger of its MFMA time (32 cycles
 // per 32x32x16 MFMA at 2.05 GHz and 88 % issue efficiency) and its load time (0.143 us + 10.1 us per MB of operands pulled by the workgroup);
 // tiles of 64 rows run two workgroups per CU, which share the MFMA pipe and the CU's load path; all workgroups together cannot pull more
 // than 18.7 TB/s out of L2; every launch pays a ramp and an epilogue per 32 x 128 outputs of a workgroup, 1.3 times as long where Q, K and
-// V^T are scattered into fragment order; split-K adds the fp32 partials, written and read.  Over those layers, weighted by their number per
-// forward, the choice is 0.46 ms off the best one in sum.  It was 2.7 ms as long as two workgroups of a CU were taken to load twice as fast as
-// one, and needed a table for two shapes (SigLIP down-projection at 768 rows, output projection at 1 024) that are within 0.7 us of the best now.  Layer
-// times: SigLIP down-projection at 512 rows 64x128/6 -> 96x128/4 69.4 -> 65.8 us, at 1 024 rows 64x128/2 -> 128x128/3 93.7 -> 89.5; Gemma
-// down-projection at 868 rows 128x128/2 -> 128x256/4 247.7 -> 236.1, output projection at 649 rows 64x128/2 -> 96x128/2 205.2 -> 200.7.
+// V^T are scattered into fragment order; split-K adds the fp32 partials, written and read.
+// What it is worth, measured again with these constants and the kernels as they are: 128 such GEMMs (the convolutions and DM0's projector among them), every tile and split of a
+// GEMM in its layer, medians of five for the chosen and the fastest.  The choice is the fastest one for 95 of them, and 0.75 ms off in sum, weighted by their number per
+// forward, of 108 ms of layers.  Most of that, layer times in us: DM0 ViT QKV with four images 192 rows 450.1, 160 rows 442.6; GeGLU at 456 and 512 rows 142.3 and 154.4, with
+// eight waves 137.1 and 146.8 (see below); down-projections 153.6 for 150.0 (512 rows, 128x128/4, 128x256/8), 136.2 for 133.7 (DM0, 876 rows, 128x128/2, 128x256/4), 76.0 for 74.5 (DM0,
+// 206 rows, 64x128/4, 128x128/8).
 enum EightWaves { EIGHT_NEVER, EIGHT_MAY, EIGHT_MUST };      // which kernels have the epilogue: csrc/gemm.hip, both, csrc/gemm8.hip
 struct TileNeeds { EightWaves eight = EIGHT_NEVER; bool scattered = false, activation = false, head = false; };      // the kind of epilogue; 128 columns
 TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittable, const char* what, TileNeeds need = {}) {
     static const int tiles[] = {TILE_224x256, TILE_192x256, TILE_160x256, TILE_128x256, TILE_64x256, TILE_128x128, TILE_96x128, TILE_64x128};
     static const int splits[] = {1, 2, 3, 4, 6, 8};
     { TileChoice forced; if (tuning_forced_tile(what, splittable, &forced.tile, &forced.nsplit) && (need.eight != EIGHT_MUST || gemm_tile_eight_waves(forced.tile))) return forced; }
-    // The eight-wave tiles (csrc/gemm8.hip) win where their workgroups fill the chip and the weights are read for many rows.  us, four / eight waves,
-    // weights cold: 8 160 x 1 024 x 1 024 23.6 / 18.7, 2 720 x 1 024 x 3 072 35 / 21, but 2 720 x 1 024 x 1 024 (88 workgroups of 128 rows) 11.5 / 14.5 and 2 028 x 9 216 x 2 048
-    // (128) 89 / 134.  The gated GEMMs are held by the clock that their MFMAs leave (GeGLU with K = 2 048, N = 16 384, by itself: 532 rows 81.4 / 83.2, 788 109 / 102;
-    // a forward with 788 takes the same with both, 10 053 / 10 057 us), unless 256 rows to a workgroup save a round that 224 need (968 rows: 131 / 116, forward 11 150 / 10 954).
+    // The eight-wave tiles (csrc/gemm8.hip) win where their workgroups fill the chip and the weights are read for many rows.  us of a whole layer with four / eight waves, the best
+    // tile of each, by blocks of 128 x 256.  88: DM0 ViT, 2 720 rows, output projection 161.9 / 167.9, down 161.8 / 182.9; 136: SigLIP up, 1 024 rows 81.2 / 83.3; 172: ViT, 5 440 rows,
+    // output projection 263.7 / 264.6, down 262.4 / 264.8; 256: 8 160 rows 354.9 / 352.7 and 352.6 / 352.4; 352: 2 720 rows up 163.8 / 161.8; 688: 5 440 rows up 268.7 / 264.5; 1 024: 369.7 / 352.7.  So
+    // 172 is the lower end of where the two are within 1 %; no GEMM of the models has a number between 172 and 256.
+    // The gated GEMMs take the same with both (GeGLU, K = 2 048, N = 16 384: 712 rows 196.9 / 196.5, 788 212.6 / 211.9, 868 227.4 / 224.3, 1 224 311.7 / 309.9) or less with four (532 rows 165.0 / 168.6,
+    // 612 175.1 / 182.4, 768 202.5 / 206.6, 1 044 279.0 / 282.0), unless 256 rows to a workgroup save a round that 224 need (968 rows 251.4 / 237.4, 1 024 257.2 / 246.3).  The 640 rows bind these alone (172
+    // blocks of fewer rows are 8 704 columns), and are too high: 449 - 512 rows save a round as well, and measure 142.3 / 137.1 at 456 and 154.4 / 146.8 at 512.
     // Among them the one whose rounds of 256 workgroups cost least: a K stage of 32 takes 0.36 us + 0.0155 us per row tile (8 160 x 4 096 x 1 024 against
     // K = 1 024), first loads and epilogue 1.6 us per row tile - 1.8 us, 2.4 us - 2 us with an activation.
     if (need.eight == EIGHT_MUST || (need.eight == EIGHT_MAY && M >= 640)) {
@@ -595,7 +599,8 @@ struct Sched {
     // 1 024 columns: 172 workgroups and more).  The sum is taken in the GEMM's epilogue, so that the stream crosses memory as bf16 (read,
     // written, read, normalised copy written) instead of as an fp32 partial beside it, and in the order in which the pass that sums
     // partials takes it: the same bits.  Measured at 8 160 rows: K = 4096 64.8 us + 16.6 us for the pass -> 67.5 + 7.0 us,
-    // K = 1024 24.7 + 16.5 -> 28.4 + 6.5 us.
+    // K = 1024 24.7 + 16.5 -> 28.4 + 6.5 us, with the four-wave kernel on both sides.  (The eight-wave one that these sizes run in now: 65.5 and 21.7 in a counter run, which is slower
+    // than a forward.)
     void gemm_residual(const bf16_t* A, int lda, int M, const bf16_t* B0, int K, int N, const bf16_t* bias, bf16_t* x, bf16_t* xn,
                        const bf16_t* nw, const bf16_t* nb, float eps, const char* what, const char* what_norm) {
         GemmP e{}; e.out = x; e.ldo = N; e.bias = bias; e.res = x; e.ldr = N;
@@ -1551,7 +1556,7 @@ int plan_linear(int M, int K, int N, int tile, int nsplit, LinearPlan* pl) {
     }
     p.tile = tc.tile; p.nsplit = tc.nsplit;
     p.partial = nsplit == 0 || tc.nsplit > 1;              // the residual-GEMM route: fp32 partials + reduce
-    if (p.partial && N > 2048) return RTVLA_ERR_LIMIT;     // the reduce kernel handles rows of at most 2048 columns
+    if (p.partial && N > 2048) return RTVLA_ERR_LIMIT;     // (of this entry point: the pass that sums takes wider rows where it does not normalise)
     p.a_off = 0;
     p.w_off = up((size_t)M * p.K128 * 2);
     p.bias_off = p.w_off + up(tiled_elems_wide(K, N, 8) * 2);
