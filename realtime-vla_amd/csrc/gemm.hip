@@ -13,6 +13,7 @@
 #include "kernels.h"
 #include "gemm_scatter.h"
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -24,19 +25,40 @@ RTVLA_DEVICE f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdg
 // workgroups per CU so that one workgroup's MFMAs run under the other's memory latency.
 // One block tile of MT 32-row tiles starting at row m0: K loop and epilogue.
 // V: a tile of V columns, whose product is taken as activations x weights (gemm_scatter.h)
-template <int WN, int MT, int NT, int EPI, bool V = false>
-RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, int n_blk, int split, int stages_total, int stages_per_split) {
+// KG: groups of WN waves that share a block tile and split its K stages among them, each with stage buffers of its own.  For launches of few workgroups, where
+// the waves of a CU wait for their loads: two groups have twice as much on the way and half as many stages one after another.  us of a whole layer with one / two
+// groups, weights cold: DM0's prefix QKV, K = 2 048, 206 rows (64 x 128) 75.8 / 74.0, 398 90.9 / 89.1, 607 (96 x 128) 105.9 / 105.0, Gemma's, 968 rows 235.4 / 232.6, ViT
+// down projection, K = 4 096, 2 720 rows 161.4 / 159.2.  With two groups a tile of 64 x 64 has eight 32 x 32 products a stage for four waves, which on its own would be two waves
+// to a CU; it doubles the workgroups where 64 x 128 leaves half of the chip idle: Gemma QKV, 256 rows, 80 workgroups of 64 x 128 105.6, 160 of 64 x 64 99.9; SigLIP QKV 256 rows 53.8 /
+// 51.7.  Where the chip is full it gives nothing (SigLIP up, 768 rows, 128 x 128 69.1 / 69.1) or less (dual tiles of 64 x 256: GeGLU, 256 rows 105.6 / 117.8), and neither do three or four
+// groups.
+template <int WN, int MT, int NT, int EPI, int KG = 1>
+struct GemmLds {
+    static constexpr bool f32 = EPI == EPI_PARTIAL || EPI == EPI_RESIDUAL;
+    static constexpr int stages = 3 * MT * 32 * 128;                                   // of one group
+    static constexpr int out_tile = 32 * (WN * (EpiTraits<EPI>::dual ? NT / 2 : NT) * 32 * (f32 ? 4 : 2) + 16);
+    static constexpr int group = stages > out_tile ? stages : out_tile;                // a group's own memory
+    static constexpr int sums = (KG - 1) * MT * WN * NT * 4096;                        // the tiles the groups hand each other
+    static constexpr int bytes = KG * group > sums ? KG * group : sums;
+};
+template <int WN, int MT, int NT, int EPI, bool V = false, int KG = 1>
+RTVLA_DEVICE void gemm_block(const GemmP& pk, unsigned char* smem_all, int m0_wg, int n_blk, int split, int stages_total, int stages_per_split) {
     constexpr int NTH = WN * 64;
+    using Lds = GemmLds<WN, MT, NT, EPI, KG>;
     constexpr int BM = MT * 32;
     constexpr int A_CHUNKS = BM * 8;                       // 16-byte chunks per 64-wide K stage
     constexpr int AIT = (A_CHUNKS + NTH - 1) / NTH;
     constexpr int STAGE_ELEMS = BM * 64;
+    const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NTH) : 0;
+    unsigned char* const smem_raw = smem_all + kg * Lds::group;
     bf16_t* lds = (bf16_t*)smem_raw;
 
-    const int tid = threadIdx.x, lane = tid & 63, wn = tid >> 6;
+    const int tid = threadIdx.x - kg * NTH, lane = tid & 63, wn = tid >> 6;
     const int h = lane >> 5, r = lane & 31;
-    const int s_begin = split * stages_per_split;
-    const int s_end = min(s_begin + stages_per_split, stages_total);
+    int m0 = m0_wg;
+    std::conditional_t<KG == 1, const GemmP&, GemmP> p = pk;
+    const int s_begin = split * stages_per_split + kg * (stages_per_split / KG);
+    const int s_end = min(s_begin + stages_per_split / KG, stages_total);
 
     // 32-column tiles of this wave
     constexpr int HALF = EpiTraits<EPI>::dual ? NT / 2 : NT;
@@ -188,6 +210,54 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
             if (s < s_end) stage(b0, b1, last, breg0, areg0, areg1);
         }
     }
+    // Each group keeps MTO of the row tiles and gets the other groups' sums of them (in the order of the groups) for its own; from here on m0 and p.M are
+    // those of its rows.
+    constexpr int MTO = (MT + KG - 1) / KG;
+    f32x16 own[MTO][NT];
+    if constexpr (KG == 1) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) own[i][j] = acc[i][j];
+    } else {
+        f32x4* const sums = (f32x4*)smem_all;
+        auto at = [&](int from, int i, int j) __attribute__((always_inline)) { return sums + ((((from - (from > i / MTO)) * MT + i) * WN + wn) * NT + j) * 256 + lane; };
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            if (i / MTO != kg)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) at(kg, i, j)[e * 64] = f32x4{acc[i][j][4 * e], acc[i][j][4 * e + 1], acc[i][j][4 * e + 2], acc[i][j][4 * e + 3]};
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < KG; ++g) {
+            if (g != kg || g * MTO >= MT) continue;
+#pragma unroll
+            for (int k = 0; k < MTO; ++k) {
+                const int i = g * MTO + k;
+                if (i >= MT) continue;
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    f32x16 v = acc[i][j];
+#pragma unroll
+                    for (int from = 0; from < KG; ++from) {
+                        if (from == g) continue;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const f32x4 o = at(from, i, j)[e * 64];
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) v[4 * e + q] += o[q];
+                        }
+                    }
+                    own[k][j] = v;
+                }
+            }
+        }
+        m0 += kg * MTO * 32;
+        p.M = min(p.M, m0_wg + min((kg + 1) * MTO, MT) * 32);
+    }
     // the bias of this wave's columns, asked for as one: a load per group of four columns is a branch and a trip to the cache for each
     // (768 x 1 152 x 4 304 with GELU, in a trace: 17.4 -> 15.9 us)
     constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU || EPI == EPI_PATCH || EPI == EPI_RESIDUAL;
@@ -213,10 +283,10 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
                     for (int e = 0; e < 4; ++e) bias[j][grp][e] = bf2f(b[j][grp][e]);
         }
     }
-    float factor[EPI == EPI_SWIGLU ? MT : 1];
+    float factor[EPI == EPI_SWIGLU ? MTO : 1];
     if constexpr (EPI == EPI_SWIGLU)
 #pragma unroll
-        for (int i = 0; i < MT; ++i) factor[i] = p.rowscale[min(m0 + i * 32 + r, p.M - 1)];
+        for (int i = 0; i < MTO; ++i) factor[i] = p.rowscale[min(m0 + i * 32 + r, p.M - 1)];
     __syncthreads();                                        // the epilogue reuses the stage buffers
 
     // ---- epilogue: lane (h, r) holds rows m = m0 + 32 i + r, columns n = 32 tile + 8 grp + 4 h + e ----
@@ -239,9 +309,9 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
         // As many 32-row tiles as fit into the stage buffers are converted and staged back to back, then copied out
         // back to back: one barrier pair per group instead of one per tile, and the stores of a group stream.
         constexpr int TILE_B = 32 * ROWB;
-        constexpr int GROUP = (3 * BM * 128) / TILE_B >= MT ? MT : ((3 * BM * 128) / TILE_B < 1 ? 1 : (3 * BM * 128) / TILE_B);
+        constexpr int GROUP = Lds::group / TILE_B >= MTO ? MTO : (Lds::group / TILE_B < 1 ? 1 : Lds::group / TILE_B);
 #pragma unroll
-        for (int g0 = 0; g0 < MT; g0 += GROUP) {
+        for (int g0 = 0; g0 < MTO; g0 += GROUP) {
           bf16x8 res[RES ? GROUP * (32 / RPP) : 1];
           if constexpr (RES) {
 #pragma unroll
@@ -251,7 +321,7 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
             }
           }
 #pragma unroll
-          for (int i = g0; i < (g0 + GROUP < MT ? g0 + GROUP : MT); ++i) {
+          for (int i = g0; i < (g0 + GROUP < MTO ? g0 + GROUP : MTO); ++i) {
             if (m0 + i * 32 >= p.M) continue;                                     // a row tile past the end (uniform)
             const int m = m0 + i * 32 + r;
             unsigned char* const tbuf = obuf + (i - g0) * TILE_B;
@@ -261,16 +331,16 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
                 for (int grp = 0; grp < 4; ++grp) {
                     const int cl = (wn * HALF + j) * 32 + 8 * grp + 4 * h;        // column inside the workgroup tile
                     const int n0 = min(nbase + cl, ncols - 4);                    // clamped: out-of-range columns are never copied out
-                    f32x4 v = {acc[i][j][4 * grp], acc[i][j][4 * grp + 1], acc[i][j][4 * grp + 2], acc[i][j][4 * grp + 3]};
+                    f32x4 v = {own[i][j][4 * grp], own[i][j][4 * grp + 1], own[i][j][4 * grp + 2], own[i][j][4 * grp + 3]};
                     unsigned char* dst = tbuf + r * ROWB + cl * ESZ;
                     if constexpr (EPI == EPI_PARTIAL) {
                         *(f32x4*)dst = v;
                     } else if constexpr (EPI == EPI_GEGLU) {
-                        const f32x4 u = {acc[i][j + HALF][4 * grp], acc[i][j + HALF][4 * grp + 1], acc[i][j + HALF][4 * grp + 2], acc[i][j + HALF][4 * grp + 3]};
+                        const f32x4 u = {own[i][j + HALF][4 * grp], own[i][j + HALF][4 * grp + 1], own[i][j + HALF][4 * grp + 2], own[i][j + HALF][4 * grp + 3]};
                         *(bf16x4*)dst = pack4(gelu_tanh(v[0]) * u[0], gelu_tanh(v[1]) * u[1], gelu_tanh(v[2]) * u[2], gelu_tanh(v[3]) * u[3]);
                     } else if constexpr (EPI == EPI_SWIGLU) {
                         const float f = factor[i];
-                        f32x4 u = {acc[i][j + HALF][4 * grp], acc[i][j + HALF][4 * grp + 1], acc[i][j + HALF][4 * grp + 2], acc[i][j + HALF][4 * grp + 3]};
+                        f32x4 u = {own[i][j + HALF][4 * grp], own[i][j + HALF][4 * grp + 1], own[i][j + HALF][4 * grp + 2], own[i][j + HALF][4 * grp + 3]};
                         v *= f; u *= f;
                         *(bf16x4*)dst = pack4(siluf(v[0]) * u[0], siluf(v[1]) * u[1], siluf(v[2]) * u[2], siluf(v[3]) * u[3]);
                     } else {
@@ -292,7 +362,7 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
           }
           __syncthreads();
 #pragma unroll
-          for (int i = g0; i < (g0 + GROUP < MT ? g0 + GROUP : MT); ++i) {
+          for (int i = g0; i < (g0 + GROUP < MTO ? g0 + GROUP : MTO); ++i) {
             const unsigned char* const tbuf = obuf + (i - g0) * TILE_B;
 #pragma unroll
             for (int ps = 0; ps < 32 / RPP; ++ps) {
@@ -316,24 +386,24 @@ RTVLA_DEVICE void gemm_block(const GemmP& p, unsigned char* smem_raw, int m0, in
                 }
             }
           }
-          if (g0 + GROUP < MT) __syncthreads();
+          if (g0 + GROUP < MTO) __syncthreads();
         }
     } else {
         static_assert(epi_scatters(EPI), "every epilogue is one of the two kinds");
         if constexpr (EPI == EPI_GQA_QKV) {
             static_assert(WN == 4 && NT == 1, "a head is 128 columns");
-            scatter_head<MT, V>(p, acc, (float*)smem_raw, m0, tile_of[0] * 32, wn, lane);
+            scatter_head<MTO, V>(p, own, (float*)smem_raw, m0, tile_of[0] * 32, wn, lane);
             return;
         }
-        else scatter_tiles<EPI, V>(p, acc, MT, m0, tile_of, lane);
+        else scatter_tiles<EPI, V>(p, own, MTO, m0, tile_of, lane);
     }
 }
 
 // Workgroup -> block tile.  Row blocks come in two sizes when MIXED: the first n_big blocks have MT 32-row tiles, the
 // others MT - 1, so that M rows are covered with ceil(M / 32) tiles instead of a multiple of MT (788 rows: 7 + 6 + 6 + 6 =
 // 25 tiles where four 7-tile blocks would compute 28).
-template <int WN, int MT, int NT, int EPI, bool MIXED>
-__global__ __launch_bounds__(WN * 64, (MT <= 2 && WN == 4 ? 2 : 1))
+template <int WN, int MT, int NT, int EPI, bool MIXED, int KG = 1>
+__global__ __launch_bounds__(WN * 64 * KG, (MT <= 2 && WN == 4 && KG == 1 ? 2 : 1))
 void gemm_mfma_kernel(GemmP p, int m_blocks, int n_blocks, int stages_total, int stages_per_split, int n_big) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int total = m_blocks * n_blocks * p.nsplit;
@@ -347,7 +417,7 @@ void gemm_mfma_kernel(GemmP p, int m_blocks, int n_blocks, int stages_total, int
             if (m_blk < n_big) gemm_block<WN, MT, NT, EPI, v.value>(p, smem_raw, m_blk * (MT * 32), n_blk, split, stages_total, stages_per_split);
             else gemm_block<WN, MT - 1, NT, EPI, v.value>(p, smem_raw, n_big * (MT * 32) + (m_blk - n_big) * ((MT - 1) * 32), n_blk, split, stages_total, stages_per_split);
         } else {
-            gemm_block<WN, MT, NT, EPI, v.value>(p, smem_raw, m_blk * (MT * 32), n_blk, split, stages_total, stages_per_split);
+            gemm_block<WN, MT, NT, EPI, v.value, KG>(p, smem_raw, m_blk * (MT * 32), n_blk, split, stages_total, stages_per_split);
         }
     };
     if constexpr (epi_scatters(EPI)) {
@@ -356,9 +426,8 @@ void gemm_mfma_kernel(GemmP p, int m_blocks, int n_blocks, int stages_total, int
     block(std::false_type{});
 }
 
-template <int WN, int MT, int NT, int EPI, bool MIXED>
+template <int WN, int MT, int NT, int EPI, bool MIXED, int KG = 1>
 int launch_cfg(const GemmP& p, hipStream_t s) {
-    constexpr int BM = MT * 32;
     constexpr int HALF = EpiTraits<EPI>::dual ? NT / 2 : NT;
     const int tiles = (p.M + 31) / 32;
     int m_blocks = (tiles + MT - 1) / MT, n_big = m_blocks;
@@ -372,16 +441,18 @@ int launch_cfg(const GemmP& p, hipStream_t s) {
     const int sps = (stages_total + nsplit - 1) / nsplit;
     if ((nsplit - 1) * sps >= stages_total) return 3;      // an empty split would leave its partial unwritten
     if (MT > 4 && ((sps & 1) || (stages_total & 1))) return 3;              // the large tiles consume K stages in pairs
+    if constexpr (KG > 1)                                  // the groups meet at every barrier, so they have as many stages each
+        if (sps % KG || stages_total % sps) return launch_cfg<4, MT, NT, EPI, MIXED>(p, s);
     GemmP q = p; q.nsplit = nsplit;
     // three K-stage buffers; the row-major epilogues stage 32-row output tiles in the same memory
-    const size_t epi_bytes = (size_t)32 * (WN * HALF * 32 * (EPI == EPI_PARTIAL || EPI == EPI_RESIDUAL ? 4 : 2) + 16);
-    const size_t smem = std::max((size_t)3 * BM * 64 * sizeof(bf16_t), epi_bytes);
-    auto kern = gemm_mfma_kernel<WN, MT, NT, EPI, MIXED>;
+    constexpr size_t smem = GemmLds<WN, MT, NT, EPI, KG>::bytes;
+    static_assert(smem <= 160 * 1024, "LDS");
+    auto kern = gemm_mfma_kernel<WN, MT, NT, EPI, MIXED, KG>;
     if (smem > 65536) {
         static std::atomic<uint64_t> done{0};
         if (int rc = ensure_dynamic_lds((const void*)kern, smem, done)) return rc;
     }
-    hipLaunchKernelGGL(kern, dim3(m_blocks * n_blocks * nsplit), dim3(WN * 64), smem, s, q, m_blocks, n_blocks, stages_total, sps, n_big);
+    hipLaunchKernelGGL(kern, dim3(m_blocks * n_blocks * nsplit), dim3(WN * 64 * KG), smem, s, q, m_blocks, n_blocks, stages_total, sps, n_big);
     return hipGetLastError() == hipSuccess ? 0 : 5;
 }
 
@@ -396,14 +467,17 @@ int launch_epi(const GemmP& p, int tile, hipStream_t s) {
         case TILE_64x128:  if constexpr (!EpiTraits<EPI>::dual) return launch_cfg<4, 2, 1, EPI, false>(p, s); else return 2;
         case TILE_128x128: if constexpr (!EpiTraits<EPI>::dual) return launch_cfg<4, 4, 1, EPI, false>(p, s); else return 2;
         case TILE_96x128:  if constexpr (!EpiTraits<EPI>::dual) return launch_cfg<4, 3, 1, EPI, false>(p, s); else return 2;
+        case TILE2_64x64:  if constexpr (!EpiTraits<EPI>::dual && EPI != EPI_GQA_QKV) return launch_cfg<2, 2, 1, EPI, false, 2>(p, s); else return 2;
+        case TILE2_64x128: if constexpr (!EpiTraits<EPI>::dual) return launch_cfg<4, 2, 1, EPI, false, 2>(p, s); else return 2;
+        case TILE2_96x128: if constexpr (!EpiTraits<EPI>::dual) return launch_cfg<4, 3, 1, EPI, false, 2>(p, s); else return 2;
     }
     return 2;
 }
 
 }  // namespace
 
-int gemm_tile_bm(int tile) { static const int v[TILE_COUNT + 1] = {224, 192, 160, 128, 64, 64, 128, 256, 224, 192, 128, 96, 160}; return v[tile]; }
-int gemm_tile_bn(int tile) { return (tile == TILE_64x128 || tile == TILE_128x128 || tile == TILE_96x128) ? 128 : 256; }
+int gemm_tile_bm(int tile) { static const int v[TILE_END] = {224, 192, 160, 128, 64, 64, 128, 256, 224, 192, 128, 96, 160, 64, 64, 96}; return v[tile]; }
+int gemm_tile_bn(int tile) { return tile == TILE2_64x64 ? 64 : (tile == TILE_64x128 || tile == TILE_128x128 || tile == TILE_96x128 || gemm_tile_two_k_groups(tile)) ? 128 : 256; }
 
 int launch_gemm(const GemmP& p, int epi, int tile, hipStream_t s) {
     if (p.M <= 0 || p.N16 <= 0 || p.K32p <= 0 || (p.K32p & 1) || p.a_rows <= 0 || p.bgroup < 1) return 1;

@@ -82,7 +82,10 @@ enum GemmTile { TILE_224x256 = 0, TILE_192x256, TILE_160x256, TILE_128x256, TILE
                 // 256-column tiles computed by eight waves (csrc/gemm8.hip)
                 TILE8_256x256, TILE8_224x256, TILE8_192x256, TILE8_128x256,
                 TILE_96x128, TILE_COUNT,
-                TILE8_160x256 = TILE_COUNT };                       // (chosen by the cost model only: callers' tile numbers end before it)
+                TILE8_160x256 = TILE_COUNT,                         // (chosen by the cost model only: callers' tile numbers end before it)
+                TILE2_64x64, TILE2_64x128, TILE2_96x128,            // two groups of waves that split K (csrc/gemm.hip); chosen likewise
+                TILE_END };
+inline bool gemm_tile_two_k_groups(int tile) { return tile >= TILE2_64x64 && tile < TILE_END; }
 inline bool gemm_tile_eight_waves(int tile) { return (tile >= TILE8_256x256 && tile <= TILE8_128x256) || tile == TILE8_160x256; }
 int gemm_tile_bm(int tile);
 int gemm_tile_bn(int tile);

@@ -217,6 +217,18 @@ TileChoice choose_tile(int M, int ncols16, int stages, bool dual, bool splittabl
             if (t <= best) { best = t; bc = TileChoice{tile, sp}; }      // (of equals the smaller tile)
         }
     }
+    // Two groups of waves that split K (csrc/gemm.hip) need as many stages each.  Tiles of 64 x 64 where 64 x 128 are 128 workgroups and fewer: us of a whole layer with 64 x 128 / with
+    // these, Gemma QKV 80 workgroups 105.6 / 99.9, 100 122.0 / 117.1, SigLIP QKV 108 53.8 / 51.7, its output projection (3 splits of 6 stages) 108 53.8 / 53.3; but QKV 180 171.6 / 171.1, 200
+    // 182.2 / 182.5, SigLIP QKV 216 60.1 / 61.4.  The others from 24 stages on: 32 stages, by rows, 64 x 128 206 75.8 / 74.0, 269 81.1 / 79.6, 398 90.9 / 89.1, 532 171.6 / 170.7, 96 x 128 607
+    // 105.9 / 105.0, 788 213.1 / 212.1, 968 235.4 / 232.6; 64: 2 720 161.4 / 159.2; 24: 64 x 128 206 75.8 / 75.0; but 18: 64 x 128 512 60.1 / 60.1, 96 x 128 768 69.2 / 69.3; 16: 96 x 128 532 165.6 / 166.3,
+    // 607 105.3 / 106.5; 8: 64 x 128 206 75.8 / 76.2.
+    const int sps = (stages + bc.nsplit - 1) / bc.nsplit;
+    if (sps % 2 == 0 && stages % sps == 0) {
+        const int blocks = (M + 63) / 64 * ((ncols16 + 7) / 8) * bc.nsplit;
+        if (bc.tile == TILE_64x128 && blocks <= 128 && !need.head) bc.tile = TILE2_64x64;
+        else if (bc.tile == TILE_64x128 && sps >= 24) bc.tile = TILE2_64x128;
+        else if (bc.tile == TILE_96x128 && sps >= 24) bc.tile = TILE2_96x128;
+    }
     tuning_report_tile(what, M, ncols16 * 16, stages, gemm_tile_bm(bc.tile), gemm_tile_bn(bc.tile), bc.nsplit, best);
     return bc;
 }
@@ -579,7 +591,7 @@ struct Sched {
         if (c->want(what)) {
             // the name a measurement reports carries the kernel variant: block tile and split-K factor
             c->last_name = std::string(what) + " [" + std::to_string(gemm_tile_bm(tc.tile)) + "x" + std::to_string(gemm_tile_bn(tc.tile)) +
-                           (gemm_tile_eight_waves(tc.tile) ? " 8 waves" : "") + " split " + std::to_string(tc.nsplit) + "]";
+                           (gemm_tile_eight_waves(tc.tile) ? " 8 waves" : gemm_tile_two_k_groups(tc.tile) ? " 2 K groups" : "") + " split " + std::to_string(tc.nsplit) + "]";
             c->note(launch_gemm(p, epi, tc.tile, s), what);
         }
     }

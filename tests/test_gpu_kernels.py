@@ -240,6 +240,37 @@ def test_eight_wave_tiles_of_the_cost_model_against_fp32(M, K, N, act):
     assert torch.equal(out[M], stream[M])
 
 
+# what the cost model gives to the tiles whose K is split between two groups of waves: 64 x 64 (128 workgroups of 64 x 128 and fewer), 64 x 128 and 96 x 128 (24 K
+# stages and more), with rows that end in the first, in the second and behind the last row tile, odd numbers of stages for a group, columns past a block, and
+# stages that the groups cannot share evenly (13 for a split: one group); bias, bias + GELU, residual, and partial sums (act None)
+@pytest.mark.parametrize("M,K,N", [
+    (33, 128, 64), (65, 264, 272), (1, 640, 16), (97, 1152, 1152), (256, 2048, 2560), (190, 1664, 2048),
+    (532, 2048, 2560), (481, 1528, 2512), (449, 4096, 1536), (788, 2048, 2560), (865, 1536, 2544), (609, 4096, 2048)])
+@pytest.mark.parametrize("act", [0, 1, 8, None])
+def test_two_k_groups_of_the_cost_model_against_fp32(M, K, N, act):
+    import rtvla_capi as capi
+    lib = capi.load()
+    if act is None:
+        res = _run(lib, capi, M, K, min(N, 2048), capi.TILE_AUTO, 0)
+    elif act == 0:
+        res = _run(lib, capi, M, K, N, capi.TILE_AUTO, 1)
+    elif act == 1:
+        res = _run_act(lib, capi, M, K, N, act, capi.TILE_AUTO)
+    else:
+        test_residual_epilogue_in_place_against_fp32(M, K, N)
+        return
+    assert res is not None and res[0] <= REL_TOL and res[1] <= 1.01, res
+
+
+def test_forward_takes_two_k_groups_where_workgroups_are_few():
+    import synthetic as syn
+    import rtvla_capi as capi
+    from pi0_infer import Pi0Inference
+    m = Pi0Inference(syn.pi0_checkpoint(5, 0, "cuda:0", 1, 1), 1, 8)
+    names = [m._engine.ctx.time_launch(stage, 0, 0, 0, 1, torch.cuda.current_stream().cuda_stream)[1] for stage in (capi.STAGE_VISION_LAYER, capi.STAGE_PREFIX_LAYER)]
+    assert names == ["vision qkv [64x64 2 K groups split 1]", "prefix qkv [64x64 2 K groups split 1]"]
+
+
 def test_eight_wave_tiles_give_what_their_offsets_cannot_reach_to_the_four_wave_kernel():
     import rtvla_capi as capi
     lib = capi.load()
