@@ -1,5 +1,6 @@
-"""Build librtvla.so (gfx950) in-tree with hipcc: python build.py [-v] [-DNAME ...] [-o OUT.so]
-(-D / -o make a variant build, e.g. -DRTVLA_TUNING with its environment knobs, next to the shipped library)."""
+"""Build librtvla.so (gfx950) and _rtvla_host.so (the per-observation calls, against the installed PyTorch) in-tree with hipcc:
+python build.py [-v] [-DNAME ...] [-o OUT.so]
+(-D / -o make a variant build of the library, e.g. -DRTVLA_TUNING with its environment knobs, next to the shipped one)."""
 import os
 import subprocess
 import sys
@@ -8,6 +9,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "librtvla.so")
+HOST_LIB = os.path.join(HERE, "_rtvla_host.so")
 SOURCES = ["gemm.hip", "gemm8.hip", "skinny.hip", "attention.hip", "misc.hip", "dm0.hip", "flash.hip", "flow.hip", "rtvla.hip", "transforms.hip"]
 # bit-exact parity with host arithmetic (Pillow, numpy): no fused multiply-adds in these files
 # flash.hip: MFMA results in ordinary VGPRs (the softmax reads every logit; the accumulator-register form costs a copy each)
@@ -35,9 +37,21 @@ def _compile(job):
     return obj, err
 
 
+def _build_host():
+    import sysconfig
+    from torch.utils.cpp_extension import include_paths, library_paths
+    cmd = [_hipcc(), "-x", "c++", "-std=c++17", "-O3", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__"]
+    cmd += ["-I" + d for d in include_paths(device_type="cuda") + [sysconfig.get_paths()["include"]]]
+    cmd += [os.path.join(CSRC, "host_calls.cpp"), "-o", HOST_LIB, "-L" + HERE, "-l:librtvla.so", "-Wl,-rpath,$ORIGIN"]
+    cmd += ["-L" + d for d in library_paths(device_type="cuda")] + ["-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("hipcc failed on host_calls.cpp:\n" + r.stderr)
+
+
 def build(force=True, verbose=False, defines=(), out=LIB):
-    """Compile every HIP source for gfx950 and link the shared library."""
-    if not force and os.path.exists(out):
+    """Compile every HIP source for gfx950 and link the shared library; with it, the module of host calls."""
+    if not force and os.path.exists(out) and (out != LIB or os.path.exists(HOST_LIB)):
         return out
     tag = "" if out == LIB else "." + os.path.splitext(os.path.basename(out))[0]
     with ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 4)) as ex:
@@ -50,6 +64,8 @@ def build(force=True, verbose=False, defines=(), out=LIB):
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stderr)
+    if out == LIB:
+        _build_host()
     return out
 
 

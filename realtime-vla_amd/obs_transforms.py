@@ -18,6 +18,7 @@ class ObservationTransforms:
         if not torch.cuda.is_available():
             raise RuntimeError("realtime-vla_amd needs a ROCm GPU (MI355X / gfx950); there is no CPU path")
         self.lib = capi.load()
+        self._host = capi.load_host()
         self.model_version = model_version
         self.mode = 0 if model_version == "pi0" else 1
         self.norm_stats = norm_stats
@@ -78,6 +79,12 @@ class ObservationTransforms:
         """_resize_with_pad + _normalize_image of one image into out_view (bf16 [224, 224, 3], e.g. one view of the
         model's observation_images_normalized buffer).  Nothing is allocated for a frame that is on the device already;
         static_scratch (frames of at most 2160 rows at full width) is kept for its callers."""
+        rc = None if static_scratch else self._host.frame(image, out_view, self._index)
+        if rc is not None:                                        # a plain frame and view: launched
+            if rc:
+                self._check(rc, "rtvla_preprocess_frame")
+            self._keep = image
+            return out_view
         if out_view.dtype is not torch.bfloat16 or out_view.shape != _VIEW_SHAPE or not out_view.is_contiguous():
             self._frame(image)                                    # (a bad image is reported first)
             raise ValueError("out_view must be a contiguous bf16 [224, 224, 3] tensor")
@@ -103,6 +110,11 @@ class ObservationTransforms:
         if "state" not in self._stats:
             return None, None
         a, b, n_stats = self._stats["state"]
+        done = self._host.state(state, a, b, n_stats, self.mode, self._row, self._bin_row if want_bins else None, out_bf16, self._index)
+        if type(done) is tuple:                                    # plain values: launched
+            return done
+        if done is not None:
+            self._check(done, "rtvla_preprocess_state_host")
         st = np.ascontiguousarray(state, dtype=np.float64)         # travels with the launch
         z = torch.empty_like(self._row)
         bins = torch.empty_like(self._bin_row) if want_bins else None
@@ -119,6 +131,11 @@ class ObservationTransforms:
         if "actions" not in self._stats:
             return None
         a, b, n_stats = self._stats["actions"]
+        done = self._host.actions(actions_bf16, ori_state, a, b, n_stats, self.mode, self.action_dim, self._row, self._index)
+        if type(done) is torch.Tensor:
+            return done
+        if done is not None:
+            self._check(done, "rtvla_postprocess_actions_host")
         if actions_bf16.dtype is not torch.bfloat16 or actions_bf16.shape[-1] != 32 or not actions_bf16.is_contiguous():
             raise ValueError("actions must be a contiguous bf16 [chunk, 32] tensor")
         chunk = actions_bf16.shape[0]

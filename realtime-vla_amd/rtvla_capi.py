@@ -4,10 +4,13 @@ The library is the only compute path: there is no eager / CPU fallback, and impo
 module on a machine where the shared library has not been built raises.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "librtvla.so")
+HOST_PATH = os.path.join(HERE, "_rtvla_host.so")
 
 PI0, PI05, DM0 = 0, 1, 2
 
@@ -110,6 +113,22 @@ def load():
             fn.restype, fn.argtypes = res, args
         _lib = lib
     return _lib
+
+
+_host = None
+
+
+def load_host():
+    """The module of csrc/host_calls.cpp; raises if it is missing."""
+    global _host
+    if _host is None:
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError("_rtvla_host.so is not built (%s); run `python realtime-vla_amd/build.py`" % HOST_PATH)
+        import torch                                           # noqa: F401  (the module links against its libraries)
+        loader = importlib.machinery.ExtensionFileLoader("_rtvla_host", HOST_PATH)
+        _host = importlib.util.module_from_spec(importlib.util.spec_from_loader("_rtvla_host", loader))
+        loader.exec_module(_host)
+    return _host
 
 
 class RtvlaError(RuntimeError):

@@ -143,3 +143,86 @@ def test_whole_observation_through_the_policy():
     ref_actions = policy.forward(imgs, st, torch.from_numpy(noise)).cpu().float().numpy()
     ref = T.postprocess_actions(ref_actions, stats["actions"], "pi0", state, 7)
     assert out.shape == (10, 7) and np.array_equal(out, ref)
+
+
+class _GeneralWay:
+    """In place of the module of host calls: every call goes the general way."""
+    frame = state = actions = staticmethod(lambda *args: None)
+
+
+def _outcome(call):
+    try:
+        return call()
+    except Exception as e:
+        return type(e), str(e)
+
+
+@pytest.mark.parametrize("version", ["pi0", "pi05"])
+def test_host_calls_and_the_general_way_agree(version):
+    """What the host calls take and what they leave to the general way, accepted or refused: the same bits, the same errors."""
+    from obs_transforms import ObservationTransforms
+    rng = np.random.RandomState(41)
+    stats = {g: {"mean": rng.randn(7).tolist(), "std": (rng.rand(7) + 0.5).tolist(), "q01": (-1 - rng.rand(7)).tolist(), "q99": (1 + rng.rand(7)).tolist()}
+             for g in ("state", "actions")}
+    plain, general = (ObservationTransforms(version, stats) for _ in range(2))
+    general._host = _GeneralWay
+    u8 = torch.from_numpy(rng.randint(0, 256, size=(61, 47, 3)).astype(np.uint8)).cuda()
+    f32 = u8.float() / 255 + 0.001
+
+    class Sub(torch.Tensor):
+        pass
+
+    frames = [u8, f32, u8.permute(2, 0, 1).contiguous(), f32.permute(2, 0, 1).contiguous(), u8.permute(1, 0, 2), f32.permute(2, 0, 1), u8[::2, 1:], u8.cpu(), u8.cpu().numpy(),
+              f32.double(), f32.half(), u8.long(), u8.as_subclass(Sub), torch.nn.Parameter(f32), u8[:0], u8[..., :2], u8[0], u8[None], u8.bool(), u8[:1].expand(9000, 47, 3).contiguous()]
+    for i, frame in enumerate(frames):
+        for view in (lambda: torch.full((224, 224, 3), 7.0, dtype=torch.bfloat16, device="cuda:0"), lambda: torch.zeros(224, 224, 3, device="cuda:0"),
+                     lambda: torch.zeros(3, 224, 224, 3, dtype=torch.bfloat16, device="cuda:0")[1], lambda: torch.zeros(224, 224, 6, dtype=torch.bfloat16, device="cuda:0")[..., :3]):
+            got, want = (_outcome(lambda: tr.resize_pad_normalize_into(frame, view())) for tr in (plain, general))
+            assert got == want if isinstance(want, tuple) else torch.equal(got, want), i
+    st = rng.randn(7)
+    states = [st, st.tolist(), st.astype(np.float32), st[::-1], np.concatenate([st, st])[::2], st.astype(">f8"), torch.from_numpy(st), np.float64(0.3), rng.randn(32), rng.randn(33),
+              np.zeros(0), rng.randn(2, 7), np.arange(7), "no"]
+    for i, values in enumerate(states):
+        for bins in (False, True):
+            for out in (None, 1):
+                outs = [torch.full((32,), 5.0, dtype=torch.bfloat16, device="cuda:0") if out else None for _ in range(2)]
+                got, want = (_outcome(lambda: tr._normalize_state(values, want_bins=bins, out_bf16=o)) for tr, o in zip((plain, general), outs))
+                if not isinstance(want[0], torch.Tensor):
+                    assert got == want, i
+                    continue
+                assert torch.equal(got[0], want[0]) and (torch.equal(got[1], want[1]) if bins else got[1] is want[1] is None), i
+                assert got[0].dtype == want[0].dtype and (not out or torch.equal(*outs))
+        acts = torch.from_numpy(rng.randn(50, 32).astype(np.float32)).to(torch.bfloat16).cuda()
+        for a in (acts, acts[:1], acts[:0], acts[::2], acts.float(), acts[:, :7].contiguous(), acts.view(2, 25, 32), acts[0], acts.as_subclass(Sub)):
+            got, want = (_outcome(lambda: tr.postprocess_actions(a, values)) for tr in (plain, general))
+            assert got == want if isinstance(want, tuple) else torch.equal(got, want), i
+
+
+def test_host_calls_follow_the_current_stream_and_are_captured():
+    from obs_transforms import ObservationTransforms
+    rng = np.random.RandomState(43)
+    stats = {g: {"mean": rng.randn(7).tolist(), "std": (rng.rand(7) + 0.5).tolist()} for g in ("state", "actions")}
+    tr = ObservationTransforms("pi0", stats)
+    frame = torch.from_numpy(rng.randint(0, 256, size=(300, 400, 3)).astype(np.uint8)).cuda()
+    out, actions, st = torch.zeros(224, 224, 3, dtype=torch.bfloat16, device="cuda:0"), torch.randn(50, 32, device="cuda:0").to(torch.bfloat16), rng.randn(7)
+
+    def observe():
+        tr.resize_pad_normalize_into(frame, out)
+        return tr._normalize_state(st, want_bins=True) + (tr.postprocess_actions(actions, st),)
+    want = [t.clone() for t in observe()] + [out.clone()]
+    torch.cuda.synchronize()
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    out.zero_()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = observe()
+    side.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip((*got, out), want))
+    with torch.cuda.graph(graph, stream=side):
+        got = observe()
+    for _ in range(3):
+        for t in (*got, out):
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip((*got, out), want))
