@@ -62,9 +62,13 @@ RTVLA_DEVICE int clip8(int v) { v >>= PRECISION_BITS; return v < 0 ? 0 : (v > 25
 // across into an 8-bit LDS tile, and that tile down into the output.  Neighbouring row blocks resample the rows they share twice
 // ((TH + 2) / TH of the work for TH output rows); in exchange nothing but the frame is read and nothing but the result written, and the
 // second launch with its round trip through memory is gone.  Measured (480 x 640 uint8, one frame): two launches, each thread deriving the
-// weights of its own pixel, 11.7 us; this one 4.9 us.  TH = 4 gives large frames (many taps per pixel) twice the workgroups.
+// weights of its own pixel, 11.7 us; this one 3.9 us.  TH = 4 gives large frames (many taps per pixel) twice the workgroups.
 enum FrameFormat { FRAME_U8_HWC = 0, FRAME_F32_HWC, FRAME_F32_CHW, FRAME_U8_CHW };
-constexpr int TW = 32, NT = 512;            // columns and threads of a workgroup
+constexpr int TW = 32;                      // columns of a workgroup
+// Threads: a thread takes a column of every (threads / TW)-th source row, and all wait for the loads of one row before those of their next.  With 1 024 instead of 512 a frame of bytes
+// of 300 x 400, 480 x 640, 719 x 1 279, 1 080 x 1 920 takes 3.51, 3.92, 4.93, 6.73 instead of 3.42, 4.11, 5.15, 7.89 us: from 24 source rows a block on (the first has 22, the second 30).
+// Staged float frames, whose loads are all on the way at once and whose bytes it converts: 3.91, 4.38, 6.46, 10.1 instead of 4.06, 5.03, 7.04, 12.1.
+constexpr int NT_MANY_ROWS = 24, STAGED_NT = 1024;
 struct FrameP { const uint8_t* src; int h, w, rw, rh, pad_top, pad_left, taps_x, taps_y, max_rows, pitch; bf16_t* dst; Axis x, y; };      // taps: rounded up to 4
 
 // numpy's / torch's float -> uint8: truncation to an integer, low byte
@@ -92,11 +96,13 @@ RTVLA_DEVICE void resize_down(const FrameP& p, const Window* win, const bf16_t* 
     const int vfirst = win[TW + rr].first - lo, vcount = win[TW + rr].count;
     if (count > 0 && vcount > 0) {
         int a0 = 1 << (PRECISION_BITS - 1), a1 = a0, a2 = a0;
-        for (int t = 0; t < vcount; ++t) {
-            const unsigned e = inter[(vfirst + t) * TW + c];
-            const int k = wy[t * TH + rr];
-            a0 += __mul24(e & 255, k); a1 += __mul24((e >> 8) & 255, k); a2 += __mul24(e >> 16, k);
-        }
+        for (int t = 0; t < vcount; t += 4)                                    // (past the window: zero weights, and rows that `inter` has room for)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const unsigned e = inter[(vfirst + t + i) * TW + c];
+                const int k = wy[(t + i) * TH + rr];
+                a0 += __mul24(e & 255, k); a1 += __mul24((e >> 8) & 255, k); a2 += __mul24((e >> 16) & 255, k);
+            }
         v0 = clip8(a0); v1 = clip8(a1); v2 = clip8(a2);
     }
     bf16_t* o = p.dst + ((size_t)(y0 + rr) * 224 + x0 + c) * 3;
@@ -105,8 +111,8 @@ RTVLA_DEVICE void resize_down(const FrameP& p, const Window* win, const bf16_t* 
 
 // Float frames, whose values cost six instructions each to become bytes: the source rectangle of the block is loaded in whole lines, converted once and
 // staged in LDS as dwords R G B - (windows overlap by half, and four-tap groups round them up, so resize_kernel loads and converts each value 2.8 times);
-// the first loads are on the way while the weights are derived.  us per frame of 300 x 400, 480 x 640, 719 x 1 279, 1 080 x 1 920: 4.6, 5.8, 8.7, 15.4
-// without and 4.3, 5.3, 7.0, 11.2 with (1.7 of it the launch).  Frames that are not reduced (4 taps) are as fast or faster without (224 x 224
+// the first loads are on the way while the weights are derived.  us per frame of 300 x 400, 480 x 640, 719 x 1 279, 1 080 x 1 920: 4.2, 4.9, 9.4, 14.8
+// without and 3.9, 4.4, 6.5, 10.1 with (1.6 of it the launch).  Frames that are not reduced (4 taps) are as fast or faster without (224 x 224
 // 3.8 / 4.0), as are bytes (480 x 640 4.3 / 4.65), and rectangles of more than half a CU's LDS stay with resize_kernel.
 struct Raw4 { f32x4 v[3]; };
 template <int FMT>
@@ -132,7 +138,7 @@ RTVLA_DEVICE uint4 px4(const Raw4& r) {
 }
 
 template <int FMT, int TH>
-__global__ __launch_bounds__(NT) void resize_staged_kernel(FrameP p) {
+__global__ __launch_bounds__(STAGED_NT) void resize_staged_kernel(FrameP p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     int4* const wx = (int4*)smem;                                              // [taps_x / 4][TW]
     unsigned* const stage = (unsigned*)(wx + (p.taps_x >> 2) * TW);            // [row][pitch] pixels as dwords
@@ -140,6 +146,7 @@ __global__ __launch_bounds__(NT) void resize_staged_kernel(FrameP p) {
     unsigned* const inter = (unsigned*)(wy + p.taps_y * TH);                   // [row][TW], three bytes each
     __shared__ Window win[TW + TH];
     __shared__ bf16_t value[256];
+    constexpr int NT = STAGED_NT;
     const int tid = threadIdx.x, x0 = blockIdx.x * TW, y0 = blockIdx.y * TH;
     // the source rectangle of this block
     const int rx0 = max(x0 - p.pad_left, 0), rx1 = min(x0 + TW - p.pad_left, p.rw) - 1, ry0 = max(y0 - p.pad_top, 0), ry1 = min(y0 + TH - p.pad_top, p.rh) - 1;
@@ -149,7 +156,7 @@ __global__ __launch_bounds__(NT) void resize_staged_kernel(FrameP p) {
         window_bounds(p.y, ry0, &lo, &skip); window_bounds(p.y, ry1, &skip, &hi);
     }
     const int groups = (hi_x - lo_x + 3) >> 2, items = (hi - lo) * groups;
-    constexpr int UN = 3;
+    constexpr int UN = 2;
     Raw4 raw[UN];
     auto pixel = [&](int i) { return (size_t)(lo + i / groups) * p.w + lo_x + 4 * (i % groups); };
 #pragma unroll
@@ -202,7 +209,7 @@ __global__ __launch_bounds__(NT) void resize_staged_kernel(FrameP p) {
     resize_down<TH>(p, win, value, wy, inter, lo, count, tid, x0, y0);
 }
 
-template <int FMT, int TH>
+template <int FMT, int TH, int NT>
 __global__ __launch_bounds__(NT) void resize_kernel(FrameP p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     int4* const wx = (int4*)smem;                                              // [taps_x / 4][TW]
@@ -316,8 +323,12 @@ __global__ void state_kernel(StateP p) {
     if (p.bins) {
         // np.digitize(z, linspace(-1, 1, 257)[:-1]) - 1: number of edges <= z, minus one; edge j is what
         // numpy's linspace yields: -1 + j * (2 / 256) (the step is exact in binary)
+        // (by bisection: 256 comparisons one after another were 3.8 of the launch's 5.4 us)
+        auto below = [&](int j) { return (-1.0 + j * (2.0 / 256.0)) <= z; };
         int cnt = 0;
-        for (int j = 0; j < 256; ++j) cnt += (-1.0 + j * (2.0 / 256.0)) <= z;
+#pragma unroll
+        for (int s = 128; s; s >>= 1) cnt += below(cnt + s - 1) ? s : 0;
+        cnt += cnt == 255 && below(255);
         p.bins[i] = cnt - 1;
     }
 }
@@ -374,10 +385,11 @@ void launch_resize(FrameP p, hipStream_t s) {
         if (p.taps_x > 4 && staged <= STAGED_LDS) {
             auto kern = resize_staged_kernel<FMT, TH>;
             static std::atomic<uint64_t> done{0};
-            if (ensure_dynamic_lds((const void*)kern, STAGED_LDS, done) == 0) { hipLaunchKernelGGL(kern, dim3(224 / TW, 224 / TH), dim3(NT), staged, s, p); return; }
+            if (ensure_dynamic_lds((const void*)kern, STAGED_LDS, done) == 0) { hipLaunchKernelGGL(kern, dim3(224 / TW, 224 / TH), dim3(STAGED_NT), staged, s, p); return; }
             (void)hipGetLastError();                                           // (the refusal is not an error of the launch below, which needs no more than the default)
         }
-    hipLaunchKernelGGL((resize_kernel<FMT, TH>), dim3(224 / TW, 224 / TH), dim3(NT), smem, s, p);
+    if (p.max_rows > NT_MANY_ROWS) hipLaunchKernelGGL((resize_kernel<FMT, TH, 1024>), dim3(224 / TW, 224 / TH), dim3(1024), smem, s, p);
+    else hipLaunchKernelGGL((resize_kernel<FMT, TH, 512>), dim3(224 / TW, 224 / TH), dim3(512), smem, s, p);
 }
 template <int FMT>
 int launch_frame(const FrameP& p, hipStream_t s) {

@@ -30,7 +30,8 @@ def test_image_preprocessing_matches_the_pillow_restatement_bit_exactly(h, w):
     assert torch.equal(got, want), "mismatching elements: %d" % (got != want).sum().item()
 
 
-@pytest.mark.parametrize("h,w", [(1, 1), (4, 5), (9, 300), (300, 9), (223, 225), (479, 641), (717, 1279), (2700, 1801)])
+# (448 and 482 rows: 24 and 25 source rows a block, either side of the rule for its threads)
+@pytest.mark.parametrize("h,w", [(1, 1), (4, 5), (9, 300), (300, 9), (223, 225), (448, 448), (482, 481), (479, 641), (717, 1279), (2700, 1801)])
 @pytest.mark.parametrize("fmt", ["u8", "u8_chw", "f32", "f32_chw"])
 def test_frame_formats_at_the_edges_of_the_tiles(h, w, fmt):
     """Every frame format on the device: single pixels, strips narrower than a tile, windows that end with the buffer, both tile heights."""
