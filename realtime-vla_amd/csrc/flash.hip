@@ -16,10 +16,11 @@
 // step in the key order of the stored V^T: no shuffles between the two products.  The loop is software-pipelined over the
 // 32-key blocks (see flash_kernel).
 //
-// Measured on MI355X (48 heads x 2705 tokens, queries without their scale): 146 us where the version without the pipeline, with register staging and a
-// rescale in most tiles took 161 us on the same machine; 71 us for 48 x 2048 tokens, which fit one round of 768
-// workgroups (0.72 PFLOP/s).  LDS reads (ds_read_b128: 256 B/clk per CU measured) are 18 % busy, the MFMA pipe 37 %, the
-// VALU 59 %; the second, a third full round of 2705-token heads (1 056 workgroups on 768 places) costs about 45 us.
+// Measured on MI355X, 16 / 32 / 48 heads x 2 705 tokens, in a ViT layer: 40 / 70 / 105 us.  Steps to there: softmax of every second block kept beside its MFMAs (see the end
+// of `step`) and waits for single LDS reads 49.6 / 75.5 / 119.9 -> 44.8 / 69.7 / 111.7; stages that K enters a tile earlier, requested by buffer loads whose addresses are
+// scalar, 43.2 / 68.9 / 108.1; last row blocks at the end of the grid, where the waves past the last row only stage, 42.1 / 68.7 / 105.5; the two kinds of MFMA in turn 40.0 / 69.6 / 104.9.
+// What the rest is spent on, left out one at a time of 111: staging 11, LDS reads 13, v_dot2_f32_bf16 of the row sums 6 (it does not run beside MFMAs: 8 of those take 145 ns a
+// wave, with 16 v_exp, 32 v_max3 or 32 v_cvt_pk between them as long, with 32 v_dot2 212), maxima and their branch 5, the barrier 1; without all of these 73.
 #include "kernels.h"
 #include <type_traits>
 
@@ -60,6 +61,15 @@ constexpr int FLASH_STAGES = 3;
 // The forward takes it: its queries are rounded to bf16 once, behind the scale.  The instance without is for callers whose queries are bf16 already
 // (rtvla_attention): rounded again behind the scale, their outputs' error against 64 bits would go from 2.3e-3 to 3.0e-3, in sharp rows (logits of
 // standard deviation 6) from 1.7e-3 to 4.8e-3.
+// All but this wave's newest N loads have landed, its LDS reads are back, and so for every wave of the workgroup
+template <int N> RTVLA_DEVICE void wait_and_meet() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(N | 7 << 4);             // vmcnt(N) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
 template <int HD, bool SCALED>
 __global__ __launch_bounds__(256, 3)
 void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
@@ -77,14 +87,16 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
     // one XCD and its K / V^T are fetched into one L2.
     int batch, item;
     if (batches_per_xcd > 0) {
-        const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-        batch = xcd * batches_per_xcd + idx / items_per_batch; item = idx % items_per_batch;
+        // (the last row blocks of the heads, which may have few rows, come last: 48 heads x 2 705 rows are 1 008 whole blocks on 768 places, and 48 of 17 rows)
+        const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3, whole = batches_per_xcd * (items_per_batch - 1);
+        batch = xcd * batches_per_xcd + (idx < whole ? idx / (items_per_batch - 1) : idx - whole);
+        item = idx < whole ? idx % (items_per_batch - 1) : items_per_batch - 1;
     } else { batch = blockIdx.x / items_per_batch; item = blockIdx.x % items_per_batch; }
     const bf16_t* const qbase = p.q + (size_t)batch * p.q_bstride;
     const uint4* const kbase = (const uint4*)(p.k + (size_t)batch * p.k_bstride);
     const uint4* const vbase = (const uint4*)(p.vt + (size_t)batch * p.vt_bstride);
     const int row0 = (item * 4 + w) * 32;
-    const bool active = row0 < p.rows;                  // a wave past the last row still stages tiles and meets the barriers
+    const bool active = __builtin_amdgcn_readfirstlane(row0) < p.rows;         // a wave past the last row still stages tiles and meets the barriers
 
     bf16x8 qf[DS];
 #pragma unroll
@@ -109,15 +121,13 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
     if (p.causal) ntiles = min(ntiles, ((min(item * 128 + 128, p.rows) - 1) / p.group >> 6) + 1);
 
     // Staging: each wave copies whole 1 KB pieces (64 lanes x 16 bytes, contiguous on both sides) from global memory straight
-    // into LDS; no staging registers and no LDS write instructions.  Tiles are requested in order, each into the stage after
-    // the previous one's.  Only the last tile can reach past the allocated rows (an odd number of 32-key blocks): its second
-    // block is then replaced by the first (finite data; those keys are masked below).  A request past the last tile repeats
-    // the last tile (into a stage nobody reads any more), so the loops below need no branch around it.
-    typedef const __attribute__((address_space(1))) void* gptr_t;
+    // into LDS; no staging registers and no LDS write instructions.  Stage T % 3 holds what tile T reads: V^T of tile T and K of tile T + 1 (step g takes
+    // S^T of block g + 1, and reads the K fragments of g + 2).  It is requested when tile T - 3 has been read by every wave and awaited two tiles later: with K and V^T of one
+    // tile in a stage, K of a tile is dead when the tile runs, and the requests had one tile's time.  Only the last tile can reach past the allocated rows (an odd number of
+    // 32-key blocks): its second block is then replaced by the first (finite data; those keys are masked below).  A request past the last tile repeats
+    // the last tile (for nobody).
     typedef __attribute__((address_space(3))) void* lptr_t;
-    const int wu = __builtin_amdgcn_readfirstlane(w);                           // wave-uniform copy: LDS addresses stay scalar
-    const unsigned char* ksrc0 = (const unsigned char*)kbase;                   // byte addresses of the next tile (wave-uniform)
-    const unsigned char* vsrc0 = (const unsigned char*)vbase;
+    const int wu = __builtin_amdgcn_readfirstlane(w);                           // wave-uniform copy: everything but the lane's offset stays scalar
     unsigned koff[NPT], voff[NPT];                                              // this lane's byte offsets inside a tile
 #pragma unroll
     for (int cc = 0; cc < NPT; ++cc) {
@@ -126,50 +136,42 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
         voff[cc] = (unsigned)(((i0 >> 7) * ldvt32 + ((i0 & 127) >> 6)) * 64 + lane) * 16u;
     }
     const int half_tile = (keys32 & 1) ? (keys32 >> 1) : -1;                    // the tile that holds a single 32-key block
-    int next_tile = 0;
-    unsigned wr_off = 0;                                                         // LDS byte offset of the stage the next request fills
-    auto stage_next = [&]() {
-        unsigned char* const dst = smem + wr_off;
-        if (next_tile + 1 < ntiles) {                                           // the common case: a whole tile, pointers move on
+    auto request = [&](const void* base, unsigned off, int at) __attribute__((always_inline)) {
+#ifdef __HIP_DEVICE_COMPILE__                                                  // (the host pass does not know the LDS load's size)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, -1, 0x00027000), (lptr_t)(smem + at), 16, (int)off, 0, 0, 0);
+#endif
+    };
+    auto stage_k = [&](int t, unsigned stage_off) __attribute__((always_inline)) {
+        t = min(t, ntiles - 1);
 #pragma unroll
-            for (int cc = 0; cc < NPT; ++cc) {
-                const int i0 = wu * 64 + 256 * cc;
-                __builtin_amdgcn_global_load_lds((gptr_t)(ksrc0 + koff[cc]), (lptr_t)(dst + (size_t)i0 * 16), 16, 0, 0);
-                __builtin_amdgcn_global_load_lds((gptr_t)(vsrc0 + voff[cc]), (lptr_t)(dst + KBYTES + (size_t)i0 * 16), 16, 0, 0);
-            }
-            ksrc0 += KBYTES;
-            vsrc0 += 128 * 16;
-        } else {
-            const bool half = ntiles - 1 == half_tile;
-#pragma unroll
-            for (int cc = 0; cc < NPT; ++cc) {
-                const int i0 = wu * 64 + 256 * cc;
-                const bool second = ((i0 / (KD * 128)) & 1) != 0;               // K: pieces of keys 32..63 of the tile
-                __builtin_amdgcn_global_load_lds((gptr_t)(ksrc0 + koff[cc] - ((half && second) ? KD * 128 * 16 : 0)),
-                                                 (lptr_t)(dst + (size_t)i0 * 16), 16, 0, 0);
-                __builtin_amdgcn_global_load_lds((gptr_t)(vsrc0 + voff[cc] - ((half && ((i0 & 127) >> 6)) ? 64 * 16 : 0)),
-                                                 (lptr_t)(dst + KBYTES + (size_t)i0 * 16), 16, 0, 0);
-            }
+        for (int cc = 0; cc < NPT; ++cc) {
+            const int i0 = wu * 64 + 256 * cc;
+            const bool second = ((i0 / (KD * 128)) & 1) != 0;                   // pieces of keys 32..63 of the tile
+            request((const unsigned char*)kbase + (size_t)t * KBYTES - (t == half_tile && second ? KD * 128 * 16 : 0), koff[cc], stage_off + i0 * 16);
         }
-        ++next_tile;
-        wr_off = wr_off == (FLASH_STAGES - 1) * 2 * KBYTES ? 0 : wr_off + 2 * KBYTES;
+    };
+    auto stage_v = [&](int t, unsigned stage_off) __attribute__((always_inline)) {
+        t = min(t, ntiles - 1);
+#pragma unroll
+        for (int cc = 0; cc < NPT; ++cc) {
+            const int i0 = wu * 64 + 256 * cc;
+            request((const unsigned char*)vbase + (size_t)t * (128 * 16) - (t == half_tile && ((i0 & 127) >> 6) ? 64 * 16 : 0), voff[cc], stage_off + KBYTES + i0 * 16);
+        }
     };
 
     // fragment reads of a 32-key block: the lane-dependent part of the address is shared by all of them, the stage is a
     // scalar byte offset that rotates once per tile
     const int lane_piece = ((n >> 4) * KD * 64 + h * 16 + (n & 15)) * 16;
     const int lane_piece_v = ((n >> 4) * 2 * 64 + h * 16 + (n & 15)) * 16 + KBYTES;
-    auto read_k = [&](unsigned stage_off, int b, bf16x8 (&kf)[DS]) __attribute__((always_inline)) {
-        const unsigned char* kt = smem + stage_off + lane_piece;
-#pragma unroll
-        for (int s4 = 0; s4 < DS; ++s4) kf[s4] = *(const bf16x8*)(kt + ((2 * b * KD + (s4 >> 1)) * 64 + 2 * (s4 & 1) * 16) * 16);
+    auto piece_k = [&](unsigned stage_off, int b, int s4) __attribute__((always_inline)) {
+        return *(const bf16x8*)(smem + stage_off + lane_piece + ((2 * b * KD + (s4 >> 1)) * 64 + 2 * (s4 & 1) * 16) * 16);
     };
-    auto read_v = [&](unsigned stage_off, int b, bf16x8 (&vf)[2][DT2]) __attribute__((always_inline)) {
-        const unsigned char* vt = smem + stage_off + lane_piece_v;
+    auto read_k = [&](unsigned stage_off, int b, bf16x8 (&kf)[DS]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int t = 0; t < DT2; ++t) vf[q][t] = *(const bf16x8*)(vt + ((2 * t * 2 + b) * 64 + 2 * q * 16) * 16);
+        for (int s4 = 0; s4 < DS; ++s4) kf[s4] = piece_k(stage_off, b, s4);
+    };
+    auto piece_v = [&](unsigned stage_off, int b, int q, int t) __attribute__((always_inline)) {
+        return *(const bf16x8*)(smem + stage_off + lane_piece_v + ((2 * t * 2 + b) * 64 + 2 * q * 16) * 16);
     };
     const bf16x2 ones = {(bf16_t)1.0f, (bf16_t)1.0f};
     // masks of block g: keys past the end, and (causal) keys after the row's own token
@@ -180,20 +182,19 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
             if (g * 32 + 8 * (e >> 2) + 4 * h + (e & 3) > last) st[e] = NEG_BIG;
     };
     auto lane_max = [&](const f32x16& st) __attribute__((always_inline)) {
-        float mx0 = st[0], mx1 = st[8];
-#pragma unroll
-        for (int e = 1; e < 8; ++e) { mx0 = fmaxf(mx0, st[e]); mx1 = fmaxf(mx1, st[8 + e]); }
-        return fmaxf(mx0, mx1);
+        const auto max3 = [](float a, float b, float c) { return fmaxf(fmaxf(a, b), c); };
+        const float mx0 = max3(max3(max3(st[0], st[1], st[2]), st[3], st[4]), st[5], st[6]), mx1 = max3(max3(max3(st[8], st[9], st[10]), st[11], st[12]), st[13], st[14]);
+        return max3(mx0, mx1, fmaxf(st[7], st[15]));
     };
     // One pipeline step for block g = 2 T + b.  On entry: s_cur = S^T(g), kf = K fragments of block g+1, vf = V^T fragments and
     // p_prev = probabilities of block g-1.  On exit: s_next = S^T(g+1), kf = K fragments of g+2, vf / p_cur those of block g.
-    // `off_v` is the stage of tile T, `off_k` that of the tile block g+2 lies in (T+1).
-    auto step = [&](auto edge_tag, int g, int b, unsigned off_v, unsigned off_k, f32x16& s_cur, f32x16& s_next, bf16x8 (&kf)[DS],
+    // `off` is the stage of tile T, which holds block g's half of V^T and, as the same half of K, block g+2.
+    auto step = [&](auto edge_tag, int g, int b, unsigned off, f32x16& s_cur, f32x16& s_next, bf16x8 (&kf)[DS],
                     bf16x8 (&vf)[2][DT2], bf16x8 (&p_prev)[2], bf16x8 (&p_cur)[2]) __attribute__((always_inline)) {
         constexpr bool EDGE = decltype(edge_tag)::value;
         if (EDGE) mask(g, s_cur);
         const float mx = SCALED ? lane_max(s_cur) : halves_max(lane_max(s_cur));
-        if (__any(mx > (SCALED ? slack : m + slack))) {
+        if (__builtin_expect(__any(mx > (SCALED ? slack : m + slack)), 0)) {
             // rare: the accumulator and the pending probabilities of block g-1 (still in the old scale) move to the new one
             const float mnew = SCALED ? m + fmaxf(halves_max(mx), 0.f) : fmaxf(m, mx);
             const float alpha = __builtin_amdgcn_exp2f((m - mnew) * c);
@@ -213,15 +214,16 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
             m = mnew;
         }
         // ---- the straight-line part: 8 MFMAs, the softmax of block g, 8 fragment reads ----
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int t = 0; t < DT2; ++t) o[t] = mfma32(vf[q][t], p_prev[q], o[t]);
-        read_v(off_v, b, vf);
+        static_assert(DS == 2 * DT2, "MFMAs in pairs");
         s_next = start;
 #pragma unroll
-        for (int s4 = 0; s4 < DS; ++s4) s_next = mfma32(kf[s4], qf[s4], s_next);
-        read_k(off_k, b, kf);
+        for (int i = 0; i < DS; ++i) {                   // (in turn: the four of S^T are a chain)
+            const int q = i / DT2, t = i % DT2;
+            o[t] = mfma32(vf[q][t], p_prev[q], o[t]);
+            s_next = mfma32(kf[i], qf[i], s_next);
+            vf[q][t] = piece_v(off, b, q, t);
+            kf[i] = piece_k(off, b, i);
+        }
         const float mc = m * c;
 #pragma unroll
         for (int e = 0; e < 16; ++e) s_cur[e] = __builtin_amdgcn_exp2f(SCALED ? s_cur[e] : s_cur[e] * c - mc);
@@ -233,30 +235,31 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
             for (int j = 0; j < 8; j += 2) l = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{p_cur[q][j], p_cur[q][j + 1]}, ones, l, false);
         }
         // issue order: one MFMA to every six (SCALED: four) VALU instructions of the softmax; the fragment reads of the next step go into
-        // the registers the MFMAs before them have consumed
+        // the registers that the pair of MFMAs before them has consumed
         constexpr int PER = SCALED ? 4 : 6;
-#pragma unroll
-        for (int i = 0; i < 2 * DT2; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x402, PER, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x100, 2 * DT2, 0);
 #pragma unroll
         for (int i = 0; i < DS; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x402, PER, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x402, PER, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
         }
-        __builtin_amdgcn_sched_group_barrier(0x100, DS, 0);
         __builtin_amdgcn_sched_barrier(0);
+        // the probabilities are made here: their first use is behind the barrier of the tile, and left to itself the compiler moves the softmax of
+        // every second block there, away from the MFMAs that it is to run beside
+        asm volatile("" :: "v"(p_cur[0]), "v"(p_cur[1]), "v"(l));
     };
 
-    for (int i = 0; i < FLASH_STAGES; ++i) stage_next();
-    __builtin_amdgcn_s_waitcnt(0x0f70);                 // vmcnt(0): this wave's pieces are in LDS
-    __syncthreads();
+    constexpr unsigned STAGE = 2 * KBYTES;
+    stage_k(0, 2 * STAGE);
+    stage_v(0, 0); stage_k(1, 0);
+    stage_v(1, STAGE); stage_k(2, STAGE);
+    wait_and_meet<2 * NPT>();                           // all but the last stage are in LDS
 
     f32x16 sA, sB;
     bf16x8 kf[DS], vf[2][DT2], pP[2], pC[2];
-    read_k(0, 0, kf);
+    read_k(2 * STAGE, 0, kf);
 #pragma unroll
     for (int e = 0; e < 16; ++e) sA[e] = 0.f;
 #pragma unroll
@@ -267,22 +270,25 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) { sA[e] -= m; start[e] = -m; }
     }
-    read_k(0, 1, kf);
+    read_k(2 * STAGE, 1, kf);
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
         pP[q] = bf16x8{};                               // "block -1": zero probabilities, any finite V^T
 #pragma unroll
         for (int t = 0; t < DT2; ++t) vf[q][t] = bf16x8{};
     }
-    unsigned off_v = 0, off_k = 2 * KBYTES;             // stages of tile T and of tile T+1
+    unsigned off = 0, off_next2 = 2 * STAGE;            // stages of tile T and of tile T+2
+    wait_and_meet<2 * NPT>();                           // everybody has read K of tile 0 (and with no scalar load under way the loop's waits are for single LDS reads)
     auto tile = [&](auto edge_tag, int T) __attribute__((always_inline)) {
-        step(edge_tag, 2 * T, 0, off_v, off_k, sA, sB, kf, vf, pP, pC);
-        step(edge_tag, 2 * T + 1, 1, off_v, off_k, sB, sA, kf, vf, pC, pP);   // (K reads past the last tile: stale LDS, never used)
-        __builtin_amdgcn_s_waitcnt(0x0f70);             // vmcnt(0): this wave's pieces of tile T+2 have landed
-        __syncthreads();                                // ... everybody's have, and everybody is done reading tile T
-        stage_next();                                   // tile T+3 into the stage of tile T
-        off_v = off_k;
-        off_k = off_k == (FLASH_STAGES - 1) * 2 * KBYTES ? 0 : off_k + 2 * KBYTES;
+        stage_v(T + 2, off_next2);
+        stage_k(T + 3, off_next2);
+        if (active) {
+            step(edge_tag, 2 * T, 0, off, sA, sB, kf, vf, pP, pC);
+            step(edge_tag, 2 * T + 1, 1, off, sB, sA, kf, vf, pC, pP);        // (K past the last tile: that one's again, never used)
+        }
+        off_next2 = off;
+        off = off == (FLASH_STAGES - 1) * STAGE ? 0 : off + STAGE;
+        wait_and_meet<2 * NPT>();                       // stage T+1 has landed, stage T has been read
     };
     // only the last tile of a non-causal pass has keys to mask
     const int plain_tiles = p.causal ? 0 : ntiles - 1;
@@ -293,6 +299,7 @@ void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {
 #pragma unroll
         for (int t = 0; t < DT2; ++t) o[t] = mfma32(vf[q][t], pP[q], o[t]);
 
+    __builtin_amdgcn_s_waitcnt(0x0f70);                 // vmcnt(0): nothing may land in LDS after the workgroup has ended
     l = halves_sum(l);
     const float inv = l > 0.f ? 1.0f / l : 0.f;
     const int row = row0 + n;

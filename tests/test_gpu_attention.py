@@ -168,11 +168,12 @@ def test_vit_flash_attention_with_a_maximum_that_keeps_growing(tokens):
 
 @pytest.mark.parametrize("tokens,heads,ramp,sharp", [(1, 16, 0.0, 1.0), (31, 8, 0.0, 1.0), (32, 1, 0.0, 1.0), (33, 8, 0.0, 1.0), (63, 3, 0.0, 1.0), (64, 8, 0.0, 1.0),
                                                      (65, 3, 0.0, 1.0), (96, 2, 0.0, 1.0), (128, 4, 0.0, 1.0), (129, 16, 0.0, 1.0), (192, 3, 0.0, 1.0), (200, 2, 0.0, 1.0),
-                                                     (257, 5, 0.0, 1.0), (2705, 16, 0.0, 1.0), (96, 3, 128.0, 1.0), (700, 3, 128.0, 1.0), (2705, 3, 128.0, 1.0),
+                                                     (257, 5, 0.0, 1.0), (385, 24, 0.0, 1.0), (449, 8, 0.0, 1.0), (512, 16, 0.0, 1.0), (2705, 16, 0.0, 1.0), (96, 3, 128.0, 1.0), (700, 3, 128.0, 1.0), (2705, 3, 128.0, 1.0),
                                                      (700, 3, -128.0, 1.0), (500, 4, 0.0, 6.0)])
 def test_vit_flash_attention_as_the_forward_runs_it(tokens, heads, ramp, sharp):
     """Queries that carry their scale, S^T started from minus the running maximum: the edges of the instance without, a sequence that ends in its first
-    block, maxima that keep growing, that lie in the first block, and sharp rows."""
+    block, last row blocks (which are dealt behind all others where the heads are a multiple of eight) of one row, of one to four waves, maxima that keep growing, that lie
+    in the first block, and sharp rows."""
     run(capi.ATTN_VIT64_EXP2, tokens, tokens, heads, seed=tokens + 2, ramp=ramp, sharp=sharp)
 
 
