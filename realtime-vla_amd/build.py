@@ -10,10 +10,11 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "librtvla.so")
 HOST_LIB = os.path.join(HERE, "_rtvla_host.so")
-SOURCES = ["gemm.hip", "gemm8.hip", "skinny.hip", "attention.hip", "misc.hip", "dm0.hip", "flash.hip", "flow.hip", "rtvla.hip", "transforms.hip"]
+SOURCES = ["gemm.hip", "gemm8.hip", "skinny.hip", "attention.hip", "prefix_attention.hip", "misc.hip", "dm0.hip", "flash.hip", "flow.hip", "rtvla.hip", "transforms.hip"]
 # bit-exact parity with host arithmetic (Pillow, numpy): no fused multiply-adds in these files
 # flash.hip: MFMA results in ordinary VGPRs (the softmax reads every logit; the accumulator-register form costs a copy each)
 EXTRA = {"transforms.hip": ["-ffp-contract=off"], "flash.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+         "prefix_attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
          "flow.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-std=c++20"]}
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", "-Wno-unused-value",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

@@ -169,17 +169,16 @@ struct AttnP {
     PrefetchP pf_attn;
     int riders;                                  // filled by the launcher: riding workgroups, first in the grid (a multiple of 8)
 };
-// Gemma (HD 256): prefix, one or two row tiles per workgroup (below) / suffix, few rows, one row tile and a key split; DM0 grouped-query
+// Gemma (HD 256): prefix, one or two (csrc/prefix_attention.hip) row tiles per workgroup (below) / suffix, few rows, one row tile and a key split; DM0 grouped-query
 // (HD 128) prefix, causal, and suffix (the ViT attention, HD 64, is launch_flash_attention)
 enum AttnVariant { ATTN_PREFIX = 0, ATTN_SUFFIX = 1, ATTN_GQA128_PREFIX, ATTN_GQA128_SUFFIX };
 
 // Row tiles per workgroup of the prefix passes.  Every workgroup reads all keys, so two halve what the chip reads from L2, and one halves
-// what a workgroup does between two waits.  us with one / two, weights cold, 256 CUs:
-//   Gemma, two or three workgroups of one row tile to a CU.  Up to one of them per CU: 256 tokens (128 tiles) 6.5 / 9.3, 512 (256) 9.3 / 12.4.
-//     More than that: 528 (264) 13.7 / 14.6, 608 (304) 14.4 / 14.3, 656 (328) 16.0 / 16.6, 704 (352) 16.5 / 16.2, 768 (384) 17.6 / 16.6,
-//     968 (484) 22.0 / 20.6, 1024 (512) 23.1 / 20.0.  A third one per CU, where two row tiles are two rounds: 1032 (516) 32.3 / 39.0,
-//     1224 (612) 37.2 / 42.6, 1536 (768) 44.0 / 47.7.  Past that: 1540 (770) 55.2 / 51.1, 2048 (1024) 72.5 / 60.0, 2524 (1262) 109 / 105,
-//     5120 (2560) 415 / 320.
+// what a workgroup does between two waits.  us, weights cold, 256 CUs:
+//   Gemma, one (two or three workgroups to a CU) / two (csrc/prefix_attention.hip, one to a CU): 256 tokens (128 tiles) 6.7 / 7.8, 356 (178) 8.4 / 8.4, 512 (256) 9.7 / 9.6, 528 (264)
+//     14.6 / 10.2, 608 (304) 15.3 / 11.1, 682 (341) 17.4 / 12.6; 768 (384) 17.6 / 13.6, 968 (484) 22.0 / 17.3, 1024 (512) 23.1 / 17.7; 1032 (516) 33.5 / 28.8, 1224 (612) 40.0 /
+//     32.9, 1536 (768) 48.8 / 38.8; 1540 (770) 55.2 / 39.1, 2048 (1024) 72.5 / 52.4.  The lines are where an earlier kernel with two tiles began to pay (528 (264) 14.6, 656 (328) 16.6,
+//     704 (352) 16.2, 1032 (516) 39.0, 1536 (768) 47.7, 1540 (770) 51.1) and are stated as such in tests/test_gpu_attention.py; for this one they would be 180 tiles and no other.
 //   Causal (DM0, 8 K/V heads), where blocks are of unlike length and small ones fill the CUs better: 206 tokens (208 tiles) 5.6 / 7.5,
 //     607 (608) 11.1 / 13.3, 807 (808) 15.1 / 17.2, 848 (848) 15.7 / 16.4, 849 (856) 16.1 / 15.3, 1007 (1008) 19.6 / 19.1, 1407 (1408) 29.3 / 28.7, 1507 (1512) 33.0 / 35.3,
 //     2107 (2112) 53.2 / 47.9, 4603 (4608) 194 / 156.  (Between 1 250 and 1 610 tokens one is better again, by 0 - 7 %; not taken.)
@@ -190,6 +189,10 @@ inline bool attn_two_row_tiles(int variant, int rows, int batch) {
 int launch_mqa_attention(const AttnP& p, int variant, hipStream_t s, int* kernels_launched = nullptr);
 // long sequences on both sides (csrc/flash.hip): 128 query rows per workgroup, K / V^T tiles shared through LDS; hd = 64
 int launch_flash_attention(const AttnP& p, int hd, hipStream_t s);
+// Gemma prefix, two row tiles per workgroup (csrc/prefix_attention.hip): one K/V head whose first keys, up to the valid length, are visible to every row; row-major output,
+// positive scale.  Others go to the general kernel with one row tile.
+bool prefix_attention_takes(const AttnP& p);
+int launch_prefix_attention(const AttnP& p, hipStream_t s);
 // SigLIP attention: q, k fragment-tiled [views*16][256][96], vt tiled [views*16][80][256], out row-major
 void launch_vision_attention(const bf16_t* q, const bf16_t* k, const bf16_t* vt, bf16_t* out, int views, hipStream_t s);
 

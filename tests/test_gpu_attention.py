@@ -126,6 +126,34 @@ def test_gemma_prefix_pass_with_a_valid_length_below_the_allocated_prefix(tokens
     assert (err.norm() / ref[:valid].norm()).item() <= REL_TOL
 
 
+# (1 024 tokens: two row tiles per workgroup)  Blocks of 32 keys over four waves: none, fewer than waves, one each, an even and an odd number of trips, ends inside and at a block
+@pytest.mark.parametrize("valid", [0, 1, 31, 32, 33, 97, 128, 129, 160, 255, 256, 257, 383, 1023])
+def test_prefix_pass_of_many_rows_with_any_number_of_key_blocks(valid):
+    if valid:
+        test_gemma_prefix_pass_with_a_valid_length_below_the_allocated_prefix(1024, valid)
+        return
+    lib, tokens = capi.load(), 1024
+    q, k, v = (torch.randn(tokens, n, 256, device="cuda:0").bfloat16() for n in (8, 1, 1))
+    out, vl = torch.full_like(q, 9.0), torch.zeros(1, dtype=torch.int32, device="cuda:0")
+    need = lib.rtvla_attention_workspace_bytes(capi.ATTN_GEMMA_PREFIX, tokens, tokens, 1)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda:0")
+    assert lib.rtvla_attention(capi.ATTN_GEMMA_PREFIX, _P(q.data_ptr()), _P(k.data_ptr()), _P(v.data_ptr()), _P(out.data_ptr()), tokens, tokens, 1,
+                               ctypes.c_float(0.0625), tokens, _P(vl.data_ptr()), 0, _P(ws.data_ptr()), need, _P(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    assert not out.any()                                    # no key is visible
+
+
+@pytest.mark.parametrize("tokens,ramp,sharp", [(700, 128.0, 1.0), (700, -128.0, 1.0), (771, 0.0, 6.0), (1600, 64.0, 1.0)])
+def test_prefix_pass_of_many_rows_with_growing_maxima_and_sharp_rows(tokens, ramp, sharp):
+    run(capi.ATTN_GEMMA_PREFIX, tokens, tokens, 1, seed=tokens, ramp=ramp, sharp=sharp)
+
+
+# masks and scales that the kernel for many rows does not take
+@pytest.mark.parametrize("prefix,state", [(900, 0), (1000, 3)])
+def test_prefix_pass_of_many_rows_with_other_masks(prefix, state):
+    run(capi.ATTN_GEMMA_PREFIX, 1000, 1000, 1, prefix_alloc=prefix, state_tokens=state, seed=prefix)
+
+
 @pytest.mark.parametrize("tokens,prefix,valid,state", [
     (51, 788, None, 1),      # the headline shape: 839 keys, 7 key splits, state-token row sees itself only
     (51, 270, None, 1),      # 321 keys = 1 mod 32: the last key block holds one key
