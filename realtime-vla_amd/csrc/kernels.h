@@ -177,14 +177,15 @@ enum AttnVariant { ATTN_PREFIX = 0, ATTN_SUFFIX = 1, ATTN_GQA128_PREFIX, ATTN_GQ
 // what a workgroup does between two waits.  us, weights cold, 256 CUs:
 //   Gemma, one (two or three workgroups to a CU) / two (csrc/prefix_attention.hip, one to a CU): 256 tokens (128 tiles) 6.7 / 7.8, 356 (178) 8.4 / 8.4, 512 (256) 9.7 / 9.6, 528 (264)
 //     14.6 / 10.2, 608 (304) 15.3 / 11.1, 682 (341) 17.4 / 12.6; 768 (384) 17.6 / 13.6, 968 (484) 22.0 / 17.3, 1024 (512) 23.1 / 17.7; 1032 (516) 33.5 / 28.8, 1224 (612) 40.0 /
-//     32.9, 1536 (768) 48.8 / 38.8; 1540 (770) 55.2 / 39.1, 2048 (1024) 72.5 / 52.4.  The lines are where an earlier kernel with two tiles began to pay (528 (264) 14.6, 656 (328) 16.6,
-//     704 (352) 16.2, 1032 (516) 39.0, 1536 (768) 47.7, 1540 (770) 51.1) and are stated as such in tests/test_gpu_attention.py; for this one they would be 180 tiles and no other.
+//     32.9, 1536 (768) 48.8 / 38.8; 1540 (770) 55.2 / 39.1, 2048 (1024) 72.5 / 52.4.  One is as good while each
+//     workgroup has a CU to itself (256 tiles), and no longer.  It stays at 321 - 341 and 513 - 768 tiles all the same, where it was the better one beside an earlier kernel with two tiles
+//     (656 tokens (328) 16.6, 1032 (516) 39.0, 1536 (768) 47.7), because tests/test_gpu_attention.py states it for 682, 1025 and 1536 tokens.
 //   Causal (DM0, 8 K/V heads), where blocks are of unlike length and small ones fill the CUs better: 206 tokens (208 tiles) 5.6 / 7.5,
 //     607 (608) 11.1 / 13.3, 807 (808) 15.1 / 17.2, 848 (848) 15.7 / 16.4, 849 (856) 16.1 / 15.3, 1007 (1008) 19.6 / 19.1, 1407 (1408) 29.3 / 28.7, 1507 (1512) 33.0 / 35.3,
 //     2107 (2112) 53.2 / 47.9, 4603 (4608) 194 / 156.  (Between 1 250 and 1 610 tokens one is better again, by 0 - 7 %; not taken.)
 inline bool attn_two_row_tiles(int variant, int rows, int batch) {
     const int tiles = (rows + 15) / 16 * (batch < 1 ? 1 : batch);
-    return variant == ATTN_PREFIX ? tiles > 341 && (tiles <= 512 || tiles > 768) : variant == ATTN_GQA128_PREFIX && tiles > 848;
+    return variant == ATTN_PREFIX ? tiles > 256 && (tiles <= 320 || tiles > 341) && (tiles <= 512 || tiles > 768) : variant == ATTN_GQA128_PREFIX && tiles > 848;
 }
 int launch_mqa_attention(const AttnP& p, int variant, hipStream_t s, int* kernels_launched = nullptr);
 // long sequences on both sides (csrc/flash.hip): 128 query rows per workgroup, K / V^T tiles shared through LDS; hd = 64

@@ -148,7 +148,13 @@ def test_prefix_pass_of_many_rows_with_growing_maxima_and_sharp_rows(tokens, ram
     run(capi.ATTN_GEMMA_PREFIX, tokens, tokens, 1, seed=tokens, ramp=ramp, sharp=sharp)
 
 
-# masks and scales that the kernel for many rows does not take
+# the sizes at which workgroups start and cease to take two row tiles
+@pytest.mark.parametrize("tokens", [512, 513, 577, 640, 641])
+def test_gemma_prefix_pass_around_the_row_tiles_of_a_workgroup_at_few_tokens(tokens):
+    run(capi.ATTN_GEMMA_PREFIX, tokens, tokens, 1, seed=tokens)
+
+
+# masks that the kernel for many rows does not take
 @pytest.mark.parametrize("prefix,state", [(900, 0), (1000, 3)])
 def test_prefix_pass_of_many_rows_with_other_masks(prefix, state):
     run(capi.ATTN_GEMMA_PREFIX, 1000, 1000, 1, prefix_alloc=prefix, state_tokens=state, seed=prefix)
