@@ -447,17 +447,23 @@ void attn_merge_kernel(AttnP p, int nsplit) {
     }
 }
 
+template <int N> RTVLA_DEVICE void wait_loads() { __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4 << 14) | (7 << 4) | (15 << 8)); }      // vmcnt(N)
+
 // SigLIP: per (view, head) Q and K are fragment-tiled [256 tokens][96] (head dim 72 zero padded),
 // V^T is [80][256] in the permuted-key tile layout; out is row-major [views*256][1152].
-// One wave per 16 query rows over all 256 keys; 4 waves per workgroup.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+// One wave per 16 query rows over all 256 keys.  Bound by latency and by the path from the L2 into a CU, 64 bytes a clock: a wave that requests the 88 KB of K and V^T into
+// registers for itself keeps it busy for 0.65 us, four in a workgroup for 2.6 of the 5.9 us that the launch took at any number of views.  WAVES = 1: a workgroup of its own;
+// 2, 4: the waves of a workgroup share the fragments through LDS, requested up front as well, in the order of their use, and awaited 64 keys at a time (launch_vision_attention
+// chooses).  us of a SigLIP layer, before and after, at 1 / 2 / 3 / 4 views: 51.4 / 59.8 / 69.3 / 82.2, 49.4 / 58.6 / 68.7 / 80.2.
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void vision_attn_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ vt,
                         bf16_t* __restrict__ out) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];       // WAVES = 4: per 64 keys 12 fragments of K and 10 of V^T
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, r = lane & 15;
-    const int blk = blockIdx.x;                  // (view*16 + head)*4 + quarter
-    const int quarter = blk & 3, vh = blk >> 2, head = vh & 15, view = vh >> 4;
-    const int mtile = quarter * 4 + w;                             // 16-row tile of this wave inside the view
+    const int blk = xcd_remap(blockIdx.x, gridDim.x) * WAVES + w;  // (view*16 + head)*16 + row tile: a head's on one XCD
+    const int mtile = blk & 15, vh = blk >> 4, head = vh & 15, view = vh >> 4;
     const int row = view * 256 + mtile * 16 + r;                   // query token (global row)
     const float scale = 0.11785113019775792f * 1.4426950408889634f; // 1 / sqrt(72), in the base-2 domain
 
@@ -467,18 +473,26 @@ void vision_attn_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     bf16x8 qf[3];
 #pragma unroll
     for (int kd = 0; kd < 3; ++kd) qf[kd] = *(const bf16x8*)(qb + (size_t)(mtile * 3 + kd) * 512);
-    // all K and V^T fragments of the 256 keys are requested up front (88 x 1 KB loads per wave)
-    bf16x8 kf[16][3];
-    bf16x8 vf[5][8];
+    constexpr int GROUP = 22, KW = 12 / WAVES, PER_WAVE = KW + (10 + WAVES - 1) / WAVES;      // fragments of 64 keys: 12 of K, 10 of V^T; per wave where they are shared
+    bf16x8 frag[WAVES == 1 ? 4 : 1][GROUP];
 #pragma unroll
-    for (int nt = 0; nt < 16; ++nt)
+    for (int kb = 0; kb < 4; ++kb) {                               // all requested up front, in the order of their use
+        auto k_at = [&](int f) __attribute__((always_inline)) { return kb_ + (kb * 12 + f) * 512; };
+        auto v_at = [&](int f) __attribute__((always_inline)) { return vb + ((f >> 1) * 8 + kb * 2 + (f & 1)) * 512; };
+        if constexpr (WAVES == 1) {
 #pragma unroll
-        for (int kd = 0; kd < 3; ++kd) kf[nt][kd] = *(const bf16x8*)(kb_ + (size_t)(nt * 3 + kd) * 512);
+            for (int f = 0; f < GROUP; ++f) frag[kb][f] = *(const bf16x8*)(f < 12 ? k_at(f) : v_at(f - 12));
+        } else {
+            typedef const __attribute__((address_space(1))) void* gptr_t;
+            typedef __attribute__((address_space(3))) void* lptr_t;
 #pragma unroll
-    for (int dt = 0; dt < 5; ++dt)
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk) vf[dt][kk] = *(const bf16x8*)(vb + (size_t)(dt * 8 + kk) * 512);
-    __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < PER_WAVE; ++i) {                   // (the last fragment twice, so that every wave has as many on the way)
+                const int f = i < KW ? w + WAVES * i : min(w + WAVES * (i - KW), 9);
+                __builtin_amdgcn_global_load_lds((gptr_t)(i < KW ? k_at(f) : v_at(f)), (lptr_t)(smem + (kb * GROUP + (i < KW ? f : 12 + f)) * 1024), 16, 0, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
 
     f32x4 o[5];
 #pragma unroll
@@ -486,12 +500,25 @@ void vision_attn_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     float mrun = NEG_BIG, lrun = 0.f;
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
+        if constexpr (WAVES > 1) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (kb == 0) wait_loads<3 * PER_WAVE>();               // (all of this wave's requests but those for the keys that follow)
+            else if (kb == 1) wait_loads<2 * PER_WAVE>();
+            else if (kb == 2) wait_loads<PER_WAVE>();
+            else wait_loads<0>();
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int f = 0; f < GROUP; ++f) frag[0][f] = *(const bf16x8*)(smem + (kb * GROUP + f) * 1024 + lane * 16);
+        }
+        const bf16x8 (&kv)[GROUP] = frag[WAVES == 1 ? kb : 0];
         f32x4 st[4];
 #pragma unroll
         for (int nt = 0; nt < 4; ++nt) {
             st[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int kd = 0; kd < 3; ++kd) st[nt] = mfma16(kf[kb * 4 + nt][kd], qf[kd], st[nt]);
+            for (int kd = 0; kd < 3; ++kd) st[nt] = mfma16(kv[nt * 3 + kd], qf[kd], st[nt]);
         }
         float mx = NEG_BIG;
 #pragma unroll
@@ -520,7 +547,7 @@ void vision_attn_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
 #pragma unroll
         for (int dt = 0; dt < 5; ++dt) {
 #pragma unroll
-            for (int kk = 0; kk < 2; ++kk) o[dt] = mfma16(vf[dt][kb * 2 + kk], pb[kk], o[dt]);
+            for (int kk = 0; kk < 2; ++kk) o[dt] = mfma16(kv[12 + dt * 2 + kk], pb[kk], o[dt]);
         }
     }
     const float inv = 1.0f / lrun;
@@ -618,6 +645,21 @@ int launch_mqa_attention(const AttnP& p0, int variant, hipStream_t s, int* nk) {
     return 2;
 }
 
-void launch_vision_attention(const bf16_t* q, const bf16_t* k, const bf16_t* vt, bf16_t* out, int views, hipStream_t s) {
-    hipLaunchKernelGGL(vision_attn_kernel, dim3(views * 16 * 4), dim3(256), 0, s, q, k, vt, out);
+// One view: 256 waves, one to a CU, each of which requests all of K and V^T.  More of them on a CU queue for its path to the L2, so they share the fragments through
+// LDS, two to a workgroup at two views (256 workgroups), four from three on.  us of a launch in its layer, by waves of a workgroup: 1 view 3.9 with one wave; 2 views 4.8, 4.5
+// with two, 4.9 with four; 3 views 5.6, 5.05 with four; 4 views 6.55, 5.15 with four (four waves that share nothing: 5.8, 5.95, 6.05, 6.3).
+int launch_vision_attention(const bf16_t* q, const bf16_t* k, const bf16_t* vt, bf16_t* out, int views, hipStream_t s) {
+    constexpr size_t smem = 88 * 1024;
+    if (views == 1) {
+        hipLaunchKernelGGL(vision_attn_kernel<1>, dim3(views * 16 * 16), dim3(64), 0, s, q, k, vt, out);
+    } else if (views == 2) {
+        static std::atomic<uint64_t> done{0};
+        if (int rc = ensure_dynamic_lds((const void*)vision_attn_kernel<2>, smem, done)) return rc;
+        hipLaunchKernelGGL(vision_attn_kernel<2>, dim3(views * 16 * 8), dim3(128), smem, s, q, k, vt, out);
+    } else {
+        static std::atomic<uint64_t> done{0};
+        if (int rc = ensure_dynamic_lds((const void*)vision_attn_kernel<4>, smem, done)) return rc;
+        hipLaunchKernelGGL(vision_attn_kernel<4>, dim3(views * 16 * 4), dim3(256), smem, s, q, k, vt, out);
+    }
+    return hipGetLastError() == hipSuccess ? 0 : 5;
 }

@@ -195,7 +195,7 @@ int launch_flash_attention(const AttnP& p, int hd, hipStream_t s);
 bool prefix_attention_takes(const AttnP& p);
 int launch_prefix_attention(const AttnP& p, hipStream_t s);
 // SigLIP attention: q, k fragment-tiled [views*16][256][96], vt tiled [views*16][80][256], out row-major
-void launch_vision_attention(const bf16_t* q, const bf16_t* k, const bf16_t* vt, bf16_t* out, int views, hipStream_t s);
+int launch_vision_attention(const bf16_t* q, const bf16_t* k, const bf16_t* vt, bf16_t* out, int views, hipStream_t s);
 
 // ----- the action expert's flow loop as one resident kernel (csrc/flow.hip) ------------------------------------
 enum FlowModel { FLOW_PI0 = 0, FLOW_PI05, FLOW_DM0 };

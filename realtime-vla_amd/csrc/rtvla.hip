@@ -648,7 +648,7 @@ struct Sched {
         const int S_v = c->S_v, V = d.vision_layers;
         GemmP e{}; e.bias = c->W("vision_attn_qkv_b", 3456, i); e.q = c->B("vision_Q"); e.k = c->B("vision_K"); e.vt = c->B("vision_Vt");
         gemm(c->B("vision_x_norm"), 1152, S_v, S_v, c->TW("t_vision_attn_qkv_w", i), nullptr, 1152, 3456, EPI_VIS_QKV, e, "vision qkv");
-        if (c->want("vision attn")) { launch_vision_attention(c->B("vision_Q"), c->B("vision_K"), c->B("vision_Vt"), c->B("vision_attn"), d.num_views, s); c->note(0, "vision attn"); }
+        if (c->want("vision attn")) { c->note(launch_vision_attention(c->B("vision_Q"), c->B("vision_K"), c->B("vision_Vt"), c->B("vision_attn"), d.num_views, s), "vision attn"); }
         gemm(c->B("vision_attn"), 1152, S_v, S_v, c->TW("t_vision_attn_o_w", i), nullptr, 1152, 1152, EPI_PARTIAL, GemmP{}, "vision o");
         reduce(S_v, 1152, c->W("vision_attn_o_b", 1152, i), c->B("vision_x"), 1152, c->B("vision_x"), 1152, c->B("vision_x_norm"), 1152,
                NORM_LAYER, c->W("vision_pre_ffn_norm_w", 1152, i), c->W("vision_pre_ffn_norm_b", 1152, i), 1e-5f, last_split, "vision o reduce");
@@ -1817,7 +1817,7 @@ int rtvla_attention(int kind, const void* q, const void* k, const void* v, void*
                               pl.keys_pad, kind == RTVLA_ATTN_SIGLIP ? 256 : 0, s);
     int rc = 0;
     if (kind == RTVLA_ATTN_SIGLIP) {
-        launch_vision_attention(qt, kt, vtt, (bf16_t*)out, tokens / 256, s);
+        rc = launch_vision_attention(qt, kt, vtt, (bf16_t*)out, tokens / 256, s);
     } else {
         AttnP a{};
         a.q = qt; a.k = kt; a.vt = vtt; a.ldvt = pl.keys_pad;

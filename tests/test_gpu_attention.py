@@ -225,6 +225,13 @@ def test_siglip_attention_keeps_views_apart(views):
     run(capi.ATTN_SIGLIP, 256 * views, 256 * views, 16, seed=views)
 
 
+@pytest.mark.parametrize("views", [1, 2, 3, 4])
+def test_siglip_attention_with_maxima_that_grow_along_the_keys(views):
+    """One, two and four waves to a workgroup: sharp logits, and keys whose logits climb, so that every block of 64 rescales what the ones before it left."""
+    run(capi.ATTN_SIGLIP, 256 * views, 256 * views, 16, seed=40 + views, sharp=4.0)
+    run(capi.ATTN_SIGLIP, 256 * views, 256 * views, 16, seed=50 + views, ramp=25.0 * views)
+
+
 def test_peaked_softmax_rows_survive_the_running_maximum():
     """Large logits (|q| scaled up): one key dominates each row, the running-maximum rescale path is exercised in every kernel."""
     run(capi.ATTN_GEMMA_PREFIX, 300, 300, 1, seed=5, sharp=6.0)
