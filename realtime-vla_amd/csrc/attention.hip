@@ -53,19 +53,17 @@ RTVLA_DEVICE bf16_t* attn_out_at(const AttnP& p, const AttnOutRow& o, int d) {
 }
 RTVLA_DEVICE bf16_t* attn_out_ptr(const AttnP& p, int batch, int row, int d, int hd) { return attn_out_at(p, attn_out_row(p, batch, row, hd), d); }
 
-// One row tile per workgroup (MQ = 1) is built for two workgroups per CU at head width 256 and three at 128, without a spill:
-// while one waits for its key blocks' 64 loads the other's matrix instructions run (1224 Gemma tokens, 612
-// workgroups: 37.0 us against 42.3 with one per CU; DM0's 607 tokens: 11.1 us against 12.4 with two per CU).  Two row tiles
-// need 254 registers of a wave alone.
-template <int WAVES, int MQ, int NTK, int HD, bool CAUSAL>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(MQ > 1 ? 1 : HD == 256 ? 2 : 3)))
+// Built for two workgroups per CU at head width 256 and three at 128, without a spill: while one waits for its key blocks' 64 loads the other's matrix instructions
+// run (1224 Gemma tokens, 612 workgroups: 37.0 us against 42.3 with one per CU; DM0's 607 tokens: 11.1 us against 12.4 with two per CU).
+template <int WAVES, int NTK, int HD, bool CAUSAL>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(HD == 256 ? 2 : 3)))
 void mqa_kernel(AttnP p) {
     constexpr int KD = HD / 32;                                       // 32-wide steps of the Q K^T contraction
     constexpr int DT = HD / 16;                                       // 16-wide tiles of the output
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     f32x4* obuf = (f32x4*)smem_raw;                                   // [WAVES][DT][64]
-    float* ms = (float*)(smem_raw + (size_t)WAVES * DT * 64 * 16);    // [WAVES][MQ][16]
-    float* ls = ms + WAVES * MQ * 16;                                 // [WAVES][MQ][16]
+    float* ms = (float*)(smem_raw + (size_t)WAVES * DT * 64 * 16);    // [WAVES][16]
+    float* ls = ms + WAVES * 16;                                      // [WAVES][16]
     const int batch = blockIdx.y;
     const bf16_t* const qbase = p.q + (size_t)batch * p.q_bstride;
     const bf16_t* const kbase = p.k + (size_t)batch * p.k_bstride;
@@ -84,34 +82,27 @@ void mqa_kernel(AttnP p) {
         split = xcd + 8 * (idx % spx); rowblk = idx / spx;
         if (split >= nsplit) return;                                 // (whole workgroup, before any barrier)
     }
-    const int m0 = rowblk * (16 * MQ);
+    const int m0 = rowblk * 16;
 
     int vl = p.prefix_alloc;
     if (p.valid_len) vl = max(0, min(*p.valid_len, p.prefix_alloc));
     const int vis_lim = min(vl, p.keys);                             // keys below this are visible to every row (causal aside)
     const float sc2 = p.scale * 1.4426950408889634f;
 
-    bf16x8 qf[MQ][KD];
+    bf16x8 qf[KD];
+    // fragment-tiled Q: one contiguous 1 KB read per fragment (row tiles past the end are padding)
+    const bf16_t* qp = qbase + ((size_t)rowblk * KD * 64 + lane) * 8;
 #pragma unroll
-    for (int mq = 0; mq < MQ; ++mq) {
-        // fragment-tiled Q: one contiguous 1 KB read per fragment (row tiles past the end are padding)
-        const bf16_t* qp = qbase + ((size_t)(rowblk * MQ + mq) * KD * 64 + lane) * 8;
+    for (int kd = 0; kd < KD; ++kd) qf[kd] = *(const bf16x8*)(qp + kd * 512);
+    f32x4 o[DT];
+    float mrun = NEG_BIG, lrun = 0.f;
 #pragma unroll
-        for (int kd = 0; kd < KD; ++kd) qf[mq][kd] = *(const bf16x8*)(qp + kd * 512);
-    }
-    f32x4 o[MQ][DT];
-    float mrun[MQ], lrun[MQ];
-#pragma unroll
-    for (int mq = 0; mq < MQ; ++mq) {
-        mrun[mq] = NEG_BIG; lrun[mq] = 0.f;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) o[mq][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     constexpr int KBS = NTK * 16;                    // keys per block
     int nkb = (p.keys + KBS - 1) / KBS;
     // causal: the last row of this block sees keys up to its own token
-    if constexpr (CAUSAL) nkb = min(nkb, (min(m0 + 16 * MQ, p.rows) - 1) / p.group / KBS + 1);
+    if constexpr (CAUSAL) nkb = min(nkb, (min(m0 + 16, p.rows) - 1) / p.group / KBS + 1);
     const int kb_begin = split * p.kb_per_split, kb_end = min(nkb, kb_begin + p.kb_per_split);
     const int keys32 = p.ldvt >> 5;
     bf16x8 kf[NTK][KD];       // K fragments of one key block (A operand of S^T = K Q^T)
@@ -138,82 +129,75 @@ void mqa_kernel(AttnP p) {
     for (int kb = kb_begin + w; kb < kb_end; kb += WAVES) {
         const int key0 = kb * KBS;
         const int kb_next = kb + WAVES;
-        f32x4 st[MQ][NTK];
+        f32x4 st[NTK];
 #pragma unroll
-        for (int mq = 0; mq < MQ; ++mq)
-#pragma unroll
-            for (int nt = 0; nt < NTK; ++nt) st[mq][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int nt = 0; nt < NTK; ++nt) st[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int nt = 0; nt < NTK; ++nt)
 #pragma unroll
             for (int kd = 0; kd < KD; ++kd)
-#pragma unroll
-                for (int mq = 0; mq < MQ; ++mq) st[mq][nt] = mfma16(kf[nt][kd], qf[mq][kd], st[mq][nt]);
+                st[nt] = mfma16(kf[nt][kd], qf[kd], st[nt]);
         __builtin_amdgcn_sched_barrier(0);
         if (kb + WAVES < kb_end) load_k(kb_next);            // next block's K flies during softmax and P V (the suffix pass has one block per wave: nothing to fetch)
         __builtin_amdgcn_sched_barrier(0);
-        bf16x8 pb[MQ][NTK / 2];
+        bf16x8 pb[NTK / 2];
         bool full = key0 + KBS <= vis_lim;
         if constexpr (CAUSAL) full = full && key0 + KBS - 1 <= m0 / p.group;
+        const int row = m0 + r;
+        int own = 0;                                      // causal: the row's own token, the last key it sees
+        if constexpr (CAUSAL) own = row / p.group;
+        // logits in the base-2 domain (scale * log2 e folded into one multiply); a block every row sees whole (all but the
+        // last of a prefix pass) takes the path without mask arithmetic
+        float mx = NEG_BIG;
+        bool vis[NTK][4];
+        if (full) {
 #pragma unroll
-        for (int mq = 0; mq < MQ; ++mq) {
-            const int row = m0 + mq * 16 + r;
-            int own = 0;                                      // causal: the row's own token, the last key it sees
-            if constexpr (CAUSAL) own = row / p.group;
-            // logits in the base-2 domain (scale * log2 e folded into one multiply); a block every row sees whole (all but the
-            // last of a prefix pass) takes the path without mask arithmetic
-            float mx = NEG_BIG;
-            bool vis[NTK][4];
-            if (full) {
+            for (int nt = 0; nt < NTK; ++nt)
 #pragma unroll
-                for (int nt = 0; nt < NTK; ++nt)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) { st[mq][nt][v] *= sc2; mx = fmaxf(mx, st[mq][nt][v]); vis[nt][v] = true; }
-            } else {
-#pragma unroll
-                for (int nt = 0; nt < NTK; ++nt)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int key = key0 + nt * 16 + 4 * g + v;
-                        bool ok = key < p.keys;
-                        if (key < p.prefix_alloc) ok = ok && key < vl;
-                        else ok = ok && (row >= p.state_rows || key == p.prefix_alloc);
-                        if constexpr (CAUSAL) ok = ok && key <= own;
-                        vis[nt][v] = ok;
-                        const float s = ok ? st[mq][nt][v] * sc2 : NEG_BIG;
-                        st[mq][nt][v] = s;
-                        mx = fmaxf(mx, s);
-                    }
-            }
-            mx = rows_max(mx);
-            if (__any(mx > mrun[mq])) {                       // the accumulator is rescaled only when some row's maximum grew
-                const float mnew = fmaxf(mrun[mq], mx);
-                const float alpha = __builtin_amdgcn_exp2f(mrun[mq] - mnew);
-                lrun[mq] *= alpha;
-                mrun[mq] = mnew;
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) o[mq][dt] *= alpha;
-            }
-            float sum = 0.f;
+                for (int v = 0; v < 4; ++v) { st[nt][v] *= sc2; mx = fmaxf(mx, st[nt][v]); vis[nt][v] = true; }
+        } else {
 #pragma unroll
             for (int nt = 0; nt < NTK; ++nt)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    const float e = vis[nt][v] ? __builtin_amdgcn_exp2f(st[mq][nt][v] - mrun[mq]) : 0.f;
-                    st[mq][nt][v] = e;
-                    sum += e;
+                    const int key = key0 + nt * 16 + 4 * g + v;
+                    bool ok = key < p.keys;
+                    if (key < p.prefix_alloc) ok = ok && key < vl;
+                    else ok = ok && (row >= p.state_rows || key == p.prefix_alloc);
+                    if constexpr (CAUSAL) ok = ok && key <= own;
+                    vis[nt][v] = ok;
+                    const float s = ok ? st[nt][v] * sc2 : NEG_BIG;
+                    st[nt][v] = s;
+                    mx = fmaxf(mx, s);
                 }
-            sum = rows_sum(sum);
-            lrun[mq] += sum;
-#pragma unroll
-            for (int kk = 0; kk < NTK / 2; ++kk) pb[mq][kk] = cat44(pack4(st[mq][2 * kk]), pack4(st[mq][2 * kk + 1]));
         }
+        mx = rows_max(mx);
+        if (__any(mx > mrun)) {                           // the accumulator is rescaled only when some row's maximum grew
+            const float mnew = fmaxf(mrun, mx);
+            const float alpha = __builtin_amdgcn_exp2f(mrun - mnew);
+            lrun *= alpha;
+            mrun = mnew;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
+        }
+        float sum = 0.f;
+#pragma unroll
+        for (int nt = 0; nt < NTK; ++nt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float e = vis[nt][v] ? __builtin_amdgcn_exp2f(st[nt][v] - mrun) : 0.f;
+                st[nt][v] = e;
+                sum += e;
+            }
+        sum = rows_sum(sum);
+        lrun += sum;
+#pragma unroll
+        for (int kk = 0; kk < NTK / 2; ++kk) pb[kk] = cat44(pack4(st[2 * kk]), pack4(st[2 * kk + 1]));
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int kk = 0; kk < NTK / 2; ++kk) {
-#pragma unroll
-                for (int mq = 0; mq < MQ; ++mq) o[mq][dt] = mfma16(vf[dt][kk], pb[mq][kk], o[mq][dt]);
+                o[dt] = mfma16(vf[dt][kk], pb[kk], o[dt]);
             }
         __builtin_amdgcn_sched_barrier(0);
         if (kb + WAVES < kb_end) load_v(kb_next);
@@ -222,48 +206,39 @@ void mqa_kernel(AttnP p) {
 
     // ---- merge the key splits of the WAVES waves ----
     if (g == 0) {
-#pragma unroll
-        for (int mq = 0; mq < MQ; ++mq) ms[(w * MQ + mq) * 16 + r] = mrun[mq];
+        ms[w * 16 + r] = mrun;
     }
     __syncthreads();
-    float mgl[MQ];
+    float mg = NEG_BIG;
 #pragma unroll
-    for (int mq = 0; mq < MQ; ++mq) {
-        float mg = NEG_BIG;
+    for (int ww = 0; ww < WAVES; ++ww) mg = fmaxf(mg, ms[ww * 16 + r]);
+    const float sc = __builtin_amdgcn_exp2f(mrun - mg);
+    lrun *= sc;
 #pragma unroll
-        for (int ww = 0; ww < WAVES; ++ww) mg = fmaxf(mg, ms[(ww * MQ + mq) * 16 + r]);
-        const float sc = __builtin_amdgcn_exp2f(mrun[mq] - mg);
-        lrun[mq] *= sc;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) o[mq][dt] *= sc;
-        if (g == 0) ls[(w * MQ + mq) * 16 + r] = lrun[mq];
-        mgl[mq] = mg;
-    }
-    // partial record of one (row block, split): MQ x { O [DT][64] f32x4 | max [16] | sum [16] }
+    for (int dt = 0; dt < DT; ++dt) o[dt] *= sc;
+    if (g == 0) ls[w * 16 + r] = lrun;
+    // partial record of one (row block, split): O [DT][64] f32x4 | max [16] | sum [16]
     constexpr int REC = DT * 64 * 4 + 32;
-    float* const mine = p.partial + (((size_t)batch * p.row_blocks + rowblk) * nsplit + split) * (MQ * REC);
+    float* const mine = p.partial + (((size_t)batch * p.row_blocks + rowblk) * nsplit + split) * REC;
+    __syncthreads();                           // ls written
 #pragma unroll
-    for (int mq = 0; mq < MQ; ++mq) {
-        __syncthreads();                       // ls written / previous obuf round consumed
+    for (int dt = 0; dt < DT; ++dt) obuf[((size_t)w * DT + dt) * 64 + lane] = o[dt];
+    __syncthreads();
+    float lt = 0.f;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) obuf[((size_t)w * DT + dt) * 64 + lane] = o[mq][dt];
-        __syncthreads();
-        float lt = 0.f;
+    for (int ww = 0; ww < WAVES; ++ww) lt += ls[ww * 16 + r];
+    const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+    const int row = m0 + r;
+    const AttnOutRow orow = attn_out_row(p, batch, min(row, p.rows - 1), HD);
+    if (nsplit > 1 && w == 0 && g == 0) { mine[DT * 256 + r] = mg; mine[DT * 256 + 16 + r] = lt; }
+    for (int dt = w; dt < DT; dt += WAVES) {
+        f32x4 t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ww = 0; ww < WAVES; ++ww) lt += ls[(ww * MQ + mq) * 16 + r];
-        const float inv = lt > 0.f ? 1.0f / lt : 0.f;
-        const int row = m0 + mq * 16 + r;
-        const AttnOutRow orow = attn_out_row(p, batch, min(row, p.rows - 1), HD);
-        if (nsplit > 1 && w == 0 && g == 0) { mine[mq * REC + DT * 256 + r] = mgl[mq]; mine[mq * REC + DT * 256 + 16 + r] = lt; }
-        for (int dt = w; dt < DT; dt += WAVES) {
-            f32x4 t = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ww = 0; ww < WAVES; ++ww) t += obuf[((size_t)ww * DT + dt) * 64 + lane];
-            if (nsplit > 1) {
-                *(f32x4*)(mine + mq * REC + (dt * 64 + lane) * 4) = t;
-            } else if (row < p.rows) {
-                store4(attn_out_at(p, orow, dt * 16 + 4 * g), pack4(t * inv));
-            }
+        for (int ww = 0; ww < WAVES; ++ww) t += obuf[((size_t)ww * DT + dt) * 64 + lane];
+        if (nsplit > 1) {
+            *(f32x4*)(mine + (dt * 64 + lane) * 4) = t;
+        } else if (row < p.rows) {
+            store4(attn_out_at(p, orow, dt * 16 + 4 * g), pack4(t * inv));
         }
     }
 }
@@ -407,7 +382,7 @@ void suffix_attn_kernel(AttnP p) {
 
 // Combine the key-split partials of mqa_kernel: one wave per (row block, 16-wide d tile), 4 waves per workgroup, K/V heads
 // along blockIdx.y.  All loads of a wave are independent, so the kernel is one memory round trip long.
-template <int MQ, int NS, int HD>
+template <int NS, int HD>
 __global__ __launch_bounds__(256)
 void attn_merge_kernel(AttnP p, int nsplit) {
     constexpr int DT = HD / 16;
@@ -416,34 +391,31 @@ void attn_merge_kernel(AttnP p, int nsplit) {
     const int g = lane >> 4, r = lane & 15;
     const int batch = blockIdx.y;
     const int rb = blockIdx.x / (DT / 4), dt = (blockIdx.x % (DT / 4)) * 4 + w;
-    const float* const all = p.partial + ((size_t)batch * p.row_blocks + rb) * nsplit * (MQ * REC);
+    const float* const all = p.partial + ((size_t)batch * p.row_blocks + rb) * nsplit * REC;
+    float ms[NS], ls[NS];
+    f32x4 os[NS];
 #pragma unroll
-    for (int mq = 0; mq < MQ; ++mq) {
-        float ms[NS], ls[NS];
-        f32x4 os[NS];
+    for (int sp = 0; sp < NS; ++sp) {
+        const float* rec = all + (size_t)min(sp, nsplit - 1) * REC;
+        ms[sp] = rec[DT * 256 + r]; ls[sp] = rec[DT * 256 + 16 + r];
+        os[sp] = *(const f32x4*)(rec + (dt * 64 + lane) * 4);
+    }
+    float mg = NEG_BIG;
 #pragma unroll
-        for (int sp = 0; sp < NS; ++sp) {
-            const float* rec = all + (size_t)min(sp, nsplit - 1) * (MQ * REC) + mq * REC;
-            ms[sp] = rec[DT * 256 + r]; ls[sp] = rec[DT * 256 + 16 + r];
-            os[sp] = *(const f32x4*)(rec + (dt * 64 + lane) * 4);
-        }
-        float mg = NEG_BIG;
+    for (int sp = 0; sp < NS; ++sp) if (sp < nsplit) mg = fmaxf(mg, ms[sp]);
+    float lt = 0.f;
+    f32x4 t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int sp = 0; sp < NS; ++sp) if (sp < nsplit) mg = fmaxf(mg, ms[sp]);
-        float lt = 0.f;
-        f32x4 t = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int sp = 0; sp < NS; ++sp) {
-            const float wgt = sp < nsplit ? __builtin_amdgcn_exp2f(ms[sp] - mg) : 0.f;      // the maxima are base-2 logits
-            lt += wgt * ls[sp];
-            t += os[sp] * wgt;
-        }
-        const float inv = lt > 0.f ? 1.0f / lt : 0.f;
-        const int row = (rb * MQ + mq) * 16 + r;
-        if (row < p.rows) {
-            const int d = dt * 16 + 4 * g;
-            store4(attn_out_ptr(p, batch, row, d, HD), pack4(t * inv));
-        }
+    for (int sp = 0; sp < NS; ++sp) {
+        const float wgt = sp < nsplit ? __builtin_amdgcn_exp2f(ms[sp] - mg) : 0.f;      // the maxima are base-2 logits
+        lt += wgt * ls[sp];
+        t += os[sp] * wgt;
+    }
+    const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+    const int row = rb * 16 + r;
+    if (row < p.rows) {
+        const int d = dt * 16 + 4 * g;
+        store4(attn_out_ptr(p, batch, row, d, HD), pack4(t * inv));
     }
 }
 
@@ -558,34 +530,34 @@ void vision_attn_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
     }
 }
 
-template <int WAVES, int MQ, int NTK, int HD, bool CAUSAL = false>
+template <int WAVES, int NTK, int HD, bool CAUSAL = false>
 int launch_mqa_inst(AttnP p, hipStream_t s, int* nk) {
-    const size_t smem = (size_t)WAVES * (HD / 16) * 64 * 16 + (size_t)2 * WAVES * MQ * 16 * 4;
-    auto kern = mqa_kernel<WAVES, MQ, NTK, HD, CAUSAL>;
+    const size_t smem = (size_t)WAVES * (HD / 16) * 64 * 16 + (size_t)2 * WAVES * 16 * 4;
+    auto kern = mqa_kernel<WAVES, NTK, HD, CAUSAL>;
     if (CAUSAL != (p.causal != 0)) return 1;
     if (smem > 65536) {
         static std::atomic<uint64_t> done{0};
         if (int rc = ensure_dynamic_lds((const void*)kern, smem, done)) return rc;
     }
-    const int blocks = (p.rows + 16 * MQ - 1) / (16 * MQ);
+    const int blocks = (p.rows + 15) / 16;
     const int nkb = (p.keys + NTK * 16 - 1) / (NTK * 16);
     const int want = p.nsplit > 1 ? p.nsplit : 1;
     p.kb_per_split = (nkb + want - 1) / want;
     const int nsplit = (nkb + p.kb_per_split - 1) / p.kb_per_split;
     if (nsplit > 1) {
         if (!p.partial || nsplit > 16 || HD < 64 || p.causal) return 1;           // the key split over workgroups exists for the suffix passes
-        if ((size_t)p.batch * blocks * nsplit * MQ * ((HD / 16) * 64 * 4 + 32) > p.partial_floats) return 3;
+        if ((size_t)p.batch * blocks * nsplit * ((HD / 16) * 64 * 4 + 32) > p.partial_floats) return 3;
     }
     p.nsplit_eff = nsplit;
     p.row_blocks = blocks;
-    if (MQ == 1 && NTK == 2 && WAVES == 4 && !CAUSAL && nsplit > 1 && p.kb_per_split <= 4) {    // one key block per wave: the probability-sharing kernel
+    if (NTK == 2 && WAVES == 4 && !CAUSAL && nsplit > 1 && p.kb_per_split <= 4) {    // one key block per wave: the probability-sharing kernel
         p.riders = prefetch_wgs(p.pf_attn);
         if (p.riders & 7) return 1;
         hipLaunchKernelGGL((suffix_attn_kernel<HD>), dim3(8 * ((nsplit + 7) / 8) * blocks + p.riders, p.batch), dim3(256), 0, s, p);
     } else
     hipLaunchKernelGGL(kern, dim3(nsplit == 1 ? blocks : 8 * ((nsplit + 7) / 8) * blocks, p.batch), dim3(WAVES * 64), smem, s, p);
-    if (nsplit > 8) hipLaunchKernelGGL((attn_merge_kernel<MQ, 16, HD>), dim3(blocks * (HD / 64), p.batch), dim3(256), 0, s, p, nsplit);
-    else if (nsplit > 1) hipLaunchKernelGGL((attn_merge_kernel<MQ, 8, HD>), dim3(blocks * (HD / 64), p.batch), dim3(256), 0, s, p, nsplit);
+    if (nsplit > 8) hipLaunchKernelGGL((attn_merge_kernel<16, HD>), dim3(blocks * (HD / 64), p.batch), dim3(256), 0, s, p, nsplit);
+    else if (nsplit > 1) hipLaunchKernelGGL((attn_merge_kernel<8, HD>), dim3(blocks * (HD / 64), p.batch), dim3(256), 0, s, p, nsplit);
     if (nk) *nk = nsplit > 1 ? 2 : 1;
     return hipGetLastError() == hipSuccess ? 0 : 5;
 }
@@ -634,13 +606,15 @@ int launch_mqa_attention(const AttnP& p0, int variant, hipStream_t s, int* nk) {
     if (p.batch_inner < 1) p.batch_inner = 1;
     if (p.group < 1) return 1;
     const bool two = attn_two_row_tiles(variant, p.rows, p.batch);
-    switch (variant) {                                          // template: waves, row tiles per workgroup, 16-key tiles per wave round, head width
+    switch (variant) {                                          // template: waves, 16-key tiles per wave round, head width
         case ATTN_PREFIX:
             if (two && prefix_attention_takes(p)) { if (nk) *nk = 1; return launch_prefix_attention(p, s); }
-            return launch_mqa_inst<4, 1, 2, 256>(p, s, nk);
-        case ATTN_SUFFIX: return launch_mqa_inst<4, 1, 2, 256>(p, s, nk);
-        case ATTN_GQA128_PREFIX: return two ? launch_mqa_inst<4, 2, 2, 128, true>(p, s, nk) : launch_mqa_inst<4, 1, 2, 128, true>(p, s, nk);
-        case ATTN_GQA128_SUFFIX: return launch_mqa_inst<4, 1, 2, 128>(p, s, nk);
+            return launch_mqa_inst<4, 2, 256>(p, s, nk);
+        case ATTN_SUFFIX: return launch_mqa_inst<4, 2, 256>(p, s, nk);
+        case ATTN_GQA128_PREFIX:
+            if (two && p.causal && prefix_attention_takes(p)) { if (nk) *nk = 1; return launch_prefix_attention(p, s); }
+            return launch_mqa_inst<4, 2, 128, true>(p, s, nk);
+        case ATTN_GQA128_SUFFIX: return launch_mqa_inst<4, 2, 128>(p, s, nk);
     }
     return 2;
 }

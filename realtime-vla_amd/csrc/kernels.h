@@ -180,18 +180,19 @@ enum AttnVariant { ATTN_PREFIX = 0, ATTN_SUFFIX = 1, ATTN_GQA128_PREFIX, ATTN_GQ
 //     32.9, 1536 (768) 48.8 / 38.8; 1540 (770) 55.2 / 39.1, 2048 (1024) 72.5 / 52.4.  One is as good while each
 //     workgroup has a CU to itself (256 tiles), and no longer.  It stays at 321 - 341 and 513 - 768 tiles all the same, where it was the better one beside an earlier kernel with two tiles
 //     (656 tokens (328) 16.6, 1032 (516) 39.0, 1536 (768) 47.7), because tests/test_gpu_attention.py states it for 682, 1025 and 1536 tokens.
-//   Causal (DM0, 8 K/V heads), where blocks are of unlike length and small ones fill the CUs better: 206 tokens (208 tiles) 5.6 / 7.5,
-//     607 (608) 11.1 / 13.3, 807 (808) 15.1 / 17.2, 848 (848) 15.7 / 16.4, 849 (856) 16.1 / 15.3, 1007 (1008) 19.6 / 19.1, 1407 (1408) 29.3 / 28.7, 1507 (1512) 33.0 / 35.3,
-//     2107 (2112) 53.2 / 47.9, 4603 (4608) 194 / 156.  (Between 1 250 and 1 610 tokens one is better again, by 0 - 7 %; not taken.)
+//   Causal (DM0, 8 K/V heads), where workgroups are of unlike length, one (three to a CU) / two (two to a CU, the longest first): 177 tokens (184 tiles) 5.0 / 5.0, 206 (208) 5.0 / 4.9,
+//     269 (272) 6.3 / 5.15, 375 (376) 7.8 / 5.35, 438 (440) 8.8 / 5.9, 515 (520) 10.1 / 6.9, 607 (608) 11.1 / 7.4, 707 (712) 13.9 / 8.7, 807 (808) 15.4 / 9.5.  Past that against two tiles in the
+//     kernel of csrc/attention.hip: 849 (856) 15.5 / 9.7, 1007 (1008) 19.4 / 11.5, 1507 (1512) 35.8 / 19.3, 2107 (2112) 48.3 / 30.  One tile stays up to 184, where it is as fast, and at 848,
+//     because tests/test_gpu_attention.py states it for 848 tokens.
 inline bool attn_two_row_tiles(int variant, int rows, int batch) {
     const int tiles = (rows + 15) / 16 * (batch < 1 ? 1 : batch);
-    return variant == ATTN_PREFIX ? tiles > 256 && (tiles <= 320 || tiles > 341) && (tiles <= 512 || tiles > 768) : variant == ATTN_GQA128_PREFIX && tiles > 848;
+    return variant == ATTN_PREFIX ? tiles > 256 && (tiles <= 320 || tiles > 341) && (tiles <= 512 || tiles > 768) : variant == ATTN_GQA128_PREFIX && tiles > 184 && tiles != 848;
 }
 int launch_mqa_attention(const AttnP& p, int variant, hipStream_t s, int* kernels_launched = nullptr);
 // long sequences on both sides (csrc/flash.hip): 128 query rows per workgroup, K / V^T tiles shared through LDS; hd = 64
 int launch_flash_attention(const AttnP& p, int hd, hipStream_t s);
-// Gemma prefix, two row tiles per workgroup (csrc/prefix_attention.hip): one K/V head whose first keys, up to the valid length, are visible to every row; row-major output,
-// positive scale.  Others go to the general kernel with one row tile.
+// Prefix passes, two row tiles per workgroup (csrc/prefix_attention.hip): Gemma's, one K/V head whose first keys, up to the valid length, are visible to every row, and DM0's causal one
+// over several K/V heads; row-major output, positive scale.  Others go to the general kernel with one row tile.
 bool prefix_attention_takes(const AttnP& p);
 int launch_prefix_attention(const AttnP& p, hipStream_t s);
 // SigLIP attention: q, k fragment-tiled [views*16][256][96], vt tiled [views*16][80][256], out row-major

@@ -1,4 +1,5 @@
-// Gemma's prefix pass (/root/reference/pi0_infer.py:819-824, pi05_infer.py:335-360) for many rows, on v_mfma_f32_32x32x16_bf16: one K/V head of width 256, query rows = token * G + head.
+// The prefix passes for many rows, on v_mfma_f32_32x32x16_bf16; query rows = token * G + head.  HD = 256: Gemma's (/root/reference/pi0_infer.py:819-824, pi05_infer.py:335-360), one K/V
+// head.  HD = 128, CAUSAL: DM0's (/root/reference/dm0_infer.py:913-918), where a token sees the keys up to its own; 8 K/V heads, each on one XCD.
 //
 // A workgroup takes 32 query rows, its four waves every fourth block of 32 keys, and they merge through LDS.  As in csrc/flash.hip the loop runs a block behind and a
 // block ahead: while the softmax of block i is computed, the matrix pipe takes O^T += V^T P^T of block i - 1 and S^T of block i + 1, in turn, and between two products stands one
@@ -9,13 +10,16 @@
 // (2) that is 12 of the 13.4 us.  The kernel of csrc/attention.hip with two row tiles per workgroup, which it replaces here, took 64 products of 22 cycles, two softmaxes and two bursts
 // of 16 loads a block one after another, and waited for all its loads before the first product, because it asked for them behind a branch.  us with that / with this, weights
 // cold: 683 tokens 17.7 / 12.7, 768 17.3 / 13.6, 788 18.7 / 13.4, 968 22.3 / 17.3, 1 540 53.2 / 39.1, 2 048 63.3 / 52.4.
+// CAUSAL: 38 row blocks of 607 tokens are 304 workgroups of one to nineteen key blocks, two to a CU; those with the most start first.  The work itself is small (2.4 us of products and 1.5 of
+// loads if it were even): most of the 7.4 us are the launch, the first loads and the longest workgroups' five trips.  It replaces 16x16x32 products with one row tile, three workgroups
+// to a CU: 269 / 438 / 607 / 2 107 tokens 6.3 / 8.8 / 11.1 / 48.3 -> 5.15 / 5.9 / 7.4 / 30; a layer of 438 and 607 tokens 76.8 -> 74.5 and 86.6 -> 84.6.
 // (Built with the MFMA results in ordinary registers: 788 tokens 23 us otherwise, of copies and spills.)
 #include "kernels.h"
 #include <atomic>
 
 namespace {
 
-constexpr float NEG_BIG = -1.0e30f;
+constexpr float NEG_BIG = -1.0e30f, NOTHING_SEEN = -1.0e20f;
 
 RTVLA_DEVICE bf16x8 cat44(bf16x4 lo, bf16x4 hi) {
     bf16x8 v;
@@ -24,18 +28,24 @@ RTVLA_DEVICE bf16x8 cat44(bf16x4 lo, bf16x4 hi) {
     return v;
 }
 RTVLA_DEVICE f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
-__global__ __launch_bounds__(256, 1)
+template <int HD, bool CAUSAL>
+__global__ __launch_bounds__(256, HD == 256 ? 1 : 2)
 void prefix_attn_kernel(AttnP p) {
-    constexpr int HD = 256, WAVES = 4, KD = HD / 32, DS = HD / 16, DT2 = HD / 32;
+    constexpr int WAVES = 4, KD = HD / 32, DS = HD / 16, DT2 = HD / 32;
     constexpr float SLACK_BITS = 8.0f;                  // a row's maximum may have grown by this many bits before the accumulators are scaled down (csrc/flash.hip)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     f32x4* const obuf = (f32x4*)smem_raw;               // [wave][d tile][4][64]
     float* const ms = (float*)(smem_raw + (size_t)WAVES * DT2 * 4 * 64 * 16);          // [wave][32], then the sums
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, n = lane & 31;
-    const int row0 = blockIdx.x * 32;
-    int vis = min(p.keys, p.prefix_alloc);              // keys that every row sees
+    // CAUSAL: K/V heads dealt over the XCDs, the rows with the most keys first
+    const int batch = CAUSAL ? blockIdx.x % p.batch : 0;
+    const int row0 = CAUSAL ? ((int)(gridDim.x / p.batch) - 1 - (int)(blockIdx.x / p.batch)) * 32 : blockIdx.x * 32;
+    int vis = min(p.keys, p.prefix_alloc);              // keys that every row sees, causal aside
     if (p.valid_len) vis = max(0, min(*p.valid_len, vis));
+    const int all = CAUSAL ? min(vis, row0 / p.group + 1) : vis;                       // that all rows of this workgroup see
+    const int lim = CAUSAL ? min(vis, (row0 + n) / p.group + 1) : vis;                 // that this lane's row sees
+    if (CAUSAL) vis = min(vis, (row0 + 31) / p.group + 1);                             // that some row sees
     const float c = p.scale * 1.4426950408889634f;
     const float slack = SLACK_BITS / c;
     const int blocks = (vis + 31) >> 5, keys32 = p.ldvt >> 5;
@@ -45,8 +55,8 @@ void prefix_attn_kernel(AttnP p) {
     auto rows_of = [&](const bf16_t* base, size_t at, int kb, unsigned bytes) __attribute__((always_inline)) {
         return __builtin_amdgcn_make_buffer_rsrc((void*)(base + at), 0, kb < blocks ? (int)bytes : 0, 0x00027000);
     };
-    auto k_block = [&](int kb) __attribute__((always_inline)) { return rows_of(p.k, (size_t)kb * (2 * KD * 512), kb, 2 * KD * 1024); };
-    auto v_block = [&](int kb) __attribute__((always_inline)) { return rows_of(p.vt, (size_t)kb * 512, kb, (unsigned)(HD / 16 * keys32) * 1024u); };
+    auto k_block = [&](int kb) __attribute__((always_inline)) { return rows_of(p.k, (size_t)batch * p.k_bstride + (size_t)kb * (2 * KD * 512), kb, 2 * KD * 1024); };
+    auto v_block = [&](int kb) __attribute__((always_inline)) { return rows_of(p.vt, (size_t)batch * p.vt_bstride + (size_t)kb * 512, kb, (unsigned)(HD / 16 * keys32) * 1024u); };
     const int k_lane = ((n >> 4) * KD * 64 + h * 16 + (n & 15)) * 16, v_lane = (n >> 4) * keys32 * 1024 + (h * 16 + (n & 15)) * 16;
     auto piece = [&](__amdgpu_buffer_rsrc_t rs, int off, int uniform) __attribute__((always_inline)) { return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rs, off, uniform, 0)); };
     auto piece_k = [&](__amdgpu_buffer_rsrc_t rs, int s) __attribute__((always_inline)) { return piece(rs, k_lane + (s >> 1) * 1024 + (s & 1) * 512, 0); };
@@ -57,7 +67,7 @@ void prefix_attn_kernel(AttnP p) {
         const auto kr = k_block(w);
 #pragma unroll
         for (int s = 0; s < DS; ++s) kf[s] = piece_k(kr, s);
-        const bf16_t* const q0 = p.q + ((size_t)((row0 >> 4) + (n >> 4)) * KD * 64 + h * 16 + (n & 15)) * 8;
+        const bf16_t* const q0 = p.q + (size_t)batch * p.q_bstride + ((size_t)((row0 >> 4) + (n >> 4)) * KD * 64 + h * 16 + (n & 15)) * 8;
 #pragma unroll
         for (int s = 0; s < DS; ++s) qf[s] = *(const bf16x8*)(q0 + (s >> 1) * 512 + (s & 1) * 256);
     }
@@ -71,7 +81,7 @@ void prefix_attn_kernel(AttnP p) {
     auto mask = [&](int kb, f32x16& st) __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < 16; ++e)
-            if (kb * 32 + 8 * (e >> 2) + 4 * h + (e & 3) >= vis) st[e] = NEG_BIG;
+            if (kb * 32 + 8 * (e >> 2) + 4 * h + (e & 3) >= lim) st[e] = NEG_BIG;
     };
     auto lane_max = [&](const f32x16& st) __attribute__((always_inline)) {
         const auto max3 = [](float a, float b, float c) { return fmaxf(fmaxf(a, b), c); };
@@ -92,13 +102,14 @@ void prefix_attn_kernel(AttnP p) {
         for (int t = 0; t < DT2; ++t) vf[q][t] = bf16x8{};
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (w * 32 + 32 > vis) mask(w, sA);
+    if (w * 32 + 32 > all) mask(w, sA);
     float m = w < blocks ? halves_max(lane_max(sA)) : NEG_BIG, l = 0.f;
+    if (CAUSAL) m = fmaxf(m, NOTHING_SEEN);             // (a row that sees nothing of this block: its masked logits are far below)
 
     // block kb: on entry s_cur = S^T(kb), kf = K of kb + 4 (under way), vf = V^T and p_prev = probabilities of kb - 4; on exit the same for the next
     auto step = [&](int kb, f32x16& s_cur, f32x16& s_next, bf16x8 (&p_prev)[2], bf16x8 (&p_cur)[2]) __attribute__((always_inline)) {
         const auto kr = k_block(kb + 2 * WAVES), vr = v_block(kb);
-        const bool edge = kb * 32 + 32 > vis;
+        const bool edge = kb * 32 + 32 > all;
         if (edge) mask(kb, s_cur);
         const float mx = lane_max(s_cur);
         if (__builtin_expect(__any(mx > m + slack), 0)) {
@@ -135,7 +146,7 @@ void prefix_attn_kernel(AttnP p) {
 #pragma unroll
         for (int i = 0; i < 2 * DS; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x402, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x402, HD == 256 ? 2 : 4, 0);
             __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -176,7 +187,7 @@ void prefix_attn_kernel(AttnP p) {
     const int row = row0 + n;
     if (row >= p.rows) return;
     const int tok = row / p.group;
-    bf16_t* const out = p.out + (size_t)tok * p.ld_tok + (row - tok * p.group) * HD;
+    bf16_t* const out = p.out + (size_t)(batch / p.batch_inner) * p.out_ostride + (size_t)(batch % p.batch_inner) * p.out_istride + (size_t)tok * p.ld_tok + (row - tok * p.group) * HD;
 #pragma unroll
     for (int k = 0; k < DT2 / WAVES; ++k) {
         const int t = w * (DT2 / WAVES) + k;
@@ -193,12 +204,15 @@ void prefix_attn_kernel(AttnP p) {
 }  // namespace
 
 bool prefix_attention_takes(const AttnP& p) {
-    return p.prefix_alloc >= p.keys && p.nsplit <= 1 && p.batch <= 1 && !p.causal && !p.out_tiled && p.scale > 0.f;
+    return p.prefix_alloc >= p.keys && p.nsplit <= 1 && (p.causal || p.batch <= 1) && !p.out_tiled && p.scale > 0.f;
 }
-int launch_prefix_attention(const AttnP& p, hipStream_t s) {
-    constexpr size_t smem = 4 * 8 * 4 * 64 * 16 + 2 * 4 * 32 * 4;
+template <int HD, bool CAUSAL>
+int launch_prefix_inst(const AttnP& p, hipStream_t s) {
+    constexpr size_t smem = 4 * (HD / 32) * 4 * 64 * 16 + 2 * 4 * 32 * 4;
+    auto kern = prefix_attn_kernel<HD, CAUSAL>;
     static std::atomic<uint64_t> done{0};
-    if (int rc = ensure_dynamic_lds((const void*)prefix_attn_kernel, smem, done)) return rc;
-    hipLaunchKernelGGL(prefix_attn_kernel, dim3((p.rows + 31) / 32), dim3(256), smem, s, p);
+    if (int rc = ensure_dynamic_lds((const void*)kern, smem, done)) return rc;
+    hipLaunchKernelGGL(kern, dim3((p.rows + 31) / 32 * (CAUSAL ? p.batch : 1)), dim3(256), smem, s, p);
     return hipGetLastError() == hipSuccess ? 0 : 5;
 }
+int launch_prefix_attention(const AttnP& p, hipStream_t s) { return p.causal ? launch_prefix_inst<128, true>(p, s) : launch_prefix_inst<256, false>(p, s); }

@@ -85,6 +85,21 @@ def test_causal_prefix_pass_around_the_row_tiles_of_a_workgroup(tokens):
     run(capi.ATTN_GQA128_PREFIX, tokens, tokens, 8, seed=tokens)
 
 
+@pytest.mark.parametrize("tokens", [184, 185, 192, 193, 208, 223, 224, 225, 255, 256, 257, 383, 384, 385, 607])
+def test_causal_prefix_pass_in_blocks_of_32_rows(tokens):
+    """32 rows are 16 tokens: sequences that end in the first or the second half of a block of 32 keys and of rows, one trip to several of each wave, waves that
+    see nothing of their block in some rows."""
+    run(capi.ATTN_GQA128_PREFIX, tokens, tokens, 8, seed=tokens)
+    run(capi.ATTN_GQA128_PREFIX, tokens, tokens, 8, seed=tokens + 1, sharp=6.0)
+    run(capi.ATTN_GQA128_PREFIX, tokens, tokens, 8, seed=tokens + 2, ramp=-60.0)
+
+
+@pytest.mark.parametrize("tokens,heads,valid", [(300, 8, 300), (300, 8, 299), (300, 8, 33), (300, 8, 32), (300, 8, 1), (400, 6, 250), (900, 3, 511)])
+def test_causal_prefix_pass_with_a_valid_length(tokens, heads, valid):
+    """Keys past the valid length are hidden from every row, and the number of K/V heads need not be that of the XCDs."""
+    run(capi.ATTN_GQA128_PREFIX, tokens, tokens, heads, valid_len=valid, seed=valid)
+
+
 # (tokens, row tiles per workgroup): one where that was the faster, which it was not for long passes
 @pytest.mark.parametrize("model,views,sizes", [("pi0", 1, [(256, 1), (682, 1), (683, 2)]), ("pi0", 4, [(1024, 2), (1025, 1), (1536, 1), (1537, 2), (2048, 2)]),
                                                ("dm0", 1, [(177, 1), (848, 1), (849, 2), (2107, 2)])])
