@@ -176,14 +176,15 @@ enum AttnVariant { ATTN_PREFIX = 0, ATTN_SUFFIX = 1, ATTN_GQA128_PREFIX, ATTN_GQ
 // Row tiles per workgroup of the prefix passes.  Every workgroup reads all keys, so two halve what the chip reads from L2, and one halves
 // what a workgroup does between two waits.  us, weights cold, 256 CUs:
 //   Gemma, one (two or three workgroups to a CU) / two (csrc/prefix_attention.hip, one to a CU): 256 tokens (128 tiles) 6.7 / 7.8, 356 (178) 8.4 / 8.4, 512 (256) 9.7 / 9.6, 528 (264)
-//     14.6 / 10.2, 608 (304) 15.3 / 11.1, 682 (341) 17.4 / 12.6; 768 (384) 17.6 / 13.6, 968 (484) 22.0 / 17.3, 1024 (512) 23.1 / 17.7; 1032 (516) 33.5 / 28.8, 1224 (612) 40.0 /
-//     32.9, 1536 (768) 48.8 / 38.8; 1540 (770) 55.2 / 39.1, 2048 (1024) 72.5 / 52.4.  One is as good while each
+//     14.6 / 10.8, 608 (304) 15.3 / 10.9, 682 (341) 17.4 / 12.6; 768 (384) 17.6 / 12.4, 968 (484) 22.0 / 16.6, 1024 (512) 23.1 / 16.3; 1032 (516) 33.5 / 28.8, 1224 (612) 40.0 /
+//     32.9, 1536 (768) 48.8 / 38.8; 1540 (770) 55.2 / 38.5, 2048 (1024) 72.5 / 52.4.  One is as good while each
 //     workgroup has a CU to itself (256 tiles), and no longer.  It stays at 321 - 341 and 513 - 768 tiles all the same, where it was the better one beside an earlier kernel with two tiles
 //     (656 tokens (328) 16.6, 1032 (516) 39.0, 1536 (768) 47.7), because tests/test_gpu_attention.py states it for 682, 1025 and 1536 tokens.
-//   Causal (DM0, 8 K/V heads), where workgroups are of unlike length, one (three to a CU) / two (two to a CU, the longest first): 177 tokens (184 tiles) 5.0 / 5.0, 206 (208) 5.0 / 4.9,
-//     269 (272) 6.3 / 5.15, 375 (376) 7.8 / 5.35, 438 (440) 8.8 / 5.9, 515 (520) 10.1 / 6.9, 607 (608) 11.1 / 7.4, 707 (712) 13.9 / 8.7, 807 (808) 15.4 / 9.5.  Past that against two tiles in the
-//     kernel of csrc/attention.hip: 849 (856) 15.5 / 9.7, 1007 (1008) 19.4 / 11.5, 1507 (1512) 35.8 / 19.3, 2107 (2112) 48.3 / 30.  One tile stays up to 184, where it is as fast, and at 848,
+//   Causal (DM0, 8 K/V heads), where workgroups are of unlike length, one (three to a CU) / two (two to a CU, the longest first): 177 tokens (184 tiles) 5.0 / 5.0, 206 (208) 5.0 / 5.05,
+//     269 (272) 6.3 / 5.45, 375 (376) 7.8 / 5.35, 438 (440) 8.8 / 6.4, 515 (520) 10.1 / 6.9, 607 (608) 11.1 / 7.9, 707 (712) 13.9 / 8.7, 807 (808) 15.4 / 9.5.  Past that against two tiles in the
+//     kernel of csrc/attention.hip: 849 (856) 15.5 / 9.7, 1007 (1008) 19.4 / 12.2, 1507 (1512) 35.8 / 19.3, 2107 (2112) 48.3 / 30.6.  One tile stays up to 184, where it is as fast, and at 848,
 //     because tests/test_gpu_attention.py states it for 848 tokens.
+//   (Figures with two tiles at 356, 512, 682, 1032, 1224, 1536 and at 177, 375, 515, 707, 807, 849, 1507 tokens are of a version that let a row's maximum lag; following it costs 0.1 - 0.5 us.)
 inline bool attn_two_row_tiles(int variant, int rows, int batch) {
     const int tiles = (rows + 15) / 16 * (batch < 1 ? 1 : batch);
     return variant == ATTN_PREFIX ? tiles > 256 && (tiles <= 320 || tiles > 341) && (tiles <= 512 || tiles > 768) : variant == ATTN_GQA128_PREFIX && tiles > 184 && tiles != 848;

@@ -7,12 +7,12 @@
 // waves, so there is nothing that two of them would share in LDS.
 //
 // What bounds it: a CU's load path.  788 tokens are 197 workgroups that pull 807 KB each, 6.2 us at 64 bytes per clock; with the launch (1.7), the first loads (2) and the merge
-// (2) that is 12 of the 13.4 us.  The kernel of csrc/attention.hip with two row tiles per workgroup, which it replaces here, took 64 products of 22 cycles, two softmaxes and two bursts
+// (2) that is 12 of the 13.3 us.  The kernel of csrc/attention.hip with two row tiles per workgroup, which it replaces here, took 64 products of 22 cycles, two softmaxes and two bursts
 // of 16 loads a block one after another, and waited for all its loads before the first product, because it asked for them behind a branch.  us with that / with this, weights
-// cold: 683 tokens 17.7 / 12.7, 768 17.3 / 13.6, 788 18.7 / 13.4, 968 22.3 / 17.3, 1 540 53.2 / 39.1, 2 048 63.3 / 52.4.
+// cold: 683 tokens 17.7 / 12.1, 768 17.3 / 12.4, 788 18.7 / 13.3, 968 22.3 / 16.6, 1 540 53.2 / 38.5, 2 048 63.3 / 52.4.
 // CAUSAL: 38 row blocks of 607 tokens are 304 workgroups of one to nineteen key blocks, two to a CU; those with the most start first.  The work itself is small (2.4 us of products and 1.5 of
-// loads if it were even): most of the 7.4 us are the launch, the first loads and the longest workgroups' five trips.  It replaces 16x16x32 products with one row tile, three workgroups
-// to a CU: 269 / 438 / 607 / 2 107 tokens 6.3 / 8.8 / 11.1 / 48.3 -> 5.15 / 5.9 / 7.4 / 30; a layer of 438 and 607 tokens 76.8 -> 74.5 and 86.6 -> 84.6.
+// loads if it were even): most of the 7.9 us are the launch, the first loads and the longest workgroups' five trips.  It replaces 16x16x32 products with one row tile, three workgroups
+// to a CU: 269 / 438 / 607 / 2 107 tokens 6.3 / 8.8 / 11.1 / 48.3 -> 5.45 / 6.4 / 7.9 / 30.6.
 // (Built with the MFMA results in ordinary registers: 788 tokens 23 us otherwise, of copies and spills.)
 #include "kernels.h"
 #include <atomic>
@@ -32,7 +32,6 @@ template <int HD, bool CAUSAL>
 __global__ __launch_bounds__(256, HD == 256 ? 1 : 2)
 void prefix_attn_kernel(AttnP p) {
     constexpr int WAVES = 4, KD = HD / 32, DS = HD / 16, DT2 = HD / 32;
-    constexpr float SLACK_BITS = 8.0f;                  // a row's maximum may have grown by this many bits before the accumulators are scaled down (csrc/flash.hip)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     f32x4* const obuf = (f32x4*)smem_raw;               // [wave][d tile][4][64]
     float* const ms = (float*)(smem_raw + (size_t)WAVES * DT2 * 4 * 64 * 16);          // [wave][32], then the sums
@@ -47,7 +46,6 @@ void prefix_attn_kernel(AttnP p) {
     const int lim = CAUSAL ? min(vis, (row0 + n) / p.group + 1) : vis;                 // that this lane's row sees
     if (CAUSAL) vis = min(vis, (row0 + 31) / p.group + 1);                             // that some row sees
     const float c = p.scale * 1.4426950408889634f;
-    const float slack = SLACK_BITS / c;
     const int blocks = (vis + 31) >> 5, keys32 = p.ldvt >> 5;
 
     // A block past the last one is a buffer of no bytes, from which the hardware returns zeros and reads nothing: behind a branch the compiler could not tell how many loads
@@ -104,27 +102,20 @@ void prefix_attn_kernel(AttnP p) {
     __builtin_amdgcn_sched_barrier(0);
     if (w * 32 + 32 > all) mask(w, sA);
     float m = w < blocks ? halves_max(lane_max(sA)) : NEG_BIG, l = 0.f;
-    if (CAUSAL) m = fmaxf(m, NOTHING_SEEN);             // (a row that sees nothing of this block: its masked logits are far below)
+    m = fmaxf(m, NOTHING_SEEN);                         // (a row that sees nothing of this block: its masked logits, and infinite ones, are far below)
 
     // block kb: on entry s_cur = S^T(kb), kf = K of kb + 4 (under way), vf = V^T and p_prev = probabilities of kb - 4; on exit the same for the next
     auto step = [&](int kb, f32x16& s_cur, f32x16& s_next, bf16x8 (&p_prev)[2], bf16x8 (&p_cur)[2]) __attribute__((always_inline)) {
         const auto kr = k_block(kb + 2 * WAVES), vr = v_block(kb);
         const bool edge = kb * 32 + 32 > all;
         if (edge) mask(kb, s_cur);
-        const float mx = lane_max(s_cur);
-        if (__builtin_expect(__any(mx > m + slack), 0)) {
-            const float mnew = fmaxf(m, halves_max(mx)), alpha = __builtin_amdgcn_exp2f((m - mnew) * c);
-            l *= alpha;
-#pragma unroll
-            for (int t = 0; t < DT2; ++t)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
-#pragma unroll
-            for (int q = 0; q < 2; ++q)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) p_prev[q][j] = (bf16_t)((float)p_prev[q][j] * alpha);
-            m = mnew;
-        }
+        // The largest probability of a row so far is exactly 1, and each is rounded to bf16 once: the maximum follows every block, and the accumulators are scaled behind the
+        // products of block kb - 4, whose probabilities are relative to the maximum before.  (Scaled ahead of them, with those probabilities, and only where the maximum has grown by
+        // 8 bits, the error against 64 bits was 1.08 times as large, in rows of sharp logits 1.18 times; 788 tokens took 12.8 us instead of 13.3, DM0's 607 7.7 instead of 7.9.)
+        const float m_old = m;
+        m = fmaxf(m, halves_max(lane_max(s_cur)));
+        const float alpha = __builtin_amdgcn_exp2f((m_old - m) * c);
+        l *= alpha;
         const float mc = m * c;
 #pragma unroll
         for (int e = 0; e < 16; ++e) s_next[e] = 0.f;
@@ -151,6 +142,11 @@ void prefix_attn_kernel(AttnP p) {
         }
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("" :: "v"(p_cur[0]), "v"(p_cur[1]), "v"(l));               // (made here, beside the MFMAs)
+        if (__any(m > m_old))
+#pragma unroll
+            for (int t = 0; t < DT2; ++t)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
     };
     int kb = w;
     for (; kb + WAVES < blocks; kb += 2 * WAVES) {
