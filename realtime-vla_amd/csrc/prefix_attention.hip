@@ -19,7 +19,7 @@
 
 namespace {
 
-constexpr float NEG_BIG = -1.0e30f, NOTHING_SEEN = -1.0e20f;
+constexpr float HIDDEN = -__builtin_inff(), LOWEST = -3.402823466e38f;
 
 RTVLA_DEVICE bf16x8 cat44(bf16x4 lo, bf16x4 hi) {
     bf16x8 v;
@@ -79,7 +79,7 @@ void prefix_attn_kernel(AttnP p) {
     auto mask = [&](int kb, f32x16& st) __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < 16; ++e)
-            if (kb * 32 + 8 * (e >> 2) + 4 * h + (e & 3) >= lim) st[e] = NEG_BIG;
+            if (kb * 32 + 8 * (e >> 2) + 4 * h + (e & 3) >= lim) st[e] = HIDDEN;
     };
     auto lane_max = [&](const f32x16& st) __attribute__((always_inline)) {
         const auto max3 = [](float a, float b, float c) { return fmaxf(fmaxf(a, b), c); };
@@ -101,8 +101,8 @@ void prefix_attn_kernel(AttnP p) {
     }
     __builtin_amdgcn_sched_barrier(0);
     if (w * 32 + 32 > all) mask(w, sA);
-    float m = w < blocks ? halves_max(lane_max(sA)) : NEG_BIG, l = 0.f;
-    m = fmaxf(m, NOTHING_SEEN);                         // (a row that sees nothing of this block: its masked logits, and infinite ones, are far below)
+    // a row's maximum is finite, so that a key it does not see (minus infinity) has no weight at any scale, also where it sees nothing of the block
+    float m = fmaxf(LOWEST, w < blocks ? halves_max(lane_max(sA)) : HIDDEN), l = 0.f;
 
     // block kb: on entry s_cur = S^T(kb), kf = K of kb + 4 (under way), vf = V^T and p_prev = probabilities of kb - 4; on exit the same for the next
     auto step = [&](int kb, f32x16& s_cur, f32x16& s_next, bf16x8 (&p_prev)[2], bf16x8 (&p_cur)[2]) __attribute__((always_inline)) {
@@ -116,7 +116,6 @@ void prefix_attn_kernel(AttnP p) {
         m = fmaxf(m, halves_max(lane_max(s_cur)));
         const float alpha = __builtin_amdgcn_exp2f((m_old - m) * c);
         l *= alpha;
-        const float mc = m * c;
 #pragma unroll
         for (int e = 0; e < 16; ++e) s_next[e] = 0.f;
 #pragma unroll
@@ -129,7 +128,7 @@ void prefix_attn_kernel(AttnP p) {
         }
         float sum[2] = {0.f, 0.f};
 #pragma unroll
-        for (int e = 0; e < 16; ++e) { s_cur[e] = __builtin_amdgcn_exp2f(s_cur[e] * c - mc); sum[e & 1] += s_cur[e]; }
+        for (int e = 0; e < 16; ++e) { s_cur[e] = __builtin_amdgcn_exp2f((s_cur[e] - m) * c); sum[e & 1] += s_cur[e]; }       // (a difference first: of equal logits it is 0, however large they are)
         l += sum[0] + sum[1];
 #pragma unroll
         for (int q = 0; q < 2; ++q) p_cur[q] = cat44(pack4(s_cur[4 * q], s_cur[4 * q + 1], s_cur[4 * q + 2], s_cur[4 * q + 3]),
@@ -137,7 +136,7 @@ void prefix_attn_kernel(AttnP p) {
 #pragma unroll
         for (int i = 0; i < 2 * DS; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x402, HD == 256 ? 2 : 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x402, HD == 256 ? 3 : 5, 0);
             __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -166,7 +165,7 @@ void prefix_attn_kernel(AttnP p) {
     l = halves_sum(l);
     if (h == 0) ms[w * 32 + n] = m;
     __syncthreads();
-    float M = NEG_BIG;
+    float M = LOWEST;
 #pragma unroll
     for (int ww = 0; ww < WAVES; ++ww) M = fmaxf(M, ms[ww * 32 + n]);
     const float f = __builtin_amdgcn_exp2f((m - M) * c);

@@ -115,6 +115,52 @@ def test_prefix_pass_rounds_each_probability_once(kind, tokens, heads):
     assert (out.float() - ref).norm().item() <= 1.06 * rounding
 
 
+# (64 and 100 tokens: the kernel for 16 rows)
+@pytest.mark.parametrize("kind,tokens,heads", [(capi.ATTN_GEMMA_PREFIX, 64, 1), (capi.ATTN_GEMMA_PREFIX, 700, 1), (capi.ATTN_GQA128_PREFIX, 100, 8), (capi.ATTN_GQA128_PREFIX, 300, 8)])
+@pytest.mark.parametrize("exponent,sign", [(20, 1), (35, 1), (35, -1), (40, 1), (40, -1)])
+def test_prefix_pass_with_logits_of_any_size(kind, tokens, heads, exponent, sign):
+    """One product to a logit, so that each is exact: +- 2^2n times 1 to 1.75, in steps of an eighth along the keys.  A row averages the keys that share its largest; those sums are of
+    bf16 values with weights 1 / n, so what is left is the rounding of the output, and of a weight to bf16 (2^-9 each of the largest element)."""
+    lib = capi.load()
+    D, G = KINDS[kind]
+    g = torch.Generator(device="cuda:0").manual_seed(tokens + exponent)
+    q, k = torch.zeros(tokens, heads, G, D, device="cuda:0"), torch.zeros(tokens, heads, D, device="cuda:0")
+    q[..., 3] = 2.0 ** exponent
+    k[..., 3] = sign * (2.0 ** exponent * (1 + ((torch.arange(tokens, device="cuda:0") * 5) % 7) / 8))[:, None]
+    q, k, v = q.bfloat16(), k.bfloat16(), torch.randn(tokens, heads, D, device="cuda:0", generator=g).bfloat16()
+    out = torch.full_like(q, 9.0)
+    need = lib.rtvla_attention_workspace_bytes(kind, tokens, tokens, heads)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda:0")
+    assert lib.rtvla_attention(kind, _P(q.data_ptr()), _P(k.data_ptr()), _P(v.data_ptr()), _P(out.data_ptr()), tokens, tokens, heads, ctypes.c_float(D ** -0.5), tokens,
+                               None, 0, _P(ws.data_ptr()), need, _P(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    ref = reference(kind, q, k, v, D ** -0.5, tokens, tokens, 0)
+    assert (out.float() - ref).abs().max().item() <= 2.0 ** -8 * v.float().abs().max().item()
+
+
+@pytest.mark.parametrize("kind,tokens,heads", [(capi.ATTN_GEMMA_PREFIX, 64, 1), (capi.ATTN_GEMMA_PREFIX, 700, 1), (capi.ATTN_GQA128_PREFIX, 100, 8), (capi.ATTN_GQA128_PREFIX, 300, 8)])
+def test_hidden_keys_have_no_weight_at_the_smallest_scales(kind, tokens, heads):
+    """A scale at which all logits are as good as equal: a row is the mean of what it sees."""
+    lib, valid = capi.load(), 33
+    D, G = KINDS[kind]
+    g = torch.Generator(device="cuda:0").manual_seed(tokens)
+    q = torch.randn(tokens, heads, G, D, device="cuda:0", generator=g).bfloat16()
+    k, v = (torch.randn(tokens, heads, D, device="cuda:0", generator=g).bfloat16() for _ in range(2))
+    out, vl = torch.full_like(q, 9.0), torch.tensor([valid], dtype=torch.int32, device="cuda:0")
+    need = lib.rtvla_attention_workspace_bytes(kind, tokens, tokens, heads)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda:0")
+    assert lib.rtvla_attention(kind, _P(q.data_ptr()), _P(k.data_ptr()), _P(v.data_ptr()), _P(out.data_ptr()), tokens, tokens, heads, ctypes.c_float(1e-30), tokens,
+                               _P(vl.data_ptr()), 0, _P(ws.data_ptr()), need, _P(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    seen = v.float()[:valid]
+    if kind == capi.ATTN_GQA128_PREFIX:
+        last = torch.arange(tokens, device="cuda:0").clamp(max=valid - 1)
+        mean = seen.cumsum(0)[last] / (last + 1)[:, None, None]
+    else:
+        mean = seen.mean(0, keepdim=True).expand(tokens, heads, D)
+    assert (out.float() - mean[:, :, None]).abs().max().item() <= 2.0 ** -8 * v.float().abs().max().item()
+
+
 @pytest.mark.parametrize("tokens,heads,valid", [(300, 8, 300), (300, 8, 299), (300, 8, 33), (300, 8, 32), (300, 8, 1), (400, 6, 250), (900, 3, 511)])
 def test_causal_prefix_pass_with_a_valid_length(tokens, heads, valid):
     """Keys past the valid length are hidden from every row, and the number of K/V heads need not be that of the XCDs."""
