@@ -79,6 +79,10 @@ PyObject* state(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const long n_stats = PyLong_AsLong(a[3]), mode = PyLong_AsLong(a[4]), index = PyLong_AsLong(a[8]);
     if (PyErr_Occurred()) return nullptr;
     if (!plain(a[1]) || !plain(a[2]) || !plain(a[5]) || (a[6] != Py_None && !plain(a[6])) || (a[7] != Py_None && !plain(a[7]))) Py_RETURN_NONE;
+    if (a[7] != Py_None) {
+        const at::Tensor& t = THPVariable_Unpack(a[7]);
+        if (t.scalar_type() != at::kBFloat16 || !ready(t, index) || t.numel() < 32) Py_RETURN_NONE;
+    }
     Doubles values(a[0]);
     if (!values.ok()) Py_RETURN_NONE;
     const at::Tensor z = like(THPVariable_Unpack(a[5]));

@@ -11,6 +11,11 @@ import rtvla_capi as capi
 _VIEW_SHAPE = (224, 224, 3)
 
 
+def _reachable(tensor):
+    """The kernels take bare pointers: device memory, or host memory that is mapped for the device."""
+    return tensor.is_cuda or tensor.is_pinned()
+
+
 class ObservationTransforms:
     def __init__(self, model_version, norm_stats=None, state_len=7, action_dim=7, device=None):
         if model_version not in ("pi0", "pi05"):
@@ -85,9 +90,9 @@ class ObservationTransforms:
                 self._check(rc, "rtvla_preprocess_frame")
             self._keep = image
             return out_view
-        if out_view.dtype is not torch.bfloat16 or out_view.shape != _VIEW_SHAPE or not out_view.is_contiguous():
+        if out_view.dtype is not torch.bfloat16 or out_view.shape != _VIEW_SHAPE or not out_view.is_contiguous() or not _reachable(out_view):
             self._frame(image)                                    # (a bad image is reported first)
-            raise ValueError("out_view must be a contiguous bf16 [224, 224, 3] tensor")
+            raise ValueError("out_view must be a contiguous bf16 [224, 224, 3] tensor in device or pinned memory")
         img, fmt, h, w = self._frame(image)
         if static_scratch:
             img = self._parse_image(img)
@@ -116,6 +121,8 @@ class ObservationTransforms:
         if done is not None:
             self._check(done, "rtvla_preprocess_state_host")
         st = np.ascontiguousarray(state, dtype=np.float64)         # travels with the launch
+        if out_bf16 is not None and (out_bf16.dtype is not torch.bfloat16 or out_bf16.numel() < 32 or not out_bf16.is_contiguous() or not _reachable(out_bf16)):
+            raise ValueError("out_bf16 must be a contiguous bf16 tensor of 32 values in device or pinned memory")
         z = torch.empty_like(self._row)
         bins = torch.empty_like(self._bin_row) if want_bins else None
         rc = self.lib.rtvla_preprocess_state_host(st.tobytes(), st.size, a.data_ptr(), b.data_ptr(), n_stats, self.mode,
@@ -136,8 +143,8 @@ class ObservationTransforms:
             return done
         if done is not None:
             self._check(done, "rtvla_postprocess_actions_host")
-        if actions_bf16.dtype is not torch.bfloat16 or actions_bf16.shape[-1] != 32 or not actions_bf16.is_contiguous():
-            raise ValueError("actions must be a contiguous bf16 [chunk, 32] tensor")
+        if actions_bf16.dtype is not torch.bfloat16 or actions_bf16.dim() < 2 or actions_bf16.shape[-1] != 32 or not actions_bf16.is_contiguous() or not _reachable(actions_bf16):
+            raise ValueError("actions must be a contiguous bf16 [chunk, 32] tensor in device or pinned memory")
         chunk = actions_bf16.shape[0]
         st = np.ascontiguousarray(ori_state, dtype=np.float64)
         out = torch.empty((chunk, self.action_dim), dtype=torch.float64, device=self.device)

@@ -199,6 +199,36 @@ def test_host_calls_and_the_general_way_agree(version):
             assert got == want if isinstance(want, tuple) else torch.equal(got, want), i
 
 
+def test_state_outputs_and_views_in_other_memory():
+    """Pinned memory is written as device memory is; other types, strides, sizes and pageable memory are refused, before any launch, by the host calls and the general way alike."""
+    from obs_transforms import ObservationTransforms
+    rng = np.random.RandomState(42)
+    stats = {"state": {"mean": rng.randn(7).tolist(), "std": (rng.rand(7) + 0.5).tolist()}, "actions": {"mean": [0.0] * 7, "std": [1.0] * 7}}
+    plain, general = (ObservationTransforms("pi0", stats) for _ in range(2))
+    general._host = _GeneralWay
+    st, frame, dev = rng.randn(7), torch.from_numpy(rng.randint(0, 256, size=(61, 47, 3)).astype(np.uint8)).cuda(), "cuda:0"
+    good, view = torch.zeros(32, dtype=torch.bfloat16, device=dev), torch.zeros(224, 224, 3, dtype=torch.bfloat16, device=dev)
+    plain._normalize_state(st, out_bf16=good)
+    plain.resize_pad_normalize_into(frame, view)
+    for tr in (plain, general):
+        for out in (torch.zeros(32, dtype=torch.bfloat16).pin_memory(), torch.zeros(2, 32, dtype=torch.bfloat16, device=dev)):
+            tr._normalize_state(st, out_bf16=out)
+            torch.cuda.synchronize()
+            assert torch.equal(out.reshape(-1)[:32].cpu(), good.cpu())
+        pinned = torch.zeros(224, 224, 3, dtype=torch.bfloat16).pin_memory()
+        tr.resize_pad_normalize_into(frame, pinned)
+        torch.cuda.synchronize()
+        assert torch.equal(pinned, view.cpu())
+        for out in (torch.zeros(32, device=dev), torch.zeros(31, dtype=torch.bfloat16, device=dev), torch.zeros(64, dtype=torch.bfloat16, device=dev)[::2], torch.zeros(32, dtype=torch.bfloat16)):
+            with pytest.raises(ValueError, match="out_bf16"):
+                tr._normalize_state(st, out_bf16=out)
+        with pytest.raises(ValueError, match="out_view"):
+            tr.resize_pad_normalize_into(frame, torch.zeros(224, 224, 3, dtype=torch.bfloat16))
+        for acts in (torch.zeros(50, 32, dtype=torch.bfloat16), torch.zeros(32, dtype=torch.bfloat16, device=dev)):
+            with pytest.raises(ValueError, match="actions"):
+                tr.postprocess_actions(acts, st)
+
+
 def test_host_calls_follow_the_current_stream_and_are_captured():
     from obs_transforms import ObservationTransforms
     rng = np.random.RandomState(43)
