@@ -192,8 +192,8 @@ inline bool attn_two_row_tiles(int variant, int rows, int batch) {
 int launch_mqa_attention(const AttnP& p, int variant, hipStream_t s, int* kernels_launched = nullptr);
 // long sequences on both sides (csrc/flash.hip): 128 query rows per workgroup, K / V^T tiles shared through LDS; hd = 64
 int launch_flash_attention(const AttnP& p, int hd, hipStream_t s);
-// Prefix passes, two row tiles per workgroup (csrc/prefix_attention.hip): Gemma's, one K/V head whose first keys, up to the valid length, are visible to every row, and DM0's causal one
-// over several K/V heads; row-major output, positive scale.  Others go to the general kernel with one row tile.
+// Prefix passes, two row tiles per workgroup (csrc/prefix_attention.hip): Gemma's, one K/V head, and DM0's causal one over several K/V heads; row-major output, positive scale.  Others
+// go to the general kernel with one row tile.
 bool prefix_attention_takes(const AttnP& p);
 int launch_prefix_attention(const AttnP& p, hipStream_t s);
 // SigLIP attention: q, k fragment-tiled [views*16][256][96], vt tiled [views*16][80][256], out row-major

@@ -236,10 +236,21 @@ def test_gemma_prefix_pass_around_the_row_tiles_of_a_workgroup_at_few_tokens(tok
     run(capi.ATTN_GEMMA_PREFIX, tokens, tokens, 1, seed=tokens)
 
 
-# masks that the kernel for many rows does not take
+# every part of the mask at once, on the edges of blocks of 32 keys: a suffix behind the prefix, a hole behind the valid keys, state rows that see the suffix's first key only
 @pytest.mark.parametrize("prefix,state", [(900, 0), (1000, 3)])
 def test_prefix_pass_of_many_rows_with_other_masks(prefix, state):
     run(capi.ATTN_GEMMA_PREFIX, 1000, 1000, 1, prefix_alloc=prefix, state_tokens=state, seed=prefix)
+
+
+@pytest.mark.parametrize("prefix,state,valid", [(900, 5, None), (0, 3, None), (0, 0, None), (999, 2, 300), (512, 1, 33), (31, 4, 31), (32, 1, 0), (960, 1000, 1), (1000, 2, 700)])
+def test_prefix_pass_of_many_rows_with_a_suffix_and_state_rows(prefix, state, valid):
+    run(capi.ATTN_GEMMA_PREFIX, 1000, 1000, 1, prefix_alloc=prefix, state_tokens=state, valid_len=valid, seed=prefix + state)
+    run(capi.ATTN_GEMMA_PREFIX, 1000, 1000, 1, prefix_alloc=prefix, state_tokens=state, valid_len=valid, seed=prefix + state, sharp=6.0)
+
+
+@pytest.mark.parametrize("prefix,state,valid", [(200, 0, None), (200, 3, 150), (33, 2, 33), (1, 1, None), (299, 4, 100), (64, 300, 1)])
+def test_causal_prefix_pass_with_a_suffix_and_state_rows(prefix, state, valid):
+    run(capi.ATTN_GQA128_PREFIX, 300, 300, 8, prefix_alloc=prefix, state_tokens=state, valid_len=valid, seed=prefix + state)
 
 
 @pytest.mark.parametrize("tokens,prefix,valid,state", [
