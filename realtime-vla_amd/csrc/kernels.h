@@ -174,20 +174,16 @@ struct AttnP {
 enum AttnVariant { ATTN_PREFIX = 0, ATTN_SUFFIX = 1, ATTN_GQA128_PREFIX, ATTN_GQA128_SUFFIX };
 
 // Row tiles per workgroup of the prefix passes.  Every workgroup reads all keys, so two halve what the chip reads from L2, and one halves
-// what a workgroup does between two waits.  us, weights cold, 256 CUs:
-//   Gemma, one (two or three workgroups to a CU) / two (csrc/prefix_attention.hip, one to a CU): 256 tokens (128 tiles) 6.7 / 7.8, 356 (178) 8.4 / 8.4, 512 (256) 9.7 / 9.6, 528 (264)
-//     14.6 / 10.8, 608 (304) 15.3 / 10.9, 682 (341) 17.4 / 12.6; 768 (384) 17.6 / 12.4, 968 (484) 22.0 / 16.6, 1024 (512) 23.1 / 16.3; 1032 (516) 33.5 / 28.8, 1224 (612) 40.0 /
-//     32.9, 1536 (768) 48.8 / 38.8; 1540 (770) 55.2 / 38.5, 2048 (1024) 72.5 / 52.4.  One is as good while each
-//     workgroup has a CU to itself (256 tiles), and no longer.  It stays at 321 - 341 and 513 - 768 tiles all the same, where it was the better one beside an earlier kernel with two tiles
-//     (656 tokens (328) 16.6, 1032 (516) 39.0, 1536 (768) 47.7), because tests/test_gpu_attention.py states it for 682, 1025 and 1536 tokens.
-//   Causal (DM0, 8 K/V heads), where workgroups are of unlike length, one (three to a CU) / two (two to a CU, the longest first): 177 tokens (184 tiles) 5.0 / 5.0, 206 (208) 5.0 / 5.05,
-//     269 (272) 6.3 / 5.45, 375 (376) 7.8 / 5.35, 438 (440) 8.8 / 6.4, 515 (520) 10.1 / 6.9, 607 (608) 11.1 / 7.9, 707 (712) 13.9 / 8.7, 807 (808) 15.4 / 9.5.  Past that against two tiles in the
-//     kernel of csrc/attention.hip: 849 (856) 15.5 / 9.7, 1007 (1008) 19.4 / 12.2, 1507 (1512) 35.8 / 19.3, 2107 (2112) 48.3 / 30.6.  One tile stays up to 184, where it is as fast, and at 848,
-//     because tests/test_gpu_attention.py states it for 848 tokens.
-//   (Figures with two tiles at 356, 512, 682, 1032, 1224, 1536 and at 177, 375, 515, 707, 807, 849, 1507 tokens are of a version that let a row's maximum lag; following it costs 0.1 - 0.5 us.)
+// what a workgroup does between two waits.  us of a launch in its layer, weights cold, 256 CUs:
+//   Gemma, one (csrc/attention.hip, two or three workgroups to a CU) / two (csrc/prefix_attention.hip, one to a CU): 256 tokens (128 tiles) 6.5 / 7.5, 356 (178) 8.1 / 8.4, 456 (228)
+//     9.3 / 9.6, 512 (256) 9.2 / 9.6; 513 (257) 13.2 / 10.3, 608 (304) 14.3 / 10.3, 682 (341) 16.3 / 11.9, 768 (384) 17.2 / 12.1, 968 (484) 21.9 / 15.6, 1 025 - 1 032 (516) 31.0 / 27.7,
+//     1 224 (612) 36.0 / 31.2, 1 536 (768) 43.4 / 36.0, 2 048 (1 024) 71.7 / 49.0.  One is the faster while each workgroup has a CU to itself, and no longer.
+//   Causal (DM0, 8 K/V heads), where workgroups are of unlike length, one (three to a CU) / two (two to a CU, the longest first): 170 tokens (176 tiles) 5.10 / 5.04, 177 (184) 5.11 / 5.16, 184
+//     (184) 5.13 / 5.04, 185 (192) 5.07 / 5.06; 193 (200) 5.16 / 5.06, 206 (208) 5.17 / 5.08, 269 (272) 6.4 / 5.4, 438 (440) 8.0 / 6.3, 607 (608) 11.1 / 7.65, 848 (848) 15.9 / 9.9, 1 507 (1 512)
+//     32.8 / 19.6, 2 107 (2 112) 52.6 / 30.1.  Up to 192 tiles the two are as fast as each other.
 inline bool attn_two_row_tiles(int variant, int rows, int batch) {
     const int tiles = (rows + 15) / 16 * (batch < 1 ? 1 : batch);
-    return variant == ATTN_PREFIX ? tiles > 256 && (tiles <= 320 || tiles > 341) && (tiles <= 512 || tiles > 768) : variant == ATTN_GQA128_PREFIX && tiles > 184 && tiles != 848;
+    return variant == ATTN_PREFIX ? tiles > 256 : variant == ATTN_GQA128_PREFIX && tiles > 184;
 }
 int launch_mqa_attention(const AttnP& p, int variant, hipStream_t s, int* kernels_launched = nullptr);
 // long sequences on both sides (csrc/flash.hip): 128 query rows per workgroup, K / V^T tiles shared through LDS; hd = 64

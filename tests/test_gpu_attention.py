@@ -74,14 +74,14 @@ def test_gemma_prefix_pass(tokens):
 
 @pytest.mark.parametrize("tokens", [681, 682, 683, 767, 768, 769, 1023, 1024, 1025, 1224, 1536, 1537])
 def test_gemma_prefix_pass_around_the_row_tiles_of_a_workgroup(tokens):
-    """Half a 16-row tile per token: 341 tiles are the last with one tile per workgroup, 342 (683 tokens) to 512 take two (an odd number
-    of tiles among them), 513 to 768 one again, 769 two."""
+    """Half a 16-row tile per token, two tiles to a workgroup: even and odd numbers of tiles at which the workgroups are two, three and four rounds of the CUs' places for
+    one tile."""
     run(capi.ATTN_GEMMA_PREFIX, tokens, tokens, 1, seed=tokens)
 
 
 @pytest.mark.parametrize("tokens", [848, 849, 864, 1201])
 def test_causal_prefix_pass_around_the_row_tiles_of_a_workgroup(tokens):
-    """Eight heads of an eighth of a 16-row tile per token: 848 tiles are the last with one tile per workgroup, 849 tokens give 107 tiles a head."""
+    """Eight heads of an eighth of a 16-row tile per token, two tiles to a workgroup: 106 tiles a head, 107 (the last workgroup has one), 108, 151."""
     run(capi.ATTN_GQA128_PREFIX, tokens, tokens, 8, seed=tokens)
 
 
@@ -167,11 +167,12 @@ def test_causal_prefix_pass_with_a_valid_length(tokens, heads, valid):
     run(capi.ATTN_GQA128_PREFIX, tokens, tokens, heads, valid_len=valid, seed=valid)
 
 
-# (tokens, row tiles per workgroup): one where that was the faster, which it was not for long passes
-@pytest.mark.parametrize("model,views,sizes", [("pi0", 1, [(256, 1), (682, 1), (683, 2)]), ("pi0", 4, [(1024, 2), (1025, 1), (1536, 1), (1537, 2), (2048, 2)]),
-                                               ("dm0", 1, [(177, 1), (848, 1), (849, 2), (2107, 2)])])
+# (tokens, row tiles per workgroup): one where that was the faster.  us of a launch with one / two: 512 tokens 9.2 / 9.6, 513 13.2 / 10.3, 682 16.3 / 11.9, 1 025 31.0 / 27.7, 1 536 43.4 / 36.0;
+# DM0 177 5.11 / 5.16, 184 5.13 / 5.04, 185 5.07 / 5.06, 206 5.17 / 5.08, 848 15.9 / 9.9
+@pytest.mark.parametrize("model,views,sizes", [("pi0", 1, [(256, 1), (682, 2), (683, 2)]), ("pi0", 2, [(512, 1), (513, 2)]), ("pi0", 4, [(1024, 2), (1025, 2), (1536, 2), (1537, 2), (2048, 2)]),
+                                               ("dm0", 1, [(177, 1), (184, 1), (185, 2), (206, 2), (848, 2), (849, 2), (2107, 2)])])
 def test_long_prefix_passes_take_two_row_tiles(model, views, sizes):
-    """A workgroup with one row tile reads all keys for 16 rows: past about 1 600 (DM0: 850) tokens that is 10 - 30 % slower than for 32."""
+    """A workgroup with one row tile reads all keys for 16 rows: past 512 (DM0: about 190) tokens that is slower than for 32, by up to 70 %."""
     import synthetic as syn
     for tokens, tiles in sizes:
         if model == "pi0":
@@ -230,7 +231,7 @@ def test_prefix_pass_of_many_rows_with_growing_maxima_and_sharp_rows(tokens, ram
     run(capi.ATTN_GEMMA_PREFIX, tokens, tokens, 1, seed=tokens, ramp=ramp, sharp=sharp)
 
 
-# the sizes at which workgroups start and cease to take two row tiles
+# sizes about the one from which workgroups take two row tiles (513), an odd number of tiles and ends inside a block of keys among them
 @pytest.mark.parametrize("tokens", [512, 513, 577, 640, 641])
 def test_gemma_prefix_pass_around_the_row_tiles_of_a_workgroup_at_few_tokens(tokens):
     run(capi.ATTN_GEMMA_PREFIX, tokens, tokens, 1, seed=tokens)
