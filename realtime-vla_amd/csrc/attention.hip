@@ -605,14 +605,13 @@ int launch_mqa_attention(const AttnP& p0, int variant, hipStream_t s, int* nk) {
     if (p.batch < 1) p.batch = 1;
     if (p.batch_inner < 1) p.batch_inner = 1;
     if (p.group < 1) return 1;
-    const bool two = attn_two_row_tiles(variant, p.rows, p.batch);
     switch (variant) {                                          // template: waves, 16-key tiles per wave round, head width
         case ATTN_PREFIX:
-            if (two && prefix_attention_takes(p)) { if (nk) *nk = 1; return launch_prefix_attention(p, s); }
+            if (prefix_attention_takes(p, variant)) { if (nk) *nk = 1; return launch_prefix_attention(p, s); }
             return launch_mqa_inst<4, 2, 256>(p, s, nk);
         case ATTN_SUFFIX: return launch_mqa_inst<4, 2, 256>(p, s, nk);
         case ATTN_GQA128_PREFIX:
-            if (two && p.causal && prefix_attention_takes(p)) { if (nk) *nk = 1; return launch_prefix_attention(p, s); }
+            if (prefix_attention_takes(p, variant)) { if (nk) *nk = 1; return launch_prefix_attention(p, s); }
             return launch_mqa_inst<4, 2, 128, true>(p, s, nk);
         case ATTN_GQA128_SUFFIX: return launch_mqa_inst<4, 2, 128>(p, s, nk);
     }

@@ -190,7 +190,7 @@ int launch_mqa_attention(const AttnP& p, int variant, hipStream_t s, int* kernel
 int launch_flash_attention(const AttnP& p, int hd, hipStream_t s);
 // Prefix passes, two row tiles per workgroup (csrc/prefix_attention.hip): Gemma's, one K/V head, and DM0's causal one over several K/V heads; row-major output, positive scale.  Others
 // go to the general kernel with one row tile.
-bool prefix_attention_takes(const AttnP& p);
+bool prefix_attention_takes(const AttnP& p, int variant);      // by its rows (above) and its form: what a launch does and what its name says
 int launch_prefix_attention(const AttnP& p, hipStream_t s);
 // SigLIP attention: q, k fragment-tiled [views*16][256][96], vt tiled [views*16][80][256], out row-major
 int launch_vision_attention(const bf16_t* q, const bf16_t* k, const bf16_t* vt, bf16_t* out, int views, hipStream_t s);

@@ -210,8 +210,9 @@ void prefix_attn_kernel(AttnP p) {
 
 }  // namespace
 
-bool prefix_attention_takes(const AttnP& p) {
-    return p.nsplit <= 1 && (p.causal || p.batch <= 1) && !p.out_tiled && p.scale > 0.f;
+bool prefix_attention_takes(const AttnP& p, int variant) {
+    const bool form = variant == ATTN_PREFIX ? !p.causal && p.batch <= 1 : variant == ATTN_GQA128_PREFIX && p.causal;
+    return form && attn_two_row_tiles(variant, p.rows, p.batch) && p.nsplit <= 1 && !p.out_tiled && p.scale > 0.f;
 }
 template <int HD, bool CAUSAL, bool SUFFIX>
 int launch_prefix_inst(const AttnP& p, hipStream_t s) {

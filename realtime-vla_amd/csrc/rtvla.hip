@@ -704,7 +704,7 @@ struct Sched {
         a.q = c->B("encoder_Q"); a.k = Kc(i); a.vt = Vt(i); a.ldvt = c->keys_pad;
         a.out = c->B("encoder_attn"); a.group = 8; a.ld_tok = 2048; a.out_tiled = 0; a.rows = 8 * S_e; a.keys = S_e; a.scale = 0.0625f;
         a.prefix_alloc = S_e; a.valid_len = valid_len(); a.state_rows = 0;
-        if (c->want(attn_two_row_tiles(ATTN_PREFIX, a.rows, a.batch) ? "prefix attn [32 rows]" : "prefix attn [16 rows]")) c->note(launch_mqa_attention(a, ATTN_PREFIX, s), "prefix attn");
+        if (c->want(prefix_attention_takes(a, ATTN_PREFIX) ? "prefix attn [32 rows]" : "prefix attn [16 rows]")) c->note(launch_mqa_attention(a, ATTN_PREFIX, s), "prefix attn");
         gemm(c->B("encoder_attn"), 2048, S_e, S_e, c->TW("t_encoder_attn_o_w", i), nullptr, 2048, 2048, EPI_PARTIAL, GemmP{}, "prefix o");
         reduce(S_e, 2048, nullptr, c->B("encoder_x"), 2048, c->B("encoder_x"), 2048, c->B("encoder_x_norm"), XN_LD, NORM_RMS, nullptr, nullptr, 1e-6f, last_split, "prefix o reduce");
         GemmP g{}; g.out = c->B("encoder_hidden"); g.ldo = EHID_LD;
@@ -929,7 +929,7 @@ struct Sched {
         a.batch = 8; a.q_bstride = qstride; a.k_bstride = (size_t)kp * 128; a.vt_bstride = (size_t)128 * kp;
         a.group = 2; a.rows = 2 * P; a.keys = P; a.scale = 0.08838834764831845f; a.prefix_alloc = P; a.causal = 1;
         a.out = c->B("prefix_attn"); a.ld_tok = 2048; a.batch_inner = 8; a.out_istride = 256;
-        if (c->want(attn_two_row_tiles(ATTN_GQA128_PREFIX, a.rows, a.batch) ? "prefix attn [32 rows]" : "prefix attn [16 rows]")) c->note(launch_mqa_attention(a, ATTN_GQA128_PREFIX, s), "prefix attn");
+        if (c->want(prefix_attention_takes(a, ATTN_GQA128_PREFIX) ? "prefix attn [32 rows]" : "prefix attn [16 rows]")) c->note(launch_mqa_attention(a, ATTN_GQA128_PREFIX, s), "prefix attn");
         gemm(c->B("prefix_attn"), 2048, P, P, c->TW("t_llm_attn_o_w", i), nullptr, 2048, 2048, EPI_PARTIAL, GemmP{}, "prefix o");
         reduce(P, 2048, nullptr, c->B("prefix_x"), 2048, c->B("prefix_x"), 2048, nullptr, 0, NORM_RMS, nullptr, nullptr, 1e-6f, last_split, "prefix o reduce",
                c->B<float>("prefix_norm_factor"));
