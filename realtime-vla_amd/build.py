@@ -43,7 +43,7 @@ def _build_host():
     from torch.utils.cpp_extension import include_paths, library_paths
     cmd = [_hipcc(), "-x", "c++", "-std=c++17", "-O3", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__"]
     cmd += ["-I" + d for d in include_paths(device_type="cuda") + [sysconfig.get_paths()["include"]]]
-    cmd += [os.path.join(CSRC, "host_calls.cpp"), "-o", HOST_LIB, "-L" + HERE, "-l:librtvla.so", "-Wl,-rpath,$ORIGIN"]
+    cmd += [os.path.join(CSRC, "host_calls.cpp"), "-o", HOST_LIB]
     cmd += ["-L" + d for d in library_paths(device_type="cuda")] + ["-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

@@ -12,6 +12,13 @@
 
 namespace {
 
+// The library's entry points as its loader found them (bind): this module is linked against none, so that there is one library in a process, whichever it is.
+struct Entries {
+    decltype(&rtvla_preprocess_frame) frame;
+    decltype(&rtvla_preprocess_state_host) state;
+    decltype(&rtvla_postprocess_actions_host) actions;
+} entry;
+
 enum { U8_HWC, F32_HWC, F32_CHW, U8_CHW };               // frame formats of rtvla_preprocess_frame
 
 bool plain(PyObject* o) { return THPVariable_CheckExact(o); }
@@ -55,7 +62,7 @@ PyObject* frame(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!arity(n, 3, "frame")) return nullptr;
     const long index = PyLong_AsLong(a[2]);
     if (index == -1 && PyErr_Occurred()) return nullptr;
-    if (!plain(a[0]) || !plain(a[1])) Py_RETURN_NONE;
+    if (!entry.frame || !plain(a[0]) || !plain(a[1])) Py_RETURN_NONE;
     const at::Tensor& img = THPVariable_Unpack(a[0]);
     const at::Tensor& out = THPVariable_Unpack(a[1]);
     const bool f32 = img.scalar_type() == at::kFloat;
@@ -68,7 +75,7 @@ PyObject* frame(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void* const src = img.data_ptr();
     void* const dst = out.data_ptr();
     void* const stream = stream_of(index);
-    return PyLong_FromLong(launch([&] { return rtvla_preprocess_frame(src, format, (int)h, (int)w, dst, stream); }));
+    return PyLong_FromLong(launch([&] { return entry.frame(src, format, (int)h, (int)w, dst, stream); }));
     END_HANDLE_TH_ERRORS
 }
 
@@ -78,7 +85,7 @@ PyObject* state(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!arity(n, 9, "state")) return nullptr;
     const long n_stats = PyLong_AsLong(a[3]), mode = PyLong_AsLong(a[4]), index = PyLong_AsLong(a[8]);
     if (PyErr_Occurred()) return nullptr;
-    if (!plain(a[1]) || !plain(a[2]) || !plain(a[5]) || (a[6] != Py_None && !plain(a[6])) || (a[7] != Py_None && !plain(a[7]))) Py_RETURN_NONE;
+    if (!entry.state || !plain(a[1]) || !plain(a[2]) || !plain(a[5]) || (a[6] != Py_None && !plain(a[6])) || (a[7] != Py_None && !plain(a[7]))) Py_RETURN_NONE;
     if (a[7] != Py_None) {
         const at::Tensor& t = THPVariable_Unpack(a[7]);
         if (t.scalar_type() != at::kBFloat16 || !ready(t, index) || t.numel() < 32) Py_RETURN_NONE;
@@ -94,7 +101,7 @@ PyObject* state(PyObject*, PyObject* const* a, Py_ssize_t n) {
     double* const zp = (double*)z.data_ptr();
     int32_t* const bp = bins.defined() ? (int32_t*)bins.data_ptr() : nullptr;
     void* const stream = stream_of(index);
-    const int rc = launch([&] { return rtvla_preprocess_state_host(values.data(), values.size(), sa, sb, (int)n_stats, (int)mode, bf16, zp, bp, stream); });
+    const int rc = launch([&] { return entry.state(values.data(), values.size(), sa, sb, (int)n_stats, (int)mode, bf16, zp, bp, stream); });
     if (rc) return PyLong_FromLong(rc);
     PyObject* const result = PyTuple_New(2);
     if (!result) return nullptr;
@@ -111,7 +118,7 @@ PyObject* actions(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!arity(n, 9, "actions")) return nullptr;
     const long n_stats = PyLong_AsLong(a[4]), mode = PyLong_AsLong(a[5]), dim = PyLong_AsLong(a[6]), index = PyLong_AsLong(a[8]);
     if (PyErr_Occurred()) return nullptr;
-    if (!plain(a[0]) || !plain(a[2]) || !plain(a[3]) || !plain(a[7])) Py_RETURN_NONE;
+    if (!entry.actions || !plain(a[0]) || !plain(a[2]) || !plain(a[3]) || !plain(a[7])) Py_RETURN_NONE;
     const at::Tensor& act = THPVariable_Unpack(a[0]);
     if (act.scalar_type() != at::kBFloat16 || act.dim() != 2 || act.size(1) != 32 || !ready(act, index) || act.size(0) > INT_MAX || dim < 0) Py_RETURN_NONE;
     Doubles values(a[1]);
@@ -123,13 +130,23 @@ PyObject* actions(PyObject*, PyObject* const* a, Py_ssize_t n) {
     double* const dst = (double*)out.data_ptr();
     void* const stream = stream_of(index);
     const int rc = launch([&] {
-        return rtvla_postprocess_actions_host(src, (int)act.size(0), sa, sb, (int)n_stats, (int)mode, values.data(), values.size(), (int)dim, dst, stream);
+        return entry.actions(src, (int)act.size(0), sa, sb, (int)n_stats, (int)mode, values.data(), values.size(), (int)dim, dst, stream);
     });
     return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(out);
     END_HANDLE_TH_ERRORS
 }
 
-PyMethodDef methods[] = {{"frame", (PyCFunction)(void*)frame, METH_FASTCALL, nullptr},
+// bind(address of rtvla_preprocess_frame, of rtvla_preprocess_state_host, of rtvla_postprocess_actions_host): once, before any other call
+PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (!arity(n, 3, "bind")) return nullptr;
+    void* const at[3] = {PyLong_AsVoidPtr(a[0]), PyLong_AsVoidPtr(a[1]), PyLong_AsVoidPtr(a[2])};
+    if (PyErr_Occurred()) return nullptr;
+    entry = {(decltype(entry.frame))at[0], (decltype(entry.state))at[1], (decltype(entry.actions))at[2]};
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {{"bind", (PyCFunction)(void*)bind, METH_FASTCALL, nullptr},
+                         {"frame", (PyCFunction)(void*)frame, METH_FASTCALL, nullptr},
                          {"state", (PyCFunction)(void*)state, METH_FASTCALL, nullptr},
                          {"actions", (PyCFunction)(void*)actions, METH_FASTCALL, nullptr},
                          {nullptr, nullptr, 0, nullptr}};

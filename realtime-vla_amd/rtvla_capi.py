@@ -119,15 +119,18 @@ _host = None
 
 
 def load_host():
-    """The module of csrc/host_calls.cpp; raises if it is missing."""
+    """The module of csrc/host_calls.cpp, with the entry points of the library that load() found; raises if it is missing."""
     global _host
     if _host is None:
         if not os.path.exists(HOST_PATH):
             raise RuntimeError("_rtvla_host.so is not built (%s); run `python realtime-vla_amd/build.py`" % HOST_PATH)
         import torch                                           # noqa: F401  (the module links against its libraries)
         loader = importlib.machinery.ExtensionFileLoader("_rtvla_host", HOST_PATH)
-        _host = importlib.util.module_from_spec(importlib.util.spec_from_loader("_rtvla_host", loader))
-        loader.exec_module(_host)
+        host = importlib.util.module_from_spec(importlib.util.spec_from_loader("_rtvla_host", loader))
+        loader.exec_module(host)
+        lib = load()
+        host.bind(*(ctypes.cast(f, _P).value for f in (lib.rtvla_preprocess_frame, lib.rtvla_preprocess_state_host, lib.rtvla_postprocess_actions_host)))
+        _host = host
     return _host
 
 

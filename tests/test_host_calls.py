@@ -1,4 +1,8 @@
 """What the observation calls refuse before a pointer reaches a kernel, on the CPU: the general way with a library that only records, and the module of host calls."""
+import shutil
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -67,6 +71,15 @@ def test_actions_without_rows_are_refused(monkeypatch):
     tr._normalize_state(np.zeros(7), out_bf16=torch.zeros(2, 32, dtype=torch.bfloat16))
     tr.resize_pad_normalize_into(torch.zeros(10, 10, 3, dtype=torch.uint8), torch.zeros(224, 224, 3, dtype=torch.bfloat16))
     assert tr.lib.calls == ["rtvla_postprocess_actions_host", "rtvla_preprocess_state_host", "rtvla_preprocess_frame"]
+
+
+def test_host_calls_use_the_library_that_was_loaded(tmp_path):
+    """Another build of the library in place of the shipped one: the host calls do not bring a second one into the process."""
+    other = shutil.copy(capi.LIB_PATH, tmp_path / "other.so")
+    code = ("import sys; sys.path.insert(0, %r); import rtvla_capi as c; c.LIB_PATH = %r; c.load(); c.load_host(); "
+            "print([l.split()[-1] for l in open('/proc/self/maps') if l.rstrip().endswith('.so')])" % (capi.HERE, str(other)))
+    maps = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, check=True, timeout=300).stdout
+    assert str(other) in maps and "_rtvla_host.so" in maps and "librtvla.so" not in maps
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="with a device its memory could be meant: the checks themselves are what is tested")
