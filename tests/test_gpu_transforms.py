@@ -146,11 +146,6 @@ def test_whole_observation_through_the_policy():
     assert out.shape == (10, 7) and np.array_equal(out, ref)
 
 
-class _GeneralWay:
-    """In place of the module of host calls: every call goes the general way."""
-    frame = state = actions = staticmethod(lambda *args: None)
-
-
 def _outcome(call):
     try:
         return call()
@@ -161,7 +156,7 @@ def _outcome(call):
 @pytest.mark.parametrize("version", ["pi0", "pi05"])
 def test_host_calls_and_the_general_way_agree(version):
     """What the host calls take and what they leave to the general way, accepted or refused: the same bits, the same errors."""
-    from obs_transforms import ObservationTransforms
+    from obs_transforms import ObservationTransforms, _GeneralWay
     rng = np.random.RandomState(41)
     stats = {g: {"mean": rng.randn(7).tolist(), "std": (rng.rand(7) + 0.5).tolist(), "q01": (-1 - rng.rand(7)).tolist(), "q99": (1 + rng.rand(7)).tolist()}
              for g in ("state", "actions")}
@@ -201,7 +196,7 @@ def test_host_calls_and_the_general_way_agree(version):
 
 def test_state_outputs_and_views_in_other_memory():
     """Pinned memory is written as device memory is; other types, strides, sizes and pageable memory are refused, before any launch, by the host calls and the general way alike."""
-    from obs_transforms import ObservationTransforms
+    from obs_transforms import ObservationTransforms, _GeneralWay
     rng = np.random.RandomState(42)
     stats = {"state": {"mean": rng.randn(7).tolist(), "std": (rng.rand(7) + 0.5).tolist()}, "actions": {"mean": [0.0] * 7, "std": [1.0] * 7}}
     plain, general = (ObservationTransforms("pi0", stats) for _ in range(2))

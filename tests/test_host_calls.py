@@ -20,13 +20,9 @@ class _Recorder:
         return lambda *args: self.calls.append(name) or 0
 
 
-class _NoHostCalls:
-    frame = state = actions = staticmethod(lambda *args: None)
-
-
 def _transforms():
     tr = obs_transforms.ObservationTransforms.__new__(obs_transforms.ObservationTransforms)
-    tr.lib, tr._host, tr.mode, tr.action_dim, tr._index, tr.device = _Recorder(), _NoHostCalls, 0, 7, 0, torch.device("cpu")
+    tr.lib, tr._host, tr.mode, tr.action_dim, tr._index, tr.device = _Recorder(), obs_transforms._GeneralWay, 0, 7, 0, torch.device("cpu")
     stat = torch.ones(7, dtype=torch.float64)
     tr._stats = {"state": (stat, stat, 7), "actions": (stat, stat, 7)}
     tr._row, tr._bin_row = torch.empty(32, dtype=torch.float64), torch.empty(32, dtype=torch.int32)
@@ -80,6 +76,21 @@ def test_host_calls_use_the_library_that_was_loaded(tmp_path):
             "print([l.split()[-1] for l in open('/proc/self/maps') if l.rstrip().endswith('.so')])" % (capi.HERE, str(other)))
     maps = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, check=True, timeout=300).stdout
     assert str(other) in maps and "_rtvla_host.so" in maps and "librtvla.so" not in maps
+
+
+@pytest.mark.parametrize("content", [None, b"not a module"])
+def test_the_library_is_enough_without_the_module_of_host_calls(content, tmp_path, monkeypatch):
+    """Not built, or built for another PyTorch (any file that does not load): said once per object, and every call goes the general way.  Asked for by name it is an error."""
+    path = tmp_path / "_rtvla_host.so"
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(capi, "HOST_PATH", str(path))
+    monkeypatch.setattr(capi, "_host", None)
+    with pytest.warns(RuntimeWarning, match="_rtvla_host"):
+        host = obs_transforms._host_calls()
+    assert host.frame(1, 2, 3) is None and host.state(*range(9)) is None and host.actions(*range(9)) is None
+    with pytest.raises((RuntimeError, ImportError)):
+        capi.load_host()
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="with a device its memory could be meant: the checks themselves are what is tested")
