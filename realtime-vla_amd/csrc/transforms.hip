@@ -66,9 +66,12 @@ RTVLA_DEVICE int clip8(int v) { v >>= PRECISION_BITS; return v < 0 ? 0 : (v > 25
 enum FrameFormat { FRAME_U8_HWC = 0, FRAME_F32_HWC, FRAME_F32_CHW, FRAME_U8_CHW };
 constexpr int TW = 32;                      // columns of a workgroup
 // Threads: a thread takes a column of every (threads / TW)-th source row, and all wait for the loads of one row before those of their next.  With 1 024 instead of 512 a frame of bytes
-// of 300 x 400, 480 x 640, 719 x 1 279, 1 080 x 1 920 takes 3.51, 3.92, 4.93, 6.73 instead of 3.42, 4.11, 5.15, 7.89 us: from 24 source rows a block on (the first has 22, the second 30).
+// of 300 x 400, 480 x 640, 719 x 1 279, 1 080 x 1 920 takes 3.99, 4.38, 5.45, 7.4 instead of 3.90, 4.56, 5.63, 8.6 us: from 24 source rows a block on (the first has 22, the second 30).
+// Not so where the blocks that hold a part of the picture are more than the CUs and have many rows: 1 920 x 1 920 (47 rows) 9.1 / 9.9, 2 448 x 2 448 (58) 11.9 / 12.0, 2 160 x 2 880 (68) 15.6 / 14.4,
+// 3 000 x 4 000 (95) 27.3 / 24.6, channels first 42.8 / 38.5; 2 250 x 4 000 (95 as well, 224 blocks) 17.0 / 20.3.  Nor for float frames that are not staged: 1 440 x 2 560 37.4 / 33.9, 2 160 x 3 840
+// 105 / 92, channels first 68 / 63.
 // Staged float frames, whose loads are all on the way at once and whose bytes it converts: 3.91, 4.38, 6.46, 10.1 instead of 4.06, 5.03, 7.04, 12.1.
-constexpr int NT_MANY_ROWS = 24, STAGED_NT = 1024;
+constexpr int NT_MANY_ROWS = 24, NT_TOO_MANY_ROWS = 60, CUS = 256, STAGED_NT = 1024;
 struct FrameP { const uint8_t* src; int h, w, rw, rh, pad_top, pad_left, taps_x, taps_y, max_rows, pitch; bf16_t* dst; Axis x, y; };      // taps: rounded up to 4
 
 // numpy's / torch's float -> uint8: truncation to an integer, low byte
@@ -388,8 +391,14 @@ void launch_resize(FrameP p, hipStream_t s) {
             if (ensure_dynamic_lds((const void*)kern, STAGED_LDS, done) == 0) { hipLaunchKernelGGL(kern, dim3(224 / TW, 224 / TH), dim3(STAGED_NT), staged, s, p); return; }
             (void)hipGetLastError();                                           // (the refusal is not an error of the launch below, which needs no more than the default)
         }
-    if (p.max_rows > NT_MANY_ROWS) hipLaunchKernelGGL((resize_kernel<FMT, TH, 1024>), dim3(224 / TW, 224 / TH), dim3(1024), smem, s, p);
-    else hipLaunchKernelGGL((resize_kernel<FMT, TH, 512>), dim3(224 / TW, 224 / TH), dim3(512), smem, s, p);
+    if constexpr (FMT == FRAME_U8_HWC || FMT == FRAME_U8_CHW) {
+        auto blocks = [](int pad, int n, int per) { return (pad + n - 1) / per - pad / per + 1; };
+        if (p.max_rows > NT_MANY_ROWS && (p.max_rows <= NT_TOO_MANY_ROWS || blocks(p.pad_left, p.rw, TW) * blocks(p.pad_top, p.rh, TH) <= CUS)) {
+            hipLaunchKernelGGL((resize_kernel<FMT, TH, 1024>), dim3(224 / TW, 224 / TH), dim3(1024), smem, s, p);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((resize_kernel<FMT, TH, 512>), dim3(224 / TW, 224 / TH), dim3(512), smem, s, p);
 }
 template <int FMT>
 int launch_frame(const FrameP& p, hipStream_t s) {

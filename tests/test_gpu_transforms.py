@@ -30,8 +30,8 @@ def test_image_preprocessing_matches_the_pillow_restatement_bit_exactly(h, w):
     assert torch.equal(got, want), "mismatching elements: %d" % (got != want).sum().item()
 
 
-# (448 and 482 rows: 24 and 25 source rows a block, either side of the rule for its threads)
-@pytest.mark.parametrize("h,w", [(1, 1), (4, 5), (9, 300), (300, 9), (223, 225), (448, 448), (482, 481), (479, 641), (717, 1279), (2700, 1801)])
+# (either side of the rule for the threads of a block: 448 and 482 rows, of which a block has 24 and 25; 2 460 and 2 640 rows of as many, of which it has 58 and 65 in more blocks than CUs)
+@pytest.mark.parametrize("h,w", [(1, 1), (4, 5), (9, 300), (300, 9), (223, 225), (448, 448), (482, 481), (479, 641), (717, 1279), (2700, 1801), (2460, 2460), (2640, 2640)])
 @pytest.mark.parametrize("fmt", ["u8", "u8_chw", "f32", "f32_chw"])
 def test_frame_formats_at_the_edges_of_the_tiles(h, w, fmt):
     """Every frame format on the device: single pixels, strips narrower than a tile, windows that end with the buffer, both tile heights."""
