@@ -62,7 +62,7 @@ RTVLA_DEVICE int clip8(int v) { v >>= PRECISION_BITS; return v < 0 ? 0 : (v > 25
 // across into an 8-bit LDS tile, and that tile down into the output.  Neighbouring row blocks resample the rows they share twice
 // ((TH + 2) / TH of the work for TH output rows); in exchange nothing but the frame is read and nothing but the result written, and the
 // second launch with its round trip through memory is gone.  Measured (480 x 640 uint8, one frame): two launches, each thread deriving the
-// weights of its own pixel, 11.7 us; this one 3.9 us.  TH = 4 gives large frames (many taps per pixel) twice the workgroups.
+// weights of its own pixel, 11.7 us; this one 4.4 us.  TH = 4 gives large frames (many taps per pixel) twice the workgroups.
 enum FrameFormat { FRAME_U8_HWC = 0, FRAME_F32_HWC, FRAME_F32_CHW, FRAME_U8_CHW };
 constexpr int TW = 32;                      // columns of a workgroup
 // Threads: a thread takes a column of every (threads / TW)-th source row, and all wait for the loads of one row before those of their next.  With 1 024 instead of 512 a frame of bytes
@@ -70,7 +70,8 @@ constexpr int TW = 32;                      // columns of a workgroup
 // Not so where the blocks that hold a part of the picture are more than the CUs and have many rows: 1 920 x 1 920 (47 rows) 9.1 / 9.9, 2 448 x 2 448 (58) 11.9 / 12.0, 2 160 x 2 880 (68) 15.6 / 14.4,
 // 3 000 x 4 000 (95) 27.3 / 24.6, channels first 42.8 / 38.5; 2 250 x 4 000 (95 as well, 224 blocks) 17.0 / 20.3.  Nor for float frames that are not staged: 1 440 x 2 560 37.4 / 33.9, 2 160 x 3 840
 // 105 / 92, channels first 68 / 63.
-// Staged float frames, whose loads are all on the way at once and whose bytes it converts: 3.91, 4.38, 6.46, 10.1 instead of 4.06, 5.03, 7.04, 12.1.
+// Staged float frames, whose loads are all on the way at once and whose bytes it converts: 4.43, 4.91, 7.24, 10.8 instead of 4.58, 5.60, 8.30, 12.8 (1 200 x 1 600 13.4 instead of 13.2).
+// (All figures of this file: launches in a graph, four frames in turn.)
 constexpr int NT_MANY_ROWS = 24, NT_TOO_MANY_ROWS = 60, CUS = 256, STAGED_NT = 1024;
 struct FrameP { const uint8_t* src; int h, w, rw, rh, pad_top, pad_left, taps_x, taps_y, max_rows, pitch; bf16_t* dst; Axis x, y; };      // taps: rounded up to 4
 
@@ -114,9 +115,9 @@ RTVLA_DEVICE void resize_down(const FrameP& p, const Window* win, const bf16_t* 
 
 // Float frames, whose values cost six instructions each to become bytes: the source rectangle of the block is loaded in whole lines, converted once and
 // staged in LDS as dwords R G B - (windows overlap by half, and four-tap groups round them up, so resize_kernel loads and converts each value 2.8 times);
-// the first loads are on the way while the weights are derived.  us per frame of 300 x 400, 480 x 640, 719 x 1 279, 1 080 x 1 920: 4.2, 4.9, 9.4, 14.8
-// without and 3.9, 4.4, 6.5, 10.1 with (1.6 of it the launch).  Frames that are not reduced (4 taps) are as fast or faster without (224 x 224
-// 3.8 / 4.0), as are bytes (480 x 640 4.3 / 4.65), and rectangles of more than half a CU's LDS stay with resize_kernel.
+// the first loads are on the way while the weights are derived.  us per frame of 300 x 400, 480 x 640, 719 x 1 279, 1 080 x 1 920: 4.8, 6.3, 10.9, 18.3
+// without and 4.4, 4.9, 7.25, 10.8 with (1.6 of it the launch).  Frames that are not reduced (4 taps) are as fast or faster without (224 x 224
+// 3.8 / 4.0 when this was introduced), as are bytes (480 x 640 4.3 / 4.65), and rectangles of more than half a CU's LDS stay with resize_kernel.
 struct Raw4 { f32x4 v[3]; };
 template <int FMT>
 RTVLA_DEVICE Raw4 load_px4(const FrameP& p, size_t at) {                       // four consecutive pixels; zero past the frame
