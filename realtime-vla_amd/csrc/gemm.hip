@@ -25,7 +25,7 @@ RTVLA_DEVICE f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdg
 // workgroups per CU so that one workgroup's MFMAs run under the other's memory latency.
 // One block tile of MT 32-row tiles starting at row m0: K loop and epilogue.
 // V: a tile of V columns, whose product is taken as activations x weights (gemm_scatter.h)
-// KG: groups of WN waves that share a block tile and split its K stages among them, each with stage buffers of its own.  For launches of few workgroups, where
+// KG: one group of WN waves, or two that share a block tile and split its K stages, each with stage buffers of its own.  For launches of few workgroups, where
 // the waves of a CU wait for their loads: two groups have twice as much on the way and half as many stages one after another.  us of a whole layer with one / two
 // groups, weights cold: DM0's prefix QKV, K = 2 048, 206 rows (64 x 128) 75.8 / 74.0, 398 90.9 / 89.1, 607 (96 x 128) 105.9 / 105.0, Gemma's, 968 rows 235.4 / 232.6, ViT
 // down projection, K = 4 096, 2 720 rows 161.4 / 159.2.  With two groups a tile of 64 x 64 has eight 32 x 32 products a stage for four waves, which on its own would be two waves
@@ -38,7 +38,7 @@ struct GemmLds {
     static constexpr int stages = 3 * MT * 32 * 128;                                   // of one group
     static constexpr int out_tile = 32 * (WN * (EpiTraits<EPI>::dual ? NT / 2 : NT) * 32 * (f32 ? 4 : 2) + 16);
     static constexpr int group = stages > out_tile ? stages : out_tile;                // a group's own memory
-    static constexpr int sums = (KG - 1) * MT * WN * NT * 4096;                        // the tiles the groups hand each other
+    static constexpr int sums = KG == 2 ? MT * WN * NT * 4096 : 0;                     // the tiles the groups hand each other
     static constexpr int bytes = KG * group > sums ? KG * group : sums;
 };
 template <int WN, int MT, int NT, int EPI, bool V = false, int KG = 1>
@@ -210,8 +210,7 @@ RTVLA_DEVICE void gemm_block(const GemmP& pk, unsigned char* smem_all, int m0_wg
             if (s < s_end) stage(b0, b1, last, breg0, areg0, areg1);
         }
     }
-    // Each group keeps MTO of the row tiles and gets the other groups' sums of them (in the order of the groups) for its own; from here on m0 and p.M are
-    // those of its rows.
+    // Each group keeps MTO of the row tiles and gets the other's sums of them for its own; from here on m0 and p.M are those of its rows.
     constexpr int MTO = (MT + KG - 1) / KG;
     f32x16 own[MTO][NT];
     if constexpr (KG == 1) {
@@ -221,7 +220,8 @@ RTVLA_DEVICE void gemm_block(const GemmP& pk, unsigned char* smem_all, int m0_wg
             for (int j = 0; j < NT; ++j) own[i][j] = acc[i][j];
     } else {
         f32x4* const sums = (f32x4*)smem_all;
-        auto at = [&](int from, int i, int j) __attribute__((always_inline)) { return sums + ((((from - (from > i / MTO)) * MT + i) * WN + wn) * NT + j) * 256 + lane; };
+        static_assert(KG == 2, "each tile has one other sum");
+        auto at = [&](int i, int j) __attribute__((always_inline)) { return sums + ((i * WN + wn) * NT + j) * 256 + lane; };
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -229,11 +229,11 @@ RTVLA_DEVICE void gemm_block(const GemmP& pk, unsigned char* smem_all, int m0_wg
 #pragma unroll
                 for (int j = 0; j < NT; ++j)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) at(kg, i, j)[e * 64] = f32x4{acc[i][j][4 * e], acc[i][j][4 * e + 1], acc[i][j][4 * e + 2], acc[i][j][4 * e + 3]};
+                    for (int e = 0; e < 4; ++e) at(i, j)[e * 64] = f32x4{acc[i][j][4 * e], acc[i][j][4 * e + 1], acc[i][j][4 * e + 2], acc[i][j][4 * e + 3]};
         __syncthreads();
 #pragma unroll
         for (int g = 0; g < KG; ++g) {
-            if (g != kg || g * MTO >= MT) continue;
+            if (g != kg) continue;
 #pragma unroll
             for (int k = 0; k < MTO; ++k) {
                 const int i = g * MTO + k;
@@ -242,14 +242,10 @@ RTVLA_DEVICE void gemm_block(const GemmP& pk, unsigned char* smem_all, int m0_wg
                 for (int j = 0; j < NT; ++j) {
                     f32x16 v = acc[i][j];
 #pragma unroll
-                    for (int from = 0; from < KG; ++from) {
-                        if (from == g) continue;
+                    for (int e = 0; e < 4; ++e) {
+                        const f32x4 o = at(i, j)[e * 64];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const f32x4 o = at(from, i, j)[e * 64];
-#pragma unroll
-                            for (int q = 0; q < 4; ++q) v[4 * e + q] += o[q];
-                        }
+                        for (int q = 0; q < 4; ++q) v[4 * e + q] += o[q];
                     }
                     own[k][j] = v;
                 }
@@ -441,7 +437,7 @@ int launch_cfg(const GemmP& p, hipStream_t s) {
     const int sps = (stages_total + nsplit - 1) / nsplit;
     if ((nsplit - 1) * sps >= stages_total) return 3;      // an empty split would leave its partial unwritten
     if (MT > 4 && ((sps & 1) || (stages_total & 1))) return 3;              // the large tiles consume K stages in pairs
-    if constexpr (KG > 1)                                  // the groups meet at every barrier, so they have as many stages each
+    if constexpr (KG > 1)                                  // the groups meet at every barrier, so they have as many stages each (a caller's own split need not give them that)
         if (sps % KG || stages_total % sps) return launch_cfg<4, MT, NT, EPI, MIXED>(p, s);
     GemmP q = p; q.nsplit = nsplit;
     // three K-stage buffers; the row-major epilogues stage 32-row output tiles in the same memory
