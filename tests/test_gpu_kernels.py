@@ -242,7 +242,8 @@ def test_eight_wave_tiles_of_the_cost_model_against_fp32(M, K, N, act):
 
 # what the cost model gives to the tiles whose K is split between two groups of waves: 64 x 64 (128 workgroups of 64 x 128 and fewer), 64 x 128 and 96 x 128 (24 K
 # stages and more), with rows that end in the first, in the second and behind the last row tile, odd numbers of stages for a group, columns past a block, and
-# stages that the groups cannot share evenly (13 for a split: one group); bias, bias + GELU, residual, and partial sums (act None)
+# columns whose K the rule leaves to one group (26 stages in 2 splits of 13); bias, bias + GELU, residual, and partial sums (act None).  That the tiles are taken is asserted by
+# name below, for launches of a forward
 @pytest.mark.parametrize("M,K,N", [
     (33, 128, 64), (65, 264, 272), (1, 640, 16), (97, 1152, 1152), (256, 2048, 2560), (190, 1664, 2048),
     (532, 2048, 2560), (481, 1528, 2512), (449, 4096, 1536), (788, 2048, 2560), (865, 1536, 2544), (609, 4096, 2048)])
@@ -269,6 +270,49 @@ def test_forward_takes_two_k_groups_where_workgroups_are_few():
     m = Pi0Inference(syn.pi0_checkpoint(5, 0, "cuda:0", 1, 1), 1, 8)
     names = [m._engine.ctx.time_launch(stage, 0, 0, 0, 1, torch.cuda.current_stream().cuda_stream)[1] for stage in (capi.STAGE_VISION_LAYER, capi.STAGE_PREFIX_LAYER)]
     assert names == ["vision qkv [64x64 2 K groups split 1]", "prefix qkv [64x64 2 K groups split 1]"]
+
+
+# the scattering epilogues of both tiles, where each group has row tiles of its own: rows that end in the first, the second and the third row tile of a block, one block of 64 x 64 as well
+@pytest.mark.parametrize("views,prompt,tile", [(1, 0, "64x64"), (1, 20, "64x64"), (2, 20, "64x128"), (2, 43, "64x128"), (3, 20, "96x128"), (3, 50, "96x128"), (3, 80, "96x128")])
+def test_prefix_qkv_of_two_k_groups(views, prompt, tile):
+    import synthetic as syn
+    import rtvla_capi as capi
+    from oracle import ops
+    from pi0_infer import Pi0Inference
+    tokens = 256 * views + prompt
+    ck = syn.pi0_checkpoint(6, prompt, "cuda:0", 1, 1)
+    e = Pi0Inference(ck, views, 8)._engine
+    assert e.ctx.time_launch(capi.STAGE_PREFIX_LAYER, 0, 0, 0, 1, torch.cuda.current_stream().cuda_stream)[1] == "prefix qkv [%s 2 K groups split 1]" % tile
+    x = torch.randn(tokens, 2048, device="cuda:0", generator=torch.Generator(device="cuda:0").manual_seed(tokens))
+    e.buffers["encoder_x_norm"].copy_(x)
+    e.buffers["encoder_Q"].fill_(3); e.buffers["encoder_K"].fill_(3); e.buffers["encoder_Vt"].fill_(3)
+    e.run_stage(capi.STAGE_PREFIX_LAYER, 0, 0)
+    torch.cuda.synchronize()
+    qkv, table = x.bfloat16().float().cpu() @ ck["encoder_attn_qkv_w"][0].float().cpu(), ops.rope_table(0, tokens)
+    # the result is rounded by at most 2^-9 of itself, the product ahead of the rotation at most likewise, which moves its pair's partner too: 2^-9 (1 + sqrt(2)) of a head's row at worst
+    for name, want in (("encoder_Q", ops.rope_interleaved(qkv[:, :2048], table).reshape(-1, 256)), ("encoder_K", ops.rope_interleaved(qkv[:, 2048:2304], table)), ("encoder_V", qkv[:, 2304:])):
+        got = e.reference_buffer(name).float().cpu().reshape(-1, 256)
+        rows = want.shape[0]
+        assert ((got[:rows] - want).norm(dim=1) / want.norm(dim=1)).max().item() <= 2.0 ** -9 * 2.42, name
+        assert name == "encoder_Q" or bool((got[rows:] == 3).all()), name
+
+
+@pytest.mark.parametrize("images,lang,tile", [(1, 7, "64x128"), (1, 37, "64x128"), (1, 69, "64x128"), (3, 100, "96x128"), (3, 109, "96x128"), (3, 139, "96x128")])
+def test_prefix_heads_of_two_k_groups(images, lang, tile):
+    """DM0, whose heads are normalised behind a barrier of the whole workgroup: by each group for the row tiles that it keeps."""
+    import rtvla_capi as capi
+    from test_gpu_dm0 import one_layer_policy, test_prefix_heads_are_normalised_by_their_gemm as heads_against_fp32
+    m = one_layer_policy(images, lang)[0]
+    assert m._engine.ctx.time_launch(capi.STAGE_PREFIX_LAYER, 0, 0, 0, 1, torch.cuda.current_stream().cuda_stream)[1] == "prefix qkv [%s 2 K groups split 1]" % tile
+    heads_against_fp32(images, lang)
+
+
+# a caller's own split with the cost model's tile: 10 stages in 2, 3 and 4 splits of 5, 4 and 3, which two groups cannot share; 32 in 2, 3 and 4
+@pytest.mark.parametrize("M,K,N,nsplit", [(65, 640, 272, 2), (65, 640, 272, 3), (65, 640, 272, 4), (532, 2048, 1536, 3), (532, 2048, 1536, 4), (788, 2048, 2048, 3), (788, 2048, 2048, 2)])
+def test_two_k_groups_with_a_callers_split(M, K, N, nsplit):
+    import rtvla_capi as capi
+    res = _run(capi.load(), capi, M, K, N, capi.TILE_AUTO, nsplit)
+    assert res is not None and res[0] <= REL_TOL and res[1] <= 1.01, res
 
 
 def test_eight_wave_tiles_give_what_their_offsets_cannot_reach_to_the_four_wave_kernel():
