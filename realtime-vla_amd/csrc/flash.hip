@@ -50,17 +50,6 @@ RTVLA_DEVICE bf16_t* flash_out_ptr(const AttnP& p, int batch, int row, int d, in
 constexpr float RESCALE_BITS = 8.0f;
 constexpr int FLASH_STAGES = 3;
 
-// The key loop is software-pipelined over 32-key blocks so that every MFMA has independent VALU work to run under: while
-// the softmax of block g is computed (VALU), the matrix pipe takes S^T of block g+1 and O^T += V^T P^T of block g-1.
-// A block needs 8 MFMAs (256 cycles) and ~65 VALU instructions of one wave; issued back to back by one wave, or by
-// several waves in turn, the two streams mostly add up on a SIMD, interleaved one MFMA to a handful of VALU
-// instructions they overlap.  Three LDS stages: tile T+2 is requested when tile T-1 has been read by every wave.
-// SCALED: the queries carry scale * log2(e), and S^T starts from minus the running maximum instead of zero, so that the logits leave the MFMAs
-// as exponents of 2: 16 multiply-adds per block less, of about 70 vector instructions beside 8 MFMAs that hardly overlap them (busy 59 + 37 % of
-// the time).  The rows' maxima are exchanged between the lane halves only where one has grown.  16 / 48 x 2 705 tokens: 57.1 / 143 us without, 53.9 / 134 with.
-// The forward takes it: its queries are rounded to bf16 once, behind the scale.  The instance without is for callers whose queries are bf16 already
-// (rtvla_attention): rounded again behind the scale, their outputs' error against 64 bits would go from 2.3e-3 to 3.0e-3, in sharp rows (logits of
-// standard deviation 6) from 1.7e-3 to 4.8e-3.
 // All but this wave's newest N loads have landed, its LDS reads are back, and so for every wave of the workgroup
 template <int N> RTVLA_DEVICE void wait_and_meet() {
     __builtin_amdgcn_sched_barrier(0);
@@ -70,6 +59,19 @@ template <int N> RTVLA_DEVICE void wait_and_meet() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
 }
+
+// The key loop is software-pipelined over 32-key blocks so that every MFMA has independent VALU work to run under: while
+// the softmax of block g is computed (VALU), the matrix pipe takes S^T of block g+1 and O^T += V^T P^T of block g-1.
+// A block needs 8 MFMAs (256 cycles) and ~65 VALU instructions of one wave; issued back to back by one wave, or by
+// several waves in turn, the two streams mostly add up on a SIMD, interleaved one MFMA to a handful of VALU
+// instructions they overlap.  Three LDS stages: tile T+2 is requested when tile T-1 has been read by every wave.
+// SCALED: the queries carry scale * log2(e), and S^T starts from minus the running maximum instead of zero, so that the logits leave the MFMAs
+// as exponents of 2: 16 multiply-adds per block less, of about 70 vector instructions beside 8 MFMAs that hardly overlap them (busy 59 + 37 % of
+// the time).  The rows' maxima are exchanged between the lane halves only where one has grown.  16 / 48 x 2 705 tokens, when this was introduced: 57.1 / 143 us
+// without, 53.9 / 134 with.
+// The forward takes it: its queries are rounded to bf16 once, behind the scale.  The instance without is for callers whose queries are bf16 already
+// (rtvla_attention): rounded again behind the scale, their outputs' error against 64 bits would go from 2.3e-3 to 3.0e-3, in sharp rows (logits of
+// standard deviation 6) from 1.7e-3 to 4.8e-3.
 template <int HD, bool SCALED>
 __global__ __launch_bounds__(256, 3)
 void flash_kernel(AttnP p, int items_per_batch, int batches_per_xcd) {

@@ -28,6 +28,7 @@ RTVLA_DEVICE bf16x8 cat44(bf16x4 lo, bf16x4 hi) {
     return v;
 }
 RTVLA_DEVICE f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+
 // SUFFIX: keys past the prefix, all of them for rows past the state's, which see the first only.  An instance of its own, without which a launch
 // of the others takes 0.1 - 0.2 us more.  us of rtvla_attention, its passes over the operands included, with a suffix of a tenth of the keys, one row tile / this: Gemma 1 000 tokens 37.4 / 30.6,
 // 2 048 95.8 / 73.8, 5 120 453 / 320; causal 607 24.4 / 19.9, 2 107 84.6 / 64.5.
