@@ -7,12 +7,12 @@
 // waves, so there is nothing that two of them would share in LDS.
 //
 // What bounds it: a CU's load path.  788 tokens are 197 workgroups that pull 807 KB each, 6.2 us at 64 bytes per clock; with the launch (1.7), the first loads (2) and the merge
-// (2) that is 12 of the 13.3 us.  The kernel of csrc/attention.hip with two row tiles per workgroup, which it replaces here, took 64 products of 22 cycles, two softmaxes and two bursts
+// (2) that is 12 of the 13.0 us.  The kernel of csrc/attention.hip with two row tiles per workgroup, which it replaces here, took 64 products of 22 cycles, two softmaxes and two bursts
 // of 16 loads a block one after another, and waited for all its loads before the first product, because it asked for them behind a branch.  us with that / with this, weights
-// cold: 683 tokens 17.7 / 12.1, 768 17.3 / 12.4, 788 18.7 / 13.3, 968 22.3 / 16.6, 1 540 53.2 / 38.5, 2 048 63.3 / 52.4.
+// cold, both in turn on one machine: 683 tokens 16.3 / 11.9, 768 16.0 / 12.4, 788 17.9 / 13.0, 968 19.7 / 15.6, 1 540 50.7 / 37.8, 2 048 60.1 / 50.5 (one row tile: csrc/kernels.h).
 // CAUSAL: 38 row blocks of 607 tokens are 304 workgroups of one to nineteen key blocks, two to a CU; those with the most start first.  The work itself is small (2.4 us of products and 1.5 of
-// loads if it were even): most of the 7.9 us are the launch, the first loads and the longest workgroups' five trips.  It replaces 16x16x32 products with one row tile, three workgroups
-// to a CU: 269 / 438 / 607 / 2 107 tokens 6.3 / 8.8 / 11.1 / 48.3 -> 5.45 / 6.4 / 7.9 / 30.6.
+// loads if it were even): most of the 7.6 us are the launch, the first loads and the longest workgroups' five trips.  It replaces 16x16x32 products with one row tile, three workgroups
+// to a CU (two row tiles at 2 107 tokens): 269 / 438 / 607 / 2 107 tokens 6.3 / 7.9 / 11.1 / 46.9 -> 5.4 / 6.4 / 7.6 / 30.4.
 // (Built with the MFMA results in ordinary registers: 788 tokens 23 us otherwise, of copies and spills.)
 #include "kernels.h"
 #include <atomic>
@@ -124,7 +124,7 @@ void prefix_attn_kernel(AttnP p) {
         if (edge) mask(kb, s_cur);
         // The largest probability of a row so far is exactly 1, and each is rounded to bf16 once: the maximum follows every block, and the accumulators are scaled behind the
         // products of block kb - 4, whose probabilities are relative to the maximum before.  (Scaled ahead of them, with those probabilities, and only where the maximum has grown by
-        // 8 bits, the error against 64 bits was 1.08 times as large, in rows of sharp logits 1.18 times; 788 tokens took 12.8 us instead of 13.3, DM0's 607 7.7 instead of 7.9.)
+        // 8 bits, the error against 64 bits was 1.08 times as large, in rows of sharp logits 1.18 times; it was 0.5 us faster at 788 tokens and 0.2 at DM0's 607.)
         const float m_old = m;
         m = fmaxf(m, halves_max(lane_max(s_cur)));
         const float alpha = __builtin_amdgcn_exp2f((m_old - m) * c);
